@@ -3,12 +3,12 @@
 // Backward semantics: include/ops/backward/embedding_backward.h:35-42. The
 // reference scatters with storage-dtype atomics (src/ops/backward/embedding_backward.cu:68-92),
 // so its rounding depends on arrival order. Here the tokens are grouped by id with a counting
-// sort over the vocabulary (integer work: histogram, scan, fill — one launch), then one wavefront
-// per vocabulary row adds that row's tokens in ascending token order with one rounding to the
+// sort over the vocabulary (integer work: histogram, scan, fill — one launch), then each
+// vocabulary row's tokens are added in ascending token order with one rounding to the
 // storage dtype per add — the arithmetic of the reference's CPU operator
-// (src/ops/cpu/backward/embedding_backward_cpu.cpp:99-112). The result is deterministic and no
-// float atomics are used. Lanes cover the hidden dimension with 128-bit accesses, so each token
-// row is read once, fully coalesced; rows that no token names are zero-filled by the same launch
+// (src/ops/cpu/backward/embedding_backward_cpu.cpp:99-112) — by one wavefront for most ids, by a
+// workgroup per 64 columns for frequent ones. The result is deterministic and no float atomics are
+// used. Token rows are read once with coalesced 128-bit accesses; rows that no token names are zero-filled by the same launch
 // when the gradient is not accumulated.
 #include "common.hpp"
 
@@ -112,12 +112,163 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
     });
 }
 
-// ---- rows: one wavefront per vocabulary row -------------------------------------------------------
+// ---- rows ------------------------------------------------------------------------------------------
 // Adds, into row `id` of the table, the rows of grad_output of the tokens with that id, in ascending token
-// order with one rounding to the storage dtype per add. Segments of up to 64 tokens are ordered in registers
-// (lane i holds the token of rank i); longer ones are walked by scanning the id list itself, 64 tokens per
-// step, which yields them in ascending order by construction. Rows without tokens are zero-filled unless the
-// gradient is accumulated.
+// order with one rounding to the storage dtype per add. Rows without tokens are zero-filled unless the gradient
+// is accumulated. Bound by HBM (three rows per token) as long as the serial chain of additions of the most
+// frequent id is short; text makes it long: the first ids of a vocabulary take several per cent of a batch each.
+//   * Segments of up to kShort tokens: one wavefront per id, tokens ordered in registers (lane i holds the token
+//     of rank i), lanes across the columns, kAhead token rows in flight.
+//   * Longer ones: one workgroup per id and kSlice columns, so that a frequent id occupies hidden / kSlice
+//     workgroups instead of one wavefront. The segment is put into ascending order window by window through a
+//     bitmap of token positions in LDS; all threads fetch the slices of the next kBatch token rows while the first
+//     wavefront adds the previous ones, one column per lane, from LDS. The chain is then bound by the latency of
+//     add + round, about 20 cycles per token.
+// Both live in one launch, the long segments' workgroups first. 32768 tokens x 1024 columns, ids Zipf distributed
+// over 32000: 1846 -> 66 us (of which the most frequent id, 6.7 per cent of the tokens, sets the end).
+constexpr unsigned int kShort = 64;      // tokens: one lane each
+constexpr unsigned int kSlice = 64;      // columns of a long segment's workgroup: one lane each, one or two cache lines
+constexpr unsigned int kBatch = 128;     // token rows per step of a long segment
+constexpr unsigned int kWindow = 4096;   // token positions covered by the bitmap at a time
+
+template <typename T, bool Vector>
+__device__ __forceinline__ void embedding_short_row(T* __restrict__ row, const T* __restrict__ grad_output,
+                                                    const unsigned int* __restrict__ segment, unsigned int tokens,
+                                                    unsigned int hidden, bool accumulate) {
+    constexpr int VEC = Vector ? kVec128<T> : 1;
+    constexpr unsigned int kAhead = 8;
+    using vec_f = vec_t<float, VEC>;
+    const unsigned int lane = threadIdx.x & (kWave - 1);
+    if (tokens == 0) {
+        if (!accumulate)
+            for (unsigned int col = lane * VEC; col < hidden; col += kWave * VEC) store_vec<T, VEC>(row + col, vec_t<T, VEC>(0));
+        return;
+    }
+    const unsigned int mine = lane < tokens ? segment[lane] : 0xFFFFFFFFu;
+    // rank = number of tokens of the segment below mine; sorted = the token of rank `lane`.
+    unsigned int rank = 0;
+    for (unsigned int j = 0; j < tokens; ++j)
+        rank += static_cast<unsigned int>(__builtin_amdgcn_readlane(static_cast<int>(mine), static_cast<int>(j))) < mine ? 1u : 0u;
+    const unsigned int sorted = static_cast<unsigned int>(
+        __builtin_amdgcn_ds_permute(static_cast<int>(rank << 2), static_cast<int>(mine)));  // lane `rank` receives mine
+    for (unsigned int col = lane * VEC; col < hidden; col += kWave * VEC) {
+        vec_f acc = accumulate ? vec_to_f32<T, VEC>(load_vec<T, VEC>(row + col)) : vec_f(0.0f);
+        // kAhead token rows are requested at a time; the additions keep their order.
+        for (unsigned int j0 = 0; j0 < tokens; j0 += kAhead) {
+            vec_t<T, VEC> dy[kAhead];
+#pragma unroll
+            for (unsigned int u = 0; u < kAhead; ++u)
+                if (j0 + u < tokens) {
+                    const auto token = static_cast<unsigned int>(
+                        __builtin_amdgcn_readlane(static_cast<int>(sorted), static_cast<int>(j0 + u)));
+                    dy[u] = load_vec<T, VEC>(grad_output + static_cast<std::size_t>(token) * hidden + col);
+                }
+#pragma unroll
+            for (unsigned int u = 0; u < kAhead; ++u)
+                if (j0 + u < tokens)  // one rounding to the storage dtype per add
+                    acc = vec_to_f32<T, VEC>(vec_from_f32<T, VEC>(acc + vec_to_f32<T, VEC>(dy[u])));
+        }
+        store_vec<T, VEC>(row + col, vec_from_f32<T, VEC>(acc));
+    }
+}
+
+template <typename T, bool Vector>
+struct LongRow {
+    static constexpr unsigned int kVec = Vector ? kVec128<T> : 1;
+    static constexpr unsigned int kChunks = kSlice / kVec;                    // loads per token and slice
+    static constexpr unsigned int kPerThread = kBatch * kChunks / kThreads;   // loads per thread and batch
+    struct Shared {
+        alignas(16) T rows[kBatch][kSlice];
+        unsigned short list[kWindow];            // token positions of the window, ascending, relative to its start
+        unsigned int words[kWindow / 32];
+        unsigned int wave_counts[kWavesPerBlock];
+    };
+};
+
+template <typename T, bool Vector>
+__device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::Shared& lds, T* __restrict__ row,
+                                                   const T* __restrict__ grad_output, const unsigned int* __restrict__ segment,
+                                                   unsigned int tokens, unsigned int count, unsigned int col0,
+                                                   unsigned int hidden, bool accumulate) {
+    using L = LongRow<T, Vector>;
+    using chunk_t = vec_t<T, static_cast<int>(L::kVec)>;
+    static_assert(kWindow / 32 <= kThreads && kThreads / kWave == kWavesPerBlock, "a thread owns at most one bitmap word");
+    const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const unsigned int col = col0 + lane;
+    float acc = 0.0f;
+    if (wave == 0 && accumulate && col < hidden) acc = to_f32(row[col]);
+    for (unsigned int base = 0; base < count; base += kWindow) {
+        // The window's tokens of this segment in ascending order.
+        if (tid < kWindow / 32) lds.words[tid] = 0;
+        __syncthreads();
+        for (unsigned int i = tid; i < tokens; i += kThreads) {
+            const unsigned int position = segment[i] - base;  // wraps below the window
+            if (position < kWindow) atomicOr(&lds.words[position / 32], 1u << (position % 32));
+        }
+        __syncthreads();
+        unsigned int word = tid < kWindow / 32 ? lds.words[tid] : 0u;
+        const unsigned int mine = __popc(word);
+        unsigned int inclusive = mine;
+#pragma unroll
+        for (int offset = 1; offset < kWave; offset <<= 1) {
+            const unsigned int other = __shfl_up(inclusive, offset, kWave);
+            if (lane >= static_cast<unsigned int>(offset)) inclusive += other;
+        }
+        if (lane == kWave - 1) lds.wave_counts[wave] = inclusive;
+        __syncthreads();
+        unsigned int slot = inclusive - mine, found = 0;
+        for (unsigned int w = 0; w < kWavesPerBlock; ++w) {
+            if (w < wave) slot += lds.wave_counts[w];
+            found += lds.wave_counts[w];
+        }
+        while (word != 0) {
+            lds.list[slot++] = static_cast<unsigned short>(tid * 32 + __builtin_ctz(word));
+            word &= word - 1;
+        }
+        __syncthreads();
+        // Loads of the batch that starts at list entry `first`, into registers.
+        chunk_t held[L::kPerThread];
+        auto fetch = [&](unsigned int first) {
+#pragma unroll
+            for (unsigned int u = 0; u < L::kPerThread; ++u) {
+                const unsigned int index = u * kThreads + tid;
+                const unsigned int entry = first + index / L::kChunks, column = col0 + index % L::kChunks * L::kVec;
+                if (entry < found && column < hidden)
+                    held[u] = load_vec<T, static_cast<int>(L::kVec)>(
+                        grad_output + static_cast<std::size_t>(base + lds.list[entry]) * hidden + column);
+            }
+        };
+        fetch(0);
+        for (unsigned int first = 0; first < found; first += kBatch) {
+#pragma unroll
+            for (unsigned int u = 0; u < L::kPerThread; ++u) {
+                const unsigned int index = u * kThreads + tid;
+                store_vec<T, static_cast<int>(L::kVec)>(&lds.rows[index / L::kChunks][index % L::kChunks * L::kVec], held[u]);
+            }
+            __syncthreads();
+            if (first + kBatch < found) fetch(first + kBatch);
+            if (wave == 0) {
+                const unsigned int n = min(kBatch, found - first);
+                unsigned int j = 0;
+                for (; j + 16 <= n; j += 16) {
+                    T dy[16];
+#pragma unroll
+                    for (unsigned int u = 0; u < 16; ++u) dy[u] = lds.rows[j + u][lane];
+#pragma unroll
+                    for (unsigned int u = 0; u < 16; ++u) acc = round_to<T>(acc + to_f32(dy[u]));
+                }
+                for (; j < n; ++j) acc = round_to<T>(acc + to_f32(lds.rows[j][lane]));
+            }
+            __syncthreads();
+        }
+    }
+    if (wave == 0 && col < hidden) row[col] = from_f32<T>(acc);
+}
+
+// Workgroups [0, long_groups): long segments. A segment of more than kShort = 64 tokens contains a position of
+// `order` that is a multiple of 64; the first one in it names the segment, so candidate j looks at the id of the
+// token at position 64 j and leaves unless that id's segment is long and 64 j its first multiple. The remaining
+// workgroups take kWavesPerBlock ids each and leave the long ones out.
 template <typename T, bool Vector>
 __global__ __launch_bounds__(kThreads) void embedding_rows_kernel(T* __restrict__ grad_weight,
                                                                  const T* __restrict__ grad_output,
@@ -125,67 +276,26 @@ __global__ __launch_bounds__(kThreads) void embedding_rows_kernel(T* __restrict_
                                                                  const unsigned int* __restrict__ offsets,
                                                                  const unsigned int* __restrict__ order,
                                                                  unsigned int count, unsigned int vocab,
-                                                                 unsigned int hidden, bool accumulate) {
-    constexpr int VEC = Vector ? kVec128<T> : 1;
-    using vec_f = vec_t<float, VEC>;
-    const unsigned int lane = threadIdx.x & (kWave - 1);
-    const unsigned int id = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+                                                                 unsigned int hidden, unsigned int slices,
+                                                                 unsigned int long_groups, bool accumulate) {
+    __shared__ typename LongRow<T, Vector>::Shared lds;
+    if (blockIdx.x < long_groups) {
+        const unsigned int candidate = blockIdx.x / slices, slice = blockIdx.x - candidate * slices;
+        const unsigned int position = candidate * kShort;
+        if (position >= offsets[vocab]) return;  // ids past the vocabulary have no place in `order`
+        const unsigned int id = ids[order[position]];
+        const unsigned int begin = offsets[id], tokens = offsets[id + 1] - begin;
+        if (tokens <= kShort || position - begin >= kShort) return;
+        embedding_long_row<T, Vector>(lds, grad_weight + static_cast<std::size_t>(id) * hidden, grad_output, order + begin,
+                                      tokens, count, slice * kSlice, hidden, accumulate);
+        return;
+    }
+    const unsigned int id = (blockIdx.x - long_groups) * kWavesPerBlock + threadIdx.x / kWave;
     if (id >= vocab) return;
     const unsigned int begin = offsets[id], tokens = offsets[id + 1] - begin;
-    T* row = grad_weight + static_cast<std::size_t>(id) * hidden;
-    if (tokens == 0) {
-        if (!accumulate)
-            for (unsigned int col = lane * VEC; col < hidden; col += kWave * VEC) store_vec<T, VEC>(row + col, vec_t<T, VEC>(0));
-        return;
-    }
-    auto add_row = [&](vec_f acc, unsigned int token, unsigned int col) {
-        const vec_f dy = vec_to_f32<T, VEC>(load_vec<T, VEC>(grad_output + static_cast<std::size_t>(token) * hidden + col));
-        return vec_to_f32<T, VEC>(vec_from_f32<T, VEC>(acc + dy));  // one rounding to the storage dtype per add
-    };
-    if (tokens <= kWave) {
-        const unsigned int mine = lane < tokens ? order[begin + lane] : 0xFFFFFFFFu;
-        // rank = number of tokens of the segment below mine; sorted = the token of rank `lane`.
-        unsigned int rank = 0;
-        for (unsigned int j = 0; j < tokens; ++j)
-            rank += static_cast<unsigned int>(__builtin_amdgcn_readlane(static_cast<int>(mine), static_cast<int>(j))) < mine ? 1u : 0u;
-        const unsigned int sorted = static_cast<unsigned int>(
-            __builtin_amdgcn_ds_permute(static_cast<int>(rank << 2), static_cast<int>(mine)));  // lane `rank` receives mine
-        for (unsigned int col = lane * VEC; col < hidden; col += kWave * VEC) {
-            vec_f acc = accumulate ? vec_to_f32<T, VEC>(load_vec<T, VEC>(row + col)) : vec_f(0.0f);
-            // Four token rows are requested at a time; the additions keep their order.
-            for (unsigned int j0 = 0; j0 < tokens; j0 += 4) {
-                vec_t<T, VEC> dy[4];
-#pragma unroll
-                for (unsigned int u = 0; u < 4; ++u)
-                    if (j0 + u < tokens) {
-                        const auto token = static_cast<unsigned int>(
-                            __builtin_amdgcn_readlane(static_cast<int>(sorted), static_cast<int>(j0 + u)));
-                        dy[u] = load_vec<T, VEC>(grad_output + static_cast<std::size_t>(token) * hidden + col);
-                    }
-#pragma unroll
-                for (unsigned int u = 0; u < 4; ++u)
-                    if (j0 + u < tokens)  // one rounding to the storage dtype per add
-                        acc = vec_to_f32<T, VEC>(vec_from_f32<T, VEC>(acc + vec_to_f32<T, VEC>(dy[u])));
-            }
-            store_vec<T, VEC>(row + col, vec_from_f32<T, VEC>(acc));
-        }
-        return;
-    }
-    for (unsigned int col0 = 0; col0 < hidden; col0 += kWave * VEC) {
-        const unsigned int col = col0 + lane * VEC;
-        const bool live = col < hidden;
-        vec_f acc = (accumulate && live) ? vec_to_f32<T, VEC>(load_vec<T, VEC>(row + col)) : vec_f(0.0f);
-        for (unsigned int first = 0; first < count; first += kWave) {
-            const unsigned int t = first + lane;
-            unsigned long long matches = __ballot(t < count && ids[t] == id);  // every lane takes part
-            while (matches != 0) {
-                const unsigned int token = first + static_cast<unsigned int>(__builtin_ctzll(matches));
-                matches &= matches - 1;
-                if (live) acc = add_row(acc, token, col);
-            }
-        }
-        if (live) store_vec<T, VEC>(row + col, vec_from_f32<T, VEC>(acc));
-    }
+    if (tokens <= kShort)
+        embedding_short_row<T, Vector>(grad_weight + static_cast<std::size_t>(id) * hidden, grad_output, order + begin, tokens,
+                                       hidden, accumulate);
 }
 
 template <typename T, bool Vector>
@@ -257,15 +367,17 @@ extern "C" int cgptx_embedding_backward(void* grad_weight, const void* grad_outp
         auto* dw = static_cast<T*>(grad_weight);
         auto* dy = static_cast<const T*>(grad_output);
         const bool vector_ok = hidden % kVec128<T> == 0 && is_aligned16(dw) && is_aligned16(dy);
-        const dim3 grid((v + kWavesPerBlock - 1) / kWavesPerBlock);
         const auto h = static_cast<unsigned int>(hidden);
-        if (vector_ok) {
-            hipLaunchKernelGGL((embedding_rows_kernel<T, true>), grid, dim3(kThreads), 0, stream, dw, dy, token_ids, offsets,
-                               order, count, v, h, accumulate_weight != 0);
-        } else {
-            hipLaunchKernelGGL((embedding_rows_kernel<T, false>), grid, dim3(kThreads), 0, stream, dw, dy, token_ids, offsets,
-                               order, count, v, h, accumulate_weight != 0);
-        }
+        // Candidates for long segments: one per kShort positions of `order` and slice of the columns.
+        const std::size_t slices = (hidden + kSlice - 1) / kSlice;
+        const std::size_t long_groups = token_count > kShort ? (token_count + kShort - 1) / kShort * slices : 0;
+        const std::size_t short_groups = (vocab + kWavesPerBlock - 1) / kWavesPerBlock;
+        if (long_groups + short_groups > static_cast<std::size_t>(std::numeric_limits<int>::max()))
+            return fail(CGPTX_OVERFLOW, std::string(name) + ": too many workgroups");
+        const dim3 grid(static_cast<unsigned int>(long_groups + short_groups));
+        auto kernel = vector_ok ? embedding_rows_kernel<T, true> : embedding_rows_kernel<T, false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, dw, dy, token_ids, offsets, order, count, v, h,
+                           static_cast<unsigned int>(slices), static_cast<unsigned int>(long_groups), accumulate_weight != 0);
         CGPTX_LAUNCH_CHECK();
         return CGPTX_OK;
     });

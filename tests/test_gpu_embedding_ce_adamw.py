@@ -301,3 +301,30 @@ def test_adamw_matches_cpu_restatement_single_tensor(device):
     assert_close(dp, p, 1e-6, "param")
     assert_close(state.first_moment, m, 1e-6, "m")
     assert_close(state.second_moment, v, 1e-6, "v")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("tokens,hidden,frequent", [
+    (64, 64, 64), (65, 64, 65),            # the longest segment of one wavefront, the shortest of a workgroup
+    (300, 72, 129), (300, 33, 130),        # one row past a batch of 128; a partial and an unaligned slice of columns
+    (4200, 128, 4097), (9000, 96, 8000),     # segments over two and three windows of 4096 positions
+])
+def test_embedding_backward_frequent_ids_bit_exact(device, tokens, hidden, frequent, dtype):
+    """Ids that take a large share of the batch, between other ids and ids past the vocabulary."""
+    vocab = 50
+    g = torch.Generator().manual_seed(tokens + hidden)
+    ids = torch.randint(0, vocab + 3, (tokens,), generator=g)
+    where = torch.randperm(tokens, generator=g)[:frequent]
+    ids[where] = torch.where(torch.arange(frequent) % 3 == 0, 7, 8) if frequent > 1000 else 7
+    dy = randn((tokens, hidden), dtype, 3)
+    for accumulate in (False, True):
+        want = randn((vocab, hidden), dtype, 4)
+        got = want.to(device)
+        # Additions in token order, each rounded to the storage type; ids past the vocabulary are skipped.
+        base = want.clone() if accumulate else torch.zeros_like(want)
+        for i in range(tokens):
+            if ids[i] < vocab:
+                base[ids[i]] = (base[ids[i]].float() + dy[i].float()).to(dtype)
+        ops.embedding_backward(got, dy.to(device), ids.to(torch.int32).to(device), tokens,
+                               options=ops.EmbeddingBackwardOptions(accumulate_weight=accumulate))
+        assert torch.equal(got.cpu(), base)
