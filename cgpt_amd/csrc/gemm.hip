@@ -39,9 +39,10 @@
 //     fp32 partial tiles go to scratch and a second kernel adds them in slice order
 //     (deterministic), applying accumulate and the dtype conversion.
 //
-// Shapes the streamed path does not cover (K not a multiple of 32, leading dimensions
-// or pointers not 16-byte aligned, fp32 storage) run on an fp32 matrix-core kernel
-// (v_mfma_f32_32x32x2_f32, register-staged operand tiles) with the same semantics.
+// Operands whose rows are not whole aligned 16-byte chunks are copied to padded rows first;
+// C may have any width and alignment (a store per element). fp32 storage, and 16-bit operands
+// beyond 32-bit offsets, run on an fp32 matrix-core kernel (v_mfma_f32_32x32x2_f32,
+// register-staged operand tiles) with the same semantics.
 #include "gemm.hpp"
 
 #include <algorithm>
@@ -57,8 +58,9 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kBK = 32;          // K step per LDS stage
 // LDS stages of a block: one being multiplied, one being refilled, the rest in flight. 256x256
-// blocks own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each).
-constexpr int stages_for(int /*bm*/, int /*bn*/) { return 5; }
+// blocks own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each), and so do 64x64
+// blocks: their K tiles are short (4 MFMAs per wavefront), so ten 8 KiB stages keep as many bytes in flight.
+constexpr int stages_for(int bm, int /*bn*/) { return bm == 64 ? 10 : 5; }
 constexpr int kXcds = 8;
 
 
@@ -113,6 +115,12 @@ struct KernelArgs {
     const float* addend;   // fp32 [M, N], row stride ld_addend, added before anything else, or null
     long ld_addend;
     int m, n, k;
+    // What the operands hold: rows or columns of A and of B (A's may exceed m, B's n: whole 16-byte chunks of padded
+    // rows), K positions of B (below k when A's padding reaches further: past them B reads as zeros).
+    int a_extent, b_extent, b_k;
+    int k_tiles;            // K tiles of kBK, the last one possibly short
+    int ragged;             // C (or an addend) has rows that are not whole 16-byte chunks: stored element by element
+    long ld_partial;        // SPLIT kernels: row length of a partial tile matrix
     long lda, ldb, ldc, ldr;
     int tiles_m, tiles_n;
     int k_tiles_per_slice;  // K tiles handled by one work item
@@ -277,15 +285,18 @@ struct KTile {
 // ---- operand stored [K, COLS] (n-contiguous): 32 x COLS slab kept in that order in LDS ---------
 // The transpose happens on the way out of LDS: ds_read_b64_tr_b16 hands lane n of a 16-lane group
 // the four k-values of column n from a 4(k) x 16(n) block, so two of them build the 8-k fragment of
-// one column. swizzle(k row) = 4*(row%4) on the chunk index: the four k rows that 32 lanes read sit
-// in four different 64-byte windows of the 256-byte bank period.
+// one column. swizzle(k row) = 4*(row%4) on the chunk index (rows of 128 bytes: 4*(row/2%2), the row's parity
+// picks the half already): the four k rows that 32 lanes read sit in four different 64-byte windows of the
+// 256-byte bank period. K rows past the operand's end are out of the buffer's range and read as zeros.
 template <typename T, int COLS>
 struct NTile {
     using frag_t = typename Mfma<T>::frag;
     static constexpr int kChunksPerRow = COLS / 8;
-    static constexpr int kRowsPerLoad = 64 / kChunksPerRow;  // k rows one load instruction covers (2 or 4)
+    static constexpr int kRowsPerLoad = 64 / kChunksPerRow;  // k rows one load instruction covers (2, 4 or 8)
     static constexpr int kElems = kBK * COLS;
     static constexpr int kLoads = kBK / kRowsPerLoad / kWaves;
+
+    __device__ __forceinline__ static int swizzle(int k_row) { return COLS >= 128 ? (k_row & 3) << 2 : (k_row & 2) << 1; }
 
     u32x4 rsrc = {0u, 0u, 0u, 0u};
     int voffset = 0;
@@ -298,7 +309,7 @@ struct NTile {
         rsrc = make_rsrc(base, (static_cast<long>(k_total - 1) * ld + cols_left) * static_cast<long>(sizeof(T)));
         const int row = lane / kChunksPerRow;                  // within the instruction's rows
         const int k_row = (wave * kRowsPerLoad + row) & 3;     // low bits of the tile row (groups step by 4*kRowsPerLoad)
-        const int chunk = min((lane % kChunksPerRow) ^ (k_row << 2), cols_left / 8 - 1);
+        const int chunk = min((lane % kChunksPerRow) ^ swizzle(k_row), cols_left / 8 - 1);
         voffset = static_cast<int>(row * ld * sizeof(T)) + chunk * 16;
         group_bytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(kRowsPerLoad * ld * sizeof(T)));
     }
@@ -312,7 +323,7 @@ struct NTile {
     // multiple of 16.
     __device__ __forceinline__ static int lane_offset(int lane, int block0) {
         const int k_row = (lane >> 4) * 8 + ((lane & 15) >> 2);
-        const int chunk = ((block0 / 8) ^ ((k_row & 3) << 2)) + ((lane & 3) >> 1);
+        const int chunk = ((block0 / 8) ^ swizzle(k_row)) + ((lane & 3) >> 1);
         return k_row * COLS + chunk * 8 + (lane & 1) * 4;
     }
     __device__ __forceinline__ static frag_t frag(const T* tile, int offset) {
@@ -417,7 +428,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         w.m0 = (first_m + in_group - column * rows_in_group) * BM;
         w.n0 = column * BN;
         w.kt_begin = w.slice * p.k_tiles_per_slice;
-        w.kt_end = min(p.k / kBK, w.kt_begin + p.k_tiles_per_slice);
+        w.kt_end = min(p.k_tiles, w.kt_begin + p.k_tiles_per_slice);
         return w;
     };
 
@@ -435,7 +446,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         src_end = w.kt_end;
         long b_shift = 0;
         if constexpr (A_K && !SEGMENTED) {
-            a_src.init(static_cast<const T*>(p.a) + static_cast<long>(m0) * p.lda, p.lda, p.m - m0, p.k, wave);
+            a_src.init(static_cast<const T*>(p.a) + static_cast<long>(m0) * p.lda, p.lda, p.a_extent - m0, p.k, wave);
         } else if constexpr (A_K) {
             // All three sources are set up unconditionally (absent segments repeat the first and
             // are never selected): conditional set-up would be merged into one piece of code that
@@ -458,7 +469,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         } else {
             // Stacked products: the tile's rows of C name the product, and the operands move with it.
             long product = 0;
-            int local_m0 = m0, rows = p.m;
+            int local_m0 = m0, rows = p.a_extent;
             if constexpr (!B_K) {
                 if (p.batch_rows > 0) {
                     product = m0 / p.batch_rows;
@@ -482,8 +493,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
             a_src.init(base + (local_m0 - first), ld, width - (local_m0 - first), p.k, wave);
         }
         if constexpr (SWIGLU) b_src.init(static_cast<const T*>(p.b) + static_cast<long>(n0 / 2) * p.ldb, p.ldb, p.n - n0 / 2, p.k, wave);
-        else if constexpr (B_K) b_src.init(static_cast<const T*>(p.b) + static_cast<long>(n0) * p.ldb, p.ldb, p.n - n0, p.k, wave);
-        else b_src.init(static_cast<const T*>(p.b) + b_shift + n0, p.ldb, p.n - n0, p.k, wave);
+        else if constexpr (B_K) b_src.init(static_cast<const T*>(p.b) + static_cast<long>(n0) * p.ldb, p.ldb, p.b_extent - n0, p.b_k, wave);
+        else b_src.init(static_cast<const T*>(p.b) + b_shift + n0, p.ldb, p.b_extent - n0, p.b_k, wave);
     };
     // K tiles past the end of the slice are still "loaded" (the loop stays free of data-dependent
     // branches and every wavefront always has the same number of loads in flight), but from an
@@ -870,7 +881,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
             return;
         }
         bool plain = false;
-        if constexpr (!SPLIT) plain = p.bias == nullptr && p.residual == nullptr && p.addend == nullptr && !p.accumulate && !p.c_f32;
+        if constexpr (!SPLIT) plain = p.bias == nullptr && p.residual == nullptr && p.addend == nullptr && !p.accumulate && !p.c_f32 && !p.ragged;
         if (plain) {
             // Straight-line code, no per-lane predicates or address arithmetic (with one wavefront per
             // SIMD every branch and every dependent wait is exposed): the stores go through a buffer
@@ -909,10 +920,11 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         }
         if constexpr (SPLIT) {
             const float* origin = static_cast<const float*>(p.c) +
-                                  (static_cast<long>(w.slice) * p.m + row0) * static_cast<long>(p.n) + (w.n0 + col0);
-            const int cols_left = min(WN, p.n - (w.n0 + col0));
-            const __amdgpu_buffer_rsrc_t rsrc = part_rsrc(origin, p.n, 4, rows_left, cols_left);
-            const int row_bytes = p.n * 4;
+                                  (static_cast<long>(w.slice) * p.m + row0) * p.ld_partial + (w.n0 + col0);
+            const int pitch = static_cast<int>(p.ld_partial);  // n rounded up to whole 16-byte chunks of storage
+            const int cols_left = min(WN, pitch - (w.n0 + col0));
+            const __amdgpu_buffer_rsrc_t rsrc = part_rsrc(origin, pitch, 4, rows_left, cols_left);
+            const int row_bytes = pitch * 4;
 #pragma unroll
             for (int r = 0; r < kRowBlocks; ++r) {
                 __builtin_amdgcn_sched_barrier(0);
@@ -932,6 +944,41 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
                         const int soffset = (r * 32 + u * kRowsF) * row_bytes;
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v0[u]), rsrc, voffset0, soffset, 0);
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v1[u]), rsrc, voffset1, soffset, 0);
+                    }
+                }
+            }
+            return;
+        }
+        if (p.ragged) {
+            // Rows of C that do not start on 16-byte boundaries: lanes along the columns of a staged half, one element
+            // each, so that a store instruction still covers one contiguous piece of a row (or of a few).
+            constexpr int kCols = WN / 2, kRowsE = kWave / kCols;
+            const int e_row = lane / kCols, e_col = lane % kCols;
+#pragma unroll
+            for (int r = 0; r < kRowBlocks; ++r) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (request) request_share(r);
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    stage.template operator()<float, TN / 2>(r, half * (TN / 2));
+                    const int col = half * kCols + e_col, n = w.n0 + col0 + col, c_col = c_col0 + col0 + col;
+                    const float bias = p.bias != nullptr && c_col < c_cols ? to_f32(static_cast<const T*>(p.bias)[n]) : 0.0f;
+#pragma unroll 4
+                    for (int u = 0; u < 32 / kRowsE; ++u) {
+                        const int row = u * kRowsE + e_row;
+                        float v = *reinterpret_cast<const float*>(region + row * kRowBytes + (((e_col / 4) ^ sw(row)) * 16) + (e_col % 4) * 4);
+                        const long m = row0 + r * 32 + row;
+                        if (m >= p.m || c_col >= c_cols) continue;
+                        if (p.addend != nullptr) v += p.addend[m * p.ld_addend + n];
+                        v += bias;
+                        if (p.residual != nullptr) v += to_f32(static_cast<const T*>(p.residual)[m * p.ldr + n]);
+                        if (p.c_f32) {
+                            float* out = static_cast<float*>(c_base) + m * c_ld + c_col;
+                            *out = p.accumulate ? v + *out : v;
+                        } else {
+                            T* out = static_cast<T*>(c_base) + m * c_ld + c_col;
+                            *out = from_f32<T>(p.accumulate ? v + to_f32(*out) : v);
+                        }
                     }
                 }
             }
@@ -1097,21 +1144,48 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     }
 }
 
-// C = Σ_slices partial (+ C) (+ bias), four columns per thread, slices in order.
+// C = Σ_slices partial (+ C) (+ bias), four columns per thread, slices in order. n: the partial rows' length, a
+// multiple of 4; columns past n_valid (rows of C that are not whole 16-byte chunks) are not stored.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(void* __restrict__ c,
                                                                 const float* __restrict__ partial,
-                                                                const T* __restrict__ bias, int m, int n, long ldc,
-                                                                int slices, int accumulate, int c_f32) {
+                                                                const T* __restrict__ bias, int m, int n, int n_valid,
+                                                                long ldc, int slices, int accumulate, int c_f32,
+                                                                int ragged) {
     const long quads = static_cast<long>(m) * (n / 4);
     const long stride = static_cast<long>(m) * n;
     for (long q = static_cast<long>(blockIdx.x) * kThreads + threadIdx.x; q < quads;
          q += static_cast<long>(gridDim.x) * kThreads) {
         const long row = q / (n / 4);
         const int col = static_cast<int>(q - row * (n / 4)) * 4;
-        vec_t<float, 4> v = *reinterpret_cast<const vec_t<float, 4>*>(partial + row * n + col);
-        for (int s = 1; s < slices; ++s)
-            v += *reinterpret_cast<const vec_t<float, 4>*>(partial + s * stride + row * n + col);
+        const float* source = partial + row * n + col;
+        // Four slices are requested at a time; the additions keep the slices' order.
+        vec_t<float, 4> v = *reinterpret_cast<const vec_t<float, 4>*>(source);
+        int s = 1;
+        for (; s + 4 <= slices; s += 4) {
+            vec_t<float, 4> part[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) part[u] = *reinterpret_cast<const vec_t<float, 4>*>(source + (s + u) * stride);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v += part[u];
+        }
+        for (; s < slices; ++s) v += *reinterpret_cast<const vec_t<float, 4>*>(source + s * stride);
+        if (ragged) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (col + e >= n_valid) continue;
+                float x = v[e];
+                if (bias != nullptr) x += to_f32(bias[col + e]);
+                if (c_f32) {
+                    float* out = static_cast<float*>(c) + row * ldc + col + e;
+                    *out = accumulate ? x + *out : x;
+                } else {
+                    T* out = static_cast<T*>(c) + row * ldc + col + e;
+                    *out = from_f32<T>(accumulate ? x + to_f32(*out) : x);
+                }
+            }
+            continue;
+        }
         if (bias != nullptr) v += vec_to_f32<T, 4>(load_vec<T, 4>(bias + col));
         if (c_f32) {
             float* out = static_cast<float*>(c) + row * ldc + col;
@@ -1122,6 +1196,27 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(void* __restric
             if (accumulate) v += vec_to_f32<T, 4>(load_vec<T, 4>(out));
             store_vec<T, 4>(out, vec_from_f32<T, 4>(v));
         }
+    }
+}
+
+// Copies a [rows, cols] matrix of 16-bit elements to rows of `pitch` elements (a multiple of 8), zeros past cols:
+// the streamed kernels read whole 16-byte chunks. Eight elements per thread; the source may start anywhere.
+__global__ __launch_bounds__(kThreads) void pad_rows_kernel(std::uint16_t* __restrict__ dst, const std::uint16_t* __restrict__ src,
+                                                            long rows, int cols, long ld, int pitch) {
+    const int chunks = pitch / 8;
+    const long total = rows * chunks;
+    for (long q = static_cast<long>(blockIdx.x) * kThreads + threadIdx.x; q < total; q += static_cast<long>(gridDim.x) * kThreads) {
+        const long row = q / chunks;
+        const int col = static_cast<int>(q - row * chunks) * 8;
+        const std::uint16_t* from = src + row * ld + col;
+        vec_t<std::uint16_t, 8> v;
+        if (col + 8 <= cols) {
+            __builtin_memcpy(&v, from, 16);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = col + e < cols ? from[e] : std::uint16_t{0};
+        }
+        store_vec<std::uint16_t, 8>(dst + row * pitch + col, v);
     }
 }
 
@@ -1170,7 +1265,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma_kernel(KernelArgs p, i
             a_regs[e] = (m < p.m && ka < p.k) ? to_f32(a_k ? A[m * p.lda + ka] : A[ka * p.lda + m]) : 0.0f;
             coordinates(e, b_k != 0, row, k);
             const long n = n0 + row, kb = k0 + k;
-            b_regs[e] = (n < p.n && kb < p.k) ? to_f32(b_k ? B[n * p.ldb + kb] : B[kb * p.ldb + n]) : 0.0f;
+            b_regs[e] = (n < p.n && n < p.b_extent && kb < p.b_k) ? to_f32(b_k ? B[n * p.ldb + kb] : B[kb * p.ldb + n]) : 0.0f;
         }
     };
     auto deposit = [&](int stage) {
@@ -1241,6 +1336,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma_kernel(KernelArgs p, i
 }
 
 // ------------------------------------------------------------------- host side
+constexpr int blocks_per_unit(int tile) { return tile == 256 ? 1 : 2; }  // resident blocks per CU: what the LDS stages allow
+
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
           bool SWIGLU = false, bool GRAD = false>
 int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
@@ -1270,7 +1367,7 @@ int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
         const bool exact = divisor > 1 && tiles * divisor < (1ul << 32);
         args.group_reciprocal = exact ? static_cast<unsigned int>(((1ul << 32) + divisor - 1) / divisor) : 0u;
     }
-    const long slots = static_cast<long>(compute_units()) * (BM == 256 ? 1 : 2) / kXcds * kXcds;
+    const long slots = static_cast<long>(compute_units()) * blocks_per_unit(BM) / kXcds * kXcds;
     const long blocks = std::min<long>((items + kXcds - 1) / kXcds * kXcds, std::max<long>(slots, kXcds));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), smem, stream, args);
     CGPTX_LAUNCH_CHECK();
@@ -1296,7 +1393,7 @@ int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream
     }
     if (p.saved != nullptr) return fail(CGPTX_RUNTIME, "gemm: the SwiGLU gradient epilogue needs 256-wide unsplit tiles");
     if constexpr (!SPLIT) {
-        if (a_k && b_k && p.bias == nullptr && p.addend == nullptr && !p.c_f32) {
+        if (a_k && b_k && p.bias == nullptr && p.addend == nullptr && !p.c_f32 && !p.ragged) {
             if (p.residual != nullptr && !p.accumulate) return launch_mfma<T, BM, BN, true, true, false, false, true>(p, slices, stream);
             if (p.residual == nullptr && p.accumulate && p.c_seg.count == 0) {
                 // C += A·B in the storage dtype is the same epilogue with C as its own residual
@@ -1315,34 +1412,59 @@ int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream
     return fail(CGPTX_RUNTIME, "gemm: unsupported operand layout");
 }
 
-// CGPTX_GEMM_TILE=128|256 pins the tile size (for experiments); anything else = automatic.
+// CGPTX_GEMM_TILE=64|128|256 pins the tile size (for experiments); anything else = automatic.
 int forced_tile() {
     static const int value = [] {
         const char* text = std::getenv("CGPTX_GEMM_TILE");
         if (text == nullptr) return 0;
         const int v = std::atoi(text);
-        return (v == 128 || v == 256) ? v : 0;
+        return (v == 64 || v == 128 || v == 256) ? v : 0;
     }();
     return value;
 }
 
-template <typename T, int BM, int BN>
-int run_config(const GemmArgs& g, KernelArgs p, hipStream_t stream) {
-    p.tiles_m = (p.m + BM - 1) / BM;
-    p.tiles_n = (p.n + BN - 1) / BN;
-    const int k_tiles = p.k / kBK;
-    const long tiles = static_cast<long>(p.tiles_m) * p.tiles_n;
-    const long want_blocks = static_cast<long>(compute_units()) * (BM == 256 ? 1 : 2);
+std::size_t round_up(std::size_t v, std::size_t unit) { return (v + unit - 1) / unit * unit; }
+
+// How a call of the streamed kernels is cut: tile edge, K slices per tile and K tiles per slice.
+struct Plan {
+    int tile = 256;
     int slices = 1;
-    const bool k_segments = g.a_k_contiguous && g.a_segments.count > 0;
-    const bool may_split = !g.no_split || g.split_workspace != nullptr;
-    if (may_split && g.residual == nullptr && g.addend_f32 == nullptr && g.swiglu_out == nullptr && g.swiglu_saved == nullptr &&
-        g.c_segments.count == 0 && !k_segments &&
-        tiles < want_blocks && k_tiles >= 32) {
+    int k_tiles_per_slice = 1;
+    std::size_t partial_bytes(const GemmArgs& g) const {
+        return slices > 1 ? static_cast<std::size_t>(slices) * g.m * round_up(g.n, 8) * sizeof(float) : 0;
+    }
+};
+
+Plan make_plan(const GemmArgs& g) {
+    Plan plan;
+    const long units = compute_units();
+    const long k_tiles = static_cast<long>((g.k + kBK - 1) / kBK);
+    auto tiles_of = [&](long edge) {
+        return static_cast<long>((g.m + edge - 1) / edge) * static_cast<long>((g.n + edge - 1) / edge);
+    };
+    const bool may_split = (!g.no_split || g.split_workspace != nullptr) && g.residual == nullptr && g.addend_f32 == nullptr &&
+                           g.swiglu_out == nullptr && g.swiglu_saved == nullptr && g.c_segments.count == 0 &&
+                           !(g.a_k_contiguous && g.a_segments.count > 0);
+    // 256x256 tiles (one block per CU, 64 MFMAs per wavefront and K step) when they still give
+    // every CU a tile, or when K is long enough to be split across the idle CUs without the
+    // fp32 partial tiles outweighing the contraction (at least 8 tiles, so at most 32 slices);
+    // otherwise 128x128 tiles, with K split when even those are too few, and 64x64 tiles where
+    // 128x128 ones would leave most of the chip idle.
+    const long big_tiles = tiles_of(256);
+    const bool fills = big_tiles * 5 >= units * 4;
+    const bool splits = may_split && big_tiles >= 8 && k_tiles >= 32 * ((units + big_tiles - 1) / big_tiles);
+    const int forced = forced_tile();
+    if (g.swiglu_out != nullptr || g.swiglu_saved != nullptr || g.batch_rows != 0) plan.tile = 256;
+    else if (forced != 0) plan.tile = forced;
+    else if (fills || splits) plan.tile = 256;
+    else plan.tile = tiles_of(128) >= units ? 128 : 64;
+    const long tiles = tiles_of(plan.tile);
+    const long want_blocks = units * blocks_per_unit(plan.tile);
+    long slices = 1;
+    if (may_split && tiles < want_blocks && k_tiles >= 32) {
         // As many slices as fit the CU slots in one go: one item more than that would cost a
         // second round of the persistent blocks.
-        slices = static_cast<int>(std::min<long>(want_blocks / tiles, k_tiles / 16));
-        if (slices < 1) slices = 1;
+        slices = std::max<long>(1, std::min<long>(want_blocks / tiles, k_tiles / 16));
     }
     if (g.batch_rows != 0 && may_split && k_tiles >= 32) {
         // A stack of products brings any number of tiles: the slice count that needs the least time, counted in
@@ -1357,22 +1479,32 @@ int run_config(const GemmArgs& g, KernelArgs p, hipStream_t stream) {
             }
         }
     }
-    if (g.no_split && static_cast<std::size_t>(slices) * g.m * g.n * sizeof(float) > g.split_workspace_bytes) slices = 1;
-    p.k_tiles_per_slice = (k_tiles + slices - 1) / slices;
-    slices = (k_tiles + p.k_tiles_per_slice - 1) / p.k_tiles_per_slice;
-    if (slices == 1) return launch_layout<T, BM, BN, false>(p, g.a_k_contiguous, g.b_k_contiguous, 1, stream);
+    plan.slices = static_cast<int>(slices);
+    if (g.no_split && plan.partial_bytes(g) > g.split_workspace_bytes) slices = 1;
+    plan.k_tiles_per_slice = static_cast<int>((k_tiles + slices - 1) / slices);
+    plan.slices = static_cast<int>((k_tiles + plan.k_tiles_per_slice - 1) / plan.k_tiles_per_slice);
+    return plan;
+}
+
+template <typename T, int BM, int BN>
+int run_config(const GemmArgs& g, const Plan& plan, KernelArgs p, hipStream_t stream) {
+    p.tiles_m = (p.m + BM - 1) / BM;
+    p.tiles_n = (p.n + BN - 1) / BN;
+    p.k_tiles_per_slice = plan.k_tiles_per_slice;
+    if (plan.slices == 1) return launch_layout<T, BM, BN, false>(p, g.a_k_contiguous, g.b_k_contiguous, 1, stream);
     void* mem = g.no_split ? g.split_workspace : nullptr;
     if (mem == nullptr) {
-        if (int s = scratch(stream, static_cast<std::size_t>(slices) * g.m * g.n * sizeof(float), &mem)) return s;
+        if (int s = scratch(stream, plan.partial_bytes(g), &mem)) return s;
     }
     KernelArgs split = p;
     split.c = mem;
-    if (int s = launch_layout<T, BM, BN, true>(split, g.a_k_contiguous, g.b_k_contiguous, slices, stream)) return s;
-    const long quads = static_cast<long>(p.m) * (p.n / 4);
+    split.ld_partial = static_cast<long>(round_up(g.n, 8));
+    if (int s = launch_layout<T, BM, BN, true>(split, g.a_k_contiguous, g.b_k_contiguous, plan.slices, stream)) return s;
+    const long quads = static_cast<long>(p.m) * (split.ld_partial / 4);
     const long blocks = std::min<long>((quads + kThreads - 1) / kThreads, static_cast<long>(compute_units()) * 8);
     hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), 0, stream,
-                       g.c, static_cast<const float*>(mem), static_cast<const T*>(g.bias), p.m, p.n, p.ldc, slices,
-                       p.accumulate, p.c_f32);
+                       g.c, static_cast<const float*>(mem), static_cast<const T*>(g.bias), p.m,
+                       static_cast<int>(split.ld_partial), p.n, p.ldc, plan.slices, p.accumulate, p.c_f32, p.ragged);
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
 }
@@ -1416,6 +1548,31 @@ bool offsets_fit_32bit(const GemmArgs& g, std::size_t elem) {
     return a_span < limit && b_span < limit && c_span < limit && r_span < limit;
 }
 
+// Which operands the streamed kernels can read as they lie: 16-byte aligned rows whose K range (k-contiguous) or
+// whose rows or columns (otherwise) are whole units of what a load instruction or a K tile covers. The K range of a
+// k-contiguous operand has to end with a K tile, since what lies behind it in the row is multiplied too; a k-strided
+// operand's may end anywhere (rows past it are out of the buffer's range).
+bool a_streams(const GemmArgs& g) {
+    return is_aligned16(g.a) && g.lda % 8 == 0 && (g.a_k_contiguous ? g.k % kBK == 0 : std::max(g.a_extent, g.m) % 8 == 0);
+}
+bool b_streams(const GemmArgs& g) {
+    return is_aligned16(g.b) && g.ldb % 8 == 0 && (g.b_k_contiguous ? g.k % kBK == 0 : std::max(g.b_extent, g.n) % 8 == 0);
+}
+// Whether C and what is added to it lie in whole aligned chunks.
+bool c_streams(const GemmArgs& g, std::size_t elem) {
+    const std::size_t c_elem = g.c_is_f32 ? 4 : elem;
+    return g.n % 8 == 0 && (g.ldc * c_elem) % 16 == 0 && is_aligned16(g.c) &&
+           (g.bias == nullptr || (reinterpret_cast<std::uintptr_t>(g.bias) & 7u) == 0) &&
+           (g.residual == nullptr || ((reinterpret_cast<std::uintptr_t>(g.residual) & 7u) == 0 && g.ldr % 4 == 0)) &&
+           (g.addend_f32 == nullptr || (is_aligned16(g.addend_f32) && g.ld_addend % 4 == 0));
+}
+
+// An operand whose rows the streamed kernels cannot read (odd widths, unaligned storage) is copied to padded rows
+// first: one pass over the operand (a few microseconds) against a contraction that ran at the fp32 matrix rate, a
+// sixteenth of the 16-bit one. Copies and split-K partial tiles share one request to the arena.
+template <typename T>
+int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream);
+
 template <typename T>
 int run_typed(const GemmArgs& g, hipStream_t stream) {
     KernelArgs p{};
@@ -1430,6 +1587,10 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
     p.m = static_cast<int>(g.m);
     p.n = static_cast<int>(g.n);
     p.k = static_cast<int>(g.k);
+    p.a_extent = static_cast<int>(std::max(g.a_extent, g.m));
+    p.b_extent = static_cast<int>(g.b_extent != 0 ? g.b_extent : g.n);
+    p.b_k = static_cast<int>(g.b_k != 0 ? g.b_k : g.k);
+    p.k_tiles = static_cast<int>((g.k + kBK - 1) / kBK);
     p.lda = static_cast<long>(g.lda);
     p.ldb = static_cast<long>(g.ldb);
     p.ldc = static_cast<long>(g.ldc);
@@ -1467,7 +1628,6 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
 
     bool fast = false;
     if constexpr (!std::is_same_v<T, float>) {
-        const std::size_t c_elem = g.c_is_f32 ? 4 : sizeof(T);
         GemmArgs whole = g;  // alignment of segmented operands was checked per segment
         if (g.a_segments.count > 0) {
             whole.a = g.a_segments.ptr[0];
@@ -1477,13 +1637,13 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
             whole.c = const_cast<void*>(g.c_segments.ptr[0]);
             whole.ldc = g.c_segments.ld[0];
         }
-        const GemmArgs& g = whole;
-        fast = g.k % kBK == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.n % 8 == 0 && g.m % 8 == 0 &&
-               is_aligned16(g.a) && is_aligned16(g.b) && (g.ldc * c_elem) % 16 == 0 && is_aligned16(g.c) &&
-               (g.bias == nullptr || (reinterpret_cast<std::uintptr_t>(g.bias) & 7u) == 0) &&
-               (g.residual == nullptr || ((reinterpret_cast<std::uintptr_t>(g.residual) & 7u) == 0 && g.ldr % 4 == 0)) &&
-               (g.addend_f32 == nullptr || (is_aligned16(g.addend_f32) && g.ld_addend % 4 == 0)) &&
-               !(!g.a_k_contiguous && g.b_k_contiguous) && offsets_fit_32bit(g, sizeof(T));
+        if ((g.a_k_contiguous || !g.b_k_contiguous) && offsets_fit_32bit(whole, sizeof(T))) {
+            const bool a_ok = a_streams(whole), b_ok = b_streams(whole);
+            fast = a_ok && b_ok;
+            p.ragged = c_streams(whole, sizeof(T)) ? 0 : 1;
+            if (!fast && !segmented && g.batch_rows == 0 && !g.no_split) return run_padded<T>(g, !a_ok, !b_ok, stream);
+        }
+        if (p.ragged && segmented) return fail(CGPTX_INVALID_ARGUMENT, "gemm: segmented operands need the aligned MFMA path");
     }
     if (!fast && segmented) return fail(CGPTX_INVALID_ARGUMENT, "gemm: segmented operands need the aligned MFMA path");
     if (!fast && g.batch_rows != 0) return fail(CGPTX_INVALID_ARGUMENT, "gemm: a stack of products needs the aligned MFMA path");
@@ -1497,23 +1657,49 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
         return CGPTX_OK;
     }
     if constexpr (!std::is_same_v<T, float>) {
-        // 256x256 tiles (one block per CU, 64 MFMAs per wavefront and K step) when they still give
-        // every CU a tile, or when K is long enough to be split across the idle CUs without the
-        // fp32 partial tiles outweighing the contraction (at least 8 tiles, so at most 32 slices);
-        // otherwise 128x128 tiles, with K split when even those are too few.
-        const long big_tiles = static_cast<long>((g.m + 255) / 256) * static_cast<long>((g.n + 255) / 256);
-        const int forced = forced_tile();
-        const long units = compute_units();
-        const bool fills = big_tiles * 5 >= units * 4;
-        const bool splits = (!g.no_split || g.split_workspace != nullptr) && g.residual == nullptr && g.addend_f32 == nullptr &&
-                            g.c_segments.count == 0 && big_tiles >= 8 &&
-                            g.k / kBK >= static_cast<std::size_t>(32 * ((units + big_tiles - 1) / big_tiles));
-        const bool big = g.swiglu_out != nullptr || g.swiglu_saved != nullptr || g.batch_rows != 0 || forced == 256 ||
-                         (forced == 0 && (fills || splits));
-        if (big) return run_config<T, 256, 256>(g, p, stream);
-        return run_config<T, 128, 128>(g, p, stream);
+        const Plan plan = make_plan(g);
+        if (plan.tile == 256) return run_config<T, 256, 256>(g, plan, p, stream);
+        if (plan.tile == 128) return run_config<T, 128, 128>(g, plan, p, stream);
+        return run_config<T, 64, 64>(g, plan, p, stream);
     }
     return CGPTX_OK;
+}
+
+template <typename T>
+int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream) {
+    GemmArgs padded = g;
+    const std::size_t k_whole = round_up(g.k, kBK);
+    std::size_t a_bytes = 0, b_bytes = 0;
+    if (pad_a) {
+        padded.lda = g.a_k_contiguous ? k_whole : round_up(g.m, 8);
+        padded.a_extent = g.a_k_contiguous ? g.m : padded.lda;
+        a_bytes = round_up((g.a_k_contiguous ? g.m : g.k) * padded.lda * sizeof(T), 256);
+    }
+    if (pad_b) {
+        padded.ldb = g.b_k_contiguous ? k_whole : round_up(g.n, 8);
+        padded.b_extent = g.b_k_contiguous ? g.n : padded.ldb;
+        b_bytes = round_up((g.b_k_contiguous ? g.n : g.k) * padded.ldb * sizeof(T), 256);
+    }
+    if (g.a_k_contiguous) padded.k = k_whole;  // A's rows then end in zeros, B's K range ends where it did
+    if (!g.b_k_contiguous) padded.b_k = g.b_k != 0 ? g.b_k : g.k;
+    const std::size_t split_bytes = make_plan(padded).partial_bytes(padded);
+    void* mem = nullptr;
+    if (int s = scratch(stream, a_bytes + b_bytes + split_bytes, &mem)) return s;
+    auto* base = static_cast<char*>(mem);
+    if (pad_a) {
+        padded.a = base;
+        const std::size_t rows = g.a_k_contiguous ? g.m : g.k, cols = g.a_k_contiguous ? g.k : g.m;
+        if (int s = pad_rows(base, g.a, rows, cols, g.lda, padded.lda, stream)) return s;
+    }
+    if (pad_b) {
+        padded.b = base + a_bytes;
+        const std::size_t rows = g.b_k_contiguous ? g.n : g.k, cols = g.b_k_contiguous ? g.k : g.n;
+        if (int s = pad_rows(base + a_bytes, g.b, rows, cols, g.ldb, padded.ldb, stream)) return s;
+    }
+    padded.no_split = true;
+    padded.split_workspace = split_bytes != 0 ? base + a_bytes + b_bytes : nullptr;
+    padded.split_workspace_bytes = split_bytes;
+    return run_typed<T>(padded, stream);
 }
 
 }  // namespace
@@ -1526,12 +1712,12 @@ bool gemm_fuses_swiglu(const GemmArgs& g) {
     const std::size_t elem = 2, inter = g.n / 2;
     // Whole 128-column units of gate and of up per tile, tiles that fill the chip (the 256x256
     // configuration), 16-byte aligned rows everywhere, and the whole weight within 32-bit offsets.
-    if (g.n % 256 != 0 || g.m % 8 != 0 || g.k % kBK != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
+    if (g.n % 256 != 0 || g.k % kBK != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
         g.ld_swiglu % 8 != 0 || g.ld_swiglu < inter || !is_aligned16(g.a) || !is_aligned16(g.b) || !is_aligned16(g.c) ||
         !is_aligned16(g.swiglu_out))
         return false;
     const long tiles = static_cast<long>((g.m + 255) / 256) * static_cast<long>(g.n / 256);
-    if (forced_tile() == 128 || tiles * 5 < static_cast<long>(compute_units()) * 4) return false;
+    if ((forced_tile() != 0 && forced_tile() != 256) || tiles * 5 < static_cast<long>(compute_units()) * 4) return false;
     constexpr std::size_t limit = (std::size_t{1} << 31) - (std::size_t{1} << 20);
     return offsets_fit_32bit(g, elem) && (g.n * g.ldb + g.k) * elem < limit && 256 * g.ld_swiglu * elem < limit;
 }
@@ -1544,12 +1730,12 @@ bool gemm_fuses_swiglu_gradient(const GemmArgs& g) {
     const std::size_t elem = 2;
     // 16-byte chunks of whole rows everywhere, tiles that fill the chip (the 256x256 configuration),
     // and a wavefront's 128 rows of the saved and of the written [gate | up] within 32-bit offsets.
-    if (g.n % 8 != 0 || g.m % 8 != 0 || g.k % kBK != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
+    if (g.n % 8 != 0 || g.k % kBK != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
         g.ld_swiglu % 8 != 0 || g.ldc < 2 * g.n || g.ld_swiglu < 2 * g.n || !is_aligned16(g.a) || !is_aligned16(g.b) ||
         !is_aligned16(g.c) || !is_aligned16(g.swiglu_saved))
         return false;
     const long tiles = static_cast<long>((g.m + 255) / 256) * static_cast<long>((g.n + 255) / 256);
-    if (forced_tile() == 128 || tiles * 5 < static_cast<long>(compute_units()) * 4) return false;
+    if ((forced_tile() != 0 && forced_tile() != 256) || tiles * 5 < static_cast<long>(compute_units()) * 4) return false;
     constexpr std::size_t limit = (std::size_t{1} << 31) - (std::size_t{1} << 20);
     return offsets_fit_32bit(g, elem) && 256 * g.ld_swiglu * elem < limit;
 }
@@ -1560,7 +1746,7 @@ bool gemm_takes_batch(const GemmArgs& g) {
         g.addend_f32 != nullptr || g.accumulate || g.c_is_f32 || g.c_segments.count > 0 || g.swiglu_out != nullptr ||
         g.swiglu_saved != nullptr || g.no_split || g.c == nullptr || g.b == nullptr)
         return false;
-    if (g.batch_rows % 256 != 0 || g.m % g.batch_rows != 0 || g.n % 8 != 0 || g.k % kBK != 0 || g.ldb % 8 != 0 ||
+    if (g.batch_rows % 256 != 0 || g.m % g.batch_rows != 0 || g.n % 8 != 0 || g.ldb % 8 != 0 ||
         g.ldc % 8 != 0 || g.b_batch_stride % 8 != 0)
         return false;
     if (g.a_segments.count == 0) return g.a != nullptr && g.lda % 8 == 0 && g.a_batch_stride % 8 == 0;
@@ -1568,6 +1754,18 @@ bool gemm_takes_batch(const GemmArgs& g) {
         if (g.a_segment_batch_stride[s] % 8 != 0) return false;
     return true;
 }
+
+int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, hipStream_t stream) {
+    const std::size_t chunks = rows * (pitch / 8);
+    const std::size_t blocks = std::min<std::size_t>((chunks + kThreads - 1) / kThreads, static_cast<std::size_t>(compute_units()) * 16);
+    hipLaunchKernelGGL(pad_rows_kernel, dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), 0, stream,
+                       static_cast<std::uint16_t*>(dst), static_cast<const std::uint16_t*>(src), static_cast<long>(rows),
+                       static_cast<int>(cols), static_cast<long>(ld), static_cast<int>(pitch));
+    CGPTX_LAUNCH_CHECK();
+    return CGPTX_OK;
+}
+
+std::size_t gemm_split_bytes(const GemmArgs& g) { return g.dtype == CGPTX_F32 ? 0 : make_plan(g).partial_bytes(g); }
 
 int gemm(const GemmArgs& g, hipStream_t stream) {
     if ((g.a == nullptr && g.a_segments.count == 0) || g.b == nullptr || (g.c == nullptr && g.c_segments.count == 0) ||

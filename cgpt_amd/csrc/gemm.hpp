@@ -31,6 +31,11 @@ struct GemmArgs {
     std::size_t ld_addend = 0;
     std::size_t m = 0, n = 0, k = 0;
     std::size_t lda = 0, ldb = 0, ldc = 0, ldr = 0;
+    // What the operands hold where that is not m, n and k (0: it is). For matrices in padded rows: a_extent >= m columns
+    // of an A that is not k-contiguous; b_extent rows of a k-contiguous B (past them C gets zeros) or columns >= n of
+    // another one; b_k <= k rows of a B that is not k-contiguous (past them it counts as zeros, whatever finite values A
+    // holds there).
+    std::size_t a_extent = 0, b_extent = 0, b_k = 0;
     bool a_k_contiguous = true;
     bool b_k_contiguous = true;
     bool accumulate = false;
@@ -71,6 +76,10 @@ struct GemmArgs {
 };
 
 int gemm(const GemmArgs& args, hipStream_t stream);
+// Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
+std::size_t gemm_split_bytes(const GemmArgs& args);
+// Copies [rows, cols] 16-bit elements (row stride ld) to rows of `pitch` elements (a multiple of 8), zeros past cols.
+int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, hipStream_t stream);
 // Whether gemm() serves args.swiglu_out for this call (shape, layout and alignment of the fused kernel).
 bool gemm_fuses_swiglu(const GemmArgs& args);
 bool gemm_fuses_swiglu_gradient(const GemmArgs& args);

@@ -6,6 +6,7 @@
 #include "gemm.hpp"
 #include "reduce.hpp"
 
+#include <algorithm>
 #include <limits>
 
 namespace cgptx {
@@ -137,8 +138,7 @@ extern "C" int cgptx_linear_backward_weights_stacked(void* grad_weight, const vo
     g.batch_rows = out_features;
     g.a_batch_stride = grad_output_stride;
     g.b_batch_stride = input_stride;
-    if (count > 1 && gemm_takes_batch(g) && is_aligned16(grad_output) && is_aligned16(input) && is_aligned16(grad_weight) &&
-        rows % 32 == 0)
+    if (count > 1 && gemm_takes_batch(g) && is_aligned16(grad_output) && is_aligned16(input) && is_aligned16(grad_weight))
         return gemm(g, stream);
     // Shapes the stacked launch does not take: one weight gradient after the other.
     const std::size_t elem = dtype_size(dtype);
@@ -162,39 +162,70 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
         (grad_weight != nullptr && input == nullptr))
         return fail(CGPTX_INVALID_ARGUMENT, "linear_backward: null tensor");
     auto stream = static_cast<hipStream_t>(stream_);
-    if (grad_input != nullptr) {  // dX[rows, in] = dY[rows, out] · W[out, in]
+    // An output gradient whose rows are not whole 16-byte chunks feeds both contractions from one padded copy (each would
+    // make its own otherwise).
+    const void* dy = grad_output;
+    std::size_t dy_pitch = out_features;
+    void* split_room = nullptr;
+    std::size_t split_bytes = 0;
+    auto input_gradient = [&]() {  // dX[rows, in] = dY[rows, out] · W[out, in]
         GemmArgs g;
-        g.a = grad_output;
+        g.a = dy;
         g.b = weight;
         g.c = grad_input;
         g.m = rows;
         g.n = in_features;
-        g.k = out_features;
-        g.lda = out_features;
+        g.k = dy_pitch;
+        g.b_k = out_features;
+        g.lda = dy_pitch;
         g.ldb = in_features;
         g.ldc = in_features;
         g.b_k_contiguous = false;
         g.accumulate = accumulate_input != 0;
         g.dtype = dtype;
-        if (int s = gemm(g, stream)) return s;
-    }
-    if (grad_weight != nullptr) {  // dW[out, in] = dYᵀ[out, rows] · X[rows, in]
+        g.no_split = split_room != nullptr;
+        g.split_workspace = split_room;
+        g.split_workspace_bytes = split_bytes;
+        return g;
+    };
+    auto weight_gradient = [&]() {  // dW[out, in] = dYᵀ[out, rows] · X[rows, in]
         GemmArgs g;
-        g.a = grad_output;
+        g.a = dy;
         g.b = input;
         g.c = grad_weight;
         g.m = out_features;
+        g.a_extent = dy_pitch;
         g.n = in_features;
         g.k = rows;
-        g.lda = out_features;
+        g.lda = dy_pitch;
         g.ldb = in_features;
         g.ldc = in_features;
         g.a_k_contiguous = false;
         g.b_k_contiguous = false;
         g.accumulate = accumulate_weight != 0;
         g.dtype = dtype;
-        if (int s = gemm(g, stream)) return s;
+        g.no_split = split_room != nullptr;
+        g.split_workspace = split_room;
+        g.split_workspace_bytes = split_bytes;
+        return g;
+    };
+    constexpr std::size_t kSpan = (std::size_t{1} << 31) - (std::size_t{1} << 21);  // the streamed kernels' 32-bit offsets
+    if (grad_input != nullptr && grad_weight != nullptr && dtype != CGPTX_F32 &&
+        (out_features % 8 != 0 || !is_aligned16(grad_output)) && in_features % 8 == 0 && is_aligned16(weight) &&
+        is_aligned16(input) && rows * (out_features + 32 + in_features) * 2 < kSpan && out_features * in_features * 2 < kSpan) {
+        dy_pitch = (out_features + 31) / 32 * 32;
+        const std::size_t copy_bytes = (rows * dy_pitch * 2 + 255) & ~std::size_t{255};
+        split_bytes = std::max(gemm_split_bytes(input_gradient()), gemm_split_bytes(weight_gradient())) + 256;
+        void* mem = nullptr;
+        if (int s = scratch(stream, copy_bytes + split_bytes, &mem)) return s;
+        if (int s = pad_rows(mem, grad_output, rows, out_features, out_features, dy_pitch, stream)) return s;
+        dy = mem;
+        split_room = static_cast<char*>(mem) + copy_bytes;
     }
+    if (grad_input != nullptr)
+        if (int s = gemm(input_gradient(), stream)) return s;
+    if (grad_weight != nullptr)
+        if (int s = gemm(weight_gradient(), stream)) return s;
     if (grad_bias != nullptr) {  // db[out] = Σ_rows dY
         const int cols = static_cast<int>(out_features);
         const int slices = rows < 256 ? 1 : (rows < 65536 ? 64 : 256);

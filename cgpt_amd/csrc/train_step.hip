@@ -369,12 +369,12 @@ int qkv_backward_weight(void* qkv_gradient, const void* dq, const void* dk, cons
 // partial tiles that a second launch adds up; the layers' tiles together fill the chip several times over and
 // (almost) nothing is split. Needs 16-bit storage, tile-aligned weight shapes and at least two layers; costs the
 // memory of every layer's output gradients.
-bool stackable_weight_gradients(const cgptx_model_config& c, std::size_t rows) {
+bool stackable_weight_gradients(const cgptx_model_config& c) {
     const char* text = std::getenv("CGPTX_STACK_DW");  // read when the model is created
     if (text != nullptr && text[0] == '0') return false;
     const std::size_t H = c.hidden_size, I = c.intermediate_size;
     const std::size_t QW = c.num_query_heads * c.head_dim, KW = c.num_kv_heads * c.head_dim;
-    return c.dtype != CGPTX_F32 && c.num_layers >= 2 && rows % 32 == 0 && H % 256 == 0 && QW % 256 == 0 && KW % 256 == 0 &&
+    return c.dtype != CGPTX_F32 && c.num_layers >= 2 && H % 256 == 0 && QW % 256 == 0 && KW % 256 == 0 &&
            (2 * I) % 256 == 0 && I % 8 == 0;
 }
 
@@ -669,7 +669,7 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
     const float eps = c.rms_epsilon;
     auto* s = static_cast<cgptx_stream>(stream);
     // One launch for the q/k/v projections needs 16-bit storage and segment widths the tiles respect.
-    const bool fused_qkv = dt != CGPTX_F32 && QW % 256 == 0 && KW % 256 == 0 && H % 32 == 0 && N % 32 == 0;
+    const bool fused_qkv = dt != CGPTX_F32 && QW % 256 == 0 && KW % 256 == 0 && H % 32 == 0;
 
     // ------------------------------------------------------------------ forward
     CGPTX_OP("embedding_fwd", cgptx_embedding_forward(m->hidden[0], m->tokens, N, m->embedding.value, c.vocabulary_size, H, dt, s));
@@ -894,7 +894,7 @@ extern "C" int cgptx_model_create(cgptx_model** out, const cgptx_model_config* c
         CGPTX_TRY(make_parameter(m, m->final_norm, "model.norm.weight", H, 1, 0.0f, seed, 1));
         m->layers.resize(c.num_layers);
         m->acts.resize(c.num_layers);
-        m->stacked_dw = stackable_weight_gradients(c, N);
+        m->stacked_dw = stackable_weight_gradients(c);
         if (m->stacked_dw) {
             const std::size_t L = c.num_layers;
             auto stack = [&](cgptx_model::Stack& st, std::size_t bytes, std::size_t count) -> int {

@@ -337,3 +337,31 @@ def test_linear_swiglu_forward_argument_errors(device):
     from cgpt_amd import capi
     with pytest.raises(ValueError):  # the C entry point rejects null tensors itself
         capi.call("cgptx_linear_swiglu_forward", None, act.data_ptr(), x.data_ptr(), w.data_ptr(), 8, 32, 32, 1, None)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("rows,fin,fout", [
+    (1, 64, 64), (63, 64, 96), (65, 96, 64), (129, 160, 136),      # 64-wide tiles with a ragged last row; short K tiles in dW
+    (3001, 512, 1024), (2049, 1024, 2048),                         # 128-wide tiles
+    (8197, 1024, 2048),                                            # 256-wide tiles
+    (77, 100, 31), (130, 33, 129), (258, 130, 66), (4099, 257, 515),  # widths that are not whole chunks: padded copies, C by elements
+    (40, 72, 24), (40, 24, 72),                                    # whole chunks, but K ends inside a K tile
+])
+@pytest.mark.parametrize("accumulate", [False, True], ids=["overwrite", "accumulate"])
+def test_linear_ragged_shapes_integer_valued_inputs_are_exact(device, rows, fin, fout, accumulate, dtype):
+    """Small integers: every product and partial sum is exact in fp32, so the result is the rounded exact value whatever
+    the order of additions."""
+    g = torch.Generator().manual_seed(rows + fin + fout)
+    integers = lambda *shape: torch.randint(-2, 3, shape, generator=g).double()
+    x, w, dy, b = integers(rows, fin), integers(fout, fin), integers(rows, fout), integers(fout)
+    base = [integers(rows, fin), integers(fout, fin), integers(fout)] if accumulate else [0, 0, 0]
+    want = [x @ w.T + b, dy @ w + base[0], dy.T @ x + base[1], dy.sum(0) + base[2]]
+    on = lambda t: t.to(dtype).to(device)
+    y = torch.full((rows, fout), float("nan"), dtype=dtype, device=device)
+    gi, gw, gb = (on(v) if accumulate else torch.full(shape, float("nan"), dtype=dtype, device=device)
+                  for v, shape in zip(base, ((rows, fin), (fout, fin), (fout,))))
+    ops.linear_forward(y, on(x), on(w), bias=on(b))
+    options = ops.LinearBackwardOptions(accumulate_input=accumulate, accumulate_weight=accumulate, accumulate_bias=accumulate)
+    ops.linear_backward(gi, gw, gb, on(dy), on(x), on(w), options=options)
+    for name, got, exact in zip(("Y", "dX", "dW", "db"), (y, gi, gw, gb), want):
+        assert torch.equal(got.cpu(), exact.to(dtype)), name
