@@ -57,7 +57,11 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         const unsigned long long asked = std::strtoull(text, nullptr, 0);
         if (asked > 0) logits_bytes = std::min<std::size_t>(static_cast<std::size_t>(asked), kMaxLogitsBytes);
     }
-    std::size_t limit = logits_bytes / (vocab * elem);
+    // Rows of logits are padded to whole K tiles of the input gradient's contraction (32 elements): an odd vocabulary
+    // then streams like any other. The padding holds zeros: columns of Z the classifier has no rows for, and cleared
+    // by the softmax pass.
+    const std::size_t pitch = dtype == CGPTX_F32 ? vocab : (vocab + 31) / 32 * 32;
+    std::size_t limit = logits_bytes / (pitch * elem);
     limit = std::max<std::size_t>(256, limit / 256 * 256);
     const std::size_t pieces = (rows + limit - 1) / limit;
     std::size_t chunk = ((rows + pieces - 1) / pieces + 255) / 256 * 256;
@@ -65,7 +69,7 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
     const bool single = chunk >= rows;
     const std::size_t loss_bytes = (rows * sizeof(float) + 255) & ~std::size_t{255};
     const std::size_t acc_bytes = single ? 0 : (vocab * hidden * sizeof(float) + 255) & ~std::size_t{255};
-    const std::size_t logit_bytes = (chunk * vocab * elem + 255) & ~std::size_t{255};
+    const std::size_t logit_bytes = (chunk * pitch * elem + 255) & ~std::size_t{255};
     // A chunk's input gradient has few output tiles ([chunk, hidden]) and a long K (the vocabulary): with several
     // chunks it is split along K into up to `units / tiles` slices, whose fp32 partial tiles need room of their own.
     const std::size_t dx_tiles = ((chunk + 255) / 256) * ((hidden + 255) / 256);
@@ -89,15 +93,16 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         z.b = classifier;
         z.c = logits;
         z.m = r;
-        z.n = vocab;
+        z.n = pitch;
+        z.b_extent = vocab;
         z.k = hidden;
         z.lda = hidden;
         z.ldb = hidden;
-        z.ldc = vocab;
+        z.ldc = pitch;
         z.dtype = dtype;
         z.no_split = true;
         if (int s = gemm(z, stream)) return s;
-        if (int s = cross_entropy_rows(row_loss + r0, logits, logits, targets + r0, r, vocab, factor, dtype, stream))
+        if (int s = cross_entropy_rows(row_loss + r0, logits, pitch, logits, pitch, targets + r0, r, vocab, factor, dtype, stream))
             return s;
         GemmArgs dx;  // dX[r, H] = dZ[r, V]·C[V, H]
         dx.a = logits;
@@ -105,8 +110,9 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         dx.c = static_cast<char*>(input_gradient) + r0 * hidden * elem;
         dx.m = r;
         dx.n = hidden;
-        dx.k = vocab;
-        dx.lda = vocab;
+        dx.k = pitch;
+        dx.b_k = vocab;
+        dx.lda = pitch;
         dx.ldb = hidden;
         dx.ldc = hidden;
         dx.b_k_contiguous = false;
@@ -124,9 +130,10 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         dc.b = x;
         dc.c = last ? classifier_gradient : static_cast<void*>(acc);
         dc.m = vocab;
+        dc.a_extent = pitch;
         dc.n = hidden;
         dc.k = r;
-        dc.lda = vocab;
+        dc.lda = pitch;
         dc.ldb = hidden;
         dc.ldc = hidden;
         dc.a_k_contiguous = false;
