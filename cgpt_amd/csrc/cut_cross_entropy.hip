@@ -60,7 +60,7 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
     // Rows of logits are padded to whole K tiles of the input gradient's contraction (32 elements): an odd vocabulary
     // then streams like any other. The padding holds zeros: columns of Z the classifier has no rows for, and cleared
     // by the softmax pass.
-    const std::size_t pitch = dtype == CGPTX_F32 ? vocab : (vocab + 31) / 32 * 32;
+    const std::size_t pitch = (vocab + 31) / 32 * 32;
     std::size_t limit = logits_bytes / (pitch * elem);
     limit = std::max<std::size_t>(256, limit / 256 * 256);
     const std::size_t pieces = (rows + limit - 1) / limit;

@@ -1,5 +1,5 @@
-// Dense contraction kernels for gfx950 (CDNA4): C[M,N] (+)= op(A)·op(B), 16-bit
-// inputs, fp32 accumulation on the matrix cores.
+// Dense contraction kernels for gfx950 (CDNA4): C[M,N] (+)= op(A)·op(B), 16-bit or
+// fp32 inputs, fp32 accumulation on the matrix cores.
 //
 // One kernel family serves the three contractions of a linear layer
 // (reference: src/ops/linear.cu:634-667, src/ops/backward/linear_backward.cu:268-285,
@@ -40,9 +40,10 @@
 //     (deterministic), applying accumulate and the dtype conversion.
 //
 // Operands whose rows are not whole aligned 16-byte chunks are copied to padded rows first;
-// C may have any width and alignment (a store per element). fp32 storage, and 16-bit operands
-// beyond 32-bit offsets, run on an fp32 matrix-core kernel (v_mfma_f32_32x32x2_f32,
-// register-staged operand tiles) with the same semantics.
+// C may have any width and alignment (a store per element). fp32 storage takes the same kernels
+// with v_mfma_f32_16x16x4_f32 and K steps of 16. Operands beyond 32-bit offsets, and unaligned ones
+// of a caller that owns the arena, run on a general fp32 matrix-core kernel
+// (v_mfma_f32_32x32x2_f32, register-staged operand tiles) with the same semantics.
 #include "gemm.hpp"
 
 #include <algorithm>
@@ -56,7 +57,9 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
-constexpr int kBK = 32;          // K step per LDS stage
+// K step per LDS stage: 64 bytes of a k-contiguous operand's row.
+template <typename T>
+constexpr int kBK = 64 / static_cast<int>(sizeof(T));
 // LDS stages of a block: one being multiplied, one being refilled, the rest in flight. 256x256
 // blocks own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each), and so do 64x64
 // blocks: their K tiles are short (4 MFMAs per wavefront), so ten 8 KiB stages keep as many bytes in flight.
@@ -66,15 +69,31 @@ constexpr int kXcds = 8;
 
 using acc_t = vec_t<float, 4>;
 
-// c += a x b with v_mfma_f32_16x16x32 (a: 16 rows x 32 k, b: 32 k x 16 columns; lane l holds row or
+// fp32 storage: four v_mfma_f32_16x16x4_f32 take the K tile of 16 (lane l holds row or column l%16 at k = 4*(l/16) + e
+// for step e; the accumulator's layout is that of the 16-bit form). 64 accumulator registers at most, left to the
+// compiler.
+template <typename T>
+struct Mfma;
+template <>
+struct Mfma<float> {
+    using frag = vec_t<float, 4>;
+    __device__ static __forceinline__ void run(acc_t& c, const frag& a, const frag& b) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+    }
+    __device__ static __forceinline__ void start(acc_t& c, const frag& a, const frag& b) {
+        c = acc_t(0.0f);
+        run(c, a, b);
+    }
+};
+
+// 16-bit storage: c += a x b with v_mfma_f32_16x16x32 (a: 16 rows x 32 k, b: 32 k x 16 columns; lane l holds row or
 // column l%16, k = 8*(l/16) .. +7; c: lane l holds rows 4*(l/16) .. +3 of column l%16). Written as
 // assembly so that the accumulator is updated in place: the four-register form of the instruction
 // does not tie its result to its addend, and with all 256 accumulator registers in use the register
 // allocator would otherwise shuffle accumulators around every MFMA. The kernel keeps the distances
 // the hardware asks for by construction: an accumulator is touched once per K tile (64 or 16 MFMAs
 // apart), zeroed long before its first MFMA and read by the epilogue only after a barrier.
-template <typename T>
-struct Mfma;
 template <>
 struct Mfma<bf16_t> {
     using frag = vec_t<bf16_t, 8>;
@@ -246,16 +265,16 @@ __device__ __forceinline__ unsigned int lds_address_of(const T* p) {
 template <typename T, int ROWS>
 struct KTile {
     using frag_t = typename Mfma<T>::frag;
-    static constexpr int kChunksPerRow = kBK / 8;
+    static constexpr int kChunksPerRow = kBK<T> / kVec128<T>;
     static constexpr int kRowsPerLoad = 64 / kChunksPerRow;
-    static constexpr int kElems = ROWS * kBK;
+    static constexpr int kElems = ROWS * kBK<T>;
     static constexpr int kLoads = ROWS / kRowsPerLoad / kWaves;  // load instructions per wavefront and tile
 
     u32x4 rsrc = {0u, 0u, 0u, 0u};
     int voffset = 0;
     unsigned int group_bytes = 0;  // kRowsPerLoad rows further in global memory
 
-    __device__ __forceinline__ static int swizzle(int row) { return (row / (128 / kBK)) % kChunksPerRow; }
+    __device__ __forceinline__ static int swizzle(int row) { return (row / 4) % kChunksPerRow; }
 
     // base: element (row0, 0) of the operand; rows past rows_left only feed C rows that are never
     // stored (they read zeros or whatever follows, never out of the allocation's last row).
@@ -273,12 +292,12 @@ struct KTile {
         return wave * group_bytes + k0 * static_cast<unsigned int>(sizeof(T));
     }
     // Element offset of the lane's fragment within a 16-row block (the whole K tile is one MFMA
-    // step): row lane%16, k = 8 (lane/16) .. +7. The swizzle of a row does not depend on the block.
+    // step): row lane%16, the lane/16-th 16 bytes of it. The swizzle of a row does not depend on the block.
     __device__ __forceinline__ static int lane_offset(int lane) {
-        return (lane & 15) * kBK + (((lane >> 4) ^ swizzle(lane & 15)) * 8);
+        return (lane & 15) * kBK<T> + (((lane >> 4) ^ swizzle(lane & 15)) * kVec128<T>);
     }
     __device__ __forceinline__ static frag_t frag(const T* tile, int block0, int offset) {
-        return *reinterpret_cast<const frag_t*>(tile + block0 * kBK + offset);
+        return *reinterpret_cast<const frag_t*>(tile + block0 * kBK<T> + offset);
     }
 };
 
@@ -291,12 +310,17 @@ struct KTile {
 template <typename T, int COLS>
 struct NTile {
     using frag_t = typename Mfma<T>::frag;
-    static constexpr int kChunksPerRow = COLS / 8;
+    static constexpr int kChunksPerRow = COLS / kVec128<T>;
     static constexpr int kRowsPerLoad = 64 / kChunksPerRow;  // k rows one load instruction covers (2, 4 or 8)
-    static constexpr int kElems = kBK * COLS;
-    static constexpr int kLoads = kBK / kRowsPerLoad / kWaves;
+    static constexpr int kElems = kBK<T> * COLS;
+    static constexpr int kLoads = kBK<T> / kRowsPerLoad / kWaves;
 
-    __device__ __forceinline__ static int swizzle(int k_row) { return COLS >= 128 ? (k_row & 3) << 2 : (k_row & 2) << 1; }
+    // fp32: the four k rows a read touches lie four apart (k = 4*(lane/16) + e); of their two low group bits those are
+    // used that a wavefront's loads have in common.
+    __device__ __forceinline__ static int swizzle(int k_row) {
+        if constexpr (std::is_same_v<T, float>) return COLS >= 128 ? k_row & 4 : k_row & 12;
+        else return COLS >= 128 ? (k_row & 3) << 2 : (k_row & 2) << 1;
+    }
 
     u32x4 rsrc = {0u, 0u, 0u, 0u};
     int voffset = 0;
@@ -308,8 +332,8 @@ struct NTile {
         const int lane = threadIdx.x & (kWave - 1);
         rsrc = make_rsrc(base, (static_cast<long>(k_total - 1) * ld + cols_left) * static_cast<long>(sizeof(T)));
         const int row = lane / kChunksPerRow;                  // within the instruction's rows
-        const int k_row = (wave * kRowsPerLoad + row) & 3;     // low bits of the tile row (groups step by 4*kRowsPerLoad)
-        const int chunk = min((lane % kChunksPerRow) ^ swizzle(k_row), cols_left / 8 - 1);
+        const int k_row = wave * kRowsPerLoad + row;           // tile row of the first load; its swizzle is that of all
+        const int chunk = min((lane % kChunksPerRow) ^ swizzle(k_row), cols_left / kVec128<T> - 1);
         voffset = static_cast<int>(row * ld * sizeof(T)) + chunk * 16;
         group_bytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(kRowsPerLoad * ld * sizeof(T)));
     }
@@ -322,11 +346,19 @@ struct NTile {
     // columns in two reads (k rows +0..3, +4..7). The offset is for the first read; block0 is a
     // multiple of 16.
     __device__ __forceinline__ static int lane_offset(int lane, int block0) {
+        if constexpr (std::is_same_v<T, float>) {  // k rows 4*(lane/16) + e, column block0 + lane%16
+            const int row = (lane >> 4) * 4, column_chunk = (block0 + (lane & 15)) / 4;
+            return row * COLS + (column_chunk ^ swizzle(row)) * 4 + (lane & 3);
+        }
         const int k_row = (lane >> 4) * 8 + ((lane & 15) >> 2);
         const int chunk = ((block0 / 8) ^ swizzle(k_row)) + ((lane & 3) >> 1);
         return k_row * COLS + chunk * 8 + (lane & 1) * 4;
     }
     __device__ __forceinline__ static frag_t frag(const T* tile, int offset) {
+        if constexpr (std::is_same_v<T, float>) {
+            const T* q = tile + offset;
+            return frag_t{q[0], q[COLS], q[2 * COLS], q[3 * COLS]};
+        } else {
         using s16x4 = vec_t<short, 4>;
         using lds_ptr = __attribute__((address_space(3))) s16x4*;
         const T* q = tile + offset;
@@ -339,6 +371,7 @@ struct NTile {
             both[4 + e] = hi[e];
         }
         return __builtin_bit_cast(frag_t, both);
+        }
     }
 };
 
@@ -503,7 +536,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     // issued one by one between MFMAs.
     auto cursors = [&](int t, TileCursor& ca, TileCursor& cb) __attribute__((always_inline)) {
         const unsigned int past_end = src_begin + t >= src_end ? 0x80000000u : 0u;
-        const int k0 = min(src_begin + t, src_end - 1) * kBK;
+        const int k0 = min(src_begin + t, src_end - 1) * kBK<T>;
         if constexpr (SEGMENTED) {
             // Values first, then selects: a conditional between the objects' members would select
             // an address and keep all three sources in memory.
@@ -613,7 +646,9 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     // staged in the storage dtype. A staged row is kRowBytes long; its 16-byte chunk c sits at
     // chunk position c ^ sw(row), which spreads both the column-wise writes and the row-wise reads
     // over all banks.
-    constexpr int kRowBytes = WN * static_cast<int>(sizeof(T));
+    constexpr bool kIsF32 = std::is_same_v<T, float>;
+    static_assert(!kIsF32 || (BM <= 128 && !SEGMENTED && !RESIDUAL && !SWIGLU && !GRAD), "fp32 storage has the plain kernels only");
+    constexpr int kRowBytes = WN * 2;  // fp32 values always pass in two halves
     constexpr int kRowChunks = kRowBytes / 16;
     static_assert(32 * kRowBytes * kWaves == static_cast<int>(kStageBytes), "staging is a quarter stage per wavefront");
     unsigned char* region = smem_raw + (kStages - 1) * kStageBytes + wave * (kStageBytes / kWaves);
@@ -635,8 +670,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
                 acc_t v;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    float x;
-                    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(acc[2 * r + ii][j0 + jj][e]));
+                    float x = acc[2 * r + ii][j0 + jj][e];
+                    if constexpr (!kIsF32) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(x));
                     v[e] = x;
                 }
                 const int byte = (jj * 16 + q_lane * 4) * static_cast<int>(sizeof(S));
@@ -882,7 +917,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         }
         bool plain = false;
         if constexpr (!SPLIT) plain = p.bias == nullptr && p.residual == nullptr && p.addend == nullptr && !p.accumulate && !p.c_f32 && !p.ragged;
-        if (plain) {
+        if constexpr (!kIsF32 && !SPLIT) if (plain) {
             // Straight-line code, no per-lane predicates or address arithmetic (with one wavefront per
             // SIMD every branch and every dependent wait is exposed): the stores go through a buffer
             // descriptor over the wavefront's part of C, whose range ends with the last valid row, so
@@ -918,11 +953,12 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
             }
             return;
         }
-        if constexpr (SPLIT) {
+        if constexpr (SPLIT || kIsF32) if (SPLIT || plain) {
+            // n rounded up to whole 16-byte chunks of 16-bit storage; plain fp32 results: C itself.
+            const int pitch = static_cast<int>(SPLIT ? p.ld_partial : p.ldc), columns = SPLIT ? pitch : p.n;
             const float* origin = static_cast<const float*>(p.c) +
-                                  (static_cast<long>(w.slice) * p.m + row0) * p.ld_partial + (w.n0 + col0);
-            const int pitch = static_cast<int>(p.ld_partial);  // n rounded up to whole 16-byte chunks of storage
-            const int cols_left = min(WN, pitch - (w.n0 + col0));
+                                  (static_cast<long>(w.slice) * p.m + row0) * pitch + (w.n0 + col0);
+            const int cols_left = min(WN, columns - (w.n0 + col0));
             const __amdgpu_buffer_rsrc_t rsrc = part_rsrc(origin, pitch, 4, rows_left, cols_left);
             const int row_bytes = pitch * 4;
 #pragma unroll
@@ -1023,21 +1059,22 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
                         } else {
                             T* out = static_cast<T*>(c_base) + static_cast<long>(m) * c_ld + c_col;
                             if (p.accumulate) {
-                                const vec_t<T, 8> old = load_vec<T, 8>(out);
+                                v0 += vec_to_f32<T, 4>(load_vec<T, 4>(out));
+                                v1 += vec_to_f32<T, 4>(load_vec<T, 4>(out + 4));
+                            }
+                            const vec_t<T, 4> r0 = vec_from_f32<T, 4>(v0), r1 = vec_from_f32<T, 4>(v1);
+                            if constexpr (kIsF32) {  // 16-byte accesses
+                                store_vec<T, 4>(out, r0);
+                                store_vec<T, 4>(out + 4, r1);
+                            } else {
+                                vec_t<T, 8> packed;
 #pragma unroll
                                 for (int e = 0; e < 4; ++e) {
-                                    v0[e] += to_f32(old[e]);
-                                    v1[e] += to_f32(old[4 + e]);
+                                    packed[e] = r0[e];
+                                    packed[4 + e] = r1[e];
                                 }
+                                store_vec<T, 8>(out, packed);
                             }
-                            vec_t<T, 8> packed;
-                            const vec_t<T, 4> r0 = vec_from_f32<T, 4>(v0), r1 = vec_from_f32<T, 4>(v1);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                packed[e] = r0[e];
-                                packed[4 + e] = r1[e];
-                            }
-                            store_vec<T, 8>(out, packed);
                         }
                     }
                 });
@@ -1199,31 +1236,32 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(void* __restric
     }
 }
 
-// Copies a [rows, cols] matrix of 16-bit elements to rows of `pitch` elements (a multiple of 8), zeros past cols:
-// the streamed kernels read whole 16-byte chunks. Eight elements per thread; the source may start anywhere.
-__global__ __launch_bounds__(kThreads) void pad_rows_kernel(std::uint16_t* __restrict__ dst, const std::uint16_t* __restrict__ src,
-                                                            long rows, int cols, long ld, int pitch) {
-    const int chunks = pitch / 8;
+// Copies a [rows, cols] matrix to rows of `pitch` elements (whole 16-byte chunks), zeros past cols: the streamed kernels
+// read whole chunks. One chunk per thread; the source may start anywhere.
+template <typename E>
+__global__ __launch_bounds__(kThreads) void pad_rows_kernel(E* __restrict__ dst, const E* __restrict__ src, long rows, int cols,
+                                                            long ld, int pitch) {
+    constexpr int VEC = kVec128<E>;
+    const int chunks = pitch / VEC;
     const long total = rows * chunks;
     for (long q = static_cast<long>(blockIdx.x) * kThreads + threadIdx.x; q < total; q += static_cast<long>(gridDim.x) * kThreads) {
         const long row = q / chunks;
-        const int col = static_cast<int>(q - row * chunks) * 8;
-        const std::uint16_t* from = src + row * ld + col;
-        vec_t<std::uint16_t, 8> v;
-        if (col + 8 <= cols) {
+        const int col = static_cast<int>(q - row * chunks) * VEC;
+        const E* from = src + row * ld + col;
+        vec_t<E, VEC> v;
+        if (col + VEC <= cols) {
             __builtin_memcpy(&v, from, 16);
         } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = col + e < cols ? from[e] : std::uint16_t{0};
+            for (int e = 0; e < VEC; ++e) v[e] = col + e < cols ? from[e] : E{0};
         }
-        store_vec<std::uint16_t, 8>(dst + row * pitch + col, v);
+        store_vec<E, VEC>(dst + row * pitch + col, v);
     }
 }
 
-// ---- fp32 matrix-core kernel for everything the streamed 16-bit path does not take ---------------
-// fp32 storage (the reference serves it through its tensor-core library too: src/ops/linear.cu:634-667,
-// src/ops/backward/linear_backward.cu:79-82), and 16-bit storage whose K is not a multiple of 32 or whose rows are
-// not 16-byte aligned. Any shape, any alignment, all three operand layouts: a 128 x 128 tile of C per block, K in
+// ---- fp32 matrix-core kernel for everything the streamed path does not take ----------------------
+// Operands that 32-bit byte offsets do not reach, and unaligned ones that cannot be copied to padded rows because the
+// caller owns the arena. Any shape, any alignment, all three operand layouts: a 128 x 128 tile of C per block, K in
 // steps of 16; the four wavefronts own 64 x 64 each and multiply with v_mfma_f32_32x32x2_f32 on fp32 operands
 // (16-bit storage is widened on the way into LDS, so the products are exact and the sums fp32, as in the streamed
 // kernels). Operand tiles go through registers into a K-major LDS layout ([k][m], [k][n]) — the fragment of an
@@ -1379,7 +1417,7 @@ int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream
     // A given in segments along K has kernels of its own (the source of a K tile is then picked
     // per tile), and only unsplit ones.
     const bool segmented = a_k && p.a_seg.count > 0;
-    if constexpr (!SPLIT) {
+    if constexpr (!SPLIT && !std::is_same_v<T, float>) {
         if (segmented && b_k) return launch_mfma<T, BM, BN, true, true, false, true>(p, slices, stream);
         if (segmented && !b_k) return launch_mfma<T, BM, BN, true, false, false, true>(p, slices, stream);
     }
@@ -1392,7 +1430,7 @@ int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream
         if (p.saved != nullptr) return launch_mfma<T, BM, BN, true, false, false, false, false, false, true>(p, slices, stream);
     }
     if (p.saved != nullptr) return fail(CGPTX_RUNTIME, "gemm: the SwiGLU gradient epilogue needs 256-wide unsplit tiles");
-    if constexpr (!SPLIT) {
+    if constexpr (!SPLIT && !std::is_same_v<T, float>) {
         if (a_k && b_k && p.bias == nullptr && p.addend == nullptr && !p.c_f32 && !p.ragged) {
             if (p.residual != nullptr && !p.accumulate) return launch_mfma<T, BM, BN, true, true, false, false, true>(p, slices, stream);
             if (p.residual == nullptr && p.accumulate && p.c_seg.count == 0) {
@@ -1438,7 +1476,9 @@ struct Plan {
 Plan make_plan(const GemmArgs& g) {
     Plan plan;
     const long units = compute_units();
-    const long k_tiles = static_cast<long>((g.k + kBK - 1) / kBK);
+    const bool f32 = g.dtype == CGPTX_F32;
+    const long k_step = f32 ? kBK<float> : kBK<bf16_t>;
+    const long k_tiles = (static_cast<long>(g.k) + k_step - 1) / k_step;
     auto tiles_of = [&](long edge) {
         return static_cast<long>((g.m + edge - 1) / edge) * static_cast<long>((g.n + edge - 1) / edge);
     };
@@ -1455,16 +1495,19 @@ Plan make_plan(const GemmArgs& g) {
     const bool splits = may_split && big_tiles >= 8 && k_tiles >= 32 * ((units + big_tiles - 1) / big_tiles);
     const int forced = forced_tile();
     if (g.swiglu_out != nullptr || g.swiglu_saved != nullptr || g.batch_rows != 0) plan.tile = 256;
+    else if (f32) plan.tile = tiles_of(128) >= 4 * units ? 128 : 64;  // bound by the fp32 matrix rate: finer is better balanced
     else if (forced != 0) plan.tile = forced;
     else if (fills || splits) plan.tile = 256;
     else plan.tile = tiles_of(128) >= units ? 128 : 64;
     const long tiles = tiles_of(plan.tile);
     const long want_blocks = units * blocks_per_unit(plan.tile);
     long slices = 1;
-    if (may_split && tiles < want_blocks && k_tiles >= 32) {
+    // K tiles a slice has at least: an fp32 K tile takes four times as long.
+    const long shortest = f32 ? 8 : 16;
+    if (may_split && tiles < want_blocks && k_tiles >= 2 * shortest) {
         // As many slices as fit the CU slots in one go: one item more than that would cost a
         // second round of the persistent blocks.
-        slices = std::max<long>(1, std::min<long>(want_blocks / tiles, k_tiles / 16));
+        slices = std::max<long>(1, std::min<long>(want_blocks / tiles, k_tiles / shortest));
     }
     if (g.batch_rows != 0 && may_split && k_tiles >= 32) {
         // A stack of products brings any number of tiles: the slice count that needs the least time, counted in
@@ -1553,17 +1596,22 @@ bool offsets_fit_32bit(const GemmArgs& g, std::size_t elem) {
 // k-contiguous operand has to end with a K tile, since what lies behind it in the row is multiplied too; a k-strided
 // operand's may end anywhere (rows past it are out of the buffer's range).
 bool a_streams(const GemmArgs& g) {
-    return is_aligned16(g.a) && g.lda % 8 == 0 && (g.a_k_contiguous ? g.k % kBK == 0 : std::max(g.a_extent, g.m) % 8 == 0);
+    const std::size_t chunk = 16 / dtype_size(g.dtype);
+    return is_aligned16(g.a) && g.lda % chunk == 0 &&
+           (g.a_k_contiguous ? g.k % (4 * chunk) == 0 : std::max(g.a_extent, g.m) % chunk == 0);
 }
 bool b_streams(const GemmArgs& g) {
-    return is_aligned16(g.b) && g.ldb % 8 == 0 && (g.b_k_contiguous ? g.k % kBK == 0 : std::max(g.b_extent, g.n) % 8 == 0);
+    const std::size_t chunk = 16 / dtype_size(g.dtype);
+    return is_aligned16(g.b) && g.ldb % chunk == 0 &&
+           (g.b_k_contiguous ? g.k % (4 * chunk) == 0 : std::max(g.b_extent, g.n) % chunk == 0);
 }
 // Whether C and what is added to it lie in whole aligned chunks.
 bool c_streams(const GemmArgs& g, std::size_t elem) {
     const std::size_t c_elem = g.c_is_f32 ? 4 : elem;
+    const std::uintptr_t four = 4 * elem - 1;  // bias and residual are read four elements at a time
     return g.n % 8 == 0 && (g.ldc * c_elem) % 16 == 0 && is_aligned16(g.c) &&
-           (g.bias == nullptr || (reinterpret_cast<std::uintptr_t>(g.bias) & 7u) == 0) &&
-           (g.residual == nullptr || ((reinterpret_cast<std::uintptr_t>(g.residual) & 7u) == 0 && g.ldr % 4 == 0)) &&
+           (g.bias == nullptr || (reinterpret_cast<std::uintptr_t>(g.bias) & four) == 0) &&
+           (g.residual == nullptr || ((reinterpret_cast<std::uintptr_t>(g.residual) & four) == 0 && g.ldr % 4 == 0)) &&
            (g.addend_f32 == nullptr || (is_aligned16(g.addend_f32) && g.ld_addend % 4 == 0));
 }
 
@@ -1590,7 +1638,7 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
     p.a_extent = static_cast<int>(std::max(g.a_extent, g.m));
     p.b_extent = static_cast<int>(g.b_extent != 0 ? g.b_extent : g.n);
     p.b_k = static_cast<int>(g.b_k != 0 ? g.b_k : g.k);
-    p.k_tiles = static_cast<int>((g.k + kBK - 1) / kBK);
+    p.k_tiles = static_cast<int>((g.k + kBK<T> - 1) / kBK<T>);
     p.lda = static_cast<long>(g.lda);
     p.ldb = static_cast<long>(g.ldb);
     p.ldc = static_cast<long>(g.ldc);
@@ -1618,7 +1666,7 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
     const bool segmented = g.a_segments.count > 0 || g.c_segments.count > 0;
     if (segmented) {
         if (int s = copy_segments(g.a_segments, g.a_k_contiguous ? g.k : (g.batch_rows != 0 ? g.batch_rows : g.m),
-                                  g.a_k_contiguous ? kBK : 256, p.a_seg))
+                                  g.a_k_contiguous ? kBK<T> : 256, p.a_seg))
             return s;
         if (int s = copy_segments(g.c_segments, g.n, 256, p.c_seg)) return s;
         if (g.c_segments.count > 0 && (g.c_is_f32 || g.residual != nullptr))
@@ -1627,7 +1675,7 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
     }
 
     bool fast = false;
-    if constexpr (!std::is_same_v<T, float>) {
+    {
         GemmArgs whole = g;  // alignment of segmented operands was checked per segment
         if (g.a_segments.count > 0) {
             whole.a = g.a_segments.ptr[0];
@@ -1656,27 +1704,26 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
         CGPTX_LAUNCH_CHECK();
         return CGPTX_OK;
     }
+    const Plan plan = make_plan(g);
     if constexpr (!std::is_same_v<T, float>) {
-        const Plan plan = make_plan(g);
         if (plan.tile == 256) return run_config<T, 256, 256>(g, plan, p, stream);
-        if (plan.tile == 128) return run_config<T, 128, 128>(g, plan, p, stream);
-        return run_config<T, 64, 64>(g, plan, p, stream);
     }
-    return CGPTX_OK;
+    if (plan.tile == 128) return run_config<T, 128, 128>(g, plan, p, stream);
+    return run_config<T, 64, 64>(g, plan, p, stream);
 }
 
 template <typename T>
 int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream) {
     GemmArgs padded = g;
-    const std::size_t k_whole = round_up(g.k, kBK);
+    const std::size_t k_whole = round_up(g.k, kBK<T>), chunk = kVec128<T>;
     std::size_t a_bytes = 0, b_bytes = 0;
     if (pad_a) {
-        padded.lda = g.a_k_contiguous ? k_whole : round_up(g.m, 8);
+        padded.lda = g.a_k_contiguous ? k_whole : round_up(g.m, chunk);
         padded.a_extent = g.a_k_contiguous ? g.m : padded.lda;
         a_bytes = round_up((g.a_k_contiguous ? g.m : g.k) * padded.lda * sizeof(T), 256);
     }
     if (pad_b) {
-        padded.ldb = g.b_k_contiguous ? k_whole : round_up(g.n, 8);
+        padded.ldb = g.b_k_contiguous ? k_whole : round_up(g.n, chunk);
         padded.b_extent = g.b_k_contiguous ? g.n : padded.ldb;
         b_bytes = round_up((g.b_k_contiguous ? g.n : g.k) * padded.ldb * sizeof(T), 256);
     }
@@ -1689,12 +1736,12 @@ int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream) {
     if (pad_a) {
         padded.a = base;
         const std::size_t rows = g.a_k_contiguous ? g.m : g.k, cols = g.a_k_contiguous ? g.k : g.m;
-        if (int s = pad_rows(base, g.a, rows, cols, g.lda, padded.lda, stream)) return s;
+        if (int s = pad_rows(base, g.a, rows, cols, g.lda, padded.lda, g.dtype, stream)) return s;
     }
     if (pad_b) {
         padded.b = base + a_bytes;
         const std::size_t rows = g.b_k_contiguous ? g.n : g.k, cols = g.b_k_contiguous ? g.k : g.n;
-        if (int s = pad_rows(base + a_bytes, g.b, rows, cols, g.ldb, padded.ldb, stream)) return s;
+        if (int s = pad_rows(base + a_bytes, g.b, rows, cols, g.ldb, padded.ldb, g.dtype, stream)) return s;
     }
     padded.no_split = true;
     padded.split_workspace = split_bytes != 0 ? base + a_bytes + b_bytes : nullptr;
@@ -1712,7 +1759,7 @@ bool gemm_fuses_swiglu(const GemmArgs& g) {
     const std::size_t elem = 2, inter = g.n / 2;
     // Whole 128-column units of gate and of up per tile, tiles that fill the chip (the 256x256
     // configuration), 16-byte aligned rows everywhere, and the whole weight within 32-bit offsets.
-    if (g.n % 256 != 0 || g.k % kBK != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
+    if (g.n % 256 != 0 || g.k % kBK<bf16_t> != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
         g.ld_swiglu % 8 != 0 || g.ld_swiglu < inter || !is_aligned16(g.a) || !is_aligned16(g.b) || !is_aligned16(g.c) ||
         !is_aligned16(g.swiglu_out))
         return false;
@@ -1730,7 +1777,7 @@ bool gemm_fuses_swiglu_gradient(const GemmArgs& g) {
     const std::size_t elem = 2;
     // 16-byte chunks of whole rows everywhere, tiles that fill the chip (the 256x256 configuration),
     // and a wavefront's 128 rows of the saved and of the written [gate | up] within 32-bit offsets.
-    if (g.n % 8 != 0 || g.k % kBK != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
+    if (g.n % 8 != 0 || g.k % kBK<bf16_t> != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ldc % 8 != 0 ||
         g.ld_swiglu % 8 != 0 || g.ldc < 2 * g.n || g.ld_swiglu < 2 * g.n || !is_aligned16(g.a) || !is_aligned16(g.b) ||
         !is_aligned16(g.c) || !is_aligned16(g.swiglu_saved))
         return false;
@@ -1755,17 +1802,21 @@ bool gemm_takes_batch(const GemmArgs& g) {
     return true;
 }
 
-int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, hipStream_t stream) {
-    const std::size_t chunks = rows * (pitch / 8);
-    const std::size_t blocks = std::min<std::size_t>((chunks + kThreads - 1) / kThreads, static_cast<std::size_t>(compute_units()) * 16);
-    hipLaunchKernelGGL(pad_rows_kernel, dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), 0, stream,
-                       static_cast<std::uint16_t*>(dst), static_cast<const std::uint16_t*>(src), static_cast<long>(rows),
-                       static_cast<int>(cols), static_cast<long>(ld), static_cast<int>(pitch));
+int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, int dtype,
+             hipStream_t stream) {
+    const std::size_t chunks = rows * (pitch * dtype_size(dtype) / 16);
+    const dim3 grid(static_cast<unsigned int>(std::min<std::size_t>((chunks + kThreads - 1) / kThreads, static_cast<std::size_t>(compute_units()) * 16)));
+    auto launch = [&]<typename E>() {
+        hipLaunchKernelGGL((pad_rows_kernel<E>), grid, dim3(kThreads), 0, stream, static_cast<E*>(dst), static_cast<const E*>(src),
+                           static_cast<long>(rows), static_cast<int>(cols), static_cast<long>(ld), static_cast<int>(pitch));
+    };
+    if (dtype == CGPTX_F32) launch.template operator()<std::uint32_t>();
+    else launch.template operator()<std::uint16_t>();
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
 }
 
-std::size_t gemm_split_bytes(const GemmArgs& g) { return g.dtype == CGPTX_F32 ? 0 : make_plan(g).partial_bytes(g); }
+std::size_t gemm_split_bytes(const GemmArgs& g) { return make_plan(g).partial_bytes(g); }
 
 int gemm(const GemmArgs& g, hipStream_t stream) {
     if ((g.a == nullptr && g.a_segments.count == 0) || g.b == nullptr || (g.c == nullptr && g.c_segments.count == 0) ||

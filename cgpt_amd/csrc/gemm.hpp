@@ -78,8 +78,9 @@ struct GemmArgs {
 int gemm(const GemmArgs& args, hipStream_t stream);
 // Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
 std::size_t gemm_split_bytes(const GemmArgs& args);
-// Copies [rows, cols] 16-bit elements (row stride ld) to rows of `pitch` elements (a multiple of 8), zeros past cols.
-int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, hipStream_t stream);
+// Copies [rows, cols] elements (row stride ld) to rows of `pitch` elements (whole 16-byte chunks), zeros past cols.
+int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, int dtype,
+             hipStream_t stream);
 // Whether gemm() serves args.swiglu_out for this call (shape, layout and alignment of the fused kernel).
 bool gemm_fuses_swiglu(const GemmArgs& args);
 bool gemm_fuses_swiglu_gradient(const GemmArgs& args);

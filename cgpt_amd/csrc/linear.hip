@@ -164,6 +164,7 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
     auto stream = static_cast<hipStream_t>(stream_);
     // An output gradient whose rows are not whole 16-byte chunks feeds both contractions from one padded copy (each would
     // make its own otherwise).
+    const std::size_t elem = dtype_size(dtype);
     const void* dy = grad_output;
     std::size_t dy_pitch = out_features;
     void* split_room = nullptr;
@@ -210,15 +211,15 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
         return g;
     };
     constexpr std::size_t kSpan = (std::size_t{1} << 31) - (std::size_t{1} << 21);  // the streamed kernels' 32-bit offsets
-    if (grad_input != nullptr && grad_weight != nullptr && dtype != CGPTX_F32 &&
-        (out_features % 8 != 0 || !is_aligned16(grad_output)) && in_features % 8 == 0 && is_aligned16(weight) &&
-        is_aligned16(input) && rows * (out_features + 32 + in_features) * 2 < kSpan && out_features * in_features * 2 < kSpan) {
+    if (grad_input != nullptr && grad_weight != nullptr &&
+        (out_features * elem % 16 != 0 || !is_aligned16(grad_output)) && in_features * elem % 16 == 0 && is_aligned16(weight) &&
+        is_aligned16(input) && rows * (out_features + 32 + in_features) * elem < kSpan && out_features * in_features * elem < kSpan) {
         dy_pitch = (out_features + 31) / 32 * 32;
-        const std::size_t copy_bytes = (rows * dy_pitch * 2 + 255) & ~std::size_t{255};
+        const std::size_t copy_bytes = (rows * dy_pitch * elem + 255) & ~std::size_t{255};
         split_bytes = std::max(gemm_split_bytes(input_gradient()), gemm_split_bytes(weight_gradient())) + 256;
         void* mem = nullptr;
         if (int s = scratch(stream, copy_bytes + split_bytes, &mem)) return s;
-        if (int s = pad_rows(mem, grad_output, rows, out_features, out_features, dy_pitch, stream)) return s;
+        if (int s = pad_rows(mem, grad_output, rows, out_features, out_features, dy_pitch, dtype, stream)) return s;
         dy = mem;
         split_room = static_cast<char*>(mem) + copy_bytes;
     }
