@@ -70,11 +70,42 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
     const std::size_t loss_bytes = (rows * sizeof(float) + 255) & ~std::size_t{255};
     const std::size_t acc_bytes = single ? 0 : (vocab * hidden * sizeof(float) + 255) & ~std::size_t{255};
     const std::size_t logit_bytes = (chunk * pitch * elem + 255) & ~std::size_t{255};
-    // A chunk's input gradient has few output tiles ([chunk, hidden]) and a long K (the vocabulary): with several
-    // chunks it is split along K into up to `units / tiles` slices, whose fp32 partial tiles need room of their own.
-    const std::size_t dx_tiles = ((chunk + 255) / 256) * ((hidden + 255) / 256);
-    const std::size_t dx_slices = single ? 1 : std::max<std::size_t>(1, static_cast<std::size_t>(compute_units()) / std::max<std::size_t>(dx_tiles, 1));
-    const std::size_t split_bytes = dx_slices > 1 ? (dx_slices * chunk * hidden * sizeof(float) + 255) & ~std::size_t{255} : 0;
+    // The gradients' contractions may be split along K (a chunk's input gradient has few output tiles and the vocabulary
+    // as its K, a small vocabulary's gradient few tiles and the rows); their partial tiles get room of their own.
+    auto input_gradient_call = [&](std::size_t r0, std::size_t r) {  // dX[r, H] = dZ[r, V]·C[V, H]
+        GemmArgs dx;
+        dx.b = classifier;
+        dx.c = static_cast<char*>(input_gradient) + r0 * hidden * elem;
+        dx.m = r;
+        dx.n = hidden;
+        dx.k = pitch;
+        dx.b_k = vocab;
+        dx.lda = pitch;
+        dx.ldb = hidden;
+        dx.ldc = hidden;
+        dx.b_k_contiguous = false;
+        dx.dtype = dtype;
+        return dx;
+    };
+    auto classifier_gradient_call = [&](std::size_t r0, std::size_t r) {  // dC[V, H] = dZᵀ[V, r]·X[r, H]
+        GemmArgs dc;
+        dc.b = static_cast<const char*>(input) + r0 * hidden * elem;
+        dc.m = vocab;
+        dc.a_extent = pitch;
+        dc.n = hidden;
+        dc.k = r;
+        dc.lda = pitch;
+        dc.ldb = hidden;
+        dc.ldc = hidden;
+        dc.a_k_contiguous = false;
+        dc.b_k_contiguous = false;
+        dc.dtype = dtype;
+        return dc;
+    };
+    std::size_t split_bytes = 0;
+    for (const std::size_t r : {chunk, (rows - 1) % chunk + 1})
+        split_bytes = std::max({split_bytes, gemm_split_bytes(input_gradient_call(0, r)), gemm_split_bytes(classifier_gradient_call(0, r))});
+    split_bytes = (split_bytes + 255) & ~std::size_t{255};
     void* mem = nullptr;
     // Arena layout: [row_loss | acc | split-K partials | logits]. The contractions below run with no_split: they
     // never ask the arena for scratch of their own, and split only into the room given to them here.
@@ -104,19 +135,8 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         if (int s = gemm(z, stream)) return s;
         if (int s = cross_entropy_rows(row_loss + r0, logits, pitch, logits, pitch, targets + r0, r, vocab, factor, dtype, stream))
             return s;
-        GemmArgs dx;  // dX[r, H] = dZ[r, V]·C[V, H]
+        GemmArgs dx = input_gradient_call(r0, r);
         dx.a = logits;
-        dx.b = classifier;
-        dx.c = static_cast<char*>(input_gradient) + r0 * hidden * elem;
-        dx.m = r;
-        dx.n = hidden;
-        dx.k = pitch;
-        dx.b_k = vocab;
-        dx.lda = pitch;
-        dx.ldb = hidden;
-        dx.ldc = hidden;
-        dx.b_k_contiguous = false;
-        dx.dtype = dtype;
         dx.no_split = true;
         dx.split_workspace = split_room;
         dx.split_workspace_bytes = split_bytes;
@@ -125,27 +145,18 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         // starts it), the last one adds acc to its own and writes the gradient, rounded once. A single chunk
         // writes the gradient itself.
         const bool last = r0 + chunk >= rows;
-        GemmArgs dc;
+        GemmArgs dc = classifier_gradient_call(r0, r);
         dc.a = logits;
-        dc.b = x;
         dc.c = last ? classifier_gradient : static_cast<void*>(acc);
-        dc.m = vocab;
-        dc.a_extent = pitch;
-        dc.n = hidden;
-        dc.k = r;
-        dc.lda = pitch;
-        dc.ldb = hidden;
-        dc.ldc = hidden;
-        dc.a_k_contiguous = false;
-        dc.b_k_contiguous = false;
         dc.accumulate = last ? accumulate_classifier != 0 : r0 != 0;
         dc.c_is_f32 = !last;
         if (last && !single) {
             dc.addend_f32 = acc;
             dc.ld_addend = hidden;
         }
-        dc.dtype = dtype;
         dc.no_split = true;
+        dc.split_workspace = split_room;
+        dc.split_workspace_bytes = split_bytes;
         if (int s = gemm(dc, stream)) return s;
     }
     return mean_reduce(loss, row_loss, rows, stream);

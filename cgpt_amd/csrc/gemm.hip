@@ -44,336 +44,19 @@
 // with v_mfma_f32_16x16x4_f32 and K steps of 16. Operands beyond 32-bit offsets, and unaligned ones
 // of a caller that owns the arena, run on a general fp32 matrix-core kernel
 // (v_mfma_f32_32x32x2_f32, register-staged operand tiles) with the same semantics.
-#include "gemm.hpp"
+#include "gemm_small.hpp"
+#include "gemm_tiles.hpp"
 
 #include <algorithm>
-#include <type_traits>
-#include <utility>
+#include <cmath>
 #include <cstdlib>
-#include <limits>
 
 namespace cgptx {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / kWave;
-// K step per LDS stage: 64 bytes of a k-contiguous operand's row.
-template <typename T>
-constexpr int kBK = 64 / static_cast<int>(sizeof(T));
 // LDS stages of a block: one being multiplied, one being refilled, the rest in flight. 256x256
-// blocks own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each), and so do 64x64
-// blocks: their K tiles are short (4 MFMAs per wavefront), so ten 8 KiB stages keep as many bytes in flight.
-constexpr int stages_for(int bm, int /*bn*/) { return bm == 64 ? 10 : 5; }
-constexpr int kXcds = 8;
-
-
-using acc_t = vec_t<float, 4>;
-
-// fp32 storage: four v_mfma_f32_16x16x4_f32 take the K tile of 16 (lane l holds row or column l%16 at k = 4*(l/16) + e
-// for step e; the accumulator's layout is that of the 16-bit form). 64 accumulator registers at most, left to the
-// compiler.
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<float> {
-    using frag = vec_t<float, 4>;
-    __device__ static __forceinline__ void run(acc_t& c, const frag& a, const frag& b) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
-    }
-    __device__ static __forceinline__ void start(acc_t& c, const frag& a, const frag& b) {
-        c = acc_t(0.0f);
-        run(c, a, b);
-    }
-};
-
-// 16-bit storage: c += a x b with v_mfma_f32_16x16x32 (a: 16 rows x 32 k, b: 32 k x 16 columns; lane l holds row or
-// column l%16, k = 8*(l/16) .. +7; c: lane l holds rows 4*(l/16) .. +3 of column l%16). Written as
-// assembly so that the accumulator is updated in place: the four-register form of the instruction
-// does not tie its result to its addend, and with all 256 accumulator registers in use the register
-// allocator would otherwise shuffle accumulators around every MFMA. The kernel keeps the distances
-// the hardware asks for by construction: an accumulator is touched once per K tile (64 or 16 MFMAs
-// apart), zeroed long before its first MFMA and read by the epilogue only after a barrier.
-template <>
-struct Mfma<bf16_t> {
-    using frag = vec_t<bf16_t, 8>;
-    __device__ static __forceinline__ void run(acc_t& c, const frag& a, const frag& b) {
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-    }
-    // c = a x b: the first K tile of an item starts the sums, so the accumulators are never cleared.
-    __device__ static __forceinline__ void start(acc_t& c, const frag& a, const frag& b) {
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-    }
-};
-template <>
-struct Mfma<f16_t> {
-    using frag = vec_t<f16_t, 8>;
-    __device__ static __forceinline__ void run(acc_t& c, const frag& a, const frag& b) {
-        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-    }
-    __device__ static __forceinline__ void start(acc_t& c, const frag& a, const frag& b) {
-        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-    }
-};
-
-using u32x4 = vec_t<unsigned int, 4>;
-
-struct KernelSegments {
-    const void* ptr[3];
-    long ld[3];
-    int cols[3];
-    int count;
-};
-
-struct KernelArgs {
-    const void* a;
-    const void* b;
-    void* c;            // T* (or float* when c_f32), or float partials when split
-    const void* bias;
-    const void* residual;  // T*, row stride ldr, or null
-    const float* addend;   // fp32 [M, N], row stride ld_addend, added before anything else, or null
-    long ld_addend;
-    int m, n, k;
-    // What the operands hold: rows or columns of A and of B (A's may exceed m, B's n: whole 16-byte chunks of padded
-    // rows), K positions of B (below k when A's padding reaches further: past them B reads as zeros).
-    int a_extent, b_extent, b_k;
-    int k_tiles;            // K tiles of kBK, the last one possibly short
-    int ragged;             // C (or an addend) has rows that are not whole 16-byte chunks: stored element by element
-    long ld_partial;        // SPLIT kernels: row length of a partial tile matrix
-    long lda, ldb, ldc, ldr;
-    int tiles_m, tiles_n;
-    int k_tiles_per_slice;  // K tiles handled by one work item
-    int slices;             // K slices per output tile
-    int accumulate;
-    int c_f32;
-    KernelSegments a_seg, c_seg;  // column segments of A (as stored) and of C; count 0 = one buffer
-    // ceil(2^32 / (group rows * tiles_n)) when multiplying by it divides every item index of the
-    // launch exactly, else 0 (the kernel then divides).
-    unsigned int group_reciprocal;
-    int group_rows_log2;  // tile-rows per L2 locality group: 1 << group_rows_log2
-    void* act;      // SWIGLU kernels: [M, inter] = silu(gate) * up, T*
-    long ld_act;
-    const void* saved;  // GRAD kernels: the forward's [M, 2 * inter] = [gate | up], T*
-    long ld_saved;
-    int inter;      // SWIGLU kernels: columns of gate (= of up); n = 2 * inter
-    // Stacked products (weight-gradient layout only): rows of C per product (0 = one product) and what a and b (or
-    // A's segments) move by from one product to the next, in elements.
-    int batch_rows;
-    long a_batch_stride, b_batch_stride;
-    long a_seg_batch_stride[3];
-};
-
-// The column segment (of up to three) that holds column `col`, picked with selects: indexing the
-// kernel-argument arrays by a run-time value would move them to private memory.
-struct SegmentPick {
-    const void* ptr;
-    long ld;
-    int first;  // first column of the segment
-    int cols;
-    int index;  // which segment
-};
-__device__ __forceinline__ SegmentPick pick_segment(const KernelSegments& seg, int col) {
-    const int end0 = seg.cols[0], end1 = end0 + seg.cols[1];
-    const bool in1 = seg.count > 1 && col >= end0;
-    const bool in2 = seg.count > 2 && col >= end1;
-    SegmentPick pick;
-    pick.ptr = in2 ? seg.ptr[2] : in1 ? seg.ptr[1] : seg.ptr[0];
-    pick.ld = in2 ? seg.ld[2] : in1 ? seg.ld[1] : seg.ld[0];
-    pick.first = in2 ? end1 : in1 ? end0 : 0;
-    pick.cols = in2 ? seg.cols[2] : in1 ? seg.cols[1] : seg.cols[0];
-    pick.index = in2 ? 2 : in1 ? 1 : 0;
-    return pick;
-}
-
-// s_waitcnt immediate that waits until at most `count` vector-memory operations are outstanding
-// (and for nothing else).
-constexpr int vmcnt_immediate(int count) { return (count & 15) | ((count >> 4) << 14) | 0x0F70; }
-
-// Buffer descriptor (raw buffer, range-checked) over `bytes` bytes starting at base (both the same
-// for all lanes). The words are pinned to scalar registers: 64-bit comparisons have no scalar form,
-// and one of them on the way would drag the descriptor, and every address derived with it, into
-// vector registers.
-__device__ __forceinline__ u32x4 make_rsrc(const void* base, long bytes) {
-    const unsigned long address = reinterpret_cast<unsigned long>(base);
-    const unsigned int size_low = static_cast<unsigned int>(bytes);
-    const unsigned int size_high = static_cast<unsigned int>(static_cast<unsigned long>(bytes) >> 32);
-    u32x4 words;
-    words[0] = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(address));
-    words[1] = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(address >> 32) & 0xFFFFu);  // stride 0
-    words[2] = __builtin_amdgcn_readfirstlane(size_high != 0 ? 0xFFFFFFFFu : size_low);
-    words[3] = 0x00020000u;
-    return words;
-}
-
-// One wavefront-wide 16-byte-per-lane load from a buffer straight into LDS: lane l's bytes land at
-// lds_base + LDS_OFFSET + 16 l. Returns soffset + step, the scalar offset of the operand's next load
-// (that addition sits between the write of M0 and the load, which need one instruction between them
-// anyway). Written as assembly on purpose: the compiler would order every later LDS read after *all*
-// outstanding loads of this kind (vmcnt(0)), which defeats keeping several K tiles in flight; the
-// kernel counts its loads itself (vmcnt_immediate). M0 is used by nothing else here.
-template <int LDS_OFFSET>
-__device__ __forceinline__ unsigned int load_to_lds(const u32x4& rsrc, unsigned int lds_base, int voffset,
-                                                    unsigned int soffset, unsigned int step) {
-    unsigned int next;
-    asm volatile("s_add_u32 m0, %1, %2\n\ts_add_u32 %0, %3, %4\n\tbuffer_load_dwordx4 %5, %6, %3 offen lds"
-                 : "=&s"(next)
-                 : "s"(lds_base), "n"(LDS_OFFSET), "s"(soffset), "s"(step), "v"(voffset), "s"(rsrc)
-                 : "scc");
-    return next;
-}
-
-// Workgroup barrier without the fence __syncthreads() carries: LDS reads still in flight may
-// cross it (their registers are waited for where they are used).
-__device__ __forceinline__ void barrier_only() { asm volatile("s_barrier" ::: "memory"); }
-
-// Where a wavefront's loads of one operand's K tile come from: load i reads at scalar offset
-// soffset + i * step.
-struct TileCursor {
-    u32x4 rsrc;
-    int voffset;
-    unsigned int soffset;
-    unsigned int step;
-    unsigned int step2;  // advance after the operand's odd-numbered loads (differs from step only for SWIGLU's B)
-};
-
-template <int BEGIN, int... I, typename F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-    (f(std::integral_constant<int, BEGIN + I>{}), ...);
-}
-// f(integral_constant<int, i>) for i = BEGIN .. END-1, unrolled at compile time.
-template <int BEGIN, int END, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl<BEGIN>(std::make_integer_sequence<int, (END > BEGIN ? END - BEGIN : 0)>{}, f);
-}
-
-template <typename T>
-__device__ __forceinline__ unsigned int lds_address_of(const T* p) {
-    return static_cast<unsigned int>(reinterpret_cast<unsigned long>((__attribute__((address_space(3))) const T*)(p)));
-}
-
-// Operand tiles travel global -> LDS with buffer_load ... lds: a wavefront-wide load drops
-// 64 x 16 B contiguously into LDS, no staging registers and no LDS stores, and the only per-lane
-// address is a loop-invariant byte offset (the K position is a scalar offset). LDS rows therefore
-// cannot be padded; bank conflicts are avoided by storing 16-byte chunk c of a row at chunk
-// position c ^ swizzle(row) — the lane that owns an LDS slot fetches the matching global chunk.
-
-// ---- operand stored [ROWS, K] (k-contiguous): ROWS x kBK slab, unpadded LDS rows ---------------
-// One load instruction covers 1024 B = kRowsPerLoad rows; wavefront w issues the loads of row
-// groups w, w+4, ... The chunk swizzle is (row / rows per 256 B) mod chunks per row: the 16 rows a
-// quarter-wavefront reads with ds_read_b128 then hit the 16 different 16-byte positions of a
-// 256-byte bank period.
-template <typename T, int ROWS>
-struct KTile {
-    using frag_t = typename Mfma<T>::frag;
-    static constexpr int kChunksPerRow = kBK<T> / kVec128<T>;
-    static constexpr int kRowsPerLoad = 64 / kChunksPerRow;
-    static constexpr int kElems = ROWS * kBK<T>;
-    static constexpr int kLoads = ROWS / kRowsPerLoad / kWaves;  // load instructions per wavefront and tile
-
-    u32x4 rsrc = {0u, 0u, 0u, 0u};
-    int voffset = 0;
-    unsigned int group_bytes = 0;  // kRowsPerLoad rows further in global memory
-
-    __device__ __forceinline__ static int swizzle(int row) { return (row / 4) % kChunksPerRow; }
-
-    // base: element (row0, 0) of the operand; rows past rows_left only feed C rows that are never
-    // stored (they read zeros or whatever follows, never out of the allocation's last row).
-    __device__ __forceinline__ void init(const T* base, long ld, int rows_left, int k_total, int wave) {
-        const int lane = threadIdx.x & (kWave - 1);
-        rsrc = make_rsrc(base, (static_cast<long>(rows_left - 1) * ld + k_total) * static_cast<long>(sizeof(T)));
-        const int row = lane / kChunksPerRow;
-        // The tile row of this lane's slot is (i*4 + wave) * kRowsPerLoad + row; its swizzle does not depend on i.
-        voffset = static_cast<int>(row * ld * sizeof(T)) +
-                  (((lane % kChunksPerRow) ^ swizzle(wave * kRowsPerLoad + row)) * 16);
-        group_bytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(kRowsPerLoad * ld * sizeof(T)));
-    }
-    // Scalar offset of wavefront `wave`'s first load of the tile that starts at column k0.
-    __device__ __forceinline__ unsigned int first_offset(int k0, int wave) const {
-        return wave * group_bytes + k0 * static_cast<unsigned int>(sizeof(T));
-    }
-    // Element offset of the lane's fragment within a 16-row block (the whole K tile is one MFMA
-    // step): row lane%16, the lane/16-th 16 bytes of it. The swizzle of a row does not depend on the block.
-    __device__ __forceinline__ static int lane_offset(int lane) {
-        return (lane & 15) * kBK<T> + (((lane >> 4) ^ swizzle(lane & 15)) * kVec128<T>);
-    }
-    __device__ __forceinline__ static frag_t frag(const T* tile, int block0, int offset) {
-        return *reinterpret_cast<const frag_t*>(tile + block0 * kBK<T> + offset);
-    }
-};
-
-// ---- operand stored [K, COLS] (n-contiguous): 32 x COLS slab kept in that order in LDS ---------
-// The transpose happens on the way out of LDS: ds_read_b64_tr_b16 hands lane n of a 16-lane group
-// the four k-values of column n from a 4(k) x 16(n) block, so two of them build the 8-k fragment of
-// one column. swizzle(k row) = 4*(row%4) on the chunk index (rows of 128 bytes: 4*(row/2%2), the row's parity
-// picks the half already): the four k rows that 32 lanes read sit in four different 64-byte windows of the
-// 256-byte bank period. K rows past the operand's end are out of the buffer's range and read as zeros.
-template <typename T, int COLS>
-struct NTile {
-    using frag_t = typename Mfma<T>::frag;
-    static constexpr int kChunksPerRow = COLS / kVec128<T>;
-    static constexpr int kRowsPerLoad = 64 / kChunksPerRow;  // k rows one load instruction covers (2, 4 or 8)
-    static constexpr int kElems = kBK<T> * COLS;
-    static constexpr int kLoads = kBK<T> / kRowsPerLoad / kWaves;
-
-    // fp32: the four k rows a read touches lie four apart (k = 4*(lane/16) + e); of their two low group bits those are
-    // used that a wavefront's loads have in common.
-    __device__ __forceinline__ static int swizzle(int k_row) {
-        if constexpr (std::is_same_v<T, float>) return COLS >= 128 ? k_row & 4 : k_row & 12;
-        else return COLS >= 128 ? (k_row & 3) << 2 : (k_row & 2) << 1;
-    }
-
-    u32x4 rsrc = {0u, 0u, 0u, 0u};
-    int voffset = 0;
-    unsigned int group_bytes = 0;  // kRowsPerLoad k rows further in global memory
-
-    // base: element (0, col0) of the operand. Column chunks past cols_left are clamped to the last
-    // valid chunk: they only feed C columns that are never stored.
-    __device__ __forceinline__ void init(const T* base, long ld, int cols_left, int k_total, int wave) {
-        const int lane = threadIdx.x & (kWave - 1);
-        rsrc = make_rsrc(base, (static_cast<long>(k_total - 1) * ld + cols_left) * static_cast<long>(sizeof(T)));
-        const int row = lane / kChunksPerRow;                  // within the instruction's rows
-        const int k_row = wave * kRowsPerLoad + row;           // tile row of the first load; its swizzle is that of all
-        const int chunk = min((lane % kChunksPerRow) ^ swizzle(k_row), cols_left / kVec128<T> - 1);
-        voffset = static_cast<int>(row * ld * sizeof(T)) + chunk * 16;
-        group_bytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(kRowsPerLoad * ld * sizeof(T)));
-    }
-    // Scalar offset of wavefront `wave`'s first load of the tile that starts at row k0.
-    __device__ __forceinline__ unsigned int first_offset(int k0, int wave) const {
-        return (wave + k0 / kRowsPerLoad) * group_bytes;
-    }
-    // Lane i of a 16-lane group addresses k row i/4, columns 4*(i%4) .. +3 of the group's 4 x 16
-    // block; group g (lanes 16g .. 16g+15) takes the k values 8g .. 8g+7 of the fragment's 16
-    // columns in two reads (k rows +0..3, +4..7). The offset is for the first read; block0 is a
-    // multiple of 16.
-    __device__ __forceinline__ static int lane_offset(int lane, int block0) {
-        if constexpr (std::is_same_v<T, float>) {  // k rows 4*(lane/16) + e, column block0 + lane%16
-            const int row = (lane >> 4) * 4, column_chunk = (block0 + (lane & 15)) / 4;
-            return row * COLS + (column_chunk ^ swizzle(row)) * 4 + (lane & 3);
-        }
-        const int k_row = (lane >> 4) * 8 + ((lane & 15) >> 2);
-        const int chunk = ((block0 / 8) ^ swizzle(k_row)) + ((lane & 3) >> 1);
-        return k_row * COLS + chunk * 8 + (lane & 1) * 4;
-    }
-    __device__ __forceinline__ static frag_t frag(const T* tile, int offset) {
-        if constexpr (std::is_same_v<T, float>) {
-            const T* q = tile + offset;
-            return frag_t{q[0], q[COLS], q[2 * COLS], q[3 * COLS]};
-        } else {
-        using s16x4 = vec_t<short, 4>;
-        using lds_ptr = __attribute__((address_space(3))) s16x4*;
-        const T* q = tile + offset;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(q));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(q + 4 * COLS));
-        vec_t<short, 8> both;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            both[e] = lo[e];
-            both[4 + e] = hi[e];
-        }
-        return __builtin_bit_cast(frag_t, both);
-        }
-    }
-};
+// blocks own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each).
+constexpr int stages_for(int /*bm*/, int /*bn*/) { return 5; }
 
 template <typename T, int BM, int BN, bool A_K, bool B_K>
 struct TileLayout {
@@ -1376,6 +1059,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma_kernel(KernelArgs p, i
 // ------------------------------------------------------------------- host side
 constexpr int blocks_per_unit(int tile) { return tile == 256 ? 1 : 2; }  // resident blocks per CU: what the LDS stages allow
 
+
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
           bool SWIGLU = false, bool GRAD = false>
 int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
@@ -1450,13 +1134,13 @@ int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream
     return fail(CGPTX_RUNTIME, "gemm: unsupported operand layout");
 }
 
-// CGPTX_GEMM_TILE=64|128|256 pins the tile size (for experiments); anything else = automatic.
+// CGPTX_GEMM_TILE=32|64|128|256 pins the tile size (for experiments); anything else = automatic.
 int forced_tile() {
     static const int value = [] {
         const char* text = std::getenv("CGPTX_GEMM_TILE");
         if (text == nullptr) return 0;
         const int v = std::atoi(text);
-        return (v == 64 || v == 128 || v == 256) ? v : 0;
+        return (v == 32 || v == 64 || v == 128 || v == 256) ? v : 0;
     }();
     return value;
 }
@@ -1468,10 +1152,45 @@ struct Plan {
     int tile = 256;
     int slices = 1;
     int k_tiles_per_slice = 1;
+    bool deep = false;  // small tiles: all of a CU's LDS for one workgroup's stages
     std::size_t partial_bytes(const GemmArgs& g) const {
         return slices > 1 ? static_cast<std::size_t>(slices) * g.m * round_up(g.n, 8) * sizeof(float) : 0;
     }
 };
+
+// Predicted time of a call in microseconds, from launches measured on random bf16 data inside a graph (operands rotated
+// through 64 MB; K tiles of 64 bytes): what a kernel costs before its K loop, plus the K loop of the busiest CU.
+//   256: one block per CU, 8.5 us for filling its pipeline and storing its tile, 0.55 per K tile on an idle chip, 0.69 at
+//        the power limit of a full one
+//   128: two blocks per CU share its matrix cores: 0.29 per K tile and block
+//    64: 0.128 per K tile and block, 0.14 where few blocks run, whose first 16 K tiles come in one latency
+//    32: 0.07 - 0.1 per K tile (k-contiguous operands stream best), up to one block per CU
+// A split along K adds a launch and the partial tiles' way to memory and back. fp32 K tiles hold 16 positions and take about
+// as long as the fp32 matrix rate asks (0.93 per K tile of 128 x 128), smaller tiles somewhat longer for their share.
+// [M, N] x K: 128 x 768 x 768 32/1 4.8, 64/1 5.1, 128/1 9.7; 1024 x 1024 x 1024 64/1 7.8, 128/1 12.7, 256/1 26; 4096 x 1024 x
+// 1024 128/1 14.5, 64/1 19, 256/1 27; 16384 x 1024 x 1024 256/1 34, 128/1 42; 768 x 768 x 8192 128/6 22, 64/3 27 - 30, 256/16
+// 30; 2048 x 768 x 50272 256/8 145 - 179, 128/8 184 - 255, 64/2 284 - 371; 16384 x 768 x 32000 256/1 688, 128/1 976; fp32
+// 256 x 1024 x 1024 32/1 10, 64/4 15, 128/8 20; 256 x 32000 x 1024 128/1 123, 64/1 149 (tile / slices).
+double predicted_us(int tile, long tiles, long slices, long k_tiles, double partial_mb, bool f32, bool a_k, bool b_k, long units) {
+    const double kt = static_cast<double>((k_tiles + slices - 1) / slices);
+    const double load = static_cast<double>(tiles * slices) / static_cast<double>(units);
+    const double blocks = std::ceil(load);
+    double time = 0.0;
+    if (f32) {
+        const double per_tile = tile == 32 ? 0.088 : tile == 64 ? 0.265 : 0.93;
+        time = (tile == 32 ? 3.0 : tile == 64 ? 4.0 : 5.0) + kt * per_tile * (tile == 32 ? std::max(1.0, load) : blocks);
+    } else if (tile == 256) {
+        time = blocks * (8.5 + kt * (0.55 + 0.14 * load / blocks));
+    } else if (tile == 128) {
+        time = 5.0 + kt * (load < 0.5 ? 0.23 : 0.29 * blocks) + 2.0 * std::max(0.0, std::ceil(blocks / 2.0) - 1.0);
+    } else if (tile == 64) {
+        time = load <= 1.0 ? 3.8 + 0.02 * std::min(kt, 16.0) + std::max(0.0, kt - 16.0) * (!a_k && load < 0.6 ? 0.095 : 0.135)
+                           : 3.8 + kt * 0.128 * blocks * (blocks > 4.0 ? 1.3 : 1.0);
+    } else {
+        time = 3.0 + kt * (!a_k ? 0.1 : b_k ? 0.07 : 0.085) * std::max(1.0, 0.92 * load);
+    }
+    return slices > 1 ? time + 3.0 + 0.45 * partial_mb + 0.3 * std::min(partial_mb, 8.0) : time;
+}
 
 Plan make_plan(const GemmArgs& g) {
     Plan plan;
@@ -1485,56 +1204,122 @@ Plan make_plan(const GemmArgs& g) {
     const bool may_split = (!g.no_split || g.split_workspace != nullptr) && g.residual == nullptr && g.addend_f32 == nullptr &&
                            g.swiglu_out == nullptr && g.swiglu_saved == nullptr && g.c_segments.count == 0 &&
                            !(g.a_k_contiguous && g.a_segments.count > 0);
-    // 256x256 tiles (one block per CU, 64 MFMAs per wavefront and K step) when they still give
-    // every CU a tile, or when K is long enough to be split across the idle CUs without the
-    // fp32 partial tiles outweighing the contraction (at least 8 tiles, so at most 32 slices);
-    // otherwise 128x128 tiles, with K split when even those are too few, and 64x64 tiles where
-    // 128x128 ones would leave most of the chip idle.
-    const long big_tiles = tiles_of(256);
-    const bool fills = big_tiles * 5 >= units * 4;
-    const bool splits = may_split && big_tiles >= 8 && k_tiles >= 32 * ((units + big_tiles - 1) / big_tiles);
-    const int forced = forced_tile();
-    if (g.swiglu_out != nullptr || g.swiglu_saved != nullptr || g.batch_rows != 0) plan.tile = 256;
-    else if (f32) plan.tile = tiles_of(128) >= 4 * units ? 128 : 64;  // bound by the fp32 matrix rate: finer is better balanced
-    else if (forced != 0) plan.tile = forced;
-    else if (fills || splits) plan.tile = 256;
-    else plan.tile = tiles_of(128) >= units ? 128 : 64;
-    const long tiles = tiles_of(plan.tile);
-    const long want_blocks = units * blocks_per_unit(plan.tile);
-    long slices = 1;
-    // K tiles a slice has at least: an fp32 K tile takes four times as long.
-    const long shortest = f32 ? 8 : 16;
-    if (may_split && tiles < want_blocks && k_tiles >= 2 * shortest) {
-        // As many slices as fit the CU slots in one go: one item more than that would cost a
-        // second round of the persistent blocks.
-        slices = std::max<long>(1, std::min<long>(want_blocks / tiles, k_tiles / shortest));
+    auto set_slices = [&](long slices) {
+        plan.k_tiles_per_slice = static_cast<int>((k_tiles + slices - 1) / slices);
+        plan.slices = static_cast<int>((k_tiles + plan.k_tiles_per_slice - 1) / plan.k_tiles_per_slice);
+    };
+    if (g.swiglu_out != nullptr || g.swiglu_saved != nullptr || (!f32 && tiles_of(256) >= 3 * units && g.batch_rows == 0)) {
+        set_slices(1);
+        return plan;
     }
-    if (g.batch_rows != 0 && may_split && k_tiles >= 32) {
+    if (g.batch_rows != 0) {
         // A stack of products brings any number of tiles: the slice count that needs the least time, counted in
         // rounds of the persistent blocks times the length of a slice (fewer slices on a tie: fewer partial tiles).
+        long slices = 1;
         double best = 0.0;
-        for (int s = 1; s <= 8 && k_tiles / s >= 16; ++s) {
-            const long rounds = (tiles * s + want_blocks - 1) / want_blocks;
-            const double time = static_cast<double>(rounds) / s * (s > 1 ? 1.02 : 1.0);
+        for (long s = 1; s <= 8 && may_split && k_tiles >= 32 && k_tiles / s >= 16; ++s) {
+            const long rounds = (tiles_of(256) * s + units - 1) / units;
+            const double time = static_cast<double>(rounds) / static_cast<double>(s) * (s > 1 ? 1.02 : 1.0);
             if (s == 1 || time < best * 0.999) {
                 best = time;
                 slices = s;
             }
         }
+        set_slices(slices);
+        return plan;
     }
-    plan.slices = static_cast<int>(slices);
-    if (g.no_split && plan.partial_bytes(g) > g.split_workspace_bytes) slices = 1;
-    plan.k_tiles_per_slice = static_cast<int>((k_tiles + slices - 1) / slices);
-    plan.slices = static_cast<int>((k_tiles + plan.k_tiles_per_slice - 1) / plan.k_tiles_per_slice);
+    const int forced = forced_tile();
+    const double slice_bytes = static_cast<double>(g.m) * static_cast<double>(round_up(g.n, 8)) * sizeof(float);
+    // Calls that 256 x 256 tiles spread over most of the chip keep the order of additions of the kernels with a SwiGLU
+    // epilogue, which take such calls only (one sum over all of K): the fused and the separate operators give the same bits.
+    const bool whole_k = !f32 && tiles_of(256) * 5 >= units * 4;
+    double best = -1.0;
+    long best_slices = 1;
+    for (int tile : {32, 64, 128, 256}) {
+        if ((whole_k && tile < 128) || (forced != 0 && tile != forced && !(f32 && forced == 256)) || (f32 && tile == 256)) continue;
+        const long tiles = tiles_of(tile);
+        if (forced == 0 && tile <= 64 && tiles > 16 * units) continue;
+        for (long s : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            if (s > 1 && (whole_k || !may_split || k_tiles / s < 8 || tiles * s > 4 * units ||
+                          (g.no_split && slice_bytes * static_cast<double>(s) > static_cast<double>(g.split_workspace_bytes))))
+                break;
+            const double time = predicted_us(tile, tiles, s, k_tiles, slice_bytes * static_cast<double>(s) * 1e-6, f32,
+                                             g.a_k_contiguous, g.b_k_contiguous, units);
+            if (best < 0.0 || time < best) {
+                best = time;
+                plan.tile = tile;
+                best_slices = s;
+            }
+        }
+    }
+    set_slices(best_slices);
+    plan.deep = tiles_of(plan.tile) * plan.slices <= units;
     return plan;
 }
 
-template <typename T, int BM, int BN>
-int run_config(const GemmArgs& g, const Plan& plan, KernelArgs p, hipStream_t stream) {
-    p.tiles_m = (p.m + BM - 1) / BM;
-    p.tiles_n = (p.n + BN - 1) / BN;
+// Arguments of the small kernel (gemm_small_kernel.hpp) from the streamed ones.
+template <typename T>
+int launch_small_call(const GemmArgs& g, const KernelArgs& p, const Plan& plan, bool split, hipStream_t stream) {
+    SmallCall call{};
+    SmallArgs& a = call.args;
+    a.a = p.a;
+    a.b = p.b;
+    a.c = p.c;
+    a.lda = p.lda;
+    a.ldb = p.ldb;
+    a.ldc = split ? p.ld_partial : p.ldc;
+    a.m = p.m;
+    a.n = p.n;
+    a.k = p.k;
+    a.a_extent = p.a_extent;
+    a.b_extent = p.b_extent;
+    a.b_k = p.b_k;
+    a.k_tiles = p.k_tiles;
+    a.k_tiles_per_slice = plan.k_tiles_per_slice;
+    a.bias = p.bias;
+    a.residual = p.residual;
+    a.addend = p.addend;
+    a.ldr = p.ldr;
+    a.ld_addend = p.ld_addend;
+    a.accumulate = p.accumulate;
+    a.c_f32 = p.c_f32;
+    a.ragged = p.ragged;
+    auto copy = [](const KernelSegments& in, SmallSegments& out) {
+        for (int i = 0; i < 3; ++i) {
+            out.ptr[i] = in.ptr[i];
+            out.ld[i] = in.ld[i];
+            out.cols[i] = in.cols[i];
+        }
+        out.count = in.count;
+    };
+    copy(p.a_seg, a.a_seg);
+    copy(p.c_seg, a.c_seg);
+    call.a_k_contiguous = g.a_k_contiguous;
+    call.b_k_contiguous = g.b_k_contiguous;
+    call.tile = plan.tile;
+    call.deep = plan.deep;
+    call.slices = plan.slices;
+    const bool plain = p.bias == nullptr && p.residual == nullptr && p.addend == nullptr && !p.accumulate &&
+                       (!p.c_f32 || std::is_same_v<T, float>) && !p.ragged;
+    call.epilogue = split ? SmallEpilogue::split : plain ? SmallEpilogue::plain : SmallEpilogue::general;
+    if constexpr (std::is_same_v<T, bf16_t>) return gemm_small_bf16(call, stream);
+    else if constexpr (std::is_same_v<T, f16_t>) return gemm_small_f16(call, stream);
+    else return gemm_small_f32(call, stream);
+}
+
+template <typename T>
+int run_plan(const GemmArgs& g, const Plan& plan, KernelArgs p, hipStream_t stream) {
+    p.tiles_m = (p.m + plan.tile - 1) / plan.tile;
+    p.tiles_n = (p.n + plan.tile - 1) / plan.tile;
     p.k_tiles_per_slice = plan.k_tiles_per_slice;
-    if (plan.slices == 1) return launch_layout<T, BM, BN, false>(p, g.a_k_contiguous, g.b_k_contiguous, 1, stream);
+    auto launch = [&]<bool SPLIT>(const KernelArgs& args) -> int {
+        if (plan.tile <= 64) return launch_small_call<T>(g, args, plan, SPLIT, stream);
+        if constexpr (!std::is_same_v<T, float>) {
+            if (plan.tile == 256) return launch_layout<T, 256, 256, SPLIT>(args, g.a_k_contiguous, g.b_k_contiguous, plan.slices, stream);
+        }
+        return launch_layout<T, 128, 128, SPLIT>(args, g.a_k_contiguous, g.b_k_contiguous, plan.slices, stream);
+    };
+    if (plan.slices == 1) return launch.template operator()<false>(p);
     void* mem = g.no_split ? g.split_workspace : nullptr;
     if (mem == nullptr) {
         if (int s = scratch(stream, plan.partial_bytes(g), &mem)) return s;
@@ -1542,7 +1327,7 @@ int run_config(const GemmArgs& g, const Plan& plan, KernelArgs p, hipStream_t st
     KernelArgs split = p;
     split.c = mem;
     split.ld_partial = static_cast<long>(round_up(g.n, 8));
-    if (int s = launch_layout<T, BM, BN, true>(split, g.a_k_contiguous, g.b_k_contiguous, plan.slices, stream)) return s;
+    if (int s = launch.template operator()<true>(split)) return s;
     const long quads = static_cast<long>(p.m) * (split.ld_partial / 4);
     const long blocks = std::min<long>((quads + kThreads - 1) / kThreads, static_cast<long>(compute_units()) * 8);
     hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), 0, stream,
@@ -1704,12 +1489,7 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
         CGPTX_LAUNCH_CHECK();
         return CGPTX_OK;
     }
-    const Plan plan = make_plan(g);
-    if constexpr (!std::is_same_v<T, float>) {
-        if (plan.tile == 256) return run_config<T, 256, 256>(g, plan, p, stream);
-    }
-    if (plan.tile == 128) return run_config<T, 128, 128>(g, plan, p, stream);
-    return run_config<T, 64, 64>(g, plan, p, stream);
+    return run_plan<T>(g, make_plan(g), p, stream);
 }
 
 template <typename T>

@@ -1,0 +1,49 @@
+// Host interface of the small-contraction kernel (gemm_small_kernel.hpp), one translation unit per storage type.
+#pragma once
+
+#include "gemm.hpp"
+
+namespace cgptx {
+
+struct SmallSegments {
+    const void* ptr[3];
+    long ld[3];
+    int cols[3];
+    int count;
+};
+
+// Everything a plain call reads comes first: a workgroup's start waits for as few scalar loads as possible.
+struct SmallArgs {
+    const void* a;
+    const void* b;
+    void* c;  // T*, float* when c_f32, float partial tiles when split
+    long lda, ldb, ldc;  // ldc: row length of a partial tile matrix when split
+    int m, n, k;
+    int a_extent, b_extent, b_k;  // see GemmArgs
+    int k_tiles, k_tiles_per_slice;
+    // the general epilogue
+    const void* bias;
+    const void* residual;
+    const float* addend;
+    long ldr, ld_addend;
+    int accumulate, c_f32, ragged;
+    // segmented operands
+    SmallSegments a_seg, c_seg;
+};
+
+enum class SmallEpilogue { plain, general, split };
+
+struct SmallCall {
+    SmallArgs args;
+    bool a_k_contiguous, b_k_contiguous;
+    int tile;   // 32 or 64
+    bool deep;  // twice the LDS stages, one workgroup per CU instead of two
+    SmallEpilogue epilogue;
+    int slices;
+};
+
+int gemm_small_bf16(const SmallCall& call, hipStream_t stream);
+int gemm_small_f16(const SmallCall& call, hipStream_t stream);
+int gemm_small_f32(const SmallCall& call, hipStream_t stream);
+
+}  // namespace cgptx

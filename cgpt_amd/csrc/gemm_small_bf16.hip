@@ -1,0 +1,6 @@
+// Small contractions, bf16 storage.
+#include "gemm_small_kernel.hpp"
+
+namespace cgptx {
+int gemm_small_bf16(const SmallCall& call, hipStream_t stream) { return launch_small<bf16_t>(call, stream); }
+}  // namespace cgptx
