@@ -31,6 +31,7 @@
 // Two families implement this scheme: the register-staged kernels (templated on the padded head
 // dimension 32 / 64 / 128) and, further down, the LDS-direct kernels (padded width 128), which
 // serve every call whose operands fit 32-bit offsets.
+#include "attention_f32.hpp"
 #include "common.hpp"
 
 #include <cmath>
@@ -1354,8 +1355,8 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
 
 
 // ============================================================================================
-// Scalar family: fp32 storage, head dimensions that are not multiples of 8, and tensors that are not
-// 16-byte aligned — what the reference serves with its warp-per-row kernels
+// Scalar family: head dimensions that are not multiples of 8 (16-bit storage) or 4 (fp32), and tensors that are
+// not 16-byte aligned — what the reference serves with its warp-per-row kernels
 // (src/ops/backward/attention_backward.cu:352-504, dispatch 2044-2068). Correct, not fast: one
 // wavefront per output row, fp32 arithmetic throughout, lane l holding head-dim elements l and l + 64.
 // No atomics: dQ rows and (key, kv-head) rows each have one owner that adds its terms in a fixed order
@@ -1558,14 +1559,39 @@ bool aligned16_all(std::initializer_list<const void*> pointers) {
 }
 
 // The matrix-core kernels take 16-bit storage, head dimensions in multiples of 8 (128-bit row chunks) and
-// 16-byte aligned tensors; everything else the interface accepts runs on the scalar family.
+// 16-byte aligned tensors, fp32 has kernels of its own (attention_f32.hip); everything else the interface
+// accepts runs on the scalar family.
 bool scalar_path(const Shape& s, std::initializer_list<const void*> pointers) {
     return s.dtype == CGPTX_F32 || s.d % 8 != 0 || !aligned16_all(pointers);
 }
 
 unsigned int scalar_blocks(std::size_t rows) { return static_cast<unsigned int>((rows + kScalarWaves - 1) / kScalarWaves); }
 
+// The call as the fp32 kernels take it.
+AttentionF32Args f32_args(const Params& p) {
+    AttentionF32Args a{};
+    a.q = static_cast<const float*>(p.q);
+    a.k = static_cast<const float*>(p.k);
+    a.v = static_cast<const float*>(p.v);
+    a.batch = p.batch;
+    a.qs = p.qs;
+    a.ks = p.ks;
+    a.hq = p.hq;
+    a.hkv = p.hkv;
+    a.d = p.d;
+    a.scale = p.scale;
+    a.causal = p.causal;
+    a.offset = p.offset;
+    return a;
+}
+
 int launch_forward(const Shape& s, Params p, bool scalar, hipStream_t stream) {
+    if (s.dtype == CGPTX_F32 && attention_f32_takes(s.d, aligned16_all({p.out0, p.q, p.k, p.v}))) {
+        AttentionF32Args a = f32_args(p);
+        a.out = static_cast<float*>(p.out0);
+        a.lse_out = p.lse_out;
+        return attention_f32_forward(a, stream);
+    }
     if (scalar) {
         const std::size_t rows = s.batch * s.qs * s.hq;
         if (rows / kScalarWaves >= (std::size_t{1} << 31)) return fail(CGPTX_OVERFLOW, "attention: grid too large");
@@ -1604,6 +1630,18 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
     p.lse = lse;
     p.delta = delta;
     p.accumulate = accumulate;
+    if (s.dtype == CGPTX_F32 && attention_f32_takes(s.d, aligned16_all({p.q, p.k, p.v, dq, dk, dv, dout, out}))) {
+        AttentionF32Args a = f32_args(p);
+        a.dout = static_cast<const float*>(dout);
+        a.o = static_cast<const float*>(out);
+        a.lse = lse;
+        a.delta = delta;
+        a.dq = static_cast<float*>(dq);
+        a.dk = static_cast<float*>(dk);
+        a.dv = static_cast<float*>(dv);
+        a.accumulate = accumulate;
+        return attention_f32_backward(a, stream);
+    }
     if (scalar) {
         const std::size_t key_rows = s.batch * s.ks * s.hkv;
         if (rows / kScalarWaves >= (std::size_t{1} << 31) || key_rows / kScalarWaves >= (std::size_t{1} << 31))

@@ -264,6 +264,39 @@ def test_scalar_family_parity(device, case, with_lse):
         assert torch.equal(a, b_)   # no atomics: results do not depend on scheduling
 
 
+F32_CASES = [
+    dict(b=1, qs=17, ks=17, hq=2, hkv=1, d=4),                             # one tile and one row, the narrowest head
+    dict(b=2, qs=16, ks=16, hq=3, hkv=3, d=64),                            # one whole tile: most wavefronts have none
+    dict(b=1, qs=130, ks=130, hq=4, hkv=2, d=64),                          # nine tiles: wavefront 0 has two
+    dict(b=1, qs=300, ks=300, hq=8, hkv=2, d=128),                         # a group of four heads, ragged end
+    dict(b=1, qs=35, ks=200, hq=4, hkv=2, d=80, off=165),                  # offset queries, padded columns
+    dict(b=1, qs=40, ks=90, hq=2, hkv=1, d=100, off=20, scale=0.2),        # keys that no query sees
+    dict(b=2, qs=33, ks=257, hq=2, hkv=1, d=96, causal=False),
+]
+
+
+@pytest.mark.parametrize("case", range(len(F32_CASES)))
+@pytest.mark.parametrize("with_lse", [True, False])
+def test_fp32_matrix_core_parity(device, case, with_lse):
+    """The fp32 kernels against the float64 formulas, 1e-4 as for every fp32 operator (sums of up to 1200 terms of
+    relative error 2^-24 each stay below 1e-4), with and without accumulation, twice with the same bits."""
+    c = F32_CASES[case]
+    q, k, v, do = make_inputs(c, torch.float32, 300 + case)
+    out, lse = run_forward(device, q, k, v, c)
+    want_out, want_lse = oracle64.attention_forward(to_np(q), to_np(k), to_np(v), *oracle_args(c))
+    assert_close(out, want_out, 1e-4, "O")
+    assert_close(lse, want_lse, 1e-4, "LSE")
+    want = oracle64.attention_backward(to_np(do), to_np(q), to_np(k), to_np(v), *oracle_args(c))
+    got = run_backward(device, do, q, k, v, c, with_lse)
+    base = (randn(q.shape, torch.float32, 91), randn(k.shape, torch.float32, 92), randn(v.shape, torch.float32, 93))
+    added = run_backward(device, do, q, k, v, c, with_lse, accumulate=True, base=base)
+    for g, a, w, start, name in zip(got, added, want, base, ("dQ", "dK", "dV")):
+        assert_close(g, w, 1e-4, name)
+        assert_close(a, w + to_np(start), 1e-4, f"{name} accumulate")
+    for g, again in zip(got, run_backward(device, do, q, k, v, c, with_lse)):
+        assert torch.equal(g, again)
+
+
 def test_unaligned_tensors_take_the_scalar_family(device):
     """Views that start 2 bytes into an allocation are not 16-byte aligned: same results as the aligned call
     to storage precision (the two families round differently)."""
