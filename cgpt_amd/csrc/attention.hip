@@ -34,6 +34,7 @@
 #include "attention_f32.hpp"
 #include "common.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <limits>
@@ -84,6 +85,8 @@ struct Params {
     float scale;
     int causal, offset, accumulate;
     int paired;  // dK/dV, LDS-direct family: a workgroup takes key blocks (i, last - i) instead of one
+    int splits;  // dK/dV, LDS-direct family: workgroups that share a key block's query tiles (never with paired)
+    float* partial;  // splits > 1: [splits][dK | dV][key, kv head, d] sums of the parts
 };
 
 template <int DP>
@@ -1124,6 +1127,8 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
     }
 
     const int key_blocks = (p.ks + kBlockRows - 1) / kBlockRows;
+    const int part = p.splits > 1 ? pair_x % p.splits : 0;
+    if (p.splits > 1) pair_x /= p.splits;
     for (int half = 0; half < (p.paired ? 2 : 1); ++half) {
         const int block_index = half == 0 ? pair_x : key_blocks - 1 - pair_x;
         if (half == 1 && block_index <= pair_x) break;
@@ -1147,7 +1152,10 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
         // pairs form one flat sequence so that the next tile is prefetched across head boundaries.
         const int q_begin = p.causal ? max(0, k_block - p.offset) / kStream * kStream : 0;
         const int tiles_per_head = q_begin < p.qs ? (p.qs - q_begin + kStream - 1) / kStream : 0;
-        const int total_tiles = tiles_per_head * group;
+        const int all_tiles = tiles_per_head * group;
+        // A shared key block: this workgroup's part of the sequence.
+        const int first_index = p.splits > 1 ? part * all_tiles / p.splits : 0;
+        const int total_tiles = p.splits > 1 ? (part + 1) * all_tiles / p.splits : all_tiles;  // end of the part
         const int wave_first_key = k_block + wave * 32;
         const int wave_last_key = wave_first_key + 31;
 
@@ -1303,13 +1311,14 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
             __syncthreads();                     // ... and everybody else's; the other stage is free
         };
         {
-            const NextTile first_tile = next_tile(0);
+            const NextTile first_tile = next_tile(first_index);
 #pragma unroll
             for (int i = 0; i <= kLoads; ++i) request_part(first_tile, i);
         }
         for (int head = 0; head < group; ++head) {
             const int tile0 = head * tiles_per_head;
-            for (int t = 0; t < masked_per_head; ++t) {
+            const int begin = max(0, first_index - tile0), end = min(tiles_per_head, total_tiles - tile0);
+            for (int t = begin; t < min(masked_per_head, end); ++t) {
                 const int tile = tile0 + t, q0 = q_begin + t * kStream;
                 const T* q_tile = lds + (tile & 1) * 2 * kWideTile<W>;
                 arrive();
@@ -1317,7 +1326,7 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
                 tile_body.template operator()<true>(q_tile, q_tile + kWideTile<W>, stats + (tile & 1) * 2 * kStream,
                                                     k_live ? causal_first : (1 << 30), next_tile(tile + 1));
             }
-            for (int t = masked_per_head; t < tiles_per_head; ++t) {
+            for (int t = max(masked_per_head, begin); t < end; ++t) {
                 const int tile = tile0 + t;
                 const T* q_tile = lds + (tile & 1) * 2 * kWideTile<W>;
                 arrive();
@@ -1326,7 +1335,26 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
             }
         }
         __syncthreads();  // the next key block's first loads overwrite stage 0
-        if (k_live) {
+        if (k_live && p.splits > 1) {
+            const long count = static_cast<long>(p.batch) * p.ks * kv_stride;
+            float* dk_out = p.partial + 2 * part * count + k_offset;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int d0 = t * 32 + g * 8 + (lane >> 5) * 4;
+                    if (d0 >= p.d) continue;
+                    vec_t<float, 4> a, c;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        a[e] = dk[t][4 * g + e] * p.scale;
+                        c[e] = dv[t][4 * g + e];
+                    }
+                    store_vec<float, 4>(dk_out + d0, a);
+                    store_vec<float, 4>(dk_out + count + d0, c);
+                }
+            }
+        } else if (k_live) {
             T* dk_out = static_cast<T*>(p.out0) + k_offset;
             T* dv_out = static_cast<T*>(p.out1) + k_offset;
 #pragma unroll
@@ -1353,6 +1381,22 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
     }
 }
 
+// dK and dV from the parts of shared key blocks, added in the order of the parts; four elements per thread.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void attention_dkv_reduce_kernel(T* __restrict__ dk, T* __restrict__ dv,
+                                                                       const float* __restrict__ partial, long count,
+                                                                       int splits, int accumulate) {
+    const long quad = static_cast<long>(blockIdx.x) * kThreads + threadIdx.x;
+    if (quad >= count / 2) return;  // count elements of dK, then of dV
+    const bool second = quad >= count / 4;
+    const long at = (second ? quad - count / 4 : quad) * 4;
+    const float* source = partial + (second ? count : 0) + at;
+    vec_t<float, 4> sum = load_vec<float, 4>(source);
+    for (int s = 1; s < splits; ++s) sum += load_vec<float, 4>(source + 2 * s * count);
+    T* out = (second ? dv : dk) + at;
+    if (accumulate) sum += vec_to_f32<T, 4>(load_vec<T, 4>(out));
+    store_vec<T, 4>(out, vec_from_f32<T, 4>(sum));
+}
 
 // ============================================================================================
 // Scalar family: head dimensions that are not multiples of 8 (16-bit storage) or 4 (fp32), and tensors that are
@@ -1567,6 +1611,46 @@ bool scalar_path(const Shape& s, std::initializer_list<const void*> pointers) {
 
 unsigned int scalar_blocks(std::size_t rows) { return static_cast<unsigned int>((rows + kScalarWaves - 1) / kScalarWaves); }
 
+// Workgroups that share a key block in the dK/dV pass. The kernel holds 128 keys of one kv head per workgroup and one
+// workgroup per CU, so short batches leave most of the chip idle while the busiest workgroup walks all heads of its group
+// over all query tiles, about 1.75 us per tile (0.9 with heads of 64). Dividing that walk costs a launch and the fp32
+// partial sums' way to memory and back: the division with the shortest predicted time is taken. Causal key blocks differ in
+// length; the parts of the first one are the longest. One sequence of 512, 32:8 heads of 128, not causal: 58 -> 28 us,
+// reduction included; 5 sequences of 1001, 8:2 heads, causal: 110 -> 61 us.
+int dkv_splits(const Shape& s) {
+    if (!wide_path(s)) return 1;
+    const long units = compute_units(), group = static_cast<long>(s.hq / s.hkv);
+    const long key_blocks = static_cast<long>((s.ks + kBlockRows - 1) / kBlockRows), pairs = static_cast<long>(s.hkv * s.batch);
+    long longest = 0, total = 0;
+    for (long i = 0; i < key_blocks; ++i) {
+        const long begin = s.causal ? std::max<long>(0, i * kBlockRows - static_cast<long>(s.offset)) / kStream * kStream : 0;
+        const long tiles = begin < static_cast<long>(s.qs) ? (static_cast<long>(s.qs) - begin + kStream - 1) / kStream * group : 0;
+        longest = std::max(longest, tiles);
+        total += tiles * pairs;
+        if (total > 16 * units * std::max<long>(longest, 1)) return 1;  // a full chip many times over
+    }
+    const double tile_us = s.d <= 64 ? 0.9 : 1.75;
+    const double megabytes = static_cast<double>(s.batch * s.ks * s.hkv * s.d) * 8e-6;
+    int best = 1;
+    double best_us = 0.0;
+    for (int parts = 1; parts <= 16 && parts <= std::max<long>(longest, 1); ++parts) {
+        const double busiest = std::max<double>(std::ceil(static_cast<double>(longest) / parts), static_cast<double>(total) / static_cast<double>(units));
+        const double us = busiest * tile_us + (parts > 1 ? 5.0 + 0.4 * megabytes * parts : 0.0);
+        if (parts == 1 || us < best_us) {
+            best = parts;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+// Scratch of the backward pass: [delta | LSE·log2 e | partial sums of shared key blocks].
+std::size_t backward_scratch_bytes(const Shape& s, bool scalar) {
+    const std::size_t stats = 2 * stat_block_bytes(s.batch * s.qs * s.hq);
+    const int splits = scalar ? 1 : dkv_splits(s);
+    return stats + (splits > 1 ? (static_cast<std::size_t>(splits) * 2 * s.batch * s.ks * s.hkv * s.d * sizeof(float) + 255) & ~std::size_t{255} : 0);
+}
+
 // The call as the fp32 kernels take it.
 AttentionF32Args f32_args(const Params& p) {
     AttentionF32Args a{};
@@ -1623,7 +1707,7 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
     const std::size_t rows = s.batch * s.qs * s.hq;
     const std::size_t stat_bytes = stat_block_bytes(rows);
     void* mem = nullptr;
-    if (int st = scratch(stream, 2 * stat_bytes, &mem)) return st;  // [delta | LSE·log2 e]
+    if (int st = scratch(stream, backward_scratch_bytes(s, scalar), &mem)) return st;
     auto* delta = static_cast<float*>(mem);
     auto* lse2 = reinterpret_cast<float*>(static_cast<char*>(mem) + stat_bytes);
     p.dout = dout;
@@ -1700,9 +1784,11 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
                 // grid that leaves compute units idle is better off with twice the workgroups (the longest single
                 // block is shorter than the pair that contains it).
                 const std::size_t single_blocks = static_cast<std::size_t>(key_blocks) * s.hkv * s.batch;
-                pk.paired = s.causal && single_blocks > static_cast<std::size_t>(compute_units());
-                const dim3 pair_grid(pk.paired ? (key_blocks + 1) / 2 : key_blocks, static_cast<unsigned int>(s.hkv),
-                                     static_cast<unsigned int>(s.batch));
+                pk.splits = dkv_splits(s);
+                pk.partial = reinterpret_cast<float*>(static_cast<char*>(mem) + 2 * stat_bytes);
+                pk.paired = pk.splits == 1 && s.causal && single_blocks > static_cast<std::size_t>(compute_units());
+                const dim3 pair_grid(pk.paired ? (key_blocks + 1) / 2 : key_blocks * static_cast<unsigned int>(pk.splits),
+                                     static_cast<unsigned int>(s.hkv), static_cast<unsigned int>(s.batch));
                 auto launch = [&]<int W>() -> int {
                     auto kernel = attention_dkv_wide_kernel<T, W>;
                     static bool configured = false;
@@ -1715,6 +1801,13 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
                     return CGPTX_OK;
                 };
                 if (int st = s.d <= 64 ? launch.template operator()<64>() : launch.template operator()<128>()) return st;
+                if (pk.splits > 1) {
+                    CGPTX_LAUNCH_CHECK();
+                    const long count = static_cast<long>(s.batch * s.ks * s.hkv * s.d);
+                    hipLaunchKernelGGL((attention_dkv_reduce_kernel<T>), dim3(static_cast<unsigned int>((count / 2 + kThreads - 1) / kThreads)),
+                                       dim3(kThreads), 0, stream, static_cast<T*>(dk), static_cast<T*>(dv), pk.partial, count,
+                                       pk.splits, accumulate);
+                }
             } else {
                 const dim3 k_grid(key_blocks, static_cast<unsigned int>(s.hkv), static_cast<unsigned int>(s.batch));
                 hipLaunchKernelGGL((attention_dkv_kernel<T, DP>), k_grid, dim3(kThreads), 0, stream, pk);
@@ -1790,15 +1883,16 @@ extern "C" int cgptx_flash_gqa_attention_backward(void* grad_query, void* grad_k
     const bool scalar = scalar_path(s, {grad_query, grad_key, grad_value, grad_output, query, key, value});
     auto stream = static_cast<hipStream_t>(stream_);
     // Recompute the output and the log-sum-exp into scratch, then run the LSE path. The scratch
-    // block is laid out [delta | LSE·log2 e | lse | output] so that launch_backward's request for
-    // the two-block prefix returns the same base pointer.
+    // block is laid out [what launch_backward asks for | lse | output], so that its request for the
+    // prefix returns the same base pointer.
     const std::size_t rows = batch * query_sequence * query_heads;
     const std::size_t stat_bytes = stat_block_bytes(rows);
     const std::size_t out_bytes = rows * head_dim * dtype_size(dtype);
     void* mem = nullptr;
-    if (int st = scratch(stream, 3 * stat_bytes + out_bytes, &mem)) return st;
-    auto* lse = reinterpret_cast<float*>(static_cast<char*>(mem) + 2 * stat_bytes);
-    void* out = static_cast<char*>(mem) + 3 * stat_bytes;
+    const std::size_t prefix = backward_scratch_bytes(s, scalar);
+    if (int st = scratch(stream, prefix + stat_bytes + out_bytes, &mem)) return st;
+    auto* lse = reinterpret_cast<float*>(static_cast<char*>(mem) + prefix);
+    void* out = static_cast<char*>(mem) + prefix + stat_bytes;
     Params p = make_params(s);
     p.q = query;
     p.k = key;
