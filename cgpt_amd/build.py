@@ -96,6 +96,32 @@ def build(force: bool = True, jobs: int | None = None) -> pathlib.Path:
     return LIB_PATH
 
 
+DISPATCH_SOURCE = ROOT / "cgpt_amd" / "host" / "dispatch.cpp"
+DISPATCH_PATH = ROOT / "cgpt_amd" / "_dispatch.so"
+
+
+def build_dispatch(force: bool = True) -> pathlib.Path:
+    """Compiles the Python extension behind cgpt_amd/ops.py (host code only: tensor checks against torch's C++ API)."""
+    deps = [DISPATCH_SOURCE, ROOT / "include" / "cgptx.h"]
+    if not force and DISPATCH_PATH.exists() and all(DISPATCH_PATH.stat().st_mtime >= d.stat().st_mtime for d in deps):
+        return DISPATCH_PATH
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], str(ROOT / "include")]
+    libraries = cpp_extension.library_paths()
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{path}" for path in includes), str(DISPATCH_SOURCE), "-o", str(DISPATCH_PATH),
+           *(f"-L{path}" for path in libraries), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           *(f"-Wl,-rpath,{path}" for path in libraries)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"dispatch extension build failed:\n{proc.stderr}")
+    return DISPATCH_PATH
+
+
 INTERFACE_TEST_SOURCES = [ROOT / "tests" / "cpp" / name
                           for name in ("ops_interface_test.cpp", "block_backward_test.cpp", "data_upload_test.cpp")]
 INTERFACE_TEST_BINARY = ROOT / "tests" / "cpp" / "ops_interface_test.bin"
@@ -117,4 +143,5 @@ def build_interface_test() -> pathlib.Path:
 if __name__ == "__main__":
     path = build(force="--incremental" not in sys.argv)
     print(path)
+    print(build_dispatch(force="--incremental" not in sys.argv))
     print(build_interface_test())

@@ -164,5 +164,18 @@ def check(status: int) -> None:
     raise CgptxRuntimeError(message)
 
 
+class _Functions(dict):
+    """Entry points by name, looked up in the library once."""
+
+    def __missing__(self, name):
+        function = self[name] = getattr(lib(), name)
+        return function
+
+
+_functions = _Functions()
+
+
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    status = _functions[name](*args)
+    if status:
+        check(status)

@@ -29,16 +29,20 @@ def _code(t: torch.Tensor) -> int:
         raise ValueError(f"unsupported dtype {t.dtype}") from None
 
 
-def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
 
 
-def _stream(stream) -> ctypes.c_void_p:
+# The current stream's handle without making a Stream object of it (2.5 us a call, about what a launch takes).
+_current_device, _current_raw_stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+
+
+def _stream(stream) -> int:
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return _current_raw_stream(_current_device())
     if isinstance(stream, torch.cuda.Stream):
-        return ctypes.c_void_p(stream.cuda_stream)
-    return ctypes.c_void_p(int(stream))
+        return stream.cuda_stream
+    return int(stream)
 
 
 def _require_device(name: str, *tensors: torch.Tensor) -> None:
@@ -53,6 +57,39 @@ def _same_dtype(name: str, *tensors: torch.Tensor) -> None:
     for t in tensors:
         if t.dtype != tensors[0].dtype or t.dtype not in _DTYPE:
             raise ValueError(f"{name}: all tensors must have the same floating dtype")
+
+
+def _load_dispatch():
+    """The native tensor checks (host/dispatch.cpp): tensors(*tensors) gives (dtype code, pointers) of contiguous device
+    tensors of one dtype, or None."""
+    try:
+        from . import _dispatch
+    except ImportError as error:
+        raise ImportError("cgpt_amd/_dispatch.so is missing or does not load: build it with `python -m cgpt_amd.build`") from error
+    globals().update(_tensors=_dispatch.tensors, _same_shape=_dispatch.same_shape, _adamw_entries=_dispatch.adamw_entries)
+
+
+def _tensors(*tensors):  # replaced by the native function on first use
+    _load_dispatch()
+    return _tensors(*tensors)
+
+
+def _same_shape(*tensors):
+    _load_dispatch()
+    return _same_shape(*tensors)
+
+
+def _adamw_entries(*args):
+    _load_dispatch()
+    return _adamw_entries(*args)
+
+
+def _reject(name: str, *tensors):
+    """Says what is wrong with tensors that the native check does not take."""
+    present = [t for t in tensors if t is not None]
+    _require_device(name, *present)
+    _same_dtype(name, *present)
+    return (_code(present[0]), *(_ptr(t) for t in tensors))
 
 
 def _ids(name: str, ids: torch.Tensor, count: int) -> None:
@@ -124,15 +161,14 @@ def rmsnorm_backward(grad_input, grad_weight, grad_output, input, weight, epsilo
     name = "rmsnorm_backward"
     if not (math.isfinite(epsilon) and epsilon > 0):
         raise ValueError(f"{name}: epsilon must be finite and positive")
-    _require_device(name, grad_input, grad_weight, grad_output, input, weight)
-    _same_dtype(name, input, grad_input, grad_weight, grad_output, weight)
-    if input.dim() != 2 or grad_output.shape != input.shape or grad_input.shape != input.shape:
+    code, dx, dw, dy, x, w = _tensors(grad_input, grad_weight, grad_output, input, weight) or \
+        _reject(name, grad_input, grad_weight, grad_output, input, weight)
+    if input.dim() != 2 or not _same_shape(input, grad_output, grad_input):
         raise ValueError(f"{name}: input, grad_output and grad_input must have shape [rows, hidden]")
-    if weight.dim() != 1 or grad_weight.dim() != 1 or weight.shape[0] != input.shape[1] or \
-            grad_weight.shape[0] != input.shape[1]:
+    rows, hidden = input.shape
+    if weight.dim() != 1 or grad_weight.dim() != 1 or weight.shape[0] != hidden or grad_weight.shape[0] != hidden:
         raise ValueError(f"{name}: weight and grad_weight must have shape [hidden]")
-    capi.call("cgptx_rmsnorm_backward", _ptr(grad_input), _ptr(grad_weight), _ptr(grad_output), _ptr(input),
-              _ptr(weight), input.shape[0], input.shape[1], epsilon, _code(input), _stream(stream))
+    capi.call("cgptx_rmsnorm_backward", dx, dw, dy, x, w, rows, hidden, epsilon, code, _stream(stream))
 
 
 def _rope_check(name, q, k, cos_cache, sin_cache, options):
@@ -152,87 +188,80 @@ def rope_backward(grad_query, grad_key, grad_rotated_query, grad_rotated_key, co
                   rope_options: RopeOptions = RopeOptions()):
     """include/ops/backward/rope_backward.h:22-31."""
     name = "rope_backward"
-    _require_device(name, grad_query, grad_key, grad_rotated_query, grad_rotated_key, cos_cache, sin_cache)
-    _same_dtype(name, grad_query, grad_key, grad_rotated_query, grad_rotated_key, cos_cache, sin_cache)
-    if grad_query.shape != grad_rotated_query.shape or grad_key.shape != grad_rotated_key.shape:
+    code, gq, gk, rq, rk, cos, sin = \
+        _tensors(grad_query, grad_key, grad_rotated_query, grad_rotated_key, cos_cache, sin_cache) or \
+        _reject(name, grad_query, grad_key, grad_rotated_query, grad_rotated_key, cos_cache, sin_cache)
+    if not (_same_shape(grad_query, grad_rotated_query) and _same_shape(grad_key, grad_rotated_key)):
         raise ValueError(f"{name}: incompatible Q/K gradient shapes")
     _rope_check(name, grad_query, grad_key, cos_cache, sin_cache, rope_options)
     b, s, hq, d = grad_query.shape
-    capi.call("cgptx_rope_backward", _ptr(grad_query), _ptr(grad_key), _ptr(grad_rotated_query),
-              _ptr(grad_rotated_key), _ptr(cos_cache), _ptr(sin_cache), b, s, hq, grad_key.shape[2], d,
-              rope_options.rotary_dim, rope_options.position_offset, cos_cache.shape[0], _code(grad_query),
-              _stream(stream))
+    capi.call("cgptx_rope_backward", gq, gk, rq, rk, cos, sin, b, s, hq, grad_key.shape[2], d, rope_options.rotary_dim,
+              rope_options.position_offset, cos_cache.shape[0], code, _stream(stream))
 
 
 def swiglu_backward(grad_gate, grad_up, grad_output, gate, up, stream=None,
                     options: SwiGLUBackwardOptions = SwiGLUBackwardOptions()):
     """include/ops/backward/swiglu_backward.h:30-38."""
     name = "swiglu_backward"
-    _require_device(name, grad_gate, grad_up, grad_output, gate, up)
-    _same_dtype(name, grad_output, grad_gate, grad_up, gate, up)
-    for t in (grad_gate, grad_up, gate, up):
-        if t.shape != grad_output.shape:
-            raise ValueError(f"{name}: all tensors must have the same shape")
-    capi.call("cgptx_swiglu_backward", _ptr(grad_gate), _ptr(grad_up), _ptr(grad_output), _ptr(gate), _ptr(up),
-              grad_output.numel(), int(options.accumulate_gate), int(options.accumulate_up), _code(gate),
-              _stream(stream))
+    code, dg, du, dy, g, u = _tensors(grad_gate, grad_up, grad_output, gate, up) or \
+        _reject(name, grad_gate, grad_up, grad_output, gate, up)
+    if not _same_shape(grad_output, grad_gate, grad_up, gate, up):
+        raise ValueError(f"{name}: all tensors must have the same shape")
+    capi.call("cgptx_swiglu_backward", dg, du, dy, g, u, grad_output.numel(), int(options.accumulate_gate),
+              int(options.accumulate_up), code, _stream(stream))
 
 
 def swiglu_backward_packed(grad_gate_up, grad_output, gate_up, stream=None,
                            options: SwiGLUBackwardOptions = SwiGLUBackwardOptions()):
     """Packed [.., 2*hidden] = [gate | up] overload (src/ops/backward/swiglu_backward.cu:830-883)."""
     name = "swiglu_backward"
-    _require_device(name, grad_gate_up, grad_output, gate_up)
-    _same_dtype(name, grad_output, grad_gate_up, gate_up)
+    code, dgu, dy, gu = _tensors(grad_gate_up, grad_output, gate_up) or _reject(name, grad_gate_up, grad_output, gate_up)
     hidden = grad_output.shape[-1]
     if gate_up.dim() < 1 or gate_up.shape[-1] != 2 * hidden or gate_up.numel() != 2 * grad_output.numel() or \
-            grad_gate_up.shape != gate_up.shape:
+            not _same_shape(grad_gate_up, gate_up):
         raise ValueError(f"{name}: invalid fused tensors")
     if grad_output.numel() == 0:
         return  # nothing to do (src/ops/backward/swiglu_backward.cu:839-841)
-    capi.call("cgptx_swiglu_backward_packed", _ptr(grad_gate_up), _ptr(grad_output), _ptr(gate_up),
-              grad_output.numel() // hidden, hidden, int(options.accumulate_gate_up), _code(gate_up), _stream(stream))
+    capi.call("cgptx_swiglu_backward_packed", dgu, dy, gu, grad_output.numel() // hidden, hidden,
+              int(options.accumulate_gate_up), code, _stream(stream))
 
 
 def linear_backward(grad_input, grad_weight, grad_bias, grad_output, input, weight, gemm_context=None, stream=None,
                     options: LinearBackwardOptions = LinearBackwardOptions()):
     """include/ops/backward/linear_backward.h:36-46 (gemm_context stands where the cuBLASLt context is)."""
     name = "linear_backward"
-    present = [t for t in (grad_input, grad_weight, grad_bias) if t is not None]
-    _require_device(name, grad_output, input, weight, *present)
-    _same_dtype(name, input, grad_output, weight, *present)
-    if input.dim() < 1 or weight.dim() != 2 or grad_output.dim() != input.dim() or \
-            input.shape[-1] != weight.shape[1] or grad_output.shape[-1] != weight.shape[0] or \
-            tuple(grad_output.shape[:-1]) != tuple(input.shape[:-1]):
+    code, dx, dw, db, dy, x, w = _tensors(grad_input, grad_weight, grad_bias, grad_output, input, weight) or \
+        _reject(name, grad_input, grad_weight, grad_bias, grad_output, input, weight)
+    x_shape, w_shape, dy_shape = input.shape, weight.shape, grad_output.shape
+    if len(x_shape) < 1 or len(w_shape) != 2 or len(dy_shape) != len(x_shape) or x_shape[-1] != w_shape[1] or \
+            dy_shape[-1] != w_shape[0] or dy_shape[:-1] != x_shape[:-1]:
         raise ValueError(f"{name}: incompatible tensors")
-    if grad_input is not None and grad_input.shape != input.shape:
+    if grad_input is not None and not _same_shape(grad_input, input):
         raise ValueError(f"{name}: grad_input must match input")
-    if grad_weight is not None and grad_weight.shape != weight.shape:
+    if grad_weight is not None and not _same_shape(grad_weight, weight):
         raise ValueError(f"{name}: grad_weight must match weight")
-    if grad_bias is not None and (grad_bias.dim() != 1 or grad_bias.shape[0] != weight.shape[0]):
+    if grad_bias is not None and (grad_bias.dim() != 1 or grad_bias.shape[0] != w_shape[0]):
         raise ValueError(f"{name}: grad_bias must have shape [out_features]")
-    out_features, in_features = weight.shape
-    capi.call("cgptx_linear_backward", _ptr(grad_input), _ptr(grad_weight), _ptr(grad_bias), _ptr(grad_output),
-              _ptr(input), _ptr(weight), input.numel() // in_features, in_features, out_features,
-              int(options.accumulate_input), int(options.accumulate_weight), int(options.accumulate_bias),
-              _code(input), _stream(stream))
+    out_features, in_features = w_shape
+    capi.call("cgptx_linear_backward", dx, dw, db, dy, x, w, input.numel() // in_features, in_features, out_features,
+              int(options.accumulate_input), int(options.accumulate_weight), int(options.accumulate_bias), code,
+              _stream(stream))
 
 
 def embedding_backward(grad_weight, grad_output, device_token_ids, token_count, stream=None,
                        options: EmbeddingBackwardOptions = EmbeddingBackwardOptions()):
     """include/ops/backward/embedding_backward.h:35-42."""
     name = "embedding_backward"
-    _require_device(name, grad_weight, grad_output)
-    _same_dtype(name, grad_weight, grad_output)
+    code, dw, dy = _tensors(grad_weight, grad_output) or _reject(name, grad_weight, grad_output)
     if token_count == 0:
         raise ValueError(f"{name}: token_count must be positive")
     _ids(name, device_token_ids, token_count)
     if grad_weight.dim() != 2 or grad_output.dim() < 1 or grad_output.shape[-1] != grad_weight.shape[1] or \
             grad_output.numel() != token_count * grad_weight.shape[1]:
         raise ValueError(f"{name}: incompatible tensors or token count")
-    capi.call("cgptx_embedding_backward", _ptr(grad_weight), _ptr(grad_output), _ptr(device_token_ids), token_count,
-              grad_weight.shape[0], grad_weight.shape[1], int(options.bounds_check), int(options.accumulate_weight),
-              _code(grad_weight), _stream(stream))
+    vocab, hidden = grad_weight.shape
+    capi.call("cgptx_embedding_backward", dw, dy, device_token_ids.data_ptr(), token_count, vocab, hidden,
+              int(options.bounds_check), int(options.accumulate_weight), code, _stream(stream))
 
 
 def _ce_check(name, loss, logits, targets, target_count):
@@ -247,23 +276,22 @@ def cross_entropy_forward_backward(loss, gradient, logits, device_targets, targe
                                    gradient_scale: float = 1.0):
     """include/ops/cross_entropy.h:25-32."""
     name = "cross_entropy_forward_backward"
-    _require_device(name, gradient, logits)
-    _same_dtype(name, logits, gradient)
+    code, g, z = _tensors(gradient, logits) or _reject(name, gradient, logits)
     _ce_check(name, loss, logits, device_targets, target_count)
-    if gradient.shape != logits.shape or not (math.isfinite(gradient_scale) and gradient_scale > 0):
+    if not _same_shape(gradient, logits) or not (math.isfinite(gradient_scale) and gradient_scale > 0):
         raise ValueError(f"{name}: invalid gradient tensor or scale")
-    capi.call("cgptx_cross_entropy_forward_backward", _ptr(loss), _ptr(gradient), _ptr(logits),
-              _ptr(device_targets), logits.shape[0], logits.shape[1], gradient_scale, _code(logits), _stream(stream))
+    rows, vocab = logits.shape
+    capi.call("cgptx_cross_entropy_forward_backward", loss.data_ptr(), g, z, device_targets.data_ptr(), rows, vocab,
+              gradient_scale, code, _stream(stream))
 
 
 def cross_entropy_forward(loss, logits, device_targets, target_count, stream=None):
     """include/ops/cross_entropy.h:37-42."""
     name = "cross_entropy_forward"
-    _require_device(name, logits)
-    _same_dtype(name, logits)
+    code, z = _tensors(logits) or _reject(name, logits)
     _ce_check(name, loss, logits, device_targets, target_count)
-    capi.call("cgptx_cross_entropy_forward", _ptr(loss), _ptr(logits), _ptr(device_targets), logits.shape[0],
-              logits.shape[1], _code(logits), _stream(stream))
+    rows, vocab = logits.shape
+    capi.call("cgptx_cross_entropy_forward", loss.data_ptr(), z, device_targets.data_ptr(), rows, vocab, code, _stream(stream))
 
 
 def cut_cross_entropy_forward_backward(loss, input_gradient, classifier_gradient, input, classifier, device_targets,
@@ -271,32 +299,32 @@ def cut_cross_entropy_forward_backward(loss, input_gradient, classifier_gradient
                                        accumulate_classifier: bool = False):
     """include/ops/cut_cross_entropy.h:25-33; gradient_scale and accumulate_classifier are extensions."""
     name = "cut_cross_entropy_forward_backward"
-    _require_device(name, input_gradient, classifier_gradient, input, classifier)
-    _same_dtype(name, input, input_gradient, classifier_gradient, classifier)
+    code, dx, dc, x, c = _tensors(input_gradient, classifier_gradient, input, classifier) or \
+        _reject(name, input_gradient, classifier_gradient, input, classifier)
     if input.dim() != 2 or classifier.dim() != 2 or input.shape[1] != classifier.shape[1] or \
-            input.shape[0] != target_count or target_count == 0 or input_gradient.shape != input.shape or \
-            classifier_gradient.shape != classifier.shape:
+            input.shape[0] != target_count or target_count == 0 or not _same_shape(input_gradient, input) or \
+            not _same_shape(classifier_gradient, classifier):
         raise ValueError(f"{name}: incompatible tensors")
     if loss.dtype != torch.float32 or loss.numel() != 1 or loss.device.type != "cuda":
         raise ValueError(f"{name}: loss must be a device F32 tensor with shape [1]")
     _ids(name, device_targets, target_count)
-    capi.call("cgptx_cut_cross_entropy_forward_backward", _ptr(loss), _ptr(input_gradient),
-              _ptr(classifier_gradient), _ptr(input), _ptr(classifier), _ptr(device_targets), input.shape[0],
-              input.shape[1], classifier.shape[0], gradient_scale, int(accumulate_classifier), _code(input),
-              _stream(stream))
+    rows, hidden = input.shape
+    capi.call("cgptx_cut_cross_entropy_forward_backward", loss.data_ptr(), dx, dc, x, c, device_targets.data_ptr(), rows,
+              hidden, classifier.shape[0], gradient_scale, int(accumulate_classifier), code, _stream(stream))
 
 
-def _attention_check(name, q, k, v, options: FlashAttentionOptions, others=()):
-    _same_dtype(name, q, k, v, *others)
-    if q.dim() != 4 or k.dim() != 4 or v.shape != k.shape or not options.num_query_heads or \
-            not options.num_kv_heads or not options.head_dim or options.num_query_heads % options.num_kv_heads or \
-            q.shape[0] != k.shape[0] or q.shape[2] != options.num_query_heads or \
-            k.shape[2] != options.num_kv_heads or q.shape[3] != options.head_dim or \
-            k.shape[3] != options.head_dim or not math.isfinite(options.attention_scale):
+def _attention_check(name, q, k, v, options: FlashAttentionOptions):
+    """Sizes of the call: (batch, query sequence, key sequence, query heads, kv heads, head_dim)."""
+    q_shape, k_shape = q.shape, k.shape
+    hq, hkv, d = options.num_query_heads, options.num_kv_heads, options.head_dim
+    if len(q_shape) != 4 or len(k_shape) != 4 or not _same_shape(v, k) or not hq or not hkv or not d or hq % hkv or \
+            q_shape[0] != k_shape[0] or q_shape[2] != hq or k_shape[2] != hkv or q_shape[3] != d or k_shape[3] != d or \
+            not math.isfinite(options.attention_scale):
         raise ValueError(f"{name}: invalid tensors or options")
-    if options.causal and (options.query_position_offset > k.shape[1] or
-                           q.shape[1] > k.shape[1] - options.query_position_offset):
+    if options.causal and (options.query_position_offset > k_shape[1] or
+                           q_shape[1] > k_shape[1] - options.query_position_offset):
         raise ValueError(f"{name}: causal range exceeds the key sequence")
+    return q_shape[0], q_shape[1], k_shape[1], hq, hkv, d
 
 
 def flash_gqa_attention_backward_with_lse(grad_query, grad_key, grad_value, grad_output, output, logsumexp, query,
@@ -305,18 +333,18 @@ def flash_gqa_attention_backward_with_lse(grad_query, grad_key, grad_value, grad
                                           accumulate_grads: bool = False):
     """include/ops/backward/attention_backward.h:57-70."""
     name = "flash_gqa_attention_backward_with_lse"
-    _require_device(name, grad_query, grad_key, grad_value, grad_output, output, logsumexp, query, key, value)
-    _attention_check(name, query, key, value, options, (grad_query, grad_key, grad_value, grad_output, output))
-    if grad_output.shape != query.shape or grad_query.shape != query.shape or grad_key.shape != key.shape or \
-            grad_value.shape != key.shape or output.shape != query.shape:
+    code, dq, dk, dv, do, o, q, k, v = \
+        _tensors(grad_query, grad_key, grad_value, grad_output, output, query, key, value) or \
+        _reject(name, grad_query, grad_key, grad_value, grad_output, output, query, key, value)
+    _require_device(name, logsumexp)
+    sizes = _attention_check(name, query, key, value, options)
+    if not _same_shape(query, grad_output, grad_query, output) or not _same_shape(key, grad_key, grad_value):
         raise ValueError(f"{name}: gradient shapes must match their tensors")
-    if logsumexp.dtype != torch.float32 or tuple(logsumexp.shape) != tuple(query.shape[:3]):
+    if logsumexp.dtype != torch.float32 or logsumexp.shape != query.shape[:3]:
         raise ValueError(f"{name}: invalid output or logsumexp")
-    capi.call("cgptx_flash_gqa_attention_backward_with_lse", _ptr(grad_query), _ptr(grad_key), _ptr(grad_value),
-              _ptr(grad_output), _ptr(output), _ptr(logsumexp), _ptr(query), _ptr(key), _ptr(value), query.shape[0],
-              query.shape[1], key.shape[1], options.num_query_heads, options.num_kv_heads, options.head_dim,
-              options.attention_scale, int(options.causal), options.query_position_offset, int(accumulate_grads),
-              _code(query), _stream(stream))
+    capi.call("cgptx_flash_gqa_attention_backward_with_lse", dq, dk, dv, do, o, logsumexp.data_ptr(), q, k, v, *sizes,
+              options.attention_scale, int(options.causal), options.query_position_offset, int(accumulate_grads), code,
+              _stream(stream))
 
 
 def flash_gqa_attention_backward(grad_query, grad_key, grad_value, grad_output, query, key, value, stream=None,
@@ -324,16 +352,13 @@ def flash_gqa_attention_backward(grad_query, grad_key, grad_value, grad_output, 
                                  accumulate_grads: bool = False):
     """include/ops/backward/attention_backward.h:24-35."""
     name = "flash_gqa_attention_backward"
-    _require_device(name, grad_query, grad_key, grad_value, grad_output, query, key, value)
-    _attention_check(name, query, key, value, options, (grad_query, grad_key, grad_value, grad_output))
-    if grad_output.shape != query.shape or grad_query.shape != query.shape or grad_key.shape != key.shape or \
-            grad_value.shape != key.shape:
+    code, dq, dk, dv, do, q, k, v = _tensors(grad_query, grad_key, grad_value, grad_output, query, key, value) or \
+        _reject(name, grad_query, grad_key, grad_value, grad_output, query, key, value)
+    sizes = _attention_check(name, query, key, value, options)
+    if not _same_shape(query, grad_output, grad_query) or not _same_shape(key, grad_key, grad_value):
         raise ValueError(f"{name}: gradient shapes must match their tensors")
-    capi.call("cgptx_flash_gqa_attention_backward", _ptr(grad_query), _ptr(grad_key), _ptr(grad_value),
-              _ptr(grad_output), _ptr(query), _ptr(key), _ptr(value), query.shape[0], query.shape[1], key.shape[1],
-              options.num_query_heads, options.num_kv_heads, options.head_dim, options.attention_scale,
-              int(options.causal), options.query_position_offset, int(accumulate_grads), _code(query),
-              _stream(stream))
+    capi.call("cgptx_flash_gqa_attention_backward", dq, dk, dv, do, q, k, v, *sizes, options.attention_scale,
+              int(options.causal), options.query_position_offset, int(accumulate_grads), code, _stream(stream))
 
 
 # ------------------------------------------------------------------------------ AdamW
@@ -387,7 +412,7 @@ class AdamWWorkspace:
         capi.call("cgptx_adamw_workspace_create", ctypes.byref(handle))
         self._handle = handle
         self._states = None
-        self._c_entries = None
+        self._array = None  # the entries as the library takes them, filled anew by each call
 
     def __del__(self):
         try:
@@ -417,16 +442,19 @@ def adamw_step_many_async(entries: Sequence[AdamWBatchEntry], options: AdamWOpti
         for e, s in zip(entries, workspace._states):
             if e.state is not s:
                 raise ValueError(f"{name}: workspace states changed")
-    array = (capi.AdamWEntry * len(entries))()
-    for i, e in enumerate(entries):
-        if e.parameter is None or e.gradient is None or e.state is None:
-            raise ValueError(f"{name}: null entry")
-        _validate_adamw_tensors(e.parameter, e.gradient, e.state, name)
-        if e.parameter.device.type != "cuda":
-            raise ValueError(f"{name}: device tensors required")
-        array[i] = capi.AdamWEntry(e.parameter.data_ptr(), e.gradient.data_ptr(), e.state.master_parameter.data_ptr(),
-                                   e.state.first_moment.data_ptr(), e.state.second_moment.data_ptr(),
-                                   e.parameter.numel(), _code(e.parameter))
+    array = workspace._array
+    if array is None or len(array) != len(entries):
+        array = workspace._array = (capi.AdamWEntry * len(entries))()
+    if not isinstance(entries, list) or not _adamw_entries(entries, workspace._states, ctypes.addressof(array)):
+        for i, e in enumerate(entries):  # another kind of sequence, or something to complain about
+            if e.parameter is None or e.gradient is None or e.state is None:
+                raise ValueError(f"{name}: null entry")
+            _validate_adamw_tensors(e.parameter, e.gradient, e.state, name)
+            if e.parameter.device.type != "cuda":
+                raise ValueError(f"{name}: device tensors required")
+            array[i] = capi.AdamWEntry(e.parameter.data_ptr(), e.gradient.data_ptr(), e.state.master_parameter.data_ptr(),
+                                       e.state.first_moment.data_ptr(), e.state.second_moment.data_ptr(),
+                                       e.parameter.numel(), _code(e.parameter))
     c_options = options.to_c()
     capi.call("cgptx_adamw_step_many_async", workspace._handle, array, len(entries), ctypes.byref(c_options),
               initial_step, _stream(stream))
@@ -469,24 +497,21 @@ def rmsnorm_forward(output, input, weight, epsilon, stream=None):
     name = "rmsnorm_forward"
     if not (math.isfinite(epsilon) and epsilon > 0):
         raise ValueError(f"{name}: epsilon must be finite and positive")
-    _require_device(name, output, input, weight)
-    _same_dtype(name, input, output, weight)
-    if input.dim() != 2 or output.shape != input.shape or weight.dim() != 1 or weight.shape[0] != input.shape[1]:
+    code, y, x, w = _tensors(output, input, weight) or _reject(name, output, input, weight)
+    if input.dim() != 2 or not _same_shape(output, input) or weight.dim() != 1 or weight.shape[0] != input.shape[1]:
         raise ValueError(f"{name}: incompatible shapes")
-    capi.call("cgptx_rmsnorm_forward", _ptr(output), _ptr(input), _ptr(weight), input.shape[0], input.shape[1],
-              epsilon, _code(input), _stream(stream))
+    rows, hidden = input.shape
+    capi.call("cgptx_rmsnorm_forward", y, x, w, rows, hidden, epsilon, code, _stream(stream))
 
 
 def rope_forward(query, key, cos_cache, sin_cache, stream=None, rope_options: RopeOptions = RopeOptions()):
     """include/ops/rope.h:32-39 (in place)."""
     name = "rope_forward"
-    _require_device(name, query, key, cos_cache, sin_cache)
-    _same_dtype(name, query, key, cos_cache, sin_cache)
+    code, q, k, cos, sin = _tensors(query, key, cos_cache, sin_cache) or _reject(name, query, key, cos_cache, sin_cache)
     _rope_check(name, query, key, cos_cache, sin_cache, rope_options)
     b, s, hq, d = query.shape
-    capi.call("cgptx_rope_forward", _ptr(query), _ptr(key), _ptr(cos_cache), _ptr(sin_cache), b, s, hq, key.shape[2],
-              d, rope_options.rotary_dim, rope_options.position_offset, cos_cache.shape[0], _code(query),
-              _stream(stream))
+    capi.call("cgptx_rope_forward", q, k, cos, sin, b, s, hq, key.shape[2], d, rope_options.rotary_dim,
+              rope_options.position_offset, cos_cache.shape[0], code, _stream(stream))
 
 
 def swiglu_forward(output, gate, up=None, stream=None):
@@ -495,8 +520,7 @@ def swiglu_forward(output, gate, up=None, stream=None):
     name = "swiglu_forward"
     if up is None:
         gate_up = gate
-        _require_device(name, output, gate_up)
-        _same_dtype(name, gate_up, output)
+        code, y, gu = _tensors(output, gate_up) or _reject(name, output, gate_up)
         if gate_up.dim() == 0 or gate_up.shape[-1] % 2 != 0:
             raise ValueError(f"{name}: the last gate_up dimension must be even")
         hidden = gate_up.shape[-1] // 2
@@ -505,28 +529,24 @@ def swiglu_forward(output, gate, up=None, stream=None):
             raise ValueError(f"{name}: output shape must match gate_up except for its last dimension")
         if output.numel() == 0:
             return  # nothing to do (src/ops/swiglu.cu:581-583)
-        capi.call("cgptx_swiglu_forward_packed", _ptr(output), _ptr(gate_up), output.numel() // hidden, hidden,
-                  _code(gate_up), _stream(stream))
+        capi.call("cgptx_swiglu_forward_packed", y, gu, output.numel() // hidden, hidden, code, _stream(stream))
         return
-    _require_device(name, output, gate, up)
-    _same_dtype(name, gate, output, up)
-    if output.shape != gate.shape or up.shape != gate.shape:
+    code, y, g, u = _tensors(output, gate, up) or _reject(name, output, gate, up)
+    if not _same_shape(gate, output, up):
         raise ValueError(f"{name}: all tensors must have the same shape")
-    capi.call("cgptx_swiglu_forward", _ptr(output), _ptr(gate), _ptr(up), gate.numel(), _code(gate), _stream(stream))
+    capi.call("cgptx_swiglu_forward", y, g, u, gate.numel(), code, _stream(stream))
 
 
 def linear_forward(output, input, weight, gemm_context=None, stream=None, bias=None):
     """include/ops/linear.h."""
     name = "linear_forward"
-    present = [bias] if bias is not None else []
-    _require_device(name, output, input, weight, *present)
-    _same_dtype(name, input, output, weight, *present)
-    if weight.dim() != 2 or input.shape[-1] != weight.shape[1] or output.shape[-1] != weight.shape[0] or \
-            tuple(output.shape[:-1]) != tuple(input.shape[:-1]):
+    code, y, x, w, b = _tensors(output, input, weight, bias) or _reject(name, output, input, weight, bias)
+    x_shape, w_shape, y_shape = input.shape, weight.shape, output.shape
+    if len(w_shape) != 2 or x_shape[-1] != w_shape[1] or y_shape[-1] != w_shape[0] or y_shape[:-1] != x_shape[:-1]:
         raise ValueError(f"{name}: incompatible tensors")
-    out_features, in_features = weight.shape
-    capi.call("cgptx_linear_forward", _ptr(output), _ptr(input), _ptr(weight), _ptr(bias),
-              input.numel() // in_features, in_features, out_features, _code(input), _stream(stream))
+    out_features, in_features = w_shape
+    capi.call("cgptx_linear_forward", y, x, w, b, input.numel() // in_features, in_features, out_features, code,
+              _stream(stream))
 
 
 def linear_swiglu_forward(gate_up, activated, input, weight, gemm_context=None, stream=None):
@@ -587,31 +607,28 @@ def linear_backward_weights_stacked(grad_weight, grad_output, input, stream=None
 def embedding_forward(output, device_token_ids, token_count, weight, stream=None):
     """include/ops/embedding.h."""
     name = "embedding_forward"
-    _require_device(name, output, weight)
-    _same_dtype(name, weight, output)
+    code, y, w = _tensors(output, weight) or _reject(name, output, weight)
     _ids(name, device_token_ids, token_count)
     if weight.dim() != 2 or output.numel() != token_count * weight.shape[1]:
         raise ValueError(f"{name}: incompatible tensors or token count")
-    capi.call("cgptx_embedding_forward", _ptr(output), _ptr(device_token_ids), token_count, _ptr(weight),
-              weight.shape[0], weight.shape[1], _code(weight), _stream(stream))
+    vocab, hidden = weight.shape
+    capi.call("cgptx_embedding_forward", y, device_token_ids.data_ptr(), token_count, w, vocab, hidden, code, _stream(stream))
 
 
 def flash_gqa_attention_forward_with_lse(output, logsumexp, query, key, value, stream=None,
                                          options: FlashAttentionOptions = FlashAttentionOptions()):
     """include/ops/attention.h:70-78."""
     name = "flash_gqa_attention_forward_with_lse"
-    tensors = [output, query, key, value] + ([logsumexp] if logsumexp is not None else [])
-    _require_device(name, *tensors)
-    _attention_check(name, query, key, value, options, (output,))
-    if output.shape != query.shape:
+    code, o, q, k, v = _tensors(output, query, key, value) or _reject(name, output, query, key, value)
+    if logsumexp is not None:
+        _require_device(name, logsumexp)
+    sizes = _attention_check(name, query, key, value, options)
+    if not _same_shape(output, query):
         raise ValueError(f"{name}: output must match query")
-    if logsumexp is not None and (logsumexp.dtype != torch.float32 or
-                                  tuple(logsumexp.shape) != tuple(query.shape[:3])):
+    if logsumexp is not None and (logsumexp.dtype != torch.float32 or logsumexp.shape != query.shape[:3]):
         raise ValueError(f"{name}: invalid logsumexp tensor")
-    capi.call("cgptx_flash_gqa_attention_forward", _ptr(output), _ptr(logsumexp), _ptr(query), _ptr(key), _ptr(value),
-              query.shape[0], query.shape[1], key.shape[1], options.num_query_heads, options.num_kv_heads,
-              options.head_dim, options.attention_scale, int(options.causal), options.query_position_offset,
-              _code(query), _stream(stream))
+    capi.call("cgptx_flash_gqa_attention_forward", o, _ptr(logsumexp), q, k, v, *sizes, options.attention_scale,
+              int(options.causal), options.query_position_offset, code, _stream(stream))
 
 
 def flash_gqa_attention_forward(output, query, key, value, stream=None,
@@ -623,8 +640,7 @@ def flash_gqa_attention_forward(output, query, key, value, stream=None,
 def add_tensors(output, a, b, stream=None):
     """src/core/transformer_block.cu:242-248."""
     name = "add"
-    _require_device(name, output, a, b)
-    _same_dtype(name, a, output, b)
-    if output.shape != a.shape or b.shape != a.shape:
+    code, y, x1, x2 = _tensors(output, a, b) or _reject(name, output, a, b)
+    if not _same_shape(a, output, b):
         raise ValueError(f"{name}: shape mismatch")
-    capi.call("cgptx_add", _ptr(output), _ptr(a), _ptr(b), a.numel(), _code(a), _stream(stream))
+    capi.call("cgptx_add", y, x1, x2, a.numel(), code, _stream(stream))
