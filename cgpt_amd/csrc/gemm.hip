@@ -1230,9 +1230,10 @@ Plan make_plan(const GemmArgs& g) {
     }
     const int forced = forced_tile();
     const double slice_bytes = static_cast<double>(g.m) * static_cast<double>(round_up(g.n, 8)) * sizeof(float);
-    // Calls that 256 x 256 tiles spread over most of the chip keep the order of additions of the kernels with a SwiGLU
-    // epilogue, which take such calls only (one sum over all of K): the fused and the separate operators give the same bits.
-    const bool whole_k = !f32 && tiles_of(256) * 5 >= units * 4;
+    // Calls that 256 x 256 tiles spread over three quarters of the chip keep the order of additions of the kernels with a
+    // SwiGLU epilogue, which take such calls only (one sum over all of K): the fused and the separate operators give the same
+    // bits. A split would fill the last quarter, less the partial tiles' way: 16384 x 768 x 32000 688 us, in four slices 650.
+    const bool whole_k = !f32 && tiles_of(256) * 4 >= units * 3;
     double best = -1.0;
     long best_slices = 1;
     for (int tile : {32, 64, 128, 256}) {
