@@ -1617,19 +1617,26 @@ unsigned int scalar_blocks(std::size_t rows) { return static_cast<unsigned int>(
 // partial sums' way to memory and back: the division with the shortest predicted time is taken. Causal key blocks differ in
 // length; the parts of the first one are the longest. One sequence of 512, 32:8 heads of 128, not causal: 58 -> 28 us,
 // reduction included; 5 sequences of 1001, 8:2 heads, causal: 110 -> 61 us.
+// The fp32 kernel holds 16 keys per workgroup and walks 16 queries per wavefront and step of 8 us, with the same trade (one
+// sequence of 256, 8:2 heads of 128, causal: 66 -> 16 us, reduction 4).
 int dkv_splits(const Shape& s) {
-    if (!wide_path(s)) return 1;
+    const bool f32 = s.dtype == CGPTX_F32;
+    if (!f32 && !wide_path(s)) return 1;
+    const std::size_t block_rows = f32 ? 16 : kBlockRows, stream_rows = f32 ? 16 : kStream;
+    const long waves = f32 ? 8 : 1;  // that walk tiles of their own
     const long units = compute_units(), group = static_cast<long>(s.hq / s.hkv);
-    const long key_blocks = static_cast<long>((s.ks + kBlockRows - 1) / kBlockRows), pairs = static_cast<long>(s.hkv * s.batch);
+    const long key_blocks = static_cast<long>((s.ks + block_rows - 1) / block_rows), pairs = static_cast<long>(s.hkv * s.batch);
     long longest = 0, total = 0;
     for (long i = 0; i < key_blocks; ++i) {
-        const long begin = s.causal ? std::max<long>(0, i * kBlockRows - static_cast<long>(s.offset)) / kStream * kStream : 0;
-        const long tiles = begin < static_cast<long>(s.qs) ? (static_cast<long>(s.qs) - begin + kStream - 1) / kStream * group : 0;
+        const long rows = static_cast<long>(stream_rows), skipped = i * static_cast<long>(block_rows) - static_cast<long>(s.offset);
+        const long begin = s.causal ? std::max<long>(0, skipped) / rows * rows : 0;
+        const long walked = begin < static_cast<long>(s.qs) ? (static_cast<long>(s.qs) - begin + rows - 1) / rows * group : 0;
+        const long tiles = (walked + waves - 1) / waves;
         longest = std::max(longest, tiles);
         total += tiles * pairs;
         if (total > 16 * units * std::max<long>(longest, 1)) return 1;  // a full chip many times over
     }
-    const double tile_us = s.d <= 64 ? 0.9 : 1.75;
+    const double tile_us = f32 ? 8.0 : s.d <= 64 ? 0.9 : 1.75;
     const double megabytes = static_cast<double>(s.batch * s.ks * s.hkv * s.d) * 8e-6;
     int best = 1;
     double best_us = 0.0;
@@ -1644,10 +1651,19 @@ int dkv_splits(const Shape& s) {
     return best;
 }
 
+template <typename T>
+int launch_dkv_reduce(const Shape& s, void* dk, void* dv, const float* partial, int splits, int accumulate, hipStream_t stream) {
+    const long count = static_cast<long>(s.batch * s.ks * s.hkv * s.d);
+    hipLaunchKernelGGL((attention_dkv_reduce_kernel<T>), dim3(static_cast<unsigned int>((count / 2 + kThreads - 1) / kThreads)),
+                       dim3(kThreads), 0, stream, static_cast<T*>(dk), static_cast<T*>(dv), partial, count, splits, accumulate);
+    CGPTX_LAUNCH_CHECK();
+    return CGPTX_OK;
+}
+
 // Scratch of the backward pass: [delta | LSE·log2 e | partial sums of shared key blocks].
 std::size_t backward_scratch_bytes(const Shape& s, bool scalar) {
     const std::size_t stats = 2 * stat_block_bytes(s.batch * s.qs * s.hq);
-    const int splits = scalar ? 1 : dkv_splits(s);
+    const int splits = scalar && s.dtype != CGPTX_F32 ? 1 : dkv_splits(s);
     return stats + (splits > 1 ? (static_cast<std::size_t>(splits) * 2 * s.batch * s.ks * s.hkv * s.d * sizeof(float) + 255) & ~std::size_t{255} : 0);
 }
 
@@ -1724,7 +1740,10 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
         a.dk = static_cast<float*>(dk);
         a.dv = static_cast<float*>(dv);
         a.accumulate = accumulate;
-        return attention_f32_backward(a, stream);
+        a.parts = dkv_splits(s);
+        a.partial = reinterpret_cast<float*>(static_cast<char*>(mem) + 2 * stat_bytes);
+        if (int st = attention_f32_backward(a, stream)) return st;
+        return a.parts > 1 ? launch_dkv_reduce<float>(s, dk, dv, a.partial, a.parts, accumulate, stream) : CGPTX_OK;
     }
     if (scalar) {
         const std::size_t key_rows = s.batch * s.ks * s.hkv;
@@ -1803,10 +1822,7 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
                 if (int st = s.d <= 64 ? launch.template operator()<64>() : launch.template operator()<128>()) return st;
                 if (pk.splits > 1) {
                     CGPTX_LAUNCH_CHECK();
-                    const long count = static_cast<long>(s.batch * s.ks * s.hkv * s.d);
-                    hipLaunchKernelGGL((attention_dkv_reduce_kernel<T>), dim3(static_cast<unsigned int>((count / 2 + kThreads - 1) / kThreads)),
-                                       dim3(kThreads), 0, stream, static_cast<T*>(dk), static_cast<T*>(dv), pk.partial, count,
-                                       pk.splits, accumulate);
+                    if (int st = launch_dkv_reduce<T>(s, dk, dv, pk.partial, pk.splits, accumulate, stream)) return st;
                 }
             } else {
                 const dim3 k_grid(key_blocks, static_cast<unsigned int>(s.hkv), static_cast<unsigned int>(s.batch));

@@ -11,8 +11,9 @@
 // output row (the scalar family of attention.hip) was latency, and the matrix rate is a sixteenth of the 16-bit one. So
 // one workgroup of eight wavefronts owns 16 stationary rows only, and the wavefronts split the streamed tiles between
 // them (tile t to wavefront t mod 8); their partial results meet in LDS at the end, in wavefront order: no atomics,
-// results independent of scheduling. One sequence of 256 tokens, 8:2 heads of 128, causal: forward 151 -> 14 us, dQ
-// 239 -> 21, dK/dV 295 -> 66.
+// results independent of scheduling. Few key tiles are shared by several workgroups in the dK/dV pass (the caller decides
+// and adds their sums up). One sequence of 256 tokens, 8:2 heads of 128, causal: forward 151 -> 14 us, dQ
+// 239 -> 21, dK/dV 295 -> 20.
 #include "attention_f32.hpp"
 
 #include <cmath>
@@ -261,7 +262,8 @@ template <int D>
 __global__ __launch_bounds__(kThreads) void attention_f32_dkv_kernel(AttentionF32Args p) {
     extern __shared__ __align__(16) float lds[];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, g = lane >> 4;
-    const int k0 = blockIdx.x * kTile, kvh = blockIdx.y, b = blockIdx.z, group = p.hq / p.hkv;  // the first keys have most queries
+    const int part = blockIdx.x % p.parts, k0 = blockIdx.x / p.parts * kTile;  // the first keys have most queries
+    const int kvh = blockIdx.y, b = blockIdx.z, group = p.hq / p.hkv;
     const int key = k0 + (lane & 15);
     const long q_stride = static_cast<long>(p.hq) * p.d, kv_stride = static_cast<long>(p.hkv) * p.d;
     const long kv_row = (static_cast<long>(b) * p.ks + key) * kv_stride + static_cast<long>(kvh) * p.d;
@@ -277,7 +279,8 @@ __global__ __launch_bounds__(kThreads) void attention_f32_dkv_kernel(AttentionF3
     for (int c = 0; c < D / 64; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) dk[c][e] = dv[c][e] = acc_t(0.0f);
-    for (int i = wave; i < tiles * group; i += kWaves) {  // (head of the group, query tile)
+    const int end = (part + 1) * (tiles * group) / p.parts;
+    for (int i = part * (tiles * group) / p.parts + wave; i < end; i += kWaves) {  // (head of the group, query tile)
         const int head = i / tiles, t = first_tile + i - head * tiles, h = kvh * group + head;
         const float* q_base = p.q + static_cast<long>(b) * p.qs * q_stride + static_cast<long>(h) * p.d;
         const float* do_base = p.dout + static_cast<long>(b) * p.qs * q_stride + static_cast<long>(h) * p.d;
@@ -305,21 +308,24 @@ __global__ __launch_bounds__(kThreads) void attention_f32_dkv_kernel(AttentionF3
         columns.load(q_base, q_stride, t * kTile, p.qs, p.d);
         accumulate<D>(dk, columns, ds);
     }
+    const long count = static_cast<long>(p.batch) * p.ks * kv_stride;
+    float* const dk_out = p.parts == 1 ? p.dk : p.partial + 2 * part * count;
+    float* const dv_out = p.parts == 1 ? p.dv : p.partial + (2 * part + 1) * count;
     auto store_to = [&](float* out) {
         return [&, out](int row, int at, f32x4 sum) {
             if (k0 + row >= p.ks) return;
             float* to = out + (static_cast<long>(b) * p.ks + k0 + row) * kv_stride + static_cast<long>(kvh) * p.d + at;
-            if (p.accumulate) sum += load_vec<float, 4>(to);
+            if (p.accumulate && p.parts == 1) sum += load_vec<float, 4>(to);
             store_vec<float, 4>(to, sum);
         };
     };
     deposit<D>(lds, wave, dk, p.scale);
     __syncthreads();
-    collect<D>(lds, p.d, store_to(p.dk));
+    collect<D>(lds, p.d, store_to(dk_out));
     __syncthreads();
     deposit<D>(lds, wave, dv, 1.0f);
     __syncthreads();
-    collect<D>(lds, p.d, store_to(p.dv));
+    collect<D>(lds, p.d, store_to(dv_out));
 }
 
 template <auto Kernel, int SMEM>
@@ -348,7 +354,9 @@ int attention_f32_forward(const AttentionF32Args& a, hipStream_t stream) {
 }
 
 int attention_f32_backward(const AttentionF32Args& a, hipStream_t stream) {
-    const dim3 q_grid = grid_over(a.qs, a.hq, a.batch), k_grid = grid_over(a.ks, a.hkv, a.batch);
+    const dim3 q_grid = grid_over(a.qs, a.hq, a.batch);
+    dim3 k_grid = grid_over(a.ks, a.hkv, a.batch);
+    k_grid.x *= static_cast<unsigned int>(a.parts);
     if (int s = a.d <= 64 ? launch<attention_f32_dq_kernel<64>, kSmemBytes<64>>(q_grid, a, stream)
                           : launch<attention_f32_dq_kernel<128>, kSmemBytes<128>>(q_grid, a, stream))
         return s;

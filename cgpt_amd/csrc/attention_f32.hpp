@@ -15,6 +15,8 @@ struct AttentionF32Args {
     int batch, qs, ks, hq, hkv, d;
     float scale;
     int causal, offset, accumulate;
+    int parts;       // dK/dV: workgroups that share a key tile; more than one leave their sums in `partial`,
+    float* partial;  // [part][dK | dV][key, kv head, d], for the caller to add up
 };
 
 // Whether these kernels take the call: head dimensions in multiples of 4 and 16-byte aligned tensors.
