@@ -1240,7 +1240,7 @@ Plan make_plan(const GemmArgs& g) {
         if ((whole_k && tile < 128) || (forced != 0 && tile != forced && !(f32 && forced == 256)) || (f32 && tile == 256)) continue;
         const long tiles = tiles_of(tile);
         if (forced == 0 && tile <= 64 && tiles > 16 * units) continue;
-        for (long s : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        for (long s = 1; s <= 16; ++s) {
             if (s > 1 && (whole_k || !may_split || k_tiles / s < 8 || tiles * s > 4 * units ||
                           (g.no_split && slice_bytes * static_cast<double>(s) > static_cast<double>(g.split_workspace_bytes))))
                 break;
