@@ -1,0 +1,95 @@
+"""GPU tests at the sizes where one kernel, tile, split or unrolling gives way to the next: the first and last sizes of each
+range, with the oracle of the operator's own tests."""
+import pytest
+import torch
+
+from cgpt_amd import ops
+from oracle import cpu_ops, oracle64
+from tests.test_gpu_attention import make_inputs, oracle_args, run_backward, run_forward
+from tests.util import DTYPE_IDS, DTYPES, STOL, TOL, assert_close, assert_scaled_close, randint, randn, to_np
+
+pytestmark = pytest.mark.gpu
+
+ATTENTION = [
+    dict(b=1, qs=64, ks=64, hq=2, hkv=1, d=128),                        # one key tile: blocks of 128 rows
+    dict(b=1, qs=65, ks=65, hq=4, hkv=2, d=128),                        # two key tiles of 64 rows, one row in the second block
+    dict(b=1, qs=1, ks=129, hq=2, hkv=1, d=64, off=128),                # one query, three key tiles: parts of two and one
+    dict(b=2, qs=63, ks=192, hq=2, hkv=2, d=96, causal=False),          # odd number of key tiles, padded columns
+    dict(b=1, qs=130, ks=300, hq=2, hkv=1, d=40, off=20, scale=0.2),    # keys that no query sees, 64-wide heads
+    dict(b=32, qs=64, ks=65, hq=8, hkv=8, d=128, causal=False),         # 256 blocks of 64 rows: the last call in two parts
+    dict(b=33, qs=64, ks=65, hq=8, hkv=8, d=128, causal=False),         # 264: the first one in blocks of 128
+    dict(b=64, qs=40, ks=65, hq=8, hkv=2, d=64, causal=False),          # 512 with 64-wide heads
+    dict(b=65, qs=40, ks=65, hq=8, hkv=2, d=64, causal=False),
+    dict(b=1, qs=390, ks=390, hq=6, hkv=2, d=128),                      # few key blocks: shared between workgroups, ragged end
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", range(len(ATTENTION)))
+def test_attention_around_the_choice_of_blocks(device, case, dtype):
+    """Bounds as in the operator's parity tests; every result twice with the same bits, gradients added to what is there."""
+    c = ATTENTION[case]
+    q, k, v, do = make_inputs(c, dtype, 700 + 10 * case)
+    out, lse = run_forward(device, q, k, v, c)
+    want_out, want_lse = oracle64.attention_forward(to_np(q), to_np(k), to_np(v), *oracle_args(c))
+    assert_close(out, want_out, TOL[dtype], "O")
+    assert_close(lse, want_lse, 1e-3, "LSE")
+    want = oracle64.attention_backward(to_np(do), to_np(q), to_np(k), to_np(v), *oracle_args(c))
+    got = run_backward(device, do, q, k, v, c)
+    base = (randn(q.shape, dtype, 91), randn(k.shape, dtype, 92), randn(v.shape, dtype, 93))
+    added = run_backward(device, do, q, k, v, c, accumulate=True, base=base)
+    for g, a, w, start, name in zip(got, added, want, base, ("dQ", "dK", "dV")):
+        assert_scaled_close(g, w, STOL[dtype], name)
+        assert_scaled_close(a, w + to_np(start), STOL[dtype], f"{name} accumulate")
+    for g, again in zip(got, run_backward(device, do, q, k, v, c)):
+        assert torch.equal(g, again)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("rows,fin,fout", [
+    (1, 4096, 64), (33, 4096, 40), (64, 5024, 96),        # few tiles, long K: 32- and 64-wide tiles in K slices
+    (3000, 64, 40), (4999, 136, 72),                      # the same for the weight gradient, K ends inside a K tile
+    (257, 2048, 264), (512, 1536, 1536),                  # tiles of 64 and 128 in slices, ragged edges
+])
+def test_contractions_in_k_slices_are_exact_on_integers(device, rows, fin, fout, dtype):
+    """Small integers: every product and partial sum is exact in fp32 (at most 4 x 5024 < 2^24), so the result is the rounded
+    exact value whatever the tile and the slices."""
+    g = torch.Generator().manual_seed(rows + fin + fout)
+    x, w, dy = (torch.randint(-2, 3, shape, generator=g).double() for shape in ((rows, fin), (fout, fin), (rows, fout)))
+    on = lambda t: t.to(dtype).to(device)
+    y, gi, gw = (torch.full(shape, float("nan"), dtype=dtype, device=device) for shape in ((rows, fout), (rows, fin), (fout, fin)))
+    ops.linear_forward(y, on(x), on(w))
+    ops.linear_backward(gi, gw, None, on(dy), on(x), on(w))
+    for name, got, exact in zip(("Y", "dX", "dW"), (y, gi, gw), (x @ w.T, dy @ w, dy.T @ x)):
+        assert torch.equal(got.cpu(), exact.to(dtype)), name
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("vectors", [1024, 1025, 4096, 4097, 8192, 8193, 16384, 16385])
+@pytest.mark.parametrize("tail", [0, 1])
+def test_cross_entropy_around_the_held_row_lengths(device, vectors, tail, dtype):
+    """Rows of exactly as many 16-byte vectors as a kernel holds and of one more, with and without a tail element."""
+    rows, vocab = 3, vectors * (16 // torch.empty(0, dtype=dtype).element_size()) + tail
+    logits, targets = randn((rows, vocab), dtype, vectors, 3.0), randint(vocab, (rows,), vectors + 1)
+    targets[0] = vocab - 1
+    loss, grad = torch.zeros(1, device=device), torch.empty((rows, vocab), dtype=dtype, device=device)
+    # A scale of the order of the vocabulary, so that the bound sees the softmax and not only the target's column.
+    ops.cross_entropy_forward_backward(loss, grad, logits.to(device), targets.to(device), rows, None, 4096.0)
+    want_loss, want = oracle64.cross_entropy(to_np(logits), targets.numpy(), 4096.0)
+    assert abs(loss.item() - want_loss) <= 1e-4 * max(1.0, abs(want_loss))
+    assert_close(grad, want, TOL[dtype], "gradient")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("more", [-1, 0, 1])
+def test_swiglu_backward_around_the_choice_of_unrolling(device, more, dtype):
+    """One vector per thread below two tiles of 1024 vectors per compute unit, four from there on."""
+    units = torch.cuda.get_device_properties(device).multi_processor_count
+    count = (units * 2 * 1024 + more) * (16 // torch.empty(0, dtype=dtype).element_size())
+    g, u, dy = randn((count,), dtype, 8, 2.0), randn((count,), dtype, 9), randn((count,), dtype, 10)
+    want_g, want_u = torch.empty_like(g), torch.empty_like(u)
+    cpu_ops.swiglu_backward(want_g, want_u, dy, g, u)
+    got_g, got_u = torch.empty_like(g, device=device), torch.empty_like(u, device=device)
+    ops.swiglu_backward(got_g, got_u, dy.to(device), g.to(device), u.to(device))
+    assert_close(got_g, want_g, TOL[dtype], "dgate")
+    assert_close(got_u, want_u, TOL[dtype], "dup")
