@@ -13,6 +13,7 @@
 #include "common.hpp"
 
 #include <cstring>
+#include <algorithm>
 #include <limits>
 
 namespace cgptx {
@@ -120,16 +121,18 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
 //   * Segments of up to kShort tokens: one wavefront per id, tokens ordered in registers (lane i holds the token
 //     of rank i), lanes across the columns, kAhead token rows in flight.
 //   * Longer ones: one workgroup per id and kSlice columns, so that a frequent id occupies hidden / kSlice
-//     workgroups instead of one wavefront. The segment is put into ascending order window by window through a
-//     bitmap of token positions in LDS; all threads fetch the slices of the next kBatch token rows while the first
-//     wavefront adds the previous ones, one column per lane, from LDS. The chain is then bound by the latency of
-//     add + round, about 20 cycles per token.
+//     workgroups instead of one wavefront. The segment is put into ascending order through a bitmap of token
+//     positions in LDS, kSpan positions at a time as long as the list of its tokens has room for the whole segment;
+//     all threads fetch the slices of the next kBatch token rows while the first wavefront adds the previous
+//     ones, one column per lane, from LDS, where it reads 16 tokens ahead of the chain. That is bound by the latency
+//     of add + round.
 // Both live in one launch, the long segments' workgroups first. 32768 tokens x 1024 columns, ids Zipf distributed
-// over 32000: 1846 -> 66 us (of which the most frequent id, 6.7 per cent of the tokens, sets the end).
+// over 32000: 1846 -> 51 us (of which the most frequent id, 6.7 per cent of the tokens, sets the end).
 constexpr unsigned int kShort = 64;      // tokens: one lane each
 constexpr unsigned int kSlice = 64;      // columns of a long segment's workgroup: one lane each, one or two cache lines
 constexpr unsigned int kBatch = 128;     // token rows per step of a long segment
-constexpr unsigned int kWindow = 4096;   // token positions covered by the bitmap at a time
+constexpr unsigned int kSpan = 65536;    // token positions covered by the bitmap at a time
+constexpr unsigned int kList = 4096;     // tokens of the ordered list; longer segments take kList positions at a time
 
 template <typename T, bool Vector>
 __device__ __forceinline__ void embedding_short_row(T* __restrict__ row, const T* __restrict__ grad_output,
@@ -172,6 +175,15 @@ __device__ __forceinline__ void embedding_short_row(T* __restrict__ row, const T
     }
 }
 
+// acc + x rounded to T and widened again. bf16: rounding into the upper half of a register whose lower half is zero is the
+// widened value already, one instruction less in the chain.
+template <typename T>
+__device__ __forceinline__ float add_rounded(float acc, T x) {
+    if constexpr (std::is_same_v<T, bf16_t>)
+        return __builtin_bit_cast(float, __builtin_convertvector(vec_t<float, 2>{0.0f, acc + to_f32(x)}, vec_t<bf16_t, 2>));
+    else return round_to<T>(acc + to_f32(x));
+}
+
 template <typename T, bool Vector>
 struct LongRow {
     static constexpr unsigned int kVec = Vector ? kVec128<T> : 1;
@@ -179,8 +191,8 @@ struct LongRow {
     static constexpr unsigned int kPerThread = kBatch * kChunks / kThreads;   // loads per thread and batch
     struct Shared {
         alignas(16) T rows[kBatch][kSlice];
-        unsigned short list[kWindow];            // token positions of the window, ascending, relative to its start
-        unsigned int words[kWindow / 32];
+        alignas(16) unsigned int words[kSpan / 32];
+        unsigned short list[kList];              // token positions of the window, ascending, relative to its start
         unsigned int wave_counts[kWavesPerBlock];
     };
 };
@@ -192,22 +204,31 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
                                                    unsigned int hidden, bool accumulate) {
     using L = LongRow<T, Vector>;
     using chunk_t = vec_t<T, static_cast<int>(L::kVec)>;
-    static_assert(kWindow / 32 <= kThreads && kThreads / kWave == kWavesPerBlock, "a thread owns at most one bitmap word");
+    using u32x4 = vec_t<unsigned int, 4>;
+    constexpr unsigned int kWords = kSpan / 32 / kThreads;  // bitmap words of a thread
+    static_assert(kWords % 4 == 0 && kThreads / kWave == kWavesPerBlock, "a thread owns whole 16-byte pieces of the bitmap");
+    const unsigned int window = tokens <= kList ? kSpan : kList;
     const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const unsigned int col = col0 + lane;
     float acc = 0.0f;
     if (wave == 0 && accumulate && col < hidden) acc = to_f32(row[col]);
-    for (unsigned int base = 0; base < count; base += kWindow) {
+    for (unsigned int base = 0; base < count; base += window) {
         // The window's tokens of this segment in ascending order.
-        if (tid < kWindow / 32) lds.words[tid] = 0;
+#pragma unroll
+        for (unsigned int i = 0; i < kWords; i += 4) *reinterpret_cast<u32x4*>(&lds.words[tid * kWords + i]) = u32x4(0u);
         __syncthreads();
         for (unsigned int i = tid; i < tokens; i += kThreads) {
             const unsigned int position = segment[i] - base;  // wraps below the window
-            if (position < kWindow) atomicOr(&lds.words[position / 32], 1u << (position % 32));
+            if (position < window) atomicOr(&lds.words[position / 32], 1u << (position % 32));
         }
         __syncthreads();
-        unsigned int word = tid < kWindow / 32 ? lds.words[tid] : 0u;
-        const unsigned int mine = __popc(word);
+        unsigned int word[kWords], mine = 0;
+#pragma unroll
+        for (unsigned int i = 0; i < kWords; i += 4) {
+            const u32x4 four = *reinterpret_cast<const u32x4*>(&lds.words[tid * kWords + i]);
+#pragma unroll
+            for (unsigned int e = 0; e < 4; ++e) mine += __popc(word[i + e] = four[e]);
+        }
         unsigned int inclusive = mine;
 #pragma unroll
         for (int offset = 1; offset < kWave; offset <<= 1) {
@@ -221,9 +242,12 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
             if (w < wave) slot += lds.wave_counts[w];
             found += lds.wave_counts[w];
         }
-        while (word != 0) {
-            lds.list[slot++] = static_cast<unsigned short>(tid * 32 + __builtin_ctz(word));
-            word &= word - 1;
+#pragma unroll
+        for (unsigned int i = 0; i < kWords; ++i) {
+            while (word[i] != 0) {
+                lds.list[slot++] = static_cast<unsigned short>((tid * kWords + i) * 32 + __builtin_ctz(word[i]));
+                word[i] &= word[i] - 1;
+            }
         }
         __syncthreads();
         // Loads of the batch that starts at list entry `first`, into registers.
@@ -249,15 +273,29 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
             if (first + kBatch < found) fetch(first + kBatch);
             if (wave == 0) {
                 const unsigned int n = min(kBatch, found - first);
-                unsigned int j = 0;
-                for (; j + 16 <= n; j += 16) {
-                    T dy[16];
+                T even[16], odd[16];
+                auto read = [&](T(&dy)[16], unsigned int j) {
+                    const unsigned int from = min(j, kBatch - 16);
 #pragma unroll
-                    for (unsigned int u = 0; u < 16; ++u) dy[u] = lds.rows[j + u][lane];
+                    for (unsigned int u = 0; u < 16; ++u) dy[u] = lds.rows[from + u][lane];
+                };
+                auto add = [&](const T(&dy)[16], unsigned int j) {
+                    if (j + 16 <= n) {
 #pragma unroll
-                    for (unsigned int u = 0; u < 16; ++u) acc = round_to<T>(acc + to_f32(dy[u]));
+                        for (unsigned int u = 0; u < 16; ++u) acc = add_rounded<T>(acc, dy[u]);
+                    } else {
+#pragma unroll
+                        for (unsigned int u = 0; u < 16; ++u)
+                            if (j + u < n) acc = add_rounded<T>(acc, dy[u]);
+                    }
+                };
+                read(even, 0);
+                for (unsigned int j = 0; j < n; j += 32) {
+                    read(odd, j + 16);
+                    add(even, j);
+                    read(even, j + 32);
+                    add(odd, j + 16);
                 }
-                for (; j < n; ++j) acc = round_to<T>(acc + to_f32(lds.rows[j][lane]));
             }
             __syncthreads();
         }
@@ -266,9 +304,11 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
 }
 
 // Workgroups [0, long_groups): long segments. A segment of more than kShort = 64 tokens contains a position of
-// `order` that is a multiple of 64; the first one in it names the segment, so candidate j looks at the id of the
-// token at position 64 j and leaves unless that id's segment is long and 64 j its first multiple. The remaining
-// workgroups take kWavesPerBlock ids each and leave the long ones out.
+// `order` that is a multiple of 64; the first one in it names the segment, so candidate j is the id of the token at
+// position 64 j if that id's segment is long and 64 j its first multiple. Each of these workgroups lists the long
+// ids itself, one candidate per thread at a time, and takes every long_groups-th (id, slice) of the list: a workgroup
+// for every candidate and slice would mostly find that there is nothing to do, after four dependent loads
+// (with the wider bitmap and the shorter chain 64 -> 51 us). The remaining workgroups take kWavesPerBlock ids each and leave the long ones out.
 template <typename T, bool Vector>
 __global__ __launch_bounds__(kThreads) void embedding_rows_kernel(T* __restrict__ grad_weight,
                                                                  const T* __restrict__ grad_output,
@@ -279,15 +319,41 @@ __global__ __launch_bounds__(kThreads) void embedding_rows_kernel(T* __restrict_
                                                                  unsigned int hidden, unsigned int slices,
                                                                  unsigned int long_groups, bool accumulate) {
     __shared__ typename LongRow<T, Vector>::Shared lds;
+    __shared__ unsigned int long_ids[kThreads], wave_longs[kWavesPerBlock];
     if (blockIdx.x < long_groups) {
-        const unsigned int candidate = blockIdx.x / slices, slice = blockIdx.x - candidate * slices;
-        const unsigned int position = candidate * kShort;
-        if (position >= offsets[vocab]) return;  // ids past the vocabulary have no place in `order`
-        const unsigned int id = ids[order[position]];
-        const unsigned int begin = offsets[id], tokens = offsets[id + 1] - begin;
-        if (tokens <= kShort || position - begin >= kShort) return;
-        embedding_long_row<T, Vector>(lds, grad_weight + static_cast<std::size_t>(id) * hidden, grad_output, order + begin,
-                                      tokens, count, slice * kSlice, hidden, accumulate);
+        const unsigned int tid = threadIdx.x, wave = tid / kWave;
+        const unsigned int placed = offsets[vocab];  // ids past the vocabulary have no place in `order`
+        const unsigned int candidates = (placed + kShort - 1) / kShort;
+        unsigned int next_item = blockIdx.x;  // among the items of the candidates from `first` on
+        for (unsigned int first = 0; first < candidates; first += kThreads) {
+            const unsigned int position = (first + tid) * kShort;
+            unsigned int id = 0;
+            bool is_long = false;
+            if (first + tid < candidates) {
+                id = ids[order[position]];
+                const unsigned int begin = offsets[id];
+                is_long = offsets[id + 1] - begin > kShort && position - begin < kShort;
+            }
+            const unsigned long long mask = __ballot(is_long);
+            if ((tid & (kWave - 1)) == 0) wave_longs[wave] = __popcll(mask);
+            __syncthreads();
+            unsigned int slot = __popcll(mask & ((1ull << (tid & (kWave - 1))) - 1)), found = 0;
+            for (unsigned int w = 0; w < kWavesPerBlock; ++w) {
+                if (w < wave) slot += wave_longs[w];
+                found += wave_longs[w];
+            }
+            if (is_long) long_ids[slot] = id;
+            __syncthreads();
+            const unsigned int items = found * slices;
+            for (; next_item < items; next_item += long_groups) {
+                const unsigned int entry = next_item / slices, row = long_ids[entry];
+                const unsigned int begin = offsets[row], tokens = offsets[row + 1] - begin;
+                embedding_long_row<T, Vector>(lds, grad_weight + static_cast<std::size_t>(row) * hidden, grad_output, order + begin,
+                                              tokens, count, (next_item - entry * slices) * kSlice, hidden, accumulate);
+            }
+            next_item -= items;
+            __syncthreads();  // the list is written again
+        }
         return;
     }
     const unsigned int id = (blockIdx.x - long_groups) * kWavesPerBlock + threadIdx.x / kWave;
@@ -368,9 +434,11 @@ extern "C" int cgptx_embedding_backward(void* grad_weight, const void* grad_outp
         auto* dy = static_cast<const T*>(grad_output);
         const bool vector_ok = hidden % kVec128<T> == 0 && is_aligned16(dw) && is_aligned16(dy);
         const auto h = static_cast<unsigned int>(hidden);
-        // Candidates for long segments: one per kShort positions of `order` and slice of the columns.
+        // Long segments: at most one per kShort + 1 tokens, each with a workgroup per slice of the columns, up to what the
+        // chip holds at a time.
         const std::size_t slices = (hidden + kSlice - 1) / kSlice;
-        const std::size_t long_groups = token_count > kShort ? (token_count + kShort - 1) / kShort * slices : 0;
+        const std::size_t long_groups =
+            std::min<std::size_t>(token_count / (kShort + 1) * slices, static_cast<std::size_t>(compute_units()) * 4);
         const std::size_t short_groups = (vocab + kWavesPerBlock - 1) / kWavesPerBlock;
         if (long_groups + short_groups > static_cast<std::size_t>(std::numeric_limits<int>::max()))
             return fail(CGPTX_OVERFLOW, std::string(name) + ": too many workgroups");
