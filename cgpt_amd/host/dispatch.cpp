@@ -5,6 +5,8 @@
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <exception>
+
 #include "cgptx.h"
 
 namespace {
@@ -21,32 +23,42 @@ int dtype_code(const at::Tensor& t) {
 
 PyObject* none() { Py_RETURN_NONE; }
 
+// A reference that is dropped on every way out, exceptions included.
+struct Owned {
+    PyObject* object = nullptr;
+    Owned() = default;
+    explicit Owned(PyObject* o) : object(o) {}
+    Owned(Owned&& other) noexcept : object(other.release()) {}
+    Owned(const Owned&) = delete;
+    ~Owned() { Py_XDECREF(object); }
+    PyObject* release() {
+        PyObject* o = object;
+        object = nullptr;
+        return o;
+    }
+};
+
 // tensors(*tensors) -> (dtype code, pointer of each), pointer 0 for None; None when one of them is no contiguous
 // device tensor or they do not share one of the library's dtypes.
 PyObject* tensors(PyObject*, PyObject* const* args, Py_ssize_t count) {
-    PyObject* out = PyTuple_New(count + 1);
-    if (out == nullptr) return nullptr;
+    Owned out(PyTuple_New(count + 1));
+    if (out.object == nullptr) return nullptr;
     int code = -1;
     for (Py_ssize_t i = 0; i < count; ++i) {
         unsigned long long pointer = 0;
         if (args[i] != Py_None) {
-            if (!THPVariable_Check(args[i])) {
-                Py_DECREF(out);
-                return none();
-            }
+            if (!THPVariable_Check(args[i])) return none();
             const at::Tensor& t = THPVariable_Unpack(args[i]);
             const int mine = dtype_code(t);
             if (code < 0) code = mine;
-            if (mine < 0 || mine != code || !t.is_cuda() || t.layout() != at::kStrided || !t.is_contiguous()) {
-                Py_DECREF(out);
+            if (mine < 0 || mine != code || !t.is_cuda() || t.layout() != at::kStrided || !t.is_contiguous())
                 return none();
-            }
             pointer = reinterpret_cast<unsigned long long>(t.data_ptr());
         }
-        PyTuple_SET_ITEM(out, i + 1, PyLong_FromUnsignedLongLong(pointer));
+        PyTuple_SET_ITEM(out.object, i + 1, PyLong_FromUnsignedLongLong(pointer));
     }
-    PyTuple_SET_ITEM(out, 0, PyLong_FromLong(code));
-    return out;
+    PyTuple_SET_ITEM(out.object, 0, PyLong_FromLong(code));
+    return out.release();
 }
 
 // same_shape(*tensors) -> bool
@@ -63,17 +75,11 @@ struct Names {
 };
 Names names;
 
-// A tensor attribute of an object; the caller drops the reference it receives. Null (no error set) if it is no tensor.
-PyObject* tensor_attribute(PyObject* object, PyObject* name) {
-    PyObject* value = PyObject_GetAttr(object, name);
-    if (value == nullptr) {
-        PyErr_Clear();
-        return nullptr;
-    }
-    if (!THPVariable_Check(value)) {
-        Py_DECREF(value);
-        return nullptr;
-    }
+// A tensor attribute of an object. Null (no error set) if it is no tensor.
+Owned tensor_attribute(PyObject* object, PyObject* name) {
+    Owned value(PyObject_GetAttr(object, name));
+    if (value.object == nullptr) PyErr_Clear();
+    else if (!THPVariable_Check(value.object)) return Owned();
     return value;
 }
 
@@ -89,46 +95,57 @@ PyObject* adamw_entries(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (PyErr_Occurred()) return nullptr;
     for (Py_ssize_t i = 0; i < n; ++i) {
         PyObject* entry = PyList_GET_ITEM(args[0], i);
-        PyObject* state = PyObject_GetAttr(entry, names.state);
+        const Owned held_state(PyObject_GetAttr(entry, names.state));
+        PyObject* state = held_state.object;
         if (state == nullptr) {
             PyErr_Clear();
             Py_RETURN_FALSE;
         }
-        PyObject* held[5] = {tensor_attribute(entry, names.parameter), tensor_attribute(entry, names.gradient),
-                             tensor_attribute(state, names.master), tensor_attribute(state, names.first),
-                             tensor_attribute(state, names.second)};
+        const Owned held[5] = {tensor_attribute(entry, names.parameter), tensor_attribute(entry, names.gradient),
+                               tensor_attribute(state, names.master), tensor_attribute(state, names.first),
+                               tensor_attribute(state, names.second)};
         bool fine = bound == nullptr || state == PyList_GET_ITEM(bound, i);
-        for (PyObject* h : held) fine = fine && h != nullptr;
+        for (const Owned& h : held) fine = fine && h.object != nullptr;
         if (fine) {
-            const at::Tensor& p = THPVariable_Unpack(held[0]);
-            const at::Tensor& g = THPVariable_Unpack(held[1]);
+            const at::Tensor& p = THPVariable_Unpack(held[0].object);
+            const at::Tensor& g = THPVariable_Unpack(held[1].object);
             const int code = dtype_code(p);
             fine = code >= 0 && p.is_cuda() && g.scalar_type() == p.scalar_type() && g.sizes() == p.sizes() && g.device() == p.device();
             for (int k = 2; k < 5; ++k) {
-                const at::Tensor& t = THPVariable_Unpack(held[k]);
+                const at::Tensor& t = THPVariable_Unpack(held[k].object);
                 fine = fine && t.scalar_type() == at::ScalarType::Float && t.sizes() == p.sizes() && t.device() == p.device();
             }
             if (fine) {
                 out[i].parameter = p.data_ptr();
                 out[i].gradient = g.data_ptr();
-                out[i].master_parameter = static_cast<float*>(THPVariable_Unpack(held[2]).data_ptr());
-                out[i].first_moment = static_cast<float*>(THPVariable_Unpack(held[3]).data_ptr());
-                out[i].second_moment = static_cast<float*>(THPVariable_Unpack(held[4]).data_ptr());
+                out[i].master_parameter = static_cast<float*>(THPVariable_Unpack(held[2].object).data_ptr());
+                out[i].first_moment = static_cast<float*>(THPVariable_Unpack(held[3].object).data_ptr());
+                out[i].second_moment = static_cast<float*>(THPVariable_Unpack(held[4].object).data_ptr());
                 out[i].count = static_cast<size_t>(p.numel());
                 out[i].dtype = code;
             }
         }
-        for (PyObject* h : held) Py_XDECREF(h);
-        Py_DECREF(state);
         if (!fine) Py_RETURN_FALSE;
     }
     Py_RETURN_TRUE;
 }
 
+// A tensor may refuse to say where or how large it is (fake tensors, symbolic sizes) with a C++ exception, which must not
+// leave a C entry: it becomes the Python exception that the tensor's own method would raise.
+template <PyObject* (*Function)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* call(PyObject* self, PyObject* const* args, Py_ssize_t count) {
+    try {
+        return Function(self, args, count);
+    } catch (const std::exception& error) {
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, error.what());
+        return nullptr;
+    }
+}
+
 PyMethodDef methods[] = {
-    {"tensors", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(tensors)), METH_FASTCALL, "(dtype code, pointers) or None"},
-    {"same_shape", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(same_shape)), METH_FASTCALL, "whether all shapes are equal"},
-    {"adamw_entries", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(adamw_entries)), METH_FASTCALL, "fills an entry array"},
+    {"tensors", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call<tensors>)), METH_FASTCALL, "(dtype code, pointers) or None"},
+    {"same_shape", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call<same_shape>)), METH_FASTCALL, "whether all shapes are equal"},
+    {"adamw_entries", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call<adamw_entries>)), METH_FASTCALL, "fills an entry array"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_dispatch", "Tensor checks of the operator mirror.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
