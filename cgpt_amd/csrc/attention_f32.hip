@@ -12,7 +12,8 @@
 // one workgroup of eight wavefronts owns 16 stationary rows only, and the wavefronts split the streamed tiles between
 // them (tile t to wavefront t mod 8); their partial results meet in LDS at the end, in wavefront order: no atomics,
 // results independent of scheduling. Few key tiles are shared by several workgroups in the dK/dV pass (the caller decides
-// and adds their sums up). One sequence of 256 tokens, 8:2 heads of 128, causal: forward 151 -> 14 us, dQ
+// and adds their sums up). A query touches no key that the causal mask hides from it, as in a walk over single rows: see
+// non_finite(). One sequence of 256 tokens, 8:2 heads of 128, causal: forward 151 -> 14 us, dQ
 // 239 -> 21, dK/dV 295 -> 20.
 #include "attention_f32.hpp"
 
@@ -79,6 +80,44 @@ __device__ __forceinline__ void accumulate(acc_t (&result)[D / 64][4], const Col
             for (int e = 0; e < 4; ++e) result[b][e] = mfma(rows.part[r][b][e], values[r], result[b][e]);
 }
 
+// Whether the tile holds an Inf or a NaN (the same answer in all lanes): 0 x is 0 for every other x. A tile on the causal
+// diagonal has rows that some stationary rows do not see. Their values are 0, but the matrix instruction multiplies them
+// all the same, and 0 x Inf is NaN. Such a tile with such a row is left out of the walk and added row by row behind it, in
+// a pass of its own so that the walk's registers do not pay for it.
+template <int D>
+__device__ __forceinline__ bool non_finite(const ColumnOperand<D>& rows) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int b = 0; b < D / 64; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = fmaf(rows.part[r][b][e], 0.0f, sum);
+    return __ballot(!(sum == 0.0f)) != 0;
+}
+// accumulate() over the rows row0 + i, below `limit`, that this lane's stationary row sees (visible(i)); no other row is
+// multiplied.
+template <int D, typename Visible>
+__device__ __forceinline__ void accumulate_visible(acc_t (&result)[D / 64][4], const float* base, long row_stride, int row0, int limit,
+                                                   int d, const acc_t& values, Visible&& visible) {
+    const int lane = threadIdx.x & (kWave - 1), at = (lane >> 4) * 16;  // the head dimension's elements of a lane: see deposit()
+#pragma unroll 1
+    for (int i = 0; i < kTile; ++i) {
+        const int r = i & 3;
+        const float value = __shfl(r == 0 ? values[0] : r == 1 ? values[1] : r == 2 ? values[2] : values[3], (lane & 15) + 16 * (i >> 2), kWave);
+        if (row0 + i >= limit || !visible(i)) continue;
+#pragma unroll
+        for (int b = 0; b < D / 64; ++b)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (64 * b + at + 4 * c >= d) continue;
+                const f32x4 row = load_vec<float, 4>(base + (row0 + i) * row_stride + 64 * b + at + 4 * c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) result[b][e][c] = fmaf(row[e], value, result[b][e][c]);
+            }
+    }
+}
+
 // Sums over the four lane groups of a stationary row.
 __device__ __forceinline__ float row_sum(float v) {
     v += __shfl_xor(v, 16, kWave);
@@ -138,6 +177,8 @@ __global__ __launch_bounds__(kThreads) void attention_f32_forward_kernel(Attenti
         const int key = t * kTile + (lane & 15);
         k.load(k_base + key * kv_stride, key < p.ks && t < tiles, p.d);
     };
+    const int first_masked = p.causal ? (p.offset + q0 + 1) / kTile : tiles;  // tile with a key that a query of the block does not see
+    bool left_out = false;
     RowOperand<D> k, ahead;
     key_rows(k, wave);
     for (int t = wave; t < tiles; t += kWaves) {
@@ -168,8 +209,21 @@ __global__ __launch_bounds__(kThreads) void attention_f32_forward_kernel(Attenti
         for (int c = 0; c < D / 64; ++c)
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[c][e] *= alpha;
-        accumulate<D>(o, v, s);
+        if (t >= first_masked && non_finite<D>(v)) left_out = true;
+        else accumulate<D>(o, v, s);
         k = ahead;
+    }
+    if (left_out) {
+        for (int t = wave; t < tiles; t += kWaves) {
+            ColumnOperand<D> v;
+            v.load(v_base, kv_stride, t * kTile, p.ks, p.d);
+            if (t < first_masked || !non_finite<D>(v)) continue;
+            key_rows(k, t);
+            acc_t s = product<D>(k, q);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] = expf(s[r] * p.scale - (m == -INFINITY ? 0.0f : m));
+            accumulate_visible<D>(o, v_base, kv_stride, t * kTile, p.ks, p.d, s, [&](int i) { return t * kTile + i <= my_last; });
+        }
     }
     // Common maximum over the wavefronts, then the weighted sums.
     if (lane < kTile) {
@@ -186,8 +240,9 @@ __global__ __launch_bounds__(kThreads) void attention_f32_forward_kernel(Attenti
     auto denominator = [&](int row, float& top) {
         top = wave_max[0][row];
         for (int w = 1; w < kWaves; ++w) top = fmaxf(top, wave_max[w][row]);
+        if (top == -INFINITY) return NAN;  // every query sees a key, so all its scores are -Inf or NaN
         float sum = 0.0f;
-        for (int w = 0; w < kWaves; ++w) sum += top == -INFINITY ? 0.0f : wave_total[w][row] * expf(wave_max[w][row] - top);
+        for (int w = 0; w < kWaves; ++w) sum += wave_total[w][row] * expf(wave_max[w][row] - top);
         return sum;
     };
     collect<D>(lds, p.d, [&](int row, int at, const f32x4& sum) {
@@ -195,7 +250,7 @@ __global__ __launch_bounds__(kThreads) void attention_f32_forward_kernel(Attenti
         float top;
         const float l = denominator(row, top);
         store_vec<float, 4>(p.out + (static_cast<long>(b) * p.qs + q0 + row) * q_stride + static_cast<long>(h) * p.d + at,
-                            sum * (l > 0.0f ? 1.0f / l : 0.0f));
+                            sum * (1.0f / l));  // l is NaN or, with the maximum's own term, at least 1
         if (at == 0 && p.lse_out != nullptr) p.lse_out[(static_cast<long>(b) * p.qs + q0 + row) * p.hq + h] = top + logf(l);
     });
 }
@@ -235,18 +290,34 @@ __global__ __launch_bounds__(kThreads) void attention_f32_dq_kernel(AttentionF32
     for (int c = 0; c < D / 64; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) dq[c][e] = acc_t(0.0f);
-    for (int t = wave; t <= last_key / kTile; t += kWaves) {
+    const int first_masked = p.causal ? (p.offset + q0 + 1) / kTile : last_key / kTile + 1;
+    bool left_out = false;
+    auto score_gradient = [&](int t) {  // lane: query l % 16, keys 4 g + r
         const int key = t * kTile + (lane & 15);
         RowOperand<D> k, v;
         k.load(k_base + key * kv_stride, key < p.ks, p.d);
         v.load(v_base + key * kv_stride, key < p.ks, p.d);
-        ColumnOperand<D> columns;
-        columns.load(k_base, kv_stride, t * kTile, p.ks, p.d);
         const acc_t s = product<D>(k, q), dp = product<D>(v, dout);
         acc_t ds;
 #pragma unroll
         for (int r = 0; r < 4; ++r) ds[r] = t * kTile + 4 * g + r <= my_last ? expf(s[r] * p.scale - lse) * (dp[r] - delta) : 0.0f;
-        accumulate<D>(dq, columns, ds);
+        return ds;
+    };
+    for (int t = wave; t <= last_key / kTile; t += kWaves) {
+        ColumnOperand<D> columns;
+        columns.load(k_base, kv_stride, t * kTile, p.ks, p.d);
+        const acc_t ds = score_gradient(t);
+        if (t >= first_masked && non_finite<D>(columns)) left_out = true;
+        else accumulate<D>(dq, columns, ds);
+    }
+    if (left_out) {
+        for (int t = wave; t <= last_key / kTile; t += kWaves) {
+            ColumnOperand<D> columns;
+            columns.load(k_base, kv_stride, t * kTile, p.ks, p.d);
+            if (t < first_masked || !non_finite<D>(columns)) continue;
+            accumulate_visible<D>(dq, k_base, kv_stride, t * kTile, p.ks, p.d, score_gradient(t),
+                                  [&](int i) { return t * kTile + i <= my_last; });
+        }
     }
     deposit<D>(lds, wave, dq, p.scale);
     __syncthreads();
@@ -258,8 +329,9 @@ __global__ __launch_bounds__(kThreads) void attention_f32_dq_kernel(AttentionF32
     });
 }
 
+// Four wavefronts per SIMD, two workgroups per CU, with heads of 64: the compiler's own choice is four registers over that.
 template <int D>
-__global__ __launch_bounds__(kThreads) void attention_f32_dkv_kernel(AttentionF32Args p) {
+__global__ __launch_bounds__(kThreads, D == 64 ? 4 : 2) void attention_f32_dkv_kernel(AttentionF32Args p) {
     extern __shared__ __align__(16) float lds[];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, g = lane >> 4;
     const int part = blockIdx.x % p.parts, k0 = blockIdx.x / p.parts * kTile;  // the first keys have most queries
@@ -279,34 +351,56 @@ __global__ __launch_bounds__(kThreads) void attention_f32_dkv_kernel(AttentionF3
     for (int c = 0; c < D / 64; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) dk[c][e] = dv[c][e] = acc_t(0.0f);
-    const int end = (part + 1) * (tiles * group) / p.parts;
-    for (int i = part * (tiles * group) / p.parts + wave; i < end; i += kWaves) {  // (head of the group, query tile)
-        const int head = i / tiles, t = first_tile + i - head * tiles, h = kvh * group + head;
-        const float* q_base = p.q + static_cast<long>(b) * p.qs * q_stride + static_cast<long>(h) * p.d;
-        const float* do_base = p.dout + static_cast<long>(b) * p.qs * q_stride + static_cast<long>(h) * p.d;
-        const int query = t * kTile + (lane & 15);
-        acc_t s, dp;
-        {
-            RowOperand<D> q, dout;
-            q.load(q_base + query * q_stride, query < p.qs, p.d);
-            dout.load(do_base + query * q_stride, query < p.qs, p.d);
-            s = product<D>(q, k);  // lane: key l % 16, queries 4 g + r
-            dp = product<D>(dout, v);
-        }
-        acc_t prob, ds;
+    const int begin = part * (tiles * group) / p.parts + wave, end = (part + 1) * (tiles * group) / p.parts;
+    bool left_out = false;
+    // Item i is (head of the group, query tile): step(its head's Q and dO, first query, probabilities and score gradients of
+    // queries 4 g + r).
+    auto walk = [&](auto&& step) __attribute__((always_inline)) {
+        for (int i = begin; i < end; i += kWaves) {
+            const int head = i / tiles, row0 = (first_tile + i - head * tiles) * kTile, h = kvh * group + head;
+            const float* q_base = p.q + static_cast<long>(b) * p.qs * q_stride + static_cast<long>(h) * p.d;
+            const float* do_base = p.dout + static_cast<long>(b) * p.qs * q_stride + static_cast<long>(h) * p.d;
+            const int query = row0 + (lane & 15);
+            acc_t s, dp;
+            {
+                RowOperand<D> q, dout;
+                q.load(q_base + query * q_stride, query < p.qs, p.d);
+                dout.load(do_base + query * q_stride, query < p.qs, p.d);
+                s = product<D>(q, k);  // lane: key l % 16, queries 4 g + r
+                dp = product<D>(dout, v);
+            }
+            acc_t prob, ds;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = t * kTile + 4 * g + r;
-            const bool seen = row >= first_query && row < p.qs && key < p.ks;
-            const long stat = (static_cast<long>(b) * p.qs + min(row, p.qs - 1)) * p.hq + h;
-            prob[r] = seen ? expf(s[r] * p.scale - p.lse[stat]) : 0.0f;
-            ds[r] = prob[r] * (dp[r] - p.delta[stat]);
+            for (int r = 0; r < 4; ++r) {
+                const int row = row0 + 4 * g + r;
+                const bool seen = row >= first_query && row < p.qs && key < p.ks;
+                const long stat = (static_cast<long>(b) * p.qs + min(row, p.qs - 1)) * p.hq + h;
+                prob[r] = seen ? expf(s[r] * p.scale - p.lse[stat]) : 0.0f;
+                ds[r] = seen ? prob[r] * (dp[r] - p.delta[stat]) : 0.0f;
+            }
+            step(q_base, do_base, row0, prob, ds);
         }
+    };
+    auto masked = [&](int row0) { return p.causal && row0 < k0 + kTile - 1 - p.offset; };  // a query that does not see a key of the block
+    walk([&](const float* q_base, const float* do_base, int row0, const acc_t& prob, const acc_t& ds) __attribute__((always_inline)) {
         ColumnOperand<D> columns;
-        columns.load(do_base, q_stride, t * kTile, p.qs, p.d);
-        accumulate<D>(dv, columns, prob);
-        columns.load(q_base, q_stride, t * kTile, p.qs, p.d);
-        accumulate<D>(dk, columns, ds);
+        columns.load(do_base, q_stride, row0, p.qs, p.d);
+        if (masked(row0) && non_finite<D>(columns)) left_out = true;
+        else accumulate<D>(dv, columns, prob);
+        columns.load(q_base, q_stride, row0, p.qs, p.d);
+        if (masked(row0) && non_finite<D>(columns)) left_out = true;
+        else accumulate<D>(dk, columns, ds);
+    });
+    if (left_out) {
+        walk([&](const float* q_base, const float* do_base, int row0, const acc_t& prob, const acc_t& ds) __attribute__((always_inline)) {
+            if (!masked(row0)) return;
+            auto visible = [&](int i) { return row0 + i >= first_query; };
+            ColumnOperand<D> columns;
+            columns.load(do_base, q_stride, row0, p.qs, p.d);
+            if (non_finite<D>(columns)) accumulate_visible<D>(dv, do_base, q_stride, row0, p.qs, p.d, prob, visible);
+            columns.load(q_base, q_stride, row0, p.qs, p.d);
+            if (non_finite<D>(columns)) accumulate_visible<D>(dk, q_base, q_stride, row0, p.qs, p.d, ds, visible);
+        });
     }
     const long count = static_cast<long>(p.batch) * p.ks * kv_stride;
     float* const dk_out = p.parts == 1 ? p.dk : p.partial + 2 * part * count;

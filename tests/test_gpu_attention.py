@@ -297,6 +297,52 @@ def test_fp32_matrix_core_parity(device, case, with_lse):
         assert torch.equal(g, again)
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
+@pytest.mark.parametrize("tensor", ["q", "k", "v", "do"])
+@pytest.mark.parametrize("case", range(3))
+def test_fp32_hidden_rows_are_not_touched(device, case, tensor, value):
+    """A row with an Inf or a NaN makes what depends on it non-finite and nothing else: a query does not touch a key that the
+    mask hides from it, although one matrix instruction multiplies the whole tile of them. The rest is compared with the
+    float64 formulas on the row's finite values, to the 1e-4 of the other fp32 tests."""
+    c = [dict(b=1, qs=40, ks=40, hq=2, hkv=1, d=64), dict(b=2, qs=37, ks=50, hq=2, hkv=1, d=128, off=13),
+         dict(b=1, qs=33, ks=60, hq=2, hkv=1, d=36, off=20)][case]
+    off, rows = c.get("off", 0), (c["qs"] if tensor in ("q", "do") else c["ks"])
+    q, k, v, do = make_inputs(c, torch.float32, 500 + case)
+    want_out, want_lse = oracle64.attention_forward(to_np(q), to_np(k), to_np(v), *oracle_args(c))
+    want = dict(zip(("dq", "dk", "dv"), oracle64.attention_backward(to_np(do), to_np(q), to_np(k), to_np(v), *oracle_args(c))))
+    want.update(out=want_out, lse=want_lse)
+    query, key = np.arange(c["qs"])[:, None], np.arange(c["ks"])
+    for row in (0, 5, 15, 16, 23, rows - 1):
+        planted = {"q": q.clone(), "k": k.clone(), "v": v.clone(), "do": do.clone()}
+        planted[tensor][0, row, 0, 1] = value
+        tensors = planted["q"], planted["k"], planted["v"]
+        out, lse = run_forward(device, *tensors, c)
+        got = dict(zip(("dq", "dk", "dv"), run_backward(device, planted["do"], *tensors, c)), out=out, lse=lse)
+        again = dict(zip(("dq", "dk", "dv"), run_backward(device, planted["do"], *tensors, c, with_lse=False)))
+        # What depends on the row: per output, [query or key, head] of the first sequence.
+        queries = np.zeros((c["qs"], c["hq"]), bool)
+        if tensor in ("q", "do"):
+            queries[row, 0] = True
+        else:
+            queries[row <= off + query[:, 0]] = True
+        keys = (queries.any(axis=1)[:, None] & (key <= off + query)).any(axis=0)[:, None]
+        none_q, none_k = np.zeros_like(queries), np.zeros_like(keys)
+        touched = {"out": none_q if tensor == "do" else queries, "lse": queries if tensor in ("q", "k") else none_q, "dq": queries,
+                   "dk": keys, "dv": none_k if tensor == "v" else keys}
+        for name, result in [*got.items(), *again.items()]:
+            result, expected = to_np(result), want[name].copy()
+            at = touched[name]
+            where = f"{tensor}[{row}] {name}"
+            if not np.isnan(value) and tensor == "v" and name == "out":
+                assert not np.isfinite(result[0][at][:, 1]).any(), where
+            elif np.isnan(value) and tensor in ("q", "k"):
+                assert np.isnan(result[0][at]).all(), where
+            elif at.any():
+                assert not np.isfinite(result[0][at]).all(), where
+            result[0][at] = expected[0][at] = 0.0
+            assert_close(result, expected, 1e-4, where)
+
+
 def test_unaligned_tensors_take_the_scalar_family(device):
     """Views that start 2 bytes into an allocation are not 16-byte aligned: same results as the aligned call
     to storage precision (the two families round differently)."""
