@@ -1753,11 +1753,24 @@ int launch_dkv_reduce(const Shape& s, void* dk, void* dv, const float* partial, 
     return CGPTX_OK;
 }
 
-// Scratch of the backward pass: [delta | LSE·log2 e | partial sums of shared key blocks].
-std::size_t backward_scratch_bytes(const Shape& s, bool scalar) {
-    const std::size_t stats = 2 * stat_block_bytes(s.batch * s.qs * s.hq);
-    const int splits = scalar && s.dtype != CGPTX_F32 ? 1 : dkv_splits(s);
-    return stats + (splits > 1 ? (static_cast<std::size_t>(splits) * 2 * s.batch * s.ks * s.hkv * s.d * sizeof(float) + 255) & ~std::size_t{255} : 0);
+// Scratch of the backward pass: [delta | LSE·log2 e | partial sums of shared key blocks | what the caller needs].
+struct BackwardScratch {
+    char* mem;
+    int splits;        // workgroups that share a key block
+    std::size_t used;  // bytes ahead of the caller's
+};
+// An arena that cannot grow shares key blocks between as many workgroups as it has room for.
+int backward_scratch(const Shape& s, bool scalar, std::size_t extra, hipStream_t stream, BackwardScratch* out) {
+    const std::size_t stats = 2 * stat_block_bytes(s.batch * s.qs * s.hq), part = 2 * s.batch * s.ks * s.hkv * s.d * sizeof(float);
+    int splits = scalar && s.dtype != CGPTX_F32 ? 1 : dkv_splits(s);
+    auto used = [&] { return stats + (splits > 1 ? (splits * part + 255) & ~std::size_t{255} : 0); };
+    void* mem = nullptr;
+    std::size_t held = 0;
+    if (int st = scratch_up_to(stream, used() + extra, &mem, &held)) return st;
+    while (splits > 1 && held < used() + extra) --splits;
+    if (int st = scratch(stream, used() + extra, &mem)) return st;
+    *out = {static_cast<char*>(mem), splits, used()};
+    return CGPTX_OK;
 }
 
 // The call as the fp32 kernels take it.
@@ -1815,13 +1828,11 @@ int launch_forward(const Shape& s, Params p, bool scalar, hipStream_t stream) {
 }
 
 int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, const void* dout, const void* out,
-                    const float* lse, int accumulate, bool scalar, hipStream_t stream) {
+                    const float* lse, int accumulate, bool scalar, const BackwardScratch& room, hipStream_t stream) {
     const std::size_t rows = s.batch * s.qs * s.hq;
     const std::size_t stat_bytes = stat_block_bytes(rows);
-    void* mem = nullptr;
-    if (int st = scratch(stream, backward_scratch_bytes(s, scalar), &mem)) return st;
-    auto* delta = static_cast<float*>(mem);
-    auto* lse2 = reinterpret_cast<float*>(static_cast<char*>(mem) + stat_bytes);
+    auto* delta = reinterpret_cast<float*>(room.mem);
+    auto* lse2 = reinterpret_cast<float*>(room.mem + stat_bytes);
     p.dout = dout;
     p.lse = lse;
     p.delta = delta;
@@ -1836,8 +1847,8 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
         a.dk = static_cast<float*>(dk);
         a.dv = static_cast<float*>(dv);
         a.accumulate = accumulate;
-        a.parts = dkv_splits(s);
-        a.partial = reinterpret_cast<float*>(static_cast<char*>(mem) + 2 * stat_bytes);
+        a.parts = room.splits;
+        a.partial = reinterpret_cast<float*>(room.mem + 2 * stat_bytes);
         if (int st = attention_f32_backward(a, stream)) return st;
         return a.parts > 1 ? launch_dkv_reduce<float>(s, dk, dv, a.partial, a.parts, accumulate, stream) : CGPTX_OK;
     }
@@ -1903,8 +1914,8 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
                 // grid that leaves compute units idle is better off with twice the workgroups (the longest single
                 // block is shorter than the pair that contains it).
                 const std::size_t single_blocks = static_cast<std::size_t>(key_blocks) * s.hkv * s.batch;
-                pk.splits = dkv_splits(s);
-                pk.partial = reinterpret_cast<float*>(static_cast<char*>(mem) + 2 * stat_bytes);
+                pk.splits = room.splits;
+                pk.partial = reinterpret_cast<float*>(room.mem + 2 * stat_bytes);
                 pk.paired = pk.splits == 1 && s.causal && single_blocks > static_cast<std::size_t>(compute_units());
                 const dim3 pair_grid(pk.paired ? (key_blocks + 1) / 2 : key_blocks * static_cast<unsigned int>(pk.splits),
                                      static_cast<unsigned int>(s.hkv), static_cast<unsigned int>(s.batch));
@@ -1977,8 +1988,10 @@ extern "C" int cgptx_flash_gqa_attention_backward_with_lse(
     p.k = key;
     p.v = value;
     const bool scalar = scalar_path(s, {grad_query, grad_key, grad_value, grad_output, output, query, key, value});
+    BackwardScratch room;
+    if (int st = backward_scratch(s, scalar, 0, static_cast<hipStream_t>(stream), &room)) return st;
     return launch_backward(s, p, grad_query, grad_key, grad_value, grad_output, output, logsumexp,
-                           accumulate_grads != 0, scalar, static_cast<hipStream_t>(stream));
+                           accumulate_grads != 0, scalar, room, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int cgptx_flash_gqa_attention_backward(void* grad_query, void* grad_key, void* grad_value,
@@ -1998,17 +2011,14 @@ extern "C" int cgptx_flash_gqa_attention_backward(void* grad_query, void* grad_k
         return fail(CGPTX_INVALID_ARGUMENT, std::string(name) + ": null tensor");
     const bool scalar = scalar_path(s, {grad_query, grad_key, grad_value, grad_output, query, key, value});
     auto stream = static_cast<hipStream_t>(stream_);
-    // Recompute the output and the log-sum-exp into scratch, then run the LSE path. The scratch
-    // block is laid out [what launch_backward asks for | lse | output], so that its request for the
-    // prefix returns the same base pointer.
+    // Recompute the output and the log-sum-exp into scratch, behind what the LSE path uses, then run that.
     const std::size_t rows = batch * query_sequence * query_heads;
     const std::size_t stat_bytes = stat_block_bytes(rows);
     const std::size_t out_bytes = rows * head_dim * dtype_size(dtype);
-    void* mem = nullptr;
-    const std::size_t prefix = backward_scratch_bytes(s, scalar);
-    if (int st = scratch(stream, prefix + stat_bytes + out_bytes, &mem)) return st;
-    auto* lse = reinterpret_cast<float*>(static_cast<char*>(mem) + prefix);
-    void* out = static_cast<char*>(mem) + prefix + stat_bytes;
+    BackwardScratch room;
+    if (int st = backward_scratch(s, scalar, stat_bytes + out_bytes, stream, &room)) return st;
+    auto* lse = reinterpret_cast<float*>(room.mem + room.used);
+    void* out = room.mem + room.used + stat_bytes;
     Params p = make_params(s);
     p.q = query;
     p.k = key;
@@ -2018,5 +2028,5 @@ extern "C" int cgptx_flash_gqa_attention_backward(void* grad_query, void* grad_k
     fwd.lse_out = lse;
     if (int st = launch_forward(s, fwd, scalar, stream)) return st;
     return launch_backward(s, p, grad_query, grad_key, grad_value, grad_output, out, lse, accumulate_grads != 0,
-                           scalar, stream);
+                           scalar, room, stream);
 }

@@ -222,6 +222,10 @@ int adamw_enqueue(cgptx_adamw_workspace* workspace, const cgptx_adamw_entry* ent
 // aligned. Grows by reallocation on eager calls; refuses to grow during capture.
 int scratch(hipStream_t stream, std::size_t bytes, void** out);
 
+// The same for scratch that a call is faster with but can do without: where the arena cannot grow to `bytes` (the stream
+// is being captured, or the memory is not there), the call gets what the arena holds. *held: its bytes, possibly 0.
+int scratch_up_to(hipStream_t stream, std::size_t bytes, void** out, std::size_t* held);
+
 // Identifies the block currently behind the (current device, stream) arena: it changes whenever that
 // arena is reallocated (a larger request) and reads 0 after cgptx_release_scratch. A captured graph
 // holds the block's address, so whoever replays one compares this value with the one at capture time

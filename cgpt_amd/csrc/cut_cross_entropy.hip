@@ -60,16 +60,21 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
     // Rows of logits are padded to whole K tiles of the input gradient's contraction (32 elements): an odd vocabulary
     // then streams like any other. The padding holds zeros: columns of Z the classifier has no rows for, and cleared
     // by the softmax pass.
-    const std::size_t pitch = (vocab + 31) / 32 * 32;
-    std::size_t limit = logits_bytes / (pitch * elem);
-    limit = std::max<std::size_t>(256, limit / 256 * 256);
-    const std::size_t pieces = (rows + limit - 1) / limit;
-    std::size_t chunk = ((rows + pieces - 1) / pieces + 255) / 256 * 256;
-    chunk = std::min(chunk, rows);
-    const bool single = chunk >= rows;
-    const std::size_t loss_bytes = (rows * sizeof(float) + 255) & ~std::size_t{255};
-    const std::size_t acc_bytes = single ? 0 : (vocab * hidden * sizeof(float) + 255) & ~std::size_t{255};
-    const std::size_t logit_bytes = (chunk * pitch * elem + 255) & ~std::size_t{255};
+    std::size_t pitch = 0, chunk = 0, loss_bytes = 0, acc_bytes = 0, logit_bytes = 0;
+    bool single = true;
+    auto lay_out = [&](std::size_t row_length) {
+        pitch = row_length;
+        std::size_t limit = logits_bytes / (pitch * elem);
+        limit = std::max<std::size_t>(256, limit / 256 * 256);
+        const std::size_t pieces = (rows + limit - 1) / limit;
+        chunk = ((rows + pieces - 1) / pieces + 255) / 256 * 256;
+        chunk = std::min(chunk, rows);
+        single = chunk >= rows;
+        loss_bytes = (rows * sizeof(float) + 255) & ~std::size_t{255};
+        acc_bytes = single ? 0 : (vocab * hidden * sizeof(float) + 255) & ~std::size_t{255};
+        logit_bytes = (chunk * pitch * elem + 255) & ~std::size_t{255};
+    };
+    lay_out((vocab + 31) / 32 * 32);
     // The gradients' contractions may be split along K (a chunk's input gradient has few output tiles and the vocabulary
     // as its K, a small vocabulary's gradient few tiles and the rows); their partial tiles get room of their own.
     auto input_gradient_call = [&](std::size_t r0, std::size_t r) {  // dX[r, H] = dZ[r, V]·C[V, H]
@@ -107,9 +112,21 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         split_bytes = std::max({split_bytes, gemm_split_bytes(input_gradient_call(0, r)), gemm_split_bytes(classifier_gradient_call(0, r))});
     split_bytes = (split_bytes + 255) & ~std::size_t{255};
     void* mem = nullptr;
+    std::size_t held = 0;
     // Arena layout: [row_loss | acc | split-K partials | logits]. The contractions below run with no_split: they
-    // never ask the arena for scratch of their own, and split only into the room given to them here.
-    if (int s = scratch(stream, loss_bytes + acc_bytes + split_bytes + logit_bytes, &mem)) return s;
+    // never ask the arena for scratch of their own, and split only into the room given to them here. An arena that
+    // cannot grow is used as it is: less room to split into, and logits without padding before none at all.
+    auto needed = [&] { return loss_bytes + acc_bytes + logit_bytes; };
+    if (int s = scratch_up_to(stream, needed() + split_bytes, &mem, &held)) return s;
+    if (held < needed()) {
+        if (int s = scratch_up_to(stream, needed(), &mem, &held)) return s;
+    }
+    if (held < needed()) {
+        lay_out(vocab);
+        if (int s = scratch(stream, needed(), &mem)) return s;
+        held = std::max(held, needed());
+    }
+    split_bytes = std::min(split_bytes, (held - needed()) & ~std::size_t{255});
     auto* base = static_cast<char*>(mem);
     auto* row_loss = reinterpret_cast<float*>(base);
     auto* acc = reinterpret_cast<float*>(base + loss_bytes);

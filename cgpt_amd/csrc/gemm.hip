@@ -42,7 +42,7 @@
 // Operands whose rows are not whole aligned 16-byte chunks are copied to padded rows first;
 // C may have any width and alignment (a store per element). fp32 storage takes the same kernels
 // with v_mfma_f32_16x16x4_f32 and K steps of 16. Operands beyond 32-bit offsets, and unaligned ones
-// of a caller that owns the arena, run on a general fp32 matrix-core kernel
+// of a caller that owns the arena or whose padded copies the arena has no room for, run on a general fp32 matrix-core kernel
 // (v_mfma_f32_32x32x2_f32, register-staged operand tiles) with the same semantics.
 #include "gemm_small.hpp"
 #include "gemm_tiles.hpp"
@@ -1321,18 +1321,14 @@ int run_plan(const GemmArgs& g, const Plan& plan, KernelArgs p, hipStream_t stre
         return launch_layout<T, 128, 128, SPLIT>(args, g.a_k_contiguous, g.b_k_contiguous, plan.slices, stream);
     };
     if (plan.slices == 1) return launch.template operator()<false>(p);
-    void* mem = g.no_split ? g.split_workspace : nullptr;
-    if (mem == nullptr) {
-        if (int s = scratch(stream, plan.partial_bytes(g), &mem)) return s;
-    }
     KernelArgs split = p;
-    split.c = mem;
+    split.c = g.split_workspace;
     split.ld_partial = static_cast<long>(round_up(g.n, 8));
     if (int s = launch.template operator()<true>(split)) return s;
     const long quads = static_cast<long>(p.m) * (split.ld_partial / 4);
     const long blocks = std::min<long>((quads + kThreads - 1) / kThreads, static_cast<long>(compute_units()) * 8);
     hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), 0, stream,
-                       g.c, static_cast<const float*>(mem), static_cast<const T*>(g.bias), p.m,
+                       g.c, static_cast<const float*>(g.split_workspace), static_cast<const T*>(g.bias), p.m,
                        static_cast<int>(split.ld_partial), p.n, p.ldc, plan.slices, p.accumulate, p.c_f32, p.ragged);
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
@@ -1403,9 +1399,20 @@ bool c_streams(const GemmArgs& g, std::size_t elem) {
 
 // An operand whose rows the streamed kernels cannot read (odd widths, unaligned storage) is copied to padded rows
 // first: one pass over the operand (a few microseconds) against a contraction that ran at the fp32 matrix rate, a
-// sixteenth of the 16-bit one. Copies and split-K partial tiles share one request to the arena.
+// sixteenth of the 16-bit one. Copies and split-K partial tiles share one request to the arena. *taken: whether the arena
+// has room for the copies; nothing was launched if not.
 template <typename T>
-int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream);
+int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream, bool* taken);
+
+// Whole aligned calls that leave at least half of the chip idle unless a long K is split (weight gradients). A graph recorded
+// without the partial tiles' memory would pay for that at every replay, so these insist on it and report that the arena
+// cannot grow; the other calls are faster split but run as they can.
+bool insists_on_split(const GemmArgs& g, bool ragged) {
+    if (g.dtype == CGPTX_F32 || ragged || g.k % kBK<bf16_t> != 0 || g.m % 8 != 0 || g.k / kBK<bf16_t> < 32) return false;
+    const std::size_t units = static_cast<std::size_t>(compute_units());
+    const std::size_t large = ((g.m + 255) / 256) * ((g.n + 255) / 256), small = ((g.m + 127) / 128) * ((g.n + 127) / 128);
+    return small <= units || (large >= 8 && 2 * large <= units && g.k / kBK<bf16_t> >= 32 * ((units + large - 1) / large));
+}
 
 template <typename T>
 int run_typed(const GemmArgs& g, hipStream_t stream) {
@@ -1475,7 +1482,11 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
             const bool a_ok = a_streams(whole), b_ok = b_streams(whole);
             fast = a_ok && b_ok;
             p.ragged = c_streams(whole, sizeof(T)) ? 0 : 1;
-            if (!fast && !segmented && g.batch_rows == 0 && !g.no_split) return run_padded<T>(g, !a_ok, !b_ok, stream);
+            if (!fast && !segmented && g.batch_rows == 0 && !g.no_split) {
+                bool taken = false;
+                const int s = run_padded<T>(g, !a_ok, !b_ok, stream, &taken);
+                if (taken || s != CGPTX_OK) return s;
+            }
         }
         if (p.ragged && segmented) return fail(CGPTX_INVALID_ARGUMENT, "gemm: segmented operands need the aligned MFMA path");
     }
@@ -1490,11 +1501,25 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
         CGPTX_LAUNCH_CHECK();
         return CGPTX_OK;
     }
-    return run_plan<T>(g, make_plan(g), p, stream);
+    Plan plan = make_plan(g);
+    if (plan.slices == 1 || g.no_split) return run_plan<T>(g, plan, p, stream);
+    GemmArgs split = g;
+    const std::size_t wanted = plan.partial_bytes(g);
+    if (int s = scratch_up_to(stream, wanted, &split.split_workspace, &split.split_workspace_bytes)) return s;
+    if (split.split_workspace_bytes < wanted) {
+        split.no_split = true;  // but into the room there is
+        const Plan smaller = make_plan(split);
+        if (g.batch_rows != 0 || (smaller.slices == 1 && insists_on_split(g, p.ragged != 0))) {
+            if (int s = scratch(stream, wanted, &split.split_workspace)) return s;  // says what is in the way
+        } else {
+            plan = smaller;
+        }
+    }
+    return run_plan<T>(split, plan, p, stream);
 }
 
 template <typename T>
-int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream) {
+int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream, bool* taken) {
     GemmArgs padded = g;
     const std::size_t k_whole = round_up(g.k, kBK<T>), chunk = kVec128<T>;
     std::size_t a_bytes = 0, b_bytes = 0;
@@ -1512,7 +1537,10 @@ int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream) {
     if (!g.b_k_contiguous) padded.b_k = g.b_k != 0 ? g.b_k : g.k;
     const std::size_t split_bytes = make_plan(padded).partial_bytes(padded);
     void* mem = nullptr;
-    if (int s = scratch(stream, a_bytes + b_bytes + split_bytes, &mem)) return s;
+    std::size_t held = 0;
+    if (int s = scratch_up_to(stream, a_bytes + b_bytes + split_bytes, &mem, &held)) return s;
+    *taken = held >= a_bytes + b_bytes;
+    if (!*taken) return CGPTX_OK;
     auto* base = static_cast<char*>(mem);
     if (pad_a) {
         padded.a = base;
@@ -1526,7 +1554,7 @@ int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream) {
     }
     padded.no_split = true;
     padded.split_workspace = split_bytes != 0 ? base + a_bytes + b_bytes : nullptr;
-    padded.split_workspace_bytes = split_bytes;
+    padded.split_workspace_bytes = std::min(split_bytes, held - a_bytes - b_bytes);
     return run_typed<T>(padded, stream);
 }
 

@@ -218,10 +218,16 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
         const std::size_t copy_bytes = (rows * dy_pitch * elem + 255) & ~std::size_t{255};
         split_bytes = std::max(gemm_split_bytes(input_gradient()), gemm_split_bytes(weight_gradient())) + 256;
         void* mem = nullptr;
-        if (int s = scratch(stream, copy_bytes + split_bytes, &mem)) return s;
-        if (int s = pad_rows(mem, grad_output, rows, out_features, out_features, dy_pitch, dtype, stream)) return s;
-        dy = mem;
-        split_room = static_cast<char*>(mem) + copy_bytes;
+        std::size_t held = 0;
+        if (int s = scratch_up_to(stream, copy_bytes + split_bytes, &mem, &held)) return s;
+        if (held >= copy_bytes) {
+            if (int s = pad_rows(mem, grad_output, rows, out_features, out_features, dy_pitch, dtype, stream)) return s;
+            dy = mem;
+            split_room = static_cast<char*>(mem) + copy_bytes;
+            split_bytes = std::min(split_bytes, held - copy_bytes);
+        } else {
+            dy_pitch = out_features;  // no room for the copy: each contraction goes its own way
+        }
     }
     if (grad_input != nullptr)
         if (int s = gemm(input_gradient(), stream)) return s;

@@ -34,7 +34,9 @@ int check_hip(hipError_t error, const char* what) {
     return fail(CGPTX_RUNTIME, std::string(what) + ": " + hipGetErrorString(error));
 }
 
-int scratch(hipStream_t stream, std::size_t bytes, void** out) {
+// Grows the stream's arena to `bytes` where that is possible. *result: the arena as it then is. *capturing, *allocation: what
+// was in the way if it holds less.
+static int grow_arena(hipStream_t stream, std::size_t bytes, Arena* result, bool* capturing, hipError_t* allocation) {
     int device = 0;
     CGPTX_HIP(hipGetDevice(&device));
     std::lock_guard<std::mutex> lock(g_arena_mutex);
@@ -42,23 +44,46 @@ int scratch(hipStream_t stream, std::size_t bytes, void** out) {
     if (arena.bytes < bytes) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         if (stream != nullptr) CGPTX_HIP(hipStreamIsCapturing(stream, &capture));
-        if (capture != hipStreamCaptureStatusNone) {
-            return fail(CGPTX_CAPTURE_ALLOC,
-                        "scratch arena would have to grow during stream capture; run the op once eagerly first");
-        }
+        *capturing = capture != hipStreamCaptureStatusNone;
         // Round up so that small variations in problem size do not reallocate.
         const std::size_t rounded = (bytes + (std::size_t{1} << 20) - 1) & ~((std::size_t{1} << 20) - 1);
         void* fresh = nullptr;
-        CGPTX_HIP(hipMalloc(&fresh, rounded));
-        if (arena.data != nullptr) {
-            // hipFree waits for outstanding work that may still read the old block.
-            CGPTX_HIP(hipFree(arena.data));
+        if (!*capturing) *allocation = hipMalloc(&fresh, rounded);
+        if (*allocation != hipSuccess) (void)hipGetLastError();  // reported from here, not by the next launch
+        if (fresh != nullptr) {
+            if (arena.data != nullptr) {
+                // hipFree waits for outstanding work that may still read the old block.
+                CGPTX_HIP(hipFree(arena.data));
+            }
+            arena.data = fresh;
+            arena.bytes = rounded;
+            arena.generation = ++g_generation;
         }
-        arena.data = fresh;
-        arena.bytes = rounded;
-        arena.generation = ++g_generation;
     }
+    *result = arena;
+    return CGPTX_OK;
+}
+
+int scratch(hipStream_t stream, std::size_t bytes, void** out) {
+    Arena arena;
+    bool capturing = false;
+    hipError_t allocation = hipSuccess;
+    if (int s = grow_arena(stream, bytes, &arena, &capturing, &allocation)) return s;
+    if (capturing)
+        return fail(CGPTX_CAPTURE_ALLOC,
+                    "scratch arena would have to grow during stream capture; run the op once eagerly first");
+    CGPTX_HIP(allocation);
     *out = arena.data;
+    return CGPTX_OK;
+}
+
+int scratch_up_to(hipStream_t stream, std::size_t bytes, void** out, std::size_t* held) {
+    Arena arena;
+    bool capturing = false;
+    hipError_t allocation = hipSuccess;
+    if (int s = grow_arena(stream, bytes, &arena, &capturing, &allocation)) return s;
+    *out = arena.data;
+    *held = arena.bytes;
     return CGPTX_OK;
 }
 

@@ -11,9 +11,11 @@
  * a per-(device, stream) arena that grows on the first eager call with a given
  * problem size. While a stream is being captured into a hipGraph the arena
  * cannot grow: a call that would need more scratch than an earlier eager call
- * reserved returns CGPTX_CAPTURE_ALLOC. Run each op once eagerly before
- * capture, exactly as the reference warms up before cudaStreamBeginCapture
- * (train/train.cpp:545-548).
+ * reserved returns CGPTX_CAPTURE_ALLOC, or is recorded in a slower form where
+ * scratch only makes it faster (padded copies of ragged operands, split-K
+ * partials of contractions other than whole, long ones, shared key blocks).
+ * Run each op once eagerly before capture, exactly as the reference warms up
+ * before cudaStreamBeginCapture (train/train.cpp:545-548).
  *
  * Threading: one host thread per stream, as in the reference.
  */
