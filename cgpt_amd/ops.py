@@ -412,7 +412,6 @@ class AdamWWorkspace:
         capi.call("cgptx_adamw_workspace_create", ctypes.byref(handle))
         self._handle = handle
         self._states = None
-        self._array = None  # the entries as the library takes them, filled anew by each call
 
     def __del__(self):
         try:
@@ -442,9 +441,7 @@ def adamw_step_many_async(entries: Sequence[AdamWBatchEntry], options: AdamWOpti
         for e, s in zip(entries, workspace._states):
             if e.state is not s:
                 raise ValueError(f"{name}: workspace states changed")
-    array = workspace._array
-    if array is None or len(array) != len(entries):
-        array = workspace._array = (capi.AdamWEntry * len(entries))()
+    array = (capi.AdamWEntry * len(entries))()  # of this call alone: the library reads it while other threads run
     if not isinstance(entries, list) or not _adamw_entries(entries, workspace._states, ctypes.addressof(array)):
         for i, e in enumerate(entries):  # another kind of sequence, or something to complain about
             if e.parameter is None or e.gradient is None or e.state is None:
