@@ -83,18 +83,22 @@ Owned tensor_attribute(PyObject* object, PyObject* name) {
     return value;
 }
 
-// adamw_entries(entries, states or None, address of the cgptx_adamw_entry array) -> bool. Fills the array when every
-// entry is what the update takes: device tensors of one dtype and shape per entry, fp32 master copy and moments of that
+// adamw_entries(entries, states or None, address of the cgptx_adamw_entry array, its length) -> bool. Fills the array when
+// there are as many entries (looked at in a copy of the list, which other code may change meanwhile) and every entry is what the update takes: device tensors of one dtype and shape per entry, fp32 master copy and moments of that
 // shape on the same device, and the states that the workspace was bound to. False otherwise (the caller says what is wrong).
 PyObject* adamw_entries(PyObject*, PyObject* const* args, Py_ssize_t count) {
-    if (count != 3 || !PyList_Check(args[0])) Py_RETURN_FALSE;
-    const Py_ssize_t n = PyList_GET_SIZE(args[0]);
+    if (count != 4 || !PyList_Check(args[0])) Py_RETURN_FALSE;
+    const Owned entries(PyList_AsTuple(args[0]));
+    if (entries.object == nullptr) return nullptr;
+    const Py_ssize_t n = PyTuple_GET_SIZE(entries.object);
     PyObject* bound = args[1] == Py_None ? nullptr : args[1];
     if (bound != nullptr && (!PyList_Check(bound) || PyList_GET_SIZE(bound) != n)) Py_RETURN_FALSE;
     auto* out = reinterpret_cast<cgptx_adamw_entry*>(PyLong_AsUnsignedLongLong(args[2]));
+    const Py_ssize_t length = PyLong_AsSsize_t(args[3]);
     if (PyErr_Occurred()) return nullptr;
+    if (length != n) Py_RETURN_FALSE;
     for (Py_ssize_t i = 0; i < n; ++i) {
-        PyObject* entry = PyList_GET_ITEM(args[0], i);
+        PyObject* entry = PyTuple_GET_ITEM(entries.object, i);
         const Owned held_state(PyObject_GetAttr(entry, names.state));
         PyObject* state = held_state.object;
         if (state == nullptr) {

@@ -442,7 +442,7 @@ def adamw_step_many_async(entries: Sequence[AdamWBatchEntry], options: AdamWOpti
             if e.state is not s:
                 raise ValueError(f"{name}: workspace states changed")
     array = (capi.AdamWEntry * len(entries))()  # of this call alone: the library reads it while other threads run
-    if not isinstance(entries, list) or not _adamw_entries(entries, workspace._states, ctypes.addressof(array)):
+    if not isinstance(entries, list) or not _adamw_entries(entries, workspace._states, ctypes.addressof(array), len(array)):
         for i, e in enumerate(entries):  # another kind of sequence, or something to complain about
             if e.parameter is None or e.gradient is None or e.state is None:
                 raise ValueError(f"{name}: null entry")
@@ -453,7 +453,7 @@ def adamw_step_many_async(entries: Sequence[AdamWBatchEntry], options: AdamWOpti
                                        e.state.first_moment.data_ptr(), e.state.second_moment.data_ptr(),
                                        e.parameter.numel(), _code(e.parameter))
     c_options = options.to_c()
-    capi.call("cgptx_adamw_step_many_async", workspace._handle, array, len(entries), ctypes.byref(c_options),
+    capi.call("cgptx_adamw_step_many_async", workspace._handle, array, len(array), ctypes.byref(c_options),
               initial_step, _stream(stream))
     if workspace._states is None:
         workspace._states = [e.state for e in entries]

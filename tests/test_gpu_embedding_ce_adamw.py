@@ -328,3 +328,16 @@ def test_embedding_backward_frequent_ids_bit_exact(device, tokens, hidden, frequ
         ops.embedding_backward(got, dy.to(device), ids.to(torch.int32).to(device), tokens,
                                options=ops.EmbeddingBackwardOptions(accumulate_weight=accumulate))
         assert torch.equal(got.cpu(), base)
+
+
+def test_adamw_entry_list_longer_than_it_says(device):
+    """The entries are written into an array of len(entries): a list with more in it than that (here one that lies, in earnest
+    one that another thread extends) is refused and nothing is written behind the array."""
+    class Short(list):
+        def __len__(self):
+            return 1
+
+    p, g = torch.ones(4, device=device), torch.ones(4, device=device)
+    entry = ops.AdamWBatchEntry(p, g, ops.AdamWState.for_parameter(p))
+    with pytest.raises(IndexError):
+        ops.adamw_step_many_async(Short([entry, entry]), ops.AdamWOptions(), ops.AdamWWorkspace())
