@@ -122,17 +122,18 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
 //     of rank i), lanes across the columns, kAhead token rows in flight.
 //   * Longer ones: one workgroup per id and kSlice columns, so that a frequent id occupies hidden / kSlice
 //     workgroups instead of one wavefront. The segment is put into ascending order through a bitmap of token
-//     positions in LDS, kSpan positions at a time as long as the list of its tokens has room for the whole segment;
-//     all threads fetch the slices of the next kBatch token rows while the first wavefront adds the previous
+//     positions in LDS, kSpan positions at a time, from which the list of the next kList tokens is drawn as often as it
+//     takes; all threads fetch the slices of the next kBatch token rows while the first wavefront adds the previous
 //     ones, one column per lane, from LDS, where it reads 16 tokens ahead of the chain. That is bound by the latency
-//     of add + round.
+//     of add + round. A segment is read once per kSpan tokens of the batch, so its work grows with its tokens up to batches
+//     of millions.
 // Both live in one launch, the long segments' workgroups first. 32768 tokens x 1024 columns, ids Zipf distributed
 // over 32000: 1846 -> 51 us (of which the most frequent id, 6.7 per cent of the tokens, sets the end).
 constexpr unsigned int kShort = 64;      // tokens: one lane each
 constexpr unsigned int kSlice = 64;      // columns of a long segment's workgroup: one lane each, one or two cache lines
 constexpr unsigned int kBatch = 128;     // token rows per step of a long segment
 constexpr unsigned int kSpan = 65536;    // token positions covered by the bitmap at a time
-constexpr unsigned int kList = 4096;     // tokens of the ordered list; longer segments take kList positions at a time
+constexpr unsigned int kList = 4096;     // tokens ordered at a time
 
 template <typename T, bool Vector>
 __device__ __forceinline__ void embedding_short_row(T* __restrict__ row, const T* __restrict__ grad_output,
@@ -207,19 +208,18 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
     using u32x4 = vec_t<unsigned int, 4>;
     constexpr unsigned int kWords = kSpan / 32 / kThreads;  // bitmap words of a thread
     static_assert(kWords % 4 == 0 && kThreads / kWave == kWavesPerBlock, "a thread owns whole 16-byte pieces of the bitmap");
-    const unsigned int window = tokens <= kList ? kSpan : kList;
     const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const unsigned int col = col0 + lane;
     float acc = 0.0f;
     if (wave == 0 && accumulate && col < hidden) acc = to_f32(row[col]);
-    for (unsigned int base = 0; base < count; base += window) {
-        // The window's tokens of this segment in ascending order.
+    for (unsigned int base = 0; base < count; base += kSpan) {
+        // The window's tokens of this segment: a bit per position.
 #pragma unroll
         for (unsigned int i = 0; i < kWords; i += 4) *reinterpret_cast<u32x4*>(&lds.words[tid * kWords + i]) = u32x4(0u);
         __syncthreads();
         for (unsigned int i = tid; i < tokens; i += kThreads) {
             const unsigned int position = segment[i] - base;  // wraps below the window
-            if (position < window) atomicOr(&lds.words[position / 32], 1u << (position % 32));
+            if (position < kSpan) atomicOr(&lds.words[position / 32], 1u << (position % 32));
         }
         __syncthreads();
         unsigned int word[kWords], mine = 0;
@@ -237,67 +237,71 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
         }
         if (lane == kWave - 1) lds.wave_counts[wave] = inclusive;
         __syncthreads();
-        unsigned int slot = inclusive - mine, found = 0;
+        unsigned int slot = inclusive - mine, window = 0;
         for (unsigned int w = 0; w < kWavesPerBlock; ++w) {
             if (w < wave) slot += lds.wave_counts[w];
-            found += lds.wave_counts[w];
+            window += lds.wave_counts[w];
         }
+        for (unsigned int listed = 0; listed < window; listed += kList) {
+            // The next kList of them in ascending order.
+            const unsigned int found = min(kList, window - listed);
 #pragma unroll
-        for (unsigned int i = 0; i < kWords; ++i) {
-            while (word[i] != 0) {
-                lds.list[slot++] = static_cast<unsigned short>((tid * kWords + i) * 32 + __builtin_ctz(word[i]));
-                word[i] &= word[i] - 1;
-            }
-        }
-        __syncthreads();
-        // Loads of the batch that starts at list entry `first`, into registers.
-        chunk_t held[L::kPerThread];
-        auto fetch = [&](unsigned int first) {
-#pragma unroll
-            for (unsigned int u = 0; u < L::kPerThread; ++u) {
-                const unsigned int index = u * kThreads + tid;
-                const unsigned int entry = first + index / L::kChunks, column = col0 + index % L::kChunks * L::kVec;
-                if (entry < found && column < hidden)
-                    held[u] = load_vec<T, static_cast<int>(L::kVec)>(
-                        grad_output + static_cast<std::size_t>(base + lds.list[entry]) * hidden + column);
-            }
-        };
-        fetch(0);
-        for (unsigned int first = 0; first < found; first += kBatch) {
-#pragma unroll
-            for (unsigned int u = 0; u < L::kPerThread; ++u) {
-                const unsigned int index = u * kThreads + tid;
-                store_vec<T, static_cast<int>(L::kVec)>(&lds.rows[index / L::kChunks][index % L::kChunks * L::kVec], held[u]);
-            }
-            __syncthreads();
-            if (first + kBatch < found) fetch(first + kBatch);
-            if (wave == 0) {
-                const unsigned int n = min(kBatch, found - first);
-                T even[16], odd[16];
-                auto read = [&](T(&dy)[16], unsigned int j) {
-                    const unsigned int from = min(j, kBatch - 16);
-#pragma unroll
-                    for (unsigned int u = 0; u < 16; ++u) dy[u] = lds.rows[from + u][lane];
-                };
-                auto add = [&](const T(&dy)[16], unsigned int j) {
-                    if (j + 16 <= n) {
-#pragma unroll
-                        for (unsigned int u = 0; u < 16; ++u) acc = add_rounded<T>(acc, dy[u]);
-                    } else {
-#pragma unroll
-                        for (unsigned int u = 0; u < 16; ++u)
-                            if (j + u < n) acc = add_rounded<T>(acc, dy[u]);
-                    }
-                };
-                read(even, 0);
-                for (unsigned int j = 0; j < n; j += 32) {
-                    read(odd, j + 16);
-                    add(even, j);
-                    read(even, j + 32);
-                    add(odd, j + 16);
+            for (unsigned int i = 0; i < kWords; ++i) {
+                while (word[i] != 0 && slot < listed + kList) {
+                    lds.list[slot++ - listed] = static_cast<unsigned short>((tid * kWords + i) * 32 + __builtin_ctz(word[i]));
+                    word[i] &= word[i] - 1;
                 }
             }
             __syncthreads();
+            // Loads of the batch that starts at list entry `first`, into registers.
+            chunk_t held[L::kPerThread];
+            auto fetch = [&](unsigned int first) {
+#pragma unroll
+                for (unsigned int u = 0; u < L::kPerThread; ++u) {
+                    const unsigned int index = u * kThreads + tid;
+                    const unsigned int entry = first + index / L::kChunks, column = col0 + index % L::kChunks * L::kVec;
+                    if (entry < found && column < hidden)
+                        held[u] = load_vec<T, static_cast<int>(L::kVec)>(
+                            grad_output + static_cast<std::size_t>(base + lds.list[entry]) * hidden + column);
+                }
+            };
+            fetch(0);
+            for (unsigned int first = 0; first < found; first += kBatch) {
+#pragma unroll
+                for (unsigned int u = 0; u < L::kPerThread; ++u) {
+                    const unsigned int index = u * kThreads + tid;
+                    store_vec<T, static_cast<int>(L::kVec)>(&lds.rows[index / L::kChunks][index % L::kChunks * L::kVec], held[u]);
+                }
+                __syncthreads();
+                if (first + kBatch < found) fetch(first + kBatch);
+                if (wave == 0) {
+                    const unsigned int n = min(kBatch, found - first);
+                    T even[16], odd[16];
+                    auto read = [&](T(&dy)[16], unsigned int j) {
+                        const unsigned int from = min(j, kBatch - 16);
+#pragma unroll
+                        for (unsigned int u = 0; u < 16; ++u) dy[u] = lds.rows[from + u][lane];
+                    };
+                    auto add = [&](const T(&dy)[16], unsigned int j) {
+                        if (j + 16 <= n) {
+#pragma unroll
+                            for (unsigned int u = 0; u < 16; ++u) acc = add_rounded<T>(acc, dy[u]);
+                        } else {
+#pragma unroll
+                            for (unsigned int u = 0; u < 16; ++u)
+                                if (j + u < n) acc = add_rounded<T>(acc, dy[u]);
+                        }
+                    };
+                    read(even, 0);
+                    for (unsigned int j = 0; j < n; j += 32) {
+                        read(odd, j + 16);
+                        add(even, j);
+                        read(even, j + 32);
+                        add(odd, j + 16);
+                    }
+                }
+                __syncthreads();
+            }
         }
     }
     if (wave == 0 && col < hidden) row[col] = from_f32<T>(acc);

@@ -307,7 +307,7 @@ def test_adamw_matches_cpu_restatement_single_tensor(device):
 @pytest.mark.parametrize("tokens,hidden,frequent", [
     (64, 64, 64), (65, 64, 65),            # the longest segment of one wavefront, the shortest of a workgroup
     (300, 72, 129), (300, 33, 130),        # one row past a batch of 128; a partial and an unaligned slice of columns
-    (4200, 128, 4097), (9000, 96, 8000),     # segments over two and three windows of 4096 positions
+    (4200, 128, 4097), (9000, 96, 8000),     # more tokens than are ordered at a time
 ])
 def test_embedding_backward_frequent_ids_bit_exact(device, tokens, hidden, frequent, dtype):
     """Ids that take a large share of the batch, between other ids and ids past the vocabulary."""
@@ -341,3 +341,42 @@ def test_adamw_entry_list_longer_than_it_says(device):
     entry = ops.AdamWBatchEntry(p, g, ops.AdamWState.for_parameter(p))
     with pytest.raises(IndexError):
         ops.adamw_step_many_async(Short([entry, entry]), ops.AdamWOptions(), ops.AdamWWorkspace())
+
+
+def _added_in_token_order(ids, dy, table, accumulate):
+    """Row by row what the scatter promises: additions in token order, each rounded to the storage type."""
+    out = table.clone() if accumulate else torch.zeros_like(table)
+    order = torch.sort(ids, stable=True).indices
+    ids_sorted, rows = ids[order], dy[order].float()
+    starts = torch.cat([torch.zeros(1, dtype=torch.long), (ids_sorted[1:] != ids_sorted[:-1]).nonzero().flatten() + 1, torch.tensor([len(ids)])])
+    lengths, first = starts[1:] - starts[:-1], starts[:-1]
+    segment_ids = ids_sorted[first]
+    keep = segment_ids < len(table)
+    lengths, first, segment_ids = lengths[keep], first[keep], segment_ids[keep]
+    acc = out[segment_ids].float()
+    for k in range(int(lengths.max())):  # the k-th token of every segment that has one
+        live = lengths > k
+        acc[live] = (acc[live] + rows[first[live] + k]).to(dy.dtype).float()
+    out[segment_ids] = acc.to(dy.dtype)
+    return out
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("tokens,vocab,hidden,frequent", [
+    (70000, 9, 8, {4: 20000, 7: 9000}),                               # two windows of positions, several lists in each
+    (66000, 5000, 7, {17: 8192, 18: 4096}),                           # whole lists
+])
+def test_embedding_backward_splits_bit_exact(device, tokens, vocab, hidden, frequent, dtype):
+    """Where the ordering of long segments changes over."""
+    g = torch.Generator().manual_seed(tokens + vocab)
+    ids = torch.randint(0, vocab + 2, (tokens,), generator=g)
+    where = torch.randperm(tokens, generator=g)
+    for id, count in frequent.items():
+        ids[where[:count]] = id
+        where = where[count:]
+    dy, table = randn((tokens, hidden), dtype, 3), randn((vocab, hidden), dtype, 4)
+    d_ids, d_dy = ids.to(torch.int32).to(device), dy.to(device)
+    for accumulate in (False, True):
+        got = table.to(device)
+        ops.embedding_backward(got, d_dy, d_ids, tokens, options=ops.EmbeddingBackwardOptions(accumulate_weight=accumulate))
+        assert torch.equal(got.cpu(), _added_in_token_order(ids, dy, table, accumulate))
