@@ -28,10 +28,15 @@ constexpr int kWavesPerBlock = kThreads / kWave;
 // no workgroup waits for another); after an exclusive scan of the histogram it hands every token of its range
 // the next free slot of its id's segment. Slots are handed out with LDS integer atomics, so the order inside a
 // segment is whatever order the lanes arrived in: the row kernel puts each segment into ascending order itself.
+// A segment of more than kShort tokens contains positions that are multiples of kShort; order's entries there are marked,
+// which is how the row kernel finds the long segments, and the offset of a workgroup's first id is marked if there is one
+// among its ids, which is how it finds out that it need not look.
 // offsets[id] .. offsets[id + 1] is id's segment of `order`; ids >= vocab belong to nobody and are skipped.
 constexpr int kGroupThreads = 1024;
 constexpr unsigned int kGroupMaxIds = 32768;  // LDS histogram entries of one workgroup (128 KiB)
 constexpr int kGroupBatch = 8;                // 128-bit id loads a thread keeps in flight
+constexpr unsigned int kShort = 64;           // tokens of a segment that one wavefront orders in registers: one lane each
+constexpr unsigned int kLong = 1u << 31;      // the mark of longer segments; positions and tokens stay below it
 
 // The id list is walked in batches of kGroupBatch x 4 ids per thread, all of a batch's loads requested before the
 // first id is looked at (one dependent load per id would cost a memory round trip each). visit(id, t) sees every
@@ -88,7 +93,11 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
     const unsigned int per = (width + kGroupThreads - 1) / kGroupThreads;
     const unsigned int first = min(tid * per, width), last = min(first + per, width);
     unsigned int mine = 0;
-    for (unsigned int i = first; i < last; ++i) mine += bins[i];
+    bool any_long = false;
+    for (unsigned int i = first; i < last; ++i) {
+        mine += bins[i];
+        any_long = any_long || bins[i] > kShort;
+    }
     unsigned int inclusive = mine;
 #pragma unroll
     for (int offset = 1; offset < kWave; offset <<= 1) {
@@ -96,20 +105,23 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
         if (lane >= static_cast<unsigned int>(offset)) inclusive += other;
     }
     if (lane == kWave - 1) wave_totals[wave] = inclusive;
-    __syncthreads();
+    any_long = __syncthreads_or(any_long);
     unsigned int before = smaller_total;
     for (unsigned int w = 0; w < wave; ++w) before += wave_totals[w];
     unsigned int running = before + inclusive - mine;
     for (unsigned int i = first; i < last; ++i) {
         const unsigned int n = bins[i];
-        bins[i] = running;
-        offsets[lo + i] = running;
+        bins[i] = n > kShort ? running | kLong : running;
+        offsets[lo + i] = i == 0 && any_long ? running | kLong : running;
         running += n;
     }
     if (lo + width == vocab && tid == kGroupThreads - 1) offsets[vocab] = running;  // the piece that ends the last range
     __syncthreads();
     for_each_id(ids, count, aligned, [&](unsigned int id, unsigned int t) {
-        if (id >= lo && id - lo < width) order[atomicAdd(&bins[id - lo], 1u)] = t;
+        if (id >= lo && id - lo < width) {
+            const unsigned int slot = atomicAdd(&bins[id - lo], 1u);
+            order[slot & ~kLong] = slot % kShort == 0 ? t | (slot & kLong) : t;
+        }
     });
 }
 
@@ -119,26 +131,31 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
 // is accumulated. Bound by HBM (three rows per token) as long as the serial chain of additions of the most
 // frequent id is short; text makes it long: the first ids of a vocabulary take several per cent of a batch each.
 //   * Segments of up to kShort tokens: one wavefront per id, tokens ordered in registers (lane i holds the token
-//     of rank i), lanes across the columns, kAhead token rows in flight.
+//     of rank i), lanes across the columns, kAhead token rows in flight. With few tokens an id it is the chain of
+//     loads that counts (offsets, token, row) and the wavefronts that are in flight against it: a wavefront takes two
+//     ids, half a vocabulary apart, and looks both up before it adds either.
 //   * Longer ones: one workgroup per id and kSlice columns, so that a frequent id occupies hidden / kSlice
 //     workgroups instead of one wavefront. The segment is put into ascending order through a bitmap of token
 //     positions in LDS, kSpan positions at a time, from which the list of the next kList tokens is drawn as often as it
-//     takes; all threads fetch the slices of the next kBatch token rows while the first wavefront adds the previous
-//     ones, one column per lane, from LDS, where it reads 16 tokens ahead of the chain. That is bound by the latency
-//     of add + round. A segment is read once per kSpan tokens of the batch, so its work grows with its tokens up to batches
-//     of millions.
-// Both live in one launch, the long segments' workgroups first. 32768 tokens x 1024 columns, ids Zipf distributed
-// over 32000: 1846 -> 51 us (of which the most frequent id, 6.7 per cent of the tokens, sets the end).
-constexpr unsigned int kShort = 64;      // tokens: one lane each
+//     takes; all threads fetch the slices of the next kBatch token rows while the first wavefront adds the
+//     previous ones, one column per lane, from LDS, where it reads kReadAhead tokens ahead of the chain. A batch of 128
+//     bf16 rows takes 3600 clocks, 2700 of them in the chain (add, round, and the reads beside them).
+// Both live in one launch, the long segments' workgroups first: the chains of the frequent ids run beside the short
+// segments (in a launch of their own they add their 50 us). So the short segments pay for the long ones' registers and LDS
+// with wavefronts in flight, which is why both are bounded (LongRow::kWavesPerSimd) and why nothing is listed where the
+// grouping found no long segment. 32768 tokens x 1024 columns in bf16 over 32000 ids, all launches: uniform ids 36 us, ids Zipf
+// distributed 64, of which the most frequent id, 9.3 per cent of the tokens, sets the end (every id by one wavefront 35 and
+// 2300; neither bounded nor told that there is nothing to list 48 and 75). A segment is read once per kSpan tokens of the batch,
+// so its work grows with its tokens up to batches of millions: 131072 of 262144 tokens in one id, 128 columns, 2.1 ms
+// (read once per 4096 tokens: 7.0).
 constexpr unsigned int kSlice = 64;      // columns of a long segment's workgroup: one lane each, one or two cache lines
-constexpr unsigned int kBatch = 128;     // token rows per step of a long segment
 constexpr unsigned int kSpan = 65536;    // token positions covered by the bitmap at a time
 constexpr unsigned int kList = 4096;     // tokens ordered at a time
 
 template <typename T, bool Vector>
 __device__ __forceinline__ void embedding_short_row(T* __restrict__ row, const T* __restrict__ grad_output,
-                                                    const unsigned int* __restrict__ segment, unsigned int tokens,
-                                                    unsigned int hidden, bool accumulate) {
+                                                    unsigned int mine, unsigned int tokens, unsigned int hidden,
+                                                    bool accumulate) {
     constexpr int VEC = Vector ? kVec128<T> : 1;
     constexpr unsigned int kAhead = 8;
     using vec_f = vec_t<float, VEC>;
@@ -148,7 +165,6 @@ __device__ __forceinline__ void embedding_short_row(T* __restrict__ row, const T
             for (unsigned int col = lane * VEC; col < hidden; col += kWave * VEC) store_vec<T, VEC>(row + col, vec_t<T, VEC>(0));
         return;
     }
-    const unsigned int mine = lane < tokens ? segment[lane] : 0xFFFFFFFFu;
     // rank = number of tokens of the segment below mine; sorted = the token of rank `lane`.
     unsigned int rank = 0;
     for (unsigned int j = 0; j < tokens; ++j)
@@ -176,6 +192,20 @@ __device__ __forceinline__ void embedding_short_row(T* __restrict__ row, const T
     }
 }
 
+// An element as it comes from LDS, in a register of its own.
+template <typename T>
+using raw_t = std::conditional_t<sizeof(T) == 2, unsigned int, float>;
+template <typename T>
+__device__ __forceinline__ raw_t<T> to_raw(T x) {
+    if constexpr (sizeof(T) == 2) return __builtin_bit_cast(unsigned short, x);
+    else return x;
+}
+template <typename T>
+__device__ __forceinline__ T from_raw(raw_t<T> x) {
+    if constexpr (sizeof(T) == 2) return __builtin_bit_cast(T, static_cast<unsigned short>(x));
+    else return x;
+}
+
 // acc + x rounded to T and widened again. bf16: rounding into the upper half of a register whose lower half is zero is the
 // widened value already, one instruction less in the chain.
 template <typename T>
@@ -187,15 +217,23 @@ __device__ __forceinline__ float add_rounded(float acc, T x) {
 
 template <typename T, bool Vector>
 struct LongRow {
-    static constexpr unsigned int kVec = Vector ? kVec128<T> : 1;
-    static constexpr unsigned int kChunks = kSlice / kVec;                    // loads per token and slice
-    static constexpr unsigned int kPerThread = kBatch * kChunks / kThreads;   // loads per thread and batch
+    static constexpr unsigned int kBatch = Vector ? (sizeof(T) == 2 ? 128 : 96) : 64;  // token rows per step
+    static constexpr unsigned int kReadAhead = Vector ? 16 : 8;  // of them that the first wavefront reads from LDS ahead of its chain
+    static constexpr unsigned int kVec = Vector ? kVec128<T> : 1;  // elements of a load
+    static constexpr unsigned int kChunks = kSlice / kVec;
+    static constexpr unsigned int kRows = kThreads / kChunks;                   // token rows of a load by all threads
+    static constexpr unsigned int kPerThread = kBatch / kRows;
+    static constexpr int kWavesPerSimd = Vector ? (sizeof(T) == 2 ? 5 : 4) : 6;  // that the launch keeps in flight
     struct Shared {
-        alignas(16) T rows[kBatch][kSlice];
-        alignas(16) unsigned int words[kSpan / 32];
-        unsigned short list[kList];              // token positions of the window, ascending, relative to its start
+        union {
+            alignas(16) T rows[kBatch][kSlice];
+            alignas(16) unsigned int words[kSpan / 32];  // until the list is there
+        };
+        unsigned short list[kList];  // token positions, ascending, relative to the window's start
         unsigned int wave_counts[kWavesPerBlock];
+        unsigned int long_ids[kThreads], wave_longs[kWavesPerBlock];
     };
+    static_assert(kThreads == 4 * kWave && sizeof(Shared) <= 160 * 1024 / kWavesPerSimd, "a workgroup is one wavefront per SIMD");
 };
 
 template <typename T, bool Vector>
@@ -208,8 +246,12 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
     using u32x4 = vec_t<unsigned int, 4>;
     constexpr unsigned int kWords = kSpan / 32 / kThreads;  // bitmap words of a thread
     static_assert(kWords % 4 == 0 && kThreads / kWave == kWavesPerBlock, "a thread owns whole 16-byte pieces of the bitmap");
-    const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    unsigned int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // what follows from it is computed per item, not held in registers over all of them
+    const unsigned int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const unsigned int col = col0 + lane;
+    // Of a load's rows and chunks this thread takes row `mine` and the chunk at `column`.
+    const unsigned int mine = tid / L::kChunks, column = col0 + tid % L::kChunks * L::kVec;
     float acc = 0.0f;
     if (wave == 0 && accumulate && col < hidden) acc = to_f32(row[col]);
     for (unsigned int base = 0; base < count; base += kSpan) {
@@ -217,19 +259,24 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
 #pragma unroll
         for (unsigned int i = 0; i < kWords; i += 4) *reinterpret_cast<u32x4*>(&lds.words[tid * kWords + i]) = u32x4(0u);
         __syncthreads();
-        for (unsigned int i = tid; i < tokens; i += kThreads) {
-            const unsigned int position = segment[i] - base;  // wraps below the window
-            if (position < kSpan) atomicOr(&lds.words[position / 32], 1u << (position % 32));
+        for (unsigned int i0 = 0; i0 < tokens; i0 += 4 * kThreads) {
+            unsigned int position[4];  // four loads in flight, none behind a branch
+#pragma unroll
+            for (unsigned int u = 0; u < 4; ++u)
+                position[u] = (segment[min(i0 + u * kThreads + tid, tokens - 1)] & ~kLong) - base;  // wraps below the window
+#pragma unroll
+            for (unsigned int u = 0; u < 4; ++u)
+                if (i0 + u * kThreads + tid < tokens && position[u] < kSpan) atomicOr(&lds.words[position[u] / 32], 1u << (position[u] % 32));
         }
         __syncthreads();
-        unsigned int word[kWords], mine = 0;
+        unsigned int word[kWords], found = 0;
 #pragma unroll
         for (unsigned int i = 0; i < kWords; i += 4) {
             const u32x4 four = *reinterpret_cast<const u32x4*>(&lds.words[tid * kWords + i]);
 #pragma unroll
-            for (unsigned int e = 0; e < 4; ++e) mine += __popc(word[i + e] = four[e]);
+            for (unsigned int e = 0; e < 4; ++e) found += __popc(word[i + e] = four[e]);
         }
-        unsigned int inclusive = mine;
+        unsigned int inclusive = found;
 #pragma unroll
         for (int offset = 1; offset < kWave; offset <<= 1) {
             const unsigned int other = __shfl_up(inclusive, offset, kWave);
@@ -237,14 +284,15 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
         }
         if (lane == kWave - 1) lds.wave_counts[wave] = inclusive;
         __syncthreads();
-        unsigned int slot = inclusive - mine, window = 0;
+        unsigned int slot = inclusive - found, window = 0;
         for (unsigned int w = 0; w < kWavesPerBlock; ++w) {
             if (w < wave) slot += lds.wave_counts[w];
             window += lds.wave_counts[w];
         }
+        window = __builtin_amdgcn_readfirstlane(window);  // the same in all lanes: what follows branches without masks
         for (unsigned int listed = 0; listed < window; listed += kList) {
             // The next kList of them in ascending order.
-            const unsigned int found = min(kList, window - listed);
+            const unsigned int entries = min(kList, window - listed);
 #pragma unroll
             for (unsigned int i = 0; i < kWords; ++i) {
                 while (word[i] != 0 && slot < listed + kList) {
@@ -253,51 +301,60 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
                 }
             }
             __syncthreads();
-            // Loads of the batch that starts at list entry `first`, into registers.
+            // The batch that starts at list entry `first`, into registers. The loads carry no condition (past the end they
+            // read the last entry's row and the last columns): a branch around each would make it wait for the one before.
             chunk_t held[L::kPerThread];
-            auto fetch = [&](unsigned int first) {
+            auto fetch = [&](unsigned int first) __attribute__((always_inline)) {
+                unsigned int token[L::kPerThread];
+#pragma unroll
+                for (unsigned int u = 0; u < L::kPerThread; ++u)
+                    token[u] = base + lds.list[min(first + u * L::kRows + mine, entries - 1)];
 #pragma unroll
                 for (unsigned int u = 0; u < L::kPerThread; ++u) {
-                    const unsigned int index = u * kThreads + tid;
-                    const unsigned int entry = first + index / L::kChunks, column = col0 + index % L::kChunks * L::kVec;
-                    if (entry < found && column < hidden)
-                        held[u] = load_vec<T, static_cast<int>(L::kVec)>(
-                            grad_output + static_cast<std::size_t>(base + lds.list[entry]) * hidden + column);
+                    const T* at = grad_output + static_cast<std::size_t>(token[u]) * hidden;
+                    held[u] = load_vec<T, static_cast<int>(L::kVec)>(at + min(column, hidden - L::kVec));
                 }
             };
             fetch(0);
-            for (unsigned int first = 0; first < found; first += kBatch) {
+            for (unsigned int first = 0; first < entries; first += L::kBatch) {
 #pragma unroll
-                for (unsigned int u = 0; u < L::kPerThread; ++u) {
-                    const unsigned int index = u * kThreads + tid;
-                    store_vec<T, static_cast<int>(L::kVec)>(&lds.rows[index / L::kChunks][index % L::kChunks * L::kVec], held[u]);
-                }
+                for (unsigned int u = 0; u < L::kPerThread; ++u)
+                    store_vec<T, static_cast<int>(L::kVec)>(&lds.rows[u * L::kRows + mine][column - col0], held[u]);
                 __syncthreads();
-                if (first + kBatch < found) fetch(first + kBatch);
+                fetch(first + L::kBatch);
                 if (wave == 0) {
-                    const unsigned int n = min(kBatch, found - first);
-                    T even[16], odd[16];
-                    auto read = [&](T(&dy)[16], unsigned int j) {
-                        const unsigned int from = min(j, kBatch - 16);
+                    const unsigned int n = min(L::kBatch, entries - first);
+                    raw_t<T> even[L::kReadAhead], odd[L::kReadAhead];
+                    auto read = [&](raw_t<T>(&dy)[L::kReadAhead], unsigned int j) __attribute__((always_inline)) {
+                        const unsigned int from = min(j, L::kBatch - L::kReadAhead);
 #pragma unroll
-                        for (unsigned int u = 0; u < 16; ++u) dy[u] = lds.rows[from + u][lane];
+                        for (unsigned int u = 0; u < L::kReadAhead; ++u) dy[u] = to_raw<T>(lds.rows[from + u][lane]);
+                        __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the additions that do not need them
                     };
-                    auto add = [&](const T(&dy)[16], unsigned int j) {
-                        if (j + 16 <= n) {
+                    auto add = [&](const raw_t<T>(&dy)[L::kReadAhead]) __attribute__((always_inline)) {
 #pragma unroll
-                            for (unsigned int u = 0; u < 16; ++u) acc = add_rounded<T>(acc, dy[u]);
-                        } else {
-#pragma unroll
-                            for (unsigned int u = 0; u < 16; ++u)
-                                if (j + u < n) acc = add_rounded<T>(acc, dy[u]);
-                        }
+                        for (unsigned int u = 0; u < L::kReadAhead; ++u) acc = add_rounded<T>(acc, from_raw<T>(dy[u]));
+                        __builtin_amdgcn_sched_barrier(0);
                     };
+                    unsigned int j = 0;
                     read(even, 0);
-                    for (unsigned int j = 0; j < n; j += 32) {
-                        read(odd, j + 16);
-                        add(even, j);
-                        read(even, j + 32);
-                        add(odd, j + 16);
+                    for (; j + 2 * L::kReadAhead <= n; j += 2 * L::kReadAhead) {
+                        read(odd, j + L::kReadAhead);
+                        add(even);
+                        read(even, j + 2 * L::kReadAhead);
+                        add(odd);
+                    }
+                    if (j < n) {  // the last batch's last rows
+                        if (j + L::kReadAhead <= n) {
+                            read(odd, j + L::kReadAhead);
+                            add(even);
+#pragma unroll
+                            for (unsigned int u = 0; u < L::kReadAhead; ++u) even[u] = odd[u];
+                            j += L::kReadAhead;
+                        }
+#pragma unroll
+                        for (unsigned int u = 0; u < L::kReadAhead; ++u)
+                            if (j + u < n) acc = add_rounded<T>(acc, from_raw<T>(even[u]));
                     }
                 }
                 __syncthreads();
@@ -307,51 +364,63 @@ __device__ __forceinline__ void embedding_long_row(typename LongRow<T, Vector>::
     if (wave == 0 && col < hidden) row[col] = from_f32<T>(acc);
 }
 
-// Workgroups [0, long_groups): long segments. A segment of more than kShort = 64 tokens contains a position of
-// `order` that is a multiple of 64; the first one in it names the segment, so candidate j is the id of the token at
-// position 64 j if that id's segment is long and 64 j its first multiple. Each of these workgroups lists the long
-// ids itself, one candidate per thread at a time, and takes every long_groups-th (id, slice) of the list: a workgroup
-// for every candidate and slice would mostly find that there is nothing to do, after four dependent loads
-// (with the wider bitmap and the shorter chain 64 -> 51 us). The remaining workgroups take kWavesPerBlock ids each and leave the long ones out.
+// Tokens of an id's segment; *begin: where it starts in `order`.
+__device__ __forceinline__ unsigned int segment_of(const unsigned int* __restrict__ offsets, unsigned int id, unsigned int* begin) {
+    *begin = offsets[id] & ~kLong;
+    return (offsets[id + 1] & ~kLong) - *begin;
+}
+
+// Workgroups [0, long_groups): long segments. Each lists the long ids itself, one mark per thread at a time, and takes every
+// long_groups-th (id, slice) of the list: a workgroup for every mark and slice would mostly find that there is nothing to do.
+// The remaining ones are wavefronts [0, row_waves) for the ids below row_waves and the ids row_waves further on; they leave
+// the long ones out.
 template <typename T, bool Vector>
-__global__ __launch_bounds__(kThreads) void embedding_rows_kernel(T* __restrict__ grad_weight,
-                                                                 const T* __restrict__ grad_output,
-                                                                 const std::uint32_t* __restrict__ ids,
-                                                                 const unsigned int* __restrict__ offsets,
-                                                                 const unsigned int* __restrict__ order,
-                                                                 unsigned int count, unsigned int vocab,
-                                                                 unsigned int hidden, unsigned int slices,
-                                                                 unsigned int long_groups, bool accumulate) {
-    __shared__ typename LongRow<T, Vector>::Shared lds;
-    __shared__ unsigned int long_ids[kThreads], wave_longs[kWavesPerBlock];
+__global__ __launch_bounds__(kThreads, (LongRow<T, Vector>::kWavesPerSimd)) void embedding_rows_kernel(
+                                                                    T* __restrict__ grad_weight,
+                                                                    const T* __restrict__ grad_output,
+                                                                    const std::uint32_t* __restrict__ ids,
+                                                                    const unsigned int* __restrict__ offsets,
+                                                                    const unsigned int* __restrict__ order,
+                                                                    unsigned int count, unsigned int vocab,
+                                                                    unsigned int hidden, unsigned int slices,
+                                                                    unsigned int long_groups, unsigned int ids_per_group, unsigned int row_waves,
+                                                                    bool accumulate) {
     if (blockIdx.x < long_groups) {
+        __shared__ typename LongRow<T, Vector>::Shared lds;
         const unsigned int tid = threadIdx.x, wave = tid / kWave;
+        if (count > kThreads * kShort) {  // fewer tokens: one look at the marks says as much
+            bool any_long = false;
+            for (unsigned int group = tid; group < (vocab + ids_per_group - 1) / ids_per_group; group += kThreads)
+                any_long = any_long || (offsets[group * ids_per_group] & kLong) != 0;
+            if (!__syncthreads_or(any_long)) return;
+        }
         const unsigned int placed = offsets[vocab];  // ids past the vocabulary have no place in `order`
-        const unsigned int candidates = (placed + kShort - 1) / kShort;
-        unsigned int next_item = blockIdx.x;  // among the items of the candidates from `first` on
-        for (unsigned int first = 0; first < candidates; first += kThreads) {
+        unsigned int next_item = blockIdx.x;  // among the items of the marks from `first` on
+        for (unsigned int first = 0; first * kShort < count; first += kThreads) {
             const unsigned int position = (first + tid) * kShort;
+            const unsigned int token = position < count ? order[position] : 0;  // read beside `placed`, not after it
             unsigned int id = 0;
-            bool is_long = false;
-            if (first + tid < candidates) {
-                id = ids[order[position]];
-                const unsigned int begin = offsets[id];
-                is_long = offsets[id + 1] - begin > kShort && position - begin < kShort;
+            bool is_long = position < placed && (token & kLong) != 0;
+            if (is_long) {  // the segment's first mark names it
+                id = ids[token & ~kLong];
+                is_long = position - (offsets[id] & ~kLong) < kShort;
             }
             const unsigned long long mask = __ballot(is_long);
-            if ((tid & (kWave - 1)) == 0) wave_longs[wave] = __popcll(mask);
+            if ((tid & (kWave - 1)) == 0) lds.wave_longs[wave] = __popcll(mask);
             __syncthreads();
             unsigned int slot = __popcll(mask & ((1ull << (tid & (kWave - 1))) - 1)), found = 0;
             for (unsigned int w = 0; w < kWavesPerBlock; ++w) {
-                if (w < wave) slot += wave_longs[w];
-                found += wave_longs[w];
+                if (w < wave) slot += lds.wave_longs[w];
+                found += lds.wave_longs[w];
             }
-            if (is_long) long_ids[slot] = id;
+            found = __builtin_amdgcn_readfirstlane(found);
+            if (is_long) lds.long_ids[slot] = id;
             __syncthreads();
             const unsigned int items = found * slices;
             for (; next_item < items; next_item += long_groups) {
-                const unsigned int entry = next_item / slices, row = long_ids[entry];
-                const unsigned int begin = offsets[row], tokens = offsets[row + 1] - begin;
+                const unsigned int entry = next_item / slices, row = __builtin_amdgcn_readfirstlane(lds.long_ids[entry]);
+                unsigned int begin;
+                const unsigned int tokens = segment_of(offsets, row, &begin);
                 embedding_long_row<T, Vector>(lds, grad_weight + static_cast<std::size_t>(row) * hidden, grad_output, order + begin,
                                               tokens, count, (next_item - entry * slices) * kSlice, hidden, accumulate);
             }
@@ -360,12 +429,20 @@ __global__ __launch_bounds__(kThreads) void embedding_rows_kernel(T* __restrict_
         }
         return;
     }
-    const unsigned int id = (blockIdx.x - long_groups) * kWavesPerBlock + threadIdx.x / kWave;
-    if (id >= vocab) return;
-    const unsigned int begin = offsets[id], tokens = offsets[id + 1] - begin;
-    if (tokens <= kShort)
-        embedding_short_row<T, Vector>(grad_weight + static_cast<std::size_t>(id) * hidden, grad_output, order + begin, tokens,
-                                       hidden, accumulate);
+    // The same for the whole wavefront, and known to be: the loads of a segment's rows then sit behind scalar branches, which
+    // wait for nothing.
+    const unsigned int first = (blockIdx.x - long_groups) * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (first >= row_waves) return;
+    const unsigned int lane = threadIdx.x & (kWave - 1), second = first + row_waves;
+    unsigned int begin0, begin1 = 0;
+    const unsigned int tokens0 = segment_of(offsets, first, &begin0);
+    const unsigned int tokens1 = second < vocab ? segment_of(offsets, second, &begin1) : kShort + 1;
+    const unsigned int mine0 = tokens0 <= kShort && lane < tokens0 ? order[begin0 + lane] : 0xFFFFFFFFu;
+    const unsigned int mine1 = tokens1 <= kShort && lane < tokens1 ? order[begin1 + lane] : 0xFFFFFFFFu;
+    if (tokens0 <= kShort)
+        embedding_short_row<T, Vector>(grad_weight + static_cast<std::size_t>(first) * hidden, grad_output, mine0, tokens0, hidden, accumulate);
+    if (tokens1 <= kShort)
+        embedding_short_row<T, Vector>(grad_weight + static_cast<std::size_t>(second) * hidden, grad_output, mine1, tokens1, hidden, accumulate);
 }
 
 template <typename T, bool Vector>
@@ -443,13 +520,17 @@ extern "C" int cgptx_embedding_backward(void* grad_weight, const void* grad_outp
         const std::size_t slices = (hidden + kSlice - 1) / kSlice;
         const std::size_t long_groups =
             std::min<std::size_t>(token_count / (kShort + 1) * slices, static_cast<std::size_t>(compute_units()) * 4);
-        const std::size_t short_groups = (vocab + kWavesPerBlock - 1) / kWavesPerBlock;
+        // Two ids a wavefront unless one each find a place on the chip together (300 tokens over 1000 ids: 7.9 us, with two 8.6;
+        // 2048 over 32000: 16.8, with one 17.6).
+        const std::size_t row_waves = vocab <= static_cast<std::size_t>(compute_units()) * 16 ? vocab : (vocab + 1) / 2;
+        const std::size_t short_groups = (row_waves + kWavesPerBlock - 1) / kWavesPerBlock;
         if (long_groups + short_groups > static_cast<std::size_t>(std::numeric_limits<int>::max()))
             return fail(CGPTX_OVERFLOW, std::string(name) + ": too many workgroups");
         const dim3 grid(static_cast<unsigned int>(long_groups + short_groups));
         auto kernel = vector_ok ? embedding_rows_kernel<T, true> : embedding_rows_kernel<T, false>;
         hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, dw, dy, token_ids, offsets, order, count, v, h,
-                           static_cast<unsigned int>(slices), static_cast<unsigned int>(long_groups), accumulate_weight != 0);
+                           static_cast<unsigned int>(slices), static_cast<unsigned int>(long_groups), ids_per_group,
+                           static_cast<unsigned int>(row_waves), accumulate_weight != 0);
         CGPTX_LAUNCH_CHECK();
         return CGPTX_OK;
     });

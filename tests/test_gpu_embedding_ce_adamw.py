@@ -307,6 +307,7 @@ def test_adamw_matches_cpu_restatement_single_tensor(device):
 @pytest.mark.parametrize("tokens,hidden,frequent", [
     (64, 64, 64), (65, 64, 65),            # the longest segment of one wavefront, the shortest of a workgroup
     (300, 72, 129), (300, 33, 130),        # one row past a batch of 128; a partial and an unaligned slice of columns
+    (200, 64, 97), (200, 40, 159), (200, 31, 71),  # past the batches of 96 and 64 rows, and up to one row short of 160
     (4200, 128, 4097), (9000, 96, 8000),     # more tokens than are ordered at a time
 ])
 def test_embedding_backward_frequent_ids_bit_exact(device, tokens, hidden, frequent, dtype):
@@ -363,11 +364,16 @@ def _added_in_token_order(ids, dy, table, accumulate):
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
 @pytest.mark.parametrize("tokens,vocab,hidden,frequent", [
+    (5000, 4096, 8, {}), (5000, 4097, 8, {}), (5000, 4098, 7, {}),  # one id per wavefront, two, and an odd number of them
+    (5000, 4099, 8, {4098: 70, 2048: 66, 2049: 65, 0: 80}),          # long and short ids in one wavefront
+    (16384, 3000, 8, {2999: 100}), (16448, 3000, 8, {2999: 100}),    # 256 positions to look at for long ids, and one more
+    (20000, 3000, 9, {5: 90, 1024: 65, 2999: 300}),                   # some in every workgroup of the grouping
+    (20000, 3000, 8, {1500: 300}),                                    # in the middle one only
     (70000, 9, 8, {4: 20000, 7: 9000}),                               # two windows of positions, several lists in each
     (66000, 5000, 7, {17: 8192, 18: 4096}),                           # whole lists
 ])
 def test_embedding_backward_splits_bit_exact(device, tokens, vocab, hidden, frequent, dtype):
-    """Where the ordering of long segments changes over."""
+    """Where the grouping's marks, the row kernel's wavefronts and the ordering of long segments change over."""
     g = torch.Generator().manual_seed(tokens + vocab)
     ids = torch.randint(0, vocab + 2, (tokens,), generator=g)
     where = torch.randperm(tokens, generator=g)
@@ -380,3 +386,15 @@ def test_embedding_backward_splits_bit_exact(device, tokens, vocab, hidden, freq
         got = table.to(device)
         ops.embedding_backward(got, d_dy, d_ids, tokens, options=ops.EmbeddingBackwardOptions(accumulate_weight=accumulate))
         assert torch.equal(got.cpu(), _added_in_token_order(ids, dy, table, accumulate))
+
+
+def test_embedding_backward_keeps_non_finite_rows_to_their_ids(device):
+    """Long segments read past their last token's row into the same row again: nothing of it is added."""
+    ids = torch.arange(1000) % 3
+    for hidden in (64, 33):
+        dy = randn((1000, hidden), torch.float32, 3)
+        dy[999] = float("inf")  # id 0
+        got = torch.empty(3, hidden, device=device)
+        ops.embedding_backward(got, dy.to(device), ids.to(torch.int32).to(device), 1000)
+        want = _added_in_token_order(ids, dy, torch.zeros(3, hidden), False)
+        assert torch.equal(got.cpu(), want) and torch.isfinite(got[1:]).all() and torch.isinf(got[0]).all()
