@@ -56,14 +56,14 @@ namespace {
 
 // LDS stages of a block: one being multiplied, one being refilled, the rest in flight. 256x256
 // blocks own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each).
-constexpr int stages_for(int /*bm*/, int /*bn*/) { return 5; }
+constexpr int kLdsStages = 5;
 
 template <typename T, int BM, int BN, bool A_K, bool B_K>
 struct TileLayout {
     using ATile = std::conditional_t<A_K, KTile<T, BM>, NTile<T, BM>>;
     using BTile = std::conditional_t<B_K, KTile<T, BN>, NTile<T, BN>>;
     static constexpr int kStage = ATile::kElems + BTile::kElems;  // elements per LDS stage: [A | B]
-    static constexpr int kStages = stages_for(BM, BN);
+    static constexpr int kStages = kLdsStages;
     static constexpr int kSmemBytes = kStages * kStage * static_cast<int>(sizeof(T));
 };
 
