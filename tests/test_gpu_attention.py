@@ -224,7 +224,11 @@ def test_long_context_variant(device):
         assert_scaled_close(g, w, STOL[dtype], name)
 
 
-SCALAR_CASES = [  # served by the scalar family: fp32 storage, head_dim not a multiple of 8, unaligned tensors
+SCALAR_CASES = [  # what the reference's scalar kernels serve: here the scalar family for a head_dim that is no multiple of 8
+    # (16-bit) or 4 (fp32), the fp32 matrix kernels for the other fp32 cases
+    (torch.float32, dict(b=1, qs=40, ks=70, hq=4, hkv=2, d=30, off=30)),
+    (torch.float32, dict(b=2, qs=33, ks=33, hq=2, hkv=1, d=7)),
+    (torch.float32, dict(b=1, qs=20, ks=31, hq=2, hkv=1, d=127, causal=False)),
     (torch.float32, dict(b=2, qs=40, ks=40, hq=8, hkv=2, d=128)),
     (torch.float32, dict(b=1, qs=33, ks=70, hq=6, hkv=2, d=64, off=37, scale=0.2)),
     (torch.float32, dict(b=1, qs=50, ks=90, hq=2, hkv=1, d=20, causal=False)),
@@ -343,11 +347,11 @@ def test_fp32_hidden_rows_are_not_touched(device, case, tensor, value):
             assert_close(result, expected, 1e-4, where)
 
 
-def test_unaligned_tensors_take_the_scalar_family(device):
-    """Views that start 2 bytes into an allocation are not 16-byte aligned: same results as the aligned call
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["f16", "f32"])
+def test_unaligned_tensors_take_the_scalar_family(device, dtype):
+    """Views that start one element into an allocation are not 16-byte aligned: same results as the aligned call
     to storage precision (the two families round differently)."""
     c = dict(b=1, qs=64, ks=64, hq=4, hkv=2, d=64)
-    dtype = torch.float16
     q, k, v, do = make_inputs(c, dtype, 3)
 
     def shifted(t):

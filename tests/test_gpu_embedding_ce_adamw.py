@@ -128,8 +128,8 @@ def test_cross_entropy_known_answers(device):
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
 @pytest.mark.parametrize("rows,vocab", [(5, 11), (64, 1000), (7, 32000), (3, 50257), (16, 8), (2, 50264), (2, 65544)])
 def test_cross_entropy_parity(device, rows, vocab, dtype):
-    # Row lengths for each kernel: unaligned rows stream (11, 50257); aligned rows of up to 8192 vectors stay
-    # in registers, in 2, 8 or 16 vectors per thread (8 .. 50264); longer ones stream again (65544).
+    # Rows of up to 16384 vectors stay in registers, wherever they start: 2, 8 or 16 vectors per thread of 512, 16 of 1024 (fp32
+    # 50257 .. 65536). Longer ones stream (fp32 65544). The edges of each: test_gpu_kernel_boundaries.py.
     logits = randn((rows, vocab), dtype, 12, 3.0)
     targets = randint(vocab, (rows,), 13)
     targets[0] = vocab + 5  # out of range: no loss, gradient stays the softmax

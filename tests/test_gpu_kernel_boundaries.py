@@ -1,5 +1,6 @@
 """GPU tests at the sizes where one kernel, tile, split or unrolling gives way to the next: the first and last sizes of each
 range, with the oracle of the operator's own tests."""
+import numpy as np
 import pytest
 import torch
 
@@ -93,3 +94,65 @@ def test_swiglu_backward_around_the_choice_of_unrolling(device, more, dtype):
     ops.swiglu_backward(got_g, got_u, dy.to(device), g.to(device), u.to(device))
     assert_close(got_g, want_g, TOL[dtype], "dgate")
     assert_close(got_u, want_u, TOL[dtype], "dup")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
+@pytest.mark.parametrize("rows,fin,fout", [
+    (1, 5, 3), (33, 50, 70), (7, 131, 257),              # operands in padded copies
+    (100, 64, 96), (33, 4096, 40),                       # 32- and 64-wide tiles, K slices
+    (257, 2048, 264), (1100, 320, 520),                  # tiles of 64 and 128, ragged edges
+])
+def test_contractions_keep_non_finite_values_to_their_row_and_column(device, rows, fin, fout, value, dtype):
+    """An Inf or a NaN in an operand reaches the row or column of the product that it belongs to and nothing beside it, whatever
+    the kernel reads past the operands' ends; the rest is exact (small integers)."""
+    g = torch.Generator().manual_seed(rows + fin)
+    x, w, dy = (torch.randint(-2, 3, shape, generator=g).double() for shape in ((rows, fin), (fout, fin), (rows, fout)))
+    for tensor, (i, j) in [("x", (rows - 1, fin - 1)), ("w", (fout - 1, fin - 1)), ("dy", (rows - 1, fout - 1)), ("x", (rows // 2, 0)),
+                           ("w", (0, fin // 2)), ("dy", (0, fout // 2))]:
+        planted = {"x": x.clone(), "w": w.clone(), "dy": dy.clone()}
+        planted[tensor][i, j] = value
+        on = lambda name: planted[name].to(dtype).to(device)
+        y, gi, gw = (torch.empty(shape, dtype=dtype, device=device) for shape in ((rows, fout), (rows, fin), (fout, fin)))
+        ops.linear_forward(y, on("x"), on("w"))
+        ops.linear_backward(gi, gw, None, on("dy"), on("x"), on("w"))
+        whole = slice(None)
+        touched = {"x": {"Y": (i, whole), "dW": (whole, j)}, "w": {"Y": (whole, i), "dX": (whole, j)},
+                   "dy": {"dX": (i, whole), "dW": (j, whole)}}[tensor]
+        for name, got, exact in zip(("Y", "dX", "dW"), (y, gi, gw), (x @ w.T, dy @ w, dy.T @ x)):
+            got, exact = got.cpu(), exact.to(dtype)
+            if name in touched:
+                assert not torch.isfinite(got[touched[name]]).any(), f"{tensor}[{i}, {j}] {name}"
+                got[touched[name]] = exact[touched[name]] = 0
+            assert torch.equal(got, exact), f"{tensor}[{i}, {j}] {name}"
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("vocab", [7, 1003, 8192, 50257, 131073])
+def test_cross_entropy_with_non_finite_logits(device, vocab, dtype):
+    """-Inf logits (masked classes) have probability 0, single ones and whole vectors of them; an Inf or a NaN spoils its own
+    row's gradient, the Inf the loss, and no other row."""
+    rows = 6
+    logits = randn((rows, vocab), dtype, vocab, 2.0)
+    targets = torch.tensor([0, 1, 2, 3, 4, 5], dtype=torch.int32)
+    logits[1, vocab - 1] = logits[1, 6] = -float("inf")
+    logits[2, vocab // 2:] = -float("inf")
+    logits[3, :3] = -float("inf")
+
+    def run(z):
+        loss, grad = torch.zeros(1, device=device), torch.empty((rows, vocab), dtype=dtype, device=device)
+        ops.cross_entropy_forward_backward(loss, grad, z.to(device), targets.to(device), rows, None, 4096.0)
+        return loss.item(), grad.cpu()
+
+    loss, grad = run(logits)
+    want_loss, want = oracle64.cross_entropy(to_np(logits), targets.numpy(), 4096.0)
+    assert abs(loss - want_loss) <= 1e-4 * max(1.0, abs(want_loss))
+    assert_close(grad, want, TOL[dtype], "gradient")
+    for value in (float("inf"), float("nan")):
+        for row, col in ((0, 0), (4, vocab - 1), (5, vocab // 2)):
+            spoiled = logits.clone()
+            spoiled[row, col] = value
+            bad_loss, bad = run(spoiled)
+            others = torch.arange(rows) != row
+            assert not torch.isfinite(bad[row]).all() and (np.isnan(value) or not np.isfinite(bad_loss))
+            assert torch.equal(bad[others], grad[others])

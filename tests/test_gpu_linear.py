@@ -1,5 +1,6 @@
-"""GPU parity tests of linear_forward / linear_backward (MFMA contraction kernels and the plain
-fallback) against the CPU checker and float64 matmuls, through the C-ABI."""
+"""GPU parity tests of linear_forward / linear_backward (MFMA contraction kernels, padded copies of ragged operands) against
+the CPU checker and float64 matmuls, through the C-ABI. The general kernel of operands that cannot be copied:
+test_zz_capture_first.py."""
 import numpy as np
 import pytest
 import torch
