@@ -10,7 +10,7 @@
 //
 // Design
 //   * 256 threads = 4 wavefronts in a 2x2 grid; a block owns a BM x BN tile of C
-//     and walks K in steps of 32. Each wavefront owns (BM/2) x (BN/2) and issues
+//     and walks K in tiles of 64, two MFMA steps each. Each wavefront owns (BM/2) x (BN/2) and issues
 //     v_mfma_f32_16x16x32 (bf16 or f16): per flop that form moves half the accumulator
 //     data of the 32x32x16 one, which counts on a chip whose clock is power-limited.
 //   * The kernel is persistent: one block per CU slot walks its share of the work items
@@ -19,15 +19,18 @@
 //     tiles in flight on one XCD share A and B panels in that XCD's L2 (2 tile-rows for
 //     the kernel whose epilogue reads and writes whole rows of a wider matrix).
 //   * Operand tiles go global -> LDS with buffer_load ... lds (no staging registers, no
-//     LDS stores, one loop-invariant per-lane offset) into a ring of five LDS stages:
-//     one being multiplied, up to three K tiles in flight, one being refilled. LDS rows
-//     cannot be padded that way; a chunk swizzle keeps the fragment reads conflict-free.
+//     LDS stores, one loop-invariant per-lane offset) into a ring of LDS slots of one operand's
+//     K tile each. A K tile takes 128 bytes of every row of a k-contiguous operand, whole cache lines: in
+//     tiles of 64 bytes the path from L2 to LDS carries two thirds as much (0.25 instead of 0.17 us per 16 KiB
+//     and CU), and that, not the matrix cores, was what a K step cost: 0.29 us per 128 x 128 tile, 0.23 now.
+//     Forward [2048, 4096] x [4096, 4096] 77 -> 60 us, [32768, 1024] x [4096, 1024] 242 -> 227, dX 218 -> 205.
+//     LDS rows cannot be padded that way; a chunk swizzle keeps the fragment reads conflict-free.
 //   * Operands that are not k-contiguous in memory (dX's weight, both dW operands) sit
 //     in LDS as they are in memory and are transposed by the LDS read itself
 //     (ds_read_b64_tr_b16): no transpose pass over HBM, no VALU shuffles.
 //   * The K loop is a software pipeline with one barrier per K tile whose issue order is
-//     pinned in the source: every MFMA is followed by its share of the fragment reads and
-//     of the loads, the wait for the next K tile sits in the middle of the tile, and the
+//     pinned in the source: every MFMA is followed by its share of the fragment reads (of the next step, into
+//     registers of their own) and of the loads, and the
 //     loop has no data-dependent branch (edges are clamped or zero-filled by the buffer
 //     range check, never predicated).
 //   * MFMA is issued as (B-fragment, A-fragment), so a lane ends up holding four
@@ -54,17 +57,21 @@
 namespace cgptx {
 namespace {
 
-// LDS stages of a block: one being multiplied, one being refilled, the rest in flight. 256x256
-// blocks own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each).
-constexpr int kLdsStages = 5;
+// LDS is a ring of slots of one operand's K tile each (two K steps: 128 bytes along K per row or column), A and B in turn:
+// four slots hold the K tile being multiplied and the next one, the rest what is in flight beyond them. 256x256 blocks
+// own a CU (5 x 32 KiB), 128x128 blocks run two per CU (5 x 16 KiB each) or, where there is no second one for a CU, one
+// with 9 slots (two K tiles more in flight).
+constexpr int kLdsSlots = 5, kDeepSlots = 9;
+constexpr int kSteps = 2;  // K steps (of one MFMA each per 16 x 16 block) of a K tile
 
-template <typename T, int BM, int BN, bool A_K, bool B_K>
+template <typename T, int BM, int BN, bool A_K, bool B_K, int SLOTS>
 struct TileLayout {
-    using ATile = std::conditional_t<A_K, KTile<T, BM>, NTile<T, BM>>;
-    using BTile = std::conditional_t<B_K, KTile<T, BN>, NTile<T, BN>>;
-    static constexpr int kStage = ATile::kElems + BTile::kElems;  // elements per LDS stage: [A | B]
-    static constexpr int kStages = kLdsStages;
-    static constexpr int kSmemBytes = kStages * kStage * static_cast<int>(sizeof(T));
+    using ATile = std::conditional_t<A_K, KTile<T, BM, kSteps>, NTile<T, BM, kSteps>>;
+    using BTile = std::conditional_t<B_K, KTile<T, BN, kSteps>, NTile<T, BN, kSteps>>;
+    static constexpr int kSlot = ATile::kElems;  // elements
+    static_assert(ATile::kElems == BTile::kElems, "both operands' tiles take any slot");
+    static constexpr int kSlots = SLOTS;
+    static constexpr int kSmemBytes = kSlots * kSlot * static_cast<int>(sizeof(T));
 };
 
 // One workgroup per CU slot walks its share of the work items (output tile x K slice) one after
@@ -82,7 +89,7 @@ struct TileLayout {
 // so only the scalar offsets of the loads change), and the epilogue computes the product from the
 // rounded gate and up values, as the separate operator would from memory.
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
-          bool SWIGLU = false, bool GRAD = false>
+          bool SWIGLU = false, bool GRAD = false, int SLOTS = kLdsSlots>
 __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     static_assert(!GRAD || (A_K && !B_K && !SPLIT && !SEGMENTED && !RESIDUAL && !SWIGLU && BN == 256),
                   "the SwiGLU gradient epilogue belongs to the plain input-gradient kernel with 256-wide tiles");
@@ -91,7 +98,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     static_assert(!SWIGLU || (A_K && B_K && !SPLIT && !SEGMENTED && !RESIDUAL && BN == 256),
                   "the SwiGLU epilogue belongs to the plain forward kernel with 256-wide tiles");
     using frag_t = typename Mfma<T>::frag;
-    using Layout = TileLayout<T, BM, BN, A_K, B_K>;
+    using Layout = TileLayout<T, BM, BN, A_K, B_K, SLOTS>;
     using ATile = typename Layout::ATile;
     using BTile = typename Layout::BTile;
     static_assert(BM == BN, "the epilogue staging assumes square tiles");
@@ -99,11 +106,12 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     constexpr int TM = WM / 16, TN = WN / 16;  // 16 x 16 MFMA blocks of a wavefront's part
     extern __shared__ __align__(1024) unsigned char smem_raw[];
     T* smem = reinterpret_cast<T*>(smem_raw);
-    // Stage s holds [A tile | B tile] at smem + s * kStage.
-    constexpr int kStage = Layout::kStage;
-    constexpr int kStages = Layout::kStages;
-    constexpr int kATile = ATile::kElems;
-    constexpr unsigned int kStageBytes = kStage * sizeof(T);
+    // Operand tile o of an item (o even: A's K tile o/2, odd: B's) lives in slot o % kSlots.
+    constexpr int kSlot = Layout::kSlot;
+    constexpr int kSlots = Layout::kSlots;
+    constexpr int kAhead = (kSlots - 1) / 2;  // K tiles between the one being multiplied and the one being requested
+    static_assert(kSlots % 2 == 1 && kSlots >= 5, "an odd number of slots: first steps request A, second steps B");
+    constexpr unsigned int kSlotBytes = kSlot * sizeof(T);
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -155,7 +163,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     ATile a_src, a_src1, a_src2;
     BTile b_src;
     int a_end0 = std::numeric_limits<int>::max(), a_end1 = std::numeric_limits<int>::max();
-    int src_begin = 0, src_end = 0;  // K tiles of that item
+    int src_begin = 0, src_end = 0;  // K steps of that item
     auto open = [&](const Item& w) __attribute__((always_inline)) {
         const int m0 = w.m0, n0 = w.n0;
         src_begin = w.kt_begin;
@@ -214,12 +222,13 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     };
     // K tiles past the end of the slice are still "loaded" (the loop stays free of data-dependent
     // branches and every wavefront always has the same number of loads in flight), but from an
-    // offset beyond the buffer: the range check answers those at once with zeros, no memory traffic.
+    // offset beyond the buffer: the range check answers those at once with zeros, no memory traffic. What the last K tile
+    // holds past an odd number of K steps is never multiplied.
     // The source of a tile is picked with scalar selects, not branches, so that the loads can be
     // issued one by one between MFMAs.
-    auto cursors = [&](int t, TileCursor& ca, TileCursor& cb) __attribute__((always_inline)) {
-        const unsigned int past_end = src_begin + t >= src_end ? 0x80000000u : 0u;
-        const int k0 = min(src_begin + t, src_end - 1) * kBK<T>;
+    auto aim_a = [&](int t, TileCursor& ca) __attribute__((always_inline)) {
+        const unsigned int past_end = src_begin + t * kSteps >= src_end ? 0x80000000u : 0u;
+        const int k0 = min(src_begin + t * kSteps, src_end - 1) * kBK<T>;
         if constexpr (SEGMENTED) {
             // Values first, then selects: a conditional between the objects' members would select
             // an address and keep all three sources in memory.
@@ -238,89 +247,89 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
             const int start = in2 ? end1 : in1 ? end0 : 0;
             ca.soffset = (wave * group_bytes + (k0 - start) * static_cast<unsigned int>(sizeof(T))) | past_end;
             ca.step = kWaves * group_bytes;
-            ca.step2 = ca.step;
         } else {
             ca.rsrc = a_src.rsrc;
             ca.voffset = a_src.voffset;
             ca.soffset = a_src.first_offset(k0, wave) | past_end;
             ca.step = kWaves * a_src.group_bytes;
-            ca.step2 = ca.step;
         }
+    };
+    auto aim_b = [&](int t, TileCursor& cb) __attribute__((always_inline)) {
+        const unsigned int past_end = src_begin + t * kSteps >= src_end ? 0x80000000u : 0u;
+        const int k0 = min(src_begin + t * kSteps, src_end - 1) * kBK<T>;
         cb.rsrc = b_src.rsrc;
         cb.voffset = b_src.voffset;
         cb.soffset = b_src.first_offset(k0, wave) | past_end;
         cb.step = kWaves * b_src.group_bytes;
-        cb.step2 = cb.step;
         if constexpr (SWIGLU) {
-            // gate unit -> up unit of the same rows (inter rows further), then back and 64 rows on.
+            // Two loads per unit of 64 rows: gate unit, up unit of the same rows (inter rows further), then back and 64
+            // rows on.
             const unsigned int up = __builtin_amdgcn_readfirstlane(
                 static_cast<unsigned int>(static_cast<long>(p.inter) * p.ldb * static_cast<long>(sizeof(T))));
-            cb.step2 = cb.step - up;
-            cb.step = up;
+            cb.step_up = up - cb.step;
+            cb.step_back = cb.step - up;
         }
     };
-    // Load l of a K tile (A's loads first, then B's) into the stage whose LDS address, advanced to
-    // this wavefront's first 1 KiB slot, is stage_lds. One load fills 1 KiB; the wavefronts' slots
-    // interleave, so a wavefront's consecutive loads are kWaves KiB apart.
+    // Load l of an operand tile into the slot whose LDS address, advanced to this wavefront's first 1 KiB, is
+    // slot_lds. One load fills 1 KiB; the wavefronts' loads interleave, so a wavefront's consecutive ones are
+    // kWaves KiB apart.
     constexpr int kLoadBytes = 64 * 16;
-    constexpr int kATileBytes = kATile * static_cast<int>(sizeof(T));
-    auto issue_one = [&](auto index, unsigned int stage_lds, TileCursor& ca, TileCursor& cb) __attribute__((always_inline)) {
+    constexpr int kLoads = ATile::kLoads;  // per wavefront and operand tile
+    static_assert(ATile::kLoads == BTile::kLoads && kSlots * kLoads < 64, "the vmcnt waits count either operand's loads");
+    auto issue_a = [&](auto index, unsigned int slot_lds, TileCursor& ca) __attribute__((always_inline)) {
         constexpr int l = decltype(index)::value;
-        if constexpr (l < ATile::kLoads) {
-            ca.soffset = load_to_lds<l * kWaves * kLoadBytes>(ca.rsrc, stage_lds, ca.voffset, ca.soffset, ca.step);
-        } else {
-            constexpr int lb = l - ATile::kLoads;
-            cb.soffset = load_to_lds<kATileBytes + lb * kWaves * kLoadBytes>(cb.rsrc, stage_lds, cb.voffset, cb.soffset,
-                                                                            (lb & 1) ? cb.step2 : cb.step);
-        }
+        ca.soffset = load_to_lds<l * kWaves * kLoadBytes>(ca.rsrc, slot_lds, ca.voffset, ca.soffset, ca.step);
     };
-    constexpr int kTileLoads = ATile::kLoads + BTile::kLoads;  // per wavefront and K tile
-    static_assert(kTileLoads % 2 == 0, "a K tile's loads are dealt out in two equal halves, and the vmcnt waits count both");
+    auto issue_b = [&](auto index, unsigned int slot_lds, TileCursor& cb) __attribute__((always_inline)) {
+        constexpr int l = decltype(index)::value;
+        const unsigned int step = !SWIGLU || l % 2 == 0 ? cb.step : l % 4 == 1 ? cb.step_up : cb.step_back;
+        cb.soffset = load_to_lds<l * kWaves * kLoadBytes>(cb.rsrc, slot_lds, cb.voffset, cb.soffset, step);
+    };
     const unsigned int lds_wave = lds_address_of(smem) + wave * kLoadBytes;
     TileCursor ca, cb;
-    // Requests K tiles FIRST .. LAST-1 of the opened item into the stages of the same numbers.
+    // Requests operand tiles FIRST .. LAST-1 of the opened item into the slots of the same numbers.
     auto request_tiles = [&]<int FIRST, int LAST>() __attribute__((always_inline)) {
         static_for<FIRST, LAST>([&](auto index) {
-            constexpr int t = decltype(index)::value;
-            cursors(t, ca, cb);
-            static_for<0, kTileLoads>([&](auto l) { issue_one(l, lds_wave + t * kStageBytes, ca, cb); });
+            constexpr int o = decltype(index)::value;
+            if constexpr (o % 2 == 0) {
+                aim_a(o / 2, ca);
+                static_for<0, kLoads>([&](auto l) { issue_a(l, lds_wave + o * kSlotBytes, ca); });
+            } else {
+                aim_b(o / 2, cb);
+                static_for<0, kLoads>([&](auto l) { issue_b(l, lds_wave + o * kSlotBytes, cb); });
+            }
         });
     };
 
-    // Per-lane LDS offsets of the fragments: one for a k-contiguous operand (the block is a
+    // Per-lane LDS offsets of the fragments: one per K step for a k-contiguous operand (the block is a
     // scalar offset), one per 16-column block for an n-contiguous one (the swizzle depends on it).
-    constexpr int kAOffsets = A_K ? 1 : TM, kBOffsets = B_K ? 1 : TN;
+    constexpr int kAOffsets = A_K ? kSteps : TM, kBOffsets = B_K ? kSteps : TN;
     int a_off[kAOffsets], b_off[kBOffsets];
-    if constexpr (A_K) {
-        a_off[0] = ATile::lane_offset(lane);
-    } else {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a_off[i] = ATile::lane_offset(lane, wm * WM + i * 16);
-    }
-    if constexpr (B_K) {
-        b_off[0] = BTile::lane_offset(lane);
-    } else {
+    for (int i = 0; i < kAOffsets; ++i) a_off[i] = A_K ? ATile::lane_offset(lane, i) : ATile::lane_offset(lane, wm * WM + i * 16);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) b_off[j] = BTile::lane_offset(lane, wn * WN + j * 16);
-    }
+    for (int j = 0; j < kBOffsets; ++j) b_off[j] = B_K ? BTile::lane_offset(lane, j) : BTile::lane_offset(lane, wn * WN + j * 16);
 
+    // Fragments of the K step being multiplied and of the next one: step s of a K tile is in af[s], bf[s].
     acc_t acc[TM][TN];
-    frag_t af[TM], bf[TN];
-    // Fragment F (A's TM blocks first, then B's TN) of the K tile in `stage_tile`.
-    auto read_frag = [&]<int F>(const T* stage_tile) __attribute__((always_inline)) {
-        if constexpr (F < TM) {
-            if constexpr (A_K) af[F] = ATile::frag(stage_tile, wm * WM + F * 16, a_off[0]);
-            else af[F] = ATile::frag(stage_tile, a_off[F]);
+    frag_t af[kSteps][TM], bf[kSteps][TN];
+    constexpr int kFrags = TM + TN;
+    // The F-th fragment in the order of first use (A's block 0, B's blocks, A's other blocks) of K step STEP.
+    auto read_frag = [&]<int STEP, int F>(const T* a_tile, const T* b_tile) __attribute__((always_inline)) {
+        if constexpr (F >= 1 && F <= TN) {
+            constexpr int j = F - 1;
+            if constexpr (B_K) bf[STEP][j] = BTile::frag(b_tile, wn * WN + j * 16, b_off[STEP]);
+            else bf[STEP][j] = BTile::frag(b_tile + STEP * BTile::kStepElems, b_off[j]);
         } else {
-            constexpr int j = F - TM;
-            if constexpr (B_K) bf[j] = BTile::frag(stage_tile + kATile, wn * WN + j * 16, b_off[0]);
-            else bf[j] = BTile::frag(stage_tile + kATile, b_off[j]);
+            constexpr int i = F == 0 ? 0 : F - TN;
+            if constexpr (A_K) af[STEP][i] = ATile::frag(a_tile, wm * WM + i * 16, a_off[STEP]);
+            else af[STEP][i] = ATile::frag(a_tile + STEP * ATile::kStepElems, a_off[i]);
         }
     };
 
     // Epilogue staging. acc[i][j][e] holds C[m, n] with m = lane%16, n = 4*(lane/16) + e, relative
     // to the 16 x 16 block (i, j) of the wavefront's WM x WN part of the tile. Each wavefront passes
-    // its part through a private quarter of the last LDS stage (the only one the first K tiles of
+    // its part through a private quarter of the last LDS slot (the only one the first operand tiles of
     // the next item do not fill), 32 rows at a time, and stores it row by row: whole contiguous
     // row segments of C per instruction instead of 32 separate 8-byte pieces, and no workgroup
     // barrier. When bias, residual or the old C are added (or the output is fp32 / a split-K
@@ -333,8 +342,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     static_assert(!kIsF32 || (BM <= 128 && !SEGMENTED && !RESIDUAL && !SWIGLU && !GRAD), "fp32 storage has the plain kernels only");
     constexpr int kRowBytes = WN * 2;  // fp32 values always pass in two halves
     constexpr int kRowChunks = kRowBytes / 16;
-    static_assert(32 * kRowBytes * kWaves == static_cast<int>(kStageBytes), "staging is a quarter stage per wavefront");
-    unsigned char* region = smem_raw + (kStages - 1) * kStageBytes + wave * (kStageBytes / kWaves);
+    static_assert(32 * kRowBytes * kWaves == static_cast<int>(kSlotBytes), "staging is a quarter slot per wavefront");
+    unsigned char* region = smem_raw + (kSlots - 1) * kSlotBytes + wave * (kSlotBytes / kWaves);
     auto sw = [](int row) { return (row / (256 / kRowBytes)) % kRowChunks; };
     const int m_lane = lane & 15, q_lane = lane >> 4;
     // Writes blocks (2r, j0 .. j0+JP-1) and (2r+1, ...) into the wavefront's staging region as element type S.
@@ -389,7 +398,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         static_for<0, kRowBlocks>([&](auto index) {
             constexpr int block = decltype(index)::value;
             if (r == block)
-                request_tiles.template operator()<block * (kStages - 1) / kRowBlocks, (block + 1) * (kStages - 1) / kRowBlocks>();
+                request_tiles.template operator()<block * (kSlots - 1) / kRowBlocks, (block + 1) * (kSlots - 1) / kRowBlocks>();
         });
     };
     // Before 32-row block r of the tile is staged and stored, its share of the first K tiles of the next item
@@ -765,56 +774,45 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         }
     };
 
-    // Software pipeline over the K tiles t = 0 .. count-1 of an item (tile t lives in LDS stage
-    // t % kStages; tiles t+1 .. t+kStages-2 are in flight or landed). A K tile is one MFMA step
-    // (k = 32) of TM x TN MFMAs, taken as two column halves (all rows x the left TN/2 blocks, then
-    // all rows x the right ones) so that one set of fragment registers suffices: a fragment is read
-    // for the next tile as soon as its last MFMA of this tile has been issued.
-    //   left half    MFMAs ‖ LDS reads of this tile's right-half B fragments ‖ the second half of the loads of
-    //                tile t+kStages-2 (into the stage freed one tile ago)
-    //   wait         this wavefront's loads of tile t+1 have landed; barrier: everybody's have, and
-    //                nobody reads stage (t-1) % kStages any more
-    //   right half   MFMAs ‖ the first half of the loads of tile t+kStages-1 into that stage ‖ tile t+1's
-    //                left-half B fragments (first thing) and its A fragment i after row i
-    // so LDS latency and kStages-2 K tiles of global latency sit in the shadow of MFMAs. With one
-    // wavefront per SIMD nothing else hides an instruction that is not next to an MFMA, so every
-    // MFMA is followed by its share of the loads and fragment reads and a scheduling fence keeps
-    // them there.
+    // Software pipeline over the K tiles t of an item, two K steps of TM x TN MFMAs each. The fragments of a step are read
+    // from LDS while the step before it is multiplied, into registers of their own:
+    //   first step   MFMAs ‖ LDS reads of this tile's second-step fragments ‖ the loads of A's K tile t+kAhead (into the slot
+    //                of B's K tile t-1)
+    //   wait         this wavefront's loads of K tile t+1 have landed and its reads of K tile t are through; barrier:
+    //                everybody's have, so K tile t's slots are free
+    //   second step  MFMAs ‖ LDS reads of K tile t+1's first-step fragments ‖ the loads of B's K tile t+kAhead (into the slot
+    //                of A's K tile t)
+    // so LDS latency and one to one and a half K tiles of global latency sit in the shadow of MFMAs, and the workgroup
+    // meets once per K tile. With one wavefront per SIMD nothing else hides an instruction that is not next to an MFMA, so
+    // every MFMA is followed by its share of the loads and fragment reads and a scheduling fence keeps them there. A
+    // wavefront's load instruction keeps it from issuing for about as long as an MFMA runs.
     constexpr int kMfmas = TM * TN;
-    constexpr int kHalf = TN / 2;
-    static_assert(TN % 2 == 0 && kHalf <= TM, "the left-half B fragments are read one per row");
-    // HALF 0: this_tile = tile t (its right-half B fragments are read); HALF 1: next_tile = tile t+1.
-    auto multiply_half = [&]<int HALF, bool FIRST>(const T* tile, unsigned int free_lds) __attribute__((always_inline)) {
-        static_for<0, kMfmas / 2>([&](auto index) {
+    constexpr int kReadEvery = kMfmas / kFrags >= 4 ? 3 : 1;  // MFMAs between fragment reads
+    static_assert(kReadEvery * kFrags <= kMfmas && kLoads <= kMfmas, "a step has room for the reads and loads it carries");
+    // STEP 0: a_tile, b_tile are K tile t's; STEP 1: K tile t+1's. slot_lds: where the step's loads (of K tile `aimed`) go.
+    auto multiply_step = [&]<int STEP, bool FIRST>(const T* a_tile, const T* b_tile, unsigned int slot_lds, int aimed) __attribute__((always_inline)) {
+        static_for<0, kMfmas>([&](auto index) {
             constexpr int m = decltype(index)::value;
             // Rows one after the other, their columns left to right and right to left alternately:
             // consecutive MFMAs always share an operand (measurably less power on a power-limited chip).
-            constexpr int i = m / kHalf, jj = m % kHalf, j = HALF * kHalf + ((i & 1) ? kHalf - 1 - jj : jj);
-            if constexpr (FIRST) Mfma<T>::start(acc[i][j], bf[j], af[i]);
-            else Mfma<T>::run(acc[i][j], bf[j], af[i]);
-            if constexpr (HALF == 0) {
-                // Right-half B fragment i of this tile after the first MFMA of row i (rows 0 .. kHalf-1).
-                if constexpr (jj == 0 && i < kHalf) read_frag.template operator()<TM + kHalf + i>(tile);
-            } else {
-                // Left-half B fragment i of the next tile after the first MFMA of row i (its last use
-                // was in the left half), A fragment i after the last MFMA of row i.
-                if constexpr (jj == 0 && i < kHalf) read_frag.template operator()<TM + i>(tile);
-                if constexpr (jj == kHalf - 1) read_frag.template operator()<i>(tile);
-                // The first half of the loads of tile t+kStages-1 (one load per kMfmas / kTileLoads MFMAs).
-                static_for<(m * (kTileLoads / 2)) / (kMfmas / 2), ((m + 1) * (kTileLoads / 2)) / (kMfmas / 2)>(
-                    [&](auto l) { issue_one(l, free_lds, ca, cb); });
-            }
-            if constexpr (HALF == 0 && !FIRST) {
-                // The second half of the loads that the previous tile's right half began: a wavefront's load
-                // instruction keeps it from issuing for about as long as an MFMA runs, so the loads are dealt out
-                // evenly over the whole tile instead of twice as densely over one half.
-                static_for<kTileLoads / 2 + (m * (kTileLoads / 2)) / (kMfmas / 2),
-                           kTileLoads / 2 + ((m + 1) * (kTileLoads / 2)) / (kMfmas / 2)>(
-                    [&](auto l) { issue_one(l, free_lds, ca, cb); });
+            constexpr int i = m / TN, jj = m % TN, j = (i & 1) ? TN - 1 - jj : jj;
+            if constexpr (FIRST && STEP == 0) Mfma<T>::start(acc[i][j], bf[STEP][j], af[STEP][i]);
+            else Mfma<T>::run(acc[i][j], bf[STEP][j], af[STEP][i]);
+            if constexpr (m % kReadEvery == 0 && m / kReadEvery < kFrags)
+                read_frag.template operator()<1 - STEP, m / kReadEvery>(a_tile, b_tile);
+            static_for<(m * kLoads) / kMfmas, ((m + 1) * kLoads) / kMfmas>([&](auto l) {
+                if constexpr (STEP == 0) issue_a(l, slot_lds, ca);
+                else issue_b(l, slot_lds, cb);
+            });
+            // The next step's cursor, where its scalar arithmetic has MFMAs around it.
+            if constexpr (m == kMfmas / 2) {
+                if constexpr (STEP == 0) aim_b(aimed, cb);
+                else aim_a(aimed + 1, ca);
             }
             __builtin_amdgcn_sched_barrier(0);
         });
     };
+    auto slot_after = [](int slot, int by) __attribute__((always_inline)) { return slot + by >= kSlots ? slot + by - kSlots : slot + by; };
 
     // Per round: multiply an item, request the first K tiles of the next one, store the finished
     // tile (its stores drain under the MFMAs that follow). The sources are opened every round, also
@@ -822,36 +820,44 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     // stay in scalar registers.
     Item current = locate(item);
     open(current);
-    request_tiles.template operator()<0, kStages - 1>();
+    request_tiles.template operator()<0, kSlots - 1>();
     while (true) {
-        const int count = current.kt_end - current.kt_begin;
-        // Loads and stores retire in the order they were issued: at most the loads of K tiles
-        // 1 .. kStages-2 (and no older store of the previous epilogue) may still be outstanding.
-        __builtin_amdgcn_s_waitcnt(vmcnt_immediate((kStages - 2) * kTileLoads));
+        const int steps = current.kt_end - current.kt_begin;
+        // Loads and stores retire in the order they were issued: at most the loads of the operand tiles
+        // after the first two (and no older store of the previous epilogue) may still be outstanding.
+        __builtin_amdgcn_s_waitcnt(vmcnt_immediate((kSlots - 3) * kLoads));
         barrier_only();
-        static_for<0, TM + kHalf>([&](auto f) { read_frag.template operator()<decltype(f)::value>(smem); });
-        int stage = 0;                 // of tile t
-        int free_stage = kStages - 1;  // of tile t-1, refilled with tile t+kStages-1
-        auto multiply_tile = [&]<bool FIRST>(int t) __attribute__((always_inline)) {
-            const int next_stage = stage + 1 == kStages ? 0 : stage + 1;
-            // The left half finishes the requests of tile t+kStages-2 (cursors and stage of the previous tile: the
-            // stage before free_stage), then the cursors move on to tile t+kStages-1.
-            const int previous_free = free_stage == 0 ? kStages - 1 : free_stage - 1;
-            multiply_half.template operator()<0, FIRST>(smem + stage * kStage, lds_wave + previous_free * kStageBytes);
-            cursors(t + kStages - 1, ca, cb);
-            __builtin_amdgcn_s_waitcnt(vmcnt_immediate((kStages - 3) * kTileLoads));
-            barrier_only();
-            multiply_half.template operator()<1, FIRST>(smem + next_stage * kStage, lds_wave + free_stage * kStageBytes);
-            free_stage = stage;
-            stage = next_stage;
+        static_for<0, kFrags>([&](auto f) { read_frag.template operator()<0, decltype(f)::value>(smem, smem + kSlot); });
+        aim_a(kAhead, ca);
+        int slot = 0;  // of A's K tile t; B's is in the one after it
+        auto first_step = [&]<bool FIRST>(int t) __attribute__((always_inline)) {
+            multiply_step.template operator()<0, FIRST>(smem + slot * kSlot, smem + slot_after(slot, 1) * kSlot,
+                                                        lds_wave + slot_after(slot, kSlots - 1) * kSlotBytes, t + kAhead);
         };
-        // The first K tile starts the sums (MFMA with a zero addend): no pass over the 256
-        // accumulator registers to clear them. Every item has at least one K tile (the host makes
+        auto second_step = [&](int t) __attribute__((always_inline)) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(vmcnt_immediate((kSlots - 4) * kLoads));
+            barrier_only();
+            const int next = slot_after(slot, 2);
+            multiply_step.template operator()<1, false>(smem + next * kSlot, smem + slot_after(slot, 3) * kSlot,
+                                                        lds_wave + slot * kSlotBytes, t + kAhead);
+            slot = next;
+        };
+        // The first K step starts the sums (MFMA with a zero addend): no pass over the 256
+        // accumulator registers to clear them. Every item has at least one K step (the host makes
         // K slices non-empty).
-        multiply_tile.template operator()<true>(0);
-        for (int t = 1; t < count; ++t) multiply_tile.template operator()<false>(t);
+        first_step.template operator()<true>(0);
+        if (steps > 1) {
+            second_step(0);
+            int t = 1;
+            for (; t * kSteps + 1 < steps; ++t) {
+                first_step.template operator()<false>(t);
+                second_step(t);
+            }
+            if (t * kSteps < steps) first_step.template operator()<false>(t);
+        }
         // The loads still outstanding are of K tiles past the end (zeros, but they do write LDS):
-        // once they have landed and every wavefront has read its last fragments, all stages are free.
+        // once they have landed and every wavefront has read its last fragments, all slots are free.
         __builtin_amdgcn_s_waitcnt(vmcnt_immediate(0));
         barrier_only();
         item += item_stride;
@@ -1061,10 +1067,15 @@ constexpr int blocks_per_unit(int tile) { return tile == 256 ? 1 : 2; }  // resi
 
 
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
-          bool SWIGLU = false, bool GRAD = false>
+          bool SWIGLU = false, bool GRAD = false, int SLOTS = kLdsSlots>
 int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
-    constexpr std::size_t smem = TileLayout<T, BM, BN, A_K, B_K>::kSmemBytes;
-    auto kernel = gemm_mfma_kernel<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD>;
+    const long items = static_cast<long>(p.tiles_m) * p.tiles_n * slices;
+    if constexpr (BM == 128 && SLOTS == kLdsSlots) {
+        if (items <= compute_units())
+            return launch_mfma<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, kDeepSlots>(p, slices, stream);
+    }
+    constexpr std::size_t smem = TileLayout<T, BM, BN, A_K, B_K, SLOTS>::kSmemBytes;
+    auto kernel = gemm_mfma_kernel<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, SLOTS>;
     static bool configured = false;
     if (!configured) {
         CGPTX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1075,7 +1086,6 @@ int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
     // so that every XCD gets the same number of blocks; fewer when there are fewer work items.
     KernelArgs args = p;
     args.slices = slices;
-    const long items = static_cast<long>(p.tiles_m) * p.tiles_n * slices;
     {
         // x * ceil(2^32 / d) >> 32 == x / d for every x with x * d < 2^32.
         // Tile-rows per L2 locality group. 8 (x 4 tile-columns = the 32 tiles in flight on an XCD) shares operand
@@ -1206,6 +1216,7 @@ Plan make_plan(const GemmArgs& g) {
                            !(g.a_k_contiguous && g.a_segments.count > 0);
     auto set_slices = [&](long slices) {
         plan.k_tiles_per_slice = static_cast<int>((k_tiles + slices - 1) / slices);
+        if (slices > 1) plan.k_tiles_per_slice = (plan.k_tiles_per_slice + kSteps - 1) / kSteps * kSteps;  // whole K tiles of the large kernels
         plan.slices = static_cast<int>((k_tiles + plan.k_tiles_per_slice - 1) / plan.k_tiles_per_slice);
     };
     if (g.swiglu_out != nullptr || g.swiglu_saved != nullptr || (!f32 && tiles_of(256) >= 3 * units && g.batch_rows == 0)) {
@@ -1459,7 +1470,7 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
     const bool segmented = g.a_segments.count > 0 || g.c_segments.count > 0;
     if (segmented) {
         if (int s = copy_segments(g.a_segments, g.a_k_contiguous ? g.k : (g.batch_rows != 0 ? g.batch_rows : g.m),
-                                  g.a_k_contiguous ? kBK<T> : 256, p.a_seg))
+                                  g.a_k_contiguous ? kSteps * kBK<T> : 256, p.a_seg))
             return s;
         if (int s = copy_segments(g.c_segments, g.n, 256, p.c_seg)) return s;
         if (g.c_segments.count > 0 && (g.c_is_f32 || g.residual != nullptr))

@@ -184,7 +184,8 @@ struct TileCursor {
     int voffset;
     unsigned int soffset;
     unsigned int step;
-    unsigned int step2;  // advance after the operand's odd-numbered loads (differs from step only for SWIGLU's B)
+    // Advance after the operand's odd-numbered loads, towards an up unit and back (differ from step only for SWIGLU's B).
+    unsigned int step_up, step_back;
 };
 
 template <int BEGIN, int... I, typename F>
@@ -208,24 +209,28 @@ __device__ __forceinline__ unsigned int lds_address_of(const T* p) {
 // cannot be padded; bank conflicts are avoided by storing 16-byte chunk c of a row at chunk
 // position c ^ swizzle(row) — the lane that owns an LDS slot fetches the matching global chunk.
 
-// ---- operand stored [ROWS, K] (k-contiguous): ROWS x kBK slab, unpadded LDS rows ---------------
+// ---- operand stored [ROWS, K] (k-contiguous): ROWS x (STEPS * kBK) slab, unpadded LDS rows -----
+// A row of the slab is STEPS * 64 bytes. With two K steps that is a whole cache line: a load instruction then touches 8
+// lines instead of 16 halves of lines, which is what the path from the L2s to a CU's LDS is bound by (16 KiB of operand
+// tiles per CU, every CU loading: 0.25 us in pieces of 64 bytes, 0.17 us in pieces of 128, no more in longer ones).
 // One load instruction covers 1024 B = kRowsPerLoad rows; wavefront w issues the loads of row
 // groups w, w+4, ... The chunk swizzle is (row / rows per 256 B) mod chunks per row: the 16 rows a
 // quarter-wavefront reads with ds_read_b128 then hit the 16 different 16-byte positions of a
 // 256-byte bank period.
-template <typename T, int ROWS>
+template <typename T, int ROWS, int STEPS = 1>
 struct KTile {
     using frag_t = typename Mfma<T>::frag;
-    static constexpr int kChunksPerRow = kBK<T> / kVec128<T>;
+    static constexpr int kRowElems = STEPS * kBK<T>;
+    static constexpr int kChunksPerRow = kRowElems / kVec128<T>;
     static constexpr int kRowsPerLoad = 64 / kChunksPerRow;
-    static constexpr int kElems = ROWS * kBK<T>;
+    static constexpr int kElems = ROWS * kRowElems;
     static constexpr int kLoads = ROWS / kRowsPerLoad / kWaves;  // load instructions per wavefront and tile
 
     u32x4 rsrc = {0u, 0u, 0u, 0u};
     int voffset = 0;
     unsigned int group_bytes = 0;  // kRowsPerLoad rows further in global memory
 
-    __device__ __forceinline__ static int swizzle(int row) { return (row / 4) % kChunksPerRow; }
+    __device__ __forceinline__ static int swizzle(int row) { return (row / (4 / STEPS)) % kChunksPerRow; }
 
     // base: element (row0, 0) of the operand; rows past rows_left only feed C rows that are never
     // stored (they read zeros or whatever follows, never out of the allocation's last row).
@@ -243,29 +248,30 @@ struct KTile {
     __device__ __forceinline__ unsigned int first_offset(int k0, int wave) const {
         return wave * group_bytes + k0 * static_cast<unsigned int>(sizeof(T));
     }
-    // Element offset of the lane's fragment within a 16-row block (the whole K tile is one MFMA
-    // step): row lane%16, the lane/16-th 16 bytes of it. The swizzle of a row does not depend on the block.
-    __device__ __forceinline__ static int lane_offset(int lane) {
-        return (lane & 15) * kBK<T> + (((lane >> 4) ^ swizzle(lane & 15)) * kVec128<T>);
+    // Element offset of the lane's fragment of K step `step` within a 16-row block: row lane%16, the lane/16-th
+    // 16 bytes of the step's part of it. The swizzle of a row does not depend on the block.
+    __device__ __forceinline__ static int lane_offset(int lane, int step = 0) {
+        return (lane & 15) * kRowElems + ((((lane >> 4) + 4 * step) ^ swizzle(lane & 15)) * kVec128<T>);
     }
     __device__ __forceinline__ static frag_t frag(const T* tile, int block0, int offset) {
-        return *reinterpret_cast<const frag_t*>(tile + block0 * kBK<T> + offset);
+        return *reinterpret_cast<const frag_t*>(tile + block0 * kRowElems + offset);
     }
 };
 
-// ---- operand stored [K, COLS] (n-contiguous): 32 x COLS slab kept in that order in LDS ---------
+// ---- operand stored [K, COLS] (n-contiguous): (STEPS * kBK) x COLS slab kept in that order in LDS
 // The transpose happens on the way out of LDS: ds_read_b64_tr_b16 hands lane n of a 16-lane group
 // the four k-values of column n from a 4(k) x 16(n) block, so two of them build the 8-k fragment of
 // one column. swizzle(k row) = 4*(row%4) on the chunk index (rows of 128 bytes: 4*(row/2%2), the row's parity
 // picks the half already): the four k rows that 32 lanes read sit in four different 64-byte windows of the
 // 256-byte bank period. K rows past the operand's end are out of the buffer's range and read as zeros.
-template <typename T, int COLS>
+template <typename T, int COLS, int STEPS = 1>
 struct NTile {
     using frag_t = typename Mfma<T>::frag;
     static constexpr int kChunksPerRow = COLS / kVec128<T>;
     static constexpr int kRowsPerLoad = 64 / kChunksPerRow;  // k rows one load instruction covers
-    static constexpr int kElems = kBK<T> * COLS;
-    static constexpr int kLoads = kBK<T> / kRowsPerLoad / kWaves;
+    static constexpr int kStepElems = kBK<T> * COLS;         // K step s starts at s * kStepElems
+    static constexpr int kElems = STEPS * kStepElems;
+    static constexpr int kLoads = STEPS * kBK<T> / kRowsPerLoad / kWaves;
 
     // fp32: the four k rows a read touches lie four apart (k = 4*(lane/16) + e).
     __device__ __forceinline__ static int swizzle(int k_row) {

@@ -66,6 +66,26 @@ def test_contractions_in_k_slices_are_exact_on_integers(device, rows, fin, fout,
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("rows,fin,fout", [
+    *((12288, k, 4096) for k in (32, 64, 96, 160, 352)),   # 256 x 256 tiles: one K step, whole K tiles, a step more
+    *((3500, k, 3496) for k in (32, 96, 128, 320, 352)),   # 128 x 128 tiles, two and more workgroups on a CU, ragged edges
+    (2000, 992, 2048), (2000, 1024, 2048), (1990, 1056, 2040),  # one workgroup per CU, more operand tiles in flight
+    (2048, 4096 + 32, 4096),                                # both gradients' K an odd number of K steps long as well
+])
+def test_contractions_whose_last_k_tile_is_half_filled_are_exact_on_integers(device, rows, fin, fout, dtype):
+    """As above (products of -1 .. 1, at most 12288 of them): K tiles are two K steps long, and what a load brings in past the
+    last step of a row is the next row, which no sum may see."""
+    g = torch.Generator(device=device).manual_seed(rows + fin + fout)
+    x, w, dy = (torch.randint(-1, 2, shape, generator=g, device=device).float() for shape in ((rows, fin), (fout, fin), (rows, fout)))
+    on = lambda t: t.to(dtype)
+    y, gi, gw = (torch.full(shape, float("nan"), dtype=dtype, device=device) for shape in ((rows, fout), (rows, fin), (fout, fin)))
+    ops.linear_forward(y, on(x), on(w))
+    ops.linear_backward(gi, gw, None, on(dy), on(x), on(w))
+    for name, got, exact in zip(("Y", "dX", "dW"), (y, gi, gw), (x @ w.T, dy @ w, dy.T.contiguous() @ x)):
+        assert torch.equal(got, exact.to(dtype)), name
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
 @pytest.mark.parametrize("vectors", [1024, 1025, 4096, 4097, 8192, 8193, 16384, 16385])
 @pytest.mark.parametrize("tail", [0, 1])
 def test_cross_entropy_around_the_held_row_lengths(device, vectors, tail, dtype):
