@@ -1270,10 +1270,8 @@ Plan make_plan(const GemmArgs& g) {
 }
 
 // Arguments of the small kernel (gemm_small_kernel.hpp) from the streamed ones.
-template <typename T>
-int launch_small_call(const GemmArgs& g, const KernelArgs& p, const Plan& plan, bool split, hipStream_t stream) {
-    SmallCall call{};
-    SmallArgs& a = call.args;
+SmallArgs small_args(const KernelArgs& p, bool split, int k_tiles_per_slice) {
+    SmallArgs a{};
     a.a = p.a;
     a.b = p.b;
     a.c = p.c;
@@ -1287,7 +1285,7 @@ int launch_small_call(const GemmArgs& g, const KernelArgs& p, const Plan& plan, 
     a.b_extent = p.b_extent;
     a.b_k = p.b_k;
     a.k_tiles = p.k_tiles;
-    a.k_tiles_per_slice = plan.k_tiles_per_slice;
+    a.k_tiles_per_slice = k_tiles_per_slice;
     a.bias = p.bias;
     a.residual = p.residual;
     a.addend = p.addend;
@@ -1306,6 +1304,13 @@ int launch_small_call(const GemmArgs& g, const KernelArgs& p, const Plan& plan, 
     };
     copy(p.a_seg, a.a_seg);
     copy(p.c_seg, a.c_seg);
+    return a;
+}
+
+template <typename T>
+int launch_small_call(const GemmArgs& g, const KernelArgs& p, const Plan& plan, bool split, hipStream_t stream) {
+    SmallCall call{};
+    call.args = small_args(p, split, plan.k_tiles_per_slice);
     call.a_k_contiguous = g.a_k_contiguous;
     call.b_k_contiguous = g.b_k_contiguous;
     call.tile = plan.tile;
@@ -1425,9 +1430,15 @@ bool insists_on_split(const GemmArgs& g, bool ragged) {
     return small <= units || (large >= 8 && 2 * large <= units && g.k / kBK<bf16_t> >= 32 * ((units + large - 1) / large));
 }
 
+// Whether a call's operands lie within the streamed kernels' 32-bit offsets, and which of them can be read as they lie.
+struct Streams {
+    bool reach = false, a = false, b = false;
+};
+
+// The kernels' arguments of a call.
 template <typename T>
-int run_typed(const GemmArgs& g, hipStream_t stream) {
-    KernelArgs p{};
+int describe(const GemmArgs& g, KernelArgs& p, Streams& streams) {
+    p = KernelArgs{};
     p.a = g.a;
     p.b = g.b;
     p.c = g.c;
@@ -1478,29 +1489,38 @@ int run_typed(const GemmArgs& g, hipStream_t stream) {
         if (std::is_same_v<T, float>) return fail(CGPTX_INVALID_ARGUMENT, "gemm: segmented operands need 16-bit storage");
     }
 
-    bool fast = false;
-    {
-        GemmArgs whole = g;  // alignment of segmented operands was checked per segment
-        if (g.a_segments.count > 0) {
-            whole.a = g.a_segments.ptr[0];
-            whole.lda = g.a_segments.ld[0];
-        }
-        if (g.c_segments.count > 0) {
-            whole.c = const_cast<void*>(g.c_segments.ptr[0]);
-            whole.ldc = g.c_segments.ld[0];
-        }
-        if ((g.a_k_contiguous || !g.b_k_contiguous) && offsets_fit_32bit(whole, sizeof(T))) {
-            const bool a_ok = a_streams(whole), b_ok = b_streams(whole);
-            fast = a_ok && b_ok;
-            p.ragged = c_streams(whole, sizeof(T)) ? 0 : 1;
-            if (!fast && !segmented && g.batch_rows == 0 && !g.no_split) {
-                bool taken = false;
-                const int s = run_padded<T>(g, !a_ok, !b_ok, stream, &taken);
-                if (taken || s != CGPTX_OK) return s;
-            }
-        }
-        if (p.ragged && segmented) return fail(CGPTX_INVALID_ARGUMENT, "gemm: segmented operands need the aligned MFMA path");
+    GemmArgs whole = g;  // alignment of segmented operands was checked per segment
+    if (g.a_segments.count > 0) {
+        whole.a = g.a_segments.ptr[0];
+        whole.lda = g.a_segments.ld[0];
     }
+    if (g.c_segments.count > 0) {
+        whole.c = const_cast<void*>(g.c_segments.ptr[0]);
+        whole.ldc = g.c_segments.ld[0];
+    }
+    streams = Streams{};
+    if ((g.a_k_contiguous || !g.b_k_contiguous) && offsets_fit_32bit(whole, sizeof(T))) {
+        streams.reach = true;
+        streams.a = a_streams(whole);
+        streams.b = b_streams(whole);
+        p.ragged = c_streams(whole, sizeof(T)) ? 0 : 1;
+    }
+    return CGPTX_OK;
+}
+
+template <typename T>
+int run_typed(const GemmArgs& g, hipStream_t stream) {
+    KernelArgs p;
+    Streams streams;
+    if (int s = describe<T>(g, p, streams)) return s;
+    const bool segmented = g.a_segments.count > 0 || g.c_segments.count > 0;
+    const bool fast = streams.a && streams.b;
+    if (streams.reach && !fast && !segmented && g.batch_rows == 0 && !g.no_split) {
+        bool taken = false;
+        const int s = run_padded<T>(g, !streams.a, !streams.b, stream, &taken);
+        if (taken || s != CGPTX_OK) return s;
+    }
+    if (p.ragged && segmented) return fail(CGPTX_INVALID_ARGUMENT, "gemm: segmented operands need the aligned MFMA path");
     if (!fast && segmented) return fail(CGPTX_INVALID_ARGUMENT, "gemm: segmented operands need the aligned MFMA path");
     if (!fast && g.batch_rows != 0) return fail(CGPTX_INVALID_ARGUMENT, "gemm: a stack of products needs the aligned MFMA path");
     if (!fast) {
@@ -1569,7 +1589,140 @@ int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream, bo
     return run_typed<T>(padded, stream);
 }
 
+// A group's tiles: those whose predicted time in one launch is least. The launch takes as long as its longest workgroup or
+// as the busiest CU's share of the work, whatever is more (us per K tile and workgroup as in predicted_us; 3.5 us before and
+// after the K loops). Joined if that is less than the calls' own predictions in turn. [M, N] x K measured apart and joined:
+// dX and dW of 128 x 768 x 768 10.4 -> 7.7 us, of 2000 x 1024 x 2048 37.4 -> 34.3; 5005 x 1024 x 256, whose dW is better
+// split along K, 23.9 -> 28.8: stays apart.
+struct GroupPlan {
+    int tile[kGroupCalls] = {};
+    long blocks = 0;
+    bool joined = false;
+};
+
+GroupPlan plan_group(const GemmArgs* calls, int count) {
+    GroupPlan best_plan;
+    const double units = static_cast<double>(compute_units());
+    double separate = 0.0;
+    for (int i = 0; i < count; ++i) {
+        const GemmArgs& g = calls[i];
+        const Plan plan = make_plan(g);
+        const long tiles = static_cast<long>((g.m + plan.tile - 1) / plan.tile) * static_cast<long>((g.n + plan.tile - 1) / plan.tile);
+        const bool f32 = g.dtype == CGPTX_F32;
+        const long k_step = f32 ? kBK<float> : kBK<bf16_t>, k_tiles = (static_cast<long>(g.k) + k_step - 1) / k_step;
+        separate += predicted_us(plan.tile, tiles, plan.slices, k_tiles, static_cast<double>(plan.partial_bytes(g)) * 1e-6, f32,
+                                 g.a_k_contiguous, g.b_k_contiguous, compute_units());
+        if (g.a_sums != nullptr) separate += 6.0;  // two launches of their own
+    }
+    double best = separate;
+    for (int choice = 0; choice < 1 << count; ++choice) {
+        double longest = 0.0, work = 0.0, blocks = 0.0;
+        for (int i = 0; i < count; ++i) {
+            const GemmArgs& g = calls[i];
+            const bool f32 = g.dtype == CGPTX_F32, small = ((choice >> i) & 1) != 0;
+            const long edge = small ? 32 : 64, k_step = f32 ? kBK<float> : kBK<bf16_t>;
+            const double kt = static_cast<double>((static_cast<long>(g.k) + k_step - 1) / k_step);
+            const double tiles = static_cast<double>((g.m + edge - 1) / edge) * static_cast<double>((g.n + edge - 1) / edge);
+            const double lone = f32 ? (small ? 0.088 : 0.265) : small ? (!g.a_k_contiguous ? 0.1 : g.b_k_contiguous ? 0.07 : 0.085) : 0.135;
+            const double shared = f32 ? lone : small ? 0.92 * lone : 0.128;
+            longest = std::max(longest, f32 || small ? kt * lone : 0.02 * std::min(kt, 16.0) + std::max(0.0, kt - 16.0) * lone);
+            work += tiles * kt * shared;
+            blocks += tiles;
+        }
+        const double load = blocks / units;
+        if (load > 1.0) longest *= 1.4;  // beside the other workgroup of its CU
+        const double time = 3.5 + std::max(longest, load <= 1.0 ? 0.0 : work / units * std::ceil(load) / load * (load > 4.0 ? 1.3 : 1.0));
+        if (time < best && blocks <= 16.0 * units) {
+            best = time;
+            best_plan.joined = true;
+            best_plan.blocks = static_cast<long>(blocks);
+            for (int i = 0; i < count; ++i) best_plan.tile[i] = ((choice >> i) & 1) != 0 ? 32 : 64;
+        }
+    }
+    return best_plan;
+}
+
+// Whether a call can be part of a group: streamed as it lies, one sum over K, nothing but the plain additions behind it.
+template <typename T>
+bool joinable(const GemmArgs& g, KernelArgs& p) {
+    if (g.a == nullptr && g.a_segments.count == 0) return false;
+    if (g.b == nullptr || g.c == nullptr || g.m == 0 || g.n == 0 || g.k == 0 || g.batch_rows != 0 || g.swiglu_out != nullptr ||
+        g.swiglu_saved != nullptr || g.c_segments.count > 0 || (g.a_sums != nullptr && g.a_k_contiguous) ||
+        (g.a_segments.count > 0 && (!g.a_k_contiguous || g.b_k_contiguous || std::is_same_v<T, float>)))
+        return false;
+    constexpr std::size_t i32max = std::numeric_limits<int>::max();
+    if (g.m > i32max || g.n > i32max || g.k > i32max) return false;
+    GemmArgs whole = g;
+    GemmSegments segments = g.a_segments;
+    whole.a_segments = GemmSegments{};
+    if (segments.count > 0) {
+        whole.a = segments.ptr[0];
+        whole.lda = segments.ld[0];
+    }
+    Streams streams;
+    if (describe<T>(whole, p, streams) != CGPTX_OK || !streams.a || !streams.b) {
+        clear_error();
+        return false;
+    }
+    if (segments.count > 0) {
+        if (copy_segments(segments, g.k, kBK<T>, p.a_seg) != CGPTX_OK || segments.cols[segments.count - 1] % kBK<T> != 0) {
+            clear_error();
+            return false;
+        }
+    }
+    return true;
+}
+
+template <typename T>
+int run_joined(const GemmArgs* calls, int count, const GroupPlan& plan, hipStream_t stream) {
+    SmallGroup group{};
+    long order[kGroupCalls];
+    for (int i = 0; i < count; ++i) order[i] = i;
+    // The workgroups with the longest K loops start first.
+    std::sort(order, order + count, [&](long x, long y) { return calls[x].k * plan.tile[x] > calls[y].k * plan.tile[y]; });
+    int blocks = 0;
+    for (int j = 0; j < count; ++j) {
+        const long i = order[j];
+        const GemmArgs& g = calls[i];
+        KernelArgs p;
+        if (!joinable<T>(g, p)) return fail(CGPTX_RUNTIME, "gemm: this call cannot be part of a group");
+        group.call[j] = small_args(p, false, p.k_tiles);
+        group.call[j].a_sums = g.a_sums;
+        group.call[j].a_sums_accumulate = g.a_sums_accumulate ? 1 : 0;
+        group.first_block[j] = blocks;
+        group.tile[j] = plan.tile[i];
+        group.tiles_m[j] = (p.m + plan.tile[i] - 1) / plan.tile[i];
+        group.layout[j] = !g.a_k_contiguous ? SmallLayout::weight_gradient
+                          : g.b_k_contiguous ? SmallLayout::forward
+                          : p.a_seg.count > 0 ? SmallLayout::segmented_input_gradient : SmallLayout::input_gradient;
+        blocks += group.tiles_m[j] * ((p.n + plan.tile[i] - 1) / plan.tile[i]);
+    }
+    group.count = count;
+    const bool deep = blocks <= compute_units();
+    if constexpr (std::is_same_v<T, bf16_t>) return gemm_small_bf16(group, blocks, deep, stream);
+    else if constexpr (std::is_same_v<T, f16_t>) return gemm_small_f16(group, blocks, deep, stream);
+    else return gemm_small_f32(group, blocks, deep, stream);
+}
+
 }  // namespace
+
+bool gemm_joins(const GemmArgs* calls, int count) {
+    if (count < 2 || count > kGroupCalls || forced_tile() != 0) return false;
+    for (int i = 0; i < count; ++i) {
+        if (calls[i].dtype != calls[0].dtype || !valid_dtype(calls[i].dtype)) return false;
+        KernelArgs p;
+        const bool fits = calls[i].dtype == CGPTX_F32 ? joinable<float>(calls[i], p)
+                          : calls[i].dtype == CGPTX_F16 ? joinable<f16_t>(calls[i], p) : joinable<bf16_t>(calls[i], p);
+        if (!fits) return false;
+    }
+    return plan_group(calls, count).joined;
+}
+
+int gemm_joined(const GemmArgs* calls, int count, hipStream_t stream) {
+    if (!gemm_joins(calls, count)) return fail(CGPTX_RUNTIME, "gemm: these calls cannot share a launch");
+    const GroupPlan plan = plan_group(calls, count);
+    return dispatch_dtype(calls[0].dtype, [&]<typename T>() -> int { return run_joined<T>(calls, count, plan, stream); });
+}
 
 bool gemm_fuses_swiglu(const GemmArgs& g) {
     if (g.swiglu_out == nullptr || g.dtype == CGPTX_F32 || !g.a_k_contiguous || !g.b_k_contiguous || g.bias != nullptr ||

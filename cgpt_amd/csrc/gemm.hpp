@@ -73,9 +73,18 @@ struct GemmArgs {
     std::size_t batch_rows = 0;
     std::size_t a_batch_stride = 0, b_batch_stride = 0;
     std::size_t a_segment_batch_stride[3] = {0, 0, 0};
+    // Weight gradient of a call in a group (gemm_joins) only: the sums of A's columns, [m] in the storage dtype (a bias's
+    // gradient), added to what is there if a_sums_accumulate.
+    void* a_sums = nullptr;
+    bool a_sums_accumulate = false;
 };
 
 int gemm(const GemmArgs& args, hipStream_t stream);
+// Up to four calls that neither read nor write each other's results, in one launch: whether that is served and faster than
+// one after the other (few tiles each, operands that stream as they lie), and the launch itself.
+constexpr int kGroupCalls = 4;
+bool gemm_joins(const GemmArgs* calls, int count);
+int gemm_joined(const GemmArgs* calls, int count, hipStream_t stream);
 // Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
 std::size_t gemm_split_bytes(const GemmArgs& args);
 // Copies [rows, cols] elements (row stride ld) to rows of `pitch` elements (whole 16-byte chunks), zeros past cols.

@@ -27,6 +27,9 @@ struct SmallArgs {
     const float* addend;
     long ldr, ld_addend;
     int accumulate, c_f32, ragged;
+    // grouped weight gradients: sums of A's columns, T*, or null
+    void* a_sums;
+    int a_sums_accumulate;
     // segmented operands
     SmallSegments a_seg, c_seg;
 };
@@ -42,8 +45,22 @@ struct SmallCall {
     int slices;
 };
 
+// Several calls in one launch: call i takes the workgroups from first_block[i] on, tile rows first.
+enum class SmallLayout { forward, input_gradient, weight_gradient, segmented_input_gradient };
+struct SmallGroup {
+    SmallArgs call[kGroupCalls];
+    int first_block[kGroupCalls];
+    int tiles_m[kGroupCalls];
+    int tile[kGroupCalls];  // 32 or 64
+    SmallLayout layout[kGroupCalls];
+    int count;
+};
+
 int gemm_small_bf16(const SmallCall& call, hipStream_t stream);
 int gemm_small_f16(const SmallCall& call, hipStream_t stream);
 int gemm_small_f32(const SmallCall& call, hipStream_t stream);
+int gemm_small_bf16(const SmallGroup& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_f16(const SmallGroup& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_f32(const SmallGroup& group, int blocks, bool deep, hipStream_t stream);
 
 }  // namespace cgptx

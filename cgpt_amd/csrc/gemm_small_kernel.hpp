@@ -25,23 +25,28 @@ __device__ __forceinline__ void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(COUNT) : "memory");
 }
 
+// One of three values, all of them read first: a choice between places would keep the arguments in memory.
+template <typename V>
+__device__ __forceinline__ V one_of(bool in1, bool in2, V v0, V v1, V v2) { return in2 ? v2 : in1 ? v1 : v0; }
+
 __device__ __forceinline__ SegmentPick pick_small_segment(const SmallSegments& seg, int col) {
-    KernelSegments s;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        s.ptr[i] = seg.ptr[i];
-        s.ld[i] = seg.ld[i];
-        s.cols[i] = seg.cols[i];
-    }
-    s.count = seg.count;
-    return pick_segment(s, col);
+    const int cols0 = seg.cols[0], cols1 = seg.cols[1], cols2 = seg.cols[2], end0 = cols0, end1 = end0 + cols1;
+    const bool in1 = seg.count > 1 && col >= end0, in2 = seg.count > 2 && col >= end1;
+    SegmentPick pick;
+    pick.ptr = one_of(in1, in2, seg.ptr[0], seg.ptr[1], seg.ptr[2]);
+    pick.ld = one_of(in1, in2, seg.ld[0], seg.ld[1], seg.ld[2]);
+    pick.first = one_of(in1, in2, 0, end0, end1);
+    pick.cols = one_of(in1, in2, cols0, cols1, cols2);
+    pick.index = one_of(in1, in2, 0, 1, 2);
+    return pick;
 }
 
 template <int TILE, bool DEEP>
 constexpr int small_smem_bytes() { return DEEP ? 128 * 1024 : 64 * 1024; }
 
-template <typename T, int TILE, bool DEEP, bool A_K, bool B_K, SmallEpilogue EPILOGUE, bool SEGMENTED>
-__global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
+// The tile at (m0, n0) of one call. SUMS: sums of A's columns beside it, by the workgroups of the first tile column.
+template <typename T, int TILE, bool DEEP, bool A_K, bool B_K, SmallEpilogue EPILOGUE, bool SEGMENTED, bool SUMS>
+__device__ __forceinline__ void small_tile(const SmallArgs& p, int m0, int n0, int slice, unsigned char* smem_raw) {
     using frag_t = typename Mfma<T>::frag;
     using ATile = std::conditional_t<A_K, KTile<T, TILE>, NTile<T, TILE>>;
     using BTile = std::conditional_t<B_K, KTile<T, TILE>, NTile<T, TILE>>;
@@ -51,21 +56,37 @@ __global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
     constexpr int kLoadBytes = 1024, kOperandLoads = kOperandBytes / kLoadBytes, kLoads = 2 * kOperandLoads;
     constexpr int STAGES = small_smem_bytes<TILE, DEEP>() / (kWaves * kStageBytes);
     static_assert(STAGES >= 2 && STAGES * kLoads < 64, "the loads in flight are counted by vmcnt");
-    extern __shared__ __align__(1024) unsigned char smem_raw[];
+    static_assert(!SUMS || !A_K, "columns of A are summed where its rows are K positions");
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
 
-    // Workgroups go to the XCDs round-robin, tile rows first: an XCD reads its share of A's panels and all of B.
-    const int m0 = blockIdx.x * TILE, n0 = blockIdx.y * TILE, slice = blockIdx.z;
     const int kt_begin = slice * p.k_tiles_per_slice, kt_end = min(p.k_tiles, kt_begin + p.k_tiles_per_slice);
     const int steps = max(0, (kt_end - kt_begin - wave + kWaves - 1) / kWaves);  // K tiles kt_begin + wave + kWaves i
 
     // Sources. A in column segments: along K (k-contiguous) the segment is picked per K tile, along M once.
     ATile a_src;
     BTile b_src;
-    if constexpr (A_K) {
-        if (!SEGMENTED || p.a_seg.count == 0)
-            a_src.init(static_cast<const T*>(p.a) + static_cast<long>(m0) * p.lda, p.lda, p.a_extent - m0, p.k, 0);
+    // In segments along K all three are set up (absent ones repeat the first and are never picked), and a K tile's is
+    // picked field by field: selecting an object would keep all of them in memory.
+    ATile a_src1, a_src2;
+    int a_end0 = std::numeric_limits<int>::max(), a_end1 = std::numeric_limits<int>::max();
+    if constexpr (A_K && SEGMENTED) {
+        const int count = p.a_seg.count;
+        const void* base0 = one_of(count == 0, false, p.a_seg.ptr[0], p.a, p.a);
+        const long ld0 = one_of(count == 0, false, p.a_seg.ld[0], p.lda, p.lda);
+        const int cols0 = one_of(count == 0, false, p.a_seg.cols[0], p.k, p.k), rows = p.m - m0;
+        auto segment = [&](ATile& source, const void* base, long ld, int cols) __attribute__((always_inline)) {
+            source.init(static_cast<const T*>(base) + static_cast<long>(m0) * ld, ld, rows, cols, 0);
+        };
+        segment(a_src, base0, ld0, cols0);
+        segment(a_src1, one_of(count > 1, false, base0, p.a_seg.ptr[1], base0), one_of(count > 1, false, ld0, p.a_seg.ld[1], ld0),
+                one_of(count > 1, false, cols0, p.a_seg.cols[1], cols0));
+        segment(a_src2, one_of(count > 2, false, base0, p.a_seg.ptr[2], base0), one_of(count > 2, false, ld0, p.a_seg.ld[2], ld0),
+                one_of(count > 2, false, cols0, p.a_seg.cols[2], cols0));
+        if (count > 1) a_end0 = cols0;
+        if (count > 2) a_end1 = cols0 + p.a_seg.cols[1];
+    } else if constexpr (A_K) {
+        a_src.init(static_cast<const T*>(p.a) + static_cast<long>(m0) * p.lda, p.lda, p.a_extent - m0, p.k, 0);
     } else {
         const T* base = static_cast<const T*>(p.a) + m0;
         long ld = p.lda;
@@ -88,22 +109,36 @@ __global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
     constexpr int kStageElems = kStageBytes / static_cast<int>(sizeof(T)), kOperandElems = kStageElems / 2;
     // Step i's loads; past the last one they read zeros from beyond the buffers, so that every step issues the same number.
     unsigned int a_soffset = 0, b_soffset = 0;
+    u32x4 a_rsrc = a_src.rsrc;
+    int a_voffset = a_src.voffset;
+    unsigned int a_step = a_src.group_bytes;
     auto aim = [&](int i) __attribute__((always_inline)) {
         const unsigned int past_end = i >= steps ? 0x80000000u : 0u;
         const int k0 = min(kt_begin + wave + kWaves * i, p.k_tiles - 1) * kBK<T>;
-        a_soffset = a_src.first_offset(k0, 0) | past_end;
         if constexpr (A_K && SEGMENTED) {
-            if (p.a_seg.count > 0) {
-                const SegmentPick pick = pick_small_segment(p.a_seg, k0);
-                a_src.init(static_cast<const T*>(pick.ptr) + static_cast<long>(m0) * pick.ld, pick.ld, p.m - m0, pick.cols, 0);
-                a_soffset = a_src.first_offset(k0 - pick.first, 0) | past_end;
+            const bool in1 = k0 >= a_end0, in2 = k0 >= a_end1;
+            const u32x4 rsrc0 = a_src.rsrc, rsrc1 = a_src1.rsrc, rsrc2 = a_src2.rsrc;
+            const int voffset0 = a_src.voffset, voffset1 = a_src1.voffset, voffset2 = a_src2.voffset;
+            const unsigned int bytes0 = a_src.group_bytes, bytes1 = a_src1.group_bytes, bytes2 = a_src2.group_bytes;
+            const int end0 = a_end0, end1 = a_end1;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned int w0 = rsrc0[e], w1 = rsrc1[e], w2 = rsrc2[e];
+                a_rsrc[e] = in2 ? w2 : in1 ? w1 : w0;
             }
+            a_voffset = in2 ? voffset2 : in1 ? voffset1 : voffset0;
+            a_step = in2 ? bytes2 : in1 ? bytes1 : bytes0;
+            a_soffset = (k0 - (in2 ? end1 : in1 ? end0 : 0)) * static_cast<unsigned int>(sizeof(T)) | past_end;
+        } else {
+            a_soffset = a_src.first_offset(k0, 0) | past_end;
         }
         b_soffset = b_src.first_offset(k0, 0) | past_end;
     };
     auto issue = [&](auto index, unsigned int stage_lds) __attribute__((always_inline)) {
         constexpr int l = decltype(index)::value;
-        if constexpr (l < kOperandLoads)
+        if constexpr (l < kOperandLoads && A_K && SEGMENTED)
+            a_soffset = load_to_lds<l * kLoadBytes>(a_rsrc, stage_lds, a_voffset, a_soffset, a_step);
+        else if constexpr (l < kOperandLoads)
             a_soffset = load_to_lds<l * kLoadBytes>(a_src.rsrc, stage_lds, a_src.load_voffset(l), a_soffset, a_src.group_bytes);
         else
             b_soffset = load_to_lds<l * kLoadBytes>(b_src.rsrc, stage_lds, b_src.load_voffset(l - kOperandLoads), b_soffset, b_src.group_bytes);
@@ -137,6 +172,18 @@ __global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
     for (int i = 0; i < kBlocks; ++i)
 #pragma unroll
         for (int j = 0; j < kBlocks; ++j) acc[i][j] = acc_t(0.0f);
+    // The column sums are one more block of columns whose B is ones.
+    const bool sums = SUMS && p.a_sums != nullptr && n0 == 0;
+    acc_t column_sums[SUMS ? kBlocks : 1];
+    frag_t ones;
+    if constexpr (SUMS) {
+#pragma unroll
+        for (int i = 0; i < kBlocks; ++i) column_sums[i] = acc_t(0.0f);
+#pragma unroll
+        for (int e = 0; e < static_cast<int>(sizeof(frag_t) / sizeof(T)); ++e) ones[e] = static_cast<T>(1.0f);
+        // Kept in registers: written again in front of its MFMA, it would need wait states that assembly has to bring itself.
+        asm volatile("" : "+v"(ones));
+    }
     wait_loads<(STAGES - 1) * kLoads>();
     static_for<0, 2 * kBlocks>([&](auto f) { read_frag.template operator()<0, decltype(f)::value>(wave_stages); });
     int stage = 0;
@@ -161,6 +208,13 @@ __global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
             }
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (SUMS) {
+            if (sums) {
+                asm volatile("s_nop 1" : "+v"(ones));
+#pragma unroll
+                for (int i = 0; i < kBlocks; ++i) Mfma<T>::run(column_sums[i], ones, af[BUFFER][i]);
+            }
+        }
         stage = next_stage;
     };
     for (int i = 0; i < steps; i += 2) {
@@ -182,8 +236,24 @@ __global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
         for (int i = 0; i < kBlocks; ++i)
 #pragma unroll
             for (int j = 0; j < kBlocks; ++j) *reinterpret_cast<acc_t*>(mine + i * 16 * kPitch + j * 16) = acc[i][j];
+        if constexpr (SUMS) {
+            // Row r's sum into the padding behind the row: every lane of row lane%16 holds it.
+#pragma unroll
+            for (int i = 0; i < kBlocks; ++i)
+                if (sums && lane < 16) partial[wave * TILE * kPitch + (i * 16 + lane) * kPitch + TILE] = column_sums[i][0];
+        }
     }
     __syncthreads();
+    if constexpr (SUMS) {
+        if (sums && threadIdx.x < TILE && m0 + static_cast<int>(threadIdx.x) < p.m) {
+            const float* from = partial + threadIdx.x * kPitch + TILE;
+            float v = from[0];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) v += from[w * TILE * kPitch];
+            T* out = static_cast<T*>(p.a_sums) + m0 + threadIdx.x;
+            *out = from_f32<T>(p.a_sums_accumulate ? v + to_f32(*out) : v);
+        }
+    }
     void* c_base = p.c;
     long c_ld = p.ldc;
     int c_col0 = n0, c_cols = p.n;
@@ -270,6 +340,81 @@ __global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
             }
         }
     }
+}
+
+template <typename T, int TILE, bool DEEP, bool A_K, bool B_K, SmallEpilogue EPILOGUE, bool SEGMENTED>
+__global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
+    extern __shared__ __align__(1024) unsigned char smem_raw[];
+    // Workgroups go to the XCDs round-robin, tile rows first: an XCD reads its share of A's panels and all of B.
+    small_tile<T, TILE, DEEP, A_K, B_K, EPILOGUE, SEGMENTED, false>(p, blockIdx.x * TILE, blockIdx.y * TILE, blockIdx.z, smem_raw);
+}
+
+// Several calls in one launch. A launch of its own costs a small call more than its work does (2 us of start and end
+// around 1 - 2 us), and two calls of a few dozen tiles each find room on the chip side by side. Both gradients of a
+// projection, us in two launches and in one: 128 x 768 x 768 bf16 10.4, 7.7; 512 x 512 x 512 11.0, 7.4; 128 x 768 x 2048 fp32
+// 23.0, 15.7; 2000 x 1024 x 2048 bf16 with bias 46, 34 (the bias's gradient took two launches more).
+template <typename T, bool DEEP>
+__global__ __launch_bounds__(kThreads) void gemm_small_group_kernel(SmallGroup group) {
+    extern __shared__ __align__(1024) unsigned char smem_raw[];
+    const int block = blockIdx.x;
+    int which = 0;
+#pragma unroll
+    for (int i = 1; i < kGroupCalls; ++i)
+        if (i < group.count && block >= group.first_block[i]) which = i;
+    int first = 0, tiles_m = 0, tile = 0;
+    SmallLayout layout = SmallLayout::forward;
+#pragma unroll
+    for (int i = 0; i < kGroupCalls; ++i) {
+        const int first_i = group.first_block[i], tiles_i = group.tiles_m[i], tile_i = group.tile[i];
+        const SmallLayout layout_i = group.layout[i];
+        first = which == i ? first_i : first;
+        tiles_m = which == i ? tiles_i : tiles_m;
+        tile = which == i ? tile_i : tile;
+        layout = which == i ? layout_i : layout;
+    }
+    // The call's arguments, read where they lie (the group is the kernel's only argument): indexing the parameter by a
+    // run-time value would copy it to private memory.
+    constexpr int kWords = sizeof(SmallArgs) / 4;
+    struct Words {
+        unsigned int w[kWords];
+    } words;
+    const auto* source = (const __attribute__((address_space(4))) unsigned int*)__builtin_amdgcn_kernarg_segment_ptr() +
+                         offsetof(SmallGroup, call) / 4 + which * kWords;
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) words.w[i] = source[i];
+    const SmallArgs p = __builtin_bit_cast(SmallArgs, words);
+    const int index = block - first;
+    const int column = index / tiles_m, row = index - column * tiles_m;
+    auto with_tile = [&]<int TILE>() __attribute__((always_inline)) {
+        const int m0 = row * TILE, n0 = column * TILE;
+        if (layout == SmallLayout::weight_gradient)
+            small_tile<T, TILE, DEEP, false, false, SmallEpilogue::general, false, true>(p, m0, n0, 0, smem_raw);
+        else if (layout == SmallLayout::input_gradient)
+            small_tile<T, TILE, DEEP, true, false, SmallEpilogue::general, false, false>(p, m0, n0, 0, smem_raw);
+        else if (layout == SmallLayout::forward)
+            small_tile<T, TILE, DEEP, true, true, SmallEpilogue::general, false, false>(p, m0, n0, 0, smem_raw);
+        else if constexpr (sizeof(T) == 2)
+            small_tile<T, TILE, DEEP, true, false, SmallEpilogue::general, true, false>(p, m0, n0, 0, smem_raw);
+    };
+    if (tile == 32) with_tile.template operator()<32>();
+    else with_tile.template operator()<64>();
+}
+
+template <typename T, bool DEEP>
+int launch_small_group_kernel(const SmallGroup& group, int blocks, hipStream_t stream) {
+    constexpr int smem = small_smem_bytes<64, DEEP>() + (DEEP ? 0 : 8192);  // 64 x 64 partial tiles need 68 KiB
+    auto kernel = gemm_small_group_kernel<T, DEEP>;
+    static const hipError_t status =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    CGPTX_HIP(status);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), smem, stream, group);
+    CGPTX_LAUNCH_CHECK();
+    return CGPTX_OK;
+}
+
+template <typename T>
+int launch_small_group(const SmallGroup& group, int blocks, bool deep, hipStream_t stream) {
+    return deep ? launch_small_group_kernel<T, true>(group, blocks, stream) : launch_small_group_kernel<T, false>(group, blocks, stream);
 }
 
 template <typename T, int TILE, bool DEEP, bool A_K, bool B_K, SmallEpilogue EPILOGUE, bool SEGMENTED>

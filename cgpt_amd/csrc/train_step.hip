@@ -270,10 +270,14 @@ int linear_backward_split(cgptx_model* m, void* dx, void* dw, const void* dy, co
                           std::size_t rows, std::size_t in_features, std::size_t out_features, int accumulate_input,
                           int dt, hipStream_t stream, const char* dx_label, const char* dw_label) {
     auto* s = static_cast<cgptx_stream>(stream);
+    // In one call, which may run both in one launch, unless each is to be timed.
+    if (!m->profiling)
+        return cgptx_linear_backward(dx, dw, nullptr, dy, x, w, rows, in_features, out_features, accumulate_input, 0, 0, dt, s);
     CGPTX_OP(dx_label, cgptx_linear_backward(dx, nullptr, nullptr, dy, x, w, rows, in_features, out_features,
                                               accumulate_input, 0, 0, dt, s));
-    CGPTX_OP(dw_label, cgptx_linear_backward(nullptr, dw, nullptr, dy, x, w, rows, in_features, out_features, 0, 0,
-                                              0, dt, s));
+    if (dw != nullptr)
+        CGPTX_OP(dw_label, cgptx_linear_backward(nullptr, dw, nullptr, dy, x, w, rows, in_features, out_features, 0, 0,
+                                                 0, dt, s));
     return CGPTX_OK;
 }
 
@@ -329,8 +333,8 @@ int qkv_forward(void* q, void* k, void* v, const void* x, const void* qkv_weight
 }
 
 // dX = [dq | dk | dv]·[Wq; Wk; Wv] in one launch.
-int qkv_backward_input(void* dx, const void* dq, const void* dk, const void* dv, const void* qkv_weight,
-                       std::size_t rows, std::size_t H, std::size_t QW, std::size_t KW, int dt, hipStream_t stream) {
+GemmArgs qkv_input_gradient(void* dx, const void* dq, const void* dk, const void* dv, const void* qkv_weight,
+                            std::size_t rows, std::size_t H, std::size_t QW, std::size_t KW, int dt) {
     GemmArgs g;
     g.a_segments = qkv_segments(dq, dk, dv, QW, KW);
     g.b = qkv_weight;
@@ -342,7 +346,43 @@ int qkv_backward_input(void* dx, const void* dq, const void* dk, const void* dv,
     g.ldc = H;
     g.b_k_contiguous = false;
     g.dtype = dt;
-    return gemm(g, stream);
+    return g;
+}
+
+// The parts of the same as calls of their own, for shapes whose tiles do not respect the segments: one launch as a group
+// where that pays (gemm_joins). Y = X·Wᵀ:
+GemmArgs projection(void* y, const void* x, const void* weight, std::size_t rows, std::size_t in_features,
+                    std::size_t out_features, int dt) {
+    GemmArgs g;
+    g.a = x;
+    g.b = weight;
+    g.c = y;
+    g.m = rows;
+    g.n = out_features;
+    g.k = in_features;
+    g.lda = in_features;
+    g.ldb = in_features;
+    g.ldc = out_features;
+    g.dtype = dt;
+    return g;
+}
+// dW = dYᵀ·X:
+GemmArgs projection_weight_gradient(void* grad_weight, const void* dy, const void* x, std::size_t rows, std::size_t in_features,
+                                    std::size_t out_features, int dt) {
+    GemmArgs g;
+    g.a = dy;
+    g.b = x;
+    g.c = grad_weight;
+    g.m = out_features;
+    g.n = in_features;
+    g.k = rows;
+    g.lda = out_features;
+    g.ldb = in_features;
+    g.ldc = in_features;
+    g.a_k_contiguous = false;
+    g.b_k_contiguous = false;
+    g.dtype = dt;
+    return g;
 }
 
 // [dWq; dWk; dWv] = [dq | dk | dv]ᵀ·X in one launch.
@@ -688,6 +728,11 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         }
         if (fused_qkv) {
             CGPTX_OP("gemm_fwd.qkv", qkv_forward(a.q_pre, a.k_pre, a.v, a.norm_a, w.q.value, N, H, QW, KW, dt, stream));
+        } else if (const GemmArgs qkv[3] = {projection(a.q_pre, a.norm_a, w.q.value, N, H, QW, dt),
+                                            projection(a.k_pre, a.norm_a, w.k.value, N, H, KW, dt),
+                                            projection(a.v, a.norm_a, w.v.value, N, H, KW, dt)};
+                   gemm_joins(qkv, 3)) {
+            CGPTX_OP("gemm_fwd.qkv", gemm_joined(qkv, 3, stream));
         } else {
             CGPTX_OP("gemm_fwd.qkv", cgptx_linear_forward(a.q_pre, a.norm_a, w.q.value, nullptr, N, H, QW, dt, s));
             CGPTX_OP("gemm_fwd.qkv", cgptx_linear_forward(a.k_pre, a.norm_a, w.k.value, nullptr, N, H, KW, dt, s));
@@ -759,9 +804,7 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             if (!stacked)
                 CGPTX_OP("gemm_dw.down", cgptx_linear_backward(nullptr, w.down.gradient, nullptr, current, a.act, w.down.value, N, I, H, 0, 0, 0, dt, s));
         } else {
-            CGPTX_OP("gemm_dx.down", cgptx_linear_backward(m->d_act, nullptr, nullptr, current, a.act, w.down.value, N, I, H, 0, 0, 0, dt, s));
-            if (!stacked)
-                CGPTX_OP("gemm_dw.down", cgptx_linear_backward(nullptr, w.down.gradient, nullptr, current, a.act, w.down.value, N, I, H, 0, 0, 0, dt, s));
+            CGPTX_TRY(linear_backward_split(m, m->d_act, stacked ? nullptr : w.down.gradient, current, a.act, w.down.value, N, I, H, 0, dt, stream, "gemm_dx.down", "gemm_dw.down"));
             CGPTX_OP("swiglu_bwd", cgptx_swiglu_backward_packed(d_gate_up, m->d_act, a.gate_up, N, I, 0, dt, s));
         }
         // The gradient of the residual stream collects the two norm branches: in one pass at the end of
@@ -770,16 +813,12 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         const bool dual_norms = fused_block_norms(m, previous, m->d_norm_in, m->d_norm_in_f, x, current) &&
                                 is_aligned16(w.attention_norm.value) && is_aligned16(w.ffn_norm.value);
         void* d_norm_f = dual_norms ? m->d_norm_in_f : m->d_norm_in;
-        CGPTX_OP("gemm_dx.gate_up", cgptx_linear_backward(d_norm_f, nullptr, nullptr, d_gate_up, a.norm_f, w.gate.value, N, H, 2 * I, 0, 0, 0, dt, s));
-        if (!stacked)
-            CGPTX_OP("gemm_dw.gate_up", cgptx_linear_backward(nullptr, w.gate.gradient, nullptr, d_gate_up, a.norm_f, w.gate.value, N, H, 2 * I, 0, 0, 0, dt, s));
+        CGPTX_TRY(linear_backward_split(m, d_norm_f, stacked ? nullptr : w.gate.gradient, d_gate_up, a.norm_f, w.gate.value, N, H, 2 * I, 0, dt, stream, "gemm_dx.gate_up", "gemm_dw.gate_up"));
         if (!dual_norms) {
             CGPTX_OP("rmsnorm_bwd", rmsnorm_backward_residual(previous, w.ffn_norm.gradient, m->d_norm_in, x, w.ffn_norm.value,
                                                               current, N, H, eps, dt, stream, sink));
         }
-        CGPTX_OP("gemm_dx.o", cgptx_linear_backward(m->d_attn_out, nullptr, nullptr, current, a.attn_out, w.o.value, N, QW, H, 0, 0, 0, dt, s));
-        if (!stacked)
-            CGPTX_OP("gemm_dw.o", cgptx_linear_backward(nullptr, w.o.gradient, nullptr, current, a.attn_out, w.o.value, N, QW, H, 0, 0, 0, dt, s));
+        CGPTX_TRY(linear_backward_split(m, m->d_attn_out, stacked ? nullptr : w.o.gradient, current, a.attn_out, w.o.value, N, QW, H, 0, dt, stream, "gemm_dx.o", "gemm_dw.o"));
         CGPTX_OP("attn_bwd", cgptx_flash_gqa_attention_backward_with_lse(d_q, d_k, d_v, m->d_attn_out, a.attn_out,
                                                               a.lse, a.q, a.k, a.v, m->batch, m->sequence,
                                                               m->sequence, HQ, HKV, D, 0.0f, 1, 0, 0, dt, s));
@@ -799,9 +838,15 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
                                                               N * HKV, D, eps, dt, stream, sink));
         }
         if (fused_qkv) {
-            CGPTX_OP("gemm_dx.qkv", qkv_backward_input(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt, stream));
+            CGPTX_OP("gemm_dx.qkv", gemm(qkv_input_gradient(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt), stream));
             if (!stacked)
                 CGPTX_OP("gemm_dw.qkv", qkv_backward_weight(w.q.gradient, d_q, d_k, d_v, a.norm_a, N, H, QW, KW, dt, stream));
+        } else if (const GemmArgs qkv[4] = {qkv_input_gradient(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt),
+                                            projection_weight_gradient(w.q.gradient, d_q, a.norm_a, N, H, QW, dt),
+                                            projection_weight_gradient(w.k.gradient, d_k, a.norm_a, N, H, KW, dt),
+                                            projection_weight_gradient(w.v.gradient, d_v, a.norm_a, N, H, KW, dt)};
+                   gemm_joins(qkv, 4)) {
+            CGPTX_OP("gemm_dx.qkv", gemm_joined(qkv, 4, stream));
         } else {
             CGPTX_TRY(linear_backward_split(m, m->d_norm_in, w.q.gradient, d_q, a.norm_a, w.q.value, N, H, QW, 0, dt, stream, "gemm_dx.qkv", "gemm_dw.qkv"));
             CGPTX_TRY(linear_backward_split(m, m->d_norm_in, w.k.gradient, d_k, a.norm_a, w.k.value, N, H, KW, 1, dt, stream, "gemm_dx.qkv", "gemm_dw.qkv"));

@@ -86,6 +86,29 @@ def test_contractions_whose_last_k_tile_is_half_filled_are_exact_on_integers(dev
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("rows,fin,fout", [
+    (1, 64, 64), (31, 64, 32), (33, 40, 72), (300, 256, 100),   # tiles of 32 and 64, one and more per gradient, ragged edges
+    (128, 768, 2048), (2000, 1024, 2048), (1999, 1000, 2040),   # more workgroups than compute units
+    (70, 256, 5003),                                            # output gradient in padded rows
+])
+def test_linear_gradients_in_one_launch_are_exact_on_integers(device, rows, fin, fout, accumulate, dtype):
+    """dX, dW and db of a small call share a launch. Products and sums of small integers are exact in fp32 (at most 4 x 5003 + 2),
+    so every result is the rounded exact value; all three overwritten and all three added to what is there."""
+    g = torch.Generator().manual_seed(rows + fin + fout)
+    ints = lambda *shape: torch.randint(-2, 3, shape, generator=g).double()
+    x, w, dy = ints(rows, fin), ints(fout, fin), ints(rows, fout)
+    start = {"dX": ints(rows, fin), "dW": ints(fout, fin), "db": ints(fout)}
+    got = {name: t.to(dtype).to(device) if accumulate else torch.full(t.shape, float("nan"), dtype=dtype, device=device)
+           for name, t in start.items()}
+    ops.linear_backward(got["dX"], got["dW"], got["db"], dy.to(dtype).to(device), x.to(dtype).to(device), w.to(dtype).to(device),
+                        options=ops.LinearBackwardOptions(accumulate_input=accumulate, accumulate_weight=accumulate,
+                                                          accumulate_bias=accumulate))
+    for name, exact in (("dX", dy @ w), ("dW", dy.T @ x), ("db", dy.sum(0))):
+        assert torch.equal(got[name].cpu(), (exact + (start[name] if accumulate else 0)).to(dtype)), name
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
 @pytest.mark.parametrize("vectors", [1024, 1025, 4096, 4097, 8192, 8193, 16384, 16385])
 @pytest.mark.parametrize("tail", [0, 1])
 def test_cross_entropy_around_the_held_row_lengths(device, vectors, tail, dtype):
