@@ -125,20 +125,18 @@ int dispatch_dtype(int dtype, Fn&& fn) {
     }
 }
 
-// ---- weight-gradient reductions of several norm-backward passes as one pair of launches ----------
+// ---- weight-gradient reductions of several norm-backward passes in one launch ---------------------
 // A norm-backward pass leaves per-workgroup partial sums of the weight gradient [parts, hidden] and reduces them
-// over the parts in two small launches. A caller that runs many such passes (the train step: four per block) may
+// over the parts in a small launch. A caller that runs many such passes (the train step: four per block) may
 // hand them a sink instead: the pass then takes its partial-sum memory from the sink (which must outlive the pass,
 // unlike the per-stream arena that the next operator reuses), records what is to be reduced, and the caller runs
-// all recorded reductions with run_column_reductions — the same arithmetic in the same order, two launches in all.
+// all recorded reductions with run_column_reductions — the same arithmetic in the same order, one launch in all.
 struct ColumnReduceEntry {
     const float* partial;  // [parts, hidden]
-    float* second;         // [slices, hidden] (used when slices > 1)
     void* out;             // T[hidden]
-    int parts, hidden, slices, dtype;
+    int parts, hidden, dtype;
     bool operator==(const ColumnReduceEntry& o) const {
-        return partial == o.partial && second == o.second && out == o.out && parts == o.parts && hidden == o.hidden &&
-               slices == o.slices && dtype == o.dtype;
+        return partial == o.partial && out == o.out && parts == o.parts && hidden == o.hidden && dtype == o.dtype;
     }
 };
 struct ColumnReduceSink {
@@ -165,9 +163,8 @@ struct ColumnReduceSink {
 // Bytes one norm-backward pass of the given kind takes from a sink (0: that shape reduces at once, from the arena).
 enum class NormPass { plain, with_rope, dual };
 std::size_t rmsnorm_backward_sink_bytes(NormPass pass, std::size_t rows, std::size_t hidden, int dtype);
-// Runs the reductions recorded in `table` (device copy of `count` entries). max_hidden / max_slices: the largest
-// values among the entries (they size the grid).
-int run_column_reductions(const ColumnReduceEntry* table, int count, int max_hidden, int max_slices, hipStream_t stream);
+// Runs the reductions recorded in `table` (device copy of `entries`).
+int run_column_reductions(const ColumnReduceEntry* table, const std::vector<ColumnReduceEntry>& entries, hipStream_t stream);
 
 // ---- fused variants used by the composed train step --------------------------
 // rmsnorm backward with grad_input = (norm gradient) + residual; residual may be null or alias

@@ -263,8 +263,7 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
                                stream, partial, static_cast<const T*>(grad_output), static_cast<long>(rows), cols,
                                rows_per_slice);
             CGPTX_LAUNCH_CHECK();
-            hipLaunchKernelGGL((column_partial_reduce_kernel<T>), dim3(col_blocks), dim3(kReduceThreads), 0, stream,
-                               static_cast<T*>(grad_bias), partial, slices, cols, accumulate_bias != 0 ? 1 : 0);
+            launch_column_partial_reduce<T>(static_cast<T*>(grad_bias), partial, slices, cols, accumulate_bias != 0 ? 1 : 0, stream);
             CGPTX_LAUNCH_CHECK();
             return CGPTX_OK;
         });

@@ -8,108 +8,79 @@ namespace cgptx {
 constexpr int kReduceThreads = 256;
 constexpr int kReduceWaves = kReduceThreads / kWave;
 
-// Sums partial[P, H] over P in a fixed order and stores (or adds) in T; `group` = which 64 columns.
-template <typename T>
+// Sums partial[P, H] over P in a fixed order and stores (or adds) in T; `group` = which kColumns columns. The partial sums
+// have just been written by the whole chip, so every load is a trip to memory: what counts is how many are in flight. A
+// workgroup of 1024 threads takes 32 columns (16 of narrow matrices, so that more workgroups share them), a thread eight
+// parts at a time; up to a few thousand parts, what the chip holds of the kernels that leave them, one launch does: 1024 x
+// 1024 4.7 us, 1792 x 128 5.7, where two launches (sums over sixteen and more parts, sums of those) took 9.4 and 9.3.
+constexpr int kFinishThreads = 1024;
+constexpr int finish_columns(int hidden) { return hidden <= 256 ? 16 : 32; }
+
+template <typename T, int COLUMNS>
 __device__ __forceinline__ void column_partial_reduce_body(T* __restrict__ out, const float* __restrict__ partial,
                                                            int parts, int hidden, int accumulate, int group) {
-    __shared__ float stage[kReduceWaves][kWave];
-    const int lane = threadIdx.x & (kWave - 1);
-    const int slice = threadIdx.x / kWave;
-    const int col = group * kWave + lane;
-    float v0 = 0.0f, v1 = 0.0f, v2 = 0.0f, v3 = 0.0f;
-    if (col < hidden) {
-        int p = slice;
-        for (; p + 3 * kReduceWaves < parts; p += 4 * kReduceWaves) {
-            v0 += partial[static_cast<std::size_t>(p) * hidden + col];
-            v1 += partial[static_cast<std::size_t>(p + kReduceWaves) * hidden + col];
-            v2 += partial[static_cast<std::size_t>(p + 2 * kReduceWaves) * hidden + col];
-            v3 += partial[static_cast<std::size_t>(p + 3 * kReduceWaves) * hidden + col];
-        }
-        for (; p < parts; p += kReduceWaves) v0 += partial[static_cast<std::size_t>(p) * hidden + col];
-    }
-    stage[slice][lane] = (v0 + v1) + (v2 + v3);
-    __syncthreads();
-    if (slice == 0 && col < hidden) {
-        float v = 0.0f;
+    constexpr int kWaves16 = kFinishThreads / kWave, kSlices = kFinishThreads / COLUMNS;
+    __shared__ float stage[kWaves16][COLUMNS];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int slice = threadIdx.x / COLUMNS;
+    const int col = group * COLUMNS + threadIdx.x % COLUMNS;
+    float v[8];
 #pragma unroll
-        for (int s = 0; s < kReduceWaves; ++s) v += stage[s][lane];
-        if (accumulate) v += to_f32(out[col]);
-        out[col] = from_f32<T>(v);
+    for (int u = 0; u < 8; ++u) v[u] = 0.0f;
+    if (col < hidden) {
+        const float* from = partial + col;
+        int p = slice;
+        for (; p + 7 * kSlices < parts; p += 8 * kSlices) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] += from[static_cast<std::size_t>(p + u * kSlices) * hidden];
+        }
+#pragma unroll
+        for (int u = 0; u < 7; ++u)
+            if (p + u * kSlices < parts) v[u] += from[static_cast<std::size_t>(p + u * kSlices) * hidden];
     }
+    float total = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+#pragma unroll
+    for (int offset = COLUMNS; offset < kWave; offset <<= 1) total += __shfl_xor(total, offset, kWave);
+    if (lane < COLUMNS) stage[wave][lane] = total;
+    __syncthreads();
+    if (threadIdx.x < COLUMNS && col < hidden) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves16; ++w) sum += stage[w][threadIdx.x];
+        if (accumulate) sum += to_f32(out[col]);
+        out[col] = from_f32<T>(sum);
+    }
+}
+template <typename T, int COLUMNS>
+__global__ __launch_bounds__(kFinishThreads) void column_partial_reduce_kernel(
+    T* __restrict__ out, const float* __restrict__ partial, int parts, int hidden, int accumulate) {
+    column_partial_reduce_body<T, COLUMNS>(out, partial, parts, hidden, accumulate, static_cast<int>(blockIdx.x));
 }
 template <typename T>
-__global__ __launch_bounds__(kReduceThreads) void column_partial_reduce_kernel(
-    T* __restrict__ out, const float* __restrict__ partial, int parts, int hidden, int accumulate) {
-    column_partial_reduce_body<T>(out, partial, parts, hidden, accumulate, static_cast<int>(blockIdx.x));
+void launch_column_partial_reduce(T* out, const float* partial, int parts, int hidden, int accumulate, hipStream_t stream) {
+    const int columns = finish_columns(hidden);
+    auto kernel = columns == 16 ? column_partial_reduce_kernel<T, 16> : column_partial_reduce_kernel<T, 32>;
+    hipLaunchKernelGGL(kernel, dim3((hidden + columns - 1) / columns), dim3(kFinishThreads), 0, stream, out, partial, parts, hidden,
+                       accumulate);
 }
 
-// First level for many parts: block (group, index) of a (column groups, slices) grid folds the parts of
-// slice `index` for its 64 columns into second[index, col]; column_partial_reduce_kernel over the `slices`
-// rows of `second` finishes. (A single launch whose last block finishes would need device-scope
-// fences, which cost more here than the second launch.)
-__device__ __forceinline__ void column_partial_fold_body(float* __restrict__ second, const float* __restrict__ partial,
-                                                         int parts, int hidden, int slices, int index, int group) {
-    __shared__ float stage[kReduceWaves][kWave];
-    const int lane = threadIdx.x & (kWave - 1);
-    const int slice = threadIdx.x / kWave;
-    const int col = group * kWave + lane;
-    const int chunk = (parts + slices - 1) / slices;
-    const int begin = index * chunk;
-    const int end = begin + chunk < parts ? begin + chunk : parts;
-    float v0 = 0.0f, v1 = 0.0f;
-    if (col < hidden) {
-        int p = begin + slice;
-        for (; p + kReduceWaves < end; p += 2 * kReduceWaves) {
-            v0 += partial[static_cast<std::size_t>(p) * hidden + col];
-            v1 += partial[static_cast<std::size_t>(p + kReduceWaves) * hidden + col];
-        }
-        if (p < end) v0 += partial[static_cast<std::size_t>(p) * hidden + col];
-    }
-    stage[slice][lane] = v0 + v1;
-    __syncthreads();
-    if (slice == 0 && col < hidden) {
-        float v = 0.0f;
-#pragma unroll
-        for (int s = 0; s < kReduceWaves; ++s) v += stage[s][lane];
-        second[static_cast<std::size_t>(index) * hidden + col] = v;
-    }
+// The same over a table of reductions (blockIdx.y picks the entry): the same additions in the same order for every entry,
+// whatever else is in the table.
+template <typename T>
+__device__ __forceinline__ void column_partial_reduce_entry(const ColumnReduceEntry& e, int group) {
+    if (finish_columns(e.hidden) == 16) column_partial_reduce_body<T, 16>(static_cast<T*>(e.out), e.partial, e.parts, e.hidden, 0, group);
+    else column_partial_reduce_body<T, 32>(static_cast<T*>(e.out), e.partial, e.parts, e.hidden, 0, group);
 }
-static __global__ __launch_bounds__(kReduceThreads) void column_partial_fold_kernel(float* __restrict__ second,
-                                                                            const float* __restrict__ partial,
-                                                                            int parts, int hidden) {
-    column_partial_fold_body(second, partial, parts, hidden, static_cast<int>(gridDim.y), static_cast<int>(blockIdx.y),
-                             static_cast<int>(blockIdx.x));
-}
-
-// The two kernels above over a table of reductions (blockIdx.z, or blockIdx.y of the second, picks the entry):
-// the same additions in the same order for every entry, whatever else is in the table.
-static __global__ __launch_bounds__(kReduceThreads) void column_partial_fold_table_kernel(
-    const ColumnReduceEntry* __restrict__ table) {
-    const ColumnReduceEntry e = table[blockIdx.z];
-    if (e.slices <= 1 || static_cast<int>(blockIdx.y) >= e.slices || static_cast<int>(blockIdx.x) * kWave >= e.hidden) return;
-    column_partial_fold_body(e.second, e.partial, e.parts, e.hidden, e.slices, static_cast<int>(blockIdx.y),
-                             static_cast<int>(blockIdx.x));
-}
-static __global__ __launch_bounds__(kReduceThreads) void column_partial_reduce_table_kernel(
+static __global__ __launch_bounds__(kFinishThreads) void column_partial_reduce_table_kernel(
     const ColumnReduceEntry* __restrict__ table) {
     const ColumnReduceEntry e = table[blockIdx.y];
-    if (static_cast<int>(blockIdx.x) * kWave >= e.hidden) return;
-    const float* source = e.slices > 1 ? e.second : e.partial;
-    const int parts = e.slices > 1 ? e.slices : e.parts;
     const int group = static_cast<int>(blockIdx.x);
+    if (group * finish_columns(e.hidden) >= e.hidden) return;
     switch (e.dtype) {
-        case CGPTX_F16: column_partial_reduce_body<f16_t>(static_cast<f16_t*>(e.out), source, parts, e.hidden, 0, group); break;
-        case CGPTX_BF16: column_partial_reduce_body<bf16_t>(static_cast<bf16_t*>(e.out), source, parts, e.hidden, 0, group); break;
-        default: column_partial_reduce_body<float>(static_cast<float*>(e.out), source, parts, e.hidden, 0, group); break;
+        case CGPTX_F16: column_partial_reduce_entry<f16_t>(e, group); break;
+        case CGPTX_BF16: column_partial_reduce_entry<bf16_t>(e, group); break;
+        default: column_partial_reduce_entry<float>(e, group); break;
     }
-}
-
-// Slices for the kernel above: enough blocks to fill the chip, at least sixteen parts each.
-inline int wide_reduce_slices(int parts, int hidden, int units) {
-    const int groups = (hidden + kWave - 1) / kWave;
-    int slices = 2 * units / groups;
-    if (slices > parts / 16) slices = parts / 16;
-    return slices < 1 ? 1 : slices;
 }
 
 // partial[blockIdx.y, col] = Σ over this block's row slice of in[row, col] (fp32).

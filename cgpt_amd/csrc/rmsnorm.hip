@@ -707,37 +707,25 @@ int partial_memory(ColumnReduceSink* sink, hipStream_t stream, std::size_t bytes
     return *deferred ? CGPTX_OK : scratch(stream, bytes, out);
 }
 
-// dw[h] = column sums of partial[blocks, h]: two small launches now, or an entry in the sink.
+// dw[h] = column sums of partial[blocks, h]: a small launch now, or an entry in the sink.
 template <typename T>
-int reduce_columns(ColumnReduceSink* sink, bool deferred, T* dw, float* partial, float* second, int blocks, int h,
-                   int slices, int dtype, hipStream_t stream) {
+int reduce_columns(ColumnReduceSink* sink, bool deferred, T* dw, const float* partial, int blocks, int h, int dtype,
+                   hipStream_t stream) {
     if (deferred) {
-        sink->entries.push_back(ColumnReduceEntry{partial, second, dw, blocks, h, slices, dtype});
+        sink->entries.push_back(ColumnReduceEntry{partial, dw, blocks, h, dtype});
         return CGPTX_OK;
     }
-    const int reduce_blocks = (h + kWave - 1) / kWave;
-    if (slices > 1) {
-        hipLaunchKernelGGL(column_partial_fold_kernel, dim3(reduce_blocks, slices), dim3(kThreads), 0, stream, second,
-                           partial, blocks, h);
-        CGPTX_LAUNCH_CHECK();
-        hipLaunchKernelGGL((column_partial_reduce_kernel<T>), dim3(reduce_blocks), dim3(kThreads), 0, stream, dw, second,
-                           slices, h, 0);
-    } else {
-        hipLaunchKernelGGL((column_partial_reduce_kernel<T>), dim3(reduce_blocks), dim3(kThreads), 0, stream, dw, partial,
-                           blocks, h, 0);
-    }
+    launch_column_partial_reduce<T>(dw, partial, blocks, h, 0, stream);
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
 }
 
-int run_column_reductions(const ColumnReduceEntry* table, int count, int max_hidden, int max_slices, hipStream_t stream) {
-    if (count <= 0) return CGPTX_OK;
-    const int groups = (max_hidden + kWave - 1) / kWave;
-    if (max_slices > 1) {
-        hipLaunchKernelGGL(column_partial_fold_table_kernel, dim3(groups, max_slices, count), dim3(kThreads), 0, stream, table);
-        CGPTX_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(column_partial_reduce_table_kernel, dim3(groups, count), dim3(kThreads), 0, stream, table);
+int run_column_reductions(const ColumnReduceEntry* table, const std::vector<ColumnReduceEntry>& entries, hipStream_t stream) {
+    if (entries.empty()) return CGPTX_OK;
+    int groups = 1;
+    for (const ColumnReduceEntry& e : entries) groups = std::max(groups, (e.hidden + finish_columns(e.hidden) - 1) / finish_columns(e.hidden));
+    hipLaunchKernelGGL(column_partial_reduce_table_kernel, dim3(groups, static_cast<unsigned int>(entries.size())), dim3(kFinishThreads),
+                       0, stream, table);
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
 }
@@ -776,24 +764,16 @@ int rmsnorm_rope_backward(void* grad_input, void* grad_weight, const void* grad_
     return dispatch_dtype(dtype, [&]<typename T>() -> int {
         const FastShape shape = pick_fast_shape<T>(h);
         const int blocks = fast_blocks(shape, r, fast_kernel<T, true>(shape, true, rope_dense<T>(r, h, rope)));
-        const int slices = wide_reduce_slices(blocks, h, compute_units());
         void* mem = nullptr;
         bool deferred = false;
-        const std::size_t partial_bytes = static_cast<std::size_t>(blocks) * head_dim * sizeof(float);
-        if (int s = partial_memory(sink, stream, partial_bytes + static_cast<std::size_t>(slices) * head_dim * sizeof(float), &mem,
-                                   &deferred))
-            return s;
+        if (int s = partial_memory(sink, stream, static_cast<std::size_t>(blocks) * head_dim * sizeof(float), &mem, &deferred)) return s;
         auto* partial = static_cast<float*>(mem);
         if (int s = launch_fast<T, true>(shape, static_cast<T*>(grad_input), partial, static_cast<const T*>(grad_output),
                                          nullptr, static_cast<const T*>(input), static_cast<const T*>(weight), r, h, epsilon,
                                          blocks, stream, &rope))
             return s;
         CGPTX_LAUNCH_CHECK();
-        auto* second = reinterpret_cast<float*>(static_cast<char*>(mem) + partial_bytes);
-        if (int s = reduce_columns<T>(sink, deferred, static_cast<T*>(grad_weight), partial, second, blocks, h, slices, dtype,
-                                      stream))
-            return s;
-        return CGPTX_OK;
+        return reduce_columns<T>(sink, deferred, static_cast<T*>(grad_weight), partial, blocks, h, dtype, stream);
     });
 }
 
@@ -879,16 +859,12 @@ int rmsnorm_backward_dual(void* grad_input, void* grad_weight_a, void* grad_weig
     return dispatch_dtype(dtype, [&]<typename T>() -> int {
         const FastShape shape = pick_fast_shape<T>(h);
         const int blocks = fast_blocks(shape, r, dual_kernel<T, true>(shape));
-        const int slices = wide_reduce_slices(blocks, h, compute_units());
         void* mem = nullptr;
         bool deferred = false;
         const std::size_t partial_bytes = static_cast<std::size_t>(blocks) * hidden * sizeof(float);
-        const std::size_t second_bytes = (static_cast<std::size_t>(slices) * hidden * sizeof(float) + 255) & ~std::size_t{255};
-        if (int s = partial_memory(sink, stream, 2 * partial_bytes + 2 * second_bytes, &mem, &deferred)) return s;
+        if (int s = partial_memory(sink, stream, 2 * partial_bytes, &mem, &deferred)) return s;
         auto* partial_a = static_cast<float*>(mem);
         auto* partial_f = reinterpret_cast<float*>(static_cast<char*>(mem) + partial_bytes);
-        auto* second_a = reinterpret_cast<float*>(static_cast<char*>(mem) + 2 * partial_bytes);
-        auto* second_f = reinterpret_cast<float*>(static_cast<char*>(mem) + 2 * partial_bytes + second_bytes);
         if (int s = launch_dual<T, true>(shape, static_cast<T*>(grad_input), nullptr, partial_a, partial_f,
                                          static_cast<const T*>(grad_output_a), static_cast<const T*>(grad_output_f),
                                          static_cast<const T*>(residual), static_cast<const T*>(input),
@@ -896,13 +872,9 @@ int rmsnorm_backward_dual(void* grad_input, void* grad_weight_a, void* grad_weig
                                          stream))
             return s;
         CGPTX_LAUNCH_CHECK();
-        if (int s = reduce_columns<T>(sink, deferred, static_cast<T*>(grad_weight_a), partial_a, second_a, blocks, h, slices,
-                                      dtype, stream))
+        if (int s = reduce_columns<T>(sink, deferred, static_cast<T*>(grad_weight_a), partial_a, blocks, h, dtype, stream))
             return s;
-        if (int s = reduce_columns<T>(sink, deferred, static_cast<T*>(grad_weight_f), partial_f, second_f, blocks, h, slices,
-                                      dtype, stream))
-            return s;
-        return CGPTX_OK;
+        return reduce_columns<T>(sink, deferred, static_cast<T*>(grad_weight_f), partial_f, blocks, h, dtype, stream);
     });
 }
 
@@ -944,10 +916,8 @@ int rmsnorm_backward_impl(void* grad_input, void* grad_weight, const void* grad_
         const int reduce_blocks = (h + kWave - 1) / kWave;
         if (shape.lpr != 0 && aligned) {
             const int blocks = fast_blocks(shape, r, fast_kernel<T, true>(shape, false));
-            const int slices = wide_reduce_slices(blocks, h, compute_units());
             void* mem = nullptr;
-            const std::size_t partial_bytes = static_cast<std::size_t>(blocks) * hidden * sizeof(float);
-            const std::size_t bytes = partial_bytes + static_cast<std::size_t>(slices) * hidden * sizeof(float);
+            const std::size_t bytes = static_cast<std::size_t>(blocks) * hidden * sizeof(float);
             if (workspace.sink != nullptr) mem = workspace.sink->take(bytes);
             const bool deferred = mem != nullptr;
             if (!deferred) {
@@ -956,8 +926,7 @@ int rmsnorm_backward_impl(void* grad_input, void* grad_weight, const void* grad_
             auto* partial = static_cast<float*>(mem);
             if (int s = launch_fast<T, true>(shape, dx, partial, dy, res, x, w, r, h, epsilon, blocks, stream)) return s;
             CGPTX_LAUNCH_CHECK();
-            auto* second = reinterpret_cast<float*>(static_cast<char*>(mem) + partial_bytes);
-            return reduce_columns<T>(workspace.sink, deferred, dw, partial, second, blocks, h, slices, dtype, stream);
+            return reduce_columns<T>(workspace.sink, deferred, dw, partial, blocks, h, dtype, stream);
         }
         const int slices = r < 256 ? 1 : (r < 65536 ? 64 : 256);
         const int rows_per_slice = (r + slices - 1) / slices;
@@ -974,8 +943,7 @@ int rmsnorm_backward_impl(void* grad_input, void* grad_weight, const void* grad_
         hipLaunchKernelGGL((rmsnorm_dgamma_generic_kernel<T>), dim3(reduce_blocks, slices), dim3(kThreads), 0, stream,
                            partial, dy, x, inv_rms, r, h, rows_per_slice);
         CGPTX_LAUNCH_CHECK();
-        hipLaunchKernelGGL((column_partial_reduce_kernel<T>), dim3(reduce_blocks), dim3(kThreads), 0, stream, dw,
-                           partial, slices, h, 0);
+        launch_column_partial_reduce<T>(dw, partial, slices, h, 0, stream);
         CGPTX_LAUNCH_CHECK();
         if (res != nullptr) return cgptx_add(dx, dx, res, rows * hidden, dtype, stream);
         return CGPTX_OK;
@@ -995,18 +963,14 @@ std::size_t rmsnorm_backward_sink_bytes(NormPass pass, std::size_t rows, std::si
         const void* kernel = pass == NormPass::dual ? dual_kernel<T, true>(shape) : fast_kernel<T, true>(shape, pass == NormPass::with_rope);
         if (kernel == nullptr) return CGPTX_OK;
         int blocks = fast_blocks(shape, r, kernel);
-        int slices = wide_reduce_slices(blocks, h, compute_units());
         if (pass == NormPass::with_rope) {
             // The pass picks between two kernels by properties of its rotary tables that are not known here: room
             // for whichever of them takes more.
             const int other = fast_blocks(shape, r, fast_kernel<T, true>(shape, true, true));
-            const int other_slices = wide_reduce_slices(other, h, compute_units());
             blocks = other > blocks ? other : blocks;
-            slices = other_slices > slices ? other_slices : slices;
         }
         const std::size_t partial_bytes = static_cast<std::size_t>(blocks) * hidden * sizeof(float);
-        const std::size_t second_bytes = static_cast<std::size_t>(slices) * hidden * sizeof(float);
-        bytes = pass == NormPass::dual ? 2 * partial_bytes + 2 * ((second_bytes + 255) & ~std::size_t{255}) : partial_bytes + second_bytes;
+        bytes = pass == NormPass::dual ? 2 * partial_bytes : partial_bytes;
         bytes = (bytes + 255) & ~std::size_t{255};  // ColumnReduceSink::take hands out multiples of 256
         return CGPTX_OK;
     });

@@ -146,7 +146,7 @@ struct cgptx_model {
         std::uint64_t scratch_generation = 0;  // scratch arena block the recorded kernels point into
     };
     RecordedStep recorded[2];
-    // weight-gradient reductions of the norm-backward passes, run as one pair of launches per step
+    // weight-gradient reductions of the norm-backward passes, run as one launch per step
     cgptx::ColumnReduceSink norm_reductions;
     cgptx::ColumnReduceEntry* norm_reduction_table = nullptr;       // device copy of the entries
     std::vector<cgptx::ColumnReduceEntry> norm_reduction_uploaded;  // what the device copy holds
@@ -485,8 +485,8 @@ bool fused_swiglu_gradient() {
     return text == nullptr || text[0] != '0';
 }
 
-// Whether the norm-backward passes of the step leave their weight-gradient reductions to one pair of launches at
-// the end of the backward pass (CGPTX_FUSE_DGAMMA=0 keeps the two small launches after each pass, for comparisons:
+// Whether the norm-backward passes of the step leave their weight-gradient reductions to one launch at
+// the end of the backward pass (CGPTX_FUSE_DGAMMA=0 keeps the small launch after each pass, for comparisons:
 // same additions in the same order, same bits).
 cgptx::ColumnReduceSink* norm_reduction_sink(cgptx_model* m) {
     const char* text = std::getenv("CGPTX_FUSE_DGAMMA");  // read per enqueue
@@ -526,13 +526,7 @@ int finish_norm_reductions(cgptx_model* m, hipStream_t stream) {
                                 hipMemcpyHostToDevice));
             m->norm_reduction_uploaded = sink.entries;
         }
-        int max_hidden = 0, max_slices = 0;
-        for (const ColumnReduceEntry& e : sink.entries) {
-            max_hidden = std::max(max_hidden, e.hidden);
-            max_slices = std::max(max_slices, e.slices);
-        }
-        if (int s = run_column_reductions(m->norm_reduction_table, static_cast<int>(sink.entries.size()), max_hidden,
-                                          max_slices, stream))
+        if (int s = run_column_reductions(m->norm_reduction_table, sink.entries, stream))
             return s;
     }
     m->norm_reductions_resized = false;
