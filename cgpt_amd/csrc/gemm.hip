@@ -74,6 +74,14 @@ struct TileLayout {
     static constexpr int kSmemBytes = kSlots * kSlot * static_cast<int>(sizeof(T));
 };
 
+// Stores a lane's 16 bytes at voffset + soffset of a buffer. The sum is taken in the vector register: behind a 16-byte store
+// with a scalar offset the compiler lets the very next instruction overwrite the data registers, and on this chip the store
+// has then not always read them (128 x 128 tiles, two wavefronts a SIMD: the first four bytes of some hundred stores in a
+// [32768, 768] result were the next value's). Without one it keeps the distance.
+__device__ __forceinline__ void store_chunk(const u32x4& data, __amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset) {
+    __builtin_amdgcn_raw_buffer_store_b128(data, rsrc, voffset + soffset, 0, 0);
+}
+
 // One workgroup per CU slot walks its share of the work items (output tile x K slice) one after
 // the other: the first K tiles of the next item are requested before the epilogue of the current
 // one, whose stores then drain under the next item's MFMAs.
@@ -478,15 +486,15 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
 #pragma unroll
                 for (int u = 0; u < kRoundsF; ++u) {
                     const int row = r * 32 + u * kRowsF;
-                    __builtin_amdgcn_raw_buffer_store_b128(gate[u], gate_rsrc, c_voffset, row * c_row_bytes, 0);
-                    __builtin_amdgcn_raw_buffer_store_b128(up[u], up_rsrc, c_voffset, row * c_row_bytes, 0);
+                    store_chunk(gate[u], gate_rsrc, c_voffset, row * c_row_bytes);
+                    store_chunk(up[u], up_rsrc, c_voffset, row * c_row_bytes);
                     const vec_t<float, 8> g = vec_to_f32<T, 8>(__builtin_bit_cast(vec_t<T, 8>, gate[u]));
                     const vec_t<float, 8> v = vec_to_f32<T, 8>(__builtin_bit_cast(vec_t<T, 8>, up[u]));
                     vec_t<float, 8> product;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) product[e] = g[e] * (1.0f / (1.0f + __expf(-g[e]))) * v[e];
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(product)), act_rsrc,
-                                                           act_voffset, row * act_row_bytes, 0);
+                    store_chunk(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(product)), act_rsrc,
+                                                           act_voffset, row * act_row_bytes);
                 }
             }
             return;
@@ -548,8 +556,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
                         du[e] = d[e] * (g[e] * sg);
                     }
                     const int soffset = (r * 32 + u * kRowsPerRound) * out_row_bytes;
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(dg)), dgate_rsrc, out_voffset, soffset, 0);
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(du)), dup_rsrc, out_voffset, soffset, 0);
+                    store_chunk(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(dg)), dgate_rsrc, out_voffset, soffset);
+                    store_chunk(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(du)), dup_rsrc, out_voffset, soffset);
                 }
             }
             return;
@@ -600,8 +608,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
                             sum[e] = v0[u][e] + add[e];
                             sum[4 + e] = v1[u][e] + add[4 + e];
                         }
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(sum)), out_rsrc, voffset,
-                                                               (r * 32 + u * kRowsF) * out_row_bytes, 0);
+                        store_chunk(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(sum)), out_rsrc, voffset,
+                                                               (r * 32 + u * kRowsF) * out_row_bytes);
                     }
                 }
             }
@@ -641,7 +649,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
                 }
 #pragma unroll
                 for (int u = 0; u < kRounds; ++u)
-                    __builtin_amdgcn_raw_buffer_store_b128(data[u], rsrc, voffset, (r * 32 + u * kRowsPerRound) * row_bytes, 0);
+                    store_chunk(data[u], rsrc, voffset, (r * 32 + u * kRowsPerRound) * row_bytes);
             }
             return;
         }
@@ -670,8 +678,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
 #pragma unroll
                     for (int u = 0; u < kRoundsF; ++u) {
                         const int soffset = (r * 32 + u * kRowsF) * row_bytes;
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v0[u]), rsrc, voffset0, soffset, 0);
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v1[u]), rsrc, voffset1, soffset, 0);
+                        store_chunk(__builtin_bit_cast(u32x4, v0[u]), rsrc, voffset0, soffset);
+                        store_chunk(__builtin_bit_cast(u32x4, v1[u]), rsrc, voffset1, soffset);
                     }
                 }
             }

@@ -753,3 +753,32 @@ def test_step_as_the_reference_call_sequence_agrees_with_the_fused_step(device, 
         separate = results[1][1][name]
         scale = separate.abs().max().item() + 1e-12
         assert (fused - separate).abs().max().item() <= 3e-2 * scale, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,seq", [(16, 313), (8, 1024), (32, 1024)], ids=["ragged", "8192", "32768"])
+def test_block_output_is_the_residual_sum_of_its_parts(device, batch, seq):
+    """hidden[1] = x + attention_output Wo + activated Wdown over every element, at row counts whose output projections run on
+    128- and 256-wide tiles: the two sums are rounded once each, so no element may be off by more than a few roundings
+    (8 bits of mantissa: 2^-8 of the larger sum each, four times that is allowed). A store that goes wrong in one element of
+    thousands shows here and in no norm."""
+    from cgpt_amd.model import LOSS_CUT, Model, ModelConfig
+
+    config = ModelConfig(vocabulary_size=512, num_layers=1, hidden_size=768, intermediate_size=2048, num_query_heads=12,
+                         num_kv_heads=4, head_dim=64, rotary_dim=64, dtype=torch.bfloat16)
+    model = Model(config, batch, seq, seed=3, device=device)
+    rng = np.random.default_rng(3)
+    model.set_tokens(rng.integers(0, 512, size=(batch, seq)), rng.integers(0, 512, size=(batch, seq)))
+    stream = torch.cuda.Stream(device=device)
+    weights = {name: p.float() for name, p, _ in model.parameters()}
+    o, down = (weights[f"model.layers.0.{name}.weight"].view(768, -1).T.contiguous() for name in ("self_attn.o_proj", "mlp.down_proj"))
+    for _ in range(3):
+        model.forward_backward(1024.0, LOSS_CUT, use_graph=False, stream=stream)
+        torch.cuda.synchronize()
+        read = lambda name, width: model.activation(name).view(-1, width).float()
+        first = read("hidden.0", 768) + read("layer.0.attention_output", 768) @ o
+        want = first + read("layer.0.activated", 2048) @ down
+        error = (read("hidden.1", 768) - want).abs()
+        assert torch.isfinite(error).all()
+        assert (error <= 4 * 2.0 ** -8 * torch.maximum(first.abs(), want.abs()) + 1e-3).all(), error.max().item()
+    model.close()
