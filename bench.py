@@ -335,11 +335,11 @@ def measured_traffic():
         return None, "no counter summary found"
     if value is None:
         return None, "the counter summary holds no traffic figure"
-    if recorded is None or recorded != source_digest("gemm.hip"):
-        note = "STALE: cgpt_amd/csrc/gemm.hip has changed since profiles/gemm_dx_256x256_gate_projection_pmc.txt was measured"
+    if recorded is None or recorded != source_digest("gemm_large_kernel.hpp"):
+        note = "STALE: cgpt_amd/csrc/gemm_large_kernel.hpp has changed since profiles/gemm_dx_256x256_gate_projection_pmc.txt was measured"
         print("bench.py: warning: roofline.traffic is " + note, file=sys.stderr)
         return value, note
-    return value, "measured with the current cgpt_amd/csrc/gemm.hip"
+    return value, "measured with the current cgpt_amd/csrc/gemm_large_kernel.hpp"
 
 
 def cpu_model_name():

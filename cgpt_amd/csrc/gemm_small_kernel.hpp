@@ -1,17 +1,18 @@
 // Small contractions: K split between the wavefronts of a workgroup.
 //
 // C of at most a few hundred tiles (short sequences, narrow layers, the weight gradients of a small batch) leaves the
-// persistent kernels of gemm.hip with little to do per K tile and a workgroup barrier around each: what such a call costs
+// persistent kernels with little to do per K tile and a workgroup barrier around each: what such a call costs
 // is the latency of its start and of its serial K loop. Here a workgroup owns one 64 x 64 or 32 x 32 tile and its four
 // wavefronts take every fourth K tile each, the whole C tile of it: the loop is four times shorter and has no barrier,
-// since a wavefront loads its K tiles into LDS stages of its own (global -> LDS) and waits for nobody. Fragments of the
-// next K tile are read, and the loads of the one STAGES further issued, between the MFMAs of the present one. At the end
+// since a wavefront loads its K tiles into LDS stages of its own (global -> LDS) and waits for nobody. A K tile is two MFMA
+// steps long, whole cache lines of a k-contiguous operand (see KTile); the fragments of the step to come are read, and the
+// loads of the K tile to come are issued, between the MFMAs of the present step. At the end
 // the four partial tiles meet in LDS and are added in wavefront order. Same swizzled operand tiles and same edges (buffer
 // range checks) as the persistent kernels.
 //
 // What bounds it: with few workgroups the latency of the loads, i.e. the K bytes of a workgroup over the bytes it keeps
-// in flight (64 or 128 KiB), which is why short rows of tiles take 32 x 32 ones; with a full chip the L2's bandwidth
-// (64 bytes per CU and cycle against 8 KiB per 16 MFMAs), where larger tiles win.
+// in flight (64 or 128 KiB), which is why short rows of tiles take 32 x 32 ones; with a full chip the path from the L2s
+// (8 KiB per 64 x 64 tile and step: 0.128 us in half cache lines, 0.09 in whole ones), where larger tiles win.
 #pragma once
 
 #include "gemm_small.hpp"
@@ -48,20 +49,22 @@ constexpr int small_smem_bytes() { return DEEP ? 128 * 1024 : 64 * 1024; }
 template <typename T, int TILE, bool DEEP, bool A_K, bool B_K, SmallEpilogue EPILOGUE, bool SEGMENTED, bool SUMS>
 __device__ __forceinline__ void small_tile(const SmallArgs& p, int m0, int n0, int slice, unsigned char* smem_raw) {
     using frag_t = typename Mfma<T>::frag;
-    using ATile = std::conditional_t<A_K, KTile<T, TILE>, NTile<T, TILE>>;
-    using BTile = std::conditional_t<B_K, KTile<T, TILE>, NTile<T, TILE>>;
+    using ATile = std::conditional_t<A_K, KTile<T, TILE, kSteps>, NTile<T, TILE, kSteps>>;
+    using BTile = std::conditional_t<B_K, KTile<T, TILE, kSteps>, NTile<T, TILE, kSteps>>;
     constexpr int kBlocks = TILE / 16;                  // 16 x 16 MFMA blocks along an edge
-    constexpr int kOperandBytes = TILE * 64;            // 64 bytes along K per row, or the same bytes k-strided
+    constexpr int kOperandBytes = TILE * 64 * kSteps;   // 128 bytes along K per row, or the same bytes k-strided
     constexpr int kStageBytes = 2 * kOperandBytes;      // [A | B]
     constexpr int kLoadBytes = 1024, kOperandLoads = kOperandBytes / kLoadBytes, kLoads = 2 * kOperandLoads;
     constexpr int STAGES = small_smem_bytes<TILE, DEEP>() / (kWaves * kStageBytes);
-    static_assert(STAGES >= 2 && STAGES * kLoads < 64, "the loads in flight are counted by vmcnt");
+    static_assert(STAGES >= 1 && STAGES * kLoads < 64, "the loads in flight are counted by vmcnt");
     static_assert(!SUMS || !A_K, "columns of A are summed where its rows are K positions");
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
 
     const int kt_begin = slice * p.k_tiles_per_slice, kt_end = min(p.k_tiles, kt_begin + p.k_tiles_per_slice);
-    const int steps = max(0, (kt_end - kt_begin - wave + kWaves - 1) / kWaves);  // K tiles kt_begin + wave + kWaves i
+    // This wavefront's K tiles: steps kt_begin + kSteps (wave + kWaves i) and the one after it, which the last may lack.
+    const int tiles = max(0, ((kt_end - kt_begin + kSteps - 1) / kSteps - wave + kWaves - 1) / kWaves);
+    const bool whole_last = kt_begin + kSteps * (wave + kWaves * (tiles - 1)) + 1 < kt_end;
 
     // Sources. A in column segments: along K (k-contiguous) the segment is picked per K tile, along M once.
     ATile a_src;
@@ -107,18 +110,17 @@ __device__ __forceinline__ void small_tile(const SmallArgs& p, int m0, int n0, i
     const unsigned int lds_wave = lds_address_of(smem_raw) + wave * (STAGES * kStageBytes);
     const T* const wave_stages = reinterpret_cast<const T*>(smem_raw + wave * (STAGES * kStageBytes));
     constexpr int kStageElems = kStageBytes / static_cast<int>(sizeof(T)), kOperandElems = kStageElems / 2;
-    // Step i's loads; past the last one they read zeros from beyond the buffers, so that every step issues the same number.
     unsigned int a_soffset = 0, b_soffset = 0;
     u32x4 a_rsrc = a_src.rsrc;
-    int a_voffset = a_src.voffset;
+    int a_voffset = a_src.voffset, a_voffset_odd = a_src.load_voffset(1);
     unsigned int a_step = a_src.group_bytes;
     auto aim = [&](int i) __attribute__((always_inline)) {
-        const unsigned int past_end = i >= steps ? 0x80000000u : 0u;
-        const int k0 = min(kt_begin + wave + kWaves * i, p.k_tiles - 1) * kBK<T>;
+        const int k0 = (kt_begin + kSteps * (wave + kWaves * i)) * kBK<T>;
         if constexpr (A_K && SEGMENTED) {
             const bool in1 = k0 >= a_end0, in2 = k0 >= a_end1;
             const u32x4 rsrc0 = a_src.rsrc, rsrc1 = a_src1.rsrc, rsrc2 = a_src2.rsrc;
             const int voffset0 = a_src.voffset, voffset1 = a_src1.voffset, voffset2 = a_src2.voffset;
+            const int odd0 = a_src.load_voffset(1), odd1 = a_src1.load_voffset(1), odd2 = a_src2.load_voffset(1);
             const unsigned int bytes0 = a_src.group_bytes, bytes1 = a_src1.group_bytes, bytes2 = a_src2.group_bytes;
             const int end0 = a_end0, end1 = a_end1;
 #pragma unroll
@@ -127,17 +129,18 @@ __device__ __forceinline__ void small_tile(const SmallArgs& p, int m0, int n0, i
                 a_rsrc[e] = in2 ? w2 : in1 ? w1 : w0;
             }
             a_voffset = in2 ? voffset2 : in1 ? voffset1 : voffset0;
+            a_voffset_odd = in2 ? odd2 : in1 ? odd1 : odd0;
             a_step = in2 ? bytes2 : in1 ? bytes1 : bytes0;
-            a_soffset = (k0 - (in2 ? end1 : in1 ? end0 : 0)) * static_cast<unsigned int>(sizeof(T)) | past_end;
+            a_soffset = (k0 - (in2 ? end1 : in1 ? end0 : 0)) * static_cast<unsigned int>(sizeof(T));
         } else {
-            a_soffset = a_src.first_offset(k0, 0) | past_end;
+            a_soffset = a_src.first_offset(k0, 0);
         }
-        b_soffset = b_src.first_offset(k0, 0) | past_end;
+        b_soffset = b_src.first_offset(k0, 0);
     };
     auto issue = [&](auto index, unsigned int stage_lds) __attribute__((always_inline)) {
         constexpr int l = decltype(index)::value;
         if constexpr (l < kOperandLoads && A_K && SEGMENTED)
-            a_soffset = load_to_lds<l * kLoadBytes>(a_rsrc, stage_lds, a_voffset, a_soffset, a_step);
+            a_soffset = load_to_lds<l * kLoadBytes>(a_rsrc, stage_lds, l % 2 == 0 ? a_voffset : a_voffset_odd, a_soffset, a_step);
         else if constexpr (l < kOperandLoads)
             a_soffset = load_to_lds<l * kLoadBytes>(a_src.rsrc, stage_lds, a_src.load_voffset(l), a_soffset, a_src.group_bytes);
         else
@@ -145,25 +148,29 @@ __device__ __forceinline__ void small_tile(const SmallArgs& p, int m0, int n0, i
     };
 
     static_for<0, STAGES>([&](auto s) {
-        aim(decltype(s)::value);
-        static_for<0, kLoads>([&](auto l) { issue(l, lds_wave + decltype(s)::value * kStageBytes); });
+        if (decltype(s)::value < tiles) {
+            aim(decltype(s)::value);
+            static_for<0, kLoads>([&](auto l) { issue(l, lds_wave + decltype(s)::value * kStageBytes); });
+        }
     });
 
-    constexpr int kAOffsets = A_K ? 1 : kBlocks, kBOffsets = B_K ? 1 : kBlocks;
+    constexpr int kAOffsets = A_K ? kSteps : kBlocks, kBOffsets = B_K ? kSteps : kBlocks;
     int a_off[kAOffsets], b_off[kBOffsets];
-    if constexpr (A_K) a_off[0] = ATile::lane_offset(lane);
-    else static_for<0, kBlocks>([&](auto i) { a_off[decltype(i)::value] = ATile::lane_offset(lane, decltype(i)::value * 16); });
-    if constexpr (B_K) b_off[0] = BTile::lane_offset(lane);
-    else static_for<0, kBlocks>([&](auto i) { b_off[decltype(i)::value] = BTile::lane_offset(lane, decltype(i)::value * 16); });
-    frag_t af[2][kBlocks], bf[2][kBlocks];
-    auto read_frag = [&]<int BUFFER, int F>(const T* stage) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kAOffsets; ++i) a_off[i] = A_K ? ATile::lane_offset(lane, i) : ATile::lane_offset(lane, i * 16);
+#pragma unroll
+    for (int j = 0; j < kBOffsets; ++j) b_off[j] = B_K ? BTile::lane_offset(lane, j) : BTile::lane_offset(lane, j * 16);
+    // Fragments of the step being multiplied and of the next one: step s of a K tile is in af[s], bf[s].
+    constexpr int kFrags = 2 * kBlocks;
+    frag_t af[kSteps][kBlocks], bf[kSteps][kBlocks];
+    auto read_frag = [&]<int STEP, int F>(const T* stage) __attribute__((always_inline)) {
         if constexpr (F < kBlocks) {
-            if constexpr (A_K) af[BUFFER][F] = ATile::frag(stage, F * 16, a_off[0]);
-            else af[BUFFER][F] = ATile::frag(stage, a_off[F]);
+            if constexpr (A_K) af[STEP][F] = ATile::frag(stage, F * 16, a_off[STEP]);
+            else af[STEP][F] = ATile::frag(stage + STEP * ATile::kStepElems, a_off[F]);
         } else {
             constexpr int j = F - kBlocks;
-            if constexpr (B_K) bf[BUFFER][j] = BTile::frag(stage + kOperandElems, j * 16, b_off[0]);
-            else bf[BUFFER][j] = BTile::frag(stage + kOperandElems, b_off[j]);
+            if constexpr (B_K) bf[STEP][j] = BTile::frag(stage + kOperandElems, j * 16, b_off[STEP]);
+            else bf[STEP][j] = BTile::frag(stage + kOperandElems + STEP * BTile::kStepElems, b_off[j]);
         }
     };
 
@@ -181,54 +188,72 @@ __device__ __forceinline__ void small_tile(const SmallArgs& p, int m0, int n0, i
         for (int i = 0; i < kBlocks; ++i) column_sums[i] = acc_t(0.0f);
 #pragma unroll
         for (int e = 0; e < static_cast<int>(sizeof(frag_t) / sizeof(T)); ++e) ones[e] = static_cast<T>(1.0f);
-        // Kept in registers: written again in front of its MFMA, it would need wait states that assembly has to bring itself.
-        asm volatile("" : "+v"(ones));
     }
-    wait_loads<(STAGES - 1) * kLoads>();
-    static_for<0, 2 * kBlocks>([&](auto f) { read_frag.template operator()<0, decltype(f)::value>(wave_stages); });
-    int stage = 0;
-    auto step = [&]<int BUFFER>(int i) __attribute__((always_inline)) {
-        const int next_stage = (stage + 1) % STAGES;
-        aim(i + STAGES);
-        // This step's fragments are in registers, so its stage can be refilled; the next step's K tile has landed.
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        wait_loads<(STAGES - 2) * kLoads>();
-        constexpr int kMfmas = kBlocks * kBlocks, kReads = 2 * kBlocks;
+    // One step's MFMAs. NEXT: the fragments of the step after it are read from `next_stage`, one per MFMA; LOADS: a K tile
+    // is requested into the stage at refill_lds, its loads dealt out over the step.
+    constexpr int kMfmas = kBlocks * kBlocks;
+    auto multiply = [&]<int STEP, bool NEXT, bool LOADS>(const T* next_stage, unsigned int refill_lds) __attribute__((always_inline)) {
         static_for<0, kMfmas>([&](auto index) {
             constexpr int m = decltype(index)::value, row = m / kBlocks, column = (row & 1) ? kBlocks - 1 - m % kBlocks : m % kBlocks;
-            Mfma<T>::run(acc[row][column], bf[BUFFER][column], af[BUFFER][row]);
-            // The fragment reads in the first half of the MFMAs, the loads in the second.
-            if constexpr (m < kMfmas / 2) {
-                static_for<m * kReads / (kMfmas / 2), (m + 1) * kReads / (kMfmas / 2)>(
-                    [&](auto f) { read_frag.template operator()<BUFFER ^ 1, decltype(f)::value>(wave_stages + next_stage * kStageElems); });
-            } else {
-                constexpr int h = m - kMfmas / 2;
-                static_for<h * kLoads / (kMfmas / 2), (h + 1) * kLoads / (kMfmas / 2)>(
-                    [&](auto l) { issue(l, lds_wave + stage * kStageBytes); });
-            }
+            Mfma<T>::add(acc[row][column], bf[STEP][column], af[STEP][row]);
+            if constexpr (NEXT && m < kFrags) read_frag.template operator()<1 - STEP, m>(next_stage);
+            if constexpr (LOADS) static_for<m * kLoads / kMfmas, (m + 1) * kLoads / kMfmas>([&](auto l) { issue(l, refill_lds); });
             __builtin_amdgcn_sched_barrier(0);
         });
         if constexpr (SUMS) {
             if (sums) {
-                asm volatile("s_nop 1" : "+v"(ones));
 #pragma unroll
-                for (int i = 0; i < kBlocks; ++i) Mfma<T>::run(column_sums[i], ones, af[BUFFER][i]);
+                for (int i = 0; i < kBlocks; ++i) Mfma<T>::add(column_sums[i], ones, af[STEP][i]);
             }
         }
-        stage = next_stage;
     };
-    for (int i = 0; i < steps; i += 2) {
-        step.template operator()<0>(i);
-        if (i + 1 < steps) step.template operator()<1>(i + 1);
+    static_assert(kFrags <= kMfmas, "a fragment read per MFMA");
+    // With one stage the next K tile's first fragments wait for its loads, which the other wavefront of the SIMD covers; with
+    // more, they are read a step ahead.
+    constexpr bool kAhead = STAGES > 1;
+    auto first_fragments = [&](const T* stage) __attribute__((always_inline)) {
+        static_for<0, kFrags>([&](auto f) { read_frag.template operator()<0, decltype(f)::value>(stage); });
+    };
+    if (kAhead && tiles > 0) {
+        if (tiles >= STAGES) wait_loads<(STAGES - 1) * kLoads>();
+        else wait_loads<0>();
+        first_fragments(wave_stages);
+    }
+    int stage = 0, t = 0;
+    // First step of K tile t, and the wait after which its stage is free.
+    auto first_step = [&]() __attribute__((always_inline)) {
+        if constexpr (!kAhead) {
+            wait_loads<0>();
+            first_fragments(wave_stages);
+        }
+        multiply.template operator()<0, true, false>(wave_stages + stage * kStageElems, 0u);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    for (; t + STAGES < tiles; ++t) {
+        first_step();
+        aim(t + STAGES);
+        const int next_stage = stage + 1 == STAGES ? 0 : stage + 1;
+        if constexpr (kAhead) wait_loads<(STAGES - (kAhead ? 2 : 1)) * kLoads>();
+        multiply.template operator()<1, kAhead, true>(wave_stages + next_stage * kStageElems, lds_wave + stage * kStageBytes);
+        stage = next_stage;
+    }
+    for (; t < tiles; ++t) {
+        first_step();
+        const int next_stage = stage + 1 == STAGES ? 0 : stage + 1;
+        if (kAhead && t + 1 < tiles) {
+            wait_loads<0>();
+            multiply.template operator()<1, true, false>(wave_stages + next_stage * kStageElems, 0u);
+        } else if (t + 1 < tiles || whole_last) {
+            multiply.template operator()<1, false, false>(wave_stages, 0u);
+        }
+        stage = next_stage;
     }
 
-    // The partial tiles, [wavefront][row][column] in fp32. Everybody's loads (of zeros, past the end) have to be through
-    // before the stages are reused; the waits also separate the last MFMA from the reads of its accumulator.
+    // The partial tiles, [wavefront][row][column] in fp32. Everybody's fragments have to be read before the stages are reused.
     constexpr int kPitch = TILE + 4;
     static_assert(kWaves * TILE * kPitch * 4 <= kWaves * STAGES * kStageBytes + 8192, "partial tiles fit where the stages were");
     float* const partial = reinterpret_cast<float*>(smem_raw);
     wait_loads<0>();
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     __syncthreads();
     {
         float* mine = partial + wave * TILE * kPitch + (lane & 15) * kPitch + (lane >> 4) * 4;

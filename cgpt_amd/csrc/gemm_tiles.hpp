@@ -1,7 +1,7 @@
 // Operand tiles and matrix instructions shared by the contraction kernels (gemm.hip, gemm_small.hpp).
 #pragma once
 
-#include "gemm.hpp"
+#include "gemm_large.hpp"
 
 #include <limits>
 #include <type_traits>
@@ -15,6 +15,8 @@ constexpr int kWaves = kThreads / kWave;
 // K step per LDS stage: 64 bytes of a k-contiguous operand's row.
 template <typename T>
 constexpr int kBK = 64 / static_cast<int>(sizeof(T));
+// K steps of one MFMA each per 16 x 16 block in a K tile of the persistent kernels: 128 bytes of a row.
+constexpr int kSteps = 2;
 constexpr int kXcds = 8;
 
 
@@ -32,6 +34,7 @@ struct Mfma<float> {
 #pragma unroll
         for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
     }
+    __device__ static __forceinline__ void add(acc_t& c, const frag& a, const frag& b) { run(c, a, b); }
     __device__ static __forceinline__ void start(acc_t& c, const frag& a, const frag& b) {
         c = acc_t(0.0f);
         run(c, a, b);
@@ -51,6 +54,10 @@ struct Mfma<bf16_t> {
     __device__ static __forceinline__ void run(acc_t& c, const frag& a, const frag& b) {
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     }
+    // The same through the compiler, which then knows the instruction's wait states: for kernels with registers to spare.
+    __device__ static __forceinline__ void add(acc_t& c, const frag& a, const frag& b) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
     // c = a x b: the first K tile of an item starts the sums, so the accumulators are never cleared.
     __device__ static __forceinline__ void start(acc_t& c, const frag& a, const frag& b) {
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
@@ -62,57 +69,15 @@ struct Mfma<f16_t> {
     __device__ static __forceinline__ void run(acc_t& c, const frag& a, const frag& b) {
         asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     }
+    __device__ static __forceinline__ void add(acc_t& c, const frag& a, const frag& b) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
     __device__ static __forceinline__ void start(acc_t& c, const frag& a, const frag& b) {
         asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
     }
 };
 
 using u32x4 = vec_t<unsigned int, 4>;
-
-struct KernelSegments {
-    const void* ptr[3];
-    long ld[3];
-    int cols[3];
-    int count;
-};
-
-struct KernelArgs {
-    const void* a;
-    const void* b;
-    void* c;            // T* (or float* when c_f32), or float partials when split
-    const void* bias;
-    const void* residual;  // T*, row stride ldr, or null
-    const float* addend;   // fp32 [M, N], row stride ld_addend, added before anything else, or null
-    long ld_addend;
-    int m, n, k;
-    // What the operands hold: rows or columns of A and of B (A's may exceed m, B's n: whole 16-byte chunks of padded
-    // rows), K positions of B (below k when A's padding reaches further: past them B reads as zeros).
-    int a_extent, b_extent, b_k;
-    int k_tiles;            // K tiles of kBK, the last one possibly short
-    int ragged;             // C (or an addend) has rows that are not whole 16-byte chunks: stored element by element
-    long ld_partial;        // SPLIT kernels: row length of a partial tile matrix
-    long lda, ldb, ldc, ldr;
-    int tiles_m, tiles_n;
-    int k_tiles_per_slice;  // K tiles handled by one work item
-    int slices;             // K slices per output tile
-    int accumulate;
-    int c_f32;
-    KernelSegments a_seg, c_seg;  // column segments of A (as stored) and of C; count 0 = one buffer
-    // ceil(2^32 / (group rows * tiles_n)) when multiplying by it divides every item index of the
-    // launch exactly, else 0 (the kernel then divides).
-    unsigned int group_reciprocal;
-    int group_rows_log2;  // tile-rows per L2 locality group: 1 << group_rows_log2
-    void* act;      // SWIGLU kernels: [M, inter] = silu(gate) * up, T*
-    long ld_act;
-    const void* saved;  // GRAD kernels: the forward's [M, 2 * inter] = [gate | up], T*
-    long ld_saved;
-    int inter;      // SWIGLU kernels: columns of gate (= of up); n = 2 * inter
-    // Stacked products (weight-gradient layout only): rows of C per product (0 = one product) and what a and b (or
-    // A's segments) move by from one product to the next, in elements.
-    int batch_rows;
-    long a_batch_stride, b_batch_stride;
-    long a_seg_batch_stride[3];
-};
 
 // The column segment (of up to three) that holds column `col`, picked with selects: indexing the
 // kernel-argument arrays by a run-time value would move them to private memory.
@@ -227,7 +192,7 @@ struct KTile {
     static constexpr int kLoads = ROWS / kRowsPerLoad / kWaves;  // load instructions per wavefront and tile
 
     u32x4 rsrc = {0u, 0u, 0u, 0u};
-    int voffset = 0;
+    int voffset = 0, voffset1 = 0;
     unsigned int group_bytes = 0;  // kRowsPerLoad rows further in global memory
 
     __device__ __forceinline__ static int swizzle(int row) { return (row / (4 / STEPS)) % kChunksPerRow; }
@@ -241,9 +206,13 @@ struct KTile {
         // The tile row of this lane's slot is (i*4 + wave) * kRowsPerLoad + row; its swizzle does not depend on i.
         voffset = static_cast<int>(row * ld * sizeof(T)) +
                   (((lane % kChunksPerRow) ^ swizzle(wave * kRowsPerLoad + row)) * 16);
+        voffset1 = static_cast<int>(row * ld * sizeof(T)) +
+                   (((lane % kChunksPerRow) ^ swizzle((wave + 1) * kRowsPerLoad + row)) * 16);
         group_bytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(kRowsPerLoad * ld * sizeof(T)));
     }
-    __device__ __forceinline__ int load_voffset(int) const { return voffset; }
+    // The lane's offset for load i of a wavefront that loads the whole tile (init with wave 0): with eight rows per load
+    // the swizzle of every other load differs.
+    __device__ __forceinline__ int load_voffset(int i) const { return STEPS == 2 && (i & 1) != 0 ? voffset1 : voffset; }
     // Scalar offset of wavefront `wave`'s first load of the tile that starts at column k0.
     __device__ __forceinline__ unsigned int first_offset(int k0, int wave) const {
         return wave * group_bytes + k0 * static_cast<unsigned int>(sizeof(T));
@@ -301,9 +270,9 @@ struct NTile {
         group_bytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(kRowsPerLoad * ld * sizeof(T)));
     }
     // The lane's offset for load i of a wavefront that loads the whole tile (init with wave 0): fp32 tiles of 64 columns
-    // cover four k rows per load, so that load i's swizzle is 4 i.
+    // cover four k rows per load, so that load i's swizzle is 4 (i % 4).
     __device__ __forceinline__ int load_voffset(int i) const {
-        if constexpr (std::is_same_v<T, float> && COLS == 64) return i == 0 ? voffset : i == 1 ? voffset1 : i == 2 ? voffset2 : voffset3;
+        if constexpr (std::is_same_v<T, float> && COLS == 64) return i % 4 == 0 ? voffset : i % 4 == 1 ? voffset1 : i % 4 == 2 ? voffset2 : voffset3;
         else return voffset;
     }
     // Scalar offset of wavefront `wave`'s first load of the tile that starts at row k0.
