@@ -244,10 +244,10 @@ struct Plan {
 
 // Predicted time of a call in microseconds, from launches measured on random bf16 data inside a graph (operands rotated
 // through 64 MB; K tiles of 64 bytes): what a kernel costs before its K loop, plus the K loop of the busiest CU.
-//   256: one block per CU, 8.5 us for filling its pipeline and storing its tile, 0.48 per K tile on an idle chip, 0.65 at
-//        the power limit of a full one
+//   256: one block per CU, 8.5 us for filling its pipeline and storing its tile (6.8 where the next tile's loads run under
+//        the store), 0.48 per K tile on an idle chip, 0.65 at the power limit of a full one
 //   128: 0.235 per K tile for a block that has a CU to itself, 0.17 each for two that share one where other CUs have less to
-//        do, 0.22 where all of them load at once
+//        do, 0.22 where all of them load at once, up to 0.245 in calls long enough to meet the power limit
 //    64: 0.09 - 0.13 per K tile with up to one block per CU, 0.11 per K tile and block with more
 //    32: 0.07 - 0.1 per K tile (k-contiguous operands stream best), up to one block per CU
 // A split along K adds a launch and the partial tiles' way to memory and back. fp32 K tiles hold 16 positions and take about
@@ -264,9 +264,10 @@ double predicted_us(int tile, long tiles, long slices, long k_tiles, double part
         const double per_tile = tile == 32 ? 0.088 : tile == 64 ? 0.265 : 0.93;
         time = (tile == 32 ? 3.0 : tile == 64 ? 4.0 : 5.0) + kt * per_tile * (tile == 32 ? std::max(1.0, load) : blocks);
     } else if (tile == 256) {
-        time = blocks * (8.5 + kt * (0.48 + 0.17 * load / blocks));
+        time = 8.5 + 6.8 * (blocks - 1.0) + blocks * kt * (0.48 + 0.17 * load / blocks);
     } else if (tile == 128) {
-        time = 5.9 + kt * (load <= 1.0 ? 0.235 : std::max(0.17 * blocks, 0.22 * load)) + 1.2 * std::max(0.0, std::ceil(blocks / 2.0) - 1.0);
+        const double crowded = std::min(0.245, 0.21 + 0.005 * load);
+        time = 5.9 + kt * (load <= 1.0 ? 0.235 : std::max(0.17 * blocks, crowded * load)) + 1.2 * std::max(0.0, std::ceil(blocks / 2.0) - 1.0);
     } else if (tile == 64) {
         time = load <= 1.0 ? 3.4 + kt * (0.09 + 0.04 * load)
                            : 3.4 + kt * 0.11 * blocks * (blocks > 4.0 ? 1.3 : 1.0);
