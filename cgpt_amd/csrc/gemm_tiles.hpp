@@ -198,10 +198,12 @@ struct KTile {
     __device__ __forceinline__ static int swizzle(int row) { return (row / (4 / STEPS)) % kChunksPerRow; }
 
     // base: element (row0, 0) of the operand; rows past rows_left only feed C rows that are never
-    // stored (they read zeros or whatever follows, never out of the allocation's last row).
+    // stored (they read zeros or whatever follows, never out of the allocation's last row). A tile may start behind the
+    // last row (C wider than the operand's rows): rows_left <= 0, and everything reads as zeros.
     __device__ __forceinline__ void init(const T* base, long ld, int rows_left, int k_total, int wave) {
         const int lane = threadIdx.x & (kWave - 1);
         rsrc = make_rsrc(base, (static_cast<long>(rows_left - 1) * ld + k_total) * static_cast<long>(sizeof(T)));
+        rsrc[2] = rows_left > 0 ? rsrc[2] : 0u;
         const int row = lane / kChunksPerRow;
         // The tile row of this lane's slot is (i*4 + wave) * kRowsPerLoad + row; its swizzle does not depend on i.
         voffset = static_cast<int>(row * ld * sizeof(T)) +

@@ -150,3 +150,18 @@ def test_argument_errors(device):
         ops.cut_cross_entropy_forward_backward(loss, x.clone(), c.clone(), x, c, t, 3)
     with pytest.raises(ValueError):
         ops.cut_cross_entropy_forward_backward(loss.half(), x.clone(), c.clone(), x, c, t, 4)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("rows,hidden,vocab", [(40, 64, 65), (54, 512, 209), (33, 128, 97), (300, 256, 1057)])
+def test_logits_rows_wider_than_the_last_tile_of_the_vocabulary(device, rows, hidden, vocab, dtype):
+    """Rows of logits are padded to 128 bytes, so that a 32-wide tile of them may start behind the classifier's last row: it
+    reads nothing and the padding is zero."""
+    x, c = randn((rows, hidden), dtype, 51), randn((vocab, hidden), dtype, 52, 0.05)
+    targets = randint(vocab, (rows,), 53)
+    targets[0] = vocab - 1
+    l64, dx64, dc64 = oracle64.cut_cross_entropy(to_np(x), to_np(c), targets.numpy(), 1024.0)
+    loss, dx, dc = run(device, x, c, targets, 1024.0)
+    assert abs(loss - l64) <= (1e-4 if dtype == torch.float32 else 5e-3) * max(1.0, l64)
+    assert_scaled_close(dx, dx64, STOL[dtype], "dX")
+    assert_scaled_close(dc, dc64, STOL[dtype], "dC")
