@@ -23,66 +23,85 @@ constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / kWave;
 
 // ---- grouping: counting sort of the token positions by id -------------------------------------------
-// Workgroup b owns the ids [b R, (b+1) R) and reads the whole id list twice: first it counts its ids in an
-// LDS histogram and, on the side, the tokens with smaller ids (which is where its part of the output begins:
-// no workgroup waits for another); after an exclusive scan of the histogram it hands every token of its range
-// the next free slot of its id's segment. Slots are handed out with LDS integer atomics, so the order inside a
-// segment is whatever order the lanes arrived in: the row kernel puts each segment into ascending order itself.
+// Workgroup b owns the ids [b R, (b+1) R) and reads the whole id list: it counts its ids in an LDS histogram and, on the
+// side, the tokens with smaller ids (which is where its part of the output begins: no workgroup waits for another); after an
+// exclusive scan of the histogram it hands every token of its range the next free slot of its id's segment. The tokens of
+// the range are listed in LDS on the way, by each wavefront in a part of its own, and handed out from there; a wavefront that
+// found more than its part holds walks the id list again instead. Slots are handed out with LDS integer atomics, so the order
+// inside a segment is whatever order the lanes arrived in: the row kernel puts each segment into ascending order itself.
 // A segment of more than kShort tokens contains positions that are multiples of kShort; order's entries there are marked,
 // which is how the row kernel finds the long segments, and the offset of a workgroup's first id is marked if there is one
 // among its ids, which is how it finds out that it need not look.
 // offsets[id] .. offsets[id + 1] is id's segment of `order`; ids >= vocab belong to nobody and are skipped.
+// Bound by the walk over the id list: 32768 ids take 8000 clocks (their way through the CU's L1 and 32 comparisons a thread),
+// and 4000 more where most of them match (text: half of the tokens are among the first 128 of 32000 ids); the scan 3000, the
+// list 5000. With a second walk in place of the list 17000: the kernel took 18.4 us and takes 12.8. Ranges are as small as one
+// workgroup per CU allows: fewer lanes match at a time (32000 ids in ranges of 128: 20900 clocks, of 1024: 22500).
 constexpr int kGroupThreads = 1024;
-constexpr unsigned int kGroupMaxIds = 32768;  // LDS histogram entries of one workgroup (128 KiB)
+constexpr unsigned int kGroupMinIds = 128, kGroupMaxIds = 32768;  // LDS histogram entries of one workgroup (up to 128 KiB)
 constexpr int kGroupBatch = 8;                // 128-bit id loads a thread keeps in flight
 constexpr unsigned int kShort = 64;           // tokens of a segment that one wavefront orders in registers: one lane each
 constexpr unsigned int kLong = 1u << 31;      // the mark of longer segments; positions and tokens stay below it
+constexpr std::size_t kGroupLds = 160 * 1024 - 512;  // for the histogram and the lists
 
 // The id list is walked in batches of kGroupBatch x 4 ids per thread, all of a batch's loads requested before the
 // first id is looked at (one dependent load per id would cost a memory round trip each). visit(id, t) sees every
-// token once; the order within a workgroup does not matter to any caller.
+// token once, in all lanes of a wavefront at a time: lanes without a token see an id that is in no range. A second walk
+// shows a wavefront the same tokens; their order does not matter to any caller.
 template <typename Visit>
 __device__ __forceinline__ void for_each_id(const std::uint32_t* __restrict__ ids, unsigned int count, bool aligned, Visit&& visit) {
     using u32x4 = vec_t<unsigned int, 4>;
+    constexpr unsigned int kNone = ~0u;
     const unsigned int quads = aligned ? count / 4 : 0;
+    const unsigned int wave_first = __builtin_amdgcn_readfirstlane(threadIdx.x);
     const auto* wide = reinterpret_cast<const u32x4*>(ids);
     for (unsigned int base = 0; base < quads; base += kGroupBatch * kGroupThreads) {
         u32x4 held[kGroupBatch];
 #pragma unroll
-        for (int k = 0; k < kGroupBatch; ++k) {
-            const unsigned int q = base + k * kGroupThreads + threadIdx.x;
-            if (q < quads) held[k] = wide[q];
-        }
+        for (int k = 0; k < kGroupBatch; ++k) held[k] = wide[min(base + k * kGroupThreads + threadIdx.x, quads - 1)];
 #pragma unroll
         for (int k = 0; k < kGroupBatch; ++k) {
+            if (base + k * kGroupThreads + wave_first >= quads) continue;
             const unsigned int q = base + k * kGroupThreads + threadIdx.x;
-            if (q < quads) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) visit(held[k][e], 4 * q + e);
-            }
+            for (int e = 0; e < 4; ++e) visit(q < quads ? held[k][e] : kNone, 4 * q + e);
         }
     }
-    for (unsigned int t = 4 * quads + threadIdx.x; t < count; t += kGroupThreads) visit(ids[t], t);
+    for (unsigned int t0 = 4 * quads; t0 + wave_first < count; t0 += kGroupThreads) {
+        const unsigned int t = t0 + threadIdx.x;
+        visit(t < count ? ids[t] : kNone, t);
+    }
 }
 
 __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned int* __restrict__ offsets,
                                                                        unsigned int* __restrict__ order,
                                                                        const std::uint32_t* __restrict__ ids,
                                                                        unsigned int count, unsigned int vocab,
-                                                                       unsigned int ids_per_group, bool aligned) {
-    extern __shared__ unsigned int bins[];  // [ids_per_group]
+                                                                       unsigned int ids_per_group, unsigned int token_bits,
+                                                                       unsigned int list_entries, bool aligned) {
+    extern __shared__ unsigned int bins[];  // [ids_per_group], then the wavefronts' lists [list_entries]
     __shared__ unsigned int wave_totals[kGroupThreads / kWave];
     __shared__ unsigned int smaller_total;
     const unsigned int lo = blockIdx.x * ids_per_group;
     const unsigned int width = min(ids_per_group, vocab - lo);
-    const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     for (unsigned int i = tid; i < width; i += kGroupThreads) bins[i] = 0;
     if (tid == 0) smaller_total = 0;
     __syncthreads();
-    unsigned int smaller = 0;
-    for_each_id(ids, count, aligned, [&](unsigned int id, unsigned int) {
-        if (id < lo) ++smaller;
-        else if (id - lo < width) atomicAdd(&bins[id - lo], 1u);
+    // An entry of a list: the token in the lower token_bits, the id's place in the range above them.
+    unsigned int* list = bins + ids_per_group + wave * list_entries;
+    unsigned int smaller = 0, listed = 0;
+    for_each_id(ids, count, aligned, [&](unsigned int id, unsigned int t) {
+        const bool match = id - lo < width;
+        smaller += id < lo ? 1u : 0u;
+        const unsigned long long mask = __ballot(match);
+        if (match) {
+            atomicAdd(&bins[id - lo], 1u);
+            const unsigned int entry = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned int>(mask >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo(static_cast<unsigned int>(mask), listed));
+            if (entry < list_entries) list[entry] = t | (id - lo) << token_bits;
+        }
+        listed += __popcll(mask);
     });
 #pragma unroll
     for (int offset = kWave / 2; offset > 0; offset >>= 1) smaller += __shfl_xor(smaller, offset, kWave);
@@ -117,12 +136,26 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
     }
     if (lo + width == vocab && tid == kGroupThreads - 1) offsets[vocab] = running;  // the piece that ends the last range
     __syncthreads();
-    for_each_id(ids, count, aligned, [&](unsigned int id, unsigned int t) {
-        if (id >= lo && id - lo < width) {
-            const unsigned int slot = atomicAdd(&bins[id - lo], 1u);
-            order[slot & ~kLong] = slot % kShort == 0 ? t | (slot & kLong) : t;
-        }
-    });
+    auto place = [&](unsigned int slot, unsigned int t) { order[slot & ~kLong] = slot % kShort == 0 ? t | (slot & kLong) : t; };
+    if (listed > list_entries) {
+        for_each_id(ids, count, aligned, [&](unsigned int id, unsigned int t) {
+            if (id - lo < width) place(atomicAdd(&bins[id - lo], 1u), t);
+        });
+        return;
+    }
+    const unsigned int token_mask = (1u << token_bits) - 1;
+    constexpr unsigned int kAhead = 4;
+    unsigned int i = lane;
+    for (; i + (kAhead - 1) * kWave < listed; i += kAhead * kWave) {
+        unsigned int entry[kAhead], slot[kAhead];
+#pragma unroll
+        for (unsigned int u = 0; u < kAhead; ++u) entry[u] = list[i + u * kWave];
+#pragma unroll
+        for (unsigned int u = 0; u < kAhead; ++u) slot[u] = atomicAdd(&bins[entry[u] >> token_bits], 1u);
+#pragma unroll
+        for (unsigned int u = 0; u < kAhead; ++u) place(slot[u], entry[u] & token_mask);
+    }
+    for (; i < listed; i += kWave) place(atomicAdd(&bins[list[i] >> token_bits], 1u), list[i] & token_mask);
 }
 
 // ---- rows ------------------------------------------------------------------------------------------
@@ -143,8 +176,8 @@ __global__ __launch_bounds__(kGroupThreads) void embedding_group_kernel(unsigned
 // Both live in one launch, the long segments' workgroups first: the chains of the frequent ids run beside the short
 // segments (in a launch of their own they add their 50 us). So the short segments pay for the long ones' registers and LDS
 // with wavefronts in flight, which is why both are bounded (LongRow::kWavesPerSimd) and why nothing is listed where the
-// grouping found no long segment. 32768 tokens x 1024 columns in bf16 over 32000 ids, all launches: uniform ids 36 us, ids Zipf
-// distributed 64, of which the most frequent id, 9.3 per cent of the tokens, sets the end (every id by one wavefront 35 and
+// grouping found no long segment. 32768 tokens x 1024 columns in bf16 over 32000 ids, all launches: uniform ids 30 us, ids Zipf
+// distributed 47 - 58, of which the most frequent id, 9.3 per cent of the tokens, sets the end (every id by one wavefront 35 and
 // 2300; neither bounded nor told that there is nothing to list 48 and 75). A segment is read once per kSpan tokens of the batch,
 // so its work grows with its tokens up to batches of millions: 131072 of 262144 tokens in one id, 128 columns, 2.1 ms
 // (read once per 4096 tokens: 7.0).
@@ -492,23 +525,30 @@ extern "C" int cgptx_embedding_backward(void* grad_weight, const void* grad_outp
     if (int s = scratch(stream, offsets_bytes + token_count * sizeof(unsigned int), &mem)) return s;
     auto* offsets = static_cast<unsigned int*>(mem);
     auto* order = reinterpret_cast<unsigned int*>(static_cast<char*>(mem) + offsets_bytes);
-    // Ranges of at least 1024 ids, at most one workgroup per compute unit, each histogram within the LDS.
-    unsigned int ids_per_group = 1024;
+    // Ranges of a power of two of ids, at most one workgroup per compute unit, each histogram within the LDS.
+    unsigned int ids_per_group = kGroupMinIds, token_bits = 25;
     const unsigned int units = static_cast<unsigned int>(compute_units());
-    while (ids_per_group < kGroupMaxIds && (v + ids_per_group - 1) / ids_per_group > units) ids_per_group *= 2;
+    while (ids_per_group < kGroupMaxIds && (v + ids_per_group - 1) / ids_per_group > units) ids_per_group *= 2, --token_bits;
+    static_assert(kGroupMinIds == 1u << (32 - 25), "an entry of a list is an id's place in its range above a token");
     const unsigned int groups = (v + ids_per_group - 1) / ids_per_group;
-    const std::size_t group_lds = ids_per_group * sizeof(unsigned int);
+    // A wavefront's list: room for all the tokens that it may see, as far as the LDS goes.
+    constexpr std::size_t kWaves = kGroupThreads / kWave;
+    const std::size_t bins_bytes = ids_per_group * sizeof(unsigned int);
+    const std::size_t seen = (token_count + 4 * kGroupThreads - 1) / (4 * kGroupThreads) * (4 * kWave);
+    const std::size_t list_entries = token_count > std::size_t{1} << token_bits
+                                         ? 0
+                                         : std::min(seen, (kGroupLds - bins_bytes) / (kWaves * sizeof(unsigned int)));
+    const std::size_t group_lds = bins_bytes + kWaves * list_entries * sizeof(unsigned int);
     {
         static bool configured = false;
         if (!configured) {
             CGPTX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(embedding_group_kernel),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          static_cast<int>(kGroupMaxIds * sizeof(unsigned int))));
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGroupLds)));
             configured = true;
         }
     }
     hipLaunchKernelGGL(embedding_group_kernel, dim3(groups), dim3(kGroupThreads), group_lds, stream, offsets, order, token_ids,
-                       count, v, ids_per_group, is_aligned16(token_ids));
+                       count, v, ids_per_group, token_bits, static_cast<unsigned int>(list_entries), is_aligned16(token_ids));
     CGPTX_LAUNCH_CHECK();
     return dispatch_dtype(dtype, [&]<typename T>() -> int {
         auto* dw = static_cast<T*>(grad_weight);

@@ -388,6 +388,26 @@ def test_embedding_backward_splits_bit_exact(device, tokens, vocab, hidden, freq
         assert torch.equal(got.cpu(), _added_in_token_order(ids, dy, table, accumulate))
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("tokens,vocab", [
+    (4097, 300),       # ranges of 128 ids, the last one partly filled; one id more than a round of loads
+    (40707, 120),      # one range: wavefronts whose list holds all of their tokens, and one token more
+    (45000, 120),      # no wavefront's list holds its tokens
+    (33000, 33000),    # ranges of 256 ids
+    (140000, 4300000), # ranges of 32768 ids: more tokens than an entry of a list can name
+])
+def test_embedding_backward_grouping_bit_exact(device, tokens, vocab, offset):
+    """The grouping with and without its lists, from an id list that does and does not begin on 16 bytes."""
+    g = torch.Generator().manual_seed(tokens + offset)
+    ids = torch.randint(0, vocab, (tokens,), generator=g)
+    dy, table = randn((tokens, 1), torch.float32, 3), randn((vocab, 1), torch.float32, 4)
+    d_ids = torch.zeros(tokens + offset, dtype=torch.int32, device=device)[offset:]
+    d_ids.copy_(ids)
+    got = table.to(device)
+    ops.embedding_backward(got, dy.to(device), d_ids, tokens, options=ops.EmbeddingBackwardOptions(accumulate_weight=False))
+    assert torch.equal(got.cpu(), _added_in_token_order(ids, dy, table, False))
+
+
 def test_embedding_backward_keeps_non_finite_rows_to_their_ids(device):
     """Long segments read past their last token's row into the same row again: nothing of it is added."""
     ids = torch.arange(1000) % 3
