@@ -1,5 +1,5 @@
 // Causal grouped-query flash attention for gfx950: forward with log-sum-exp,
-// and the backward (delta, dQ, dK/dV) on the matrix cores.
+// and the backward (delta and dQ, dK/dV) on the matrix cores.
 //
 // Reference semantics: include/ops/attention.h:47-78, include/ops/backward/attention_backward.h:24-70,
 // formulas of src/ops/cpu/backward/attention_backward_cpu.cpp:206-280:
@@ -79,8 +79,11 @@ struct Params {
     const void* k;
     const void* v;
     const void* dout;
-    const float* lse;
-    const float* delta;
+    const void* o;         // dq: O
+    const float* lse;      // dq, dkv of the register-staged family: LSE | dkv, LDS-direct family: LSE·log2 e
+    const float* delta;    // dkv
+    float* delta_out;      // dq: delta = rowsum(dO∘O)
+    float* lse2_out;       // dq: LSE·log2 e
     int batch, qs, ks, hq, hkv, d;
     float scale;
     int causal, offset, accumulate;
@@ -346,31 +349,28 @@ __global__ __launch_bounds__(kThreads) void attention_forward_kernel(Params p) {
         p.lse_out[(static_cast<long>(b) * p.qs + q_row) * p.hq + h] = (m + log2f(l)) * kLn2;
 }
 
-// --------------------------------------------------------------------- delta
-// delta[b, t, h] = Σ_d dO·O (and LSE·log2 e next to it), one group of LPR lanes per row, 128-bit loads.
-template <typename T, int LPR>
-__global__ __launch_bounds__(kThreads) void attention_delta_kernel(float* __restrict__ delta,
-                                                                  float* __restrict__ lse2,
-                                                                  const float* __restrict__ lse,
-                                                                  const T* __restrict__ dout,
-                                                                  const T* __restrict__ out, long rows, int d) {
-    const long row = (static_cast<long>(blockIdx.x) * kThreads + threadIdx.x) / LPR;
-    const int sub = threadIdx.x % LPR;
-    float sum = 0.0f;
-    if (row < rows && sub * 8 < d) {
-        const vec_t<float, 8> a = vec_to_f32<T, 8>(load_vec<T, 8>(dout + row * d + sub * 8));
-        const vec_t<float, 8> b = vec_to_f32<T, 8>(load_vec<T, 8>(out + row * d + sub * 8));
+// ------------------------------------------------------------------------ dQ
+// delta = Σ_d dO·O of the rows whose dO fragments a wavefront holds, in all lanes of a row, left in memory (with LSE·log2 e
+// beside it) for the dK/dV pass. A pass of its own read dO once more and was one launch more: backward in a graph, batch x length
+// x heads x width, 3 x 100 x 4:2 x 64 16.2 -> 15.3 us, 1 x 512 x 32:8 x 128 42.8 -> 42.4, 8 x 4096 x 12:4 x 64 748 -> 736,
+// 32 x 1024 x 8:2 x 128 the same. The order of additions is that of a butterfly over the row's groups of eight columns.
+template <typename T, int STEPS>
+__device__ __forceinline__ float row_delta(const typename Mma<T>::frag (&dof)[STEPS], const T* o_row, bool live, int d) {
+    float sum[STEPS];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sum = fmaf(a[e], b[e], sum);
+    for (int s = 0; s < STEPS; ++s) {
+        const auto o = vec_to_f32<T, 8>(global_frag<T>(o_row, live, s, d)), dout = vec_to_f32<T, 8>(dof[s]);
+        sum[s] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[s] = fmaf(dout[e], o[e], sum[s]);
     }
-    sum = wave_sum<LPR>(sum);
-    if (row < rows && sub == 0) {
-        delta[row] = sum;
-        lse2[row] = lse[row] * kLog2e;  // the exponent the wide backward kernels subtract, in base 2
-    }
+#pragma unroll
+    for (int w = STEPS / 2; w > 0; w /= 2)
+#pragma unroll
+        for (int s = 0; s < w; ++s) sum[s] += sum[s + w];
+    return sum[0] + __shfl_xor(sum[0], 32, kWave);
 }
 
-// ------------------------------------------------------------------------ dQ
 template <typename T, int DP>
 __global__ __launch_bounds__(kThreads) void attention_dq_kernel(Params p) {
     constexpr int STEPS = DP / 16, DT = DP / 32;
@@ -395,7 +395,11 @@ __global__ __launch_bounds__(kThreads) void attention_dq_kernel(Params p) {
     }
     const long stat_index = (static_cast<long>(b) * p.qs + q_row) * p.hq + h;
     const float lse2 = q_live ? p.lse[stat_index] * kLog2e : 0.0f;
-    const float delta = q_live ? p.delta[stat_index] : 0.0f;
+    const float delta = row_delta<T, STEPS>(dof, static_cast<const T*>(p.o) + q_offset, q_live, p.d);
+    if (q_live && lane < 32) {
+        p.delta_out[stat_index] = delta;
+        p.lse2_out[stat_index] = lse2;
+    }
 
     acc_t dq[DT];
 #pragma unroll
@@ -986,7 +990,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_forward_wide_kernel(Par
 
 // dQ, LDS-direct family: the forward kernel's streaming scheme; per 32-key half tile
 // Sᵀ = K·Qᵀ and dPᵀ = V·dOᵀ (two independent MFMA chains), dS = P∘(dP − delta) in registers,
-// dQᵀ += Kᵀ·dSᵀ with K read back transposed. lse2 holds LSE·log2(e).
+// dQᵀ += Kᵀ·dSᵀ with K read back transposed.
 template <typename T, int W, int PARTS>
 __global__ __launch_bounds__(kThreads, 2) void attention_dq_wide_kernel(Params p) {
     using frag = typename Mma<T>::frag;
@@ -1028,8 +1032,12 @@ __global__ __launch_bounds__(kThreads, 2) void attention_dq_wide_kernel(Params p
         dof[s] = global_frag<T>(static_cast<const T*>(p.dout) + q_offset, q_live, s, p.d);
     }
     const long stat_index = (static_cast<long>(b) * p.qs + q_row) * p.hq + h;
-    const float lse2 = q_live ? p.lse[stat_index] : 0.0f;
-    const float delta = q_live ? p.delta[stat_index] : 0.0f;
+    const float lse2 = q_live ? p.lse[stat_index] * kLog2e : 0.0f;  // the exponent that both backward kernels subtract, in base 2
+    const float delta = row_delta<T, STEPS>(dof, static_cast<const T*>(p.o) + q_offset, q_live, p.d);
+    if (q_live && part == 0 && lane < 32) {
+        p.delta_out[stat_index] = delta;
+        p.lse2_out[stat_index] = lse2;
+    }
     int k_off[STEPS], kt_off[DT][2];
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) k_off[s] = wide_direct_offset<W>(lane, s);
@@ -1871,29 +1879,15 @@ int launch_backward(const Shape& s, Params p, void* dq, void* dk, void* dv, cons
         });
     }
     return dispatch_16bit(s.dtype, [&]<typename T>() -> int {
-        const int lpr = s.d <= 32 ? 4 : (s.d <= 64 ? 8 : 16);
-        const unsigned int delta_blocks = static_cast<unsigned int>((rows * lpr + kThreads - 1) / kThreads);
-        auto* dout_t = static_cast<const T*>(dout);
-        auto* out_t = static_cast<const T*>(out);
-        const long r = static_cast<long>(rows);
-        const int d = static_cast<int>(s.d);
-        if (lpr == 4)
-            hipLaunchKernelGGL((attention_delta_kernel<T, 4>), dim3(delta_blocks), dim3(kThreads), 0, stream, delta,
-                               lse2, lse, dout_t, out_t, r, d);
-        else if (lpr == 8)
-            hipLaunchKernelGGL((attention_delta_kernel<T, 8>), dim3(delta_blocks), dim3(kThreads), 0, stream, delta,
-                               lse2, lse, dout_t, out_t, r, d);
-        else
-            hipLaunchKernelGGL((attention_delta_kernel<T, 16>), dim3(delta_blocks), dim3(kThreads), 0, stream, delta,
-                               lse2, lse, dout_t, out_t, r, d);
-        CGPTX_LAUNCH_CHECK();
         return dispatch_head_dim(s.d, [&]<int DP>() -> int {
             Params pq = p;
             pq.out0 = dq;
+            pq.o = out;
+            pq.delta_out = delta;
+            pq.lse2_out = lse2;
             const dim3 q_grid(static_cast<unsigned int>((s.qs + kBlockRows - 1) / kBlockRows),
                               static_cast<unsigned int>(s.hq), static_cast<unsigned int>(s.batch));
             if (wide_path(s)) {
-                pq.lse = lse2;
                 if (two_parts(s)) {
                     const int st = s.d <= 64 ? launch_two_parts<attention_dq_wide_kernel<T, 64, 2>, 64>(s, pq, stream)
                                              : launch_two_parts<attention_dq_wide_kernel<T, 128, 2>, 128>(s, pq, stream);
