@@ -160,7 +160,8 @@ struct ColumnReduceSink {
         return block;
     }
 };
-// Bytes one norm-backward pass of the given kind takes from a sink (0: that shape reduces at once, from the arena).
+// Bytes one norm-backward pass of the given kind takes from a sink (0: that shape reduces at once, from the arena). with_rope: at
+// most, for q's and k's rows together.
 enum class NormPass { plain, with_rope, dual };
 std::size_t rmsnorm_backward_sink_bytes(NormPass pass, std::size_t rows, std::size_t hidden, int dtype);
 // Runs the reductions recorded in `table` (device copy of `entries`).
@@ -173,19 +174,26 @@ int rmsnorm_backward_residual(void* grad_input, void* grad_weight, const void* g
                               const void* weight, const void* residual, std::size_t rows, std::size_t hidden,
                               float epsilon, int dtype, hipStream_t stream, ColumnReduceSink* sink = nullptr);
 
-// Per-head RMSNorm and rotary embedding in one pass over [rows = tokens x heads, head_dim]:
-//   forward   output = rope(rmsnorm(input));   backward   the gradient of that, with the weight gradient.
+// Per-head RMSNorm and rotary embedding of q and k in one pass over their [rows = tokens x heads, head_dim]:
+//   forward   output = rope(rmsnorm(input));   backward   output = the gradient of that, with the weight gradient.
 // Bit for bit what the separate operators give (their intermediate roundings are kept). Positions are
 // position_offset + token % sequence, token = row / heads. `rmsnorm_rope_fusable` says whether the shape,
 // dtype and alignment are served; callers run the separate operators otherwise.
+struct NormRopeTensors {
+    void* output;
+    const void* input;
+    const void* weight;
+    std::size_t heads;
+    const void* grad_output = nullptr;  // backward; may be output itself
+    void* grad_weight = nullptr;        // backward
+};
 bool rmsnorm_rope_fusable(const void* a, const void* b, const void* c, const void* weight, const void* cos_cache,
                           const void* sin_cache, std::size_t head_dim, std::size_t rotary_dim, int dtype);
-int rmsnorm_rope_forward(void* output, const void* input, const void* weight, const void* cos_cache, const void* sin_cache,
-                         std::size_t rows, std::size_t head_dim, std::size_t heads, std::size_t sequence,
-                         std::size_t rotary_dim, std::size_t position_offset, float epsilon, int dtype, hipStream_t stream);
-int rmsnorm_rope_backward(void* grad_input, void* grad_weight, const void* grad_output, const void* input,
-                          const void* weight, const void* cos_cache, const void* sin_cache, std::size_t rows,
-                          std::size_t head_dim, std::size_t heads, std::size_t sequence, std::size_t rotary_dim,
+int rmsnorm_rope_forward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
+                         std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
+                         std::size_t position_offset, float epsilon, int dtype, hipStream_t stream);
+int rmsnorm_rope_backward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
+                          std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
                           std::size_t position_offset, float epsilon, int dtype, hipStream_t stream,
                           ColumnReduceSink* sink = nullptr);
 

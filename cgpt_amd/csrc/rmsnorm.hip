@@ -83,14 +83,15 @@ __device__ __forceinline__ vec_t<float, kVec128<T>> rope_vector(vec_t<float, kVe
 }
 
 // ------------------------------------------------------------------ fast path
-template <typename T, int LPR, int K, bool Backward, bool Rope = false>
-__global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(
+// Workgroup `block` of `blocks`.
+template <typename T, int LPR, int K, bool Backward, bool Rope>
+__device__ __forceinline__ void rmsnorm_rows(
     T* out,                         // dx (backward) or y (forward)
-    float* __restrict__ partial,    // [gridDim.x, H] dgamma partials (backward)
+    float* __restrict__ partial,    // [blocks, H] dgamma partials (backward)
     const T* dy,                    // backward only; may be out itself
     const T* residual,              // backward only, optional: added to dx (may be out itself)
     const T* __restrict__ x, const T* __restrict__ w, int rows, int hidden, float inv_hidden, float eps,
-    RopeArgs rope = RopeArgs{}) {
+    const RopeArgs& rope, int block, int blocks) {
     constexpr int VEC = kVec128<T>;
     constexpr int RPW = kWave / LPR;  // rows per wavefront iteration
     using F = vec_t<float, VEC>;
@@ -112,8 +113,8 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(
     }
 
     const int groups = (rows + RPW - 1) / RPW;
-    const int wave_global = blockIdx.x * kWavesPerBlock + wave;
-    const int wave_count = gridDim.x * kWavesPerBlock;
+    const int wave_global = block * kWavesPerBlock + wave;
+    const int wave_count = blocks * kWavesPerBlock;
     for (int g = wave_global; g < groups; g += wave_count) {
         const int row = g * RPW + rsel;
         const bool row_live = row < rows;
@@ -196,22 +197,30 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(
             float v = 0.0f;
 #pragma unroll
             for (int s = 0; s < kWavesPerBlock; ++s) v += stage[s][col];
-            partial[static_cast<std::size_t>(blockIdx.x) * hidden + col] = v;
+            partial[static_cast<std::size_t>(block) * hidden + col] = v;
         }
     }
 }
 
+template <typename T, int LPR, int K, bool Backward>
+__global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(T* out, float* __restrict__ partial, const T* dy, const T* residual,
+                                                                const T* __restrict__ x, const T* __restrict__ w, int rows,
+                                                                int hidden, float inv_hidden, float eps) {
+    rmsnorm_rows<T, LPR, K, Backward, false>(out, partial, dy, residual, x, w, rows, hidden, inv_hidden, eps, RopeArgs{}, blockIdx.x,
+                                             gridDim.x);
+}
+
 // The fused per-head norm + rotary pass at the shape a training step gives it: rows of exactly 16 vectors (head_dim 128
 // in 16-bit storage), all of them rotated, a multiple of four rows, tensors and tables below 4 GiB. Same arithmetic,
-// in the same order, as rmsnorm_rows_kernel<T, 16, 1, Backward, true>; what differs is the bookkeeping, which at 2 KiB
+// in the same order, as rmsnorm_rows<T, 16, 1, Backward, true>; what differs is the bookkeeping, which at 2 KiB
 // of rows per wavefront and trip is what that kernel spends most of its instructions on: no per-lane predicates, 32-bit
 // byte offsets that advance by a constant, and the token position carried from trip to trip (head index and position
 // advance by constants with one carry each) instead of two integer divisions per trip. A trip requests U groups of
 // four rows before it uses the first, so that a wavefront has U times the bytes in flight.
 template <typename T, bool Backward, int U>
-__global__ __launch_bounds__(kThreads) void rmsnorm_rope_dense_kernel(
+__device__ __forceinline__ void rmsnorm_rope_dense(
     T* out, float* __restrict__ partial, const T* dy /* may be out itself */, const T* __restrict__ x,
-    const T* __restrict__ w, int rows, float inv_hidden, float eps, RopeArgs rope) {
+    const T* __restrict__ w, int rows, float inv_hidden, float eps, const RopeArgs& rope, int block, int blocks) {
     constexpr int VEC = kVec128<T>;
     constexpr int HALF = VEC / 2;
     constexpr int LPR = 16;
@@ -228,8 +237,8 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rope_dense_kernel(
     F acc(0.0f);
 
     const int groups = rows / RPW;
-    const int wave_global = blockIdx.x * kWavesPerBlock + wave;
-    const int wave_count = gridDim.x * kWavesPerBlock;
+    const int wave_global = block * kWavesPerBlock + wave;
+    const int wave_count = blocks * kWavesPerBlock;
     const int first_row = wave_global * RPW + rsel;
     const int stride_rows = wave_count * RPW;
     int head = first_row % rope.heads;
@@ -343,9 +352,36 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rope_dense_kernel(
             float v = 0.0f;
 #pragma unroll
             for (int s = 0; s < kWavesPerBlock; ++s) v += stage[s][col];
-            partial[static_cast<std::size_t>(blockIdx.x) * HIDDEN + col] = v;
+            partial[static_cast<std::size_t>(block) * HIDDEN + col] = v;
         }
     }
+}
+
+// q and k in one launch: the first blocks_q workgroups take q's rows, the others k's. In a call of a few hundred tokens each of the
+// two is a launch of 4.5 us for less than one of work.
+template <typename T>
+struct RopeRows {
+    T* out;
+    float* partial;
+    const T* dy;
+    const T* x;
+    const T* w;
+    int rows, heads;
+};
+template <typename T, bool Backward, bool Dense>
+__global__ __launch_bounds__(kThreads) void rmsnorm_rope_pair_kernel(RopeRows<T> q, RopeRows<T> k, int blocks_q, int hidden,
+                                                                     float inv_hidden, float eps, RopeArgs rope) {
+    const bool second = static_cast<int>(blockIdx.x) >= blocks_q;
+    const int block = static_cast<int>(blockIdx.x) - (second ? blocks_q : 0);
+    const int blocks = second ? static_cast<int>(gridDim.x) - blocks_q : blocks_q;
+    const RopeRows<T> of = second ? k : q;
+    rope.heads = of.heads;
+    if constexpr (Dense)
+        rmsnorm_rope_dense<T, Backward, kRopeDenseUnroll<Backward>>(of.out, of.partial, of.dy, of.x, of.w, of.rows, inv_hidden, eps, rope,
+                                                                    block, blocks);
+    else
+        rmsnorm_rows<T, 16, 1, Backward, true>(of.out, of.partial, of.dy, nullptr, of.x, of.w, of.rows, hidden, inv_hidden, eps, rope,
+                                               block, blocks);
 }
 
 // Two RMSNorms of the same rows with different weights (the block's attention and feed-forward norms
@@ -586,19 +622,8 @@ bool rope_dense(int rows, int hidden, const RopeArgs& rope) {
 
 template <typename T, bool Backward>
 int launch_fast(const FastShape shape, T* out, float* partial, const T* dy, const T* residual, const T* x, const T* w,
-                int rows, int hidden, float eps, int blocks, hipStream_t stream, const RopeArgs* rope = nullptr) {
+                int rows, int hidden, float eps, int blocks, hipStream_t stream) {
     const float inv_hidden = 1.0f / static_cast<float>(hidden);
-    if (rope != nullptr) {
-        if (shape.lpr != 16 || shape.k != 1) return fail(CGPTX_RUNTIME, "rmsnorm: no rotary kernel for shape");
-        if (rope_dense<T>(rows, hidden, *rope)) {
-            hipLaunchKernelGGL((rmsnorm_rope_dense_kernel<T, Backward, kRopeDenseUnroll<Backward>>), dim3(blocks), dim3(kThreads), 0, stream, out,
-                               partial, dy, x, w, rows, inv_hidden, eps, *rope);
-            return CGPTX_OK;
-        }
-        hipLaunchKernelGGL((rmsnorm_rows_kernel<T, 16, 1, Backward, true>), dim3(blocks), dim3(kThreads), 0, stream, out,
-                           partial, dy, residual, x, w, rows, hidden, inv_hidden, eps, *rope);
-        return CGPTX_OK;
-    }
 #define CGPTX_RMS_CASE(L, KK)                                                                             \
     if (shape.lpr == L && shape.k == KK) {                                                                \
         hipLaunchKernelGGL((rmsnorm_rows_kernel<T, L, KK, Backward>), dim3(blocks), dim3(kThreads), 0,   \
@@ -616,12 +641,7 @@ int launch_fast(const FastShape shape, T* out, float* partial, const T* dy, cons
 
 // The kernel launch_fast would launch (null when there is none).
 template <typename T, bool Backward>
-const void* fast_kernel(const FastShape shape, bool rope, bool dense = false) {
-    if (rope) {
-        if (shape.lpr != 16 || shape.k != 1) return nullptr;
-        return dense ? reinterpret_cast<const void*>(&rmsnorm_rope_dense_kernel<T, Backward, kRopeDenseUnroll<Backward>>)
-                     : reinterpret_cast<const void*>(&rmsnorm_rows_kernel<T, 16, 1, Backward, true>);
-    }
+const void* fast_kernel(const FastShape shape) {
 #define CGPTX_RMS_CASE(L, KK) \
     if (shape.lpr == L && shape.k == KK) return reinterpret_cast<const void*>(&rmsnorm_rows_kernel<T, L, KK, Backward>);
     CGPTX_RMS_CASE(16, 1)
@@ -730,50 +750,85 @@ int run_column_reductions(const ColumnReduceEntry* table, const std::vector<Colu
     return CGPTX_OK;
 }
 
-int rmsnorm_rope_forward(void* output, const void* input, const void* weight, const void* cos_cache, const void* sin_cache,
-                         std::size_t rows, std::size_t head_dim, std::size_t heads, std::size_t sequence,
-                         std::size_t rotary_dim, std::size_t position_offset, float epsilon, int dtype, hipStream_t stream) {
-    if (int s = validate(output, input, weight, rows, head_dim, epsilon, dtype, "rmsnorm_rope_forward")) return s;
-    if (cos_cache == nullptr || sin_cache == nullptr || heads == 0 || sequence == 0 ||
-        !rmsnorm_rope_fusable(output, input, nullptr, weight, cos_cache, sin_cache, head_dim, rotary_dim, dtype))
-        return fail(CGPTX_INVALID_ARGUMENT, "rmsnorm_rope_forward: shape or alignment not served by the fused pass");
-    const int r = static_cast<int>(rows), h = static_cast<int>(head_dim);
-    const RopeArgs rope = make_rope(cos_cache, sin_cache, heads, sequence, rotary_dim, position_offset);
+namespace {
+// Workgroups that rows of 16 vectors fill, four rows a wavefront.
+int pair_blocks(int rows) { return static_cast<int>((static_cast<long>(rows) + 4 * kWavesPerBlock - 1) / (4 * kWavesPerBlock)); }
+
+// The pair kernel's form for these rows, and how many workgroups each of the two takes: in the ratio of their rows where the chip
+// does not hold one per group of rows.
+template <typename T, bool Backward>
+struct PairPlan {
+    bool dense;
+    int blocks_q, blocks_k;
+    PairPlan(int rows_q, int rows_k, int head_dim, RopeArgs rope) : dense(rope_dense<T>(std::max(rows_q, rows_k), head_dim, rope) &&
+                                                                          rows_q % 4 == 0 && rows_k % 4 == 0) {
+        const long q = pair_blocks(rows_q), k = pair_blocks(rows_k);
+        const long cap = resident_blocks(dense ? reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, true>)
+                                               : reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, false>));
+        blocks_q = static_cast<int>(q + k <= cap ? q : std::max(1L, std::min(cap - 1, cap * q / (q + k))));
+        blocks_k = static_cast<int>(q + k <= cap ? k : std::min(k, cap - blocks_q));
+    }
+};
+template <typename T, bool Backward>
+int launch_pair(const PairPlan<T, Backward>& plan, const RopeRows<T>& q, const RopeRows<T>& k, int head_dim, float epsilon,
+                const RopeArgs& rope, hipStream_t stream) {
+    auto kernel = plan.dense ? rmsnorm_rope_pair_kernel<T, Backward, true> : rmsnorm_rope_pair_kernel<T, Backward, false>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(plan.blocks_q + plan.blocks_k)), dim3(kThreads), 0, stream, q, k,
+                       plan.blocks_q, head_dim, 1.0f / static_cast<float>(head_dim), epsilon, rope);
+    CGPTX_LAUNCH_CHECK();
+    return CGPTX_OK;
+}
+}  // namespace
+
+int rmsnorm_rope_forward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
+                         std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
+                         std::size_t position_offset, float epsilon, int dtype, hipStream_t stream) {
+    for (const NormRopeTensors* t : {&q, &k}) {
+        if (int s = validate(t->output, t->input, t->weight, tokens * t->heads, head_dim, epsilon, dtype, "rmsnorm_rope_forward")) return s;
+        if (cos_cache == nullptr || sin_cache == nullptr || sequence == 0 ||
+            !rmsnorm_rope_fusable(t->output, t->input, nullptr, t->weight, cos_cache, sin_cache, head_dim, rotary_dim, dtype))
+            return fail(CGPTX_INVALID_ARGUMENT, "rmsnorm_rope_forward: shape or alignment not served by the fused pass");
+    }
+    const int h = static_cast<int>(head_dim);
+    const RopeArgs rope = make_rope(cos_cache, sin_cache, 0, sequence, rotary_dim, position_offset);
     return dispatch_dtype(dtype, [&]<typename T>() -> int {
-        const FastShape shape = pick_fast_shape<T>(h);
-        if (int s = launch_fast<T, false>(shape, static_cast<T*>(output), nullptr, nullptr, nullptr,
-                                          static_cast<const T*>(input), static_cast<const T*>(weight), r, h, epsilon,
-                                          fast_blocks(shape, r, fast_kernel<T, false>(shape, true, rope_dense<T>(r, h, rope))), stream, &rope))
-            return s;
-        CGPTX_LAUNCH_CHECK();
-        return CGPTX_OK;
+        const auto rows = [&](const NormRopeTensors& t) {
+            return RopeRows<T>{static_cast<T*>(t.output), nullptr, nullptr, static_cast<const T*>(t.input),
+                               static_cast<const T*>(t.weight), static_cast<int>(tokens * t.heads), static_cast<int>(t.heads)};
+        };
+        const RopeRows<T> of_q = rows(q), of_k = rows(k);
+        return launch_pair<T, false>(PairPlan<T, false>(of_q.rows, of_k.rows, h, rope), of_q, of_k, h, epsilon, rope, stream);
     });
 }
 
-int rmsnorm_rope_backward(void* grad_input, void* grad_weight, const void* grad_output, const void* input,
-                          const void* weight, const void* cos_cache, const void* sin_cache, std::size_t rows,
-                          std::size_t head_dim, std::size_t heads, std::size_t sequence, std::size_t rotary_dim,
+int rmsnorm_rope_backward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
+                          std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
                           std::size_t position_offset, float epsilon, int dtype, hipStream_t stream, ColumnReduceSink* sink) {
-    if (int s = validate(grad_input, grad_output, input, rows, head_dim, epsilon, dtype, "rmsnorm_rope_backward")) return s;
-    if (grad_weight == nullptr || weight == nullptr || cos_cache == nullptr || sin_cache == nullptr || heads == 0 ||
-        sequence == 0 ||
-        !rmsnorm_rope_fusable(grad_input, grad_output, input, weight, cos_cache, sin_cache, head_dim, rotary_dim, dtype))
-        return fail(CGPTX_INVALID_ARGUMENT, "rmsnorm_rope_backward: shape or alignment not served by the fused pass");
-    const int r = static_cast<int>(rows), h = static_cast<int>(head_dim);
-    const RopeArgs rope = make_rope(cos_cache, sin_cache, heads, sequence, rotary_dim, position_offset);
+    for (const NormRopeTensors* t : {&q, &k}) {
+        if (int s = validate(t->output, t->grad_output, t->input, tokens * t->heads, head_dim, epsilon, dtype, "rmsnorm_rope_backward"))
+            return s;
+        if (t->grad_weight == nullptr || t->weight == nullptr || cos_cache == nullptr || sin_cache == nullptr || sequence == 0 ||
+            !rmsnorm_rope_fusable(t->output, t->grad_output, t->input, t->weight, cos_cache, sin_cache, head_dim, rotary_dim, dtype))
+            return fail(CGPTX_INVALID_ARGUMENT, "rmsnorm_rope_backward: shape or alignment not served by the fused pass");
+    }
+    const int h = static_cast<int>(head_dim);
+    const RopeArgs rope = make_rope(cos_cache, sin_cache, 0, sequence, rotary_dim, position_offset);
     return dispatch_dtype(dtype, [&]<typename T>() -> int {
-        const FastShape shape = pick_fast_shape<T>(h);
-        const int blocks = fast_blocks(shape, r, fast_kernel<T, true>(shape, true, rope_dense<T>(r, h, rope)));
+        const PairPlan<T, true> plan(static_cast<int>(tokens * q.heads), static_cast<int>(tokens * k.heads), h, rope);
         void* mem = nullptr;
         bool deferred = false;
-        if (int s = partial_memory(sink, stream, static_cast<std::size_t>(blocks) * head_dim * sizeof(float), &mem, &deferred)) return s;
-        auto* partial = static_cast<float*>(mem);
-        if (int s = launch_fast<T, true>(shape, static_cast<T*>(grad_input), partial, static_cast<const T*>(grad_output),
-                                         nullptr, static_cast<const T*>(input), static_cast<const T*>(weight), r, h, epsilon,
-                                         blocks, stream, &rope))
+        if (int s = partial_memory(sink, stream, static_cast<std::size_t>(plan.blocks_q + plan.blocks_k) * head_dim * sizeof(float), &mem,
+                                   &deferred))
             return s;
-        CGPTX_LAUNCH_CHECK();
-        return reduce_columns<T>(sink, deferred, static_cast<T*>(grad_weight), partial, blocks, h, dtype, stream);
+        auto* partial_q = static_cast<float*>(mem);
+        float* partial_k = partial_q + static_cast<std::size_t>(plan.blocks_q) * head_dim;
+        const auto rows = [&](const NormRopeTensors& t, float* partial) {
+            return RopeRows<T>{static_cast<T*>(t.output), partial, static_cast<const T*>(t.grad_output), static_cast<const T*>(t.input),
+                               static_cast<const T*>(t.weight), static_cast<int>(tokens * t.heads), static_cast<int>(t.heads)};
+        };
+        if (int s = launch_pair<T, true>(plan, rows(q, partial_q), rows(k, partial_k), h, epsilon, rope, stream)) return s;
+        if (int s = reduce_columns<T>(sink, deferred, static_cast<T*>(q.grad_weight), partial_q, plan.blocks_q, h, dtype, stream)) return s;
+        return reduce_columns<T>(sink, deferred, static_cast<T*>(k.grad_weight), partial_k, plan.blocks_k, h, dtype, stream);
     });
 }
 
@@ -915,7 +970,7 @@ int rmsnorm_backward_impl(void* grad_input, void* grad_weight, const void* grad_
         const bool aligned = is_aligned16(dx) && is_aligned16(dy) && is_aligned16(x) && is_aligned16(w) && is_aligned16(res);
         const int reduce_blocks = (h + kWave - 1) / kWave;
         if (shape.lpr != 0 && aligned) {
-            const int blocks = fast_blocks(shape, r, fast_kernel<T, true>(shape, false));
+            const int blocks = fast_blocks(shape, r, fast_kernel<T, true>(shape));
             void* mem = nullptr;
             const std::size_t bytes = static_cast<std::size_t>(blocks) * hidden * sizeof(float);
             if (workspace.sink != nullptr) mem = workspace.sink->take(bytes);
@@ -960,14 +1015,17 @@ std::size_t rmsnorm_backward_sink_bytes(NormPass pass, std::size_t rows, std::si
     dispatch_dtype(dtype, [&]<typename T>() -> int {
         const FastShape shape = pick_fast_shape<T>(h);
         if (shape.lpr == 0) return CGPTX_OK;
-        const void* kernel = pass == NormPass::dual ? dual_kernel<T, true>(shape) : fast_kernel<T, true>(shape, pass == NormPass::with_rope);
-        if (kernel == nullptr) return CGPTX_OK;
-        int blocks = fast_blocks(shape, r, kernel);
+        int blocks = 0;
         if (pass == NormPass::with_rope) {
             // The pass picks between two kernels by properties of its rotary tables that are not known here: room
-            // for whichever of them takes more.
-            const int other = fast_blocks(shape, r, fast_kernel<T, true>(shape, true, true));
-            blocks = other > blocks ? other : blocks;
+            // for whichever of them takes more. q's and k's last workgroups may both be partly filled.
+            for (const void* kernel : {reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, true, false>),
+                                       reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, true, true>)})
+                blocks = std::max(blocks, std::min(pair_blocks(r) + 1, resident_blocks(kernel)));
+        } else {
+            const void* kernel = pass == NormPass::dual ? dual_kernel<T, true>(shape) : fast_kernel<T, true>(shape);
+            if (kernel == nullptr) return CGPTX_OK;
+            blocks = fast_blocks(shape, r, kernel);
         }
         const std::size_t partial_bytes = static_cast<std::size_t>(blocks) * hidden * sizeof(float);
         bytes = pass == NormPass::dual ? 2 * partial_bytes : partial_bytes;
@@ -1046,7 +1104,7 @@ extern "C" int cgptx_rmsnorm_forward(void* output, const void* input, const void
         auto* w = static_cast<const T*>(weight);
         const FastShape shape = pick_fast_shape<T>(h);
         if (shape.lpr != 0 && is_aligned16(y) && is_aligned16(x) && is_aligned16(w)) {
-            const int blocks = fast_blocks(shape, r, fast_kernel<T, false>(shape, false));
+            const int blocks = fast_blocks(shape, r, fast_kernel<T, false>(shape));
             if (int s = launch_fast<T, false>(shape, y, nullptr, nullptr, nullptr, x, w, r, h, epsilon, blocks, stream)) return s;
             CGPTX_LAUNCH_CHECK();
             return CGPTX_OK;

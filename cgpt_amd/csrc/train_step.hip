@@ -733,10 +733,8 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             CGPTX_OP("gemm_fwd.qkv", cgptx_linear_forward(a.v, a.norm_a, w.v.value, nullptr, N, H, KW, dt, s));
         }
         if (fused_qk_norm_rope(m, a.q, a.q_pre, nullptr, w.q_norm.value) && fused_qk_norm_rope(m, a.k, a.k_pre, nullptr, w.k_norm.value)) {
-            CGPTX_OP("rmsnorm_fwd", rmsnorm_rope_forward(a.q, a.q_pre, w.q_norm.value, m->cos_cache, m->sin_cache, N * HQ, D, HQ,
-                                                         m->sequence, c.rotary_dim, 0, eps, dt, stream));
-            CGPTX_OP("rmsnorm_fwd", rmsnorm_rope_forward(a.k, a.k_pre, w.k_norm.value, m->cos_cache, m->sin_cache, N * HKV, D, HKV,
-                                                         m->sequence, c.rotary_dim, 0, eps, dt, stream));
+            CGPTX_OP("rmsnorm_fwd", rmsnorm_rope_forward({a.q, a.q_pre, w.q_norm.value, HQ}, {a.k, a.k_pre, w.k_norm.value, HKV},
+                                                         m->cos_cache, m->sin_cache, N, D, m->sequence, c.rotary_dim, 0, eps, dt, stream));
         } else {
             CGPTX_OP("rmsnorm_fwd", cgptx_rmsnorm_forward(a.q, a.q_pre, w.q_norm.value, N * HQ, D, eps, dt, s));
             CGPTX_OP("rmsnorm_fwd", cgptx_rmsnorm_forward(a.k, a.k_pre, w.k_norm.value, N * HKV, D, eps, dt, s));
@@ -819,10 +817,9 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         // In place over the attention gradients (a lane reads and writes the same elements).
         if (fused_qk_norm_rope(m, d_q, d_q, a.q_pre, w.q_norm.value) &&
             fused_qk_norm_rope(m, d_k, d_k, a.k_pre, w.k_norm.value)) {
-            CGPTX_OP("rmsnorm_bwd", rmsnorm_rope_backward(d_q, w.q_norm.gradient, d_q, a.q_pre, w.q_norm.value, m->cos_cache,
-                                                          m->sin_cache, N * HQ, D, HQ, m->sequence, c.rotary_dim, 0, eps, dt, stream, sink));
-            CGPTX_OP("rmsnorm_bwd", rmsnorm_rope_backward(d_k, w.k_norm.gradient, d_k, a.k_pre, w.k_norm.value, m->cos_cache,
-                                                          m->sin_cache, N * HKV, D, HKV, m->sequence, c.rotary_dim, 0, eps, dt, stream, sink));
+            CGPTX_OP("rmsnorm_bwd", rmsnorm_rope_backward({d_q, a.q_pre, w.q_norm.value, HQ, d_q, w.q_norm.gradient},
+                                                          {d_k, a.k_pre, w.k_norm.value, HKV, d_k, w.k_norm.gradient}, m->cos_cache,
+                                                          m->sin_cache, N, D, m->sequence, c.rotary_dim, 0, eps, dt, stream, sink));
         } else {
             CGPTX_OP("rope_bwd", cgptx_rope_backward(m->d_q_pre, m->d_k_pre, d_q, d_k, m->cos_cache, m->sin_cache, m->batch,
                                           m->sequence, HQ, HKV, D, c.rotary_dim, 0, m->sequence, dt, s));
@@ -1065,7 +1062,7 @@ extern "C" int cgptx_model_create(cgptx_model** out, const cgptx_model_config* c
             auto bytes = [&](NormPass pass, std::size_t rows, std::size_t width) {
                 return rmsnorm_backward_sink_bytes(pass, rows, width, c.dtype);
             };
-            const std::size_t heads = std::max(bytes(NormPass::with_rope, N * HQ, D) + bytes(NormPass::with_rope, N * HKV, D),
+            const std::size_t heads = std::max(bytes(NormPass::with_rope, N * (HQ + HKV), D),
                                                bytes(NormPass::plain, N * HQ, D) + bytes(NormPass::plain, N * HKV, D));
             const std::size_t block = std::max(bytes(NormPass::dual, N, H), 2 * bytes(NormPass::plain, N, H));
             const std::size_t total = c.num_layers * (heads + block) + bytes(NormPass::plain, N, H);

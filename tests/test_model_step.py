@@ -378,6 +378,34 @@ def test_fused_qk_norm_rope_is_bit_identical_to_the_separate_operators(device, m
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("head_dim,kv_heads", [(128, 3), (64, 1), (128, 6)], ids=["ragged-split", "general", "equal"])
+def test_fused_qk_norm_rope_of_more_rows_than_the_chip_holds(device, monkeypatch, head_dim, kv_heads):
+    """q and k share the workgroups of one launch in the ratio of their rows once they are more than the chip holds. All but the
+    order of additions in the two norms' weight gradients is that of the separate operators: fp32 sums over up to 72000 rows, one
+    rounding to bf16 (2^-9), beside sums of rounded terms whose error grows with the gradient's largest element."""
+    from cgpt_amd.model import LOSS_DENSE, Model, ModelConfig
+    config = ModelConfig(vocabulary_size=64, num_layers=1, hidden_size=6 * head_dim, intermediate_size=64, num_query_heads=6,
+                         num_kv_heads=kv_heads, head_dim=head_dim, rotary_dim=head_dim, dtype=torch.bfloat16)
+    batch, seq = 60, 200
+    rng = np.random.default_rng(3)
+    inputs, targets = (rng.integers(0, 64, size=batch * seq).astype(np.uint32) for _ in range(2))
+    results = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("CGPTX_FUSE_QK", fuse)
+        model = Model(config, batch, seq, seed=4, device=device)
+        model.set_tokens(inputs, targets)
+        model.forward_backward(loss_scale=4.0, loss_mode=LOSS_DENSE)
+        results.append((model.status()[0], [(name, g.clone()) for name, _, g in model.parameters()]))
+    assert results[0][0] == results[1][0]
+    for (name, a), (_, b) in zip(results[0][1], results[1][1]):
+        if "q_norm" in name or "k_norm" in name:
+            a, b = a.float(), b.float()
+            assert (a - b).abs().max() <= 2.0 ** -8 * b.abs().max()
+        else:
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
 def test_norm_weight_gradients_reduced_at_the_end_of_the_backward_pass_are_bit_identical(device, monkeypatch):
     """The norm-backward passes of a step leave the reduction of their weight-gradient partial sums to one pair of
     launches at the end of the backward pass (same additions, same order); CGPTX_FUSE_DGAMMA=0 reduces after each
