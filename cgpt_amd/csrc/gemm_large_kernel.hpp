@@ -79,6 +79,13 @@ __device__ __forceinline__ void store_chunk(const u32x4& data, __amdgpu_buffer_r
     __builtin_amdgcn_raw_buffer_store_b128(data, rsrc, voffset + soffset, 0, 0);
 }
 
+// Nothing is added to the result, and it is stored in the operands' type on rows of whole 16 bytes.
+__device__ __host__ __forceinline__ bool stored_as_it_is(const KernelArgs& p) {
+    return p.bias == nullptr && p.residual == nullptr && p.addend == nullptr && !p.accumulate && !p.c_f32 && !p.ragged;
+}
+template <int BM, bool SPLIT, bool RESIDUAL, bool SWIGLU, bool GRAD>
+constexpr bool plain_apart = BM == 128 && !SPLIT && !RESIDUAL && !SWIGLU && !GRAD;  // such calls have a kernel of their own
+
 // One workgroup per CU slot walks its share of the work items (output tile x K slice) one after
 // the other: the first K tiles of the next item are requested before the epilogue of the current
 // one, whose stores then drain under the next item's MFMAs.
@@ -93,8 +100,11 @@ __device__ __forceinline__ void store_chunk(const u32x4& data, __amdgpu_buffer_r
 // [gate 0-63 | up 0-63 | gate 64-127 | up 64-127] (one unit per load instruction of a wavefront,
 // so only the scalar offsets of the loads change), and the epilogue computes the product from the
 // rounded gate and up values, as the separate operator would from memory.
+// PLAIN: the result is stored as it is, in the operands' type, by kernels of their own: with the general epilogue beside it the
+// compiler spills 35 - 60 scalar registers (256-wide tiles: 120 - 150) and asks for private memory that nothing touches, without
+// it 0 - 29 and none.
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
-          bool SWIGLU = false, bool GRAD = false, bool DEEP = false>
+          bool SWIGLU = false, bool GRAD = false, bool DEEP = false, bool PLAIN = false>
 __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     static_assert(!GRAD || (A_K && !B_K && !SPLIT && !SEGMENTED && !RESIDUAL && !SWIGLU && BN == 256),
                   "the SwiGLU gradient epilogue belongs to the plain input-gradient kernel with 256-wide tiles");
@@ -613,8 +623,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
             }
             return;
         }
-        bool plain = false;
-        if constexpr (!SPLIT) plain = p.bias == nullptr && p.residual == nullptr && p.addend == nullptr && !p.accumulate && !p.c_f32 && !p.ragged;
+        bool plain = PLAIN;
+        if constexpr (!SPLIT && !plain_apart<BM, SPLIT, RESIDUAL, SWIGLU, GRAD>) plain = stored_as_it_is(p);
         if constexpr (!kIsF32 && !SPLIT) if (plain) {
             // Straight-line code, no per-lane predicates or address arithmetic (with one wavefront per
             // SIMD every branch and every dependent wait is exposed): the stores go through a buffer
@@ -883,15 +893,19 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
 constexpr int blocks_per_unit(int tile) { return tile == 256 ? 1 : 2; }  // resident blocks per CU: what the LDS slots allow
 
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
-          bool SWIGLU = false, bool GRAD = false, bool DEEP = false>
+          bool SWIGLU = false, bool GRAD = false, bool DEEP = false, bool PLAIN = false>
 int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
     const long items = static_cast<long>(p.tiles_m) * p.tiles_n * slices;
-    if constexpr (BM == 128 && !DEEP) {
+    if constexpr (BM == 128 && !DEEP && !PLAIN) {
         if (items <= compute_units())
             return launch_mfma<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, true>(p, slices, stream);
     }
+    if constexpr (plain_apart<BM, SPLIT, RESIDUAL, SWIGLU, GRAD> && !PLAIN) {
+        if (stored_as_it_is(p))
+            return launch_mfma<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP, true>(p, slices, stream);
+    }
     constexpr std::size_t smem = TileLayout<T, BM, BN, A_K, B_K, DEEP>::kSmemBytes;
-    auto kernel = gemm_mfma_kernel<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP>;
+    auto kernel = gemm_mfma_kernel<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP, PLAIN>;
     static bool configured = false;
     if (!configured) {
         CGPTX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
