@@ -291,7 +291,10 @@ Plan make_plan(const GemmArgs& g) {
                            !(g.a_k_contiguous && g.a_segments.count > 0);
     auto set_slices = [&](long slices) {
         plan.k_tiles_per_slice = static_cast<int>((k_tiles + slices - 1) / slices);
-        if (slices > 1) plan.k_tiles_per_slice = (plan.k_tiles_per_slice + kSteps - 1) / kSteps * kSteps;  // whole K tiles
+        // Slices of a k-contiguous operand begin at whole K tiles: its rows are read in whole cache lines. A K step of k-strided
+        // operands is whole rows of memory wherever it begins, and their slices are as long as each other.
+        if (slices > 1 && (g.a_k_contiguous || g.b_k_contiguous))
+            plan.k_tiles_per_slice = (plan.k_tiles_per_slice + kSteps - 1) / kSteps * kSteps;
         plan.slices = static_cast<int>((k_tiles + plan.k_tiles_per_slice - 1) / plan.k_tiles_per_slice);
     };
     if (g.swiglu_out != nullptr || g.swiglu_saved != nullptr || (!f32 && tiles_of(256) >= 3 * units && g.batch_rows == 0)) {

@@ -86,6 +86,33 @@ def test_contractions_whose_last_k_tile_is_half_filled_are_exact_on_integers(dev
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("steps", [1026, 1028, 1033])
+def test_weight_gradients_are_cut_into_equal_k_slices(device, steps, dtype):
+    """A long weight gradient's K steps (32 rows, 16 in fp32) are dealt out to its slices evenly, an odd number each where that
+    is what they come to. The cuts are read off the sums: column j of dY holds 2^24 in step 0, 1 in step j and -2^24 in step
+    j + 1 (as products). A 1 behind the 2^24 of its own slice is lost, 2^24 + 1 being no float; so is one that is the last of
+    a later slice, where it meets the 2^24 alone."""
+    rows = steps * (16 if dtype == torch.float32 else 32)
+    width = 1024
+    dy = torch.zeros(steps, rows // steps, width, dtype=dtype, device=device)
+    column = torch.arange(width, device=device)
+    dy[0, 0] = 4096
+    dy[column + 1, 0, column] = 2.0 ** -12
+    dy[column + 2, 0, column] = -4096
+    x = torch.full((rows, width), 4096, dtype=dtype, device=device)
+    gw = torch.full((width, width), float("nan"), dtype=dtype, device=device)
+    ops.linear_backward(None, gw, None, dy.view(rows, width), x, x[:width])
+    assert torch.equal(gw, gw[:, :1].expand_as(gw))
+    kept = gw[:, 0].cpu()
+    assert ((kept == 0) | (kept == 1)).all()
+    length = int(kept.nonzero()[0]) + 1  # the first step that is not slice 0's
+    slices = -(-steps // length)
+    assert slices > 1 and length == -(-steps // slices), (length, slices)
+    lost = {j for j in range(1, width + 1) if j < length or (j + 1) % length == 0}
+    assert set((kept == 0).nonzero().flatten().add(1).tolist()) == lost
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("rows,fin,fout", [
     (1, 64, 64), (31, 64, 32), (33, 40, 72), (300, 256, 100),   # tiles of 32 and 64, one and more per gradient, ragged edges
