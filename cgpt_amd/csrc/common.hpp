@@ -176,7 +176,9 @@ int rmsnorm_backward_residual(void* grad_input, void* grad_weight, const void* g
 
 // Per-head RMSNorm and rotary embedding of q and k in one pass over their [rows = tokens x heads, head_dim]:
 //   forward   output = rope(rmsnorm(input));   backward   output = the gradient of that, with the weight gradient.
-// Bit for bit what the separate operators give (their intermediate roundings are kept). Positions are
+// Bit for bit what the separate operators give (their intermediate roundings are kept); only the weight gradients of more rows
+// than the chip holds at once in 16-bit storage, where the separate norm fits more workgroups on it, add fp32 sums in another order.
+// Positions are
 // position_offset + token % sequence, token = row / heads. `rmsnorm_rope_fusable` says whether the shape,
 // dtype and alignment are served; callers run the separate operators otherwise.
 struct NormRopeTensors {

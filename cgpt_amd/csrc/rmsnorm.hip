@@ -608,7 +608,7 @@ FastShape pick_fast_shape(int hidden) {
     return {};
 }
 
-// Whether rmsnorm_rope_dense_kernel serves the pass: rows of exactly 16 vectors, all of them rotated, whole groups of
+// Whether rmsnorm_rope_dense serves the pass: rows of exactly 16 vectors, all of them rotated, whole groups of
 // four rows, and every byte offset it forms (tensor and table) below 2^32.
 template <typename T>
 bool rope_dense(int rows, int hidden, const RopeArgs& rope) {
@@ -754,19 +754,21 @@ namespace {
 // Workgroups that rows of 16 vectors fill, four rows a wavefront.
 int pair_blocks(int rows) { return static_cast<int>((static_cast<long>(rows) + 4 * kWavesPerBlock - 1) / (4 * kWavesPerBlock)); }
 
-// The pair kernel's form for these rows, and how many workgroups each of the two takes: in the ratio of their rows where the chip
-// does not hold one per group of rows.
+// The pair kernel's form for these rows, and how many workgroups each of the two takes: as many as in a launch of its own, up to
+// what the chip holds, since each leaves one partial sum of the weight gradient and their number is the order of its additions.
+// More than the chip holds together, k's start as q's end; shared out in the ratio of their rows instead, all resident at once, the
+// launches took longer: backward of 32768 tokens, 8:2 heads of 128, 45.6 us and 42.5 so, forward 31.9 and 29.5; 12:4 heads of 64,
+// 50.4 and 45.7, 38.9 and 35.0.
 template <typename T, bool Backward>
 struct PairPlan {
     bool dense;
     int blocks_q, blocks_k;
     PairPlan(int rows_q, int rows_k, int head_dim, RopeArgs rope) : dense(rope_dense<T>(std::max(rows_q, rows_k), head_dim, rope) &&
                                                                           rows_q % 4 == 0 && rows_k % 4 == 0) {
-        const long q = pair_blocks(rows_q), k = pair_blocks(rows_k);
-        const long cap = resident_blocks(dense ? reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, true>)
-                                               : reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, false>));
-        blocks_q = static_cast<int>(q + k <= cap ? q : std::max(1L, std::min(cap - 1, cap * q / (q + k))));
-        blocks_k = static_cast<int>(q + k <= cap ? k : std::min(k, cap - blocks_q));
+        const int cap = resident_blocks(dense ? reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, true>)
+                                              : reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, false>));
+        blocks_q = std::min(pair_blocks(rows_q), cap);
+        blocks_k = std::min(pair_blocks(rows_k), cap);
     }
 };
 template <typename T, bool Backward>
@@ -1021,7 +1023,7 @@ std::size_t rmsnorm_backward_sink_bytes(NormPass pass, std::size_t rows, std::si
             // for whichever of them takes more. q's and k's last workgroups may both be partly filled.
             for (const void* kernel : {reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, true, false>),
                                        reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, true, true>)})
-                blocks = std::max(blocks, std::min(pair_blocks(r) + 1, resident_blocks(kernel)));
+                blocks = std::max(blocks, std::min(pair_blocks(r) + 1, 2 * resident_blocks(kernel)));
         } else {
             const void* kernel = pass == NormPass::dual ? dual_kernel<T, true>(shape) : fast_kernel<T, true>(shape);
             if (kernel == nullptr) return CGPTX_OK;

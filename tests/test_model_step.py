@@ -380,9 +380,10 @@ def test_fused_qk_norm_rope_is_bit_identical_to_the_separate_operators(device, m
 @pytest.mark.gpu
 @pytest.mark.parametrize("head_dim,kv_heads", [(128, 3), (64, 1), (128, 6)], ids=["ragged-split", "general", "equal"])
 def test_fused_qk_norm_rope_of_more_rows_than_the_chip_holds(device, monkeypatch, head_dim, kv_heads):
-    """q and k share the workgroups of one launch in the ratio of their rows once they are more than the chip holds. All but the
-    order of additions in the two norms' weight gradients is that of the separate operators: fp32 sums over up to 72000 rows, one
-    rounding to bf16 (2^-9), beside sums of rounded terms whose error grows with the gradient's largest element."""
+    """More rows than the chip holds at once: the separate norm, which fits more workgroups on it than the fused pass, groups the
+    additions of the two norms' weight gradients otherwise. All else is that of the separate operators, bit for bit; those are fp32
+    sums over up to 72000 rows, one rounding to bf16 (2^-9), beside sums of rounded terms whose error grows with the gradient's
+    largest element."""
     from cgpt_amd.model import LOSS_DENSE, Model, ModelConfig
     config = ModelConfig(vocabulary_size=64, num_layers=1, hidden_size=6 * head_dim, intermediate_size=64, num_query_heads=6,
                          num_kv_heads=kv_heads, head_dim=head_dim, rotary_dim=head_dim, dtype=torch.bfloat16)
@@ -403,6 +404,29 @@ def test_fused_qk_norm_rope_of_more_rows_than_the_chip_holds(device, monkeypatch
             assert (a - b).abs().max() <= 2.0 ** -8 * b.abs().max()
         else:
             assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_heads,rotary_dim", [(3, 64), (1, 64), (6, 32)], ids=["dense", "few-k-rows", "partly-rotated"])
+def test_fused_qk_norm_rope_in_fp32_adds_as_the_separate_operators_do(device, monkeypatch, kv_heads, rotary_dim):
+    """More rows than the chip holds at once, in fp32 storage, where no rounding hides another order of additions: q's and k's
+    workgroups leave the partial sums of the weight gradients that launches of their own leave, so all gradients are
+    bit-identical. (In 16-bit storage the separate norm fits more workgroups on a compute unit than the fused one.)"""
+    from cgpt_amd.model import LOSS_DENSE, Model, ModelConfig
+    config = ModelConfig(vocabulary_size=64, num_layers=1, hidden_size=6 * 64, intermediate_size=64, num_query_heads=6,
+                         num_kv_heads=kv_heads, head_dim=64, rotary_dim=rotary_dim, dtype=torch.float32)
+    batch, seq = 60, 200
+    rng = np.random.default_rng(3)
+    inputs, targets = (rng.integers(0, 64, size=batch * seq).astype(np.uint32) for _ in range(2))
+    results = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("CGPTX_FUSE_QK", fuse)
+        model = Model(config, batch, seq, seed=4, device=device)
+        model.set_tokens(inputs, targets)
+        model.forward_backward(loss_scale=4.0, loss_mode=LOSS_DENSE)
+        results.append([(name, g.clone()) for name, _, g in model.parameters()])
+    for (name, a), (_, b) in zip(*results):
+        assert torch.equal(a, b), name
 
 
 @pytest.mark.gpu
