@@ -745,7 +745,7 @@ int run_column_reductions(const ColumnReduceEntry* table, const std::vector<Colu
     int groups = 1;
     for (const ColumnReduceEntry& e : entries) groups = std::max(groups, (e.hidden + finish_columns(e.hidden) - 1) / finish_columns(e.hidden));
     hipLaunchKernelGGL(column_partial_reduce_table_kernel, dim3(groups, static_cast<unsigned int>(entries.size())), dim3(kFinishThreads),
-                       0, stream, table);
+                       0, stream, table, compute_units());
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
 }

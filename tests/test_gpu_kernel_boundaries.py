@@ -112,6 +112,56 @@ def test_weight_gradients_are_cut_into_equal_k_slices(device, steps, dtype):
     assert set((kept == 0).nonzero().flatten().add(1).tolist()) == lost
 
 
+def column_sums_in_order(parts, hidden, units):
+    """parts [P, H] in float32, added over P in the order that the column reductions promise."""
+    count = len(parts)
+    slices = max(1, min(2 * units // -(-hidden // 64), count // 16, 4096 // (16 if hidden <= 256 else 32)))
+    if slices > 1:
+        chunk = -(-count // slices)
+        folded = np.zeros((slices, hidden), np.float32)
+        for i in range(slices):
+            own = parts[i * chunk:(i + 1) * chunk]
+            eighths = np.zeros((8, hidden), np.float32)
+            for p, row in enumerate(own):
+                eighths[p % 8] += row
+            for w in range(4):
+                folded[i] += eighths[w] + eighths[w + 4]
+        parts, count = folded, slices
+    total = np.zeros(hidden, np.float32)
+    for w in range(4):
+        running = np.zeros((4, hidden), np.float32)
+        p = w
+        while p + 12 < count:
+            for u in range(4):
+                running[u] += parts[p + 4 * u]
+            p += 16
+        for q in range(p, count, 4):
+            running[0] += parts[q]
+        total += (running[0] + running[1]) + (running[2] + running[3])
+    return total
+
+
+@pytest.mark.parametrize("rows,width", [
+    *((rows, width) for rows in (300, 4096, 65536) for width in (1, 16, 20, 256, 300, 1024)),  # 60, 64, 256 parts; 16 or 32 columns
+    (4096, 9000), (4096, 16448),                                                               # few slices, one slice
+])
+def test_column_sums_add_in_their_order(device, rows, width):
+    """A bias's gradient in fp32 whose parts are one row each, so that the order of additions is all there is to it: that order
+    is part of what the norms' weight gradients promise a training step."""
+    parts = 64 if rows < 65536 else 256
+    per_part = -(-rows // parts)
+    values = (torch.randn(parts, width, generator=torch.Generator().manual_seed(width)) * 3).float()
+    values[-(-rows // per_part):] = 0
+    dy = torch.zeros(rows, width, device=device)
+    dy[torch.arange(0, rows, per_part, device=device)] = values[:-(-rows // per_part)].to(device)
+    x = torch.zeros(rows, 4, device=device)
+    db = torch.full((width,), float("nan"), device=device)
+    ops.linear_backward(None, None, db, dy, x, torch.zeros(width, 4, device=device))
+    units = torch.cuda.get_device_properties(device).multi_processor_count
+    want = column_sums_in_order(values.numpy(), width, units)
+    assert np.array_equal(db.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("rows,fin,fout", [
