@@ -230,9 +230,10 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
         }
     }
     if (grad_input != nullptr && grad_weight != nullptr) {
-        // Small calls: both gradients, and the bias's, in one launch, whose parts run in no order. None may write what
-        // another one reads.
+        // Small calls: both gradients, and the bias's, in one launch, whose parts run in no order. None may write what another
+        // one reads, nor what another one writes: overlapping results hold what the last of the separate launches leaves.
         const std::size_t dy_bytes = rows * out_features * elem, x_bytes = rows * in_features * elem, w_bytes = out_features * in_features * elem;
+        const std::size_t bias_bytes = out_features * elem;
         auto apart = [](const void* a, std::size_t a_bytes, const void* b, std::size_t b_bytes) {
             const auto x = reinterpret_cast<std::uintptr_t>(a), y = reinterpret_cast<std::uintptr_t>(b);
             return a == nullptr || x >= y + b_bytes || y >= x + a_bytes;
@@ -242,8 +243,9 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
         calls[1].a_sums_accumulate = accumulate_bias != 0;
         if (apart(grad_input, x_bytes, grad_output, dy_bytes) && apart(grad_input, x_bytes, input, x_bytes) &&
             apart(grad_weight, w_bytes, grad_output, dy_bytes) && apart(grad_weight, w_bytes, weight, w_bytes) &&
-            apart(grad_bias, out_features * elem, grad_output, dy_bytes) && apart(grad_bias, out_features * elem, weight, w_bytes) &&
-            apart(grad_bias, out_features * elem, input, x_bytes) && gemm_joins(calls, 2))
+            apart(grad_bias, bias_bytes, grad_output, dy_bytes) && apart(grad_bias, bias_bytes, weight, w_bytes) &&
+            apart(grad_bias, bias_bytes, input, x_bytes) && apart(grad_weight, w_bytes, grad_input, x_bytes) &&
+            apart(grad_bias, bias_bytes, grad_input, x_bytes) && apart(grad_bias, bias_bytes, grad_weight, w_bytes) && gemm_joins(calls, 2))
             return gemm_joined(calls, 2, stream);
     }
     if (grad_input != nullptr)

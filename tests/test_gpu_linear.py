@@ -7,7 +7,7 @@ import torch
 
 from cgpt_amd import ops
 from oracle import cpu_ops, oracle64
-from tests.util import DTYPES, DTYPE_IDS, TOL, assert_close, randn, to_np
+from tests.util import DTYPES, DTYPE_IDS, TOL, assert_close, launches, randn, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -366,3 +366,34 @@ def test_linear_ragged_shapes_integer_valued_inputs_are_exact(device, rows, fin,
     ops.linear_backward(gi, gw, gb, on(dy), on(x), on(w), options=options)
     for name, got, exact in zip(("Y", "dX", "dW", "db"), (y, gi, gw, gb), want):
         assert torch.equal(got.cpu(), exact.to(dtype)), name
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("behind,before", [("db", "dW"), ("dW", "dX"), ("db", "dX")])
+def test_overlapping_gradients_are_written_one_after_the_other(device, behind, before, dtype):
+    """Gradients that share memory hold what the last of dX, dW, db leaves. Small calls run all three in one launch, whose
+    workgroups are in no order: not these."""
+    rows, fin, fout = 128, 256, 192
+    g = torch.Generator().manual_seed(rows)
+    x, w, dy = (torch.randint(-2, 3, shape, generator=g).to(dtype).to(device) for shape in ((rows, fin), (fout, fin), (rows, fout)))
+    shapes = {"dX": (rows, fin), "dW": (fout, fin), "db": (fout,)}
+    # `behind` begins within the last sixteen elements of `before`.
+    size = {name: int(np.prod(shape)) for name, shape in shapes.items()}
+    shared = torch.zeros(size[before] + size[behind], dtype=dtype, device=device)
+    place = {name: torch.zeros(shape, dtype=dtype, device=device) for name, shape in shapes.items()}
+    place[before] = shared[:size[before]].view(shapes[before])
+    place[behind] = shared[size[before] - 16:][:size[behind]].view(shapes[behind])
+
+    def at_once(to):
+        ops.linear_backward(to["dX"], to["dW"], to["db"], dy, x, w)
+
+    assert launches(lambda: at_once(place)) > 1
+    shared.zero_()
+    at_once(place)
+    got = shared.clone()
+    shared.zero_()
+    for name in ("dX", "dW", "db"):
+        ops.linear_backward(*(place[n] if n == name else None for n in ("dX", "dW", "db")), dy, x, w)
+    assert torch.equal(got, shared)
+    apart = {name: torch.zeros(shape, dtype=dtype, device=device) for name, shape in shapes.items()}
+    assert launches(lambda: at_once(apart)) == 1

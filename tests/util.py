@@ -1,8 +1,12 @@
 """Shared helpers for the parity tests: seeded inputs, tolerances, comparisons."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
+
+from cgpt_amd import capi
 
 # Tolerances of the parity bar: max |a-b| / max(1, |b|).
 TOL = {torch.float32: 1e-4, torch.float16: 2e-2, torch.bfloat16: 2e-2}
@@ -70,3 +74,19 @@ def bits(t: torch.Tensor) -> np.ndarray:
     if t.dtype == torch.float32:
         return t.view(torch.int32).numpy()
     return t.view(torch.int16).numpy()
+
+
+def launches(call) -> int:
+    """Kernels that `call` enqueues: the nodes of a graph that it is recorded into and that is never run. Called once before,
+    so that its scratch memory is there."""
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        call()
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        call()
+    count = ctypes.c_size_t()
+    assert capi.lib().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
