@@ -667,22 +667,21 @@ int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream, bo
     return run_typed<T>(padded, stream);
 }
 
+constexpr double kGroupBlocksPerUnit = 16.0;  // of a group, at most
+
 // A group's tiles: those whose predicted time in one launch is least. The launch takes as long as its longest workgroup or
 // as the busiest CU's share of the work, whatever is more (us per K tile and workgroup as in predicted_us; 3.5 us before and
 // after the K loops). Two workgroups share a CU and its LDS, or, deep, each has one to itself: then the longest is not held
 // up by another, but 3.5 us of start and end of every workgroup are in nobody's shadow. Joined if that is less than the calls'
 // own predictions in turn. [M, N] x K measured apart and joined: dX and dW of 128 x 768 x 768 10.4 -> 7.4 us, of 2000 x 1024 x
 // 2048 35.7 -> 32.3; 5005 x 1024 x 256, whose dW is better split along K, 23.7 -> 28.8: stays apart.
-struct GroupPlan {
-    int tile[kGroupCalls] = {};
-    long blocks = 0;
-    bool deep = false;
-    bool joined = false;
-};
-
-GroupPlan plan_group(const GemmArgs* calls, int count) {
-    GroupPlan best_plan;
+GemmGroup plan_group(const GemmArgs* calls, int count) {
+    GemmGroup best_plan;
     const double units = static_cast<double>(compute_units());
+    // Large calls are told apart by their tiles alone: whatever is spent here, they pay beside their own plans.
+    double fewest = 0.0;
+    for (int i = 0; i < count; ++i) fewest += static_cast<double>((calls[i].m + 63) / 64) * static_cast<double>((calls[i].n + 63) / 64);
+    if (fewest > kGroupBlocksPerUnit * units) return best_plan;
     double separate = 0.0;
     for (int i = 0; i < count; ++i) {
         const GemmArgs& g = calls[i];
@@ -711,14 +710,13 @@ GroupPlan plan_group(const GemmArgs* calls, int count) {
             lone_work += tiles * (loop + 3.5);
             blocks += tiles;
         }
-        if (blocks > 16.0 * units) continue;
+        if (blocks > kGroupBlocksPerUnit * units) continue;
         const double load = blocks / units;
         const double two = load <= 1.0 ? longest : std::max(1.4 * longest, work / units * std::ceil(load) / load * (load > 4.0 ? 1.3 : 1.0));
         const double one = load <= 1.0 ? longest : std::max(longest, lone_work / units * std::ceil(load) / load);
         if (3.5 + std::min(one, two) < best) {
             best = 3.5 + std::min(one, two);
             best_plan.joined = true;
-            best_plan.blocks = static_cast<long>(blocks);
             best_plan.deep = one <= two;
             for (int i = 0; i < count; ++i) best_plan.tile[i] = ((choice >> i) & 1) != 0 ? 32 : 64;
         }
@@ -758,7 +756,7 @@ bool joinable(const GemmArgs& g, KernelArgs& p) {
 }
 
 template <typename T>
-int run_joined(const GemmArgs* calls, int count, const GroupPlan& plan, hipStream_t stream) {
+int run_joined(const GemmArgs* calls, int count, const GemmGroup& plan, hipStream_t stream) {
     SmallGroup group{};
     long order[kGroupCalls];
     for (int i = 0; i < count; ++i) order[i] = i;
@@ -789,22 +787,21 @@ int run_joined(const GemmArgs* calls, int count, const GroupPlan& plan, hipStrea
 
 }  // namespace
 
-bool gemm_joins(const GemmArgs* calls, int count) {
-    if (count < 2 || count > kGroupCalls || forced_tile() != 0) return false;
+GemmGroup gemm_joins(const GemmArgs* calls, int count) {
+    if (count < 2 || count > kGroupCalls || forced_tile() != 0) return {};
     for (int i = 0; i < count; ++i) {
-        if (calls[i].dtype != calls[0].dtype || !valid_dtype(calls[i].dtype)) return false;
+        if (calls[i].dtype != calls[0].dtype || !valid_dtype(calls[i].dtype)) return {};
         KernelArgs p;
         const bool fits = calls[i].dtype == CGPTX_F32 ? joinable<float>(calls[i], p)
                           : calls[i].dtype == CGPTX_F16 ? joinable<f16_t>(calls[i], p) : joinable<bf16_t>(calls[i], p);
-        if (!fits) return false;
+        if (!fits) return {};
     }
-    return plan_group(calls, count).joined;
+    return plan_group(calls, count);
 }
 
-int gemm_joined(const GemmArgs* calls, int count, hipStream_t stream) {
-    if (!gemm_joins(calls, count)) return fail(CGPTX_RUNTIME, "gemm: these calls cannot share a launch");
-    const GroupPlan plan = plan_group(calls, count);
-    return dispatch_dtype(calls[0].dtype, [&]<typename T>() -> int { return run_joined<T>(calls, count, plan, stream); });
+int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream) {
+    if (!group.joined || count < 2 || count > kGroupCalls) return fail(CGPTX_RUNTIME, "gemm: these calls cannot share a launch");
+    return dispatch_dtype(calls[0].dtype, [&]<typename T>() -> int { return run_joined<T>(calls, count, group, stream); });
 }
 
 bool gemm_fuses_swiglu(const GemmArgs& g) {

@@ -81,10 +81,15 @@ struct GemmArgs {
 
 int gemm(const GemmArgs& args, hipStream_t stream);
 // Up to four calls that neither read nor write each other's results, in one launch: whether that is served and faster than
-// one after the other (few tiles each, operands that stream as they lie), and the launch itself.
+// one after the other (few tiles each, operands that stream as they lie) and how their tiles are cut then, and the launch itself.
 constexpr int kGroupCalls = 4;
-bool gemm_joins(const GemmArgs* calls, int count);
-int gemm_joined(const GemmArgs* calls, int count, hipStream_t stream);
+struct GemmGroup {
+    int tile[kGroupCalls] = {};
+    bool deep = false;  // one workgroup per CU
+    bool joined = false;
+};
+GemmGroup gemm_joins(const GemmArgs* calls, int count);
+int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream);
 // Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
 std::size_t gemm_split_bytes(const GemmArgs& args);
 // Copies [rows, cols] elements (row stride ld) to rows of `pitch` elements (whole 16-byte chunks), zeros past cols.

@@ -245,8 +245,9 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
             apart(grad_weight, w_bytes, grad_output, dy_bytes) && apart(grad_weight, w_bytes, weight, w_bytes) &&
             apart(grad_bias, bias_bytes, grad_output, dy_bytes) && apart(grad_bias, bias_bytes, weight, w_bytes) &&
             apart(grad_bias, bias_bytes, input, x_bytes) && apart(grad_weight, w_bytes, grad_input, x_bytes) &&
-            apart(grad_bias, bias_bytes, grad_input, x_bytes) && apart(grad_bias, bias_bytes, grad_weight, w_bytes) && gemm_joins(calls, 2))
-            return gemm_joined(calls, 2, stream);
+            apart(grad_bias, bias_bytes, grad_input, x_bytes) && apart(grad_bias, bias_bytes, grad_weight, w_bytes)) {
+            if (const GemmGroup group = gemm_joins(calls, 2); group.joined) return gemm_joined(calls, 2, group, stream);
+        }
     }
     if (grad_input != nullptr)
         if (int s = gemm(input_gradient(), stream)) return s;

@@ -720,13 +720,14 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         } else {
             CGPTX_OP("rmsnorm_fwd", cgptx_rmsnorm_forward(a.norm_a, x, w.attention_norm.value, N, H, eps, dt, s));
         }
+        const GemmArgs qkv_parts[3] = {projection(a.q_pre, a.norm_a, w.q.value, N, H, QW, dt),
+                                       projection(a.k_pre, a.norm_a, w.k.value, N, H, KW, dt),
+                                       projection(a.v, a.norm_a, w.v.value, N, H, KW, dt)};
+        const GemmGroup qkv_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_parts, 3);
         if (fused_qkv) {
             CGPTX_OP("gemm_fwd.qkv", qkv_forward(a.q_pre, a.k_pre, a.v, a.norm_a, w.q.value, N, H, QW, KW, dt, stream));
-        } else if (const GemmArgs qkv[3] = {projection(a.q_pre, a.norm_a, w.q.value, N, H, QW, dt),
-                                            projection(a.k_pre, a.norm_a, w.k.value, N, H, KW, dt),
-                                            projection(a.v, a.norm_a, w.v.value, N, H, KW, dt)};
-                   gemm_joins(qkv, 3)) {
-            CGPTX_OP("gemm_fwd.qkv", gemm_joined(qkv, 3, stream));
+        } else if (qkv_group.joined) {
+            CGPTX_OP("gemm_fwd.qkv", gemm_joined(qkv_parts, 3, qkv_group, stream));
         } else {
             CGPTX_OP("gemm_fwd.qkv", cgptx_linear_forward(a.q_pre, a.norm_a, w.q.value, nullptr, N, H, QW, dt, s));
             CGPTX_OP("gemm_fwd.qkv", cgptx_linear_forward(a.k_pre, a.norm_a, w.k.value, nullptr, N, H, KW, dt, s));
@@ -828,16 +829,17 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             CGPTX_OP("rmsnorm_bwd", rmsnorm_backward_residual(d_k, w.k_norm.gradient, m->d_k_pre, a.k_pre, w.k_norm.value, nullptr,
                                                               N * HKV, D, eps, dt, stream, sink));
         }
+        const GemmArgs qkv_gradients[4] = {qkv_input_gradient(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt),
+                                           projection_weight_gradient(w.q.gradient, d_q, a.norm_a, N, H, QW, dt),
+                                           projection_weight_gradient(w.k.gradient, d_k, a.norm_a, N, H, KW, dt),
+                                           projection_weight_gradient(w.v.gradient, d_v, a.norm_a, N, H, KW, dt)};
+        const GemmGroup gradient_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_gradients, 4);
         if (fused_qkv) {
-            CGPTX_OP("gemm_dx.qkv", gemm(qkv_input_gradient(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt), stream));
+            CGPTX_OP("gemm_dx.qkv", gemm(qkv_gradients[0], stream));
             if (!stacked)
                 CGPTX_OP("gemm_dw.qkv", qkv_backward_weight(w.q.gradient, d_q, d_k, d_v, a.norm_a, N, H, QW, KW, dt, stream));
-        } else if (const GemmArgs qkv[4] = {qkv_input_gradient(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt),
-                                            projection_weight_gradient(w.q.gradient, d_q, a.norm_a, N, H, QW, dt),
-                                            projection_weight_gradient(w.k.gradient, d_k, a.norm_a, N, H, KW, dt),
-                                            projection_weight_gradient(w.v.gradient, d_v, a.norm_a, N, H, KW, dt)};
-                   gemm_joins(qkv, 4)) {
-            CGPTX_OP("gemm_dx.qkv", gemm_joined(qkv, 4, stream));
+        } else if (gradient_group.joined) {
+            CGPTX_OP("gemm_dx.qkv", gemm_joined(qkv_gradients, 4, gradient_group, stream));
         } else {
             CGPTX_TRY(linear_backward_split(m, m->d_norm_in, w.q.gradient, d_q, a.norm_a, w.q.value, N, H, QW, 0, dt, stream, "gemm_dx.qkv", "gemm_dw.qkv"));
             CGPTX_TRY(linear_backward_split(m, m->d_norm_in, w.k.gradient, d_k, a.norm_a, w.k.value, N, H, KW, 1, dt, stream, "gemm_dx.qkv", "gemm_dw.qkv"));
