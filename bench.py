@@ -531,9 +531,12 @@ def main() -> int:
     for label, ms in labelled.items():
         kind = label.split(".")[0]
         breakdown[kind] = breakdown.get(kind, 0.0) + ms
-    # The probe's launch inside the step: one per layer in the event-timed eager pass.
-    in_step_seconds = labelled["gemm_dx.gate_up"] * 1e-3 / cfg.num_layers
+    # The probe's launch inside the step: one per layer in the event-timed eager pass (small batches share it with the weight's).
+    in_step_seconds = labelled["gemm_dx.gate_up"] * 1e-3 / cfg.num_layers if "gemm_dx.gate_up" in labelled else probe["seconds"]
     work = op_work(cfg, args.batch, args.seq, args.loss)
+    if "gemm_dx_dw" in breakdown:
+        work["gemm_dx_dw"] = (work["gemm_dx"][0], work["gemm_dx"][1] + work["gemm_dw"][1])
+        breakdown["gemm_dx_dw"] = sum(breakdown.pop(kind, 0.0) for kind in ("gemm_dx", "gemm_dw", "gemm_dx_dw"))
     # When the per-head norms carry the rotary embedding (one pass), its algorithmic bytes count with theirs.
     for rope, norm in (("rope_fwd", "rmsnorm_fwd"), ("rope_bwd", "rmsnorm_bwd")):
         if rope not in breakdown:

@@ -174,6 +174,17 @@ int rmsnorm_backward_residual(void* grad_input, void* grad_weight, const void* g
                               const void* weight, const void* residual, std::size_t rows, std::size_t hidden,
                               float epsilon, int dtype, hipStream_t stream, ColumnReduceSink* sink = nullptr);
 
+// cgptx_linear_backward that says when it has enqueued each contraction: for a caller that times them.
+struct LinearParts {
+    enum Part { input, weight, joined };
+    virtual int done(Part part) = 0;
+    virtual ~LinearParts() = default;
+};
+int linear_backward(void* grad_input, void* grad_weight, void* grad_bias, const void* grad_output, const void* input,
+                    const void* weight, std::size_t rows, std::size_t in_features, std::size_t out_features,
+                    int accumulate_input, int accumulate_weight, int accumulate_bias, int dtype, hipStream_t stream,
+                    LinearParts* parts);
+
 // Per-head RMSNorm and rotary embedding of q and k in one pass over their [rows = tokens x heads, head_dim]:
 //   forward   output = rope(rmsnorm(input));   backward   output = the gradient of that, with the weight gradient.
 // Bit for bit what the separate operators give (their intermediate roundings are kept); only the weight gradients of more rows

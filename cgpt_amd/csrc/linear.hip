@@ -156,12 +156,18 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
                                      const void* input, const void* weight, size_t rows, size_t in_features,
                                      size_t out_features, int accumulate_input, int accumulate_weight,
                                      int accumulate_bias, int dtype, cgptx_stream stream_) {
-    using namespace cgptx;
+    return cgptx::linear_backward(grad_input, grad_weight, grad_bias, grad_output, input, weight, rows, in_features, out_features,
+                                  accumulate_input, accumulate_weight, accumulate_bias, dtype, static_cast<hipStream_t>(stream_), nullptr);
+}
+
+int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias, const void* grad_output, const void* input,
+                           const void* weight, std::size_t rows, std::size_t in_features, std::size_t out_features,
+                           int accumulate_input, int accumulate_weight, int accumulate_bias, int dtype, hipStream_t stream,
+                           LinearParts* parts) {
     if (int s = validate("linear_backward", rows, in_features, out_features, dtype)) return s;
     if (grad_output == nullptr || (grad_input != nullptr && weight == nullptr) ||
         (grad_weight != nullptr && input == nullptr))
         return fail(CGPTX_INVALID_ARGUMENT, "linear_backward: null tensor");
-    auto stream = static_cast<hipStream_t>(stream_);
     // An output gradient whose rows are not whole 16-byte chunks feeds both contractions from one padded copy (each would
     // make its own otherwise).
     const std::size_t elem = dtype_size(dtype);
@@ -246,13 +252,22 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
             apart(grad_bias, bias_bytes, grad_output, dy_bytes) && apart(grad_bias, bias_bytes, weight, w_bytes) &&
             apart(grad_bias, bias_bytes, input, x_bytes) && apart(grad_weight, w_bytes, grad_input, x_bytes) &&
             apart(grad_bias, bias_bytes, grad_input, x_bytes) && apart(grad_bias, bias_bytes, grad_weight, w_bytes)) {
-            if (const GemmGroup group = gemm_joins(calls, 2); group.joined) return gemm_joined(calls, 2, group, stream);
+            if (const GemmGroup group = gemm_joins(calls, 2); group.joined) {
+                if (int s = gemm_joined(calls, 2, group, stream)) return s;
+                return parts != nullptr ? parts->done(LinearParts::joined) : CGPTX_OK;
+            }
         }
     }
-    if (grad_input != nullptr)
+    if (grad_input != nullptr) {
         if (int s = gemm(input_gradient(), stream)) return s;
-    if (grad_weight != nullptr)
+        if (parts != nullptr)
+            if (int s = parts->done(LinearParts::input)) return s;
+    }
+    if (grad_weight != nullptr) {
         if (int s = gemm(weight_gradient(), stream)) return s;
+        if (parts != nullptr)
+            if (int s = parts->done(LinearParts::weight)) return s;
+    }
     if (grad_bias != nullptr) {  // db[out] = Σ_rows dY
         const int cols = static_cast<int>(out_features);
         const int slices = rows < 256 ? 1 : (rows < 65536 ? 64 : 256);

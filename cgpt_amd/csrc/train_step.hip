@@ -265,20 +265,46 @@ void collect(cgptx_model* m, std::vector<Parameter*>& out) {
         }                                                                       \
     } while (0)
 
-// linear_backward as two single-kernel calls so that each can be timed on its own.
-int linear_backward_split(cgptx_model* m, void* dx, void* dw, const void* dy, const void* x, const void* w,
-                          std::size_t rows, std::size_t in_features, std::size_t out_features, int accumulate_input,
-                          int dt, hipStream_t stream, const char* dx_label, const char* dw_label) {
-    auto* s = static_cast<cgptx_stream>(stream);
-    // In one call, which may run both in one launch, unless each is to be timed.
-    if (!m->profiling)
-        return cgptx_linear_backward(dx, dw, nullptr, dy, x, w, rows, in_features, out_features, accumulate_input, 0, 0, dt, s);
-    CGPTX_OP(dx_label, cgptx_linear_backward(dx, nullptr, nullptr, dy, x, w, rows, in_features, out_features,
-                                              accumulate_input, 0, 0, dt, s));
-    if (dw != nullptr)
-        CGPTX_OP(dw_label, cgptx_linear_backward(nullptr, dw, nullptr, dy, x, w, rows, in_features, out_features, 0, 0,
-                                                 0, dt, s));
-    return CGPTX_OK;
+// The two gradients of a projection. When profiling, each launch is timed under its label: input, weight, or both in one.
+struct TimedParts final : LinearParts {
+    cgptx_model* m;
+    hipStream_t stream;
+    const char* const (&labels)[3];
+    cgptx_model::Timed open{};
+    TimedParts(cgptx_model* model, hipStream_t on, const char* const (&names)[3]) : m(model), stream(on), labels(names) {}
+    int start() {
+        CGPTX_HIP(hipEventCreate(&open.start));
+        CGPTX_HIP(hipEventCreate(&open.stop));
+        CGPTX_HIP(hipEventRecord(open.start, stream));
+        return CGPTX_OK;
+    }
+    int done(Part part) override {
+        CGPTX_HIP(hipEventRecord(open.stop, stream));
+        open.label = labels[part];
+        m->timed.push_back(open);
+        open = {};
+        return part == input ? start() : CGPTX_OK;
+    }
+    ~TimedParts() override {  // nothing followed the last start
+        if (open.start != nullptr) (void)hipEventDestroy(open.start);
+        if (open.stop != nullptr) (void)hipEventDestroy(open.stop);
+    }
+};
+#define CGPTX_GRADIENT_LABELS(projection) {"gemm_dx." projection, "gemm_dw." projection, "gemm_dx_dw." projection}
+constexpr const char* kQkvLabels[3] = CGPTX_GRADIENT_LABELS("qkv");
+constexpr const char* kOutputLabels[3] = CGPTX_GRADIENT_LABELS("o");
+constexpr const char* kGateUpLabels[3] = CGPTX_GRADIENT_LABELS("gate_up");
+constexpr const char* kDownLabels[3] = CGPTX_GRADIENT_LABELS("down");
+constexpr const char* kClassifierLabels[3] = CGPTX_GRADIENT_LABELS("classifier");
+#undef CGPTX_GRADIENT_LABELS
+
+int linear_gradients(cgptx_model* m, void* dx, void* dw, const void* dy, const void* x, const void* w, std::size_t rows,
+                     std::size_t in_features, std::size_t out_features, int accumulate_input, int dt, hipStream_t stream,
+                     const char* const (&labels)[3]) {
+    TimedParts timed(m, stream, labels);
+    if (m->profiling) CGPTX_TRY(timed.start());
+    return linear_backward(dx, dw, nullptr, dy, x, w, rows, in_features, out_features, accumulate_input, 0, 0, dt, stream,
+                           m->profiling ? &timed : nullptr);
 }
 
 // Y = X·Wᵀ + residual (accumulate: + Y): the block's residual additions ride in the projection's
@@ -600,10 +626,10 @@ int enqueue_reference_sequence(cgptx_model* m, float loss_scale, int loss_mode, 
         CGPTX_OP(label, cgptx_linear_forward(out, in, w, nullptr, N, in_features, out_features, dt, s));
         return CGPTX_OK;
     };
-    auto project_bwd = [&](const char* dx_label, const char* dw_label, void* dx, void* dw, const void* dy, const void* x, const void* w,
+    auto project_bwd = [&](const char* const (&labels)[3], void* dx, void* dw, const void* dy, const void* x, const void* w,
                            std::size_t in_features, std::size_t out_features, int accumulate_input) -> int {
         note_call(m, "linear_backward", {dx, dw, dy, x, w}, {N, in_features, out_features}, {accumulate_input});
-        return linear_backward_split(m, dx, dw, dy, x, w, N, in_features, out_features, accumulate_input, dt, stream, dx_label, dw_label);
+        return linear_gradients(m, dx, dw, dy, x, w, N, in_features, out_features, accumulate_input, dt, stream, labels);
     };
     auto add = [&](void* out, const void* a, const void* b) -> int {
         note_call(m, "add", {out, a, b}, {N * H});
@@ -650,7 +676,7 @@ int enqueue_reference_sequence(cgptx_model* m, float loss_scale, int loss_mode, 
         CGPTX_TRY(project("gemm_fwd.classifier", m->logits, m->normalized, m->embedding.value, H, V));
         note_call(m, "cross_entropy_forward_backward", {m->loss, m->grad_logits, m->logits, m->targets}, {N, V}, {}, loss_scale);
         CGPTX_OP("dense_ce", cgptx_cross_entropy_forward_backward(m->loss, m->grad_logits, m->logits, m->targets, N, V, loss_scale, dt, s));
-        CGPTX_TRY(project_bwd("gemm_dx.classifier", "gemm_dw.classifier", m->d_normalized, m->embedding.gradient, m->grad_logits,
+        CGPTX_TRY(project_bwd(kClassifierLabels, m->d_normalized, m->embedding.gradient, m->grad_logits,
                               m->normalized, m->embedding.value, H, V, 0));
     }
 
@@ -663,14 +689,14 @@ int enqueue_reference_sequence(cgptx_model* m, float loss_scale, int loss_mode, 
         void *gate = a.gate_up, *up = second_half(a.gate_up);
         void *d_gate = m->d_gate_up, *d_up = second_half(m->d_gate_up);
         void* grad_residual = m->d_norm_in_f;
-        CGPTX_TRY(project_bwd("gemm_dx.down", "gemm_dw.down", m->d_act, w.down.gradient, current, a.act, w.down.value, I, H, 0));
+        CGPTX_TRY(project_bwd(kDownLabels, m->d_act, w.down.gradient, current, a.act, w.down.value, I, H, 0));
         note_call(m, "swiglu_backward", {d_gate, d_up, m->d_act, gate, up}, {N * I}, {0, 0});
         CGPTX_OP("swiglu_bwd", cgptx_swiglu_backward(d_gate, d_up, m->d_act, gate, up, N * I, 0, 0, dt, s));
-        CGPTX_TRY(project_bwd("gemm_dx.gate_up", "gemm_dw.gate_up", m->d_norm_in, w.gate.gradient, d_gate, a.norm_f, w.gate.value, H, I, 0));
-        CGPTX_TRY(project_bwd("gemm_dx.gate_up", "gemm_dw.gate_up", m->d_norm_in, w.up.gradient, d_up, a.norm_f, w.up.value, H, I, 1));
+        CGPTX_TRY(project_bwd(kGateUpLabels, m->d_norm_in, w.gate.gradient, d_gate, a.norm_f, w.gate.value, H, I, 0));
+        CGPTX_TRY(project_bwd(kGateUpLabels, m->d_norm_in, w.up.gradient, d_up, a.norm_f, w.up.value, H, I, 1));
         CGPTX_TRY(norm_bwd(grad_residual, w.ffn_norm.gradient, m->d_norm_in, x, w.ffn_norm.value, N, H));
         CGPTX_TRY(add(previous, current, grad_residual));  // grad_input = grad_output + grad_residual
-        CGPTX_TRY(project_bwd("gemm_dx.o", "gemm_dw.o", m->d_attn_out, w.o.gradient, current, a.attn_out, w.o.value, QW, H, 0));
+        CGPTX_TRY(project_bwd(kOutputLabels, m->d_attn_out, w.o.gradient, current, a.attn_out, w.o.value, QW, H, 0));
         note_call(m, "flash_gqa_attention_backward_with_lse", {m->d_q, m->d_k, m->d_v, m->d_attn_out, a.attn_out, a.lse, a.q, a.k, a.v},
                   {B, T, T, HQ, HKV, D, 0}, {1, 0});
         CGPTX_OP("attn_bwd", cgptx_flash_gqa_attention_backward_with_lse(m->d_q, m->d_k, m->d_v, m->d_attn_out, a.attn_out, a.lse,
@@ -681,9 +707,9 @@ int enqueue_reference_sequence(cgptx_model* m, float loss_scale, int loss_mode, 
                                                  c.rotary_dim, 0, T, dt, s));
         CGPTX_TRY(norm_bwd(m->d_q, w.q_norm.gradient, m->d_q_pre, a.q_pre, w.q_norm.value, N * HQ, D));
         CGPTX_TRY(norm_bwd(m->d_k, w.k_norm.gradient, m->d_k_pre, a.k_pre, w.k_norm.value, N * HKV, D));
-        CGPTX_TRY(project_bwd("gemm_dx.qkv", "gemm_dw.qkv", m->d_norm_in, w.q.gradient, m->d_q, a.norm_a, w.q.value, H, QW, 0));
-        CGPTX_TRY(project_bwd("gemm_dx.qkv", "gemm_dw.qkv", m->d_norm_in, w.k.gradient, m->d_k, a.norm_a, w.k.value, H, KW, 1));
-        CGPTX_TRY(project_bwd("gemm_dx.qkv", "gemm_dw.qkv", m->d_norm_in, w.v.gradient, m->d_v, a.norm_a, w.v.value, H, KW, 1));
+        CGPTX_TRY(project_bwd(kQkvLabels, m->d_norm_in, w.q.gradient, m->d_q, a.norm_a, w.q.value, H, QW, 0));
+        CGPTX_TRY(project_bwd(kQkvLabels, m->d_norm_in, w.k.gradient, m->d_k, a.norm_a, w.k.value, H, KW, 1));
+        CGPTX_TRY(project_bwd(kQkvLabels, m->d_norm_in, w.v.gradient, m->d_v, a.norm_a, w.v.value, H, KW, 1));
         CGPTX_TRY(norm_bwd(grad_residual, w.attention_norm.gradient, m->d_norm_in, x, w.attention_norm.value, N, H));
         CGPTX_TRY(add(previous, previous, grad_residual));
         std::swap(current, previous);
@@ -768,7 +794,7 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
                                        c.vocabulary_size, dt, s));
         CGPTX_OP("dense_ce", cgptx_cross_entropy_forward_backward(m->loss, m->grad_logits, m->logits, m->targets, N,
                                                        c.vocabulary_size, loss_scale, dt, s));
-        CGPTX_TRY(linear_backward_split(m, m->d_normalized, m->embedding.gradient, m->grad_logits, m->normalized, m->embedding.value, N, H, c.vocabulary_size, 0, dt, stream, "gemm_dx.classifier", "gemm_dw.classifier"));
+        CGPTX_TRY(linear_gradients(m, m->d_normalized, m->embedding.gradient, m->grad_logits, m->normalized, m->embedding.value, N, H, c.vocabulary_size, 0, dt, stream, kClassifierLabels));
     }
 
     // ----------------------------------------------------------------- backward
@@ -797,7 +823,7 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             if (!stacked)
                 CGPTX_OP("gemm_dw.down", cgptx_linear_backward(nullptr, w.down.gradient, nullptr, current, a.act, w.down.value, N, I, H, 0, 0, 0, dt, s));
         } else {
-            CGPTX_TRY(linear_backward_split(m, m->d_act, stacked ? nullptr : w.down.gradient, current, a.act, w.down.value, N, I, H, 0, dt, stream, "gemm_dx.down", "gemm_dw.down"));
+            CGPTX_TRY(linear_gradients(m, m->d_act, stacked ? nullptr : w.down.gradient, current, a.act, w.down.value, N, I, H, 0, dt, stream, kDownLabels));
             CGPTX_OP("swiglu_bwd", cgptx_swiglu_backward_packed(d_gate_up, m->d_act, a.gate_up, N, I, 0, dt, s));
         }
         // The gradient of the residual stream collects the two norm branches: in one pass at the end of
@@ -806,12 +832,12 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         const bool dual_norms = fused_block_norms(m, previous, m->d_norm_in, m->d_norm_in_f, x, current) &&
                                 is_aligned16(w.attention_norm.value) && is_aligned16(w.ffn_norm.value);
         void* d_norm_f = dual_norms ? m->d_norm_in_f : m->d_norm_in;
-        CGPTX_TRY(linear_backward_split(m, d_norm_f, stacked ? nullptr : w.gate.gradient, d_gate_up, a.norm_f, w.gate.value, N, H, 2 * I, 0, dt, stream, "gemm_dx.gate_up", "gemm_dw.gate_up"));
+        CGPTX_TRY(linear_gradients(m, d_norm_f, stacked ? nullptr : w.gate.gradient, d_gate_up, a.norm_f, w.gate.value, N, H, 2 * I, 0, dt, stream, kGateUpLabels));
         if (!dual_norms) {
             CGPTX_OP("rmsnorm_bwd", rmsnorm_backward_residual(previous, w.ffn_norm.gradient, m->d_norm_in, x, w.ffn_norm.value,
                                                               current, N, H, eps, dt, stream, sink));
         }
-        CGPTX_TRY(linear_backward_split(m, m->d_attn_out, stacked ? nullptr : w.o.gradient, current, a.attn_out, w.o.value, N, QW, H, 0, dt, stream, "gemm_dx.o", "gemm_dw.o"));
+        CGPTX_TRY(linear_gradients(m, m->d_attn_out, stacked ? nullptr : w.o.gradient, current, a.attn_out, w.o.value, N, QW, H, 0, dt, stream, kOutputLabels));
         CGPTX_OP("attn_bwd", cgptx_flash_gqa_attention_backward_with_lse(d_q, d_k, d_v, m->d_attn_out, a.attn_out,
                                                               a.lse, a.q, a.k, a.v, m->batch, m->sequence,
                                                               m->sequence, HQ, HKV, D, 0.0f, 1, 0, 0, dt, s));
@@ -839,11 +865,11 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             if (!stacked)
                 CGPTX_OP("gemm_dw.qkv", qkv_backward_weight(w.q.gradient, d_q, d_k, d_v, a.norm_a, N, H, QW, KW, dt, stream));
         } else if (gradient_group.joined) {
-            CGPTX_OP("gemm_dx.qkv", gemm_joined(qkv_gradients, 4, gradient_group, stream));
+            CGPTX_OP("gemm_dx_dw.qkv", gemm_joined(qkv_gradients, 4, gradient_group, stream));
         } else {
-            CGPTX_TRY(linear_backward_split(m, m->d_norm_in, w.q.gradient, d_q, a.norm_a, w.q.value, N, H, QW, 0, dt, stream, "gemm_dx.qkv", "gemm_dw.qkv"));
-            CGPTX_TRY(linear_backward_split(m, m->d_norm_in, w.k.gradient, d_k, a.norm_a, w.k.value, N, H, KW, 1, dt, stream, "gemm_dx.qkv", "gemm_dw.qkv"));
-            CGPTX_TRY(linear_backward_split(m, m->d_norm_in, w.v.gradient, d_v, a.norm_a, w.v.value, N, H, KW, 1, dt, stream, "gemm_dx.qkv", "gemm_dw.qkv"));
+            CGPTX_TRY(linear_gradients(m, m->d_norm_in, w.q.gradient, d_q, a.norm_a, w.q.value, N, H, QW, 0, dt, stream, kQkvLabels));
+            CGPTX_TRY(linear_gradients(m, m->d_norm_in, w.k.gradient, d_k, a.norm_a, w.k.value, N, H, KW, 1, dt, stream, kQkvLabels));
+            CGPTX_TRY(linear_gradients(m, m->d_norm_in, w.v.gradient, d_v, a.norm_a, w.v.value, N, H, KW, 1, dt, stream, kQkvLabels));
         }
         if (dual_norms) {
             CGPTX_OP("rmsnorm_bwd", rmsnorm_backward_dual(previous, w.attention_norm.gradient, w.ffn_norm.gradient, m->d_norm_in,

@@ -112,7 +112,8 @@ int cgptx_model_status(cgptx_model* model, float* loss, int* all_finite, uint64_
 
 /* Runs one eager forward + loss + backward with HIP events around every operator call on
  * `stream` and keeps the time per operator kind ("gemm_fwd", "gemm_dx", "gemm_dw", "attn_fwd",
- * "attn_bwd", "rmsnorm_bwd", ...), summed over the calls of that kind. Synchronises. */
+ * "attn_bwd", "rmsnorm_bwd", ...), summed over the calls of that kind. The launches are those of every other
+ * pass: small projections whose gradients share one are found under "gemm_dx_dw". Synchronises. */
 int cgptx_model_profile(cgptx_model* model, float loss_scale, int loss_mode, cgptx_stream stream);
 size_t cgptx_model_profile_count(const cgptx_model* model);
 int cgptx_model_profile_entry(const cgptx_model* model, size_t index, const char** label, float* milliseconds);

@@ -470,6 +470,31 @@ def test_norm_weight_gradients_reduced_at_the_end_of_the_backward_pass_are_bit_i
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("batch,seq,together", [(3, 100, True), (16, 1024, False)], ids=["small", "large"])
+def test_profile_times_the_launches_of_the_step(device, batch, seq, together):
+    """The profiled pass makes the launches of every other pass, so it gives the same bits, and its labels tell what they were:
+    a small model's gradients share launches, a large one's have their own."""
+    from cgpt_amd.model import LOSS_CUT, Model, ModelConfig
+    config = ModelConfig(vocabulary_size=503, num_layers=2, hidden_size=256, intermediate_size=704, num_query_heads=4,
+                         num_kv_heads=2, head_dim=64, rotary_dim=64, dtype=torch.float16)
+    rng = np.random.default_rng(5)
+    inputs, targets = (rng.integers(0, 503, size=batch * seq).astype(np.uint32) for _ in range(2))
+    model = Model(config, batch, seq, seed=6, device=device)
+    model.set_tokens(inputs, targets)
+    model.forward_backward(loss_scale=64.0, loss_mode=LOSS_CUT)
+    torch.cuda.synchronize()
+    want = [g.clone() for _, _, g in model.parameters()]
+    labels = model.profile(64.0, LOSS_CUT)
+    for (name, _, got), expected in zip(model.parameters(), want):
+        assert torch.equal(got, expected), name
+    assert all(ms > 0 for ms in labels.values())
+    for projection in ("gate_up", "o", "qkv"):
+        assert (f"gemm_dx_dw.{projection}" in labels) == together, labels
+        assert (f"gemm_dx.{projection}" in labels) != together and (f"gemm_dw.{projection}" in labels) != together, labels
+    model.close()
+
+
+@pytest.mark.gpu
 def test_swiglu_in_the_projection_epilogues_is_bit_identical_to_the_separate_operators(device, monkeypatch):
     """The SwiGLU product rides in the gate/up projection's epilogue and its gradient in the epilogue of the
     down projection's input gradient when the shapes fill the chip (here 4096 rows x 3328 feed-forward
