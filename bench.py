@@ -310,18 +310,24 @@ def published_kernel_shapes(torch, stream, seed):
     return out
 
 
-def source_digest(name):
-    """sha256 of a kernel source file (the summaries under profiles/ record the one they were made with)."""
+PROBE_SOURCES = ("gemm_large_kernel.hpp", "gemm_tiles.hpp")  # the probe's kernel and its operand loads
+CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cgpt_amd", "csrc")
+
+
+def source_digest():
+    """sha256 of PROBE_SOURCES, one after the other (the summary under profiles/ records the one it was made with)."""
     import hashlib
 
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cgpt_amd", "csrc", name)
-    with open(path, "rb") as handle:
-        return hashlib.sha256(handle.read()).hexdigest()
+    digest = hashlib.sha256()
+    for name in PROBE_SOURCES:
+        with open(os.path.join(CSRC, name), "rb") as handle:
+            digest.update(handle.read())
+    return digest.hexdigest()
 
 
 def measured_traffic():
     """(HBM bytes per launch of the probe kernel from the committed counter summary or None, note). The summary
-    names the sha256 of the kernel source it was measured with; when the source has changed since, the figure is
+    names the sha256 of the kernel sources it was measured with; when one has changed since, the figure is
     reported with a warning (stderr and `traffic_note`) instead of silently."""
     value, recorded = None, None
     try:
@@ -335,11 +341,12 @@ def measured_traffic():
         return None, "no counter summary found"
     if value is None:
         return None, "the counter summary holds no traffic figure"
-    if recorded is None or recorded != source_digest("gemm_large_kernel.hpp"):
-        note = "STALE: cgpt_amd/csrc/gemm_large_kernel.hpp has changed since profiles/gemm_dx_256x256_gate_projection_pmc.txt was measured"
+    sources = " and ".join(PROBE_SOURCES) + " in cgpt_amd/csrc"
+    if recorded is None or recorded != source_digest():
+        note = f"STALE: {sources} are not what profiles/gemm_dx_256x256_gate_projection_pmc.txt was measured with"
         print("bench.py: warning: roofline.traffic is " + note, file=sys.stderr)
         return value, note
-    return value, "measured with the current cgpt_amd/csrc/gemm_large_kernel.hpp"
+    return value, f"measured with the current {sources}"
 
 
 def cpu_model_name():
