@@ -48,7 +48,7 @@ struct GemmArgs {
     int dtype = CGPTX_BF16;
     // Column segments of A as stored (its K range when k-contiguous, its M range otherwise) and of
     // C (written through; not combined with split-K, residual or fp32 output). Segment widths are
-    // multiples of 256 (of 32 for a k-contiguous A) except the last; a and lda / c and ldc are
+    // multiples of 256 (of 64 for a k-contiguous A) except the last; a and lda / c and ldc are
     // ignored for a segmented operand.
     GemmSegments a_segments, c_segments;
     // Forward projection into the concatenated [gate | up] layout (n = 2·inter, b = [gate; up]

@@ -1,0 +1,183 @@
+// The projections of q, k and v as the step of a small model makes them: several contractions in one launch
+// (cgpt_amd/csrc/gemm.hpp), forward as a group of three, backward as one of four whose input gradient reads its operand from
+// three buffers. Operands of -1 .. 1: sums of at most 8192 products are exact in fp32 in any order, so every result is the
+// rounded exact value. Built by `python -m cgpt_amd.build`; run by tests/test_cpp_interface.py on the GPU.
+#include <cstdio>
+#include <cstring>
+#include <random>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "gemm.hpp"
+
+namespace {
+
+using cgptx::GemmArgs;
+using Bits = std::vector<std::uint16_t>;
+
+int failures = 0;
+void expect(bool ok, const std::string& what) {
+    if (!ok) {
+        ++failures;
+        std::printf("FAIL %s\n", what.c_str());
+    }
+}
+void hip_ok(hipError_t status, const char* what) {
+    if (status != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(status));
+}
+
+// Nearest even, of whole numbers far from either type's limits.
+std::uint16_t rounded(int value, int dtype) {
+    std::uint16_t out;
+    if (dtype == CGPTX_F16) {
+        const auto half = static_cast<_Float16>(value);
+        std::memcpy(&out, &half, 2);
+        return out;
+    }
+    const auto f = static_cast<float>(value);
+    std::uint32_t bits;
+    std::memcpy(&bits, &f, 4);
+    return static_cast<std::uint16_t>((bits + 0x7fff + (bits >> 16 & 1)) >> 16);
+}
+
+struct Matrix {
+    std::size_t rows, cols;
+    std::vector<int> values;
+    int at(std::size_t r, std::size_t c) const { return values[r * cols + c]; }
+};
+Matrix random_matrix(std::size_t rows, std::size_t cols, std::mt19937& rng) {
+    Matrix m{rows, cols, std::vector<int>(rows * cols)};
+    for (int& v : m.values) v = static_cast<int>(rng() % 3) - 1;
+    return m;
+}
+// Sum over t of a(t) b(t), for element (i, j) of a result.
+template <typename A, typename B>
+Bits product(std::size_t m, std::size_t n, std::size_t k, int dtype, A&& a, B&& b) {
+    Bits out(m * n);
+    for (std::size_t i = 0; i < m; ++i)
+        for (std::size_t j = 0; j < n; ++j) {
+            int sum = 0;
+            for (std::size_t t = 0; t < k; ++t) sum += a(i, t) * b(t, j);
+            out[i * n + j] = rounded(sum, dtype);
+        }
+    return out;
+}
+
+// Device memory with guards before and behind it.
+class Buffer {
+public:
+    explicit Buffer(std::size_t count) : count_(count), host_(count + 2 * kGuard, kPoison) { allocate(); }
+    Buffer(const Matrix& m, int dtype) : count_(m.values.size()), host_(count_ + 2 * kGuard, kPoison) {
+        for (std::size_t i = 0; i < count_; ++i) host_[kGuard + i] = rounded(m.values[i], dtype);
+        allocate();
+    }
+    Buffer(const Buffer&) = delete;
+    ~Buffer() { (void)hipFree(base_); }
+    std::uint16_t* data() const { return base_ + kGuard; }
+    bool holds(const Bits& want) {
+        hip_ok(hipMemcpy(host_.data(), base_, host_.size() * 2, hipMemcpyDeviceToHost), "hipMemcpy");
+        for (std::size_t i = 0; i < kGuard; ++i)
+            if (host_[i] != kPoison || host_[kGuard + count_ + i] != kPoison) return false;
+        return want.size() == count_ && std::memcmp(host_.data() + kGuard, want.data(), count_ * 2) == 0;
+    }
+
+private:
+    void allocate() {
+        hip_ok(hipMalloc(reinterpret_cast<void**>(&base_), host_.size() * 2), "hipMalloc");
+        hip_ok(hipMemcpy(base_, host_.data(), host_.size() * 2, hipMemcpyHostToDevice), "hipMemcpy");
+    }
+    static constexpr std::size_t kGuard = 512;
+    static constexpr std::uint16_t kPoison = 0x7fc1;  // no number in either type
+    std::size_t count_;
+    std::vector<std::uint16_t> host_;
+    std::uint16_t* base_ = nullptr;
+};
+
+void check(std::size_t rows, std::size_t hidden, std::size_t q, std::size_t k, std::size_t v, int dtype, hipStream_t stream) {
+    const std::string name = std::to_string(rows) + " x " + std::to_string(hidden) + ", " + std::to_string(q) + " + " +
+                             std::to_string(k) + " + " + std::to_string(v) + (dtype == CGPTX_F16 ? " f16" : " bf16");
+    std::printf("%s\n", name.c_str());
+    std::fflush(stdout);
+    std::mt19937 rng(static_cast<unsigned int>(rows + hidden + q + v));
+    const std::size_t width[3] = {q, k, v}, total = q + k + v;
+    const Matrix x = random_matrix(rows, hidden, rng), w = random_matrix(total, hidden, rng);
+    const Matrix dy[3] = {random_matrix(rows, q, rng), random_matrix(rows, k, rng), random_matrix(rows, v, rng)};
+    const Buffer on_x(x, dtype), on_w(w, dtype), on_dq(dy[0], dtype), on_dk(dy[1], dtype), on_dv(dy[2], dtype);
+    const Buffer* on_dy[3] = {&on_dq, &on_dk, &on_dv};
+    Buffer y_q(rows * q), y_k(rows * k), y_v(rows * v), dw_q(q * hidden), dw_k(k * hidden), dw_v(v * hidden), dx(rows * hidden);
+    Buffer *y[3] = {&y_q, &y_k, &y_v}, *dw[3] = {&dw_q, &dw_k, &dw_v};
+
+    GemmArgs forward[3], backward[4];
+    GemmArgs& input = backward[0];  // dX = [dq | dk | dv]·W
+    input.b = on_w.data();
+    input.c = dx.data();
+    input.m = rows;
+    input.n = input.ldb = input.ldc = hidden;
+    input.k = total;
+    input.b_k_contiguous = false;
+    input.dtype = dtype;
+    input.a_segments.count = 3;
+    std::size_t first[3] = {0, q, q + k};
+    for (int i = 0; i < 3; ++i) {
+        GemmArgs& f = forward[i];  // Y = X·Wᵀ
+        f.a = on_x.data();
+        f.b = on_w.data() + first[i] * hidden;
+        f.c = y[i]->data();
+        f.m = rows;
+        f.n = f.ldc = width[i];
+        f.k = f.lda = f.ldb = hidden;
+        f.dtype = dtype;
+        GemmArgs& b = backward[i + 1];  // dW = dYᵀ·X
+        b.a = on_dy[i]->data();
+        b.b = on_x.data();
+        b.c = dw[i]->data();
+        b.m = b.lda = width[i];
+        b.n = b.ldb = b.ldc = hidden;
+        b.k = rows;
+        b.a_k_contiguous = b.b_k_contiguous = false;
+        b.dtype = dtype;
+        input.a_segments.ptr[i] = on_dy[i]->data();
+        input.a_segments.ld[i] = input.a_segments.cols[i] = width[i];
+    }
+    const cgptx::GemmGroup forward_group = cgptx::gemm_joins(forward, 3), backward_group = cgptx::gemm_joins(backward, 4);
+    expect(forward_group.joined, name + ": the projections share no launch");
+    expect(backward_group.joined, name + ": the gradients share no launch");
+    if (!forward_group.joined || !backward_group.joined) return;
+    expect(cgptx::gemm_joined(forward, 3, forward_group, stream) == CGPTX_OK, name + ": forward launch");
+    expect(cgptx::gemm_joined(backward, 4, backward_group, stream) == CGPTX_OK, name + ": backward launch");
+    hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize");
+
+    const auto dy_at = [&](std::size_t r, std::size_t c) { return c < q ? dy[0].at(r, c) : c < q + k ? dy[1].at(r, c - q) : dy[2].at(r, c - q - k); };
+    expect(dx.holds(product(rows, hidden, total, dtype, dy_at, [&](std::size_t t, std::size_t j) { return w.at(t, j); })), name + ": dX");
+    for (int i = 0; i < 3; ++i) {
+        expect(y[i]->holds(product(rows, width[i], hidden, dtype, [&](std::size_t r, std::size_t t) { return x.at(r, t); },
+                                   [&](std::size_t t, std::size_t j) { return w.at(first[i] + j, t); })),
+               name + ": Y " + std::to_string(i));
+        expect(dw[i]->holds(product(width[i], hidden, rows, dtype, [&](std::size_t c, std::size_t t) { return dy[i].at(t, c); },
+                                    [&](std::size_t t, std::size_t j) { return x.at(t, j); })),
+               name + ": dW " + std::to_string(i));
+    }
+}
+
+}  // namespace
+
+int main() {
+    try {
+        hipStream_t stream = nullptr;
+        hip_ok(hipStreamCreate(&stream), "hipStreamCreate");
+        for (const int dtype : {CGPTX_F16, CGPTX_BF16}) {
+            check(1, 64, 64, 64, 32, dtype, stream);        // the last segment is half a K tile
+            check(33, 96, 128, 64, 96, dtype, stream);      // one row behind a 32-wide tile, a step more than whole K tiles
+            check(100, 256, 256, 128, 128, dtype, stream);  // 3 x 100 tokens' kind: segments of whole K tiles
+            check(131, 224, 192, 64, 160, dtype, stream);   // ragged rows and columns, five steps in the last segment
+            check(300, 512, 512, 64, 224, dtype, stream);   // more rows than one tile of either size
+        }
+        hip_ok(hipStreamDestroy(stream), "hipStreamDestroy");
+    } catch (const std::exception& e) {
+        std::printf("FAIL %s\n", e.what());
+        ++failures;
+    }
+    std::printf("%d failure(s)\n", failures);
+    return failures == 0 ? 0 : 1;
+}

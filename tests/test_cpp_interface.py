@@ -91,3 +91,14 @@ def test_callers_of_the_headers_reproduce_the_library_step():
     proc = subprocess.run([str(binary)], capture_output=True, text=True, timeout=120)
     assert proc.returncode == 0, proc.stdout + proc.stderr
     assert "0 failure(s)" in proc.stdout
+
+
+@pytest.mark.gpu
+def test_projections_of_a_small_block_share_exact_launches():
+    """tests/cpp/gemm_group_test.cpp: the forward projections of q, k and v as one launch, and their four gradients as one whose
+    input gradient reads three buffers; ragged rows and segments that end inside a K tile, exact on whole numbers."""
+    binary = ROOT / "tests" / "cpp" / "gemm_group_test.bin"
+    assert binary.exists(), "build it with `python -m cgpt_amd.build` (there is no fallback)"
+    proc = subprocess.run([str(binary)], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+    assert "\n0 failure(s)" in proc.stdout

@@ -7,7 +7,7 @@ import torch
 from cgpt_amd import ops
 from oracle import cpu_ops, oracle64
 from tests.test_gpu_attention import make_inputs, oracle_args, run_backward, run_forward
-from tests.util import DTYPE_IDS, DTYPES, STOL, TOL, assert_close, assert_scaled_close, randint, randn, to_np
+from tests.util import DTYPE_IDS, DTYPES, STOL, TOL, assert_close, assert_scaled_close, launches, randint, randn, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -168,13 +168,23 @@ def test_column_sums_add_in_their_order(device, rows, width):
     (1, 64, 64), (31, 64, 32), (33, 40, 72), (300, 256, 100),   # tiles of 32 and 64, one and more per gradient, ragged edges
     (128, 768, 2048), (2000, 1024, 2048), (1999, 1000, 2040),   # more workgroups than compute units
     (70, 256, 5003),                                            # output gradient in padded rows
+    (33, 40, 96), (131, 72, 160), (1999, 1000, 2048),           # ragged edges in the shared launch
 ])
 def test_linear_gradients_in_one_launch_are_exact_on_integers(device, rows, fin, fout, accumulate, dtype):
-    """dX, dW and db of a small call share a launch. Products and sums of small integers are exact in fp32 (at most 4 x 5003 + 2),
+    """dX, dW and db of a small call share a launch, behind a copy of 16-bit output gradients whose rows are no whole K steps (the
+    other ragged calls go their own way, several launches). Products and sums of small integers are exact in fp32 (at most 4 x 5003 + 2),
     so every result is the rounded exact value; all three overwritten and all three added to what is there."""
     g = torch.Generator().manual_seed(rows + fin + fout)
     ints = lambda *shape: torch.randint(-2, 3, shape, generator=g).double()
     x, w, dy = ints(rows, fin), ints(fout, fin), ints(rows, fout)
+    blank = [torch.zeros(shape, dtype=dtype, device=device) for shape in ((rows, fin), (fout, fin), fout, (rows, fout), (rows, fin), (fout, fin))]
+    enqueued = launches(lambda: ops.linear_backward(*blank))
+    if fout % 32 == 0:
+        assert enqueued == 1
+    elif fin % 32 == 0 and dtype != torch.float32:
+        assert enqueued == 2
+    else:
+        assert enqueued > 2
     start = {"dX": ints(rows, fin), "dW": ints(fout, fin), "db": ints(fout)}
     got = {name: t.to(dtype).to(device) if accumulate else torch.full(t.shape, float("nan"), dtype=dtype, device=device)
            for name, t in start.items()}
