@@ -49,8 +49,8 @@ namespace {
 // CU, DEEP: one with 5 + 4 slots.
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool DEEP>
 struct TileLayout {
-    using ATile = std::conditional_t<A_K, KTile<T, BM, kSteps>, NTile<T, BM, kSteps>>;
-    using BTile = std::conditional_t<B_K, KTile<T, BN, kSteps>, NTile<T, BN, kSteps>>;
+    using ATile = std::conditional_t<A_K, KTile<T, BM>, NTile<T, BM>>;
+    using BTile = std::conditional_t<B_K, KTile<T, BN>, NTile<T, BN>>;
     static constexpr int kASlots = DEEP ? 5 : 3, kBSlots = DEEP ? 4 : 2;
     static constexpr int kSmemBytes = (kASlots * ATile::kElems + kBSlots * BTile::kElems) * static_cast<int>(sizeof(T));
     // The order of an item's requests: A's K tile x is requested in the first step of K tile x + 1 - kASlots, B's in the
@@ -83,8 +83,8 @@ __device__ __forceinline__ void store_chunk(const u32x4& data, __amdgpu_buffer_r
 __device__ __host__ __forceinline__ bool stored_as_it_is(const KernelArgs& p) {
     return p.bias == nullptr && p.residual == nullptr && p.addend == nullptr && !p.accumulate && !p.c_f32 && !p.ragged;
 }
-template <int BM, bool SPLIT, bool RESIDUAL, bool SWIGLU, bool GRAD>
 // Such calls have a kernel of their own. Not on 256 x 256 tiles, which gain nothing by it (0.996 - 1.009 over four workloads).
+template <int BM, bool SPLIT, bool RESIDUAL, bool SWIGLU, bool GRAD>
 constexpr bool plain_apart = BM == 128 && !SPLIT && !RESIDUAL && !SWIGLU && !GRAD;
 
 // One workgroup per CU slot walks its share of the work items (output tile x K slice) one after
@@ -109,7 +109,8 @@ template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGME
 __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     static_assert(!GRAD || (A_K && !B_K && !SPLIT && !SEGMENTED && !RESIDUAL && !SWIGLU && BN == 256),
                   "the SwiGLU gradient epilogue belongs to the plain input-gradient kernel with 256-wide tiles");
-    static_assert(!SEGMENTED || (A_K && !SPLIT), "segments along K are read by the unsplit kernels only");
+    static_assert(!SEGMENTED || (A_K && !B_K && !SPLIT && (PLAIN || BM == 256)),
+                  "segments along K are read by unsplit input gradients that nothing is added to");
     static_assert(!RESIDUAL || (!SPLIT && !SEGMENTED), "the residual epilogue belongs to plain unsplit kernels");
     static_assert(!SWIGLU || (A_K && B_K && !SPLIT && !SEGMENTED && !RESIDUAL && BN == 256),
                   "the SwiGLU epilogue belongs to the plain forward kernel with 256-wide tiles");
@@ -893,18 +894,10 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
 // ------------------------------------------------------------------- host side
 constexpr int blocks_per_unit(int tile) { return tile == 256 ? 1 : 2; }  // resident blocks per CU: what the LDS slots allow
 
-template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
-          bool SWIGLU = false, bool GRAD = false, bool DEEP = false, bool PLAIN = false>
-int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
+template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL, bool SWIGLU, bool GRAD,
+          bool DEEP, bool PLAIN>
+int launch_kernel(const KernelArgs& p, int slices, hipStream_t stream) {
     const long items = static_cast<long>(p.tiles_m) * p.tiles_n * slices;
-    if constexpr (BM == 128 && !DEEP && !PLAIN) {
-        if (items <= compute_units())
-            return launch_mfma<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, true>(p, slices, stream);
-    }
-    if constexpr (plain_apart<BM, SPLIT, RESIDUAL, SWIGLU, GRAD> && !PLAIN) {
-        if (stored_as_it_is(p))
-            return launch_mfma<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP, true>(p, slices, stream);
-    }
     constexpr std::size_t smem = TileLayout<T, BM, BN, A_K, B_K, DEEP>::kSmemBytes;
     auto kernel = gemm_mfma_kernel<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP, PLAIN>;
     static bool configured = false;
@@ -937,16 +930,33 @@ int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
     return CGPTX_OK;
 }
 
+template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
+          bool SWIGLU = false, bool GRAD = false>
+int launch_mfma(const KernelArgs& p, int slices, hipStream_t stream) {
+    auto with_depth = [&]<bool DEEP>() -> int {
+        if constexpr (plain_apart<BM, SPLIT, RESIDUAL, SWIGLU, GRAD>) {
+            if (stored_as_it_is(p))
+                return launch_kernel<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP, true>(p, slices, stream);
+            if constexpr (SEGMENTED) return fail(CGPTX_RUNTIME, "gemm: an operand in segments along K takes nothing added to its product");
+        }
+        if constexpr (!(SEGMENTED && BM == 128))
+            return launch_kernel<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP, false>(p, slices, stream);
+    };
+    if constexpr (BM == 128) {
+        if (static_cast<long>(p.tiles_m) * p.tiles_n * slices <= compute_units()) return with_depth.template operator()<true>();
+    }
+    return with_depth.template operator()<false>();
+}
+
 template <typename T, int BM, int BN, bool SPLIT>
 int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream_t stream) {
     // A given in segments along K has kernels of its own (the source of a K tile is then picked
-    // per tile), and only unsplit ones.
+    // per tile), and only unsplit ones of input gradients.
     const bool segmented = a_k && p.a_seg.count > 0;
     if constexpr (!SPLIT && !std::is_same_v<T, float>) {
-        if (segmented && b_k) return launch_mfma<T, BM, BN, true, true, false, true>(p, slices, stream);
         if (segmented && !b_k) return launch_mfma<T, BM, BN, true, false, false, true>(p, slices, stream);
     }
-    if (segmented) return fail(CGPTX_RUNTIME, "gemm: a segmented operand cannot be split along K");
+    if (segmented) return fail(CGPTX_RUNTIME, "gemm: an operand in segments along K is that of an unsplit input gradient");
     if constexpr (!SPLIT && BN == 256) {
         if (p.act != nullptr) return launch_mfma<T, BM, BN, true, true, false, false, false, true>(p, slices, stream);
     }

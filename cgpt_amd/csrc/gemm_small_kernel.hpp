@@ -49,8 +49,8 @@ constexpr int small_smem_bytes() { return DEEP ? 128 * 1024 : 64 * 1024; }
 template <typename T, int TILE, bool DEEP, bool A_K, bool B_K, SmallEpilogue EPILOGUE, bool SEGMENTED, bool SUMS>
 __device__ __forceinline__ void small_tile(const SmallArgs& p, int m0, int n0, int slice, unsigned char* smem_raw) {
     using frag_t = typename Mfma<T>::frag;
-    using ATile = std::conditional_t<A_K, KTile<T, TILE, kSteps>, NTile<T, TILE, kSteps>>;
-    using BTile = std::conditional_t<B_K, KTile<T, TILE, kSteps>, NTile<T, TILE, kSteps>>;
+    using ATile = std::conditional_t<A_K, KTile<T, TILE>, NTile<T, TILE>>;
+    using BTile = std::conditional_t<B_K, KTile<T, TILE>, NTile<T, TILE>>;
     constexpr int kBlocks = TILE / 16;                  // 16 x 16 MFMA blocks along an edge
     constexpr int kOperandBytes = TILE * 64 * kSteps;   // 128 bytes along K per row, or the same bytes k-strided
     constexpr int kStageBytes = 2 * kOperandBytes;      // [A | B]

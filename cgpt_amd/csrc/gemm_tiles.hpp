@@ -174,18 +174,18 @@ __device__ __forceinline__ unsigned int lds_address_of(const T* p) {
 // cannot be padded; bank conflicts are avoided by storing 16-byte chunk c of a row at chunk
 // position c ^ swizzle(row) — the lane that owns an LDS slot fetches the matching global chunk.
 
-// ---- operand stored [ROWS, K] (k-contiguous): ROWS x (STEPS * kBK) slab, unpadded LDS rows -----
-// A row of the slab is STEPS * 64 bytes. With two K steps that is a whole cache line: a load instruction then touches 8
+// ---- operand stored [ROWS, K] (k-contiguous): ROWS x (kSteps * kBK) slab, unpadded LDS rows -----
+// A row of the slab is two K steps, a whole cache line: a load instruction then touches 8
 // lines instead of 16 halves of lines, which is what the path from the L2s to a CU's LDS is bound by (16 KiB of operand
 // tiles per CU, every CU loading: 0.25 us in pieces of 64 bytes, 0.17 us in pieces of 128, no more in longer ones).
 // One load instruction covers 1024 B = kRowsPerLoad rows; wavefront w issues the loads of row
 // groups w, w+4, ... The chunk swizzle is (row / rows per 256 B) mod chunks per row: the 16 rows a
 // quarter-wavefront reads with ds_read_b128 then hit the 16 different 16-byte positions of a
 // 256-byte bank period.
-template <typename T, int ROWS, int STEPS = 1>
+template <typename T, int ROWS>
 struct KTile {
     using frag_t = typename Mfma<T>::frag;
-    static constexpr int kRowElems = STEPS * kBK<T>;
+    static constexpr int kRowElems = kSteps * kBK<T>;
     static constexpr int kChunksPerRow = kRowElems / kVec128<T>;
     static constexpr int kRowsPerLoad = 64 / kChunksPerRow;
     static constexpr int kElems = ROWS * kRowElems;
@@ -195,7 +195,7 @@ struct KTile {
     int voffset = 0, voffset1 = 0;
     unsigned int group_bytes = 0;  // kRowsPerLoad rows further in global memory
 
-    __device__ __forceinline__ static int swizzle(int row) { return (row / (4 / STEPS)) % kChunksPerRow; }
+    __device__ __forceinline__ static int swizzle(int row) { return (row / 2) % kChunksPerRow; }
 
     // base: element (row0, 0) of the operand; rows past rows_left only feed C rows that are never
     // stored (they read zeros or whatever follows, never out of the allocation's last row). A tile may start behind the
@@ -214,7 +214,7 @@ struct KTile {
     }
     // The lane's offset for load i of a wavefront that loads the whole tile (init with wave 0): with eight rows per load
     // the swizzle of every other load differs.
-    __device__ __forceinline__ int load_voffset(int i) const { return STEPS == 2 && (i & 1) != 0 ? voffset1 : voffset; }
+    __device__ __forceinline__ int load_voffset(int i) const { return (i & 1) != 0 ? voffset1 : voffset; }
     // Scalar offset of wavefront `wave`'s first load of the tile that starts at column k0.
     __device__ __forceinline__ unsigned int first_offset(int k0, int wave) const {
         return wave * group_bytes + k0 * static_cast<unsigned int>(sizeof(T));
@@ -229,20 +229,20 @@ struct KTile {
     }
 };
 
-// ---- operand stored [K, COLS] (n-contiguous): (STEPS * kBK) x COLS slab kept in that order in LDS
+// ---- operand stored [K, COLS] (n-contiguous): (kSteps * kBK) x COLS slab kept in that order in LDS
 // The transpose happens on the way out of LDS: ds_read_b64_tr_b16 hands lane n of a 16-lane group
 // the four k-values of column n from a 4(k) x 16(n) block, so two of them build the 8-k fragment of
 // one column. swizzle(k row) = 4*(row%4) on the chunk index (rows of 128 bytes: 4*(row/2%2), the row's parity
 // picks the half already): the four k rows that 32 lanes read sit in four different 64-byte windows of the
 // 256-byte bank period. K rows past the operand's end are out of the buffer's range and read as zeros.
-template <typename T, int COLS, int STEPS = 1>
+template <typename T, int COLS>
 struct NTile {
     using frag_t = typename Mfma<T>::frag;
     static constexpr int kChunksPerRow = COLS / kVec128<T>;
     static constexpr int kRowsPerLoad = 64 / kChunksPerRow;  // k rows one load instruction covers
     static constexpr int kStepElems = kBK<T> * COLS;         // K step s starts at s * kStepElems
-    static constexpr int kElems = STEPS * kStepElems;
-    static constexpr int kLoads = STEPS * kBK<T> / kRowsPerLoad / kWaves;
+    static constexpr int kElems = kSteps * kStepElems;
+    static constexpr int kLoads = kSteps * kBK<T> / kRowsPerLoad / kWaves;
 
     // fp32: the four k rows a read touches lie four apart (k = 4*(lane/16) + e).
     __device__ __forceinline__ static int swizzle(int k_row) {
