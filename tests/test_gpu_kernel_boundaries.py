@@ -65,6 +65,24 @@ def test_contractions_in_k_slices_are_exact_on_integers(device, rows, fin, fout,
         assert torch.equal(got.cpu(), exact.to(dtype)), name
 
 
+@pytest.mark.parametrize("rows,fin,fout", [(33, 480, 576), (121, 192, 896), (690, 352, 512), (2837, 256, 128), (5399, 608, 640)])
+def test_fp32_gradients_of_one_call_are_as_near_to_64_bits_as_one_by_one(device, rows, fin, fout):
+    """Whatever shares a launch adds no longer chains in fp32 than the calls by themselves. The error of a sum of random terms,
+    taken over a whole gradient, varies by a few per cent from one order of additions to another of the same length (the
+    smallest gradient here has 128 elements: 1 / sqrt(2 x 128)); a chain twice as long has 1.4 times the error."""
+    g = torch.Generator(device=device).manual_seed(rows)
+    x, w, dy = (torch.randn(shape, device=device, generator=g) for shape in ((rows, fin), (fout, fin), (rows, fout)))
+    together, alone = ({name: torch.empty(shape, device=device) for name, shape in (("dX", (rows, fin)), ("dW", (fout, fin)), ("db", (fout,)))}
+                       for _ in range(2))
+    ops.linear_backward(*together.values(), dy, x, w)
+    for name in alone:
+        ops.linear_backward(*(alone[n] if n == name else None for n in alone), dy, x, w)
+    exact = {"dX": dy.double() @ w.double(), "dW": dy.double().T.contiguous() @ x.double(), "db": dy.double().sum(0)}
+    for name in ("db",):
+        off, before = ((t[name].double() - exact[name]).norm() / exact[name].norm() for t in (together, alone))
+        assert off <= 1.25 * before, (name, float(off), float(before))
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
 @pytest.mark.parametrize("rows,fin,fout", [
     *((12288, k, 4096) for k in (32, 64, 96, 160, 352)),   # 256 x 256 tiles: one K step, whole K tiles, a step more
