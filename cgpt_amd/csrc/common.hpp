@@ -244,6 +244,12 @@ int scratch(hipStream_t stream, std::size_t bytes, void** out);
 // is being captured, or the memory is not there), the call gets what the arena holds. *held: its bytes, possibly 0.
 int scratch_up_to(hipStream_t stream, std::size_t bytes, void** out, std::size_t* held);
 
+// kTickets counters bound to (current device, stream), all zero between launches: a kernel's workgroups count themselves by them
+// (the last one to end goes on with what the others left) and the last one leaves them at zero. Null where they cannot be had
+// (first asked for under capture, no memory): the caller does without.
+constexpr int kTickets = 4096;
+unsigned int* tickets(hipStream_t stream);
+
 // Identifies the block currently behind the (current device, stream) arena: it changes whenever that
 // arena is reallocated (a larger request) and reads 0 after cgptx_release_scratch. A captured graph
 // holds the block's address, so whoever replays one compares this value with the one at capture time

@@ -669,19 +669,76 @@ int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream, bo
 
 constexpr double kGroupBlocksPerUnit = 16.0;  // of a group, at most
 
+// An input and a weight gradient that gemm_pair_kernel takes together (the small kernels' groups take more).
+bool pairs(const GemmArgs* calls, int count) {
+    return count == 2 && calls[0].dtype != CGPTX_F32 && calls[0].a_k_contiguous && !calls[0].b_k_contiguous && calls[0].a_segments.count == 0 &&
+           !calls[1].a_k_contiguous && !calls[1].b_k_contiguous && calls[1].a_segments.count == 0;
+}
+long tiles_128(const GemmArgs& g) { return static_cast<long>((g.m + 127) / 128) * static_cast<long>((g.n + 127) / 128); }
+long k_steps_16bit(const GemmArgs& g) { return static_cast<long>((g.k + kBK<bf16_t> - 1) / kBK<bf16_t>); }
+// K steps of a slice: whole K tiles, as the kernels read them.
+long slice_steps(long steps, long slices) { return ((steps + slices - 1) / slices + kSteps - 1) / kSteps * kSteps; }
+
+// Predicted time of a pair in microseconds: the dispatch of its workgroups, the longer ones first, onto two slots per CU, in K steps
+// (0.22 us of a workgroup that has a CU to itself, 0.47 each of two that share one, no CU faster than 0.237 a step), 5.6 before and
+// after the K loops, and the way of the partial tiles to memory and back. Fitted to 33 shapes from 300 x 768 x 768 to 32768 x 768 x 768
+// in up to 12 slices each: within 15 per cent where it matters, the slice count it picks within 6 of the best one. Both gradients
+// of [rows, in] x out, us, calls of their own (or the small group) and a pair: 2000 x 1024 x 2048 34.3 -> 22.3, 5005 x 1024 x 1024 38.0 -> 29.6,
+// 5005 x 1024 x 2048 59.0 -> 50.3, 4096 x 768 x 2048 45.0 -> 32.5, 8192 x 1024 x 2048 74.7 -> 65.0; 1000 x 1024 x 1024 12.4 and 13.0,
+// 8192 x 256 x 256 17.0 and 20.6 (partial tiles), 16384 x 1024 x 4096 225 and 229 (256 x 256 tiles): those stay as they were.
+double predicted_pair_us(long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units) {
+    const long kt = slices > 1 ? slice_steps(steps_w, slices) : steps_w, items_w = tiles_w * slices, items = tiles_x + items_w;
+    const bool weight_first = kt >= steps_x;
+    const long counts[2] = {weight_first ? items_w : tiles_x, weight_first ? tiles_x : items_w};
+    const long lengths[2] = {weight_first ? kt : steps_x, weight_first ? steps_x : kt};
+    const double work = static_cast<double>(tiles_x * steps_x + items_w * kt) / static_cast<double>(units);
+    // K steps of the CU that ends last: of its longer slot, and of the one beside it.
+    double longest = static_cast<double>(lengths[0]), beside = 0.0;
+    if (items > 2 * units) {
+        // Slots by the steps they have been given: the least loaded ones take the next workgroups.
+        struct Slots {
+            long steps, count;
+        } slots[64] = {{0, 2 * units}};
+        int groups = 1;
+        for (int kind = 0; kind < 2; ++kind) {
+            for (long left = counts[kind]; left > 0;) {
+                int least = 0;
+                for (int i = 1; i < groups; ++i)
+                    if (slots[i].steps < slots[least].steps) least = i;
+                const long taken = std::min(left, slots[least].count), steps = slots[least].steps + lengths[kind];
+                left -= taken;
+                slots[least].count -= taken;
+                if (slots[least].count == 0) slots[least] = slots[--groups];
+                int same = 0;
+                while (same < groups && slots[same].steps != steps) ++same;
+                if (same == groups && groups < 64) slots[groups++] = {steps, 0};
+                slots[std::min(same, groups - 1)].count += taken;
+            }
+        }
+        long most = 0;
+        for (int i = 0; i < groups; ++i) most = std::max(most, slots[i].steps);
+        longest = static_cast<double>(most);
+        beside = std::min(longest, work / 2.0);
+    } else if (items > units) {
+        beside = static_cast<double>(counts[0] > units ? lengths[0] : lengths[1]);
+    }
+    const double fold = slices > 1 ? 3.0 * static_cast<double>(items_w) / static_cast<double>(units) + 0.9 * static_cast<double>(slices) : 0.0;
+    return 5.6 + std::max(0.22 * (longest - beside) + 0.47 * beside + fold, 0.237 * work);
+}
+
 // A group's tiles: those whose predicted time in one launch is least. The launch takes as long as its longest workgroup or
 // as the busiest CU's share of the work, whatever is more (us per K tile and workgroup as in predicted_us; 3.5 us before and
 // after the K loops). Two workgroups share a CU and its LDS, or, deep, each has one to itself: then the longest is not held
 // up by another, but 3.5 us of start and end of every workgroup are in nobody's shadow. Joined if that is less than the calls'
 // own predictions in turn. [M, N] x K measured apart and joined: dX and dW of 128 x 768 x 768 10.4 -> 7.4 us, of 2000 x 1024 x
 // 2048 35.7 -> 32.3; 5005 x 1024 x 256, whose dW is better split along K, 23.7 -> 28.8: stays apart.
-GemmGroup plan_group(const GemmArgs* calls, int count) {
+GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
     GemmGroup best_plan;
     const double units = static_cast<double>(compute_units());
     // Large calls are told apart by their tiles alone: whatever is spent here, they pay beside their own plans.
     double fewest = 0.0;
     for (int i = 0; i < count; ++i) fewest += static_cast<double>((calls[i].m + 63) / 64) * static_cast<double>((calls[i].n + 63) / 64);
-    if (fewest > kGroupBlocksPerUnit * units) return best_plan;
+    if (fewest > (pair ? 4.0 : 1.0) * kGroupBlocksPerUnit * units) return best_plan;
     double separate = 0.0;
     for (int i = 0; i < count; ++i) {
         const GemmArgs& g = calls[i];
@@ -694,6 +751,19 @@ GemmGroup plan_group(const GemmArgs* calls, int count) {
         if (g.a_sums != nullptr) separate += 6.0;  // two launches of their own
     }
     double best = separate;
+    if (pair) {
+        const long tiles_x = tiles_128(calls[0]), tiles_w = tiles_128(calls[1]), steps_x = k_steps_16bit(calls[0]), steps_w = k_steps_16bit(calls[1]);
+        for (long s = 1; s <= 16 && tiles_w <= kTickets && (s == 1 || steps_w / s >= 8); ++s) {
+            if (slice_steps(steps_w, s) * (s - 1) >= steps_w) continue;
+            const double time = predicted_pair_us(tiles_x, steps_x, tiles_w, steps_w, s, compute_units());
+            if (time < best) {
+                best = time;
+                best_plan.joined = best_plan.pair = true;
+                best_plan.slices = static_cast<int>(s);
+            }
+        }
+    }
+    if (fewest > kGroupBlocksPerUnit * units) return best_plan;
     for (int choice = 0; choice < 1 << count; ++choice) {
         double longest = 0.0, work = 0.0, lone_work = 0.0, blocks = 0.0;
         for (int i = 0; i < count; ++i) {
@@ -717,6 +787,7 @@ GemmGroup plan_group(const GemmArgs* calls, int count) {
         if (3.5 + std::min(one, two) < best) {
             best = 3.5 + std::min(one, two);
             best_plan.joined = true;
+            best_plan.pair = false;
             best_plan.deep = one <= two;
             for (int i = 0; i < count; ++i) best_plan.tile[i] = ((choice >> i) & 1) != 0 ? 32 : 64;
         }
@@ -755,8 +826,58 @@ bool joinable(const GemmArgs& g, KernelArgs& p) {
     return true;
 }
 
+// What a pair's weight gradient in K slices needs: partial tiles and counters.
+struct FoldRoom {
+    void* partial = nullptr;
+    unsigned int* counters = nullptr;
+    bool enough = false;
+};
+int fold_room(const GemmArgs& g, int slices, hipStream_t stream, FoldRoom* room) {
+    const std::size_t wanted = static_cast<std::size_t>(tiles_128(g)) * static_cast<std::size_t>(slices) * kFoldTileBytes;
+    room->partial = g.split_workspace;
+    std::size_t held = g.split_workspace_bytes;
+    if (!g.no_split)
+        if (int s = scratch_up_to(stream, wanted, &room->partial, &held)) return s;
+    room->counters = tickets(stream);
+    room->enough = room->partial != nullptr && held >= wanted && room->counters != nullptr;
+    return CGPTX_OK;
+}
+
+template <typename T>
+int run_pair(const GemmArgs* calls, const GemmGroup& plan, hipStream_t stream) {
+    if constexpr (std::is_same_v<T, float>) {
+        return fail(CGPTX_RUNTIME, "gemm: fp32 calls run in groups of small tiles");
+    } else {
+        PairArgs pair{};
+        for (int i = 0; i < 2; ++i) {
+            KernelArgs& p = i == 0 ? pair.input : pair.weight;
+            if (!joinable<T>(calls[i], p)) return fail(CGPTX_RUNTIME, "gemm: this call cannot be part of a group");
+            p.tiles_m = (p.m + 127) / 128;
+            p.tiles_n = (p.n + 127) / 128;
+            p.slices = 1;
+            p.k_tiles_per_slice = p.k_tiles;
+        }
+        KernelArgs& w = pair.weight;
+        const GemmArgs& g = calls[1];
+        w.a_sums = g.a_sums;
+        w.a_sums_accumulate = g.a_sums_accumulate ? 1 : 0;
+        if (plan.slices > 1) {
+            FoldRoom room;
+            if (int s = fold_room(g, plan.slices, stream, &room)) return s;
+            if (!room.enough) return fail(CGPTX_RUNTIME, "gemm: no room for the partial tiles of a pair");
+            w.fold_partial = static_cast<unsigned char*>(room.partial);
+            w.fold_tickets = room.counters;
+            w.k_tiles_per_slice = static_cast<int>(slice_steps(w.k_tiles, plan.slices));
+            w.slices = (w.k_tiles + w.k_tiles_per_slice - 1) / w.k_tiles_per_slice;
+        }
+        if constexpr (std::is_same_v<T, bf16_t>) return gemm_pair_bf16(pair, stream);
+        else return gemm_pair_f16(pair, stream);
+    }
+}
+
 template <typename T>
 int run_joined(const GemmArgs* calls, int count, const GemmGroup& plan, hipStream_t stream) {
+    if (plan.pair) return run_pair<T>(calls, plan, stream);
     SmallGroup group{};
     long order[kGroupCalls];
     for (int i = 0; i < count; ++i) order[i] = i;
@@ -787,7 +908,7 @@ int run_joined(const GemmArgs* calls, int count, const GemmGroup& plan, hipStrea
 
 }  // namespace
 
-GemmGroup gemm_joins(const GemmArgs* calls, int count) {
+GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream) {
     if (count < 2 || count > kGroupCalls || forced_tile() != 0) return {};
     for (int i = 0; i < count; ++i) {
         if (calls[i].dtype != calls[0].dtype || !valid_dtype(calls[i].dtype)) return {};
@@ -796,7 +917,16 @@ GemmGroup gemm_joins(const GemmArgs* calls, int count) {
                           : calls[i].dtype == CGPTX_F16 ? joinable<f16_t>(calls[i], p) : joinable<bf16_t>(calls[i], p);
         if (!fits) return {};
     }
-    return plan_group(calls, count);
+    const bool pair = pairs(calls, count);
+    GemmGroup group = plan_group(calls, count, pair);
+    if (group.pair && group.slices > 1) {
+        FoldRoom room;
+        if (fold_room(calls[1], group.slices, stream, &room) != CGPTX_OK || !room.enough) {
+            clear_error();
+            group = plan_group(calls, count, false);
+        }
+    }
+    return group;
 }
 
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream) {

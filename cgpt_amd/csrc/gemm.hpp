@@ -86,9 +86,11 @@ constexpr int kGroupCalls = 4;
 struct GemmGroup {
     int tile[kGroupCalls] = {};
     bool deep = false;  // one workgroup per CU
+    bool pair = false;  // an input and a weight gradient on 128 x 128 tiles, the weight gradient in `slices` along K
+    int slices = 1;
     bool joined = false;
 };
-GemmGroup gemm_joins(const GemmArgs* calls, int count);
+GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream = nullptr);
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream);
 // Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
 std::size_t gemm_split_bytes(const GemmArgs& args);

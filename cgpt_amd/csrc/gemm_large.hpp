@@ -48,6 +48,19 @@ struct KernelArgs {
     int batch_rows;
     long a_batch_stride, b_batch_stride;
     long a_seg_batch_stride[3];
+    // Calls of a pair: partial tiles of K slices and a ticket per tile (slices > 1); weight gradients: sums of A's columns, T*, or null.
+    unsigned char* fold_partial;
+    unsigned int* fold_tickets;
+    void* a_sums;
+    int a_sums_accumulate;
+};
+
+// The input and the weight gradient of a projection in one launch, on 128 x 128 tiles; each call's tiles_m, tiles_n, slices and
+// k_tiles_per_slice are set.
+constexpr int kFoldTileBytes = 128 * 128 * 4 + 128 * 4;  // of a tile's slice: accumulators, and sums of A's columns
+struct PairArgs {
+    KernelArgs input, weight;
+    int first_blocks, weight_first;  // set by the launch: the workgroups of the call that starts first
 };
 
 struct LargeCall {
@@ -61,5 +74,7 @@ struct LargeCall {
 int gemm_large_bf16(const LargeCall& call, hipStream_t stream);
 int gemm_large_f16(const LargeCall& call, hipStream_t stream);
 int gemm_large_f32(const LargeCall& call, hipStream_t stream);
+int gemm_pair_bf16(const PairArgs& pair, hipStream_t stream);
+int gemm_pair_f16(const PairArgs& pair, hipStream_t stream);
 
 }  // namespace cgptx

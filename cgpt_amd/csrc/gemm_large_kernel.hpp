@@ -87,6 +87,81 @@ __device__ __host__ __forceinline__ bool stored_as_it_is(const KernelArgs& p) {
 template <int BM, bool SPLIT, bool RESIDUAL, bool SWIGLU, bool GRAD>
 constexpr bool plain_apart = BM == 128 && !SPLIT && !RESIDUAL && !SWIGLU && !GRAD;
 
+// The K slices of a 128 x 128 tile, each in the accumulators of a workgroup: everybody leaves its own in memory, takes a ticket, and
+// the last one adds them up in slice order (whoever it is) and goes on with the sum. Written through to the memory behind the XCDs'
+// L2s and read from there: the workgroups of a tile run on any XCD. In the accumulators' own layout, 16 bytes per lane: whole
+// cache lines, and no way through LDS. The ticket is left at zero. True for the last one.
+template <typename T, int TM, int TN, bool SUMS>
+__device__ __forceinline__ bool fold_slices(const KernelArgs& p, acc_t (&acc)[TM][TN], acc_t (&column_sums)[SUMS ? TM : 1], bool sums,
+                                            int slice, int tiles, int tile, int wm, unsigned char* smem_raw) {
+    constexpr int kAgent = 16;  // sc1
+    const int lane = threadIdx.x & (kWave - 1);
+    auto rsrc_of = [&](int s) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(p.fold_partial + (static_cast<long>(s) * tiles + tile) * kFoldTileBytes, 0, kFoldTileBytes, 0x00020000);
+    };
+    const int voffset = threadIdx.x * 16, sum_voffset = 128 * 128 * 4 + (wm * 64 + lane) * 4;
+    {
+        const auto rsrc = rsrc_of(slice);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                acc_t v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float x = acc[i][j][e];
+                    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(x));
+                    v[e] = x;
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, voffset + (i * TN + j) * kThreads * 16, 0, kAgent);
+            }
+        if constexpr (SUMS) {
+            if (sums && lane < 16) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, static_cast<float>(column_sums[i][0])), rsrc, sum_voffset + i * 64, 0, kAgent);
+            }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_immediate(0));
+    __syncthreads();
+    auto* const arrived = reinterpret_cast<unsigned int*>(smem_raw);
+    if (threadIdx.x == 0) {
+        unsigned int* const ticket = p.fold_tickets + tile;
+        const unsigned int before = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (before + 1 == static_cast<unsigned int>(p.slices)) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *arrived = before;
+    }
+    __syncthreads();
+    const bool last = __builtin_amdgcn_readfirstlane(*arrived) + 1 == static_cast<unsigned int>(p.slices);
+    __syncthreads();
+    if (!last) return false;
+    for (int s = 0; s < p.slices; ++s) {
+        const auto rsrc = rsrc_of(s);
+        u32x4 part[TM][TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) part[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voffset + (i * TN + j) * kThreads * 16, 0, kAgent);
+        float sum[TM];
+        if constexpr (SUMS) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) sum[i] = sums && lane < 16 ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, sum_voffset + i * 64, 0, kAgent)) : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const acc_t v = __builtin_bit_cast(acc_t, part[i][j]);
+                if (s == 0) acc[i][j] = v;
+                else acc[i][j] += v;
+            }
+            if constexpr (SUMS) column_sums[i][0] = s == 0 ? sum[i] : column_sums[i][0] + sum[i];
+        }
+    }
+    return true;
+}
+
 // One workgroup per CU slot walks its share of the work items (output tile x K slice) one after
 // the other: the first K tiles of the next item are requested before the epilogue of the current
 // one, whose stores then drain under the next item's MFMAs.
@@ -104,9 +179,11 @@ constexpr bool plain_apart = BM == 128 && !SPLIT && !RESIDUAL && !SWIGLU && !GRA
 // PLAIN: the result is stored as it is, in the operands' type, by kernels of their own: with the general epilogue beside it the
 // compiler spills 35 - 60 scalar registers (256-wide tiles: 120 - 150) and asks for private memory that nothing touches, without
 // it 0 - 29 and none.
-template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
-          bool SWIGLU = false, bool GRAD = false, bool DEEP = false, bool PLAIN = false>
-__global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
+// FOLD: one item, whose K slice is added to the tile's others by whichever workgroup ends last (fold_slices), with the sums of A's
+// columns beside it: the two gradients of a projection in one launch (gemm_pair_kernel).
+template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL, bool SWIGLU, bool GRAD, bool DEEP,
+          bool PLAIN, bool FOLD>
+__device__ __forceinline__ void contract(const KernelArgs& p, int item, const int item_end, const int item_stride, unsigned char* smem_raw) {
     static_assert(!GRAD || (A_K && !B_K && !SPLIT && !SEGMENTED && !RESIDUAL && !SWIGLU && BN == 256),
                   "the SwiGLU gradient epilogue belongs to the plain input-gradient kernel with 256-wide tiles");
     static_assert(!SEGMENTED || (A_K && !B_K && !SPLIT && (PLAIN || BM == 256)),
@@ -114,13 +191,14 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     static_assert(!RESIDUAL || (!SPLIT && !SEGMENTED), "the residual epilogue belongs to plain unsplit kernels");
     static_assert(!SWIGLU || (A_K && B_K && !SPLIT && !SEGMENTED && !RESIDUAL && BN == 256),
                   "the SwiGLU epilogue belongs to the plain forward kernel with 256-wide tiles");
+    static_assert(!FOLD || (BM == 128 && BN == 128 && !SPLIT && !SEGMENTED && !RESIDUAL && !SWIGLU && !GRAD && !std::is_same_v<T, float>),
+                  "slices are folded in the accumulators' layout of 128 x 128 tiles");
     using frag_t = typename Mfma<T>::frag;
     using Layout = TileLayout<T, BM, BN, A_K, B_K, DEEP>;
     using ATile = typename Layout::ATile;
     using BTile = typename Layout::BTile;
     constexpr int WM = BM / 2, WN = BN / 2;
     constexpr int TM = WM / 16, TN = WN / 16;  // 16 x 16 MFMA blocks of a wavefront's part
-    extern __shared__ __align__(1024) unsigned char smem_raw[];
     T* smem = reinterpret_cast<T*>(smem_raw);
     // K tile x of A lives in A's slot x % kASlots, of B in B's slot x % kBSlots.
     constexpr int kASlots = Layout::kASlots, kBSlots = Layout::kBSlots;
@@ -131,17 +209,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int wm = wave >> 1, wn = wave & 1;
 
-    // Work items are numbered slice-major (all tiles of K slice 0, then of slice 1, ...), tiles in
-    // groups of 1 << group_rows_log2 tile-rows, down the rows first. Blocks are dealt round-robin to the 8
-    // XCDs, so XCD x takes the x-th eighth of the items and its blocks walk it side by side: the
-    // items in flight on one XCD are neighbours and share A and B panels in that XCD's L2.
     const int tiles = p.tiles_m * p.tiles_n;
-    const int items = tiles * p.slices;
-    const int per_xcd = (items + kXcds - 1) / kXcds;
-    const int item_stride = gridDim.x / kXcds;
-    const int item_end = min(items, static_cast<int>(blockIdx.x % kXcds + 1) * per_xcd);
-    int item = static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
-    if (item >= item_end) return;
 
     struct Item {
         int m0, n0, slice, kt_begin, kt_end;
@@ -327,6 +395,12 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
 #pragma unroll
     for (int j = 0; j < kBOffsets; ++j) b_off[j] = B_K ? BTile::lane_offset(lane, j) : BTile::lane_offset(lane, wn * WN + j * 16);
 
+    // FOLD, weight gradients: the sums of A's columns are one more block of columns whose B is ones, in the tiles of the first
+    // tile column.
+    constexpr bool kSums = FOLD && !A_K;
+    bool sums = false;
+    acc_t column_sums[kSums ? TM : 1];
+    frag_t ones;
     // Fragments of the K step being multiplied and of the next one: step s of a K tile is in af[s], bf[s].
     acc_t acc[TM][TN];
     frag_t af[kSteps][TM], bf[kSteps][TN];
@@ -572,7 +646,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
             }
             return;
         }
-        if constexpr (RESIDUAL) {
+        // Of a pair's calls either the result is stored as it is or C is its own residual.
+        if constexpr (RESIDUAL || (FOLD && PLAIN)) if (RESIDUAL || p.residual != nullptr) {
             const int cols_left = min(WN, c_cols - (c_col0 + col0));
             const T* out_origin = static_cast<const T*>(c_base) + static_cast<long>(row0) * c_ld + (c_col0 + col0);
             const T* res_origin = static_cast<const T*>(p.residual) + static_cast<long>(row0) * p.ldr + (w.n0 + col0);
@@ -830,6 +905,13 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
             }
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (kSums) {
+            if (sums) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) Mfma<T>::add(column_sums[i], ones, af[STEP][i]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     };
     auto next_slot = []<int SLOTS>(int slot) __attribute__((always_inline)) { return slot + 1 == SLOTS ? 0 : slot + 1; };
 
@@ -839,6 +921,13 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     // stay in scalar registers.
     Item current = locate(item);
     open(current);
+    if constexpr (kSums) {
+        sums = p.a_sums != nullptr && current.n0 == 0 && wn == 0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) column_sums[i] = acc_t(0.0f);
+#pragma unroll
+        for (int e = 0; e < static_cast<int>(sizeof(frag_t) / sizeof(T)); ++e) ones[e] = static_cast<T>(1.0f);
+    }
     request_due.template operator()<Layout::kFirstDue, 0>();
     while (true) {
         const int steps = current.kt_end - current.kt_begin;
@@ -881,6 +970,24 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
         // once they have landed and every wavefront has read its last fragments, all slots are free.
         __builtin_amdgcn_s_waitcnt(vmcnt_immediate(0));
         barrier_only();
+        if constexpr (FOLD) {
+            const int first_row = current.m0 + wm * WM + lane;  // of A's columns whose sums this lane stores, 16 apart
+            const bool last = p.slices == 1 || fold_slices<T, TM, TN, kSums>(p, acc, column_sums, sums, current.slice, tiles,
+                                                                             current.m0 / BM * p.tiles_n + current.n0 / BN, wm, smem_raw);
+            if (!last) return;
+            if constexpr (kSums) {
+                if (sums && lane < 16) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        if (first_row + i * 16 >= p.m) continue;
+                        T* out = static_cast<T*>(p.a_sums) + first_row + i * 16;
+                        *out = from_f32<T>(p.a_sums_accumulate ? column_sums[i][0] + to_f32(*out) : column_sums[i][0]);
+                    }
+                }
+            }
+            store_tile(current, false);
+            return;
+        }
         item += item_stride;
         const bool more = item < item_end;
         const Item next = locate(more ? item : item_end - 1);
@@ -891,8 +998,63 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
     }
 }
 
+template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL = false,
+          bool SWIGLU = false, bool GRAD = false, bool DEEP = false, bool PLAIN = false>
+__global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(KernelArgs p) {
+    extern __shared__ __align__(1024) unsigned char smem_raw[];
+    // Work items are numbered slice-major (all tiles of K slice 0, then of slice 1, ...), tiles in
+    // groups of 1 << group_rows_log2 tile-rows, down the rows first. Blocks are dealt round-robin to the 8
+    // XCDs, so XCD x takes the x-th eighth of the items and its blocks walk it side by side: the
+    // items in flight on one XCD are neighbours and share A and B panels in that XCD's L2.
+    const int items = p.tiles_m * p.tiles_n * p.slices;
+    const int per_xcd = (items + kXcds - 1) / kXcds;
+    const int item_end = min(items, static_cast<int>(blockIdx.x % kXcds + 1) * per_xcd);
+    const int item = static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
+    if (item >= item_end) return;
+    contract<T, BM, BN, A_K, B_K, SPLIT, SEGMENTED, RESIDUAL, SWIGLU, GRAD, DEEP, PLAIN, false>(p, item, item_end, gridDim.x / kXcds, smem_raw);
+}
+
+// Both gradients of a projection on 128 x 128 tiles in one launch, a workgroup per tile and K slice, the longer ones first. Either
+// gradient by itself leaves CUs idle (a weight gradient of 1024 x 1024 has 64 tiles, an input gradient of 5005 x 1024 320 for 256
+// CUs) and pays a launch, a pipeline fill and an epilogue of its own; a weight gradient split along K paid one more launch for its
+// partial tiles. Not persistent: the dispatcher deals the workgroups out to the two slots of a CU as they become free, and one's
+// epilogue runs beside the other's K loop. What bounds it is the path from the L2s (0.22 - 0.24 us per K step and CU), and with few
+// rounds the last one. Inputs from memory, bf16, us before and now: 2000 x 1024 x 2048 with bias, added to old gradients 32 -> 24
+// (on 64 x 64 tiles before); a block of 5 x 1001 tokens, 1024 wide, forward and backward 752 -> 699.
+template <typename T, bool DEEP, bool PLAIN>
+__global__ __launch_bounds__(kThreads, DEEP ? 1 : 2) void gemm_pair_kernel(PairArgs pair) {
+    extern __shared__ __align__(1024) unsigned char smem_raw[];
+    const int block = blockIdx.x;
+    const bool weight = (block < pair.first_blocks) == (pair.weight_first != 0);
+    const int local = block < pair.first_blocks ? block : block - pair.first_blocks;
+    auto item_of = [&](const KernelArgs& p) __attribute__((always_inline)) {
+        const int items = p.tiles_m * p.tiles_n * p.slices, per_xcd = (items + kXcds - 1) / kXcds;
+        const int within = local / kXcds, item = local % kXcds * per_xcd + within;
+        return within < per_xcd && item < items ? item : -1;
+    };
+    if (weight) {
+        const int item = item_of(pair.weight);
+        if (item < 0) return;
+        contract<T, 128, 128, false, false, false, false, false, false, false, DEEP, PLAIN, true>(pair.weight, item, item + 1, 1, smem_raw);
+    } else {
+        const int item = item_of(pair.input);
+        if (item < 0) return;
+        contract<T, 128, 128, true, false, false, false, false, false, false, DEEP, PLAIN, true>(pair.input, item, item + 1, 1, smem_raw);
+    }
+}
+
 // ------------------------------------------------------------------- host side
 constexpr int blocks_per_unit(int tile) { return tile == 256 ? 1 : 2; }  // resident blocks per CU: what the LDS slots allow
+
+// Groups of 1 << rows_log2 tile-rows, and what divides by their size.
+inline void set_groups(KernelArgs& p, int rows_log2) {
+    p.group_rows_log2 = rows_log2;
+    // x * ceil(2^32 / d) >> 32 == x / d for every x with x * d < 2^32.
+    const unsigned long divisor = (1ul << rows_log2) * static_cast<unsigned long>(p.tiles_n);
+    const unsigned long tiles = static_cast<unsigned long>(p.tiles_m) * static_cast<unsigned long>(p.tiles_n);
+    const bool exact = divisor > 1 && tiles * divisor < (1ul << 32);
+    p.group_reciprocal = exact ? static_cast<unsigned int>(((1ul << 32) + divisor - 1) / divisor) : 0u;
+}
 
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool SPLIT, bool SEGMENTED, bool RESIDUAL, bool SWIGLU, bool GRAD,
           bool DEEP, bool PLAIN>
@@ -910,19 +1072,12 @@ int launch_kernel(const KernelArgs& p, int slices, hipStream_t stream) {
     // so that every XCD gets the same number of blocks; fewer when there are fewer work items.
     KernelArgs args = p;
     args.slices = slices;
-    {
-        // x * ceil(2^32 / d) >> 32 == x / d for every x with x * d < 2^32.
-        // Tile-rows per L2 locality group. 8 (x 4 tile-columns = the 32 tiles in flight on an XCD) shares operand
-        // panels best. The SwiGLU-gradient epilogue moves four times the bytes of a plain one, two loads and two
-        // stores of whole [gate | up] rows: there the tiles in flight on an XCD are better spread along the rows
-        // (2 tile-rows x all 8 tile-columns of the training shape: 250 -> 212 us per launch; 1, 2 and 4 tile-rows
-        // measure the same, every other kernel is at its best with 8).
-        args.group_rows_log2 = GRAD ? 1 : 3;
-        const unsigned long divisor = (1ul << args.group_rows_log2) * static_cast<unsigned long>(p.tiles_n);
-        const unsigned long tiles = static_cast<unsigned long>(p.tiles_m) * static_cast<unsigned long>(p.tiles_n);
-        const bool exact = divisor > 1 && tiles * divisor < (1ul << 32);
-        args.group_reciprocal = exact ? static_cast<unsigned int>(((1ul << 32) + divisor - 1) / divisor) : 0u;
-    }
+    // Tile-rows per L2 locality group. 8 (x 4 tile-columns = the 32 tiles in flight on an XCD) shares operand
+    // panels best. The SwiGLU-gradient epilogue moves four times the bytes of a plain one, two loads and two
+    // stores of whole [gate | up] rows: there the tiles in flight on an XCD are better spread along the rows
+    // (2 tile-rows x all 8 tile-columns of the training shape: 250 -> 212 us per launch; 1, 2 and 4 tile-rows
+    // measure the same, every other kernel is at its best with 8).
+    set_groups(args, GRAD ? 1 : 3);
     const long slots = static_cast<long>(compute_units()) * blocks_per_unit(BM) / kXcds * kXcds;
     const long blocks = std::min<long>((items + kXcds - 1) / kXcds * kXcds, std::max<long>(slots, kXcds));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), smem, stream, args);
@@ -983,6 +1138,48 @@ int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream
     if (a_k && !b_k) return launch_mfma<T, BM, BN, true, false, SPLIT, false>(p, slices, stream);
     if (!a_k && !b_k) return launch_mfma<T, BM, BN, false, false, SPLIT, false>(p, slices, stream);
     return fail(CGPTX_RUNTIME, "gemm: unsupported operand layout");
+}
+
+template <typename T, bool DEEP, bool PLAIN>
+int launch_pair_kernel(const PairArgs& pair, int blocks, hipStream_t stream) {
+    constexpr int smem = std::max(TileLayout<T, 128, 128, true, false, DEEP>::kSmemBytes, TileLayout<T, 128, 128, false, false, DEEP>::kSmemBytes);
+    auto kernel = gemm_pair_kernel<T, DEEP, PLAIN>;
+    static const hipError_t status =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    CGPTX_HIP(status);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), smem, stream, pair);
+    CGPTX_LAUNCH_CHECK();
+    return CGPTX_OK;
+}
+
+template <typename T>
+int launch_pair(const PairArgs& pair_in, hipStream_t stream) {
+    PairArgs pair = pair_in;
+    long items[2];
+    int blocks[2], i = 0;
+    for (KernelArgs* p : {&pair.input, &pair.weight}) {
+        set_groups(*p, 3);
+        items[i] = static_cast<long>(p->tiles_m) * p->tiles_n * p->slices;
+        if (items[i] > std::numeric_limits<int>::max() / 4) return fail(CGPTX_OVERFLOW, "gemm: too many tiles");
+        blocks[i] = static_cast<int>((items[i] + kXcds - 1) / kXcds * kXcds);
+        ++i;
+    }
+    // C += A·B in the storage dtype: C as its own residual, see launch_layout.
+    const bool plain = !pair.input.ragged && !pair.weight.ragged;
+    if (plain) {
+        for (KernelArgs* p : {&pair.input, &pair.weight}) {
+            if (!p->accumulate) continue;
+            p->residual = p->c;
+            p->ldr = p->ldc;
+            p->accumulate = 0;
+        }
+    }
+    pair.weight_first = pair.weight.k_tiles_per_slice >= pair.input.k_tiles_per_slice ? 1 : 0;
+    pair.first_blocks = blocks[pair.weight_first];
+    const int total = blocks[0] + blocks[1];
+    const bool deep = items[0] + items[1] <= compute_units();
+    if (deep) return plain ? launch_pair_kernel<T, true, true>(pair, total, stream) : launch_pair_kernel<T, true, false>(pair, total, stream);
+    return plain ? launch_pair_kernel<T, false, true>(pair, total, stream) : launch_pair_kernel<T, false, false>(pair, total, stream);
 }
 
 template <typename T>

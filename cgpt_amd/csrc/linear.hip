@@ -252,7 +252,7 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
             apart(grad_bias, bias_bytes, grad_output, dy_bytes) && apart(grad_bias, bias_bytes, weight, w_bytes) &&
             apart(grad_bias, bias_bytes, input, x_bytes) && apart(grad_weight, w_bytes, grad_input, x_bytes) &&
             apart(grad_bias, bias_bytes, grad_input, x_bytes) && apart(grad_bias, bias_bytes, grad_weight, w_bytes)) {
-            if (const GemmGroup group = gemm_joins(calls, 2); group.joined) {
+            if (const GemmGroup group = gemm_joins(calls, 2, stream); group.joined) {
                 if (int s = gemm_joined(calls, 2, group, stream)) return s;
                 return parts != nullptr ? parts->done(LinearParts::joined) : CGPTX_OK;
             }

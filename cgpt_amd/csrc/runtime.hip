@@ -14,6 +14,7 @@ struct Arena {
     void* data = nullptr;
     std::size_t bytes = 0;
     std::uint64_t generation = 0;  // value of g_generation when this block was allocated
+    unsigned int* tickets = nullptr;
 };
 
 std::mutex g_arena_mutex;
@@ -87,6 +88,29 @@ int scratch_up_to(hipStream_t stream, std::size_t bytes, void** out, std::size_t
     return CGPTX_OK;
 }
 
+unsigned int* tickets(hipStream_t stream) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return nullptr;
+    std::lock_guard<std::mutex> lock(g_arena_mutex);
+    Arena& arena = g_arenas[{device, stream}];
+    if (arena.tickets != nullptr) return arena.tickets;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (stream != nullptr && hipStreamIsCapturing(stream, &capture) != hipSuccess) capture = hipStreamCaptureStatusActive;
+    void* fresh = nullptr;
+    constexpr std::size_t bytes = kTickets * sizeof(unsigned int);
+    if (capture != hipStreamCaptureStatusNone || hipMalloc(&fresh, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (hipMemsetAsync(fresh, 0, bytes, stream) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(fresh);
+        return nullptr;
+    }
+    arena.tickets = static_cast<unsigned int*>(fresh);
+    return arena.tickets;
+}
+
 std::uint64_t scratch_generation(hipStream_t stream) {
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return 0;
@@ -132,6 +156,7 @@ extern "C" int cgptx_release_scratch(void) {
     for (auto it = g_arenas.begin(); it != g_arenas.end();) {
         if (it->first.first == device) {
             if (it->second.data != nullptr) CGPTX_HIP(hipFree(it->second.data));
+            if (it->second.tickets != nullptr) CGPTX_HIP(hipFree(it->second.tickets));
             it = g_arenas.erase(it);
         } else {
             ++it;

@@ -749,7 +749,7 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         const GemmArgs qkv_parts[3] = {projection(a.q_pre, a.norm_a, w.q.value, N, H, QW, dt),
                                        projection(a.k_pre, a.norm_a, w.k.value, N, H, KW, dt),
                                        projection(a.v, a.norm_a, w.v.value, N, H, KW, dt)};
-        const GemmGroup qkv_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_parts, 3);
+        const GemmGroup qkv_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_parts, 3, stream);
         if (fused_qkv) {
             CGPTX_OP("gemm_fwd.qkv", qkv_forward(a.q_pre, a.k_pre, a.v, a.norm_a, w.q.value, N, H, QW, KW, dt, stream));
         } else if (qkv_group.joined) {
@@ -859,7 +859,7 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
                                            projection_weight_gradient(w.q.gradient, d_q, a.norm_a, N, H, QW, dt),
                                            projection_weight_gradient(w.k.gradient, d_k, a.norm_a, N, H, KW, dt),
                                            projection_weight_gradient(w.v.gradient, d_v, a.norm_a, N, H, KW, dt)};
-        const GemmGroup gradient_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_gradients, 4);
+        const GemmGroup gradient_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
         if (fused_qkv) {
             CGPTX_OP("gemm_dx.qkv", gemm(qkv_gradients[0], stream));
             if (!stacked)

@@ -397,3 +397,30 @@ def test_overlapping_gradients_are_written_one_after_the_other(device, behind, b
     assert torch.equal(got, shared)
     apart = {name: torch.zeros(shape, dtype=dtype, device=device) for name, shape in shapes.items()}
     assert launches(lambda: at_once(apart)) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("rows,fin,fout", [
+    (2000, 1024, 2048),                      # a workgroup per CU, one sum over K; dW's K ends inside a K tile
+    (4100, 768, 768), (5005, 1032, 288),     # dW in K slices, rows and columns that end inside a tile, an odd last slice
+    (8193, 1024, 1024),                      # more workgroups than the chip holds at once
+])
+@pytest.mark.parametrize("accumulate", [False, True], ids=["overwrite", "accumulate"])
+def test_both_gradients_on_large_tiles_share_a_launch(device, rows, fin, fout, accumulate, dtype):
+    """Small integers: exact in any order of additions. Three passes into poisoned memory: the counters by which the last
+    workgroup of a tile knows itself start each from zero."""
+    g = torch.Generator().manual_seed(rows + fin)
+    integers = lambda *shape: torch.randint(-1, 2, shape, generator=g).float()
+    x, w, dy = integers(rows, fin), integers(fout, fin), integers(rows, fout)
+    base = [integers(rows, fin), integers(fout, fin), integers(fout)]
+    want = [dy @ w, dy.T @ x, dy.sum(0)]  # whole numbers far below 2^24: exact in fp32
+    x, w, dy = (t.to(dtype).to(device) for t in (x, w, dy))
+    outputs = [torch.empty(shape, dtype=dtype, device=device) for shape in ((rows, fin), (fout, fin), (fout,))]
+    options = ops.LinearBackwardOptions(accumulate_input=accumulate, accumulate_weight=accumulate, accumulate_bias=accumulate)
+    for _ in range(3):
+        for out, old in zip(outputs, base):
+            out.copy_(old) if accumulate else out.fill_(float("nan"))
+        ops.linear_backward(*outputs, dy, x, w, options=options)
+        for name, got, exact, old in zip(("dX", "dW", "db"), outputs, want, base):
+            assert torch.equal(got.cpu(), (exact + old if accumulate else exact).to(dtype)), name
+    assert launches(lambda: ops.linear_backward(*outputs, dy, x, w, options=options)) == 1
