@@ -183,7 +183,7 @@ struct LinearParts {
 int linear_backward(void* grad_input, void* grad_weight, void* grad_bias, const void* grad_output, const void* input,
                     const void* weight, std::size_t rows, std::size_t in_features, std::size_t out_features,
                     int accumulate_input, int accumulate_weight, int accumulate_bias, int dtype, hipStream_t stream,
-                    LinearParts* parts);
+                    LinearParts* parts, bool large_pairs = true);
 
 // Per-head RMSNorm and rotary embedding of q and k in one pass over their [rows = tokens x heads, head_dim]:
 //   forward   output = rope(rmsnorm(input));   backward   output = the gradient of that, with the weight gradient.
@@ -202,13 +202,22 @@ struct NormRopeTensors {
 };
 bool rmsnorm_rope_fusable(const void* a, const void* b, const void* c, const void* weight, const void* cos_cache,
                           const void* sin_cache, std::size_t head_dim, std::size_t rotary_dim, int dtype);
+// SwiGLU on [rows, 2 hidden] = [gate | up] in the same launch: forward output[rows, hidden] = silu(gate) up, backward output[rows, 2 hidden] =
+// the gradient of [gate | up]. The bits of the operators. `swiglu_beside_norms`: whether alignment and width are served.
+struct SwigluTensors {
+    void* output;
+    const void* grad_activated;  // backward
+    const void* gate_up;
+    std::size_t rows, hidden;
+};
+bool swiglu_beside_norms(const SwigluTensors& tensors, int dtype);
 int rmsnorm_rope_forward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
                          std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
-                         std::size_t position_offset, float epsilon, int dtype, hipStream_t stream);
+                         std::size_t position_offset, float epsilon, int dtype, hipStream_t stream, const SwigluTensors* swiglu = nullptr);
 int rmsnorm_rope_backward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
                           std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
                           std::size_t position_offset, float epsilon, int dtype, hipStream_t stream,
-                          ColumnReduceSink* sink = nullptr);
+                          ColumnReduceSink* sink = nullptr, const SwigluTensors* swiglu = nullptr);
 
 // Two RMSNorms of the same rows with different weights in one pass (x is read once):
 //   forward   output_a = rmsnorm(input; weight_a), output_f = rmsnorm(input; weight_f)

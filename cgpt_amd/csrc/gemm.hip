@@ -908,7 +908,7 @@ int run_joined(const GemmArgs* calls, int count, const GemmGroup& plan, hipStrea
 
 }  // namespace
 
-GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream) {
+GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream, bool large_pairs) {
     if (count < 2 || count > kGroupCalls || forced_tile() != 0) return {};
     for (int i = 0; i < count; ++i) {
         if (calls[i].dtype != calls[0].dtype || !valid_dtype(calls[i].dtype)) return {};
@@ -917,7 +917,7 @@ GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream) {
                           : calls[i].dtype == CGPTX_F16 ? joinable<f16_t>(calls[i], p) : joinable<bf16_t>(calls[i], p);
         if (!fits) return {};
     }
-    const bool pair = pairs(calls, count);
+    const bool pair = large_pairs && pairs(calls, count);
     GemmGroup group = plan_group(calls, count, pair);
     if (group.pair && group.slices > 1) {
         FoldRoom room;

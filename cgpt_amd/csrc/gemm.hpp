@@ -80,9 +80,9 @@ struct GemmArgs {
 };
 
 int gemm(const GemmArgs& args, hipStream_t stream);
-// Up to four calls that neither read nor write each other's results, in one launch: whether that is served and faster than
+// Up to kGroupCalls calls that neither read nor write each other's results, in one launch: whether that is served and faster than
 // one after the other (few tiles each, operands that stream as they lie) and how their tiles are cut then, and the launch itself.
-constexpr int kGroupCalls = 4;
+constexpr int kGroupCalls = 6;
 struct GemmGroup {
     int tile[kGroupCalls] = {};
     bool deep = false;  // one workgroup per CU
@@ -90,7 +90,8 @@ struct GemmGroup {
     int slices = 1;
     bool joined = false;
 };
-GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream = nullptr);
+// large_pairs: whether an input and a weight gradient may share a launch on 128 x 128 tiles too.
+GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream = nullptr, bool large_pairs = true);
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream);
 // Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
 std::size_t gemm_split_bytes(const GemmArgs& args);

@@ -163,7 +163,7 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
 int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias, const void* grad_output, const void* input,
                            const void* weight, std::size_t rows, std::size_t in_features, std::size_t out_features,
                            int accumulate_input, int accumulate_weight, int accumulate_bias, int dtype, hipStream_t stream,
-                           LinearParts* parts) {
+                           LinearParts* parts, bool large_pairs) {
     if (int s = validate("linear_backward", rows, in_features, out_features, dtype)) return s;
     if (grad_output == nullptr || (grad_input != nullptr && weight == nullptr) ||
         (grad_weight != nullptr && input == nullptr))
@@ -252,7 +252,7 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
             apart(grad_bias, bias_bytes, grad_output, dy_bytes) && apart(grad_bias, bias_bytes, weight, w_bytes) &&
             apart(grad_bias, bias_bytes, input, x_bytes) && apart(grad_weight, w_bytes, grad_input, x_bytes) &&
             apart(grad_bias, bias_bytes, grad_input, x_bytes) && apart(grad_bias, bias_bytes, grad_weight, w_bytes)) {
-            if (const GemmGroup group = gemm_joins(calls, 2, stream); group.joined) {
+            if (const GemmGroup group = gemm_joins(calls, 2, stream, large_pairs); group.joined) {
                 if (int s = gemm_joined(calls, 2, group, stream)) return s;
                 return parts != nullptr ? parts->done(LinearParts::joined) : CGPTX_OK;
             }

@@ -16,6 +16,7 @@
 // read, then a column kernel over saved 1/rms.
 #include "common.hpp"
 #include "reduce.hpp"
+#include "swiglu.hpp"
 
 #include <cmath>
 #include <limits>
@@ -368,19 +369,44 @@ struct RopeRows {
     const T* w;
     int rows, heads;
 };
-template <typename T, bool Backward, bool Dense>
-__global__ __launch_bounds__(kThreads) void rmsnorm_rope_pair_kernel(RopeRows<T> q, RopeRows<T> k, int blocks_q, int hidden,
-                                                                     float inv_hidden, float eps, RopeArgs rope) {
+// SWIGLU: the workgroups behind them take the SwiGLU product of the feed-forward branch or its gradient, which neither reads nor writes
+// what the attention branch does: a step of 3 x 100 tokens gives each of the two launches 3 - 4 us for less than one of work.
+template <typename T>
+struct SwigluRows {
+    T* out;
+    const T* grad_activated;  // backward
+    const T* gate_up;
+    unsigned int rows, hidden;
+};
+// LPR: lanes per row, 16, or 32 for heads of 128 in fp32 (three launches before, q's norm, k's and the rotation: 14.4 us of a step of
+// 256 tokens in each direction and layer, now 4.8).
+template <typename T, int LPR, bool Backward, bool Dense, bool SWIGLU>
+__global__ __launch_bounds__(kThreads) void rmsnorm_rope_pair_kernel(RopeRows<T> q, RopeRows<T> k, int blocks_q, int blocks_k, int hidden,
+                                                                     float inv_hidden, float eps, RopeArgs rope, SwigluRows<T> swiglu) {
+    if constexpr (SWIGLU) {
+        const int block = static_cast<int>(blockIdx.x) - blocks_q - blocks_k, blocks = static_cast<int>(gridDim.x) - blocks_q - blocks_k;
+        if (block >= 0) {
+            const std::size_t row_elems = swiglu.hidden;
+            const unsigned int row_vectors = swiglu.hidden / kVec128<T>;
+            if constexpr (Backward)
+                swiglu_backward_vectors<T, false, false, 1>(swiglu.out, swiglu.out + row_elems, swiglu.grad_activated, swiglu.gate_up,
+                                                            swiglu.gate_up + row_elems, static_cast<std::size_t>(swiglu.rows) * row_vectors,
+                                                            row_vectors, -1, 2 * row_elems, block, blocks);
+            else
+                swiglu_forward_packed_vectors<T>(swiglu.out, swiglu.gate_up, swiglu.rows, swiglu.hidden, block, blocks);
+            return;
+        }
+    }
     const bool second = static_cast<int>(blockIdx.x) >= blocks_q;
     const int block = static_cast<int>(blockIdx.x) - (second ? blocks_q : 0);
-    const int blocks = second ? static_cast<int>(gridDim.x) - blocks_q : blocks_q;
+    const int blocks = second ? blocks_k : blocks_q;
     const RopeRows<T> of = second ? k : q;
     rope.heads = of.heads;
     if constexpr (Dense)
         rmsnorm_rope_dense<T, Backward, kRopeDenseUnroll<Backward>>(of.out, of.partial, of.dy, of.x, of.w, of.rows, inv_hidden, eps, rope,
                                                                     block, blocks);
     else
-        rmsnorm_rows<T, 16, 1, Backward, true>(of.out, of.partial, of.dy, nullptr, of.x, of.w, of.rows, hidden, inv_hidden, eps, rope,
+        rmsnorm_rows<T, LPR, 1, Backward, true>(of.out, of.partial, of.dy, nullptr, of.x, of.w, of.rows, hidden, inv_hidden, eps, rope,
                                                block, blocks);
 }
 
@@ -694,6 +720,12 @@ int validate(const void* a, const void* b, const void* c, std::size_t rows, std:
     return CGPTX_OK;
 }
 
+// Lanes per row of the norm + rotary kernels (0: not served): rows of up to 16 vectors, in fp32 of up to 32.
+template <typename T>
+int pair_lanes(int head_dim) {
+    const FastShape shape = pick_fast_shape<T>(head_dim);
+    return shape.k == 1 && (shape.lpr == 16 || (shape.lpr == 32 && std::is_same_v<T, float>)) ? shape.lpr : 0;
+}
 }  // namespace
 
 bool rmsnorm_rope_fusable(const void* a, const void* b, const void* c, const void* weight, const void* cos_cache,
@@ -702,8 +734,7 @@ bool rmsnorm_rope_fusable(const void* a, const void* b, const void* c, const voi
     const std::size_t elem = dtype_size(dtype), vec = 16 / elem;
     bool shape_ok = false;
     dispatch_dtype(dtype, [&]<typename T>() -> int {
-        const FastShape shape = pick_fast_shape<T>(static_cast<int>(head_dim));
-        shape_ok = shape.lpr == 16 && shape.k == 1;
+        shape_ok = pair_lanes<T>(static_cast<int>(head_dim)) != 0;
         return CGPTX_OK;
     });
     const auto half_aligned = [&](const void* p) { return (reinterpret_cast<std::uintptr_t>(p) % (vec / 2 * elem)) == 0; };
@@ -751,8 +782,21 @@ int run_column_reductions(const ColumnReduceEntry* table, const std::vector<Colu
 }
 
 namespace {
-// Workgroups that rows of 16 vectors fill, four rows a wavefront.
-int pair_blocks(int rows) { return static_cast<int>((static_cast<long>(rows) + 4 * kWavesPerBlock - 1) / (4 * kWavesPerBlock)); }
+// Workgroups that the rows fill, 64 / lanes of them a wavefront.
+int pair_blocks(int rows, int lanes) {
+    const long rows_per_block = kWave / lanes * kWavesPerBlock;
+    return static_cast<int>((static_cast<long>(rows) + rows_per_block - 1) / rows_per_block);
+}
+template <typename T, bool Backward>
+using PairKernel = void (*)(RopeRows<T>, RopeRows<T>, int, int, int, float, float, RopeArgs, SwigluRows<T>);
+template <typename T, bool Backward>
+PairKernel<T, Backward> pair_kernel(int lanes, bool dense, bool swiglu) {
+    if constexpr (std::is_same_v<T, float>) {
+        if (lanes == 32) return swiglu ? rmsnorm_rope_pair_kernel<T, 32, Backward, false, true> : rmsnorm_rope_pair_kernel<T, 32, Backward, false, false>;
+    }
+    if (dense) return swiglu ? rmsnorm_rope_pair_kernel<T, 16, Backward, true, true> : rmsnorm_rope_pair_kernel<T, 16, Backward, true, false>;
+    return swiglu ? rmsnorm_rope_pair_kernel<T, 16, Backward, false, true> : rmsnorm_rope_pair_kernel<T, 16, Backward, false, false>;
+}
 
 // The pair kernel's form for these rows, and how many workgroups each of the two takes: as many as in a launch of its own, up to
 // what the chip holds, since each leaves one partial sum of the weight gradient and their number is the order of its additions.
@@ -761,30 +805,51 @@ int pair_blocks(int rows) { return static_cast<int>((static_cast<long>(rows) + 4
 // 50.4 and 45.7, 38.9 and 35.0.
 template <typename T, bool Backward>
 struct PairPlan {
+    int lanes;
     bool dense;
     int blocks_q, blocks_k;
-    PairPlan(int rows_q, int rows_k, int head_dim, RopeArgs rope) : dense(rope_dense<T>(std::max(rows_q, rows_k), head_dim, rope) &&
-                                                                          rows_q % 4 == 0 && rows_k % 4 == 0) {
-        const int cap = resident_blocks(dense ? reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, true>)
-                                              : reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, Backward, false>));
-        blocks_q = std::min(pair_blocks(rows_q), cap);
-        blocks_k = std::min(pair_blocks(rows_k), cap);
+    PairPlan(int rows_q, int rows_k, int head_dim, RopeArgs rope) : lanes(pair_lanes<T>(head_dim)), dense(rope_dense<T>(std::max(rows_q, rows_k), head_dim, rope) &&
+                                                                                                         rows_q % 4 == 0 && rows_k % 4 == 0) {
+        const int cap = resident_blocks(reinterpret_cast<const void*>(pair_kernel<T, Backward>(lanes, dense, false)));
+        blocks_q = std::min(pair_blocks(rows_q, lanes), cap);
+        blocks_k = std::min(pair_blocks(rows_k, lanes), cap);
     }
 };
 template <typename T, bool Backward>
 int launch_pair(const PairPlan<T, Backward>& plan, const RopeRows<T>& q, const RopeRows<T>& k, int head_dim, float epsilon,
-                const RopeArgs& rope, hipStream_t stream) {
-    auto kernel = plan.dense ? rmsnorm_rope_pair_kernel<T, Backward, true> : rmsnorm_rope_pair_kernel<T, Backward, false>;
+                const RopeArgs& rope, const SwigluTensors* beside, hipStream_t stream) {
+    SwigluRows<T> swiglu{};
+    int blocks_s = 0;
+    if (beside != nullptr) {
+        swiglu = {static_cast<T*>(beside->output), static_cast<const T*>(beside->grad_activated), static_cast<const T*>(beside->gate_up),
+                  static_cast<unsigned int>(beside->rows), static_cast<unsigned int>(beside->hidden)};
+        const std::size_t vectors = beside->rows * (beside->hidden / kVec128<T>);
+        blocks_s = static_cast<int>(std::min<std::size_t>((vectors + kThreads - 1) / kThreads, static_cast<std::size_t>(compute_units()) * 16));
+        auto kernel = pair_kernel<T, Backward>(plan.lanes, plan.dense, true);
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(plan.blocks_q + plan.blocks_k + blocks_s)), dim3(kThreads), 0, stream, q, k,
+                           plan.blocks_q, plan.blocks_k, head_dim, 1.0f / static_cast<float>(head_dim), epsilon, rope, swiglu);
+        CGPTX_LAUNCH_CHECK();
+        return CGPTX_OK;
+    }
+    auto kernel = pair_kernel<T, Backward>(plan.lanes, plan.dense, false);
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(plan.blocks_q + plan.blocks_k)), dim3(kThreads), 0, stream, q, k,
-                       plan.blocks_q, head_dim, 1.0f / static_cast<float>(head_dim), epsilon, rope);
+                       plan.blocks_q, plan.blocks_k, head_dim, 1.0f / static_cast<float>(head_dim), epsilon, rope, swiglu);
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
 }
 }  // namespace
 
+bool swiglu_beside_norms(const SwigluTensors& s, int dtype) {
+    constexpr std::size_t limit = std::size_t{1} << 31;
+    return s.output != nullptr && s.gate_up != nullptr && is_aligned16(s.output) && is_aligned16(s.grad_activated) && is_aligned16(s.gate_up) &&
+           s.rows != 0 && s.rows < limit && s.hidden != 0 && s.hidden < limit && s.hidden % (16 / dtype_size(dtype)) == 0;
+}
+
 int rmsnorm_rope_forward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
                          std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
-                         std::size_t position_offset, float epsilon, int dtype, hipStream_t stream) {
+                         std::size_t position_offset, float epsilon, int dtype, hipStream_t stream, const SwigluTensors* swiglu) {
+    if (swiglu != nullptr && !swiglu_beside_norms(*swiglu, dtype))
+        return fail(CGPTX_INVALID_ARGUMENT, "rmsnorm_rope_forward: SwiGLU tensors that the fused pass does not serve");
     for (const NormRopeTensors* t : {&q, &k}) {
         if (int s = validate(t->output, t->input, t->weight, tokens * t->heads, head_dim, epsilon, dtype, "rmsnorm_rope_forward")) return s;
         if (cos_cache == nullptr || sin_cache == nullptr || sequence == 0 ||
@@ -799,13 +864,16 @@ int rmsnorm_rope_forward(const NormRopeTensors& q, const NormRopeTensors& k, con
                                static_cast<const T*>(t.weight), static_cast<int>(tokens * t.heads), static_cast<int>(t.heads)};
         };
         const RopeRows<T> of_q = rows(q), of_k = rows(k);
-        return launch_pair<T, false>(PairPlan<T, false>(of_q.rows, of_k.rows, h, rope), of_q, of_k, h, epsilon, rope, stream);
+        return launch_pair<T, false>(PairPlan<T, false>(of_q.rows, of_k.rows, h, rope), of_q, of_k, h, epsilon, rope, swiglu, stream);
     });
 }
 
 int rmsnorm_rope_backward(const NormRopeTensors& q, const NormRopeTensors& k, const void* cos_cache, const void* sin_cache,
                           std::size_t tokens, std::size_t head_dim, std::size_t sequence, std::size_t rotary_dim,
-                          std::size_t position_offset, float epsilon, int dtype, hipStream_t stream, ColumnReduceSink* sink) {
+                          std::size_t position_offset, float epsilon, int dtype, hipStream_t stream, ColumnReduceSink* sink,
+                          const SwigluTensors* swiglu) {
+    if (swiglu != nullptr && (!swiglu_beside_norms(*swiglu, dtype) || swiglu->grad_activated == nullptr))
+        return fail(CGPTX_INVALID_ARGUMENT, "rmsnorm_rope_backward: SwiGLU tensors that the fused pass does not serve");
     for (const NormRopeTensors* t : {&q, &k}) {
         if (int s = validate(t->output, t->grad_output, t->input, tokens * t->heads, head_dim, epsilon, dtype, "rmsnorm_rope_backward"))
             return s;
@@ -828,7 +896,7 @@ int rmsnorm_rope_backward(const NormRopeTensors& q, const NormRopeTensors& k, co
             return RopeRows<T>{static_cast<T*>(t.output), partial, static_cast<const T*>(t.grad_output), static_cast<const T*>(t.input),
                                static_cast<const T*>(t.weight), static_cast<int>(tokens * t.heads), static_cast<int>(t.heads)};
         };
-        if (int s = launch_pair<T, true>(plan, rows(q, partial_q), rows(k, partial_k), h, epsilon, rope, stream)) return s;
+        if (int s = launch_pair<T, true>(plan, rows(q, partial_q), rows(k, partial_k), h, epsilon, rope, swiglu, stream)) return s;
         if (int s = reduce_columns<T>(sink, deferred, static_cast<T*>(q.grad_weight), partial_q, plan.blocks_q, h, dtype, stream)) return s;
         return reduce_columns<T>(sink, deferred, static_cast<T*>(k.grad_weight), partial_k, plan.blocks_k, h, dtype, stream);
     });
@@ -1021,9 +1089,11 @@ std::size_t rmsnorm_backward_sink_bytes(NormPass pass, std::size_t rows, std::si
         if (pass == NormPass::with_rope) {
             // The pass picks between two kernels by properties of its rotary tables that are not known here: room
             // for whichever of them takes more. q's and k's last workgroups may both be partly filled.
-            for (const void* kernel : {reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, true, false>),
-                                       reinterpret_cast<const void*>(&rmsnorm_rope_pair_kernel<T, true, true>)})
-                blocks = std::max(blocks, std::min(pair_blocks(r) + 1, 2 * resident_blocks(kernel)));
+            const int lanes = pair_lanes<T>(h);
+            if (lanes == 0) return CGPTX_OK;
+            for (const bool dense : {false, true})
+                blocks = std::max(blocks, std::min(pair_blocks(r, lanes) + 1,
+                                                   2 * resident_blocks(reinterpret_cast<const void*>(pair_kernel<T, true>(lanes, dense, false)))));
         } else {
             const void* kernel = pass == NormPass::dual ? dual_kernel<T, true>(shape) : fast_kernel<T, true>(shape);
             if (kernel == nullptr) return CGPTX_OK;

@@ -156,6 +156,8 @@ struct cgptx_model {
     struct Timed {
         const char* label;
         hipEvent_t start, stop;
+        double share = 1.0;   // of the time between them: launches that serve several projections
+        bool borrowed = false;  // the events belong to another entry
     };
     bool profiling = false;
     std::vector<Timed> timed;
@@ -265,6 +267,32 @@ void collect(cgptx_model* m, std::vector<Parameter*>& out) {
         }                                                                       \
     } while (0)
 
+// A launch that serves two projections: its time goes to both labels, by their multiplications.
+#define CGPTX_SHARED_OP(first_label, second_label, calls, count, split, expr)                       \
+    do {                                                                                            \
+        CGPTX_OP(first_label, expr);                                                                      \
+        if (m->profiling) {                                                                         \
+            cgptx_model::Timed& first_ = m->timed.back();                                           \
+            cgptx_model::Timed second_ = first_;                                                    \
+            first_.share = share_of(calls, split, count);                                           \
+            second_.label = second_label;                                                           \
+            second_.share = 1.0 - first_.share;                                                     \
+            second_.borrowed = true;                                                                \
+            m->timed.push_back(second_);                                                            \
+        }                                                                                           \
+    } while (0)
+
+// The first `split` calls' part of the multiplications of all `count`.
+double share_of(const GemmArgs* calls, int split, int count) {
+    double first = 0.0, all = 0.0;
+    for (int i = 0; i < count; ++i) {
+        const double work = static_cast<double>(calls[i].m) * static_cast<double>(calls[i].n) * static_cast<double>(calls[i].k);
+        all += work;
+        if (i < split) first += work;
+    }
+    return first / all;
+}
+
 // The two gradients of a projection. When profiling, each launch is timed under its label: input, weight, or both in one.
 struct TimedParts final : LinearParts {
     cgptx_model* m;
@@ -298,13 +326,18 @@ constexpr const char* kDownLabels[3] = CGPTX_GRADIENT_LABELS("down");
 constexpr const char* kClassifierLabels[3] = CGPTX_GRADIENT_LABELS("classifier");
 #undef CGPTX_GRADIENT_LABELS
 
+// Steps of more rows keep the launches of an input and a weight gradient apart. Each of the two fills the chip by itself there
+// (16384 x 1024 x 1024 80 us apart, 77 in one launch; x 4096 225 and 229), and the embedding's gradient, whose additions are rounded to the
+// storage type one by one, passes on enlarged whatever other order of additions the layers above it take.
+constexpr std::size_t kPairedRows = 8192;
+
 int linear_gradients(cgptx_model* m, void* dx, void* dw, const void* dy, const void* x, const void* w, std::size_t rows,
                      std::size_t in_features, std::size_t out_features, int accumulate_input, int dt, hipStream_t stream,
-                     const char* const (&labels)[3]) {
+                     const char* const (&labels)[3], bool may_pair = true) {
     TimedParts timed(m, stream, labels);
     if (m->profiling) CGPTX_TRY(timed.start());
     return linear_backward(dx, dw, nullptr, dy, x, w, rows, in_features, out_features, accumulate_input, 0, 0, dt, stream,
-                           m->profiling ? &timed : nullptr);
+                           m->profiling ? &timed : nullptr, may_pair && rows <= kPairedRows);
 }
 
 // Y = X·Wᵀ + residual (accumulate: + Y): the block's residual additions ride in the projection's
@@ -406,6 +439,24 @@ GemmArgs projection_weight_gradient(void* grad_weight, const void* dy, const voi
     g.ldb = in_features;
     g.ldc = in_features;
     g.a_k_contiguous = false;
+    g.b_k_contiguous = false;
+    g.dtype = dt;
+    return g;
+}
+
+// dX = dY·W:
+GemmArgs projection_input_gradient(void* dx, const void* dy, const void* weight, std::size_t rows, std::size_t in_features,
+                                   std::size_t out_features, int dt) {
+    GemmArgs g;
+    g.a = dy;
+    g.b = weight;
+    g.c = dx;
+    g.m = rows;
+    g.n = in_features;
+    g.k = out_features;
+    g.lda = out_features;
+    g.ldb = in_features;
+    g.ldc = in_features;
     g.b_k_contiguous = false;
     g.dtype = dt;
     return g;
@@ -749,8 +800,20 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         const GemmArgs qkv_parts[3] = {projection(a.q_pre, a.norm_a, w.q.value, N, H, QW, dt),
                                        projection(a.k_pre, a.norm_a, w.k.value, N, H, KW, dt),
                                        projection(a.v, a.norm_a, w.v.value, N, H, KW, dt)};
-        const GemmGroup qkv_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_parts, 3, stream);
-        if (fused_qkv) {
+        // Few tokens: the attention branch's and the feed-forward branch's first projections, which read the two norms, in one
+        // launch, and the SwiGLU product beside the next one, q's and k's norms and rotations.
+        const GemmArgs first_parts[4] = {qkv_parts[0], qkv_parts[1], qkv_parts[2], projection(a.gate_up, a.norm_f, w.gate.value, N, H, 2 * I, dt)};
+        const SwigluTensors swiglu{a.act, nullptr, a.gate_up, N, I};
+        GemmArgs fused_first = first_parts[3];
+        fused_first.swiglu_out = a.act;
+        fused_first.ld_swiglu = I;
+        const bool qk_in_one = fused_qk_norm_rope(m, a.q, a.q_pre, nullptr, w.q_norm.value) && fused_qk_norm_rope(m, a.k, a.k_pre, nullptr, w.k_norm.value);
+        const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && !gemm_fuses_swiglu(fused_first) && swiglu_beside_norms(swiglu, dt);
+        const GemmGroup first_group = branches_together ? gemm_joins(first_parts, 4, stream) : GemmGroup{};
+        const GemmGroup qkv_group = fused_qkv || first_group.joined ? GemmGroup{} : gemm_joins(qkv_parts, 3, stream);
+        if (first_group.joined) {
+            CGPTX_SHARED_OP("gemm_fwd.qkv", "gemm_fwd.gate_up", first_parts, 4, 3, gemm_joined(first_parts, 4, first_group, stream));
+        } else if (fused_qkv) {
             CGPTX_OP("gemm_fwd.qkv", qkv_forward(a.q_pre, a.k_pre, a.v, a.norm_a, w.q.value, N, H, QW, KW, dt, stream));
         } else if (qkv_group.joined) {
             CGPTX_OP("gemm_fwd.qkv", gemm_joined(qkv_parts, 3, qkv_group, stream));
@@ -759,9 +822,10 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             CGPTX_OP("gemm_fwd.qkv", cgptx_linear_forward(a.k_pre, a.norm_a, w.k.value, nullptr, N, H, KW, dt, s));
             CGPTX_OP("gemm_fwd.qkv", cgptx_linear_forward(a.v, a.norm_a, w.v.value, nullptr, N, H, KW, dt, s));
         }
-        if (fused_qk_norm_rope(m, a.q, a.q_pre, nullptr, w.q_norm.value) && fused_qk_norm_rope(m, a.k, a.k_pre, nullptr, w.k_norm.value)) {
+        if (qk_in_one) {
             CGPTX_OP("rmsnorm_fwd", rmsnorm_rope_forward({a.q, a.q_pre, w.q_norm.value, HQ}, {a.k, a.k_pre, w.k_norm.value, HKV},
-                                                         m->cos_cache, m->sin_cache, N, D, m->sequence, c.rotary_dim, 0, eps, dt, stream));
+                                                         m->cos_cache, m->sin_cache, N, D, m->sequence, c.rotary_dim, 0, eps, dt, stream,
+                                                         first_group.joined ? &swiglu : nullptr));
         } else {
             CGPTX_OP("rmsnorm_fwd", cgptx_rmsnorm_forward(a.q, a.q_pre, w.q_norm.value, N * HQ, D, eps, dt, s));
             CGPTX_OP("rmsnorm_fwd", cgptx_rmsnorm_forward(a.k, a.k_pre, w.k_norm.value, N * HKV, D, eps, dt, s));
@@ -773,7 +837,8 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         // out = x + attention_projection, then out += ffn_output (src/core/transformer_block.cu:594-595)
         CGPTX_OP("gemm_fwd.o", linear_forward_residual(out, a.attn_out, w.o.value, x, false, N, QW, H, dt, stream));
         if (!dual_norms) CGPTX_OP("rmsnorm_fwd", cgptx_rmsnorm_forward(a.norm_f, x, w.ffn_norm.value, N, H, eps, dt, s));
-        if (fused_swiglu()) {
+        if (first_group.joined) {
+        } else if (fused_swiglu()) {
             CGPTX_OP("gemm_fwd.gate_up", cgptx_linear_swiglu_forward(a.gate_up, a.act, a.norm_f, w.gate.value, N, H, I, dt, s));
         } else {
             CGPTX_OP("gemm_fwd.gate_up", cgptx_linear_forward(a.gate_up, a.norm_f, w.gate.value, nullptr, N, H, 2 * I, dt, s));
@@ -817,36 +882,75 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         void* d_k = stacked ? m->d_k_all.at(reverse) : m->d_k;
         void* d_v = stacked ? m->d_v_all.at(reverse) : m->d_v;
         if (stacked) previous = m->d_hidden_slot(reverse);
-        if (fused_swiglu() && fused_swiglu_gradient()) {
-            // The SwiGLU gradient rides in the epilogue of the down projection's input gradient.
-            CGPTX_OP("gemm_dx.down", cgptx_linear_swiglu_backward(d_gate_up, m->d_act, current, w.down.value, a.gate_up, N, I, H, dt, s));
-            if (!stacked)
-                CGPTX_OP("gemm_dw.down", cgptx_linear_backward(nullptr, w.down.gradient, nullptr, current, a.act, w.down.value, N, I, H, 0, 0, 0, dt, s));
-        } else {
-            CGPTX_TRY(linear_gradients(m, m->d_act, stacked ? nullptr : w.down.gradient, current, a.act, w.down.value, N, I, H, 0, dt, stream, kDownLabels));
-            CGPTX_OP("swiglu_bwd", cgptx_swiglu_backward_packed(d_gate_up, m->d_act, a.gate_up, N, I, 0, dt, s));
-        }
         // The gradient of the residual stream collects the two norm branches: in one pass at the end of
         // the block when the shape allows (previous = current + d(ffn norm) + d(attention norm)), else as
         // they are produced (previous = current + d(ffn branch), later previous += d(attention branch)).
         const bool dual_norms = fused_block_norms(m, previous, m->d_norm_in, m->d_norm_in_f, x, current) &&
                                 is_aligned16(w.attention_norm.value) && is_aligned16(w.ffn_norm.value);
+        // Few tokens: what the two branches make of the block's output gradient in one launch (the down and the output projection's
+        // gradients), the gradient of the SwiGLU beside q's and k's norms and rotations, and the gradients of the branches' first
+        // projections in one launch again. Stacked weight gradients come at the end.
+        GemmArgs last_parts[4], first_parts[6];
+        int last_count = 0, last_down = 0, first_count = 0, first_gate_up = 0;
+        last_parts[last_count++] = projection_input_gradient(m->d_act, current, w.down.value, N, I, H, dt);
+        if (!stacked) last_parts[last_count++] = projection_weight_gradient(w.down.gradient, current, a.act, N, I, H, dt);
+        last_down = last_count;
+        last_parts[last_count++] = projection_input_gradient(m->d_attn_out, current, w.o.value, N, QW, H, dt);
+        if (!stacked) last_parts[last_count++] = projection_weight_gradient(w.o.gradient, current, a.attn_out, N, QW, H, dt);
+        first_parts[first_count++] = projection_input_gradient(m->d_norm_in_f, d_gate_up, w.gate.value, N, H, 2 * I, dt);
+        if (!stacked) first_parts[first_count++] = projection_weight_gradient(w.gate.gradient, d_gate_up, a.norm_f, N, H, 2 * I, dt);
+        first_gate_up = first_count;
+        first_parts[first_count++] = qkv_input_gradient(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt);
+        if (!stacked) {
+            first_parts[first_count++] = projection_weight_gradient(w.q.gradient, d_q, a.norm_a, N, H, QW, dt);
+            first_parts[first_count++] = projection_weight_gradient(w.k.gradient, d_k, a.norm_a, N, H, KW, dt);
+            first_parts[first_count++] = projection_weight_gradient(w.v.gradient, d_v, a.norm_a, N, H, KW, dt);
+        }
+        const SwigluTensors swiglu{d_gate_up, m->d_act, a.gate_up, N, I};
+        GemmArgs fused_last = last_parts[0];
+        fused_last.c = d_gate_up;
+        fused_last.ldc = 2 * I;
+        fused_last.swiglu_saved = a.gate_up;
+        fused_last.ld_swiglu = 2 * I;
+        const bool qk_in_one = fused_qk_norm_rope(m, d_q, d_q, a.q_pre, w.q_norm.value) && fused_qk_norm_rope(m, d_k, d_k, a.k_pre, w.k_norm.value);
+        const bool fills_chip = gemm_fuses_swiglu_gradient(fused_last);
+        const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && fused_swiglu_gradient() && !fills_chip &&
+                                       swiglu_beside_norms(swiglu, dt);
+        const GemmGroup last_group = branches_together ? gemm_joins(last_parts, last_count, stream, false) : GemmGroup{};
+        const GemmGroup first_group = last_group.joined ? gemm_joins(first_parts, first_count, stream, false) : GemmGroup{};
+        if (last_group.joined) {
+            CGPTX_SHARED_OP(stacked ? "gemm_dx.down" : "gemm_dx_dw.down", stacked ? "gemm_dx.o" : "gemm_dx_dw.o", last_parts, last_count, last_down,
+                            gemm_joined(last_parts, last_count, last_group, stream));
+        } else if (fills_chip && fused_swiglu() && fused_swiglu_gradient()) {
+            // The SwiGLU gradient rides in the epilogue of the down projection's input gradient.
+            CGPTX_OP("gemm_dx.down", cgptx_linear_swiglu_backward(d_gate_up, m->d_act, current, w.down.value, a.gate_up, N, I, H, dt, s));
+            if (!stacked)
+                CGPTX_OP("gemm_dw.down", cgptx_linear_backward(nullptr, w.down.gradient, nullptr, current, a.act, w.down.value, N, I, H, 0, 0, 0, dt, s));
+        } else {
+            // Either way the weight gradient adds up in one order.
+            CGPTX_TRY(linear_gradients(m, m->d_act, stacked ? nullptr : w.down.gradient, current, a.act, w.down.value, N, I, H, 0, dt, stream, kDownLabels, !fills_chip));
+            CGPTX_OP("swiglu_bwd", cgptx_swiglu_backward_packed(d_gate_up, m->d_act, a.gate_up, N, I, 0, dt, s));
+        }
         void* d_norm_f = dual_norms ? m->d_norm_in_f : m->d_norm_in;
-        CGPTX_TRY(linear_gradients(m, d_norm_f, stacked ? nullptr : w.gate.gradient, d_gate_up, a.norm_f, w.gate.value, N, H, 2 * I, 0, dt, stream, kGateUpLabels));
+        auto gate_up_gradients = [&]() -> int {
+            return linear_gradients(m, d_norm_f, stacked ? nullptr : w.gate.gradient, d_gate_up, a.norm_f, w.gate.value, N, H, 2 * I, 0, dt, stream, kGateUpLabels);
+        };
+        if (!last_group.joined) CGPTX_TRY(gate_up_gradients());
         if (!dual_norms) {
             CGPTX_OP("rmsnorm_bwd", rmsnorm_backward_residual(previous, w.ffn_norm.gradient, m->d_norm_in, x, w.ffn_norm.value,
                                                               current, N, H, eps, dt, stream, sink));
         }
-        CGPTX_TRY(linear_gradients(m, m->d_attn_out, stacked ? nullptr : w.o.gradient, current, a.attn_out, w.o.value, N, QW, H, 0, dt, stream, kOutputLabels));
+        if (!last_group.joined)
+            CGPTX_TRY(linear_gradients(m, m->d_attn_out, stacked ? nullptr : w.o.gradient, current, a.attn_out, w.o.value, N, QW, H, 0, dt, stream, kOutputLabels));
         CGPTX_OP("attn_bwd", cgptx_flash_gqa_attention_backward_with_lse(d_q, d_k, d_v, m->d_attn_out, a.attn_out,
                                                               a.lse, a.q, a.k, a.v, m->batch, m->sequence,
                                                               m->sequence, HQ, HKV, D, 0.0f, 1, 0, 0, dt, s));
         // In place over the attention gradients (a lane reads and writes the same elements).
-        if (fused_qk_norm_rope(m, d_q, d_q, a.q_pre, w.q_norm.value) &&
-            fused_qk_norm_rope(m, d_k, d_k, a.k_pre, w.k_norm.value)) {
+        if (qk_in_one) {
             CGPTX_OP("rmsnorm_bwd", rmsnorm_rope_backward({d_q, a.q_pre, w.q_norm.value, HQ, d_q, w.q_norm.gradient},
                                                           {d_k, a.k_pre, w.k_norm.value, HKV, d_k, w.k_norm.gradient}, m->cos_cache,
-                                                          m->sin_cache, N, D, m->sequence, c.rotary_dim, 0, eps, dt, stream, sink));
+                                                          m->sin_cache, N, D, m->sequence, c.rotary_dim, 0, eps, dt, stream, sink,
+                                                          last_group.joined ? &swiglu : nullptr));
         } else {
             CGPTX_OP("rope_bwd", cgptx_rope_backward(m->d_q_pre, m->d_k_pre, d_q, d_k, m->cos_cache, m->sin_cache, m->batch,
                                           m->sequence, HQ, HKV, D, c.rotary_dim, 0, m->sequence, dt, s));
@@ -855,12 +959,13 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             CGPTX_OP("rmsnorm_bwd", rmsnorm_backward_residual(d_k, w.k_norm.gradient, m->d_k_pre, a.k_pre, w.k_norm.value, nullptr,
                                                               N * HKV, D, eps, dt, stream, sink));
         }
-        const GemmArgs qkv_gradients[4] = {qkv_input_gradient(m->d_norm_in, d_q, d_k, d_v, w.q.value, N, H, QW, KW, dt),
-                                           projection_weight_gradient(w.q.gradient, d_q, a.norm_a, N, H, QW, dt),
-                                           projection_weight_gradient(w.k.gradient, d_k, a.norm_a, N, H, KW, dt),
-                                           projection_weight_gradient(w.v.gradient, d_v, a.norm_a, N, H, KW, dt)};
-        const GemmGroup gradient_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
-        if (fused_qkv) {
+        if (last_group.joined && !first_group.joined) CGPTX_TRY(gate_up_gradients());
+        const GemmArgs* const qkv_gradients = first_parts + first_gate_up;  // with the weights' unless those are stacked
+        const GemmGroup gradient_group = fused_qkv || first_group.joined ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
+        if (first_group.joined) {
+            CGPTX_SHARED_OP(stacked ? "gemm_dx.gate_up" : "gemm_dx_dw.gate_up", stacked ? "gemm_dx.qkv" : "gemm_dx_dw.qkv", first_parts, first_count,
+                            first_gate_up, gemm_joined(first_parts, first_count, first_group, stream));
+        } else if (fused_qkv) {
             CGPTX_OP("gemm_dx.qkv", gemm(qkv_gradients[0], stream));
             if (!stacked)
                 CGPTX_OP("gemm_dw.qkv", qkv_backward_weight(w.q.gradient, d_q, d_k, d_v, a.norm_a, N, H, QW, KW, dt, stream));
@@ -1427,8 +1532,7 @@ extern "C" int cgptx_model_profile(cgptx_model* m, float loss_scale, int loss_mo
     for (auto& t : m->timed) {
         float ms = 0.0f;
         if (status == CGPTX_OK) (void)hipEventElapsedTime(&ms, t.start, t.stop);
-        (void)hipEventDestroy(t.start);
-        (void)hipEventDestroy(t.stop);
+        ms *= static_cast<float>(t.share);
         bool found = false;
         for (auto& entry : m->profile) {
             if (entry.first == t.label) {
@@ -1437,6 +1541,11 @@ extern "C" int cgptx_model_profile(cgptx_model* m, float loss_scale, int loss_mo
             }
         }
         if (!found) m->profile.emplace_back(t.label, ms);
+    }
+    for (auto& t : m->timed) {
+        if (t.borrowed) continue;
+        (void)hipEventDestroy(t.start);
+        (void)hipEventDestroy(t.stop);
     }
     m->timed.clear();
     return status;

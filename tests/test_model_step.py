@@ -859,3 +859,34 @@ def test_block_output_is_the_residual_sum_of_its_parts(device, batch, seq):
         assert torch.isfinite(error).all()
         assert (error <= 4 * 2.0 ** -8 * torch.maximum(first.abs(), want.abs()) + 1e-3).all(), error.max().item()
     model.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("batch,seq,heads,kv_heads,head_dim,inter,layers", [
+    (3, 100, 4, 2, 64, 704, 2),   # one weight gradient per layer and projection
+    (1, 33, 2, 2, 128, 520, 2),   # all dimensions multiples of 256 but the last: stacked weight gradients in 16-bit storage
+    (2, 16, 3, 1, 32, 72, 1),
+])
+def test_branches_of_a_small_step_share_launches(device, monkeypatch, dtype, batch, seq, heads, kv_heads, head_dim, inter, layers):
+    """A few hundred tokens: the attention and the feed-forward branch's first projections run in one launch, so do the gradients
+    of their last and of their first ones, and the SwiGLU product and its gradient ride beside q's and k's norms.
+    CGPTX_FUSE_SWIGLU=0 keeps the branches apart: more launches, the same step but for the order of some sums."""
+    from cgpt_amd.model import LOSS_DENSE, Model, ModelConfig
+    from tests.util import STOL, assert_scaled_close, launches
+    config = ModelConfig(vocabulary_size=203, num_layers=layers, hidden_size=heads * head_dim, intermediate_size=inter,
+                         num_query_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, rotary_dim=head_dim, dtype=dtype)
+    rng = np.random.default_rng(batch + seq)
+    inputs, targets = (rng.integers(0, 203, size=batch * seq).astype(np.uint32) for _ in range(2))
+    results, counts = [], []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("CGPTX_FUSE_SWIGLU", fuse)
+        model = Model(config, batch, seq, seed=4, device=device)
+        model.set_tokens(inputs, targets)
+        model.forward_backward(loss_scale=4.0, loss_mode=LOSS_DENSE)
+        results.append([(name, g.clone()) for name, _, g in model.parameters()])
+        counts.append(launches(lambda: model.forward_backward(4.0, LOSS_DENSE, use_graph=False, stream=torch.cuda.current_stream())))
+        model.close()
+    assert counts[0] <= counts[1] - 3 * layers, counts
+    for (name, a), (_, b) in zip(*results):
+        assert_scaled_close(a, b, STOL[dtype], name)
