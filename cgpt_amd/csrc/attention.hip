@@ -1144,11 +1144,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_dq_wide_kernel(Params p
 // dK/dV, LDS-direct family. A block owns 128 keys of one (batch, kv-head) — 32 per
 // wavefront, K and V fragments and the two accumulator tiles in registers — and streams the 64-query
 // Q/dO tiles (plus their LSE·log2 e and delta values) of every q-head of the group through two LDS
-// stages with LDS-direct loads. Registers allow one wavefront per SIMD here; the tile is handled
-// as two 32-query halves, each as Sᵀ,dPᵀ (MFMAs with the fragment reads placed between them by
-// sched_group_barrier) | P, dS (VALU) | dV, dK (MFMAs over transposed fragment reads). Issuing one
-// half's P, dS arithmetic between the other half's MFMAs (a software pipeline over the halves, the
-// mask applied as selects) was measured 3 % slower than this plain order.
+// stages with LDS-direct loads; the tile is handled as two 32-query halves (tile_body below).
 // Key blocks are handled in pairs (i, last-i) by one block: under a causal mask block i sees
 // (last-i+1)/(last+1) of the queries, so every pair carries the same work and 256 equal blocks fill
 // 256 CUs exactly at the training shape.
@@ -1157,8 +1153,14 @@ __global__ __launch_bounds__(kThreads, 2) void attention_dq_wide_kernel(Params p
 template <int W>
 constexpr int kWideDkvSmem = 4 * kWideTile<W> * 2 + 4 * kStream * static_cast<int>(sizeof(float));
 
+// Registers allow one wavefront per SIMD with heads of 128. With heads of 64 the kernel fits 256 of them (253, none
+// spilled, operands read two slots ahead instead of four), and two wavefronts share a SIMD: there a tile's exponentials,
+// products and converts take as long as its matrix instructions, and what one wavefront cannot hide under its own falls
+// under the other's. Same order of additions, same bits. dQ and dK/dV of 8 x 4096 x 12:4 x 64, causal: 765 -> 719 us,
+// 32 x 1024: 257 -> 235, one short sequence 17.8 as before (one half after the other inside a wavefront: 734, 238 and
+// 18.4; look-ahead of one or three slots: short calls 3 % longer).
 template <typename T, int W>
-__global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params p) {
+__global__ __launch_bounds__(kThreads, W == 64 ? 2 : 1) void attention_dkv_wide_kernel(Params p) {
     using frag = typename Mma<T>::frag;
     constexpr int STEPS = W / 16, DT = W / 32;
     extern __shared__ __align__(1024) unsigned char wide_smem[];
@@ -1287,7 +1289,7 @@ __global__ __launch_bounds__(kThreads, 1) void attention_dkv_wide_kernel(Params 
         // MASKED: some (query, key) pairs of this wavefront are hidden (causal mask, keys past the end);
         // first = first visible register coordinate for this lane's key. Two separate straight-line bodies.
         auto tile_body = [&]<bool MASKED>(const T* q_tile, const T* do_tile, const float* stat, int first, const NextTile& next) {
-            constexpr int N = W / 8, kLookAhead = 4;
+            constexpr int N = W / 8, kLookAhead = W == 64 ? 2 : 4;
             acc_t s_acc[2], dp_acc[2];
             vec_t<unsigned int, 4> p_words[2][2], ds_words[2][2];  // [half][16-query step]: the k-operands of dV, dK
             vec_t<float, 4> lse_q[2][4], delta_q[2][4];
