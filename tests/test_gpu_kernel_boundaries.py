@@ -22,6 +22,8 @@ ATTENTION = [
     dict(b=64, qs=40, ks=65, hq=8, hkv=2, d=64, causal=False),          # 512 with 64-wide heads
     dict(b=65, qs=40, ks=65, hq=8, hkv=2, d=64, causal=False),
     dict(b=1, qs=390, ks=390, hq=6, hkv=2, d=128),                      # few key blocks: shared between workgroups, ragged end
+    dict(b=3, qs=330, ks=330, hq=4, hkv=2, d=64),                       # 6 (batch, kv-head) pairs: shared key blocks, no even share of the XCDs
+    dict(b=8, qs=260, ks=300, hq=8, hkv=2, d=128, off=40),              # 16 pairs: two for each XCD
 ]
 
 
