@@ -929,6 +929,15 @@ GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream, bool 
     return group;
 }
 
+bool gemm_adds_as_joined(const GemmArgs* calls, int count, hipStream_t stream) {
+    if (gemm_joins(calls, count, stream, false).joined) return true;
+    for (int i = 0; i < count; ++i) {
+        const Plan plan = make_plan(calls[i]);
+        if (plan.tile > 64 || plan.slices != 1) return false;
+    }
+    return true;
+}
+
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream) {
     if (!group.joined || count < 2 || count > kGroupCalls) return fail(CGPTX_RUNTIME, "gemm: these calls cannot share a launch");
     return dispatch_dtype(calls[0].dtype, [&]<typename T>() -> int { return run_joined<T>(calls, count, group, stream); });

@@ -93,6 +93,8 @@ struct GemmGroup {
 // large_pairs: whether an input and a weight gradient may share a launch on 128 x 128 tiles too.
 GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream = nullptr, bool large_pairs = true);
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream);
+// Whether calls by themselves, or as a group of their own, add in the order that a group gives them: small tiles, one sum over K.
+bool gemm_adds_as_joined(const GemmArgs* calls, int count, hipStream_t stream);
 // Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
 std::size_t gemm_split_bytes(const GemmArgs& args);
 // Copies [rows, cols] elements (row stride ld) to rows of `pitch` elements (whole 16-byte chunks), zeros past cols.

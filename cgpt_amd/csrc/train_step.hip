@@ -326,18 +326,17 @@ constexpr const char* kDownLabels[3] = CGPTX_GRADIENT_LABELS("down");
 constexpr const char* kClassifierLabels[3] = CGPTX_GRADIENT_LABELS("classifier");
 #undef CGPTX_GRADIENT_LABELS
 
-// Steps of more rows keep the launches of an input and a weight gradient apart. Each of the two fills the chip by itself there
-// (16384 x 1024 x 1024 80 us apart, 77 in one launch; x 4096 225 and 229), and the embedding's gradient, whose additions are rounded to the
-// storage type one by one, passes on enlarged whatever other order of additions the layers above it take.
-constexpr std::size_t kPairedRows = 8192;
-
+// A step's input and weight gradients do not share a launch of 128 x 128 tiles. Where both are small they run in a group of
+// small tiles anyway, where they are large each fills the chip by itself (16384 x 1024 x 1024 80 us apart, 77 in one launch; x 4096
+// 225 and 229; steps of 600 to 8000 tokens measured alike either way), and the embedding's gradient, whose additions are rounded to the storage
+// type one by one, passes on enlarged whatever other order of additions the layers above it take.
 int linear_gradients(cgptx_model* m, void* dx, void* dw, const void* dy, const void* x, const void* w, std::size_t rows,
                      std::size_t in_features, std::size_t out_features, int accumulate_input, int dt, hipStream_t stream,
-                     const char* const (&labels)[3], bool may_pair = true) {
+                     const char* const (&labels)[3]) {
     TimedParts timed(m, stream, labels);
     if (m->profiling) CGPTX_TRY(timed.start());
     return linear_backward(dx, dw, nullptr, dy, x, w, rows, in_features, out_features, accumulate_input, 0, 0, dt, stream,
-                           m->profiling ? &timed : nullptr, may_pair && rows <= kPairedRows);
+                           m->profiling ? &timed : nullptr, false);
 }
 
 // Y = X·Wᵀ + residual (accumulate: + Y): the block's residual additions ride in the projection's
@@ -376,8 +375,8 @@ GemmSegments qkv_segments(const void* q, const void* k, const void* v, std::size
 }
 
 // [q | k | v] = X·[Wq; Wk; Wv]ᵀ in one launch; qkv_weight is the shared [QW + 2 KW, H] block.
-int qkv_forward(void* q, void* k, void* v, const void* x, const void* qkv_weight, std::size_t rows, std::size_t H,
-                std::size_t QW, std::size_t KW, int dt, hipStream_t stream) {
+GemmArgs qkv_projection(void* q, void* k, void* v, const void* x, const void* qkv_weight, std::size_t rows, std::size_t H,
+                        std::size_t QW, std::size_t KW, int dt) {
     GemmArgs g;
     g.a = x;
     g.b = qkv_weight;
@@ -388,7 +387,7 @@ int qkv_forward(void* q, void* k, void* v, const void* x, const void* qkv_weight
     g.lda = H;
     g.ldb = H;
     g.dtype = dt;
-    return gemm(g, stream);
+    return g;
 }
 
 // dX = [dq | dk | dv]·[Wq; Wk; Wv] in one launch.
@@ -463,8 +462,8 @@ GemmArgs projection_input_gradient(void* dx, const void* dy, const void* weight,
 }
 
 // [dWq; dWk; dWv] = [dq | dk | dv]ᵀ·X in one launch.
-int qkv_backward_weight(void* qkv_gradient, const void* dq, const void* dk, const void* dv, const void* x,
-                        std::size_t rows, std::size_t H, std::size_t QW, std::size_t KW, int dt, hipStream_t stream) {
+GemmArgs qkv_weight_gradient(void* qkv_gradient, const void* dq, const void* dk, const void* dv, const void* x,
+                             std::size_t rows, std::size_t H, std::size_t QW, std::size_t KW, int dt) {
     GemmArgs g;
     g.a_segments = qkv_segments(dq, dk, dv, QW, KW);
     g.b = x;
@@ -477,7 +476,7 @@ int qkv_backward_weight(void* qkv_gradient, const void* dq, const void* dk, cons
     g.a_k_contiguous = false;
     g.b_k_contiguous = false;
     g.dtype = dt;
-    return gemm(g, stream);
+    return g;
 }
 
 // Whether the projections' weight gradients of all layers run as four launches at the end of the backward pass
@@ -800,21 +799,25 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         const GemmArgs qkv_parts[3] = {projection(a.q_pre, a.norm_a, w.q.value, N, H, QW, dt),
                                        projection(a.k_pre, a.norm_a, w.k.value, N, H, KW, dt),
                                        projection(a.v, a.norm_a, w.v.value, N, H, KW, dt)};
+        const GemmArgs fused_qkv_projection = qkv_projection(a.q_pre, a.k_pre, a.v, a.norm_a, w.q.value, N, H, QW, KW, dt);
         // Few tokens: the attention branch's and the feed-forward branch's first projections, which read the two norms, in one
-        // launch, and the SwiGLU product beside the next one, q's and k's norms and rotations.
+        // launch, and the SwiGLU product beside the next one, q's and k's norms and rotations. Only where that changes no order of
+        // additions (see linear_gradients).
         const GemmArgs first_parts[4] = {qkv_parts[0], qkv_parts[1], qkv_parts[2], projection(a.gate_up, a.norm_f, w.gate.value, N, H, 2 * I, dt)};
         const SwigluTensors swiglu{a.act, nullptr, a.gate_up, N, I};
         GemmArgs fused_first = first_parts[3];
         fused_first.swiglu_out = a.act;
         fused_first.ld_swiglu = I;
         const bool qk_in_one = fused_qk_norm_rope(m, a.q, a.q_pre, nullptr, w.q_norm.value) && fused_qk_norm_rope(m, a.k, a.k_pre, nullptr, w.k_norm.value);
-        const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && !gemm_fuses_swiglu(fused_first) && swiglu_beside_norms(swiglu, dt);
+        const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && !gemm_fuses_swiglu(fused_first) && swiglu_beside_norms(swiglu, dt) &&
+                                       gemm_adds_as_joined(fused_qkv ? &fused_qkv_projection : qkv_parts, fused_qkv ? 1 : 3, stream) &&
+                                       gemm_adds_as_joined(first_parts + 3, 1, stream);
         const GemmGroup first_group = branches_together ? gemm_joins(first_parts, 4, stream) : GemmGroup{};
         const GemmGroup qkv_group = fused_qkv || first_group.joined ? GemmGroup{} : gemm_joins(qkv_parts, 3, stream);
         if (first_group.joined) {
             CGPTX_SHARED_OP("gemm_fwd.qkv", "gemm_fwd.gate_up", first_parts, 4, 3, gemm_joined(first_parts, 4, first_group, stream));
         } else if (fused_qkv) {
-            CGPTX_OP("gemm_fwd.qkv", qkv_forward(a.q_pre, a.k_pre, a.v, a.norm_a, w.q.value, N, H, QW, KW, dt, stream));
+            CGPTX_OP("gemm_fwd.qkv", gemm(fused_qkv_projection, stream));
         } else if (qkv_group.joined) {
             CGPTX_OP("gemm_fwd.qkv", gemm_joined(qkv_parts, 3, qkv_group, stream));
         } else {
@@ -906,6 +909,8 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             first_parts[first_count++] = projection_weight_gradient(w.k.gradient, d_k, a.norm_a, N, H, KW, dt);
             first_parts[first_count++] = projection_weight_gradient(w.v.gradient, d_v, a.norm_a, N, H, KW, dt);
         }
+        const GemmArgs fused_qkv_gradients[2] = {first_parts[first_gate_up],
+                                                 qkv_weight_gradient(w.q.gradient, d_q, d_k, d_v, a.norm_a, N, H, QW, KW, dt)};
         const SwigluTensors swiglu{d_gate_up, m->d_act, a.gate_up, N, I};
         GemmArgs fused_last = last_parts[0];
         fused_last.c = d_gate_up;
@@ -914,21 +919,26 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         fused_last.ld_swiglu = 2 * I;
         const bool qk_in_one = fused_qk_norm_rope(m, d_q, d_q, a.q_pre, w.q_norm.value) && fused_qk_norm_rope(m, d_k, d_k, a.k_pre, w.k_norm.value);
         const bool fills_chip = gemm_fuses_swiglu_gradient(fused_last);
+        bool down_alike = true;  // the down projection's gradients, each by itself, add as a group would
+        for (int i = 0; i < last_down; ++i) down_alike = down_alike && gemm_adds_as_joined(last_parts + i, 1, stream);
         const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && fused_swiglu_gradient() && !fills_chip &&
-                                       swiglu_beside_norms(swiglu, dt);
+                                       swiglu_beside_norms(swiglu, dt) && down_alike &&
+                                       gemm_adds_as_joined(last_parts + last_down, last_count - last_down, stream);
+        const bool first_together = gemm_adds_as_joined(first_parts, first_gate_up, stream) && (fused_qkv
+            ? gemm_adds_as_joined(fused_qkv_gradients, 1, stream) && (stacked || gemm_adds_as_joined(fused_qkv_gradients + 1, 1, stream))
+            : gemm_adds_as_joined(first_parts + first_gate_up, first_count - first_gate_up, stream));
         const GemmGroup last_group = branches_together ? gemm_joins(last_parts, last_count, stream, false) : GemmGroup{};
-        const GemmGroup first_group = last_group.joined ? gemm_joins(first_parts, first_count, stream, false) : GemmGroup{};
+        const GemmGroup first_group = last_group.joined && first_together ? gemm_joins(first_parts, first_count, stream, false) : GemmGroup{};
         if (last_group.joined) {
             CGPTX_SHARED_OP(stacked ? "gemm_dx.down" : "gemm_dx_dw.down", stacked ? "gemm_dx.o" : "gemm_dx_dw.o", last_parts, last_count, last_down,
                             gemm_joined(last_parts, last_count, last_group, stream));
-        } else if (fills_chip && fused_swiglu() && fused_swiglu_gradient()) {
-            // The SwiGLU gradient rides in the epilogue of the down projection's input gradient.
+        } else if ((fills_chip || !down_alike) && fused_swiglu() && fused_swiglu_gradient()) {
+            // The SwiGLU gradient rides in the epilogue of the down projection's input gradient, where that fills the chip.
             CGPTX_OP("gemm_dx.down", cgptx_linear_swiglu_backward(d_gate_up, m->d_act, current, w.down.value, a.gate_up, N, I, H, dt, s));
             if (!stacked)
                 CGPTX_OP("gemm_dw.down", cgptx_linear_backward(nullptr, w.down.gradient, nullptr, current, a.act, w.down.value, N, I, H, 0, 0, 0, dt, s));
         } else {
-            // Either way the weight gradient adds up in one order.
-            CGPTX_TRY(linear_gradients(m, m->d_act, stacked ? nullptr : w.down.gradient, current, a.act, w.down.value, N, I, H, 0, dt, stream, kDownLabels, !fills_chip));
+            CGPTX_TRY(linear_gradients(m, m->d_act, stacked ? nullptr : w.down.gradient, current, a.act, w.down.value, N, I, H, 0, dt, stream, kDownLabels));
             CGPTX_OP("swiglu_bwd", cgptx_swiglu_backward_packed(d_gate_up, m->d_act, a.gate_up, N, I, 0, dt, s));
         }
         void* d_norm_f = dual_norms ? m->d_norm_in_f : m->d_norm_in;
@@ -968,7 +978,7 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         } else if (fused_qkv) {
             CGPTX_OP("gemm_dx.qkv", gemm(qkv_gradients[0], stream));
             if (!stacked)
-                CGPTX_OP("gemm_dw.qkv", qkv_backward_weight(w.q.gradient, d_q, d_k, d_v, a.norm_a, N, H, QW, KW, dt, stream));
+                CGPTX_OP("gemm_dw.qkv", gemm(fused_qkv_gradients[1], stream));
         } else if (gradient_group.joined) {
             CGPTX_OP("gemm_dx_dw.qkv", gemm_joined(qkv_gradients, 4, gradient_group, stream));
         } else {
