@@ -24,6 +24,7 @@ ATTENTION = [
     dict(b=1, qs=390, ks=390, hq=6, hkv=2, d=128),                      # few key blocks: shared between workgroups, ragged end
     dict(b=3, qs=330, ks=330, hq=4, hkv=2, d=64),                       # 6 (batch, kv-head) pairs: shared key blocks, no even share of the XCDs
     dict(b=8, qs=260, ks=300, hq=8, hkv=2, d=128, off=40),              # 16 pairs: two for each XCD
+    dict(b=30, qs=130, ks=150, hq=4, hkv=2, d=128, off=20),             # 360 blocks of 64 rows: causal blocks of 128, ragged end
 ]
 
 
@@ -45,6 +46,20 @@ def test_attention_around_the_choice_of_blocks(device, case, dtype):
         assert_scaled_close(g, w, STOL[dtype], name)
         assert_scaled_close(a, w + to_np(start), STOL[dtype], f"{name} accumulate")
     for g, again in zip(got, run_backward(device, do, q, k, v, c)):
+        assert torch.equal(g, again)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", range(len(ATTENTION)))
+def test_attention_gradients_without_saved_statistics_around_the_choice_of_blocks(device, case, dtype):
+    """The launch that makes the statistics itself, in one and in two parts: the bounds of the one that is given them."""
+    c = ATTENTION[case]
+    q, k, v, do = make_inputs(c, dtype, 900 + 10 * case)
+    want = oracle64.attention_backward(to_np(do), to_np(q), to_np(k), to_np(v), *oracle_args(c))
+    got = run_backward(device, do, q, k, v, c, with_lse=False)
+    for g, w, name in zip(got, want, ("dQ", "dK", "dV")):
+        assert_scaled_close(g, w, STOL[dtype], name)
+    for g, again in zip(got, run_backward(device, do, q, k, v, c, with_lse=False)):
         assert torch.equal(g, again)
 
 
