@@ -356,11 +356,11 @@ __global__ __launch_bounds__(kThreads) void attention_forward_kernel(Params p) {
 // x heads x width, 3 x 100 x 4:2 x 64 16.2 -> 15.3 us, 1 x 512 x 32:8 x 128 42.8 -> 42.4, 8 x 4096 x 12:4 x 64 748 -> 736,
 // 32 x 1024 x 8:2 x 128 the same. The order of additions is that of a butterfly over the row's groups of eight columns.
 template <typename T, int STEPS>
-__device__ __forceinline__ float row_delta(const typename Mma<T>::frag (&dof)[STEPS], const T* o_row, bool live, int d) {
+__device__ __forceinline__ float row_delta(const typename Mma<T>::frag (&dof)[STEPS], const typename Mma<T>::frag (&of)[STEPS]) {
     float sum[STEPS];
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
-        const auto o = vec_to_f32<T, 8>(global_frag<T>(o_row, live, s, d)), dout = vec_to_f32<T, 8>(dof[s]);
+        const auto o = vec_to_f32<T, 8>(of[s]), dout = vec_to_f32<T, 8>(dof[s]);
         sum[s] = 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) sum[s] = fmaf(dout[e], o[e], sum[s]);
@@ -370,6 +370,13 @@ __device__ __forceinline__ float row_delta(const typename Mma<T>::frag (&dof)[ST
 #pragma unroll
         for (int s = 0; s < w; ++s) sum[s] += sum[s + w];
     return sum[0] + __shfl_xor(sum[0], 32, kWave);
+}
+template <typename T, int STEPS>
+__device__ __forceinline__ float row_delta(const typename Mma<T>::frag (&dof)[STEPS], const T* o_row, bool live, int d) {
+    typename Mma<T>::frag of[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) of[s] = global_frag<T>(o_row, live, s, d);
+    return row_delta<T, STEPS>(dof, of);
 }
 
 template <typename T, int DP>
@@ -979,20 +986,34 @@ __device__ __forceinline__ void forward_block(Params p, T* lds, T* meet_at, floa
     l += other_half(l);
     if (!q_live) return;
     if constexpr (STATISTICS) {
-        delta = 0.0f;
+        // The bits of a launch that stores O and LSE and of one that reads them back. A lane has quads of O's columns, its partner
+        // in the other half of the wavefront the quads between: swapped, they are the fragments that dO comes in.
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
         const T* dout = static_cast<const T*>(p.dout) + (static_cast<long>(b) * p.qs + q_row) * q_stride + h * p.d;
+        frag dof[STEPS], of[STEPS];
 #pragma unroll
-        for (int t = 0; t < DT; ++t)
+        for (int s = 0; s < STEPS; ++s) {
+            dof[s] = global_frag<T>(dout, true, s, p.d);
+            vec_t<unsigned int, 2> quads[2];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d0 = t * 32 + g * 8 + (lane >> 5) * 4;
-                if (d0 >= p.d) continue;
-                const vec_t<float, 4> v = vec_to_f32<T, 4>(load_vec<T, 4>(dout + d0));
+            for (int i = 0; i < 2; ++i) {
+                vec_t<float, 4> v;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) delta = fmaf(v[e], o[t][4 * g + e], delta);
+                for (int e = 0; e < 4; ++e) v[e] = o[s / 2][(s % 2 * 2 + i) * 4 + e] * inv;
+                quads[i] = __builtin_bit_cast(vec_t<unsigned int, 2>, vec_from_f32<T, 4>(v));
             }
-        delta = l > 0.0f ? (delta + other_half(delta)) / l : 0.0f;
-        lse2 = mb + log2f(l);
+            vec_t<unsigned int, 4> words;
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                const auto swapped = __builtin_amdgcn_permlane32_swap(quads[0][w], quads[1][w], false, false);
+                words[w] = swapped[0];
+                words[2 + w] = swapped[1];
+            }
+            of[s] = __builtin_bit_cast(frag, words);
+        }
+        delta = row_delta<T, STEPS>(dof, of);
+        const float lse = (mb + log2f(l)) * kLn2;
+        lse2 = lse * kLog2e;
         return;
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
@@ -1023,10 +1044,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_forward_wide_kernel(Par
 // dQ, LDS-direct family: the forward kernel's streaming scheme; per 32-key half tile
 // Sᵀ = K·Qᵀ and dPᵀ = V·dOᵀ (two independent MFMA chains), dS = P∘(dP − delta) in registers,
 // dQᵀ += Kᵀ·dSᵀ with K read back transposed.
-// STATISTICS: nobody has saved the forward pass's. The workgroup walks its keys twice, first for LSE and delta; O stays in the
-// registers and is not rounded for delta. Against a forward launch into scratch before the other, backward of 1 x 512 x 32:8 x
-// 128, not causal: 52.1 -> 50.8 us, 32 x 1024 x 8:2 x 128 causal 368 -> 342, 5 x 1001 107 -> 101, 20 x 700 x 8:2 x 64 125 -> 119,
-// 3 x 100 x 4:2 x 64 19.5 -> 17.4.
+// STATISTICS: nobody has saved the forward pass's. The workgroup walks its keys twice, first for LSE and delta, O stays in the
+// registers, and the bits are those of a call that is given what the forward pass saved. Against a forward launch into scratch
+// before the other, backward of 1 x 512 x 32:8 x 128, not causal: 52.1 -> 49.7 us, 32 x 1024 x 8:2 x 128 causal 374 -> 347,
+// 5 x 1001 109 -> 100, 20 x 700 x 8:2 x 64 127 -> 119, 3 x 100 x 4:2 x 64 19.5 -> 17.1.
 template <typename T, int W, int PARTS, bool STATISTICS>
 __global__ __launch_bounds__(kThreads, 2) void attention_dq_wide_kernel(Params p) {
     using frag = typename Mma<T>::frag;

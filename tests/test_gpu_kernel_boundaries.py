@@ -52,15 +52,11 @@ def test_attention_around_the_choice_of_blocks(device, case, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("case", range(len(ATTENTION)))
 def test_attention_gradients_without_saved_statistics_around_the_choice_of_blocks(device, case, dtype):
-    """The launch that makes the statistics itself, in one and in two parts: the bounds of the one that is given them."""
+    """The launch that makes the statistics itself, in one and in two parts: the bits of the one that is given them."""
     c = ATTENTION[case]
     q, k, v, do = make_inputs(c, dtype, 900 + 10 * case)
-    want = oracle64.attention_backward(to_np(do), to_np(q), to_np(k), to_np(v), *oracle_args(c))
-    got = run_backward(device, do, q, k, v, c, with_lse=False)
-    for g, w, name in zip(got, want, ("dQ", "dK", "dV")):
-        assert_scaled_close(g, w, STOL[dtype], name)
-    for g, again in zip(got, run_backward(device, do, q, k, v, c, with_lse=False)):
-        assert torch.equal(g, again)
+    for got, want in zip(run_backward(device, do, q, k, v, c, with_lse=False), run_backward(device, do, q, k, v, c)):
+        assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
