@@ -218,13 +218,13 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma_kernel(KernelArgs p, i
 
 // ------------------------------------------------------------------- host side
 
-// CGPTX_GEMM_TILE=32|64|128|256 pins the tile size (for experiments); anything else = automatic.
+// CGPTX_GEMM_TILE=32|64|128|192|256 pins the tile size (for experiments); anything else = automatic.
 int forced_tile() {
     static const int value = [] {
         const char* text = std::getenv("CGPTX_GEMM_TILE");
         if (text == nullptr) return 0;
         const int v = std::atoi(text);
-        return (v == 32 || v == 64 || v == 128 || v == 256) ? v : 0;
+        return (v == 32 || v == 64 || v == 128 || v == 192 || v == 256) ? v : 0;
     }();
     return value;
 }
@@ -233,7 +233,11 @@ std::size_t round_up(std::size_t v, std::size_t unit) { return (v + unit - 1) / 
 
 // How a call of the streamed kernels is cut: tile, K slices per tile and K steps per slice.
 struct Plan {
-    int tile = 256;
+    int tile = 256;  // square, but 192: 256 rows of 192 columns
+    static long tiles_of(const GemmArgs& g, int tile) {
+        const std::size_t rows = tile == 192 ? 256 : tile, columns = tile;
+        return static_cast<long>((g.m + rows - 1) / rows) * static_cast<long>((g.n + columns - 1) / columns);
+    }
     int slices = 1;
     int k_tiles_per_slice = 1;
     bool deep = false;  // small tiles: all of a CU's LDS for one workgroup's stages
@@ -246,6 +250,7 @@ struct Plan {
 // through 64 MB; K tiles of 64 bytes): what a kernel costs before its K loop, plus the K loop of the busiest CU.
 //   256: one block per CU, 8.5 us for filling its pipeline and storing its tile (6.8 where the next tile's loads run under
 //        the store), 0.48 per K tile on an idle chip, 0.65 at the power limit of a full one
+//   256 x 192: one block per CU, 10 us and 7.5 for a further one, 0.40 per K tile on an idle chip, 0.55 on a full one
 //   128: 0.235 per K tile for a block that has a CU to itself, 0.17 each for two that share one where other CUs have less to
 //        do, 0.22 where all of them load at once, up to 0.245 in calls long enough to meet the power limit
 //    64: 0.09 - 0.13 per K tile with up to one block per CU, 0.11 per K tile and block with more
@@ -254,7 +259,7 @@ struct Plan {
 // as long as the fp32 matrix rate asks (0.93 per K tile of 128 x 128), smaller tiles somewhat longer for their share.
 // [M, N] x K: 128 x 768 x 768 32/1 4.4, 64/1 5.4; 1000 x 1024 x 1024 64/1 7.5, 32/1 9.5; 2000 x 2048 x 1024 128/1 13.3, 64/1
 // 17.2, 256/1 25.2; 5005 x 1024 x 1024 128/1 17.3, 256/1 25.6; 5005 x 2048 x 1024 128/1 26.4, 256/1 27.1; 16384 x 1024 x 1024
-// 256/1 31.1, 128/1 35.6; 2048 x 4096 x 4096 128/1 60.1, 256/1 77.5; 8192 x 4096 x 1024 256/1 62.5, 128/1 68.2 (tile / slices).
+// 256/1 31.1, 128/1 35.6; 32768 x 768 x 768 128/1 41.5, 192/1 44.2, 256/1 46.3; 32768 x 768 x 2048 192/1 85.3, 128/1 91.1, 256/1 91.2; 2048 x 4096 x 4096 128/1 60.1, 256/1 77.5; 8192 x 4096 x 1024 256/1 62.5, 128/1 68.2 (tile / slices).
 double predicted_us(int tile, long tiles, long slices, long k_tiles, double partial_mb, bool f32, bool a_k, bool b_k, long units) {
     const double kt = static_cast<double>((k_tiles + slices - 1) / slices);
     const double load = static_cast<double>(tiles * slices) / static_cast<double>(units);
@@ -263,6 +268,8 @@ double predicted_us(int tile, long tiles, long slices, long k_tiles, double part
     if (f32) {
         const double per_tile = tile == 32 ? 0.088 : tile == 64 ? 0.265 : 0.93;
         time = (tile == 32 ? 3.0 : tile == 64 ? 4.0 : 5.0) + kt * per_tile * (tile == 32 ? std::max(1.0, load) : blocks);
+    } else if (tile == 192) {
+        time = 10.0 + 7.5 * (blocks - 1.0) + blocks * kt * (0.40 + 0.15 * load / blocks);
     } else if (tile == 256) {
         time = 8.5 + 6.8 * (blocks - 1.0) + blocks * kt * (0.48 + 0.17 * load / blocks);
     } else if (tile == 128) {
@@ -277,15 +284,25 @@ double predicted_us(int tile, long tiles, long slices, long k_tiles, double part
     return slices > 1 ? time + 3.0 + 0.45 * partial_mb + 0.3 * std::min(partial_mb, 8.0) : time;
 }
 
+// Whether 256 x 192 tiles take a call: 16-bit storage, nothing but products, a residual, an fp32 addend and what C holds added, C
+// in one buffer on rows of whole 16 bytes.
+bool takes_narrow_tiles(const GemmArgs& g) {
+    constexpr std::size_t kMostPitch = std::size_t{1} << 21;  // 32-bit offsets within a wavefront's 128 rows of fp32
+    const std::size_t c_elem = g.c_is_f32 ? 4 : 2;
+    return g.dtype != CGPTX_F32 && g.bias == nullptr && g.a_sums == nullptr && g.swiglu_out == nullptr && g.swiglu_saved == nullptr &&
+           g.c_segments.count == 0 && g.batch_rows == 0 && (g.a_k_contiguous || (!g.b_k_contiguous && g.a_segments.count == 0)) &&
+           (g.a_segments.count == 0 || !g.b_k_contiguous) && !(g.residual != nullptr && (g.c_is_f32 || g.accumulate)) &&
+           !(g.addend_f32 != nullptr && g.c_is_f32 && g.accumulate) && g.n % 8 == 0 && (g.ldc * c_elem) % 16 == 0 && is_aligned16(g.c) &&
+           g.ldc < kMostPitch && g.ldr < kMostPitch && g.ld_addend < kMostPitch;
+}
+
 Plan make_plan(const GemmArgs& g) {
     Plan plan;
     const long units = compute_units();
     const bool f32 = g.dtype == CGPTX_F32;
     const long k_step = f32 ? kBK<float> : kBK<bf16_t>;
     const long k_tiles = (static_cast<long>(g.k) + k_step - 1) / k_step;
-    auto tiles_of = [&](long edge) {
-        return static_cast<long>((g.m + edge - 1) / edge) * static_cast<long>((g.n + edge - 1) / edge);
-    };
+    auto tiles_of = [&](int tile) { return Plan::tiles_of(g, tile); };
     const bool may_split = (!g.no_split || g.split_workspace != nullptr) && g.residual == nullptr && g.addend_f32 == nullptr &&
                            g.swiglu_out == nullptr && g.swiglu_saved == nullptr && g.c_segments.count == 0 &&
                            !(g.a_k_contiguous && g.a_segments.count > 0);
@@ -341,6 +358,12 @@ Plan make_plan(const GemmArgs& g) {
                 best_slices = s;
             }
         }
+    }
+    // 256 x 192 tiles where one sum over K on a large tile is best anyway: they add in the same order.
+    if (takes_narrow_tiles(g) && (forced == 192 || (forced == 0 && plan.tile >= 128 && best_slices == 1)) &&
+        (forced == 192 || predicted_us(192, tiles_of(192), 1, k_tiles, 0.0, f32, g.a_k_contiguous, g.b_k_contiguous, units) < best)) {
+        plan.tile = 192;
+        best_slices = 1;
     }
     set_slices(best_slices);
     plan.deep = tiles_of(plan.tile) * plan.slices <= units;
@@ -404,7 +427,8 @@ int launch_small_call(const GemmArgs& g, const KernelArgs& p, const Plan& plan, 
 
 template <typename T>
 int run_plan(const GemmArgs& g, const Plan& plan, KernelArgs p, hipStream_t stream) {
-    p.tiles_m = (p.m + plan.tile - 1) / plan.tile;
+    const int tile_rows = plan.tile == 192 ? 256 : plan.tile;
+    p.tiles_m = (p.m + tile_rows - 1) / tile_rows;
     p.tiles_n = (p.n + plan.tile - 1) / plan.tile;
     p.k_tiles_per_slice = plan.k_tiles_per_slice;
     auto launch = [&](const KernelArgs& args, bool split) -> int {
@@ -743,7 +767,7 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
     for (int i = 0; i < count; ++i) {
         const GemmArgs& g = calls[i];
         const Plan plan = make_plan(g);
-        const long tiles = static_cast<long>((g.m + plan.tile - 1) / plan.tile) * static_cast<long>((g.n + plan.tile - 1) / plan.tile);
+        const long tiles = Plan::tiles_of(g, plan.tile);
         const bool f32 = g.dtype == CGPTX_F32;
         const long k_step = f32 ? kBK<float> : kBK<bf16_t>, k_tiles = (static_cast<long>(g.k) + k_step - 1) / k_step;
         separate += predicted_us(plan.tile, tiles, plan.slices, k_tiles, static_cast<double>(plan.partial_bytes(g)) * 1e-6, f32,

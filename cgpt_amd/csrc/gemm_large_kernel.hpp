@@ -1,4 +1,4 @@
-// Persistent contraction kernels: C[M,N] (+)= op(A)·op(B) on 256 x 256 and 128 x 128 tiles.
+// Persistent contraction kernels: C[M,N] (+)= op(A)·op(B) on 256 x 256, 256 x 192 and 128 x 128 tiles.
 //
 // Design
 //   * 256 threads = 4 wavefronts in a 2x2 grid; a block owns a BM x BN tile of C
@@ -43,14 +43,24 @@
 namespace cgptx {
 namespace {
 
+// An n-contiguous operand's tile.
+template <typename T, int COLS>
+struct ColumnTile {
+    using type = NTile<T, COLS>;
+};
+template <typename T>
+struct ColumnTile<T, 192> {
+    using type = NTile192<T>;
+};
+
 // LDS holds a ring of K tiles of A and one of B (a K tile: two K steps, 128 bytes along K per row or column). Two slots of
 // each hold the K tile being multiplied and the next one, the rest what is in flight beyond them. 256 x 256 blocks own a CU
-// (3 x 32 + 2 x 32 KiB), 128 x 128 blocks run two per CU (3 x 16 + 2 x 16 KiB each) or, where there is no second one for a
+// (3 x 32 + 2 x 32 KiB; 256 x 192: 3 x 32 + 2 x 24), 128 x 128 blocks run two per CU (3 x 16 + 2 x 16 KiB each) or, where there is no second one for a
 // CU, DEEP: one with 5 + 4 slots.
 template <typename T, int BM, int BN, bool A_K, bool B_K, bool DEEP>
 struct TileLayout {
     using ATile = std::conditional_t<A_K, KTile<T, BM>, NTile<T, BM>>;
-    using BTile = std::conditional_t<B_K, KTile<T, BN>, NTile<T, BN>>;
+    using BTile = std::conditional_t<B_K, KTile<T, BN>, typename ColumnTile<T, BN>::type>;
     static constexpr int kASlots = DEEP ? 5 : 3, kBSlots = DEEP ? 4 : 2;
     static constexpr int kSmemBytes = (kASlots * ATile::kElems + kBSlots * BTile::kElems) * static_cast<int>(sizeof(T));
     // The order of an item's requests: A's K tile x is requested in the first step of K tile x + 1 - kASlots, B's in the
@@ -208,6 +218,11 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int wm = wave >> 1, wn = wave & 1;
+    // 256 x 192 tiles: a wavefront has half of the tile's first 128 columns and half of its last 64, so that each of its blocks
+    // of 16 columns lies in one part of the operand's tile and C is stored in half lines at least.
+    constexpr bool kNarrow = BN == 192;
+    static_assert(!kNarrow || (BM == 256 && !SPLIT && !RESIDUAL && !SWIGLU && !GRAD && !FOLD), "256 x 192 tiles have an epilogue of their own");
+    auto column_of = [&](int j) { return !kNarrow ? wn * WN + j * 16 : j < 4 ? wn * 64 + j * 16 : 128 + wn * 32 + (j - 4) * 16; };
 
     const int tiles = p.tiles_m * p.tiles_n;
 
@@ -336,6 +351,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
             ca.step = kWaves * a_src.group_bytes;
         }
     };
+    TileCursor cn;  // 256 x 192 tiles, B as [K, N]: its 64 columns' loads
     auto aim_b = [&](int t, TileCursor& cb) __attribute__((always_inline)) {
         const unsigned int past_end = src_begin + t * kSteps >= src_end ? 0x80000000u : 0u;
         const int k0 = min(src_begin + t * kSteps, src_end - 1) * kBK<T>;
@@ -343,6 +359,11 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
         cb.voffset = b_src.voffset;
         cb.soffset = b_src.first_offset(k0, wave) | past_end;
         cb.step = kWaves * b_src.group_bytes;
+        if constexpr (kNarrow && !B_K) {
+            cn.voffset = b_src.narrow_voffset;
+            cn.soffset = b_src.narrow_first_offset(k0, wave) | past_end;
+            cn.step = 2 * kWaves * b_src.group_bytes;
+        }
         if constexpr (SWIGLU) {
             // Two loads per unit of 64 rows: gate unit, up unit of the same rows (inter rows further), then back and 64
             // rows on.
@@ -364,6 +385,10 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     };
     auto issue_b = [&](auto index, unsigned int slot_lds, TileCursor& cb) __attribute__((always_inline)) {
         constexpr int l = decltype(index)::value;
+        if constexpr (kNarrow && !B_K && l % 3 == 2) {
+            cn.soffset = load_to_lds<l * kWaves * kLoadBytes>(cb.rsrc, slot_lds, cn.voffset, cn.soffset, cn.step);
+            return;
+        }
         const unsigned int step = !SWIGLU || l % 2 == 0 ? cb.step : l % 4 == 1 ? cb.step_up : cb.step_back;
         cb.soffset = load_to_lds<l * kWaves * kLoadBytes>(cb.rsrc, slot_lds, cb.voffset, cb.soffset, step);
     };
@@ -393,7 +418,10 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
 #pragma unroll
     for (int i = 0; i < kAOffsets; ++i) a_off[i] = A_K ? ATile::lane_offset(lane, i) : ATile::lane_offset(lane, wm * WM + i * 16);
 #pragma unroll
-    for (int j = 0; j < kBOffsets; ++j) b_off[j] = B_K ? BTile::lane_offset(lane, j) : BTile::lane_offset(lane, wn * WN + j * 16);
+    for (int j = 0; j < kBOffsets; ++j) {
+        if constexpr (kNarrow && !B_K) b_off[j] = j < 4 ? BTile::wide_offset(lane, column_of(j)) : BTile::narrow_offset(lane, column_of(j) - 128);
+        else b_off[j] = B_K ? BTile::lane_offset(lane, j) : BTile::lane_offset(lane, column_of(j));
+    }
 
     // FOLD, weight gradients: the sums of A's columns are one more block of columns whose B is ones, in the tiles of the first
     // tile column.
@@ -409,7 +437,9 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     auto read_frag = [&]<int STEP, int F>(const T* a_tile, const T* b_tile) __attribute__((always_inline)) {
         if constexpr (F >= 1 && F <= TN) {
             constexpr int j = F - 1;
-            if constexpr (B_K) bf[STEP][j] = BTile::frag(b_tile, wn * WN + j * 16, b_off[STEP]);
+            if constexpr (B_K) bf[STEP][j] = BTile::frag(b_tile, column_of(j), b_off[STEP]);
+            else if constexpr (kNarrow && j < 4) bf[STEP][j] = NTile<T, 128>::frag(b_tile + STEP * BTile::kStepElems, b_off[j]);
+            else if constexpr (kNarrow) bf[STEP][j] = NTile<T, 64>::frag(b_tile + STEP * BTile::kStepElems, b_off[j]);
             else bf[STEP][j] = BTile::frag(b_tile + STEP * BTile::kStepElems, b_off[j]);
         } else {
             constexpr int i = F == 0 ? 0 : F - TN;
@@ -431,7 +461,8 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     // over all banks.
     constexpr bool kIsF32 = std::is_same_v<T, float>;
     static_assert(!kIsF32 || (BM <= 128 && !SEGMENTED && !RESIDUAL && !SWIGLU && !GRAD), "fp32 storage has the plain kernels only");
-    constexpr int kRowBytes = WN * 2;  // fp32 values always pass in two halves
+    constexpr int kStaged = kNarrow ? 4 : TN;  // 16-bit blocks of a staged row
+    constexpr int kRowBytes = kStaged * 32;    // fp32 values always pass in two halves
     constexpr int kRowChunks = kRowBytes / 16;
     static_assert(32 * kRowBytes * kWaves <= static_cast<int>(kASlotBytes), "staging fits a slot of A");
     unsigned char* region = smem_raw + (kASlots - 1) * kASlotBytes + wave * (32 * kRowBytes);
@@ -513,7 +544,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
         // partial tiles (nothing added, fp32 out) and a residual added to a 16-bit result. Half the
         // columns are staged per pass; lane l of round u holds 8 consecutive columns (group l%8) of
         // row 8u + l/8.
-        constexpr int kGroups = WN / 2 / 8, kRowsF = kWave / kGroups, kRoundsF = 32 / kRowsF;
+        constexpr int kGroups = kStaged, kRowsF = kWave / kGroups, kRoundsF = 32 / kRowsF;
         const int f_row = lane / kGroups, f_col = (lane % kGroups) * 8;  // f_col within the staged half
         auto read_staged = [&](int u, vec_t<float, 4>& v0, vec_t<float, 4>& v1) __attribute__((always_inline)) {
             const int row = u * kRowsF + f_row;
@@ -538,6 +569,79 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
             return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(origin), 0, static_cast<int>(extent), 0x00020000);
         };
         const int rows_left = min(WM, p.m - row0);
+        if constexpr (kNarrow) {
+            // 32 columns at a time through fp32 staging, 8 consecutive ones of row 16u + l/4 to lane l in round u. What is added is
+            // requested one pass ahead.
+            const int cols_left = min(BN, p.n - w.n0);
+            const int c_elem = p.c_f32 ? 4 : static_cast<int>(sizeof(T)), c_row_bytes = static_cast<int>(p.ldc) * c_elem;
+            char* const c_origin = static_cast<char*>(p.c) + (static_cast<long>(row0) * p.ldc + w.n0) * c_elem;
+            const __amdgpu_buffer_rsrc_t out_rsrc = part_rsrc(c_origin, p.ldc, c_elem, rows_left, cols_left);
+            // fp32: the addend, or the old C of an fp32 result; 16 bits: the residual, or the old C of a 16-bit result.
+            const bool old_f32 = p.c_f32 && p.accumulate, old_16 = !p.c_f32 && p.accumulate;
+            const bool adds_f32 = p.addend != nullptr || old_f32, adds_16 = p.residual != nullptr || old_16;
+            const long f32_ld = p.addend != nullptr ? p.ld_addend : p.ldc, ld_16 = p.residual != nullptr ? p.ldr : p.ldc;
+            const float* f32_origin = (p.addend != nullptr ? p.addend : static_cast<const float*>(p.c)) + static_cast<long>(row0) * f32_ld + w.n0;
+            const T* origin_16 = static_cast<const T*>(p.residual != nullptr ? p.residual : p.c) + static_cast<long>(row0) * ld_16 + w.n0;
+            const __amdgpu_buffer_rsrc_t f32_rsrc = part_rsrc(f32_origin, f32_ld, 4, rows_left, cols_left);
+            const __amdgpu_buffer_rsrc_t rsrc_16 = part_rsrc(origin_16, ld_16, sizeof(T), rows_left, cols_left);
+            const int n_row = lane / 4, n_col = (lane % 4) * 8;
+            constexpr int kPasses = kRowBlocks * 3;
+            u32x4 ahead_f32[2][2][2], ahead_16[2][2];
+            auto column = [&](int q) { return (q % 3 < 2 ? wn * 64 + q % 3 * 32 : 128 + wn * 32) + n_col; };
+            auto voffset_of = [&](int q, long ld, int elem) {
+                return column(q) < cols_left ? n_row * static_cast<int>(ld) * elem + column(q) * elem : std::numeric_limits<int>::min();
+            };
+            auto request_added = [&](int q) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int row = q / 3 * 32 + u * 16;
+                    if (adds_f32) {
+                        const int voffset = voffset_of(q, f32_ld, 4), soffset = row * static_cast<int>(f32_ld) * 4;
+                        ahead_f32[q & 1][u][0] = __builtin_amdgcn_raw_buffer_load_b128(f32_rsrc, voffset, soffset, 0);
+                        ahead_f32[q & 1][u][1] = __builtin_amdgcn_raw_buffer_load_b128(f32_rsrc, voffset + 16, soffset, 0);
+                    }
+                    if (adds_16)
+                        ahead_16[q & 1][u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_16, voffset_of(q, ld_16, sizeof(T)),
+                                                                                  row * static_cast<int>(ld_16) * static_cast<int>(sizeof(T)), 0);
+                }
+            };
+            request_added(0);
+#pragma unroll
+            for (int q = 0; q < kPasses; ++q) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (q % 3 == 0 && request) request_share(q / 3);
+                if (q + 1 < kPasses) request_added(q + 1);
+                stage.template operator()<float, 2>(q / 3, q % 3 * 2);
+                const int voffset = voffset_of(q, p.ldc, c_elem);
+                vec_t<float, 4> v[2][2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const int row = u * 16 + n_row;
+                        v[u][c] = *reinterpret_cast<const vec_t<float, 4>*>(region + row * kRowBytes + (((n_col / 4 + c) ^ sw(row)) * 16));
+                    }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    if (adds_f32) {
+                        v[u][0] += __builtin_bit_cast(acc_t, ahead_f32[q & 1][u][0]);
+                        v[u][1] += __builtin_bit_cast(acc_t, ahead_f32[q & 1][u][1]);
+                    }
+                    vec_t<float, 8> sum;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) sum[e] = v[u][e / 4][e % 4];
+                    if (adds_16) sum += vec_to_f32<T, 8>(__builtin_bit_cast(vec_t<T, 8>, ahead_16[q & 1][u]));
+                    const int soffset = (q / 3 * 32 + u * 16) * c_row_bytes;
+                    if (p.c_f32) {
+                        store_chunk(__builtin_bit_cast(u32x4, v[u][0]), out_rsrc, voffset, soffset);
+                        store_chunk(__builtin_bit_cast(u32x4, v[u][1]), out_rsrc, voffset + 16, soffset);
+                    } else {
+                        store_chunk(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(sum)), out_rsrc, voffset, soffset);
+                    }
+                }
+            }
+            return;
+        }
         if constexpr (SWIGLU) {
             // The wavefront's 128 staged columns are gate g0 .. g0+63 and up g0 .. g0+63. Lane l of
             // round u takes 8 gate and the 8 matching up values of row 8u + l/8 from the staging
@@ -558,7 +662,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
             for (int r = 0; r < kRowBlocks; ++r) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (request) request_share(r);
-                stage.template operator()<T, TN>(r, 0);
+                stage.template operator()<T, kStaged>(r, 0);
                 u32x4 gate[kRoundsF], up[kRoundsF];
 #pragma unroll
                 for (int u = 0; u < kRoundsF; ++u) {
@@ -620,7 +724,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                 __builtin_amdgcn_sched_barrier(0);
                 if (request) request_share(r);
                 if (r + 1 < kRowBlocks) request_saved(r + 1, ahead[(r + 1) & 1]);
-                stage.template operator()<T, TN>(r, 0);
+                stage.template operator()<T, kStaged>(r, 0);
                 u32x4 data[kRounds];
 #pragma unroll
                 for (int u = 0; u < kRounds; ++u) {
@@ -677,7 +781,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                 if (r + 1 < kRowBlocks) request_residual(r + 1, ahead[(r + 1) & 1]);
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
-                    stage.template operator()<float, TN / 2>(r, half * (TN / 2));
+                    stage.template operator()<float, kStaged / 2>(r, half * (kStaged / 2));
                     const int col = half * (WN / 2) + f_col;
                     const int voffset = col < cols_left ? f_row * out_row_bytes + col * static_cast<int>(sizeof(T))
                                                         : std::numeric_limits<int>::min();
@@ -725,7 +829,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                 // would not fit the vector registers.
                 __builtin_amdgcn_sched_barrier(0);
                 if (request) request_share(r);
-                stage.template operator()<T, TN>(r, 0);
+                stage.template operator()<T, kStaged>(r, 0);
                 u32x4 data[kRounds];
 #pragma unroll
                 for (int u = 0; u < kRounds; ++u) {
@@ -752,7 +856,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                 if (request) request_share(r);
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
-                    stage.template operator()<float, TN / 2>(r, half * (TN / 2));
+                    stage.template operator()<float, kStaged / 2>(r, half * (kStaged / 2));
                     const int col = half * (WN / 2) + l_col;
                     constexpr int kSecond = kGroups * 4;  // columns between a lane's two quads
                     const int voffset0 = col < cols_left ? f_row * row_bytes + col * 4 : std::numeric_limits<int>::min();
@@ -773,7 +877,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
         if (p.ragged) {
             // Rows of C that do not start on 16-byte boundaries: lanes along the columns of a staged half, one element
             // each, so that a store instruction still covers one contiguous piece of a row (or of a few).
-            constexpr int kCols = WN / 2, kRowsE = kWave / kCols;
+            constexpr int kCols = kStaged * 8, kRowsE = kWave / kCols;
             const int e_row = lane / kCols, e_col = lane % kCols;
 #pragma unroll
             for (int r = 0; r < kRowBlocks; ++r) {
@@ -781,7 +885,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                 if (request) request_share(r);
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
-                    stage.template operator()<float, TN / 2>(r, half * (TN / 2));
+                    stage.template operator()<float, kStaged / 2>(r, half * (kStaged / 2));
                     const int col = half * kCols + e_col, n = w.n0 + col0 + col, c_col = c_col0 + col0 + col;
                     const float bias = p.bias != nullptr && c_col < c_cols ? to_f32(static_cast<const T*>(p.bias)[n]) : 0.0f;
 #pragma unroll 4
@@ -811,7 +915,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
             if (request) request_share(r);
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
-                pass.template operator()<float, TN / 2>(r, half * (TN / 2), [&](int, int row, int col, const unsigned char* lo,
+                pass.template operator()<float, kStaged / 2>(r, half * (kStaged / 2), [&](int, int row, int col, const unsigned char* lo,
                                                                               const unsigned char* hi) {
                     const int m = row0 + row, n = w.n0 + col0 + col, c_col = c_col0 + col0 + col;
                     vec_t<float, 4> v0 = *reinterpret_cast<const vec_t<float, 4>*>(lo);
@@ -880,7 +984,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     // every MFMA is followed by its share of the loads and fragment reads and a scheduling fence keeps them there. A
     // wavefront's load instruction keeps it from issuing for about as long as an MFMA runs.
     constexpr int kMfmas = TM * TN;
-    constexpr int kReadEvery = kMfmas / kFrags >= 4 ? 3 : 1;  // MFMAs between fragment reads
+    constexpr int kReadEvery = kMfmas / kFrags >= 3 ? 3 : 1;  // MFMAs between fragment reads
     static_assert(kReadEvery * kFrags <= kMfmas && kALoads <= kMfmas && kBLoads <= kMfmas, "a step has room for its reads and loads");
     // STEP 0: a_tile, b_tile are K tile t's; STEP 1: K tile t+1's. slot_lds: where the step's loads go.
     auto multiply_step = [&]<int STEP, bool FIRST>(int t, const T* a_tile, const T* b_tile, unsigned int slot_lds) __attribute__((always_inline)) {
@@ -1140,6 +1244,28 @@ int launch_layout(const KernelArgs& p, bool a_k, bool b_k, int slices, hipStream
     return fail(CGPTX_RUNTIME, "gemm: unsupported operand layout");
 }
 
+// 256 x 192 tiles (call.tile 192): for results whose columns are not near a multiple of 256, or whose 256 x 256 tiles leave part of the
+// last round of CUs idle. 768 columns are three tiles of 256, 192 of them for 16384 rows, and four of 192, 256 of them. Same sums in
+// the same order. The K loop is 0.77 of a 256 x 256 tile's (48 MFMAs a step for 64, 56 KiB of operands a K tile for 64); that a
+// filled chip runs at a lower clock than one of which a quarter idles takes most of the rest. us, 256 and 192 columns: 16384 x 768 x
+// 32000 626 -> 587, 32000 x 768 x 16384 (weight gradient) 661 -> 630, 32768 x 768 x 4096 172 -> 159, 32768 x 768 x 2048 91 -> 85;
+// 32768 x 768 x 768 46 -> 44 (128 x 128: 41.5), 32768 x 960 x 960 56 -> 70. The step of 8 x 4096 tokens, 768 wide, 10294 -> 10002.
+template <typename T>
+int launch_narrow(const LargeCall& call, hipStream_t stream) {
+    const KernelArgs& p = call.args;
+    const bool a_k = call.a_k_contiguous, b_k = call.b_k_contiguous;
+    if (call.split || p.bias != nullptr || p.ragged || p.act != nullptr || p.saved != nullptr || p.c_seg.count > 0 || p.batch_rows > 0)
+        return fail(CGPTX_RUNTIME, "gemm: 256 x 192 tiles take plain products");
+    if (a_k && p.a_seg.count > 0) {
+        if (b_k) return fail(CGPTX_RUNTIME, "gemm: an operand in segments along K is that of an input gradient");
+        return launch_kernel<T, 256, 192, true, false, false, true, false, false, false, false, false>(p, 1, stream);
+    }
+    if (a_k && b_k) return launch_kernel<T, 256, 192, true, true, false, false, false, false, false, false, false>(p, 1, stream);
+    if (a_k) return launch_kernel<T, 256, 192, true, false, false, false, false, false, false, false, false>(p, 1, stream);
+    if (!b_k) return launch_kernel<T, 256, 192, false, false, false, false, false, false, false, false, false>(p, 1, stream);
+    return fail(CGPTX_RUNTIME, "gemm: unsupported operand layout");
+}
+
 template <typename T, bool DEEP, bool PLAIN>
 int launch_pair_kernel(const PairArgs& pair, int blocks, hipStream_t stream) {
     constexpr int smem = std::max(TileLayout<T, 128, 128, true, false, DEEP>::kSmemBytes, TileLayout<T, 128, 128, false, false, DEEP>::kSmemBytes);
@@ -1190,6 +1316,7 @@ int launch_large(const LargeCall& call, hipStream_t stream) {
     };
     if constexpr (!std::is_same_v<T, float>) {
         if (call.tile == 256) return with_tile.template operator()<256>();
+        if (call.tile == 192) return launch_narrow<T>(call, stream);
     }
     return with_tile.template operator()<128>();
 }

@@ -315,5 +315,44 @@ struct NTile {
     }
 };
 
+// ---- operand stored [K, 192] (n-contiguous), 16-bit: 128 columns and 64 columns side by side -----
+// 384 bytes are no power of two of chunks for a load instruction's lanes, so each K step's slab is that of NTile<128>, then
+// that of NTile<64>. Of a wavefront's six loads per K tile the third and the sixth are the 64 columns', at scalar offsets of
+// their own.
+template <typename T>
+struct NTile192 {
+    using frag_t = typename Mfma<T>::frag;
+    using Wide = NTile<T, 128>;
+    using Narrow = NTile<T, 64>;
+    static constexpr int kStepElems = kBK<T> * 192;
+    static constexpr int kNarrowElems = kBK<T> * 128;  // where a step's 64 columns start
+    static constexpr int kElems = kSteps * kStepElems;
+    static constexpr int kLoads = Wide::kLoads + Narrow::kLoads;
+    static_assert(kSteps == 2 && Wide::kLoads == 4 && Narrow::kLoads == 2, "two loads of the 128 columns, one of the 64 per K step");
+
+    u32x4 rsrc = {0u, 0u, 0u, 0u};
+    int voffset = 0, narrow_voffset = 0;
+    unsigned int group_bytes = 0;  // of the 128 columns; the 64 columns' loads cover twice the k rows
+
+    __device__ __forceinline__ void init(const T* base, long ld, int cols_left, int k_total, int wave) {
+        const int lane = threadIdx.x & (kWave - 1);
+        rsrc = make_rsrc(base, (static_cast<long>(k_total - 1) * ld + cols_left) * static_cast<long>(sizeof(T)));
+        const int last = cols_left / kVec128<T> - 1;
+        auto at = [&](int per_row, int first, int swizzle) {
+            const int row = lane / per_row;
+            return static_cast<int>(row * ld * sizeof(T)) + min(first + ((lane % per_row) ^ swizzle), last) * 16;
+        };
+        voffset = at(Wide::kChunksPerRow, 0, Wide::swizzle(wave * Wide::kRowsPerLoad + lane / Wide::kChunksPerRow));
+        narrow_voffset = at(Narrow::kChunksPerRow, Wide::kChunksPerRow,
+                            Narrow::swizzle(wave * Narrow::kRowsPerLoad + lane / Narrow::kChunksPerRow));
+        group_bytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(Wide::kRowsPerLoad * ld * sizeof(T)));
+    }
+    __device__ __forceinline__ unsigned int first_offset(int k0, int wave) const { return (wave + k0 / Wide::kRowsPerLoad) * group_bytes; }
+    __device__ __forceinline__ unsigned int narrow_first_offset(int k0, int wave) const { return (2 * wave + k0 / Wide::kRowsPerLoad) * group_bytes; }
+    // A block of 16 columns lies in one of the two parts.
+    __device__ __forceinline__ static int wide_offset(int lane, int block0) { return Wide::lane_offset(lane, block0); }
+    __device__ __forceinline__ static int narrow_offset(int lane, int block0) { return kNarrowElems + Narrow::lane_offset(lane, block0); }
+};
+
 }  // namespace
 }  // namespace cgptx

@@ -75,11 +75,17 @@ public:
     Buffer(const Buffer&) = delete;
     ~Buffer() { (void)hipFree(base_); }
     std::uint16_t* data() const { return base_ + kGuard; }
-    bool holds(const Bits& want) {
+    // What the buffer holds; false if a guard does not.
+    bool copy(Bits& out) {
         hip_ok(hipMemcpy(host_.data(), base_, host_.size() * 2, hipMemcpyDeviceToHost), "hipMemcpy");
         for (std::size_t i = 0; i < kGuard; ++i)
             if (host_[i] != kPoison || host_[kGuard + count_ + i] != kPoison) return false;
-        return want.size() == count_ && std::memcmp(host_.data() + kGuard, want.data(), count_ * 2) == 0;
+        out.assign(host_.begin() + kGuard, host_.begin() + kGuard + static_cast<std::ptrdiff_t>(count_));
+        return true;
+    }
+    bool holds(const Bits& want) {
+        Bits held;
+        return copy(held) && held == want;
     }
 
 private:
@@ -160,6 +166,47 @@ void check(std::size_t rows, std::size_t hidden, std::size_t q, std::size_t k, s
     }
 }
 
+// The input gradient of q, k and v over many rows, whose operand comes from three buffers: few enough columns and rows that tiles of
+// 256 x 192 fill the chip where 256 x 256 do not, ragged both ways. Some rows are compared, the last ones among them.
+void check_many_rows(std::size_t rows, std::size_t hidden, std::size_t q, std::size_t k, std::size_t v, int dtype, hipStream_t stream) {
+    const std::string name = "input gradient of " + std::to_string(rows) + " rows" + (dtype == CGPTX_F16 ? " f16" : " bf16");
+    std::printf("%s\n", name.c_str());
+    std::fflush(stdout);
+    std::mt19937 rng(static_cast<unsigned int>(rows + hidden));
+    const std::size_t width[3] = {q, k, v}, total = q + k + v;
+    const Matrix w = random_matrix(total, hidden, rng);
+    const Matrix dy[3] = {random_matrix(rows, q, rng), random_matrix(rows, k, rng), random_matrix(rows, v, rng)};
+    const Buffer on_w(w, dtype), on_dq(dy[0], dtype), on_dk(dy[1], dtype), on_dv(dy[2], dtype);
+    const Buffer* on_dy[3] = {&on_dq, &on_dk, &on_dv};
+    Buffer dx(rows * hidden);
+    GemmArgs input;
+    input.b = on_w.data();
+    input.c = dx.data();
+    input.m = rows;
+    input.n = input.ldb = input.ldc = hidden;
+    input.k = total;
+    input.b_k_contiguous = false;
+    input.dtype = dtype;
+    input.a_segments.count = 3;
+    for (int i = 0; i < 3; ++i) {
+        input.a_segments.ptr[i] = on_dy[i]->data();
+        input.a_segments.ld[i] = input.a_segments.cols[i] = width[i];
+    }
+    expect(cgptx::gemm(input, stream) == CGPTX_OK, name + ": launch");
+    hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    std::vector<std::size_t> some;
+    for (std::size_t r = 0; r < rows; r += 331) some.push_back(r);
+    for (std::size_t r = rows - 3; r < rows; ++r) some.push_back(r);
+    const auto dy_at = [&](std::size_t i, std::size_t c) {
+        return c < q ? dy[0].at(some[i], c) : c < q + k ? dy[1].at(some[i], c - q) : dy[2].at(some[i], c - q - k);
+    };
+    const Bits want = product(some.size(), hidden, total, dtype, dy_at, [&](std::size_t t, std::size_t j) { return w.at(t, j); });
+    Bits got(rows * hidden);
+    expect(dx.copy(got), name + ": guards");
+    for (std::size_t i = 0; i < some.size(); ++i)
+        expect(std::memcmp(&got[some[i] * hidden], &want[i * hidden], hidden * 2) == 0, name + ": row " + std::to_string(some[i]));
+}
+
 }  // namespace
 
 int main() {
@@ -172,6 +219,7 @@ int main() {
             check(100, 256, 256, 128, 128, dtype, stream);  // 3 x 100 tokens' kind: segments of whole K tiles
             check(131, 224, 192, 64, 160, dtype, stream);   // ragged rows and columns, five steps in the last segment
             check(300, 512, 512, 64, 224, dtype, stream);   // more rows than one tile of either size
+            check_many_rows(16300, 760, 1024, 512, 512, dtype, stream);
         }
         hip_ok(hipStreamDestroy(stream), "hipStreamDestroy");
     } catch (const std::exception& e) {

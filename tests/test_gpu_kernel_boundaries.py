@@ -78,6 +78,31 @@ def test_contractions_in_k_slices_are_exact_on_integers(device, rows, fin, fout,
         assert torch.equal(got.cpu(), exact.to(dtype)), name
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("rows,fin,fout", [
+    (16300, 2048, 760), (16300, 760, 2048),  # Y and dX on 256 x 192 tiles, ragged rows and columns
+    (2048, 760, 16304), (2040, 768, 16384),  # dW: both operands as they lie, a K tile half empty
+])
+def test_contractions_whose_columns_leave_square_tiles_idle_are_exact_on_integers(device, rows, fin, fout, dtype):
+    """Some 750 columns are three tiles of 256, which is 192 of them for 256 compute units, or four of 192. Every sum is exact in
+    fp32 (at most 4 x 16304 < 2^24), so each result is the rounded exact value, alone and added to what is there."""
+    g = torch.Generator(device=device).manual_seed(rows + fin)
+    x, w, dy = (torch.randint(-2, 3, shape, generator=g, device=device).float() for shape in ((rows, fin), (fout, fin), (rows, fout)))
+    on = lambda t: t.to(dtype)
+    y, gi, gw = (torch.full(shape, float("nan"), dtype=dtype, device=device) for shape in ((rows, fout), (rows, fin), (fout, fin)))
+    ops.linear_forward(y, on(x), on(w))
+    ops.linear_backward(gi, None, None, on(dy), on(x), on(w))
+    ops.linear_backward(None, gw, None, on(dy), on(x), on(w))
+    exact = (x @ w.T.contiguous(), dy @ w, dy.T.contiguous() @ x)
+    for name, got, want in zip(("Y", "dX", "dW"), (y, gi, gw), exact):
+        assert torch.equal(got, on(want)), name
+    added = ops.LinearBackwardOptions(accumulate_input=True, accumulate_weight=True)
+    ops.linear_backward(gi, None, None, on(dy), on(x), on(w), options=added)
+    ops.linear_backward(None, gw, None, on(dy), on(x), on(w), options=added)
+    for name, got, want in zip(("dX", "dW"), (gi, gw), exact[1:]):
+        assert torch.equal(got, on(want + on(want).float())), name
+
+
 @pytest.mark.parametrize("rows,fin,fout", [(33, 480, 576), (121, 192, 896), (690, 352, 512), (2837, 256, 128), (5399, 608, 640)])
 def test_fp32_gradients_of_one_call_are_as_near_to_64_bits_as_one_by_one(device, rows, fin, fout):
     """Whatever shares a launch adds no longer chains in fp32 than the calls by themselves. The error of a sum of random terms,
