@@ -755,7 +755,9 @@ double predicted_pair_us(long tiles_x, long steps_x, long tiles_w, long steps_w,
 // after the K loops). Two workgroups share a CU and its LDS, or, deep, each has one to itself: then the longest is not held
 // up by another, but 3.5 us of start and end of every workgroup are in nobody's shadow. Joined if that is less than the calls'
 // own predictions in turn. [M, N] x K measured apart and joined: dX and dW of 128 x 768 x 768 10.4 -> 7.4 us, of 2000 x 1024 x
-// 2048 35.7 -> 32.3; 5005 x 1024 x 256, whose dW is better split along K, 23.7 -> 28.8: stays apart.
+// 2048 35.7 -> 32.3; 5005 x 1024 x 256, whose dW is better split along K, 23.7 -> 28.8: stays apart. fp32, 256 rows, 1024 wide, 8:2
+// heads of 128, feed-forward of 2048: the gradients of gate|up, q, k and v in turn 83, joined 66; q, k, v and gate|up forward on 64 x 64
+// tiles 42, gate|up on those and the others on 32 x 32 37.
 GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
     GemmGroup best_plan;
     const double units = static_cast<double>(compute_units());
@@ -764,9 +766,13 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
     for (int i = 0; i < count; ++i) fewest += static_cast<double>((calls[i].m + 63) / 64) * static_cast<double>((calls[i].n + 63) / 64);
     if (fewest > (pair ? 4.0 : 1.0) * kGroupBlocksPerUnit * units) return best_plan;
     double separate = 0.0;
+    // fp32 pairs whose own plans have no K slices: a group gives neither a longer chain of additions. (Who makes larger groups has
+    // looked at that, see gemm_adds_as_joined.)
+    bool f32_group = calls[0].dtype == CGPTX_F32;
     for (int i = 0; i < count; ++i) {
         const GemmArgs& g = calls[i];
         const Plan plan = make_plan(g);
+        f32_group = f32_group && (count > 2 || plan.slices == 1);
         const long tiles = Plan::tiles_of(g, plan.tile);
         const bool f32 = g.dtype == CGPTX_F32;
         const long k_step = f32 ? kBK<float> : kBK<bf16_t>, k_tiles = (static_cast<long>(g.k) + k_step - 1) / k_step;
@@ -789,7 +795,7 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
     }
     if (fewest > kGroupBlocksPerUnit * units) return best_plan;
     for (int choice = 0; choice < 1 << count; ++choice) {
-        double longest = 0.0, work = 0.0, lone_work = 0.0, blocks = 0.0;
+        double longest = 0.0, work = 0.0, lone_work = 0.0, blocks = 0.0, loops[kGroupCalls], counts[kGroupCalls];
         for (int i = 0; i < count; ++i) {
             const GemmArgs& g = calls[i];
             const bool f32 = g.dtype == CGPTX_F32, small = ((choice >> i) & 1) != 0;
@@ -803,10 +809,19 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
             work += tiles * kt * shared;
             lone_work += tiles * (loop + 3.5);
             blocks += tiles;
+            loops[i] = loop;
+            counts[i] = tiles;
         }
         if (blocks > kGroupBlocksPerUnit * units) continue;
         const double load = blocks / units;
-        const double two = load <= 1.0 ? longest : std::max(1.4 * longest, work / units * std::ceil(load) / load * (load > 4.0 ? 1.3 : 1.0));
+        double two = load <= 1.0 ? longest : std::max(1.4 * longest, work / units * std::ceil(load) / load * (load > 4.0 && !f32_group ? 1.3 : 1.0));
+        // fp32: the matrix cores are what binds, two tiles on a CU take twice as long, and a CU that has one long tile more than the
+        // others ends that much later.
+        for (int i = 0; i < count && f32_group; ++i) {
+            double as_long = 0.0;
+            for (int j = 0; j < count; ++j) as_long += loops[j] >= loops[i] ? counts[j] : 0.0;
+            two = std::max(two, std::ceil(as_long / units) * loops[i]);
+        }
         const double one = load <= 1.0 ? longest : std::max(longest, lone_work / units * std::ceil(load) / load);
         if (3.5 + std::min(one, two) < best) {
             best = 3.5 + std::min(one, two);
@@ -825,7 +840,7 @@ bool joinable(const GemmArgs& g, KernelArgs& p) {
     if (g.a == nullptr && g.a_segments.count == 0) return false;
     if (g.b == nullptr || g.c == nullptr || g.m == 0 || g.n == 0 || g.k == 0 || g.batch_rows != 0 || g.swiglu_out != nullptr ||
         g.swiglu_saved != nullptr || g.c_segments.count > 0 || (g.a_sums != nullptr && g.a_k_contiguous) ||
-        (g.a_segments.count > 0 && (!g.a_k_contiguous || g.b_k_contiguous || std::is_same_v<T, float>)))
+        (g.a_segments.count > 0 && (!g.a_k_contiguous || g.b_k_contiguous)))
         return false;
     constexpr std::size_t i32max = std::numeric_limits<int>::max();
     if (g.m > i32max || g.n > i32max || g.k > i32max) return false;

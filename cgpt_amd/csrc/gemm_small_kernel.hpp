@@ -441,7 +441,7 @@ __global__ __launch_bounds__(kThreads) void gemm_small_group_kernel(SmallGroup g
             small_tile<T, TILE, DEEP, true, false, SmallEpilogue::general, false, false>(p, m0, n0, 0, smem_raw);
         else if (layout == SmallLayout::forward)
             small_tile<T, TILE, DEEP, true, true, SmallEpilogue::general, false, false>(p, m0, n0, 0, smem_raw);
-        else if constexpr (sizeof(T) == 2)
+        else
             small_tile<T, TILE, DEEP, true, false, SmallEpilogue::general, true, false>(p, m0, n0, 0, smem_raw);
     };
     if (tile == 32) with_tile.template operator()<32>();
