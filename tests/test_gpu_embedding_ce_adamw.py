@@ -288,6 +288,30 @@ def test_adamw_many_parity_three_steps(device, dtype):
         assert torch.equal(p, s.master_parameter.to(dtype))
 
 
+@pytest.mark.parametrize("sizes", [
+    [4096 * (i % 3) + i for i in range(1, 65)], [4096 * (i % 2) + 7 * i for i in range(1, 66)],  # one and two starts a lane
+    [1 + 37 * i % 5000 for i in range(256)], [1 + 37 * i % 5000 for i in range(257)],            # the most that are read at once, and one more
+    [3, 2045 * 4096, 4096], [3, 2046 * 4096, 4097, 5],                                           # 2047 chunks, one a block, and 2050, four
+], ids=["64", "65", "256", "257", "one-chunk", "four-chunks"])
+def test_adamw_finds_every_chunk(device, sizes):
+    """One clipped step over many tensors, and over as many chunks as the statistics pass changes its blocks at, against float64:
+    a chunk that is taken for another tensor's or left out moves the norm and its elements."""
+    params = [randn((n,), torch.float32, 500 + i, 0.5) for i, n in enumerate(sizes)]
+    grads = [randn((n,), torch.float32, 900 + i, 1.0 + i % 7) for i, n in enumerate(sizes)]
+    d_params = [dev(p, device).clone() for p in params]
+    states = [ops.AdamWState.for_parameter(p) for p in d_params]
+    entries = [ops.AdamWBatchEntry(p, dev(g, device), s) for p, g, s in zip(d_params, grads, states)]
+    ws = ops.AdamWWorkspace()
+    ops.adamw_step_many_async(entries, ops.AdamWOptions(learning_rate=3e-4, beta1=0.9, beta2=0.95, epsilon=1e-8, weight_decay=0.1,
+                                                        loss_scale=2.0, max_grad_norm=1.0), ws)
+    ok, masters, ms, vs, step = oracle64.adamw(None, [to_np(g) for g in grads], [to_np(p) for p in params], [np.zeros(n) for n in sizes],
+                                               [np.zeros(n) for n in sizes], 0, 3e-4, 0.9, 0.95, 1e-8, 0.1, 2.0, 1.0)
+    assert ok and ops.adamw_check(ws)
+    for s, m64, mm in zip(states, masters, ms):
+        assert_close(s.master_parameter, m64, 1e-5, "master")
+        assert np.abs(to_np(s.first_moment) - mm).max() <= 1e-5 * max(1e-12, np.abs(mm).max())
+
+
 def test_adamw_matches_cpu_restatement_single_tensor(device):
     n = 10007
     p, g = randn((n,), torch.float32, 300), randn((n,), torch.float32, 301, 5.0)
