@@ -46,7 +46,7 @@ struct Mfma<float> {
 // assembly so that the accumulator is updated in place: the four-register form of the instruction
 // does not tie its result to its addend, and with all 256 accumulator registers in use the register
 // allocator would otherwise shuffle accumulators around every MFMA. The kernel keeps the distances
-// the hardware asks for by construction: an accumulator is touched once per K tile (64 or 16 MFMAs
+// the hardware asks for by construction: an accumulator is touched once per K step (64, 48 or 16 MFMAs
 // apart), zeroed long before its first MFMA and read by the epilogue only after a barrier.
 template <>
 struct Mfma<bf16_t> {
