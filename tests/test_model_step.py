@@ -871,7 +871,8 @@ def test_block_output_is_the_residual_sum_of_its_parts(device, batch, seq):
 def test_branches_of_a_small_step_share_launches(device, monkeypatch, dtype, batch, seq, heads, kv_heads, head_dim, inter, layers):
     """A few hundred tokens: the attention and the feed-forward branch's first projections run in one launch, so do the gradients
     of their last and of their first ones, and the SwiGLU product and its gradient ride beside q's and k's norms.
-    CGPTX_FUSE_SWIGLU=0 keeps the branches apart: more launches, the same step but for the order of some sums."""
+    CGPTX_FUSE_SWIGLU=0 keeps the branches apart: more launches and the same step, in 16-bit storage to the bit (fp32 steps share
+    launches also where that changes the order of a sum)."""
     from cgpt_amd.model import LOSS_DENSE, Model, ModelConfig
     from tests.util import STOL, assert_scaled_close, launches
     config = ModelConfig(vocabulary_size=203, num_layers=layers, hidden_size=heads * head_dim, intermediate_size=inter,
@@ -889,4 +890,32 @@ def test_branches_of_a_small_step_share_launches(device, monkeypatch, dtype, bat
         model.close()
     assert counts[0] <= counts[1] - 3 * layers, counts
     for (name, a), (_, b) in zip(*results):
-        assert_scaled_close(a, b, STOL[dtype], name)
+        if dtype == torch.float32:
+            assert_scaled_close(a, b, STOL[dtype], name)
+        else:
+            assert torch.equal(a, b), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("batch,seq,heads,kv_heads,head_dim,inter,layers", [
+    (21, 112, 16, 4, 32, 1024, 1), (32, 140, 8, 4, 64, 1024, 2), (7, 22, 8, 4, 128, 2752, 2), (32, 111, 6, 2, 32, 512, 2),
+])
+def test_sharing_launches_changes_no_sum(device, monkeypatch, dtype, batch, seq, heads, kv_heads, head_dim, inter, layers):
+    """Steps some of whose projections, by themselves, run on large tiles or in K slices: those stay apart, since a group would add
+    them up in another order, and the gradients are those of a step whose branches share nothing, bit for bit."""
+    from cgpt_amd.model import LOSS_DENSE, Model, ModelConfig
+    config = ModelConfig(vocabulary_size=203, num_layers=layers, hidden_size=heads * head_dim, intermediate_size=inter,
+                         num_query_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, rotary_dim=head_dim, dtype=dtype)
+    rng = np.random.default_rng(batch + seq)
+    inputs, targets = (rng.integers(0, 203, size=batch * seq).astype(np.uint32) for _ in range(2))
+    results = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("CGPTX_FUSE_SWIGLU", fuse)
+        model = Model(config, batch, seq, seed=4, device=device)
+        model.set_tokens(inputs, targets)
+        model.forward_backward(loss_scale=4.0, loss_mode=LOSS_DENSE)
+        results.append([(name, g.clone()) for name, _, g in model.parameters()])
+        model.close()
+    for (name, a), (_, b) in zip(*results):
+        assert torch.equal(a, b), name
