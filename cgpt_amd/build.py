@@ -124,16 +124,19 @@ def build_dispatch(force: bool = True) -> pathlib.Path:
 
 INTERFACE_TEST_SOURCES = [ROOT / "tests" / "cpp" / name
                           for name in ("ops_interface_test.cpp", "block_backward_test.cpp", "data_upload_test.cpp",
-                                       "gemm_group_test.cpp")]
+                                       "gemm_group_test.cpp", "gemm_plan_test.cpp")]
 INTERFACE_TEST_BINARY = ROOT / "tests" / "cpp" / "ops_interface_test.bin"
 
 
 def build_interface_test() -> pathlib.Path:
     """Compiles the C++ programs that drive include/core, include/ops/**, include/optim/** and the library's internal
-    cgpt_amd/csrc/gemm.hpp against the library (tests/cpp/*.cpp -> *.bin). Host code only (the headers under include/ are
-    inline wrappers over the C-ABI); linked with an rpath relative to the binary so that they run from any checkout location."""
+    cgpt_amd/csrc/gemm.hpp against the library, and the one that reads the rules of cgpt_amd/csrc/gemm.hip itself (tests/cpp/*.cpp
+    -> *.bin). Host code only (the headers under include/ are inline wrappers over the C-ABI); linked with an rpath relative to the
+    binary so that they run from any checkout location."""
     for source in INTERFACE_TEST_SOURCES:
-        cmd = [HIPCC, "-std=c++20", "-O1", f"-I{ROOT / 'include'}", f"-I{CSRC}", str(source), "-o", str(source.with_suffix(".bin")),
+        # gemm.hip is included as source: HIP, with its kernels.
+        hip = [*DEVICE_FLAGS, "-x", "hip"] if source.name == "gemm_plan_test.cpp" else []
+        cmd = [HIPCC, *hip, "-std=c++20", "-O1", f"-I{ROOT / 'include'}", f"-I{CSRC}", str(source), "-o", str(source.with_suffix(".bin")),
                f"-L{LIB_DIR}", "-lcgptx", "-Wl,-rpath,$ORIGIN/../../cgpt_amd/lib"]
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:

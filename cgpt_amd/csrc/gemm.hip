@@ -218,7 +218,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma_kernel(KernelArgs p, i
 
 // ------------------------------------------------------------------- host side
 
-// CGPTX_GEMM_TILE=32|64|128|192|256 pins the tile size (for experiments); anything else = automatic.
+// CGPTX_GEMM_TILE=32|64|128|192|256 pins the tile size (for experiments); anything else = automatic, and so is a size that a call's
+// kernels do not have (192 where takes_narrow_tiles says no, 256 in fp32).
 int forced_tile() {
     static const int value = [] {
         const char* text = std::getenv("CGPTX_GEMM_TILE");
@@ -334,7 +335,8 @@ Plan make_plan(const GemmArgs& g) {
         set_slices(slices);
         return plan;
     }
-    const int forced = forced_tile();
+    const int pinned = forced_tile();
+    const int forced = (pinned == 192 && !takes_narrow_tiles(g)) || (f32 && pinned == 256) ? 0 : pinned;
     const double slice_bytes = static_cast<double>(g.m) * static_cast<double>(round_up(g.n, 8)) * sizeof(float);
     // Calls that 256 x 256 tiles spread over three quarters of the chip keep the order of additions of the kernels with a
     // SwiGLU epilogue, which take such calls only (one sum over all of K): the fused and the separate operators give the same
@@ -343,7 +345,7 @@ Plan make_plan(const GemmArgs& g) {
     double best = -1.0;
     long best_slices = 1;
     for (int tile : {32, 64, 128, 256}) {
-        if ((whole_k && tile < 128) || (forced != 0 && tile != forced && !(f32 && forced == 256)) || (f32 && tile == 256)) continue;
+        if ((whole_k && tile < 128) || (forced != 0 && tile != forced) || (f32 && tile == 256)) continue;
         const long tiles = tiles_of(tile);
         if (forced == 0 && tile <= 64 && tiles > 16 * units) continue;
         for (long s = 1; s <= 16; ++s) {

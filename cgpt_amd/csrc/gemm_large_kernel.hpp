@@ -1318,6 +1318,7 @@ int launch_large(const LargeCall& call, hipStream_t stream) {
         if (call.tile == 256) return with_tile.template operator()<256>();
         if (call.tile == 192) return launch_narrow<T>(call, stream);
     }
+    if (call.tile != 128) return fail(CGPTX_RUNTIME, "gemm: no large tiles of this size for the storage type");
     return with_tile.template operator()<128>();
 }
 

@@ -4,6 +4,7 @@ CPU part: every header of the interface is self-contained C++20 and the set decl
 the reference's callers use, in the reference's argument order. GPU part: the compiled test program
 replays the reference tests' known answers through that interface (tests/cpp/ops_interface_test.cpp).
 """
+import os
 import pathlib
 import re
 import shutil
@@ -102,3 +103,17 @@ def test_projections_of_a_small_block_share_exact_launches():
     proc = subprocess.run([str(binary)], capture_output=True, text=True, timeout=120)
     assert proc.returncode == 0, proc.stdout + proc.stderr
     assert "\n0 failure(s)" in proc.stdout
+
+
+def run_plan_test(mode, **environment):
+    binary = ROOT / "tests" / "cpp" / "gemm_plan_test.bin"
+    assert binary.exists(), "build it with `python -m cgpt_amd.build` (there is no fallback)"
+    proc = subprocess.run([str(binary), mode], capture_output=True, text=True, timeout=120, env={**os.environ, **environment})
+    assert proc.returncode == 0, proc.stdout[-4000:] + proc.stderr
+    assert proc.stdout.endswith("\n0 failure(s)\n") or proc.stdout == "0 failure(s)\n"
+
+
+def test_a_pinned_tile_size_is_one_that_the_call_has():
+    """tests/cpp/gemm_plan_test.cpp: with CGPTX_GEMM_TILE=192 fp32 calls, and those that add a bias, are planned for tiles they have
+    kernels of (fp32 results once lacked three quarters of their elements)."""
+    run_plan_test("pinned", CGPTX_GEMM_TILE="192")
