@@ -924,9 +924,13 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && fused_swiglu_gradient() && !fills_chip &&
                                        swiglu_beside_norms(swiglu, dt) && down_alike &&
                                        gemm_adds_as_joined(last_parts + last_down, last_count - last_down, stream);
+        const GemmArgs* const qkv_gradients = first_parts + first_gate_up;  // with the weights' unless those are stacked
+        // Without a launch of their own q's, k's and v's input gradients are added up in storage, rounded each time: a group of all
+        // six would add them in fp32.
+        const GemmGroup qkv_gradient_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
         const bool first_together = gemm_adds_as_joined(first_parts, first_gate_up, stream) && (fused_qkv
             ? gemm_adds_as_joined(fused_qkv_gradients, 1, stream) && (stacked || gemm_adds_as_joined(fused_qkv_gradients + 1, 1, stream))
-            : gemm_adds_as_joined(first_parts + first_gate_up, first_count - first_gate_up, stream));
+            : qkv_gradient_group.joined);
         const GemmGroup last_group = branches_together ? gemm_joins(last_parts, last_count, stream, false) : GemmGroup{};
         const GemmGroup first_group = last_group.joined && first_together ? gemm_joins(first_parts, first_count, stream, false) : GemmGroup{};
         if (last_group.joined) {
@@ -970,8 +974,6 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
                                                               N * HKV, D, eps, dt, stream, sink));
         }
         if (last_group.joined && !first_group.joined) CGPTX_TRY(gate_up_gradients());
-        const GemmArgs* const qkv_gradients = first_parts + first_gate_up;  // with the weights' unless those are stacked
-        const GemmGroup gradient_group = fused_qkv || first_group.joined ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
         if (first_group.joined) {
             CGPTX_SHARED_OP(stacked ? "gemm_dx.gate_up" : "gemm_dx_dw.gate_up", stacked ? "gemm_dx.qkv" : "gemm_dx_dw.qkv", first_parts, first_count,
                             first_gate_up, gemm_joined(first_parts, first_count, first_group, stream));
@@ -979,8 +981,8 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
             CGPTX_OP("gemm_dx.qkv", gemm(qkv_gradients[0], stream));
             if (!stacked)
                 CGPTX_OP("gemm_dw.qkv", gemm(fused_qkv_gradients[1], stream));
-        } else if (gradient_group.joined) {
-            CGPTX_OP("gemm_dx_dw.qkv", gemm_joined(qkv_gradients, 4, gradient_group, stream));
+        } else if (qkv_gradient_group.joined) {
+            CGPTX_OP("gemm_dx_dw.qkv", gemm_joined(qkv_gradients, 4, qkv_gradient_group, stream));
         } else {
             CGPTX_TRY(linear_gradients(m, m->d_norm_in, w.q.gradient, d_q, a.norm_a, w.q.value, N, H, QW, 0, dt, stream, kQkvLabels));
             CGPTX_TRY(linear_gradients(m, m->d_norm_in, w.k.gradient, d_k, a.norm_a, w.k.value, N, H, KW, 1, dt, stream, kQkvLabels));

@@ -900,6 +900,7 @@ def test_branches_of_a_small_step_share_launches(device, monkeypatch, dtype, bat
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("batch,seq,heads,kv_heads,head_dim,inter,layers", [
     (21, 112, 16, 4, 32, 1024, 1), (32, 140, 8, 4, 64, 1024, 2), (7, 22, 8, 4, 128, 2752, 2), (32, 111, 6, 2, 32, 512, 2),
+    (8, 255, 7, 7, 128, 576, 1),  # q, k and v too wide for a group of their own: their input gradients are added up in storage
 ])
 def test_sharing_launches_changes_no_sum(device, monkeypatch, dtype, batch, seq, heads, kv_heads, head_dim, inter, layers):
     """Steps some of whose projections, by themselves, run on large tiles or in K slices: those stay apart, since a group would add
