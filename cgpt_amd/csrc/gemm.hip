@@ -768,8 +768,9 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
     for (int i = 0; i < count; ++i) fewest += static_cast<double>((calls[i].m + 63) / 64) * static_cast<double>((calls[i].n + 63) / 64);
     if (fewest > (pair ? 4.0 : 1.0) * kGroupBlocksPerUnit * units) return best_plan;
     double separate = 0.0;
-    // fp32 pairs whose own plans have no K slices: a group gives neither a longer chain of additions. (Who makes larger groups has
-    // looked at that, see gemm_adds_as_joined.)
+    // fp32 pairs whose own plans have no K slices: a group gives neither a longer chain of additions. (Who makes larger groups of
+    // gradients has looked at that, see gemm_adds_as_joined and gemm_segments_add_as_joined; the three forward projections, whose
+    // chains are a layer's width, always shared a launch.)
     bool f32_group = calls[0].dtype == CGPTX_F32;
     for (int i = 0; i < count; ++i) {
         const GemmArgs& g = calls[i];
@@ -975,6 +976,22 @@ bool gemm_adds_as_joined(const GemmArgs* calls, int count, hipStream_t stream) {
     for (int i = 0; i < count; ++i) {
         const Plan plan = make_plan(calls[i]);
         if (plan.tile > 64 || plan.slices != 1) return false;
+    }
+    return true;
+}
+
+bool gemm_segments_add_as_joined(const GemmArgs* calls, hipStream_t stream) {
+    const GemmSegments& segments = calls[0].a_segments;
+    std::size_t first = 0;
+    for (int i = 0; i < segments.count; ++i) {
+        GemmArgs pair[2] = {calls[0], calls[1 + i]};
+        pair[0].a_segments = GemmSegments{};
+        pair[0].a = segments.ptr[i];
+        pair[0].lda = segments.ld[i];
+        pair[0].k = segments.cols[i];
+        pair[0].b = static_cast<const char*>(calls[0].b) + first * calls[0].ldb * dtype_size(calls[0].dtype);
+        if (!gemm_adds_as_joined(pair, 2, stream)) return false;
+        first += segments.cols[i];
     }
     return true;
 }

@@ -95,6 +95,10 @@ GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream = null
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream);
 // Whether calls by themselves, or as a group of their own, add in the order that a group gives them: small tiles, one sum over K.
 bool gemm_adds_as_joined(const GemmArgs* calls, int count, hipStream_t stream);
+// The same of an input gradient in segments along K (calls[0]) and each segment's weight gradient (calls[1 ..]) against what they
+// stand for, a pair of calls per segment. fp32 sums show it: in K slices, 1221 rows make a weight gradient of chains of 34 additions, in
+// one sum of 305.
+bool gemm_segments_add_as_joined(const GemmArgs* calls, hipStream_t stream);
 // Bytes of split-K partial tiles that gemm() asks the arena for in this call (operands that stream as they lie).
 std::size_t gemm_split_bytes(const GemmArgs& args);
 // Copies [rows, cols] elements (row stride ld) to rows of `pitch` elements (whole 16-byte chunks), zeros past cols.

@@ -927,7 +927,8 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         const GemmArgs* const qkv_gradients = first_parts + first_gate_up;  // with the weights' unless those are stacked
         // Without a launch of their own q's, k's and v's input gradients are added up in storage, rounded each time: a group of all
         // six would add them in fp32.
-        const GemmGroup qkv_gradient_group = fused_qkv ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
+        const bool qkv_gradients_alike = dt != CGPTX_F32 || gemm_segments_add_as_joined(qkv_gradients, stream);
+        const GemmGroup qkv_gradient_group = fused_qkv || !qkv_gradients_alike ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
         const bool first_together = gemm_adds_as_joined(first_parts, first_gate_up, stream) && (fused_qkv
             ? gemm_adds_as_joined(fused_qkv_gradients, 1, stream) && (stacked || gemm_adds_as_joined(fused_qkv_gradients + 1, 1, stream))
             : qkv_gradient_group.joined);

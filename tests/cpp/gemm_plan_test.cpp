@@ -64,10 +64,55 @@ void check_pinned() {
                 }
 }
 
+// q's, k's and v's gradients over `rows` tokens as one group: their input gradients as one call in segments, then the weight gradients.
+struct Gradients {
+    GemmArgs calls[4], input[3];
+    Gradients(std::size_t rows, std::size_t hidden, std::size_t q, std::size_t k, int dtype) {
+        const std::size_t width[3] = {q, k, k};
+        calls[0] = contraction(Kind::input_gradient, rows, hidden, q + 2 * k, dtype);
+        calls[0].a = nullptr;
+        calls[0].a_segments.count = 3;
+        for (int i = 0; i < 3; ++i) {
+            calls[0].a_segments.ptr[i] = address();
+            calls[0].a_segments.ld[i] = calls[0].a_segments.cols[i] = width[i];
+            calls[1 + i] = contraction(Kind::weight_gradient, width[i], hidden, rows, dtype);
+            input[i] = contraction(Kind::input_gradient, rows, hidden, width[i], dtype);
+        }
+    }
+};
+// Additions that follow each other in a sum of a call by itself: four wavefronts share a small tile's K range.
+double chain(const GemmArgs& g) {
+    const Plan plan = make_plan(g);
+    return static_cast<double>(g.k) / (plan.slices * (plan.tile <= 64 ? 4 : 1));
+}
+
+// fp32: a group gives no sum a longer chain of additions than the calls that it stands for have, each with its weight gradient.
+void check_chains() {
+    int joined = 0, refused = 0;
+    for (const std::size_t head_dim : {32, 64, 128})
+        for (const std::size_t kv : {1, 2, 4})
+            for (const std::size_t group : {1, 2, 4})
+                for (std::size_t rows = 32; rows <= 2048; rows += rows / 8) {
+                    const std::size_t q = head_dim * kv * group, k = head_dim * kv;
+                    const Gradients of(rows, q, q, k, CGPTX_F32);
+                    const bool together = gemm_segments_add_as_joined(of.calls, nullptr) && gemm_joins(of.calls, 4).joined;
+                    (together ? joined : refused) += 1;
+                    if (!together) continue;
+                    for (int i = 0; i < 3; ++i) {
+                        const GemmArgs pair[2] = {of.input[i], of.calls[1 + i]};
+                        if (gemm_joins(pair, 2).joined) continue;
+                        for (const GemmArgs& g : pair)
+                            expect(static_cast<double>(g.k) / 4 <= 1.01 * chain(g), name_of(g) + ": a chain of " + std::to_string(g.k / 4) + " for " + std::to_string(chain(g)));
+                    }
+                }
+    expect(joined > 100 && refused > 10, std::to_string(joined) + " groups joined, " + std::to_string(refused) + " not");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "pinned") == 0) check_pinned();
+    if (argc > 1 && std::strcmp(argv[1], "chains") == 0) check_chains();
     std::printf("%d failure(s)\n", failures);
     return failures == 0 ? 0 : 1;
 }

@@ -117,3 +117,9 @@ def test_a_pinned_tile_size_is_one_that_the_call_has():
     """tests/cpp/gemm_plan_test.cpp: with CGPTX_GEMM_TILE=192 fp32 calls, and those that add a bias, are planned for tiles they have
     kernels of (fp32 results once lacked three quarters of their elements)."""
     run_plan_test("pinned", CGPTX_GEMM_TILE="192")
+
+
+def test_fp32_gradients_that_share_a_launch_have_no_longer_chains():
+    """tests/cpp/gemm_plan_test.cpp: q's, k's and v's gradients in fp32 join only where no sum becomes a longer chain of additions
+    than it is in the launches they stand for (the rounding error of a chain grows with its length)."""
+    run_plan_test("chains")
