@@ -2,6 +2,7 @@
 // (cgpt_amd/csrc/gemm.hpp), forward as a group of three, backward as one of four whose input gradient reads its operand from
 // three buffers. Operands of -1 .. 1: sums of at most 8192 products are exact in fp32 in any order, so every result is the
 // rounded exact value. Built by `python -m cgpt_amd.build`; run by tests/test_cpp_interface.py on the GPU.
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <random>
@@ -207,6 +208,110 @@ void check_many_rows(std::size_t rows, std::size_t hidden, std::size_t q, std::s
         expect(std::memcmp(&got[some[i] * hidden], &want[i * hidden], hidden * 2) == 0, name + ": row " + std::to_string(some[i]));
 }
 
+class Floats {
+public:
+    explicit Floats(std::size_t count) : count_(count) { hip_ok(hipMalloc(reinterpret_cast<void**>(&data_), count * 4), "hipMalloc"); }
+    explicit Floats(const std::vector<float>& from) : Floats(from.size()) {
+        hip_ok(hipMemcpy(data_, from.data(), count_ * 4, hipMemcpyHostToDevice), "hipMemcpy");
+    }
+    Floats(const Floats&) = delete;
+    ~Floats() { (void)hipFree(data_); }
+    float* data() const { return data_; }
+    std::vector<float> copy() const {  // after all that was launched
+        std::vector<float> out(count_);
+        hip_ok(hipDeviceSynchronize(), "hipDeviceSynchronize");
+        hip_ok(hipMemcpy(out.data(), data_, count_ * 4, hipMemcpyDeviceToHost), "hipMemcpy");
+        return out;
+    }
+
+private:
+    std::size_t count_;
+    float* data_ = nullptr;
+};
+
+// The same input gradient in fp32, where the group is launched for its one call in segments: its error against 64 bits is that of
+// three calls which add to each other's result, not that of one sum over all segments. A sum's error grows with its length: one
+// chain of three equal parts has some 1.7 times the error of three.
+void check_segment_sums(std::size_t rows, std::size_t hidden, std::size_t q, std::size_t k, hipStream_t stream) {
+    const std::string name = "fp32 input gradient, " + std::to_string(rows) + " x " + std::to_string(hidden) + ", " + std::to_string(q) + " + 2 x " + std::to_string(k);
+    std::printf("%s\n", name.c_str());
+    std::fflush(stdout);
+    std::mt19937 rng(static_cast<unsigned int>(rows + q));
+    std::normal_distribution<float> normal;
+    const std::size_t width[3] = {q, k, k}, total = q + 2 * k;
+    auto random = [&](std::size_t count) {
+        std::vector<float> v(count);
+        for (float& x : v) x = normal(rng);
+        return v;
+    };
+    const std::vector<float> w = random(total * hidden), x = random(rows * hidden), dy[3] = {random(rows * q), random(rows * k), random(rows * k)};
+    Floats on_w(w), on_x(x), dx(rows * hidden), dw(total * hidden);
+    Floats on_dy[3] = {Floats(dy[0]), Floats(dy[1]), Floats(dy[2])};
+    GemmArgs calls[4];
+    GemmArgs& input = calls[0];
+    input.b = on_w.data();
+    input.c = dx.data();
+    input.m = rows;
+    input.n = input.ldb = input.ldc = hidden;
+    input.k = total;
+    input.b_k_contiguous = false;
+    input.dtype = CGPTX_F32;
+    input.a_segments.count = 3;
+    std::size_t first = 0;
+    for (int i = 0; i < 3; ++i) {
+        GemmArgs& b = calls[1 + i];
+        b.a = on_dy[i].data();
+        b.b = on_x.data();
+        b.c = dw.data() + first * hidden;
+        b.m = b.lda = width[i];
+        b.n = b.ldb = b.ldc = hidden;
+        b.k = rows;
+        b.a_k_contiguous = b.b_k_contiguous = false;
+        b.dtype = CGPTX_F32;
+        input.a_segments.ptr[i] = on_dy[i].data();
+        input.a_segments.ld[i] = input.a_segments.cols[i] = width[i];
+        first += width[i];
+    }
+    // Root mean square of the error of some rows.
+    auto error = [&](const std::vector<float>& got) {
+        double sum = 0.0;
+        for (std::size_t r = 0; r < rows; r += 7)
+            for (std::size_t c = 0; c < hidden; ++c) {
+                double exact = 0.0;
+                std::size_t t = 0;
+                for (int i = 0; i < 3; ++i)
+                    for (std::size_t j = 0; j < width[i]; ++j, ++t) exact += static_cast<double>(dy[i][r * width[i] + j]) * w[t * hidden + c];
+                sum += (got[r * hidden + c] - exact) * (got[r * hidden + c] - exact);
+            }
+        return std::sqrt(sum / static_cast<double>((rows + 6) / 7 * hidden));
+    };
+    cgptx::GemmGroup group = cgptx::gemm_joins(calls, 4, stream);
+    expect(group.joined, name + ": the gradients share no launch");
+    if (!group.joined) return;
+    for (const int tile : {32, 64})
+        for (const bool deep : {false, true}) {
+            for (int& t : group.tile) t = tile;
+            group.deep = deep;
+            expect(cgptx::gemm_joined(calls, 4, group, stream) == CGPTX_OK, name + ": launch");
+            const double joined = error(dx.copy());
+            // What it stands for, in the same tiles: each projection's pair of gradients, the input gradients added up.
+            first = 0;
+            for (int i = 0; i < 3; ++i) {
+                GemmArgs pair[2] = {input, calls[1 + i]};
+                pair[0].a_segments = {};
+                pair[0].a = on_dy[i].data();
+                pair[0].lda = pair[0].k = width[i];
+                pair[0].b = on_w.data() + first * hidden;
+                pair[0].accumulate = i > 0;
+                first += width[i];
+                expect(cgptx::gemm_joined(pair, 2, group, stream) == CGPTX_OK, name + ": launch of a pair");
+            }
+            const double apart = error(dx.copy());
+            std::printf("  tiles of %d%s: error %.3g, apart %.3g\n", tile, deep ? ", deep" : "", joined, apart);
+            expect(joined <= 1.1 * apart, name + ": larger error in one launch");
+        }
+}
+
 }  // namespace
 
 int main() {
@@ -221,6 +326,9 @@ int main() {
             check(300, 512, 512, 64, 224, dtype, stream);   // more rows than one tile of either size
             check_many_rows(16300, 760, 1024, 512, 512, dtype, stream);
         }
+        check_segment_sums(300, 512, 512, 512, stream);
+        check_segment_sums(131, 768, 768, 256, stream);
+        check_segment_sums(70, 224, 96, 32, stream);  // wavefronts without a K tile of some segments
         hip_ok(hipStreamDestroy(stream), "hipStreamDestroy");
     } catch (const std::exception& e) {
         std::printf("FAIL %s\n", e.what());
