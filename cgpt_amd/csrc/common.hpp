@@ -254,8 +254,9 @@ int scratch(hipStream_t stream, std::size_t bytes, void** out);
 int scratch_up_to(hipStream_t stream, std::size_t bytes, void** out, std::size_t* held);
 
 // kTickets counters bound to (current device, stream), all zero between launches: a kernel's workgroups count themselves by them
-// (the last one to end goes on with what the others left) and the last one leaves them at zero. Null where they cannot be had
-// (first asked for under capture, no memory): the caller does without.
+// (the last one to end goes on with what the others left). What a launch adds to a counter in all is 2^32, so that no order of
+// launches and no meeting of two leaves one that the next launch miscounts from. Null where they cannot be had (first asked for under
+// capture, no memory): the caller does without.
 constexpr int kTickets = 4096;
 unsigned int* tickets(hipStream_t stream);
 

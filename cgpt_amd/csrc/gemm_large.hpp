@@ -58,6 +58,13 @@ struct KernelArgs {
 // The input and the weight gradient of a projection in one launch, on 128 x 128 tiles; each call's tiles_m, tiles_n, slices and
 // k_tiles_per_slice are set.
 constexpr int kFoldTileBytes = 128 * 128 * 4 + 128 * 4;  // of a tile's slice: accumulators, and sums of A's columns
+// What a K slice adds to the counter of its tile: shares that make 2^32 together, none of them zero. The workgroup that brings the
+// counter back to zero is the tile's last one, and a launch leaves the counter as it found it: also where two launches met on the same
+// counters (a graph replayed beside other work of the stream it was captured on), whatever slices each has, the next one counts from zero.
+__host__ __device__ constexpr unsigned int fold_share(int slice, int slices) {
+    const unsigned int even = 0xFFFFFFFFu / static_cast<unsigned int>(slices);
+    return slice == 0 ? 0u - even * static_cast<unsigned int>(slices - 1) : even;
+}
 struct PairArgs {
     KernelArgs input, weight;
     int first_blocks, weight_first;  // set by the launch: the workgroups of the call that starts first

@@ -100,7 +100,7 @@ constexpr bool plain_apart = BM == 128 && !SPLIT && !RESIDUAL && !SWIGLU && !GRA
 // The K slices of a 128 x 128 tile, each in the accumulators of a workgroup: everybody leaves its own in memory, takes a ticket, and
 // the last one adds them up in slice order (whoever it is) and goes on with the sum. Written through to the memory behind the XCDs'
 // L2s and read from there: the workgroups of a tile run on any XCD. In the accumulators' own layout, 16 bytes per lane: whole
-// cache lines, and no way through LDS. The ticket is left at zero. True for the last one.
+// cache lines, and no way through LDS. True for the last one (fold_share says how it knows).
 template <typename T, int TM, int TN, bool SUMS>
 __device__ __forceinline__ bool fold_slices(const KernelArgs& p, acc_t (&acc)[TM][TN], acc_t (&column_sums)[SUMS ? TM : 1], bool sums,
                                             int slice, int tiles, int tile, int wm, unsigned char* smem_raw) {
@@ -137,13 +137,11 @@ __device__ __forceinline__ bool fold_slices(const KernelArgs& p, acc_t (&acc)[TM
     __syncthreads();
     auto* const arrived = reinterpret_cast<unsigned int*>(smem_raw);
     if (threadIdx.x == 0) {
-        unsigned int* const ticket = p.fold_tickets + tile;
-        const unsigned int before = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (before + 1 == static_cast<unsigned int>(p.slices)) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *arrived = before;
+        const unsigned int share = fold_share(slice, p.slices);
+        *arrived = __hip_atomic_fetch_add(p.fold_tickets + tile, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + share;
     }
     __syncthreads();
-    const bool last = __builtin_amdgcn_readfirstlane(*arrived) + 1 == static_cast<unsigned int>(p.slices);
+    const bool last = __builtin_amdgcn_readfirstlane(*arrived) == 0u;
     __syncthreads();
     if (!last) return false;
     for (int s = 0; s < p.slices; ++s) {

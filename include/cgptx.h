@@ -15,7 +15,11 @@
  * scratch only makes it faster (padded copies of ragged operands, split-K
  * partials of contractions other than whole, long ones, shared key blocks).
  * Run each op once eagerly before capture, exactly as the reference warms up
- * before cudaStreamBeginCapture (train/train.cpp:545-548).
+ * before cudaStreamBeginCapture (train/train.cpp:545-548). A recorded call keeps
+ * the scratch of the stream it was captured on: replays, on whatever stream, have
+ * to be ordered with the library's other work on that stream and with other graphs
+ * captured there, or their results and that work's are undefined (later calls are
+ * not touched). cgptx_release_scratch ends the use of such graphs.
  *
  * Threading: one host thread per stream, as in the reference.
  */

@@ -1,9 +1,11 @@
 // How contractions are cut and which of them share a launch: the rules of cgpt_amd/csrc/gemm.hip, read where they stand. Host code
 // only, no GPU needed. Built by `python -m cgpt_amd.build`; run by tests/test_cpp_interface.py.
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <random>
 #include <string>
+#include <vector>
 
 #include "gemm.hip"
 
@@ -108,11 +110,43 @@ void check_chains() {
     expect(joined > 100 && refused > 10, std::to_string(joined) + " groups joined, " + std::to_string(refused) + " not");
 }
 
+// The counters of tiles in K slices: the last workgroup of a launch, and only it, finds zero; launches that meet on a counter, whose
+// workgroups come in any order, may mistake each other's for the last one, but leave zero for the next.
+void check_counters() {
+    std::mt19937 rng(3);
+    unsigned int counter = 0;
+    auto launch = [&](std::vector<int> slice_counts) {  // how often somebody found zero
+        std::vector<unsigned int> shares;
+        for (const int slices : slice_counts)
+            for (int s = 0; s < slices; ++s) shares.push_back(fold_share(s, slices));
+        std::shuffle(shares.begin(), shares.end(), rng);
+        int last = 0;
+        for (std::size_t i = 0; i < shares.size(); ++i) {
+            counter += shares[i];
+            if (counter == 0) {
+                ++last;
+                if (slice_counts.size() == 1) expect(i + 1 == shares.size(), "an early last workgroup of " + std::to_string(slice_counts[0]));
+            }
+        }
+        return last;
+    };
+    for (int slices = 2; slices <= 16; ++slices)
+        for (int other = 2; other <= 16; ++other) {
+            const std::string name = std::to_string(slices) + " and " + std::to_string(other) + " slices";
+            launch({slices, other});
+            expect(counter == 0, name + ": the counter is left at " + std::to_string(counter));
+            launch({other, slices, other});
+            expect(counter == 0, name + ": the counter is left at " + std::to_string(counter) + " by three");
+            for (const int alone : {slices, other}) expect(launch({alone}) == 1, name + ": not one last workgroup afterwards");
+        }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "pinned") == 0) check_pinned();
     if (argc > 1 && std::strcmp(argv[1], "chains") == 0) check_chains();
+    if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
     std::printf("%d failure(s)\n", failures);
     return failures == 0 ? 0 : 1;
 }

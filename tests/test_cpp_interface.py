@@ -123,3 +123,9 @@ def test_fp32_gradients_that_share_a_launch_have_no_longer_chains():
     """tests/cpp/gemm_plan_test.cpp: q's, k's and v's gradients in fp32 join only where no sum becomes a longer chain of additions
     than it is in the launches they stand for (the rounding error of a chain grows with its length)."""
     run_plan_test("chains")
+
+
+def test_launches_that_meet_on_a_tile_counter_leave_it_at_zero():
+    """tests/cpp/gemm_plan_test.cpp: the shares by which the K slices of a tile count themselves, in random orders of arrival, alone
+    and with other launches between (counting by ones, two such launches left every later one on the stream with a wrong count)."""
+    run_plan_test("counters")

@@ -424,3 +424,54 @@ def test_both_gradients_on_large_tiles_share_a_launch(device, rows, fin, fout, a
         for name, got, exact, old in zip(("dX", "dW", "db"), outputs, want, base):
             assert torch.equal(got.cpu(), (exact + old if accumulate else exact).to(dtype)), name
     assert launches(lambda: ops.linear_backward(*outputs, dy, x, w, options=options)) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_gradients_in_k_slices_replay_from_a_graph(device, dtype):
+    """dW in K slices, recorded: replays between eager calls with another number of slices on the same counters, which all start
+    from zero. Then a replay on another stream beside eager work of the first: those two share scratch and their results are
+    undefined, but what comes after them is not."""
+    shapes = [(4100, 768, 768), (5005, 1024, 1024)]  # five slices, three
+    g = torch.Generator().manual_seed(5)
+    integers = lambda *shape: torch.randint(-1, 2, shape, generator=g).float()
+    calls = []
+    for rows, fin, fout in shapes:
+        x, w, dy = integers(rows, fin), integers(fout, fin), integers(rows, fout)
+        want = [t.to(dtype).to(device) for t in (dy @ w, dy.T @ x, dy.sum(0))]  # whole numbers: exact in any order of additions
+        operands = [t.to(dtype).to(device) for t in (dy, x, w)]
+        calls.append((operands, want, [torch.empty_like(t) for t in want]))
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def run(which):
+        operands, _, outputs = calls[which]
+        ops.linear_backward(*outputs, *operands)
+
+    def check(which, call):
+        for out in calls[which][2]:
+            out.fill_(float("nan"))
+        call()
+        torch.cuda.synchronize()
+        for name, got, exact in zip(("dX", "dW", "db"), calls[which][2], calls[which][1]):
+            assert torch.equal(got, exact), name
+
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        assert launches(lambda: run(0)) == 1 and launches(lambda: run(1)) == 1
+        check(0, lambda: run(0))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+            run(0)
+        for _ in range(3):
+            check(0, graph.replay)
+            check(1, lambda: run(1))
+    torch.cuda.synchronize()
+    for _ in range(4):
+        with torch.cuda.stream(other):
+            graph.replay()
+        with torch.cuda.stream(stream):
+            run(1)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(2):
+            check(1, lambda: run(1))
+            check(0, graph.replay)
