@@ -285,15 +285,16 @@ double predicted_us(int tile, long tiles, long slices, long k_tiles, double part
     return slices > 1 ? time + 3.0 + 0.45 * partial_mb + 0.3 * std::min(partial_mb, 8.0) : time;
 }
 
+bool c_streams(const GemmArgs& g, std::size_t elem);
+
 // Whether 256 x 192 tiles take a call: 16-bit storage, nothing but products, a residual, an fp32 addend and what C holds added, C
-// in one buffer on rows of whole 16 bytes.
+// in one buffer, it and what is added in whole aligned chunks.
 bool takes_narrow_tiles(const GemmArgs& g) {
     constexpr std::size_t kMostPitch = std::size_t{1} << 21;  // 32-bit offsets within a wavefront's 128 rows of fp32
-    const std::size_t c_elem = g.c_is_f32 ? 4 : 2;
     return g.dtype != CGPTX_F32 && g.bias == nullptr && g.a_sums == nullptr && g.swiglu_out == nullptr && g.swiglu_saved == nullptr &&
            g.c_segments.count == 0 && g.batch_rows == 0 && (g.a_k_contiguous || (!g.b_k_contiguous && g.a_segments.count == 0)) &&
            (g.a_segments.count == 0 || !g.b_k_contiguous) && !(g.residual != nullptr && (g.c_is_f32 || g.accumulate)) &&
-           !(g.addend_f32 != nullptr && g.c_is_f32 && g.accumulate) && g.n % 8 == 0 && (g.ldc * c_elem) % 16 == 0 && is_aligned16(g.c) &&
+           !(g.addend_f32 != nullptr && g.c_is_f32 && g.accumulate) && c_streams(g, 2) &&
            g.ldc < kMostPitch && g.ldr < kMostPitch && g.ld_addend < kMostPitch;
 }
 

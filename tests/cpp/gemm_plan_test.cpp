@@ -66,6 +66,42 @@ void check_pinned() {
                 }
 }
 
+// Calls whose columns leave square tiles idle take 256 x 192 ones where C and all that is added lie in whole aligned chunks: those
+// tiles have no other epilogue. The rest is served by square tiles, element by element.
+void check_narrow() {
+    for (const int dtype : {CGPTX_BF16, CGPTX_F16})
+        for (const Kind kind : {Kind::forward, Kind::input_gradient}) {
+            const GemmArgs plain = contraction(kind, 16384, 768, 4096, dtype);
+            auto expect_tile = [&](const GemmArgs& g, bool narrow, const char* what) {
+                expect((make_plan(g).tile == 192) == narrow, name_of(g) + ", " + what + ": tiles of " + std::to_string(make_plan(g).tile));
+                expect(make_plan(g).tile != 192 || c_streams(g, 2), name_of(g) + ", " + what + ": tiles without an epilogue for it");
+            };
+            expect_tile(plain, true, "plain");
+            for (const std::size_t offset : {0, 2, 8}) {  // residuals are read four elements at a time
+                GemmArgs g = plain;
+                g.residual = address(offset);
+                g.ldr = 768;
+                expect_tile(g, offset != 2, "residual");
+                g.ldr = 770;
+                expect_tile(g, false, "residual in rows of 770");
+            }
+            for (const std::size_t offset : {0, 4, 8}) {
+                GemmArgs g = plain;
+                g.addend_f32 = static_cast<const float*>(address(offset));
+                g.ld_addend = 768;
+                expect_tile(g, offset == 0, "addend");
+                g.ld_addend = 770;
+                expect_tile(g, false, "addend in rows of 770");
+            }
+            GemmArgs g = plain;
+            g.c = address(8);
+            expect_tile(g, false, "C on 8 bytes");
+            g.c = address();
+            g.ldc = 772;
+            expect_tile(g, false, "C in rows of 772");
+        }
+}
+
 // q's, k's and v's gradients over `rows` tokens as one group: their input gradients as one call in segments, then the weight gradients.
 struct Gradients {
     GemmArgs calls[4], input[3];
@@ -146,6 +182,7 @@ void check_counters() {
 int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "pinned") == 0) check_pinned();
     if (argc > 1 && std::strcmp(argv[1], "chains") == 0) check_chains();
+    if (argc > 1 && std::strcmp(argv[1], "narrow") == 0) check_narrow();
     if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
     std::printf("%d failure(s)\n", failures);
     return failures == 0 ? 0 : 1;

@@ -129,3 +129,9 @@ def test_launches_that_meet_on_a_tile_counter_leave_it_at_zero():
     """tests/cpp/gemm_plan_test.cpp: the shares by which the K slices of a tile count themselves, in random orders of arrival, alone
     and with other launches between (counting by ones, two such launches left every later one on the stream with a wrong count)."""
     run_plan_test("counters")
+
+
+def test_tiles_of_192_columns_take_what_their_epilogue_serves():
+    """tests/cpp/gemm_plan_test.cpp: a residual or an fp32 addend that does not lie in whole aligned chunks keeps a call on square
+    tiles (on 256 x 192 ones it would end in an error)."""
+    run_plan_test("narrow")
