@@ -795,8 +795,8 @@ __device__ __forceinline__ void deposit_sums(vec_t<float, 4>* to, const acc_t (&
         for (int q = 0; q < 4; ++q)
             to[(4 * t + q) * kWave] = vec_t<float, 4>{sums[t][4 * q], sums[t][4 * q + 1], sums[t][4 * q + 2], sums[t][4 * q + 3]};
 }
-// Which of the two products is rounded is written out: left to the compiler it changed with the code around the call, and the
-// bits of a training step hang on it.
+// Which of the two products is rounded is written out, here and where the parts' sums of probabilities meet: left to the compiler it
+// may change with the code around it, and two kernels that promise each other's bits would differ.
 template <int DT>
 __device__ __forceinline__ void add_sums(const vec_t<float, 4>* from, acc_t (&sums)[DT], float mine, float other) {
 #pragma unroll
@@ -805,10 +805,7 @@ __device__ __forceinline__ void add_sums(const vec_t<float, 4>* from, acc_t (&su
         for (int q = 0; q < 4; ++q) {
             const vec_t<float, 4> v = from[(4 * t + q) * kWave];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float sum = sums[t][4 * q + e];
-                sums[t][4 * q + e] = 4 * t + q < (DT == 2 ? 6 : 3) ? fmaf(v[e], other, sum * mine) : fmaf(sum, mine, v[e] * other);
-            }
+            for (int e = 0; e < 4; ++e) sums[t][4 * q + e] = fmaf(sums[t][4 * q + e], mine, v[e] * other);
         }
 }
 
@@ -979,7 +976,7 @@ __device__ __forceinline__ void forward_block(Params p, T* lds, T* meet_at, floa
         const float top_b = top == -INFINITY ? 0.0f : top * scale2;
         const float mine = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mb - top_b);
         const float other = theirs[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(theirs[0] * scale2 - top_b);
-        l = l * mine + theirs[1] * other;
+        l = fmaf(l, mine, theirs[1] * other);
         add_sums<DT>(meet, o, mine, other);
         mb = top_b;
     }
