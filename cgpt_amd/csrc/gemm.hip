@@ -713,15 +713,22 @@ long slice_steps(long steps, long slices) { return ((steps + slices - 1) / slice
 // of [rows, in] x out, us, calls of their own (or the small group) and a pair: 2000 x 1024 x 2048 34.3 -> 22.3, 5005 x 1024 x 1024 38.0 -> 29.6,
 // 5005 x 1024 x 2048 59.0 -> 50.3, 4096 x 768 x 2048 45.0 -> 32.5, 8192 x 1024 x 2048 74.7 -> 65.0; 1000 x 1024 x 1024 12.4 and 13.0,
 // 8192 x 256 x 256 17.0 and 20.6 (partial tiles), 16384 x 1024 x 4096 225 and 229 (256 x 256 tiles): those stay as they were.
-double predicted_pair_us(long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units) {
+// The slots are only walked where the answer can be below `worth`: a bound is returned where not (the walk is most of what planning a
+// large call costs, up to 1.5 us).
+double predicted_pair_us(long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units, double worth) {
     const long kt = slices > 1 ? slice_steps(steps_w, slices) : steps_w, items_w = tiles_w * slices, items = tiles_x + items_w;
     const bool weight_first = kt >= steps_x;
     const long counts[2] = {weight_first ? items_w : tiles_x, weight_first ? tiles_x : items_w};
     const long lengths[2] = {weight_first ? kt : steps_x, weight_first ? steps_x : kt};
     const double work = static_cast<double>(tiles_x * steps_x + items_w * kt) / static_cast<double>(units);
+    const double fold = slices > 1 ? 3.0 * static_cast<double>(items_w) / static_cast<double>(units) + 0.9 * static_cast<double>(slices) : 0.0;
     // K steps of the CU that ends last: of its longer slot, and of the one beside it.
     double longest = static_cast<double>(lengths[0]), beside = 0.0;
+    auto time = [&]() { return 5.6 + std::max(0.22 * (longest - beside) + 0.47 * beside + fold, 0.237 * work); };
     if (items > 2 * units) {
+        longest = std::max(longest, work / 2.0);  // no slot order has a shorter longest one
+        beside = work / 2.0;
+        if (time() >= worth) return time();
         // Slots by the steps they have been given: the least loaded ones take the next workgroups.
         struct Slots {
             long steps, count;
@@ -749,8 +756,7 @@ double predicted_pair_us(long tiles_x, long steps_x, long tiles_w, long steps_w,
     } else if (items > units) {
         beside = static_cast<double>(counts[0] > units ? lengths[0] : lengths[1]);
     }
-    const double fold = slices > 1 ? 3.0 * static_cast<double>(items_w) / static_cast<double>(units) + 0.9 * static_cast<double>(slices) : 0.0;
-    return 5.6 + std::max(0.22 * (longest - beside) + 0.47 * beside + fold, 0.237 * work);
+    return time();
 }
 
 // A group's tiles: those whose predicted time in one launch is least. The launch takes as long as its longest workgroup or
@@ -789,7 +795,7 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
         const long tiles_x = tiles_128(calls[0]), tiles_w = tiles_128(calls[1]), steps_x = k_steps_16bit(calls[0]), steps_w = k_steps_16bit(calls[1]);
         for (long s = 1; s <= 16 && tiles_w <= kTickets && (s == 1 || steps_w / s >= 8); ++s) {
             if (slice_steps(steps_w, s) * (s - 1) >= steps_w) continue;
-            const double time = predicted_pair_us(tiles_x, steps_x, tiles_w, steps_w, s, compute_units());
+            const double time = predicted_pair_us(tiles_x, steps_x, tiles_w, steps_w, s, compute_units(), best);
             if (time < best) {
                 best = time;
                 best_plan.joined = best_plan.pair = true;

@@ -146,6 +146,25 @@ void check_chains() {
     expect(joined > 100 && refused > 10, std::to_string(joined) + " groups joined, " + std::to_string(refused) + " not");
 }
 
+// The prediction of a pair stops short where it cannot be below what the caller has already; it never says otherwise than the whole one.
+void check_predictions() {
+    std::mt19937 rng(4);
+    int stopped = 0;
+    for (int i = 0; i < 3000; ++i) {
+        const long tiles_x = 1 + static_cast<long>(rng() % 4000), tiles_w = 1 + static_cast<long>(rng() % 1000), steps_x = 2 + static_cast<long>(rng() % 128);
+        const long steps_w = 2 + static_cast<long>(rng() % 1024), slices = 1 + static_cast<long>(rng() % 12);
+        auto predicted = [&](double worth) { return predicted_pair_us(tiles_x, steps_x, tiles_w, steps_w, slices, 256, worth); };
+        const double whole = predicted(std::numeric_limits<double>::infinity());
+        for (const double worth : {0.5 * whole, 0.97 * whole, 1.03 * whole}) {
+            const double short_of = predicted(worth);
+            stopped += short_of != whole;
+            expect((short_of < worth) == (whole < worth) && (short_of >= worth || short_of == whole),
+                   std::to_string(whole) + " predicted as " + std::to_string(short_of) + " for " + std::to_string(worth));
+        }
+    }
+    expect(stopped > 100, "nothing was stopped short");
+}
+
 // The counters of tiles in K slices: the last workgroup of a launch, and only it, finds zero; launches that meet on a counter, whose
 // workgroups come in any order, may mistake each other's for the last one, but leave zero for the next.
 void check_counters() {
@@ -184,6 +203,7 @@ int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "chains") == 0) check_chains();
     if (argc > 1 && std::strcmp(argv[1], "narrow") == 0) check_narrow();
     if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
+    if (argc > 1 && std::strcmp(argv[1], "predictions") == 0) check_predictions();
     std::printf("%d failure(s)\n", failures);
     return failures == 0 ? 0 : 1;
 }

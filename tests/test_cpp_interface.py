@@ -135,3 +135,9 @@ def test_tiles_of_192_columns_take_what_their_epilogue_serves():
     """tests/cpp/gemm_plan_test.cpp: a residual or an fp32 addend that does not lie in whole aligned chunks keeps a call on square
     tiles (on 256 x 192 ones it would end in an error)."""
     run_plan_test("narrow")
+
+
+def test_predictions_that_stop_short_decide_as_whole_ones():
+    """tests/cpp/gemm_plan_test.cpp: what both gradients of a projection take in one launch, predicted only as far as the answer
+    can matter."""
+    run_plan_test("predictions")
