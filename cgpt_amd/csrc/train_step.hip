@@ -840,10 +840,9 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         // out = x + attention_projection, then out += ffn_output (src/core/transformer_block.cu:594-595)
         CGPTX_OP("gemm_fwd.o", linear_forward_residual(out, a.attn_out, w.o.value, x, false, N, QW, H, dt, stream));
         if (!dual_norms) CGPTX_OP("rmsnorm_fwd", cgptx_rmsnorm_forward(a.norm_f, x, w.ffn_norm.value, N, H, eps, dt, s));
-        if (first_group.joined) {
-        } else if (fused_swiglu()) {
+        if (!first_group.joined && fused_swiglu()) {
             CGPTX_OP("gemm_fwd.gate_up", cgptx_linear_swiglu_forward(a.gate_up, a.act, a.norm_f, w.gate.value, N, H, I, dt, s));
-        } else {
+        } else if (!first_group.joined) {
             CGPTX_OP("gemm_fwd.gate_up", cgptx_linear_forward(a.gate_up, a.norm_f, w.gate.value, nullptr, N, H, 2 * I, dt, s));
             CGPTX_OP("swiglu_fwd", cgptx_swiglu_forward_packed(a.act, a.gate_up, N, I, dt, s));
         }
@@ -919,25 +918,25 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
         fused_last.ld_swiglu = 2 * I;
         const bool qk_in_one = fused_qk_norm_rope(m, d_q, d_q, a.q_pre, w.q_norm.value) && fused_qk_norm_rope(m, d_k, d_k, a.k_pre, w.k_norm.value);
         const bool fills_chip = gemm_fuses_swiglu_gradient(fused_last);
-        bool down_alike = true;  // the down projection's gradients, each by itself, add as a group would
-        for (int i = 0; i < last_down; ++i) down_alike = down_alike && gemm_adds_as_joined(last_parts + i, 1, stream);
-        const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && fused_swiglu_gradient() && !fills_chip &&
-                                       swiglu_beside_norms(swiglu, dt) && down_alike &&
+        bool down_alike = !fills_chip;  // and each of the down projection's gradients by itself adds as a group would
+        for (int i = 0; i < last_down && down_alike; ++i) down_alike = gemm_adds_as_joined(last_parts + i, 1, stream);
+        const bool branches_together = dual_norms && qk_in_one && fused_swiglu() && fused_swiglu_gradient() && down_alike &&
+                                       swiglu_beside_norms(swiglu, dt) &&
                                        gemm_adds_as_joined(last_parts + last_down, last_count - last_down, stream);
+        const GemmGroup last_group = branches_together ? gemm_joins(last_parts, last_count, stream, false) : GemmGroup{};
         const GemmArgs* const qkv_gradients = first_parts + first_gate_up;  // with the weights' unless those are stacked
         // Without a launch of their own q's, k's and v's input gradients are added up in storage, rounded each time: a group of all
         // six would add them in fp32.
-        const bool qkv_gradients_alike = dt != CGPTX_F32 || gemm_segments_add_as_joined(qkv_gradients, stream);
-        const GemmGroup qkv_gradient_group = fused_qkv || !qkv_gradients_alike ? GemmGroup{} : gemm_joins(qkv_gradients, 4, stream);
-        const bool first_together = gemm_adds_as_joined(first_parts, first_gate_up, stream) && (fused_qkv
+        const bool qkv_gradients_alike = !fused_qkv && (dt != CGPTX_F32 || gemm_segments_add_as_joined(qkv_gradients, stream));
+        const GemmGroup qkv_gradient_group = qkv_gradients_alike ? gemm_joins(qkv_gradients, 4, stream) : GemmGroup{};
+        const bool first_together = last_group.joined && gemm_adds_as_joined(first_parts, first_gate_up, stream) && (fused_qkv
             ? gemm_adds_as_joined(fused_qkv_gradients, 1, stream) && (stacked || gemm_adds_as_joined(fused_qkv_gradients + 1, 1, stream))
             : qkv_gradient_group.joined);
-        const GemmGroup last_group = branches_together ? gemm_joins(last_parts, last_count, stream, false) : GemmGroup{};
-        const GemmGroup first_group = last_group.joined && first_together ? gemm_joins(first_parts, first_count, stream, false) : GemmGroup{};
+        const GemmGroup first_group = first_together ? gemm_joins(first_parts, first_count, stream, false) : GemmGroup{};
         if (last_group.joined) {
             CGPTX_SHARED_OP(stacked ? "gemm_dx.down" : "gemm_dx_dw.down", stacked ? "gemm_dx.o" : "gemm_dx_dw.o", last_parts, last_count, last_down,
                             gemm_joined(last_parts, last_count, last_group, stream));
-        } else if ((fills_chip || !down_alike) && fused_swiglu() && fused_swiglu_gradient()) {
+        } else if (!down_alike && fused_swiglu() && fused_swiglu_gradient()) {
             // The SwiGLU gradient rides in the epilogue of the down projection's input gradient, where that fills the chip.
             CGPTX_OP("gemm_dx.down", cgptx_linear_swiglu_backward(d_gate_up, m->d_act, current, w.down.value, a.gate_up, N, I, H, dt, s));
             if (!stacked)
