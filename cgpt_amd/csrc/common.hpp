@@ -265,6 +265,14 @@ unsigned int* tickets(hipStream_t stream);
 // holds the block's address, so whoever replays one compares this value with the one at capture time
 // and captures again when they differ.
 std::uint64_t scratch_generation(hipStream_t stream);
+// While one lives on a thread, what is recorded there is only replayed behind a look at scratch_generation: the arena's block may go when
+// it grows. The block that any other recorded call works in is kept.
+struct ScratchWatch {
+    ScratchWatch();
+    ~ScratchWatch();
+    ScratchWatch(const ScratchWatch&) = delete;
+    ScratchWatch& operator=(const ScratchWatch&) = delete;
+};
 
 // Number of compute units of the current device (cached).
 int compute_units();

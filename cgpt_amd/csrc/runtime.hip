@@ -4,6 +4,7 @@
 #include <map>
 #include <mutex>
 #include <utility>
+#include <vector>
 
 namespace cgptx {
 namespace {
@@ -15,7 +16,10 @@ struct Arena {
     std::size_t bytes = 0;
     std::uint64_t generation = 0;  // value of g_generation when this block was allocated
     unsigned int* tickets = nullptr;
+    bool recorded = false;       // a caller's graph may hold this block's address
+    std::vector<void*> retired;  // earlier blocks of which that was so
 };
+thread_local int g_watches = 0;  // see ScratchWatch
 
 std::mutex g_arena_mutex;
 std::map<std::pair<int, hipStream_t>, Arena> g_arenas;
@@ -35,17 +39,21 @@ int check_hip(hipError_t error, const char* what) {
     return fail(CGPTX_RUNTIME, std::string(what) + ": " + hipGetErrorString(error));
 }
 
-// Grows the stream's arena to `bytes` where that is possible. *result: the arena as it then is. *capturing, *allocation: what
+ScratchWatch::ScratchWatch() { ++g_watches; }
+ScratchWatch::~ScratchWatch() { --g_watches; }
+
+// Grows the stream's arena to `bytes` where that is possible. *data, *held: the arena as it then is. *capturing, *allocation: what
 // was in the way if it holds less.
-static int grow_arena(hipStream_t stream, std::size_t bytes, Arena* result, bool* capturing, hipError_t* allocation) {
+static int grow_arena(hipStream_t stream, std::size_t bytes, void** data, std::size_t* held, bool* capturing, hipError_t* allocation) {
     int device = 0;
     CGPTX_HIP(hipGetDevice(&device));
     std::lock_guard<std::mutex> lock(g_arena_mutex);
     Arena& arena = g_arenas[{device, stream}];
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (stream != nullptr && (arena.bytes < bytes || !arena.recorded)) CGPTX_HIP(hipStreamIsCapturing(stream, &capture));
+    *capturing = capture != hipStreamCaptureStatusNone;
+    if (*capturing && g_watches == 0) arena.recorded = true;
     if (arena.bytes < bytes) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (stream != nullptr) CGPTX_HIP(hipStreamIsCapturing(stream, &capture));
-        *capturing = capture != hipStreamCaptureStatusNone;
         // Round up so that small variations in problem size do not reallocate.
         const std::size_t rounded = (bytes + (std::size_t{1} << 20) - 1) & ~((std::size_t{1} << 20) - 1);
         void* fresh = nullptr;
@@ -53,39 +61,38 @@ static int grow_arena(hipStream_t stream, std::size_t bytes, Arena* result, bool
         if (*allocation != hipSuccess) (void)hipGetLastError();  // reported from here, not by the next launch
         if (fresh != nullptr) {
             if (arena.data != nullptr) {
-                // hipFree waits for outstanding work that may still read the old block.
-                CGPTX_HIP(hipFree(arena.data));
+                // hipFree waits for outstanding work that may still read the old block. One that a recorded call of the caller's works
+                // in stays until cgptx_release_scratch: its graph may be replayed at any time.
+                if (arena.recorded) arena.retired.push_back(arena.data);
+                else CGPTX_HIP(hipFree(arena.data));
             }
             arena.data = fresh;
             arena.bytes = rounded;
+            arena.recorded = false;
             arena.generation = ++g_generation;
         }
     }
-    *result = arena;
+    *data = arena.data;
+    *held = arena.bytes;
     return CGPTX_OK;
 }
 
 int scratch(hipStream_t stream, std::size_t bytes, void** out) {
-    Arena arena;
+    std::size_t held = 0;
     bool capturing = false;
     hipError_t allocation = hipSuccess;
-    if (int s = grow_arena(stream, bytes, &arena, &capturing, &allocation)) return s;
-    if (capturing)
+    if (int s = grow_arena(stream, bytes, out, &held, &capturing, &allocation)) return s;
+    if (held < bytes && capturing)
         return fail(CGPTX_CAPTURE_ALLOC,
                     "scratch arena would have to grow during stream capture; run the op once eagerly first");
     CGPTX_HIP(allocation);
-    *out = arena.data;
     return CGPTX_OK;
 }
 
 int scratch_up_to(hipStream_t stream, std::size_t bytes, void** out, std::size_t* held) {
-    Arena arena;
     bool capturing = false;
     hipError_t allocation = hipSuccess;
-    if (int s = grow_arena(stream, bytes, &arena, &capturing, &allocation)) return s;
-    *out = arena.data;
-    *held = arena.bytes;
-    return CGPTX_OK;
+    return grow_arena(stream, bytes, out, held, &capturing, &allocation);
 }
 
 unsigned int* tickets(hipStream_t stream) {
@@ -157,6 +164,7 @@ extern "C" int cgptx_release_scratch(void) {
         if (it->first.first == device) {
             if (it->second.data != nullptr) CGPTX_HIP(hipFree(it->second.data));
             if (it->second.tickets != nullptr) CGPTX_HIP(hipFree(it->second.tickets));
+            for (void* block : it->second.retired) CGPTX_HIP(hipFree(block));
             it = g_arenas.erase(it);
         } else {
             ++it;

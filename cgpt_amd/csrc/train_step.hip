@@ -1471,6 +1471,7 @@ int run_step(cgptx_model* m, float loss_scale, int loss_mode, int use_graph, boo
         step.exec = nullptr;
     }
     CGPTX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+    const ScratchWatch watch;
     const int status = enqueue_step(m, loss_scale, loss_mode, with_optimizer, stream);
     hipGraph_t graph = nullptr;
     const hipError_t end = hipStreamEndCapture(stream, &graph);

@@ -19,7 +19,8 @@
  * the scratch of the stream it was captured on: replays, on whatever stream, have
  * to be ordered with the library's other work on that stream and with other graphs
  * captured there, or their results and that work's are undefined (later calls are
- * not touched). cgptx_release_scratch ends the use of such graphs.
+ * not touched). An arena that grows later leaves the block that a recorded call
+ * works in until cgptx_release_scratch, which ends the use of such graphs.
  *
  * Threading: one host thread per stream, as in the reference.
  */
@@ -53,7 +54,8 @@ typedef void* cgptx_stream; /* hipStream_t */
 const char* cgptx_last_error(void);
 /* Library version string. */
 const char* cgptx_version(void);
-/* Releases every scratch arena of the current device (synchronises the device). */
+/* Releases every scratch arena of the current device (synchronises the device). Graphs of calls that work in one, recorded before, must
+ * not be replayed any more; the composed step (cgptx_train.h) records its own anew. */
 int cgptx_release_scratch(void);
 /* Bytes of the scratch arena bound to (current device, stream): the largest request any operator has made on
  * that stream so far, rounded up to 1 MiB; 0 when the stream has none. For a train step it is dominated by the

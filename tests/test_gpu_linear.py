@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from cgpt_amd import ops
+from cgpt_amd import capi, ops
 from oracle import cpu_ops, oracle64
 from tests.util import DTYPES, DTYPE_IDS, TOL, assert_close, launches, randn, to_np
 
@@ -429,8 +429,9 @@ def test_both_gradients_on_large_tiles_share_a_launch(device, rows, fin, fout, a
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 def test_gradients_in_k_slices_replay_from_a_graph(device, dtype):
     """dW in K slices, recorded: replays between eager calls with another number of slices on the same counters, which all start
-    from zero. Then a replay on another stream beside eager work of the first: those two share scratch and their results are
-    undefined, but what comes after them is not."""
+    from zero, and with partial tiles that make the arena grow, under which the recorded ones stay where they were. Then replays on
+    another stream beside eager work of the first: they share the counters and their results are undefined, but what comes after
+    them is not."""
     shapes = [(4100, 768, 768), (5005, 1024, 1024)]  # five slices, three
     g = torch.Generator().manual_seed(5)
     integers = lambda *shape: torch.randint(-1, 2, shape, generator=g).float()
@@ -454,9 +455,10 @@ def test_gradients_in_k_slices_replay_from_a_graph(device, dtype):
         for name, got, exact in zip(("dX", "dW", "db"), calls[which][2], calls[which][1]):
             assert torch.equal(got, exact), name
 
+    assert launches(lambda: run(0)) == 1 and launches(lambda: run(1)) == 1
     torch.cuda.synchronize()
+    capi.call("cgptx_release_scratch")
     with torch.cuda.stream(stream):
-        assert launches(lambda: run(0)) == 1 and launches(lambda: run(1)) == 1
         check(0, lambda: run(0))
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):

@@ -113,3 +113,39 @@ def test_cut_cross_entropy(device, dtype):
     arena = 4 if dtype == torch.float32 else 2  # 2000 rows of 521 logits take 4.0 or 2.0 MiB, padded 4.15 or 2.08
     for room in (arena, arena + 1):
         check_recorded(device, lambda s: ops.cut_cross_entropy_forward_backward(loss, dx, dw, x, w, targets, 2000, s), [loss, dx, dw], room * MIB)
+
+
+def test_a_recorded_call_keeps_its_scratch(device):
+    """A caller's graph, whose kernels work in the arena as it was: a later call that makes the arena grow leaves that block where it
+    is, replays give what they gave, and cgptx_release_scratch gives all of it back."""
+    stream = torch.cuda.Stream(device=device)
+    rows = 2 << 20  # 4 bytes of scratch per row
+    logits, targets = torch.randn(2 * rows, 2, device=device), torch.zeros(2 * rows, dtype=torch.int32, device=device)
+    loss = torch.empty(1, device=device)
+
+    def call(count):
+        ops.cross_entropy_forward(loss, logits[:count], targets[:count], count, stream)
+
+    free = []
+    for _ in range(20):
+        torch.cuda.synchronize()
+        capi.call("cgptx_release_scratch")
+        free.append(torch.cuda.mem_get_info()[0])
+        call(rows)
+        stream.synchronize()
+        want = loss.clone()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+            call(rows)
+        for _ in range(3):
+            call(2 * rows)
+            stream.synchronize()
+            assert capi.lib().cgptx_scratch_bytes(stream.cuda_stream) == 8 * rows
+            loss.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(loss, want)
+        del graph
+    assert free[1] - free[-1] <= 18 * 4 * rows // 2  # the smaller blocks, kept in every round, would be twice that
