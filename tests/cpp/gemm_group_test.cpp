@@ -312,6 +312,72 @@ void check_segment_sums(std::size_t rows, std::size_t hidden, std::size_t q, std
         }
 }
 
+// Y = X·Wᵀ on tiles of 256 x 192, ragged both ways, with all that their epilogue adds: a residual, sums in fp32, what C holds, into C of
+// either kind. Whole numbers, exact in fp32 whatever the order. Some rows are compared, and the guards around C.
+void check_narrow_epilogue(int dtype, hipStream_t stream) {
+    const std::size_t rows = 16300, columns = 760, k = 1024;
+    std::mt19937 rng(7);
+    const Matrix x = random_matrix(rows, k, rng), w = random_matrix(columns, k, rng);
+    auto wide = [&](int most) {
+        Matrix m{rows, columns, std::vector<int>(rows * columns)};
+        for (int& v : m.values) v = static_cast<int>(rng() % (2 * most + 1)) - most;
+        return m;
+    };
+    const Matrix residual = wide(100), addend = wide(1000), old = wide(100);
+    const Buffer on_x(x, dtype), on_w(w, dtype), on_residual(residual, dtype);
+    const Floats on_addend(std::vector<float>(addend.values.begin(), addend.values.end()));
+    std::vector<std::size_t> some;
+    for (std::size_t r = 0; r < rows; r += 331) some.push_back(r);
+    for (std::size_t r = rows - 3; r < rows; ++r) some.push_back(r);
+    std::vector<int> products;
+    for (const std::size_t r : some)
+        for (std::size_t c = 0; c < columns; ++c) {
+            int sum = 0;
+            for (std::size_t t = 0; t < k; ++t) sum += x.at(r, t) * w.at(c, t);
+            products.push_back(sum);
+        }
+    struct Form {
+        const char* name;
+        bool residual, addend, accumulate, f32;
+    };
+    for (const Form form : {Form{"residual", true, false, false, false}, {"addend", false, true, false, false}, {"addend and residual", true, true, false, false},
+                            {"old C", false, false, true, false}, {"addend and old C", false, true, true, false}, {"fp32", false, false, false, true},
+                            {"fp32, old C", false, false, true, true}, {"fp32, addend", false, true, false, true}}) {
+        const std::string name = std::string("256 x 192 tiles, ") + form.name + (dtype == CGPTX_F16 ? " f16" : " bf16");
+        std::printf("%s\n", name.c_str());
+        std::fflush(stdout);
+        Buffer c16(old, dtype);
+        Floats c32(std::vector<float>(old.values.begin(), old.values.end()));
+        GemmArgs g;
+        g.a = on_x.data();
+        g.b = on_w.data();
+        g.c = form.f32 ? static_cast<void*>(c32.data()) : c16.data();
+        g.m = rows;
+        g.n = g.ldc = columns;
+        g.k = g.lda = g.ldb = k;
+        g.dtype = dtype;
+        g.c_is_f32 = form.f32;
+        g.accumulate = form.accumulate;
+        if (form.residual) g.residual = on_residual.data(), g.ldr = columns;
+        if (form.addend) g.addend_f32 = on_addend.data(), g.ld_addend = columns;
+        expect(cgptx::gemm(g, stream) == CGPTX_OK, name + ": launch");
+        hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        Bits got;
+        expect(c16.copy(got), name + ": guards");
+        const std::vector<float> got32 = c32.copy();
+        for (std::size_t i = 0; i < some.size(); ++i)
+            for (std::size_t c = 0; c < columns; ++c) {
+                const std::size_t at = some[i] * columns + c;
+                const int want = products[i * columns + c] + (form.residual ? residual.values[at] : 0) + (form.addend ? addend.values[at] : 0) +
+                                 (form.accumulate ? old.values[at] : 0);
+                const bool same = form.f32 ? got32[at] == static_cast<float>(want) : got[at] == rounded(want, dtype);
+                if (same) continue;
+                expect(false, name + ": row " + std::to_string(some[i]) + ", column " + std::to_string(c));
+                break;
+            }
+    }
+}
+
 }  // namespace
 
 int main() {
@@ -325,6 +391,7 @@ int main() {
             check(131, 224, 192, 64, 160, dtype, stream);   // ragged rows and columns, five steps in the last segment
             check(300, 512, 512, 64, 224, dtype, stream);   // more rows than one tile of either size
             check_many_rows(16300, 760, 1024, 512, 512, dtype, stream);
+            check_narrow_epilogue(dtype, stream);
         }
         check_segment_sums(300, 512, 512, 512, stream);
         check_segment_sums(131, 768, 768, 256, stream);

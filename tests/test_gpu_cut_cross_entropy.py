@@ -140,6 +140,28 @@ def test_training_shape_against_the_dense_path_and_float64_rows(device, monkeypa
     assert again[0] == loss and torch.equal(again[1], dx) and torch.equal(again[2], dc)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("accumulate", [False, True], ids=["overwrite", "accumulate"])
+def test_chunks_on_tiles_of_192_columns(device, monkeypatch, dtype, accumulate):
+    """[4096, 768] x [32000, 768] in four chunks of 1024 rows: the classifier gradient's 768 columns are four tiles of 192, in fp32
+    the first time, added to the fp32 sums by the second and third, with the sums (and the old gradient) added by the last. Against
+    the gradients of fp32 softmax probabilities."""
+    monkeypatch.setenv("CGPTX_CUT_CE_LOGITS_BYTES", str(64 << 20))
+    rows, hidden, vocab, scale = 4096, 768, 32000, 4096.0
+    x, c = randn((rows, hidden), dtype, 51).to(device), randn((vocab, hidden), dtype, 52, 0.02).to(device)
+    targets = randint(vocab, (rows,), 53).to(device)
+    old = randn((vocab, hidden), dtype, 54, 0.5).to(device)
+    loss, dx, dc = run(device, x, c, targets, scale, accumulate, old)
+    z = x.float() @ c.float().T.contiguous()
+    want_loss = torch.nn.functional.cross_entropy(z, targets.long()).item()
+    z = torch.softmax(z, dim=1)
+    z[torch.arange(rows, device=device), targets.long()] -= 1.0
+    z *= scale / rows
+    assert abs(loss - want_loss) <= 1e-4 * want_loss
+    assert_scaled_close(dx, z @ c.float(), STOL[dtype], "dX")
+    assert_scaled_close(dc, z.T.contiguous() @ x.float() + (old.float() if accumulate else 0.0), STOL[dtype], "dC")
+
+
 def test_argument_errors(device):
     x, c = torch.zeros(4, 8, device=device), torch.zeros(5, 8, device=device)
     t = torch.zeros(4, dtype=torch.int32, device=device)

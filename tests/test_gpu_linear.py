@@ -427,6 +427,37 @@ def test_both_gradients_on_large_tiles_share_a_launch(device, rows, fin, fout, a
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("rows,fin,fout", [
+    (2000, 1024, 2048),   # a workgroup per CU and all of its LDS
+    (4100, 768, 768),     # two per CU, dW in K slices
+])
+@pytest.mark.parametrize("shifted", ["dX", "dW", "both"])
+@pytest.mark.parametrize("accumulate", [False, True], ids=["overwrite", "accumulate"])
+def test_large_gradients_wherever_they_start(device, rows, fin, fout, accumulate, shifted, dtype):
+    """Gradients that start on no multiple of 16 bytes are stored element by element, by one launch all the same, and nothing
+    beside them is written."""
+    g = torch.Generator().manual_seed(rows + fin)
+    integers = lambda *shape: torch.randint(-1, 2, shape, generator=g).float()
+    x, w, dy = integers(rows, fin), integers(fout, fin), integers(rows, fout)
+    base = [integers(rows, fin), integers(fout, fin), integers(fout)]
+    want = [dy @ w, dy.T @ x, dy.sum(0)]  # whole numbers far below 2^24: exact in fp32
+    x, w, dy = (t.to(dtype).to(device) for t in (x, w, dy))
+    buffers, outputs = [], []
+    for name, old in zip(("dX", "dW", "db"), base):
+        first = 16 + (3 if shifted in (name, "both") else 0)
+        buffer = torch.full((old.numel() + 48,), 7.0, dtype=dtype, device=device)
+        outputs.append(buffer[first:first + old.numel()].view(old.shape))
+        outputs[-1].copy_(old) if accumulate else outputs[-1].fill_(float("nan"))
+        buffers.append((buffer, first))
+    options = ops.LinearBackwardOptions(accumulate_input=accumulate, accumulate_weight=accumulate, accumulate_bias=accumulate)
+    ops.linear_backward(*outputs, dy, x, w, options=options)
+    for name, got, exact, old, (buffer, first) in zip(("dX", "dW", "db"), outputs, want, base, buffers):
+        assert torch.equal(got.cpu(), (exact + old if accumulate else exact).to(dtype)), name
+        assert (buffer[:first] == 7.0).all() and (buffer[first + old.numel():] == 7.0).all(), name
+    assert launches(lambda: ops.linear_backward(*outputs, dy, x, w, options=options)) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 def test_gradients_in_k_slices_replay_from_a_graph(device, dtype):
     """dW in K slices, recorded: replays between eager calls with another number of slices on the same counters, which all start
     from zero, and with partial tiles that make the arena grow, under which the recorded ones stay where they were. Then replays on
