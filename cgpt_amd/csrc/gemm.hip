@@ -924,10 +924,9 @@ int run_pair(const GemmArgs* calls, const GemmGroup& plan, hipStream_t stream) {
     }
 }
 
-template <typename T>
-int run_joined(const GemmArgs* calls, int count, const GemmGroup& plan, hipStream_t stream) {
-    if (plan.pair) return run_pair<T>(calls, plan, stream);
-    SmallGroup group{};
+template <typename T, int CALLS>
+int run_group(const GemmArgs* calls, int count, const GemmGroup& plan, hipStream_t stream) {
+    SmallGroup<CALLS> group{};
     long order[kGroupCalls];
     for (int i = 0; i < count; ++i) order[i] = i;
     // The workgroups with the longest K loops start first.
@@ -955,6 +954,12 @@ int run_joined(const GemmArgs* calls, int count, const GemmGroup& plan, hipStrea
     else return gemm_small_f32(group, blocks, plan.deep, stream);
 }
 
+template <typename T>
+int run_joined(const GemmArgs* calls, int count, const GemmGroup& plan, hipStream_t stream) {
+    if (plan.pair) return run_pair<T>(calls, plan, stream);
+    return plan.few ? run_group<T, kFewCalls>(calls, count, plan, stream) : run_group<T, kGroupCalls>(calls, count, plan, stream);
+}
+
 }  // namespace
 
 GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream, bool large_pairs) {
@@ -975,6 +980,7 @@ GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream, bool 
             group = plan_group(calls, count, false);
         }
     }
+    group.few = large_pairs && count <= kFewCalls;
     return group;
 }
 
@@ -1004,7 +1010,7 @@ bool gemm_segments_add_as_joined(const GemmArgs* calls, hipStream_t stream) {
 }
 
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream) {
-    if (!group.joined || count < 2 || count > kGroupCalls) return fail(CGPTX_RUNTIME, "gemm: these calls cannot share a launch");
+    if (!group.joined || count < 2 || count > (group.few ? kFewCalls : kGroupCalls)) return fail(CGPTX_RUNTIME, "gemm: these calls cannot share a launch");
     return dispatch_dtype(calls[0].dtype, [&]<typename T>() -> int { return run_joined<T>(calls, count, group, stream); });
 }
 

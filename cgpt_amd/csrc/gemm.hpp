@@ -82,15 +82,17 @@ struct GemmArgs {
 int gemm(const GemmArgs& args, hipStream_t stream);
 // Up to kGroupCalls calls that neither read nor write each other's results, in one launch: whether that is served and faster than
 // one after the other (few tiles each, operands that stream as they lie) and how their tiles are cut then, and the launch itself.
-constexpr int kGroupCalls = 6;
+constexpr int kGroupCalls = 6, kFewCalls = 2;
 struct GemmGroup {
     int tile[kGroupCalls] = {};
     bool deep = false;  // one workgroup per CU
+    bool few = false;   // launched by the kernel whose arguments hold kFewCalls calls
     bool pair = false;  // an input and a weight gradient on 128 x 128 tiles, the weight gradient in `slices` along K
     int slices = 1;
     bool joined = false;
 };
-// large_pairs: whether an input and a weight gradient may share a launch on 128 x 128 tiles too.
+// large_pairs: whether an input and a weight gradient may share a launch on 128 x 128 tiles too. Left out by steps, which also launch
+// all their groups by one kernel: a second one, fetched cold in between, takes the step of 3 x 100 tokens from 234.2 to 236.2 us.
 GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream = nullptr, bool large_pairs = true);
 int gemm_joined(const GemmArgs* calls, int count, const GemmGroup& group, hipStream_t stream);
 // Whether calls by themselves, or as a group of their own, add in the order that a group gives them: small tiles, one sum over K.

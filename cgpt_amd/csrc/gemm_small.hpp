@@ -47,20 +47,25 @@ struct SmallCall {
 
 // Several calls in one launch: call i takes the workgroups from first_block[i] on, tile rows first.
 enum class SmallLayout { forward, input_gradient, weight_gradient, segmented_input_gradient };
+// The launch's arguments hold as many calls as its kernel is made for.
+template <int CALLS>
 struct SmallGroup {
-    SmallArgs call[kGroupCalls];
-    int first_block[kGroupCalls];
-    int tiles_m[kGroupCalls];
-    int tile[kGroupCalls];  // 32 or 64
-    SmallLayout layout[kGroupCalls];
+    SmallArgs call[CALLS];
+    int first_block[CALLS];
+    int tiles_m[CALLS];
+    int tile[CALLS];  // 32 or 64
+    SmallLayout layout[CALLS];
     int count;
 };
 
 int gemm_small_bf16(const SmallCall& call, hipStream_t stream);
 int gemm_small_f16(const SmallCall& call, hipStream_t stream);
 int gemm_small_f32(const SmallCall& call, hipStream_t stream);
-int gemm_small_bf16(const SmallGroup& group, int blocks, bool deep, hipStream_t stream);
-int gemm_small_f16(const SmallGroup& group, int blocks, bool deep, hipStream_t stream);
-int gemm_small_f32(const SmallGroup& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_bf16(const SmallGroup<kFewCalls>& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_bf16(const SmallGroup<kGroupCalls>& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_f16(const SmallGroup<kFewCalls>& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_f16(const SmallGroup<kGroupCalls>& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_f32(const SmallGroup<kFewCalls>& group, int blocks, bool deep, hipStream_t stream);
+int gemm_small_f32(const SmallGroup<kGroupCalls>& group, int blocks, bool deep, hipStream_t stream);
 
 }  // namespace cgptx

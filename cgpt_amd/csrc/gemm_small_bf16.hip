@@ -3,5 +3,5 @@
 
 namespace cgptx {
 int gemm_small_bf16(const SmallCall& call, hipStream_t stream) { return launch_small<bf16_t>(call, stream); }
-int gemm_small_bf16(const SmallGroup& group, int blocks, bool deep, hipStream_t stream) { return launch_small_group<bf16_t>(group, blocks, deep, stream); }
+int gemm_small_bf16(const SmallGroup<kGroupCalls>& group, int blocks, bool deep, hipStream_t stream) { return launch_small_group<bf16_t>(group, blocks, deep, stream); }
 }  // namespace cgptx

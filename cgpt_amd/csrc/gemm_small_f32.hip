@@ -3,5 +3,5 @@
 
 namespace cgptx {
 int gemm_small_f32(const SmallCall& call, hipStream_t stream) { return launch_small<float>(call, stream); }
-int gemm_small_f32(const SmallGroup& group, int blocks, bool deep, hipStream_t stream) { return launch_small_group<float>(group, blocks, deep, stream); }
+int gemm_small_f32(const SmallGroup<kGroupCalls>& group, int blocks, bool deep, hipStream_t stream) { return launch_small_group<float>(group, blocks, deep, stream); }
 }  // namespace cgptx

@@ -434,18 +434,21 @@ __global__ __launch_bounds__(kThreads) void gemm_small_kernel(SmallArgs p) {
 // around 1 - 2 us), and two calls of a few dozen tiles each find room on the chip side by side. Both gradients of a
 // projection, us in two launches and in one: 128 x 768 x 768 bf16 10.4, 7.7; 512 x 512 x 512 11.0, 7.4; 128 x 768 x 2048 fp32
 // 23.0, 15.7; 2000 x 1024 x 2048 bf16 with bias 46, 34 (the bias's gradient took two launches more).
-template <typename T, bool DEEP>
-__global__ __launch_bounds__(kThreads) void gemm_small_group_kernel(SmallGroup group) {
+// CALLS: six, or two in translation units of their own, for the gradients of one projection. The host writes a launch's arguments across
+// the bus, 1784 bytes for six: linear_backward of 128 x 768 x 768 takes 4.6 us of host time a call with them, 4.0 with two, and the block of
+// 128 tokens, seven such calls of 46 and bound by the host, 200 and 187 us (one stream, calls in a row).
+template <typename T, bool DEEP, int CALLS>
+__global__ __launch_bounds__(kThreads) void gemm_small_group_kernel(SmallGroup<CALLS> group) {
     extern __shared__ __align__(1024) unsigned char smem_raw[];
     const int block = blockIdx.x;
     int which = 0;
 #pragma unroll
-    for (int i = 1; i < kGroupCalls; ++i)
+    for (int i = 1; i < CALLS; ++i)
         if (i < group.count && block >= group.first_block[i]) which = i;
     int first = 0, tiles_m = 0, tile = 0;
     SmallLayout layout = SmallLayout::forward;
 #pragma unroll
-    for (int i = 0; i < kGroupCalls; ++i) {
+    for (int i = 0; i < CALLS; ++i) {
         const int first_i = group.first_block[i], tiles_i = group.tiles_m[i], tile_i = group.tile[i];
         const SmallLayout layout_i = group.layout[i];
         first = which == i ? first_i : first;
@@ -460,7 +463,7 @@ __global__ __launch_bounds__(kThreads) void gemm_small_group_kernel(SmallGroup g
         unsigned int w[kWords];
     } words;
     const auto* source = (const __attribute__((address_space(4))) unsigned int*)__builtin_amdgcn_kernarg_segment_ptr() +
-                         offsetof(SmallGroup, call) / 4 + which * kWords;
+                         offsetof(SmallGroup<CALLS>, call) / 4 + which * kWords;
 #pragma unroll
     for (int i = 0; i < kWords; ++i) words.w[i] = source[i];
     const SmallArgs p = __builtin_bit_cast(SmallArgs, words);
@@ -481,10 +484,10 @@ __global__ __launch_bounds__(kThreads) void gemm_small_group_kernel(SmallGroup g
     else with_tile.template operator()<64>();
 }
 
-template <typename T, bool DEEP>
-int launch_small_group_kernel(const SmallGroup& group, int blocks, hipStream_t stream) {
+template <typename T, bool DEEP, int CALLS>
+int launch_small_group_kernel(const SmallGroup<CALLS>& group, int blocks, hipStream_t stream) {
     constexpr int smem = small_smem_bytes<64, DEEP>() + (DEEP ? 0 : 8192);  // 64 x 64 partial tiles need 68 KiB
-    auto kernel = gemm_small_group_kernel<T, DEEP>;
+    auto kernel = gemm_small_group_kernel<T, DEEP, CALLS>;
     static const hipError_t status =
         hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     CGPTX_HIP(status);
@@ -493,9 +496,9 @@ int launch_small_group_kernel(const SmallGroup& group, int blocks, hipStream_t s
     return CGPTX_OK;
 }
 
-template <typename T>
-int launch_small_group(const SmallGroup& group, int blocks, bool deep, hipStream_t stream) {
-    return deep ? launch_small_group_kernel<T, true>(group, blocks, stream) : launch_small_group_kernel<T, false>(group, blocks, stream);
+template <typename T, int CALLS>
+int launch_small_group(const SmallGroup<CALLS>& group, int blocks, bool deep, hipStream_t stream) {
+    return deep ? launch_small_group_kernel<T, true, CALLS>(group, blocks, stream) : launch_small_group_kernel<T, false, CALLS>(group, blocks, stream);
 }
 
 template <typename T, int TILE, bool DEEP, bool A_K, bool B_K, SmallEpilogue EPILOGUE, bool SEGMENTED>
