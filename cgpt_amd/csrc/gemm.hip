@@ -218,14 +218,35 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma_kernel(KernelArgs p, i
 
 // ------------------------------------------------------------------- host side
 
-// CGPTX_GEMM_TILE=32|64|128|192|256 pins the tile size (for experiments); anything else = automatic, and so is a size that a call's
-// kernels do not have (192 where takes_narrow_tiles says no, 256 in fp32).
+// Oblong tiles run one block per CU: us before and after a block's K loop, of a further one, of a K step on an idle chip and what a
+// full one (whose clock and L2s are shared) adds. Measured as predicted_us says, K from 128 to 4096 and 0.4 to 4 rounds: within 8 per
+// cent. They are taken where they are predicted to take 5 per cent less than the best square tiles or 256 x 192 ones. [M, N] x K, us,
+// best of those and chosen: 5005 x 1024 x 1024 17.7 -> 15.7 (160 x 128), x 2048 27.4 -> 22.5; 7000 x 768 x 2048 28.2 -> 25.2 (192 x 128);
+// 5005 x 2048 x 1024 26.4 -> 23.3 (160 x 256), 10000 x 1024 x 1024 26.3 -> 22.3; 13000 x 4096 x 1024 109 -> 99 (224 x 256). Where a call's
+// square tiles fill the chip they stay: 16384 x 1024 x 1024 30.6 and 35.5 (256 x 128), 2000 x 2048 x 1024 12.0 (128 x 128) and 12.9.
+struct OblongCost {
+    int tile;
+    double first, further, step, step_full;
+};
+constexpr OblongCost kOblongCosts[] = {{oblong_tile(160, 128), 5.6, 2.8, 0.165, 0.085}, {oblong_tile(192, 128), 5.8, 3.2, 0.20, 0.09},
+                                       {oblong_tile(256, 128), 6.2, 4.0, 0.23, 0.13},   {oblong_tile(160, 256), 7.2, 4.2, 0.24, 0.19},
+                                       {oblong_tile(192, 256), 7.5, 4.5, 0.32, 0.17},   {oblong_tile(224, 256), 7.8, 5.0, 0.37, 0.19}};
+const OblongCost& oblong_cost(int tile) {
+    for (const OblongCost& c : kOblongCosts)
+        if (c.tile == tile) return c;
+    return kOblongCosts[0];
+}
+
+// CGPTX_GEMM_TILE=32|64|128|192|256|160128|... pins the tile size (for experiments); anything else = automatic, and so is a size that a call's
+// kernels do not have (192 where takes_narrow_tiles says no, oblong ones where takes_oblong_tiles does, 256 in fp32).
 int forced_tile() {
     static const int value = [] {
         const char* text = std::getenv("CGPTX_GEMM_TILE");
         if (text == nullptr) return 0;
         const int v = std::atoi(text);
-        return (v == 32 || v == 64 || v == 128 || v == 192 || v == 256) ? v : 0;
+        bool oblong = false;
+        for (const OblongCost& c : kOblongCosts) oblong = oblong || c.tile == v;
+        return (v == 32 || v == 64 || v == 128 || v == 192 || v == 256 || oblong) ? v : 0;
     }();
     return value;
 }
@@ -234,9 +255,9 @@ std::size_t round_up(std::size_t v, std::size_t unit) { return (v + unit - 1) / 
 
 // How a call of the streamed kernels is cut: tile, K slices per tile and K steps per slice.
 struct Plan {
-    int tile = 256;  // square, but 192: 256 rows of 192 columns
+    int tile = 256;  // see tile_rows
     static long tiles_of(const GemmArgs& g, int tile) {
-        const std::size_t rows = tile == 192 ? 256 : tile, columns = tile;
+        const std::size_t rows = tile_rows(tile), columns = tile_columns(tile);
         return static_cast<long>((g.m + rows - 1) / rows) * static_cast<long>((g.n + columns - 1) / columns);
     }
     int slices = 1;
@@ -266,7 +287,11 @@ double predicted_us(int tile, long tiles, long slices, long k_tiles, double part
     const double load = static_cast<double>(tiles * slices) / static_cast<double>(units);
     const double blocks = std::ceil(load);
     double time = 0.0;
-    if (f32) {
+    if (tile > 256) {
+        const OblongCost& c = oblong_cost(tile);
+        const double filled = load / blocks;
+        time = c.first + 1.3 * filled + c.further * (blocks - 1.0) + blocks * kt * (c.step + c.step_full * filled);
+    } else if (f32) {
         const double per_tile = tile == 32 ? 0.088 : tile == 64 ? 0.265 : 0.93;
         time = (tile == 32 ? 3.0 : tile == 64 ? 4.0 : 5.0) + kt * per_tile * (tile == 32 ? std::max(1.0, load) : blocks);
     } else if (tile == 192) {
@@ -298,6 +323,14 @@ bool takes_narrow_tiles(const GemmArgs& g) {
            g.ldc < kMostPitch && g.ldr < kMostPitch && g.ld_addend < kMostPitch;
 }
 
+// Whether oblong tiles take a call: 16-bit storage, k-contiguous A, one sum over K, the result stored as it is or with a residual or
+// what C holds added.
+bool takes_oblong_tiles(const GemmArgs& g) {
+    return g.dtype != CGPTX_F32 && g.a_k_contiguous && g.bias == nullptr && g.addend_f32 == nullptr && !g.c_is_f32 && g.a_sums == nullptr &&
+           g.swiglu_out == nullptr && g.swiglu_saved == nullptr && g.batch_rows == 0 && !(g.a_segments.count > 0 && (g.b_k_contiguous || g.residual != nullptr || g.accumulate)) &&
+           !(g.residual != nullptr && g.accumulate) && !(g.c_segments.count > 0 && (g.residual != nullptr || g.accumulate)) && c_streams(g, 2);
+}
+
 Plan make_plan(const GemmArgs& g) {
     Plan plan;
     const long units = compute_units();
@@ -316,7 +349,21 @@ Plan make_plan(const GemmArgs& g) {
             plan.k_tiles_per_slice = (plan.k_tiles_per_slice + kSteps - 1) / kSteps * kSteps;
         plan.slices = static_cast<int>((k_tiles + plan.k_tiles_per_slice - 1) / plan.k_tiles_per_slice);
     };
+    const int pinned = forced_tile();
+    // Oblong tiles in place of plan.tile's, predicted to take `best`: the same sums in the same order.
+    auto try_oblong = [&](double best) {
+        for (const OblongCost& c : kOblongCosts) {
+            if (pinned > 256 && c.tile != pinned) continue;
+            const double time = 1.05 * predicted_us(c.tile, tiles_of(c.tile), 1, k_tiles, 0.0, f32, true, g.b_k_contiguous, units);
+            if (pinned == 0 && time >= best) continue;
+            best = time;
+            plan.tile = c.tile;
+        }
+    };
     if (g.swiglu_out != nullptr || g.swiglu_saved != nullptr || (!f32 && tiles_of(256) >= 3 * units && g.batch_rows == 0)) {
+        // Of more rounds the last one is too small a part.
+        if ((pinned == 0 || pinned > 256) && tiles_of(256) <= 8 * units && takes_oblong_tiles(g))
+            try_oblong(predicted_us(256, tiles_of(256), 1, k_tiles, 0.0, f32, true, g.b_k_contiguous, units));
         set_slices(1);
         return plan;
     }
@@ -336,8 +383,7 @@ Plan make_plan(const GemmArgs& g) {
         set_slices(slices);
         return plan;
     }
-    const int pinned = forced_tile();
-    const int forced = (pinned == 192 && !takes_narrow_tiles(g)) || (f32 && pinned == 256) ? 0 : pinned;
+    const int forced = (pinned == 192 && !takes_narrow_tiles(g)) || (pinned > 256 && !takes_oblong_tiles(g)) || (f32 && pinned == 256) ? 0 : pinned;
     const double slice_bytes = static_cast<double>(g.m) * static_cast<double>(round_up(g.n, 8)) * sizeof(float);
     // Calls that 256 x 256 tiles spread over three quarters of the chip keep the order of additions of the kernels with a
     // SwiGLU epilogue, which take such calls only (one sum over all of K): the fused and the separate operators give the same
@@ -363,10 +409,18 @@ Plan make_plan(const GemmArgs& g) {
         }
     }
     // 256 x 192 tiles where one sum over K on a large tile is best anyway: they add in the same order.
-    if (takes_narrow_tiles(g) && (forced == 192 || (forced == 0 && plan.tile >= 128 && best_slices == 1)) &&
-        (forced == 192 || predicted_us(192, tiles_of(192), 1, k_tiles, 0.0, f32, g.a_k_contiguous, g.b_k_contiguous, units) < best)) {
-        plan.tile = 192;
-        best_slices = 1;
+    const bool large = plan.tile >= 128 && best_slices == 1;
+    if (takes_narrow_tiles(g) && (forced == 192 || (forced == 0 && large))) {
+        const double time = predicted_us(192, tiles_of(192), 1, k_tiles, 0.0, f32, g.a_k_contiguous, g.b_k_contiguous, units);
+        if (forced == 192 || time < best) {
+            best = time;
+            plan.tile = 192;
+            best_slices = 1;
+        }
+    }
+    if (takes_oblong_tiles(g) && (forced > 256 || (forced == 0 && large))) {
+        try_oblong(best);
+        best_slices = plan.tile > 256 ? 1 : best_slices;
     }
     set_slices(best_slices);
     plan.deep = tiles_of(plan.tile) * plan.slices <= units;
@@ -430,15 +484,15 @@ int launch_small_call(const GemmArgs& g, const KernelArgs& p, const Plan& plan, 
 
 template <typename T>
 int run_plan(const GemmArgs& g, const Plan& plan, KernelArgs p, hipStream_t stream) {
-    const int tile_rows = plan.tile == 192 ? 256 : plan.tile;
-    p.tiles_m = (p.m + tile_rows - 1) / tile_rows;
-    p.tiles_n = (p.n + plan.tile - 1) / plan.tile;
+    const int rows = tile_rows(plan.tile), columns = tile_columns(plan.tile);
+    p.tiles_m = (p.m + rows - 1) / rows;
+    p.tiles_n = (p.n + columns - 1) / columns;
     p.k_tiles_per_slice = plan.k_tiles_per_slice;
     auto launch = [&](const KernelArgs& args, bool split) -> int {
         if (plan.tile <= 64) return launch_small_call<T>(g, args, plan, split, stream);
         const LargeCall call{args, g.a_k_contiguous, g.b_k_contiguous, plan.tile, split, plan.slices};
-        if constexpr (std::is_same_v<T, bf16_t>) return gemm_large_bf16(call, stream);
-        else if constexpr (std::is_same_v<T, f16_t>) return gemm_large_f16(call, stream);
+        if constexpr (std::is_same_v<T, bf16_t>) return plan.tile > 256 ? gemm_oblong_bf16(call, stream) : gemm_large_bf16(call, stream);
+        else if constexpr (std::is_same_v<T, f16_t>) return plan.tile > 256 ? gemm_oblong_f16(call, stream) : gemm_large_f16(call, stream);
         else return gemm_large_f32(call, stream);
     };
     if (plan.slices == 1) return launch(p, false);

@@ -5,6 +5,8 @@
 
 namespace cgptx {
 
+constexpr int kLdsBytes = 160 * 1024;  // of a CU
+
 struct KernelSegments {
     const void* ptr[3];
     long ld[3];
@@ -70,10 +72,15 @@ struct PairArgs {
     int first_blocks, weight_first;  // set by the launch: the workgroups of the call that starts first
 };
 
+// Tiles by a number: the edge of a square one, 192 for 256 rows of 192 columns, and these for oblong ones (16-bit storage).
+constexpr int oblong_tile(int rows, int columns) { return rows * 1000 + columns; }
+constexpr int tile_rows(int tile) { return tile > 256 ? tile / 1000 : tile == 192 ? 256 : tile; }
+constexpr int tile_columns(int tile) { return tile > 256 ? tile % 1000 : tile; }
+
 struct LargeCall {
     KernelArgs args;
     bool a_k_contiguous, b_k_contiguous;
-    int tile;    // 256 (16-bit storage) or 128
+    int tile;    // 128 or, in 16-bit storage, 256, 192 or an oblong one
     bool split;  // fp32 partial tiles of K slices
     int slices;
 };
@@ -81,6 +88,8 @@ struct LargeCall {
 int gemm_large_bf16(const LargeCall& call, hipStream_t stream);
 int gemm_large_f16(const LargeCall& call, hipStream_t stream);
 int gemm_large_f32(const LargeCall& call, hipStream_t stream);
+int gemm_oblong_bf16(const LargeCall& call, hipStream_t stream);
+int gemm_oblong_f16(const LargeCall& call, hipStream_t stream);
 int gemm_pair_bf16(const PairArgs& pair, hipStream_t stream);
 int gemm_pair_f16(const PairArgs& pair, hipStream_t stream);
 

@@ -53,6 +53,30 @@ struct ColumnTile<T, 192> {
     using type = NTile192<T>;
 };
 
+// Tiles that are not square, but 256 x 192 ones: more heights between 128 and 256 rows, for calls whose square tiles would leave CUs
+// idle (oblong_tiles).
+template <int BM, int BN>
+constexpr bool is_oblong = BM != BN && BN != 192;
+
+// The rings' slots of a tile that has a CU to itself: whatever lets the operand that is requested last be requested earliest (A's K
+// tile 2 kASlots - 3 steps before it is read, B's 2 kBSlots - 2), in as little of the LDS as that takes.
+struct RingSlots {
+    int a, b;
+};
+constexpr RingSlots ring_slots(int a_bytes, int b_bytes) {
+    RingSlots best{0, 0};
+    int best_lead = 0, best_bytes = 0;
+    for (int a = 3; a <= 8; ++a)
+        for (int b = 2; b <= 8; ++b) {
+            const int bytes = a * a_bytes + b * b_bytes, lead = 2 * a - 3 < 2 * b - 2 ? 2 * a - 3 : 2 * b - 2;
+            if (bytes > kLdsBytes || lead < best_lead || (lead == best_lead && bytes >= best_bytes)) continue;
+            best = {a, b};
+            best_lead = lead;
+            best_bytes = bytes;
+        }
+    return best;
+}
+
 // LDS holds a ring of K tiles of A and one of B (a K tile: two K steps, 128 bytes along K per row or column). Two slots of
 // each hold the K tile being multiplied and the next one, the rest what is in flight beyond them. 256 x 256 blocks own a CU
 // (3 x 32 + 2 x 32 KiB; 256 x 192: 3 x 32 + 2 x 24), 128 x 128 blocks run two per CU (3 x 16 + 2 x 16 KiB each) or, where there is no second one for a
@@ -61,7 +85,8 @@ template <typename T, int BM, int BN, bool A_K, bool B_K, bool DEEP>
 struct TileLayout {
     using ATile = std::conditional_t<A_K, KTile<T, BM>, NTile<T, BM>>;
     using BTile = std::conditional_t<B_K, KTile<T, BN>, typename ColumnTile<T, BN>::type>;
-    static constexpr int kASlots = DEEP ? 5 : 3, kBSlots = DEEP ? 4 : 2;
+    static constexpr RingSlots kOblong = ring_slots(ATile::kElems * static_cast<int>(sizeof(T)), BTile::kElems * static_cast<int>(sizeof(T)));
+    static constexpr int kASlots = is_oblong<BM, BN> ? kOblong.a : DEEP ? 5 : 3, kBSlots = is_oblong<BM, BN> ? kOblong.b : DEEP ? 4 : 2;
     static constexpr int kSmemBytes = (kASlots * ATile::kElems + kBSlots * BTile::kElems) * static_cast<int>(sizeof(T));
     // The order of an item's requests: A's K tile x is requested in the first step of K tile x + 1 - kASlots, B's in the
     // second step of x - kBSlots. Steps are numbered 2 t (first) and 2 t + 1 (second); what is due before step 0 is
@@ -219,6 +244,8 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     // 256 x 192 tiles: a wavefront has half of the tile's first 128 columns and half of its last 64, so that each of its blocks
     // of 16 columns lies in one part of the operand's tile and C is stored in half lines at least.
     constexpr bool kNarrow = BN == 192;
+    constexpr bool kOblong = is_oblong<BM, BN>;
+    static_assert(!kOblong || (A_K && !SPLIT && !RESIDUAL && !SWIGLU && !GRAD && !FOLD && PLAIN), "oblong tiles take unsplit calls of k-contiguous A that are stored as they are or with a residual");
     static_assert(!kNarrow || (BM == 256 && !SPLIT && !RESIDUAL && !SWIGLU && !GRAD && !FOLD), "256 x 192 tiles have an epilogue of their own");
     auto column_of = [&](int j) { return !kNarrow ? wn * WN + j * 16 : j < 4 ? wn * 64 + j * 16 : 128 + wn * 32 + (j - 4) * 16; };
 
@@ -462,16 +489,17 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     constexpr int kStaged = kNarrow ? 4 : TN;  // 16-bit blocks of a staged row
     constexpr int kRowBytes = kStaged * 32;    // fp32 values always pass in two halves
     constexpr int kRowChunks = kRowBytes / 16;
-    static_assert(32 * kRowBytes * kWaves <= static_cast<int>(kASlotBytes), "staging fits a slot of A");
-    unsigned char* region = smem_raw + (kASlots - 1) * kASlotBytes + wave * (32 * kRowBytes);
+    constexpr int kPassRows = kOblong ? 16 : 32;  // 80 and 112 rows of a wavefront are no multiple of 32, and the slot may be smaller
+    static_assert(kPassRows * kRowBytes * kWaves <= static_cast<int>(kASlotBytes), "staging fits a slot of A");
+    unsigned char* region = smem_raw + (kASlots - 1) * kASlotBytes + wave * (kPassRows * kRowBytes);
     auto sw = [](int row) { return (row / (256 / kRowBytes)) % kRowChunks; };
     const int m_lane = lane & 15, q_lane = lane >> 4;
-    // Writes blocks (2r, j0 .. j0+JP-1) and (2r+1, ...) into the wavefront's staging region as element type S.
+    // Writes blocks (r, j0 .. j0+JP-1) of kPassRows rows into the wavefront's staging region as element type S.
     auto stage = [&]<typename S, int JP>(int r, int j0) __attribute__((always_inline)) {
         static_assert(JP * 16 * sizeof(S) == kRowBytes, "a pass fills whole staged rows");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int ii = 0; ii < 2; ++ii) {
+        for (int ii = 0; ii < kPassRows / 16; ++ii) {
             const int row = ii * 16 + m_lane;
             unsigned char* write_row = region + row * kRowBytes;
 #pragma unroll
@@ -482,7 +510,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                 acc_t v;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    float x = acc[2 * r + ii][j0 + jj][e];
+                    float x = acc[r * (kPassRows / 16) + ii][j0 + jj][e];
                     if constexpr (!kIsF32) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(x));
                     v[e] = x;
                 }
@@ -494,26 +522,26 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
         }
         __builtin_amdgcn_wave_barrier();
     };
-    // Stages those blocks, 32 rows, and hands each lane 8 consecutive staged elements at a time:
+    // Stages those blocks and hands each lane 8 consecutive staged elements at a time:
     // consume(round, row, col, pointer to the 8 elements' first chunk, to the second chunk when S is
     // float), row/col relative to the wavefront's part; in round u the lane gets element
-    // q = 64 u + lane of the 32 x (8-element groups per row) grid, row-major.
+    // q = 64 u + lane of the kPassRows x (8-element groups per row) grid, row-major.
     auto pass = [&]<typename S, int JP>(int r, int j0, auto&& consume) __attribute__((always_inline)) {
         stage.template operator()<S, JP>(r, j0);
         constexpr int kLanesPerRow = kRowBytes / (8 * static_cast<int>(sizeof(S)));
         constexpr int kChunksPerLane = 8 * static_cast<int>(sizeof(S)) / 16;
-        constexpr int kRounds = 32 * kLanesPerRow / kWave;
+        constexpr int kRounds = kPassRows * kLanesPerRow / kWave;
 #pragma unroll
         for (int u = 0; u < kRounds; ++u) {
             const int q = u * kWave + lane;
             const int row = q / kLanesPerRow, part = q % kLanesPerRow;
             const unsigned char* base = region + row * kRowBytes;
             const int first = part * kChunksPerLane;
-            consume(u, r * 32 + row, j0 * 16 + part * 8, base + ((first ^ sw(row)) * 16),
+            consume(u, r * kPassRows + row, j0 * 16 + part * 8, base + ((first ^ sw(row)) * 16),
                     base + (((first + kChunksPerLane - 1) ^ sw(row)) * 16));
         }
     };
-    constexpr int kRowBlocks = WM / 32;  // 32-row blocks of a wavefront's part
+    constexpr int kRowBlocks = WM / kPassRows;  // passes over a wavefront's rows
     auto request_share = [&](int r) __attribute__((always_inline)) {
         static_for<0, kRowBlocks>([&](auto index) {
             constexpr int block = decltype(index)::value;
@@ -522,7 +550,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                                                 Layout::kFirstDue - Layout::kFirstDue * (block + 1) / kRowBlocks>();
         });
     };
-    // Before 32-row block r of the tile is staged and stored, its share of the first K tiles of the next item
+    // Before block r of the tile's rows is staged and stored, its share of the first K tiles of the next item
     // are requested (if there is one): a burst of requests would hold the wavefront up for as long as
     // the memory system takes to accept them, between the stores it costs nothing.
     auto store_tile = [&](const Item& w, bool request) __attribute__((always_inline)) {
@@ -542,7 +570,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
         // partial tiles (nothing added, fp32 out) and a residual added to a 16-bit result. Half the
         // columns are staged per pass; lane l of round u holds 8 consecutive columns (group l%8) of
         // row 8u + l/8.
-        constexpr int kGroups = kStaged, kRowsF = kWave / kGroups, kRoundsF = 32 / kRowsF;
+        constexpr int kGroups = kStaged, kRowsF = kWave / kGroups, kRoundsF = kPassRows / kRowsF;
         const int f_row = lane / kGroups, f_col = (lane % kGroups) * 8;  // f_col within the staged half
         auto read_staged = [&](int u, vec_t<float, 4>& v0, vec_t<float, 4>& v1) __attribute__((always_inline)) {
             const int row = u * kRowsF + f_row;
@@ -748,8 +776,8 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
             }
             return;
         }
-        // Of a pair's calls either the result is stored as it is or C is its own residual.
-        if constexpr (RESIDUAL || (FOLD && PLAIN)) if (RESIDUAL || p.residual != nullptr) {
+        // Of a pair's calls, and on oblong tiles, either the result is stored as it is or a residual is all that is added (C its own).
+        if constexpr (RESIDUAL || (FOLD && PLAIN) || kOblong) if (RESIDUAL || p.residual != nullptr) {
             const int cols_left = min(WN, c_cols - (c_col0 + col0));
             const T* out_origin = static_cast<const T*>(c_base) + static_cast<long>(row0) * c_ld + (c_col0 + col0);
             const T* res_origin = static_cast<const T*>(p.residual) + static_cast<long>(row0) * p.ldr + (w.n0 + col0);
@@ -768,7 +796,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                                                         : std::numeric_limits<int>::min();
 #pragma unroll
                     for (int u = 0; u < kRoundsF; ++u)
-                        into[half][u] = __builtin_amdgcn_raw_buffer_load_b128(res_rsrc, voffset, (r * 32 + u * kRowsF) * res_row_bytes, 0);
+                        into[half][u] = __builtin_amdgcn_raw_buffer_load_b128(res_rsrc, voffset, (r * kPassRows + u * kRowsF) * res_row_bytes, 0);
                 }
             };
             request_residual(0, ahead[0]);
@@ -796,7 +824,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                             sum[4 + e] = v1[u][e] + add[4 + e];
                         }
                         store_chunk(__builtin_bit_cast(u32x4, vec_from_f32<T, 8>(sum)), out_rsrc, voffset,
-                                                               (r * 32 + u * kRowsF) * out_row_bytes);
+                                                               (r * kPassRows + u * kRowsF) * out_row_bytes);
                     }
                 }
             }
@@ -817,7 +845,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                                     ? (static_cast<long>(rows_left - 1) * c_ld + cols_left) * static_cast<long>(sizeof(T))
                                     : 0;
             const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(part, 0, static_cast<int>(extent), 0x00020000);
-            constexpr int kLanesPerRow = kRowBytes / 16, kRowsPerRound = kWave / kLanesPerRow, kRounds = 32 / kRowsPerRound;
+            constexpr int kLanesPerRow = kRowBytes / 16, kRowsPerRound = kWave / kLanesPerRow, kRounds = kPassRows / kRowsPerRound;
             const int lane_row = lane / kLanesPerRow, lane_chunk = lane % kLanesPerRow;
             const int row_bytes = static_cast<int>(c_ld * static_cast<long>(sizeof(T)));
             const int voffset = lane_chunk * 8 < cols_left ? lane_row * row_bytes + lane_chunk * 16 : std::numeric_limits<int>::min();
@@ -836,7 +864,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                 }
 #pragma unroll
                 for (int u = 0; u < kRounds; ++u)
-                    store_chunk(data[u], rsrc, voffset, (r * 32 + u * kRowsPerRound) * row_bytes);
+                    store_chunk(data[u], rsrc, voffset, (r * kPassRows + u * kRowsPerRound) * row_bytes);
             }
             return;
         }
@@ -1146,7 +1174,7 @@ __global__ __launch_bounds__(kThreads, DEEP ? 1 : 2) void gemm_pair_kernel(PairA
 }
 
 // ------------------------------------------------------------------- host side
-constexpr int blocks_per_unit(int tile) { return tile == 256 ? 1 : 2; }  // resident blocks per CU: what the LDS slots allow
+constexpr int blocks_per_unit(std::size_t smem) { return smem * 2 <= kLdsBytes ? 2 : 1; }  // resident blocks per CU: what the LDS slots allow
 
 // Groups of 1 << rows_log2 tile-rows, and what divides by their size.
 inline void set_groups(KernelArgs& p, int rows_log2) {
@@ -1180,7 +1208,7 @@ int launch_kernel(const KernelArgs& p, int slices, hipStream_t stream) {
     // (2 tile-rows x all 8 tile-columns of the training shape: 250 -> 212 us per launch; 1, 2 and 4 tile-rows
     // measure the same, every other kernel is at its best with 8).
     set_groups(args, GRAD ? 1 : 3);
-    const long slots = static_cast<long>(compute_units()) * blocks_per_unit(BM) / kXcds * kXcds;
+    const long slots = static_cast<long>(compute_units()) * blocks_per_unit(smem) / kXcds * kXcds;
     const long blocks = std::min<long>((items + kXcds - 1) / kXcds * kXcds, std::max<long>(slots, kXcds));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(blocks)), dim3(kThreads), smem, stream, args);
     CGPTX_LAUNCH_CHECK();
@@ -1264,6 +1292,28 @@ int launch_narrow(const LargeCall& call, hipStream_t stream) {
     return fail(CGPTX_RUNTIME, "gemm: unsupported operand layout");
 }
 
+// Oblong tiles, one block per CU: 160, 192 or 256 rows of 128 columns, 160, 192 or 224 of 256. A few thousand rows are 1.2 or 2.3
+// rounds of square tiles: 5005 x 1024 is 320 tiles of 128 x 128, of which 64 CUs get two, or 80 of 256 x 256. A tile of 160 x 128 is
+// one round. A call of one round costs 6 to 9 us that are no K loop (launch, first loads, store) and then what the L2s deliver
+// (128 columns: 0.25 us a K step, 1.34 PFLOP/s over a full chip) or the matrix cores at the power limit (160 x 256: 0.44 us, 1.5 PFLOP/s). Same
+// sums in the same order as square tiles. Block of 5 x 1001 tokens, 1024 wide, forward and backward 695 -> 671 us.
+template <typename T, int BM, int BN>
+int launch_oblong_tile(const LargeCall& call, hipStream_t stream) {
+    KernelArgs p = call.args;
+    const bool a_k = call.a_k_contiguous, b_k = call.b_k_contiguous;
+    if (p.accumulate && p.residual == nullptr) {  // C as its own residual, see launch_layout
+        p.residual = p.c;
+        p.ldr = p.ldc;
+        p.accumulate = 0;
+    }
+    if (call.split || !a_k || p.bias != nullptr || p.addend != nullptr || p.accumulate || p.c_f32 || p.ragged || p.act != nullptr ||
+        p.saved != nullptr || p.batch_rows > 0 || (p.residual != nullptr && p.c_seg.count > 0) || (p.a_seg.count > 0 && b_k))
+        return fail(CGPTX_RUNTIME, "gemm: oblong tiles take products that are stored as they are or with a residual");
+    if (p.a_seg.count > 0) return launch_kernel<T, BM, BN, true, false, false, true, false, false, false, false, true>(p, 1, stream);
+    if (b_k) return launch_kernel<T, BM, BN, true, true, false, false, false, false, false, false, true>(p, 1, stream);
+    return launch_kernel<T, BM, BN, true, false, false, false, false, false, false, false, true>(p, 1, stream);
+}
+
 template <typename T, bool DEEP, bool PLAIN>
 int launch_pair_kernel(const PairArgs& pair, int blocks, hipStream_t stream) {
     constexpr int smem = std::max(TileLayout<T, 128, 128, true, false, DEEP>::kSmemBytes, TileLayout<T, 128, 128, false, false, DEEP>::kSmemBytes);
@@ -1318,6 +1368,17 @@ int launch_large(const LargeCall& call, hipStream_t stream) {
     }
     if (call.tile != 128) return fail(CGPTX_RUNTIME, "gemm: no large tiles of this size for the storage type");
     return with_tile.template operator()<128>();
+}
+
+template <typename T>
+int launch_oblong(const LargeCall& call, hipStream_t stream) {
+    if (call.tile == oblong_tile(160, 128)) return launch_oblong_tile<T, 160, 128>(call, stream);
+    if (call.tile == oblong_tile(192, 128)) return launch_oblong_tile<T, 192, 128>(call, stream);
+    if (call.tile == oblong_tile(256, 128)) return launch_oblong_tile<T, 256, 128>(call, stream);
+    if (call.tile == oblong_tile(160, 256)) return launch_oblong_tile<T, 160, 256>(call, stream);
+    if (call.tile == oblong_tile(192, 256)) return launch_oblong_tile<T, 192, 256>(call, stream);
+    if (call.tile == oblong_tile(224, 256)) return launch_oblong_tile<T, 224, 256>(call, stream);
+    return fail(CGPTX_RUNTIME, "gemm: no oblong tiles of this size");
 }
 
 }  // namespace

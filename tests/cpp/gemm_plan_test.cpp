@@ -102,6 +102,42 @@ void check_narrow() {
         }
 }
 
+// Oblong tiles take the place of large square ones only, where the call is one sum over K and has nothing but a residual or its own C
+// added: results keep their bits, and every such plan has a kernel.
+void check_oblong() {
+    int taken = 0;
+    for (const int dtype : {CGPTX_BF16, CGPTX_F16, CGPTX_F32})
+        for (const Kind kind : {Kind::forward, Kind::input_gradient, Kind::weight_gradient})
+            for (std::size_t m = 100; m <= 40000; m += m / 7)
+                for (const std::size_t n : {640, 768, 1000, 1024, 1536, 2048, 4096})
+                    for (const std::size_t k : {64, 768, 1024, 4096})
+                        for (const int extra : {0, 1, 2, 3, 4, 5}) {
+                            GemmArgs g = contraction(kind, m, n, k, dtype);
+                            if (extra == 1) g.residual = address(), g.ldr = n;
+                            if (extra == 2) g.accumulate = true;
+                            if (extra == 3) g.bias = address();
+                            if (extra == 4) g.c = address(8);
+                            if (extra == 5) g.c_is_f32 = true;
+                            const Plan plan = make_plan(g);
+                            if (plan.tile <= 256) continue;
+                            ++taken;
+                            const std::string name = name_of(g) + ": tiles of " + std::to_string(plan.tile);
+                            expect(extra < 3 && dtype != CGPTX_F32 && kind != Kind::weight_gradient && plan.slices == 1, name);
+                            expect(tile_rows(plan.tile) % 32 == 0 && tile_columns(plan.tile) % 128 == 0, name);
+                            GemmArgs square = g;  // as it was planned without them
+                            square.bias = address();
+                            const Plan other = make_plan(square);
+                            expect(other.slices == 1 && other.tile >= 128, name + " for " + std::to_string(other.tile) + " in " + std::to_string(other.slices));
+                        }
+    expect(taken > 500, std::to_string(taken) + " calls on oblong tiles");
+    // Columns in segments are whole tiles of 256; an input gradient's segments along K take nothing added.
+    GemmArgs g = contraction(Kind::input_gradient, 5005, 1024, 1536, CGPTX_BF16);
+    g.a_segments.count = 3;
+    expect(make_plan(g).tile > 256, "segments along K");
+    g.accumulate = true;
+    expect(make_plan(g).tile <= 256, "segments along K, added to C");
+}
+
 // q's, k's and v's gradients over `rows` tokens as one group: their input gradients as one call in segments, then the weight gradients.
 struct Gradients {
     GemmArgs calls[4], input[3];
@@ -202,6 +238,7 @@ int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "pinned") == 0) check_pinned();
     if (argc > 1 && std::strcmp(argv[1], "chains") == 0) check_chains();
     if (argc > 1 && std::strcmp(argv[1], "narrow") == 0) check_narrow();
+    if (argc > 1 && std::strcmp(argv[1], "oblong") == 0) check_oblong();
     if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
     if (argc > 1 && std::strcmp(argv[1], "predictions") == 0) check_predictions();
     std::printf("%d failure(s)\n", failures);

@@ -137,6 +137,11 @@ def test_tiles_of_192_columns_take_what_their_epilogue_serves():
     run_plan_test("narrow")
 
 
+def test_calls_on_oblong_tiles_keep_their_bits_and_have_a_kernel():
+    """Oblong tiles replace large square ones of calls that are one sum over K, stored as it is or with a residual."""
+    run_plan_test("oblong")
+
+
 def test_predictions_that_stop_short_decide_as_whole_ones():
     """tests/cpp/gemm_plan_test.cpp: what both gradients of a projection take in one launch, predicted only as far as the answer
     can matter."""

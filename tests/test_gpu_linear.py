@@ -508,3 +508,36 @@ def test_gradients_in_k_slices_replay_from_a_graph(device, dtype):
         for _ in range(2):
             check(1, lambda: run(1))
             check(0, graph.replay)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("rows,k,n", [  # what the plan takes on 256 compute units
+    (5005, 1024, 1024), (4833, 992, 1000),     # 160 x 128
+    (7000, 2048, 768), (8999, 1728, 640),      # 192 x 128
+    (8161, 4096, 1024),                        # 256 x 128 where nothing else fits better
+    (5005, 1024, 2048), (10000, 1024, 1016),   # 160 x 256
+    (11900, 1024, 1024), (11871, 352, 1024),   # 192 x 256
+    (12500, 1024, 1024), (13001, 1024, 4096),  # 224 x 256, one round and four
+])
+def test_oblong_tiles_give_the_bits_of_square_ones(device, rows, k, n, dtype):
+    """Forward products with a bias of zeros run on square tiles of the general epilogue; without one, and as an input gradient,
+    on whatever the plan takes: one sum over K each, in the same order. Integers small enough that all sums are exact check both."""
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randint(-2, 3, (rows, k), generator=g).to(dtype).to(device)
+    w = torch.randint(-1, 2, (n, k), generator=g).to(dtype).to(device)
+    for scale in (1.0, 0.37):
+        a, b = (x * scale).to(dtype), (w * 0.11 if scale != 1.0 else w).to(dtype)
+        plain, square, dx = (torch.full((rows, n), float("nan"), dtype=dtype, device=device) for _ in range(3))
+        ops.linear_forward(plain, a, b)
+        ops.linear_forward(square, a, b, bias=torch.zeros(n, dtype=dtype, device=device))
+        assert torch.equal(plain, square)
+        ops.linear_backward(dx, None, None, a, torch.empty_like(dx), b.t().contiguous())
+        assert torch.equal(dx, square)
+        if scale == 1.0:
+            exact = a.float() @ b.float().t()
+            assert torch.equal(plain, exact.to(dtype))
+            old = torch.randint(-8, 9, (rows, n), generator=g).to(dtype).to(device)
+            added = old.clone()
+            ops.linear_backward(added, None, None, a, torch.empty_like(dx), b.t().contiguous(),
+                                options=ops.LinearBackwardOptions(accumulate_input=True))
+            assert torch.equal(added, (exact + old.float()).to(dtype))
