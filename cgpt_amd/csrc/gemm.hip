@@ -755,7 +755,12 @@ bool pairs(const GemmArgs* calls, int count) {
     return count == 2 && calls[0].dtype != CGPTX_F32 && calls[0].a_k_contiguous && !calls[0].b_k_contiguous && calls[0].a_segments.count == 0 &&
            !calls[1].a_k_contiguous && !calls[1].b_k_contiguous && calls[1].a_segments.count == 0;
 }
-long tiles_128(const GemmArgs& g) { return static_cast<long>((g.m + 127) / 128) * static_cast<long>((g.n + 127) / 128); }
+long tiles_of_size(const GemmArgs& g, std::size_t rows, std::size_t columns) {
+    return static_cast<long>((g.m + rows - 1) / rows) * static_cast<long>((g.n + columns - 1) / columns);
+}
+// The weight gradient's tile of a pair, by the input gradient's.
+int pair_weight_rows(const GemmGroup& plan) { return plan.tile[0] > 256 ? kPairWeightRows : 128; }
+int pair_weight_columns(const GemmGroup& plan) { return plan.tile[0] > 256 ? kPairWeightColumns : 128; }
 long k_steps_16bit(const GemmArgs& g) { return static_cast<long>((g.k + kBK<bf16_t> - 1) / kBK<bf16_t>); }
 // K steps of a slice: whole K tiles, as the kernels read them.
 long slice_steps(long steps, long slices) { return ((steps + slices - 1) / slices + kSteps - 1) / kSteps * kSteps; }
@@ -813,6 +818,23 @@ double predicted_pair_us(long tiles_x, long steps_x, long tiles_w, long steps_w,
     return time();
 }
 
+// The same with an oblong tile for the input gradient and 256 x 128 for the weight gradient, where every workgroup has a CU to itself:
+// the longer of the two. Both operands of the weight gradient are read transposed from LDS, 0.30 - 0.39 us a K step. Fitted to 16 shapes from
+// 3000 x 1024 x 4096 to 12000 x 768 x 768, six tiles and one to four slices each: within 5 per cent where one round is enough; what several
+// rounds take varies by a third with the order in which workgroups end, so those keep to 128 x 128 tiles, and so do short sums, whose
+// slices cost more to add up than the tiles save. us, 128 x 128 and chosen: 5005 x 1024 x 2048 53.4 -> 45.7, 6000 x 1024 x 2048 59.1 -> 52.0,
+// 7000 x 768 x 2048 52.0 -> 47.4, 3000 x 1024 x 4096 52.7 -> 47.8; 5005 x 1024 x 1024 30.8 and 33.6, 4096 x 768 x 2048 33.6 and 34.8.
+double predicted_oblong_pair_us(const OblongCost& c, long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units) {
+    const long items = tiles_x + tiles_w * slices;
+    if (items > units) return std::numeric_limits<double>::infinity();
+    const long kt = slices > 1 ? slice_steps(steps_w, slices) : steps_w;
+    const double filled = static_cast<double>(items) / static_cast<double>(units);
+    const double fold = slices > 1 ? 3.6 * static_cast<double>(slices * tiles_w * slices) / static_cast<double>(units) : 0.0;
+    const double input = 4.2 + static_cast<double>(steps_x) * (1.09 * c.step + 0.565 * c.step_full * filled);
+    const double weight = 6.5 + static_cast<double>(kt) * (0.30 + 0.087 * filled) + fold;
+    return 4.5 + std::max(input, weight);
+}
+
 // A group's tiles: those whose predicted time in one launch is least. The launch takes as long as its longest workgroup or
 // as the busiest CU's share of the work, whatever is more (us per K tile and workgroup as in predicted_us; 3.5 us before and
 // after the K loops). Two workgroups share a CU and its LDS, or, deep, each has one to itself: then the longest is not held
@@ -846,15 +868,29 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
     }
     double best = separate;
     if (pair) {
-        const long tiles_x = tiles_128(calls[0]), tiles_w = tiles_128(calls[1]), steps_x = k_steps_16bit(calls[0]), steps_w = k_steps_16bit(calls[1]);
+        const long tiles_x = tiles_of_size(calls[0], 128, 128), tiles_w = tiles_of_size(calls[1], 128, 128), steps_x = k_steps_16bit(calls[0]), steps_w = k_steps_16bit(calls[1]);
         for (long s = 1; s <= 16 && tiles_w <= kTickets && (s == 1 || steps_w / s >= 8); ++s) {
             if (slice_steps(steps_w, s) * (s - 1) >= steps_w) continue;
             const double time = predicted_pair_us(tiles_x, steps_x, tiles_w, steps_w, s, compute_units(), best);
             if (time < best) {
                 best = time;
                 best_plan.joined = best_plan.pair = true;
+                best_plan.tile[0] = 128;
                 best_plan.slices = static_cast<int>(s);
             }
+        }
+        if (takes_oblong_tiles(calls[0]) && calls[0].a_segments.count == 0 && c_streams(calls[1], 2)) {
+            const long tiles = tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns);
+            for (const OblongCost& c : kOblongCosts)
+                for (long s = 1; s <= 3; ++s) {
+                    if (s > 1 && slice_steps(steps_w, s) * (s - 1) >= steps_w) continue;
+                    const double time = 1.06 * predicted_oblong_pair_us(c, Plan::tiles_of(calls[0], c.tile), steps_x, tiles, steps_w, s, compute_units());
+                    if (time >= best) continue;
+                    best = time;
+                    best_plan.joined = best_plan.pair = true;
+                    best_plan.tile[0] = c.tile;
+                    best_plan.slices = static_cast<int>(s);
+                }
         }
     }
     if (fewest > kGroupBlocksPerUnit * units) return best_plan;
@@ -935,8 +971,9 @@ struct FoldRoom {
     unsigned int* counters = nullptr;
     bool enough = false;
 };
-int fold_room(const GemmArgs& g, int slices, hipStream_t stream, FoldRoom* room) {
-    const std::size_t wanted = static_cast<std::size_t>(tiles_128(g)) * static_cast<std::size_t>(slices) * kFoldTileBytes;
+int fold_room(const GemmArgs& g, const GemmGroup& plan, hipStream_t stream, FoldRoom* room) {
+    const int rows = pair_weight_rows(plan), columns = pair_weight_columns(plan);
+    const std::size_t wanted = static_cast<std::size_t>(tiles_of_size(g, rows, columns)) * static_cast<std::size_t>(plan.slices) * fold_tile_bytes(rows, columns);
     room->partial = g.split_workspace;
     std::size_t held = g.split_workspace_bytes;
     if (!g.no_split)
@@ -955,8 +992,9 @@ int run_pair(const GemmArgs* calls, const GemmGroup& plan, hipStream_t stream) {
         for (int i = 0; i < 2; ++i) {
             KernelArgs& p = i == 0 ? pair.input : pair.weight;
             if (!joinable<T>(calls[i], p)) return fail(CGPTX_RUNTIME, "gemm: this call cannot be part of a group");
-            p.tiles_m = (p.m + 127) / 128;
-            p.tiles_n = (p.n + 127) / 128;
+            const int rows = i == 0 ? tile_rows(plan.tile[0]) : pair_weight_rows(plan), columns = i == 0 ? tile_columns(plan.tile[0]) : pair_weight_columns(plan);
+            p.tiles_m = (p.m + rows - 1) / rows;
+            p.tiles_n = (p.n + columns - 1) / columns;
             p.slices = 1;
             p.k_tiles_per_slice = p.k_tiles;
         }
@@ -966,15 +1004,17 @@ int run_pair(const GemmArgs* calls, const GemmGroup& plan, hipStream_t stream) {
         w.a_sums_accumulate = g.a_sums_accumulate ? 1 : 0;
         if (plan.slices > 1) {
             FoldRoom room;
-            if (int s = fold_room(g, plan.slices, stream, &room)) return s;
+            if (int s = fold_room(g, plan, stream, &room)) return s;
             if (!room.enough) return fail(CGPTX_RUNTIME, "gemm: no room for the partial tiles of a pair");
             w.fold_partial = static_cast<unsigned char*>(room.partial);
             w.fold_tickets = room.counters;
             w.k_tiles_per_slice = static_cast<int>(slice_steps(w.k_tiles, plan.slices));
             w.slices = (w.k_tiles + w.k_tiles_per_slice - 1) / w.k_tiles_per_slice;
         }
-        if constexpr (std::is_same_v<T, bf16_t>) return gemm_pair_bf16(pair, stream);
-        else return gemm_pair_f16(pair, stream);
+        pair.input_tile = plan.tile[0];
+        const bool oblong = plan.tile[0] > 256;
+        if constexpr (std::is_same_v<T, bf16_t>) return oblong ? gemm_oblong_pair_bf16(pair, stream) : gemm_pair_bf16(pair, stream);
+        else return oblong ? gemm_oblong_pair_f16(pair, stream) : gemm_pair_f16(pair, stream);
     }
 }
 
@@ -1029,7 +1069,7 @@ GemmGroup gemm_joins(const GemmArgs* calls, int count, hipStream_t stream, bool 
     GemmGroup group = plan_group(calls, count, pair);
     if (group.pair && group.slices > 1) {
         FoldRoom room;
-        if (fold_room(calls[1], group.slices, stream, &room) != CGPTX_OK || !room.enough) {
+        if (fold_room(calls[1], group, stream, &room) != CGPTX_OK || !room.enough) {
             clear_error();
             group = plan_group(calls, count, false);
         }

@@ -87,7 +87,7 @@ struct GemmGroup {
     int tile[kGroupCalls] = {};
     bool deep = false;  // one workgroup per CU
     bool few = false;   // launched by the kernel whose arguments hold kFewCalls calls
-    bool pair = false;  // an input and a weight gradient on 128 x 128 tiles, the weight gradient in `slices` along K
+    bool pair = false;  // an input and a weight gradient on large tiles (the input gradient's is tile[0]), the weight gradient in `slices` along K
     int slices = 1;
     bool joined = false;
 };

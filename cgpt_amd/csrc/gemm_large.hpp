@@ -57,9 +57,10 @@ struct KernelArgs {
     int a_sums_accumulate;
 };
 
-// The input and the weight gradient of a projection in one launch, on 128 x 128 tiles; each call's tiles_m, tiles_n, slices and
+// The input and the weight gradient of a projection in one launch; each call's tiles_m, tiles_n, slices and
 // k_tiles_per_slice are set.
-constexpr int kFoldTileBytes = 128 * 128 * 4 + 128 * 4;  // of a tile's slice: accumulators, and sums of A's columns
+constexpr int fold_tile_bytes(int rows, int columns) { return rows * columns * 4 + rows * 4; }  // of a tile's slice: accumulators, and sums of A's columns
+constexpr int kPairWeightRows = 256, kPairWeightColumns = 128;  // the weight gradient's tile beside an oblong one of the input gradient
 // What a K slice adds to the counter of its tile: shares that make 2^32 together, none of them zero. The workgroup that brings the
 // counter back to zero is the tile's last one, and a launch leaves the counter as it found it: also where two launches met on the same
 // counters (a graph replayed beside other work of the stream it was captured on), whatever slices each has, the next one counts from zero.
@@ -69,6 +70,7 @@ __host__ __device__ constexpr unsigned int fold_share(int slice, int slices) {
 }
 struct PairArgs {
     KernelArgs input, weight;
+    int input_tile;  // 128: both on 128 x 128 tiles
     int first_blocks, weight_first;  // set by the launch: the workgroups of the call that starts first
 };
 
@@ -92,5 +94,7 @@ int gemm_oblong_bf16(const LargeCall& call, hipStream_t stream);
 int gemm_oblong_f16(const LargeCall& call, hipStream_t stream);
 int gemm_pair_bf16(const PairArgs& pair, hipStream_t stream);
 int gemm_pair_f16(const PairArgs& pair, hipStream_t stream);
+int gemm_oblong_pair_bf16(const PairArgs& pair, hipStream_t stream);
+int gemm_oblong_pair_f16(const PairArgs& pair, hipStream_t stream);
 
 }  // namespace cgptx

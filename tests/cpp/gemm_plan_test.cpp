@@ -130,6 +130,24 @@ void check_oblong() {
                             expect(other.slices == 1 && other.tile >= 128, name + " for " + std::to_string(other.tile) + " in " + std::to_string(other.slices));
                         }
     expect(taken > 500, std::to_string(taken) + " calls on oblong tiles");
+    // Both gradients of a projection: one round of workgroups, C of either in whole aligned chunks.
+    int pairs_taken = 0;
+    for (std::size_t rows = 500; rows <= 20000; rows += rows / 9)
+        for (const std::size_t in : {640, 768, 1000, 1024, 2048})
+            for (const std::size_t out : {256, 1024, 2048, 4096})
+                for (const int extra : {0, 1, 2, 3, 4}) {
+                    GemmArgs calls[2] = {contraction(Kind::input_gradient, rows, in, out, CGPTX_BF16), contraction(Kind::weight_gradient, out, in, rows, CGPTX_BF16)};
+                    if (extra == 1) calls[0].accumulate = true;
+                    if (extra == 2) calls[1].accumulate = true, calls[1].a_sums = address();
+                    if (extra == 3) calls[0].c = address(8);
+                    if (extra == 4) calls[1].c = address(8);
+                    const GemmGroup plan = plan_group(calls, 2, true);
+                    if (!plan.pair || plan.tile[0] <= 256) continue;
+                    ++pairs_taken;
+                    const long items = Plan::tiles_of(calls[0], plan.tile[0]) + tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns) * plan.slices;
+                    expect(extra < 3 && items <= compute_units(), name_of(calls[0]) + ": " + std::to_string(items) + " workgroups for a pair");
+                }
+    expect(pairs_taken > 20, std::to_string(pairs_taken) + " pairs on oblong tiles");
     // Columns in segments are whole tiles of 256; an input gradient's segments along K take nothing added.
     GemmArgs g = contraction(Kind::input_gradient, 5005, 1024, 1536, CGPTX_BF16);
     g.a_segments.count = 3;

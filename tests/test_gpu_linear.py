@@ -541,3 +541,13 @@ def test_oblong_tiles_give_the_bits_of_square_ones(device, rows, k, n, dtype):
             ops.linear_backward(added, None, None, a, torch.empty_like(dx), b.t().contiguous(),
                                 options=ops.LinearBackwardOptions(accumulate_input=True))
             assert torch.equal(added, (exact + old.float()).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("rows,fin,fout", [
+    (5005, 1024, 2048), (6983, 760, 2048),   # dX on 224 x 256, dW in two and three slices; rows, columns and K end inside tiles
+    (3000, 1024, 4096), (2993, 1016, 4064),  # dX on 192 x 128, dW one sum over K
+])
+@pytest.mark.parametrize("accumulate", [False, True], ids=["overwrite", "accumulate"])
+def test_both_gradients_on_oblong_tiles_share_a_launch(device, rows, fin, fout, accumulate, dtype):
+    test_both_gradients_on_large_tiles_share_a_launch(device, rows, fin, fout, accumulate, dtype)
