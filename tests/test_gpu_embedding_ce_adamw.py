@@ -442,3 +442,30 @@ def test_embedding_backward_keeps_non_finite_rows_to_their_ids(device):
         ops.embedding_backward(got, dy.to(device), ids.to(torch.int32).to(device), 1000)
         want = _added_in_token_order(ids, dy, torch.zeros(3, hidden), False)
         assert torch.equal(got.cpu(), want) and torch.isfinite(got[1:]).all() and torch.isinf(got[0]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_adamw_of_more_state_than_the_memory_cache_gives_the_bits_of_less(device, dtype):
+    """22.4 million elements are 256 MiB of fp32 state: beyond them the update accesses it as what is used once. Without clipping
+    every element is updated by itself, so one call over all gives what calls over parts give."""
+    count = (256 << 20) // 12 + 4096 * 3 + 17
+    generator = torch.Generator(device=device).manual_seed(3)
+    start = torch.randn(count, device=device, generator=generator).to(dtype)
+    grads = [torch.randn(count, device=device, generator=generator).mul_(0.01).to(dtype) for _ in range(2)]
+    options = ops.AdamWOptions(learning_rate=3e-4, weight_decay=0.1, max_grad_norm=float("inf"))
+    results = []
+    for parts in (1, 3):
+        edges = [count * i // parts // 64 * 64 for i in range(parts)] + [count]
+        parameter, gradient, master = start.clone(), torch.empty_like(start), start.to(torch.float32, copy=True)
+        first, second = torch.zeros_like(master), torch.zeros_like(master)
+        calls = []
+        for a, b in zip(edges, edges[1:]):
+            state = ops.AdamWState(master[a:b], first[a:b], second[a:b])
+            calls.append(([ops.AdamWBatchEntry(parameter[a:b], gradient[a:b], state)], ops.AdamWWorkspace()))
+        for g in grads:
+            gradient.copy_(g)
+            for entries, workspace in calls:
+                ops.adamw_step_many_async(entries, options, workspace)
+        results.append((parameter, master, first, second))
+    for name, one, three in zip(("parameter", "master", "first", "second"), *results):
+        assert torch.equal(one, three), name
