@@ -469,3 +469,27 @@ def test_adamw_of_more_state_than_the_memory_cache_gives_the_bits_of_less(device
         results.append((parameter, master, first, second))
     for name, one, three in zip(("parameter", "master", "first", "second"), *results):
         assert torch.equal(one, three), name
+
+
+@pytest.mark.parametrize("dtype,rows,vocab", [(torch.bfloat16, 1511, 50257), (torch.float32, 2311, 16381), (torch.float16, 19, 8 * 1024 * 1024 // 64 - 3)],
+                         ids=["bf16", "f32", "f16"])
+def test_cross_entropy_of_more_logits_than_the_memory_cache_gives_the_rows_of_few(device, dtype, rows, vocab):
+    """Beyond 288 MiB logits and gradients are accessed as what is used once; a row's gradient is what a call over few rows gives for it
+    (the same scale / rows). The last shape is a small one of long rows at odd addresses."""
+    generator = torch.Generator(device=device).manual_seed(5)
+    logits = torch.randn(rows, vocab, device=device, generator=generator).to(dtype)
+    targets = torch.randint(0, vocab, (rows,), device=device, generator=generator, dtype=torch.int32)
+    loss, gradient = torch.empty(1, device=device), torch.empty_like(logits)
+    ops.cross_entropy_forward_backward(loss, gradient, logits, targets, rows, gradient_scale=float(rows))
+    total = 0.0
+    for first in range(0, rows, 300):
+        part = slice(first, min(first + 300, rows))
+        few = part.stop - part.start
+        part_loss, part_gradient = torch.empty(1, device=device), torch.empty_like(logits[part])
+        ops.cross_entropy_forward_backward(part_loss, part_gradient, logits[part], targets[part].contiguous(), few, gradient_scale=float(few))
+        assert torch.equal(gradient[part], part_gradient)
+        total += part_loss.item() * few
+    assert abs(loss.item() - total / rows) <= 1e-6 * abs(loss.item())
+    only = torch.empty(1, device=device)
+    ops.cross_entropy_forward(only, logits, targets, rows)
+    assert only.item() == loss.item()
