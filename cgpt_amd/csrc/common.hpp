@@ -274,6 +274,22 @@ int scratch_up_to(hipStream_t stream, std::size_t bytes, void** out, std::size_t
 // capture, no memory): the caller does without.
 constexpr int kTickets = 4096;
 unsigned int* tickets(hipStream_t stream);
+// What one of `slices` workgroups adds to their counter: shares that make 2^32 together, none of them zero. The workgroup that brings
+// the counter back to zero is the last one, and a launch leaves the counter as it found it: also where two launches met on the same
+// counters (a graph replayed beside other work of the stream it was captured on), whatever slices each has, the next one counts from zero.
+__host__ __device__ constexpr unsigned int fold_share(int slice, int slices) {
+    const unsigned int even = 0xFFFFFFFFu / static_cast<unsigned int>(slices);
+    return slice == 0 ? 0u - even * static_cast<unsigned int>(slices - 1) : even;
+}
+// A thread leaves a value that the last workgroup of the launch reads, behind the L2s (each XCD has its own), and counts its
+// workgroup: true for the last one. Every workgroup calls it once, with one thread.
+__device__ __forceinline__ bool leave_and_count(float* where, float value, unsigned int* counter, unsigned int share) {
+    __hip_atomic_store(where, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return __hip_atomic_fetch_add(counter, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + share == 0u;
+}
+// What leave_and_count left.
+__device__ __forceinline__ float read_left(const float* where) { return __hip_atomic_load(where, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // Identifies the block currently behind the (current device, stream) arena: it changes whenever that
 // arena is reallocated (a larger request) and reads 0 after cgptx_release_scratch. A captured graph

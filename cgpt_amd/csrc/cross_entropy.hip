@@ -48,6 +48,41 @@ __device__ __forceinline__ MaxSum block_combine(MaxSum v, MaxSum* stage) {
     return total;
 }
 
+// (Σ row_loss) / rows by a workgroup of THREADS. 1024 partial sums of four running ones each: the order of additions is fixed by
+// the rows alone, so the result is reproducible. read: how a row's loss is read.
+constexpr int kMeanSums = 1024;
+template <int THREADS, typename Read>
+__device__ __forceinline__ void mean_of_rows(float* __restrict__ loss, Read&& read, unsigned int rows, float inv_rows, double* stage) {
+    for (unsigned int t = threadIdx.x; t < kMeanSums; t += THREADS) {
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+        unsigned int i = t;
+        for (; i + 3 * kMeanSums < rows; i += 4 * kMeanSums) {
+            s0 += static_cast<double>(read(i));
+            s1 += static_cast<double>(read(i + kMeanSums));
+            s2 += static_cast<double>(read(i + 2 * kMeanSums));
+            s3 += static_cast<double>(read(i + 3 * kMeanSums));
+        }
+        for (; i < rows; i += kMeanSums) s0 += static_cast<double>(read(i));
+        stage[t] = (s0 + s1) + (s2 + s3);
+    }
+    __syncthreads();
+    for (unsigned int stride = kMeanSums / 2; stride > 0; stride >>= 1) {
+        for (unsigned int t = threadIdx.x; t < stride; t += THREADS) stage[t] += stage[t + stride];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) loss[0] = static_cast<float>(stage[0]) * inv_rows;
+}
+
+// The mean that the last workgroup of a row launch takes, in place of a launch that begins when all of this one has ended: bf16 [16, 1000] 8.3 -> 6.2 us,
+// [100, 32000] 9.8 -> 7.8. The workgroups meet on one counter, which takes one of them every 12 ns: [4096, 1000] would take 52 us for 12, fp32
+// [512, 50257] 24 for 22.
+struct MeanArgs {
+    float* loss;
+    unsigned int* counter;  // null: no mean
+    float inv_rows;
+};
+constexpr std::size_t kMostMeanRows = 128;
+
 // Streaming kernel for rows that are too long to hold: each row is split into the elements before its first
 // 16-byte boundary (a vocabulary that is not a multiple of the vector width moves every row's start), whole 128-bit
 // vectors, and the rest. vector_ok: logits and gradient rows have the same alignment phase (or there is no gradient).
@@ -152,10 +187,12 @@ template <typename T, int THREADS, int SLOTS, bool WithGradient, bool ONCE>
 __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
     float* __restrict__ row_loss, T* gradient /* may alias logits */, const T* logits,
     const std::uint32_t* __restrict__ targets, unsigned int vocab, std::size_t ld_logits, std::size_t ld_gradient,
-    float factor) {
+    float factor, MeanArgs mean) {
     constexpr int VEC = kVec128<T>;
     constexpr int WAVES = THREADS / kWave;
     __shared__ MaxSum stage[WAVES];
+    __shared__ double mean_stage[kMeanSums];
+    __shared__ bool last;
     const T* row = logits + blockIdx.x * ld_logits;
     const unsigned int vectors = vocab / VEC, tail = vectors * VEC + threadIdx.x;  // tail: this thread's element behind them
     const std::uint32_t target = targets[blockIdx.x];
@@ -193,7 +230,9 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
     if (threadIdx.x == 0) {
         float loss = 0.0f;
         if (target < vocab) loss = __logf(total.s) + total.m - target_logit;
-        row_loss[blockIdx.x] = loss;
+        if (mean.counter != nullptr)  // before the gradient's stores, which it would wait for
+            last = leave_and_count(row_loss + blockIdx.x, loss, mean.counter, fold_share(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)));
+        else row_loss[blockIdx.x] = loss;
     }
     if constexpr (WithGradient) {
         const float inv = 1.0f / total.s;
@@ -227,11 +266,14 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
         }
         for (std::size_t i = vocab + threadIdx.x; i < ld_gradient; i += THREADS) out[i] = from_f32<T>(0.0f);
     }
+    if (mean.counter == nullptr) return;
+    __syncthreads();
+    if (last) mean_of_rows<THREADS>(mean.loss, [row_loss](unsigned int i) { return read_left(row_loss + i); }, gridDim.x, mean.inv_rows, mean_stage);
 }
 
 template <typename T, int THREADS, int SLOTS>
 void launch_resident(float* row_loss, T* gradient, const T* logits, const std::uint32_t* targets, unsigned int rows,
-                     unsigned int vocab, std::size_t ld_logits, std::size_t ld_gradient, float factor, hipStream_t stream) {
+                     unsigned int vocab, std::size_t ld_logits, std::size_t ld_gradient, float factor, const MeanArgs& mean, hipStream_t stream) {
     // More logits and gradients than the memory-side cache holds until somebody reads them again: bf16 [16384, 32000] in place 367 -> 342 us,
     // fp32 [2048, 32000] 107 -> 98, f16 [4096, 20011] (328 MB) 78 -> 72; fp32 [700, 50257] (281 MB), of which a part is still found there, 60 and 64.
     const std::size_t bytes = static_cast<std::size_t>(rows) * vocab * sizeof(T) * (gradient != nullptr && gradient != logits ? 2 : 1);
@@ -241,7 +283,7 @@ void launch_resident(float* row_loss, T* gradient, const T* logits, const std::u
                                       : (once ? cross_entropy_row_resident_kernel<T, THREADS, SLOTS, true, true>
                                               : cross_entropy_row_resident_kernel<T, THREADS, SLOTS, true, false>);
     hipLaunchKernelGGL(kernel, dim3(rows), dim3(THREADS), 0, stream, row_loss, gradient, logits, targets, vocab, ld_logits,
-                       ld_gradient, factor);
+                       ld_gradient, factor, mean);
 }
 
 }  // namespace
@@ -250,42 +292,28 @@ void launch_resident(float* row_loss, T* gradient, const T* logits, const std::u
 __global__ __launch_bounds__(1024) void mean_reduce_kernel(float* __restrict__ loss,
                                                           const float* __restrict__ row_loss, unsigned int rows,
                                                           float inv_rows) {
-    __shared__ double stage[1024];
-    // Four independent partial sums per thread keep four loads in flight; the order of additions is
-    // fixed by (rows, thread count), so the result is reproducible.
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    unsigned int i = threadIdx.x;
-    for (; i + 3 * 1024 < rows; i += 4 * 1024) {
-        s0 += static_cast<double>(row_loss[i]);
-        s1 += static_cast<double>(row_loss[i + 1024]);
-        s2 += static_cast<double>(row_loss[i + 2 * 1024]);
-        s3 += static_cast<double>(row_loss[i + 3 * 1024]);
-    }
-    for (; i < rows; i += 1024) s0 += static_cast<double>(row_loss[i]);
-    stage[threadIdx.x] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    for (int stride = 512; stride > 0; stride >>= 1) {
-        if (threadIdx.x < static_cast<unsigned int>(stride)) stage[threadIdx.x] += stage[threadIdx.x + stride];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) loss[0] = static_cast<float>(stage[0]) * inv_rows;
+    __shared__ double stage[kMeanSums];
+    mean_of_rows<1024>(loss, [row_loss](unsigned int i) { return row_loss[i]; }, rows, inv_rows, stage);
 }
 
 // Per-row pass: row_loss[r] and (optionally) the gradient, factor = gradient_scale / total_rows.
 int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient, const void* logits, std::size_t ld_logits,
                        const std::uint32_t* targets, std::size_t rows, std::size_t vocab, float factor, int dtype,
-                       hipStream_t stream) {
+                       hipStream_t stream, float* loss) {
+    MeanArgs mean{loss, nullptr, 1.0f / static_cast<float>(rows)};
+    if (loss != nullptr && rows <= kMostMeanRows) mean.counter = tickets(stream);
     const auto r = static_cast<unsigned int>(rows), v = static_cast<unsigned int>(vocab);
     return dispatch_dtype(dtype, [&]<typename T>() -> int {
         auto* g = static_cast<T*>(gradient);
         auto* z = static_cast<const T*>(logits);
         // A thread holds up to 16 vectors; 1024 threads where 512 would not reach.
         const unsigned int vectors = v / kVec128<T>;
-        if (vectors <= 2u * 512) launch_resident<T, 512, 2>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, stream);
-        else if (vectors <= 8u * 512) launch_resident<T, 512, 8>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, stream);
-        else if (vectors <= 16u * 512) launch_resident<T, 512, 16>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, stream);
-        else if (vectors <= 16u * 1024) launch_resident<T, 1024, 16>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, stream);
+        if (vectors <= 2u * 512) launch_resident<T, 512, 2>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
+        else if (vectors <= 8u * 512) launch_resident<T, 512, 8>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
+        else if (vectors <= 16u * 512) launch_resident<T, 512, 16>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
+        else if (vectors <= 16u * 1024) launch_resident<T, 1024, 16>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
         else {
+            mean.counter = nullptr;
             // The streaming kernel finds each row's own 16-byte boundary; logits and gradient rows must share it.
             const bool same_phase = g == nullptr || (((reinterpret_cast<std::uintptr_t>(z) ^ reinterpret_cast<std::uintptr_t>(g)) & 15u) == 0 &&
                                                      (ld_logits - ld_gradient) % kVec128<T> == 0);
@@ -294,7 +322,7 @@ int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient,
                                factor, same_phase);
         }
         CGPTX_LAUNCH_CHECK();
-        return CGPTX_OK;
+        return loss != nullptr && mean.counter == nullptr ? mean_reduce(loss, row_loss, rows, stream) : CGPTX_OK;
     });
 }
 
@@ -322,10 +350,8 @@ int run(float* loss, void* gradient, const void* logits, const std::uint32_t* ta
     if (int s = scratch(stream, rows * sizeof(float), &mem)) return s;
     auto* row_loss = static_cast<float*>(mem);
     const float factor = gradient_scale / static_cast<float>(rows);
-    if (int s = cross_entropy_rows(row_loss, with_gradient ? gradient : nullptr, vocab, logits, vocab, targets, rows, vocab,
-                                   factor, dtype, stream))
-        return s;
-    return mean_reduce(loss, row_loss, rows, stream);
+    return cross_entropy_rows(row_loss, with_gradient ? gradient : nullptr, vocab, logits, vocab, targets, rows, vocab, factor,
+                              dtype, stream, loss);
 }
 
 }  // namespace

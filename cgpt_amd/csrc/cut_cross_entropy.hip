@@ -150,7 +150,7 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         z.dtype = dtype;
         z.no_split = true;
         if (int s = gemm(z, stream)) return s;
-        if (int s = cross_entropy_rows(row_loss + r0, logits, pitch, logits, pitch, targets + r0, r, vocab, factor, dtype, stream))
+        if (int s = cross_entropy_rows(row_loss + r0, logits, pitch, logits, pitch, targets + r0, r, vocab, factor, dtype, stream, r == rows ? loss : nullptr))
             return s;
         GemmArgs dx = input_gradient_call(r0, r);
         dx.a = logits;
@@ -176,5 +176,5 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         dc.split_workspace_bytes = split_bytes;
         if (int s = gemm(dc, stream)) return s;
     }
-    return mean_reduce(loss, row_loss, rows, stream);
+    return single ? CGPTX_OK : mean_reduce(loss, row_loss, rows, stream);
 }

@@ -61,13 +61,6 @@ struct KernelArgs {
 // k_tiles_per_slice are set.
 constexpr int fold_tile_bytes(int rows, int columns) { return rows * columns * 4 + rows * 4; }  // of a tile's slice: accumulators, and sums of A's columns
 constexpr int kPairWeightRows = 256, kPairWeightColumns = 128;  // the weight gradient's tile beside an oblong one of the input gradient
-// What a K slice adds to the counter of its tile: shares that make 2^32 together, none of them zero. The workgroup that brings the
-// counter back to zero is the tile's last one, and a launch leaves the counter as it found it: also where two launches met on the same
-// counters (a graph replayed beside other work of the stream it was captured on), whatever slices each has, the next one counts from zero.
-__host__ __device__ constexpr unsigned int fold_share(int slice, int slices) {
-    const unsigned int even = 0xFFFFFFFFu / static_cast<unsigned int>(slices);
-    return slice == 0 ? 0u - even * static_cast<unsigned int>(slices - 1) : even;
-}
 struct PairArgs {
     KernelArgs input, weight;
     int input_tile;  // 128: both on 128 x 128 tiles

@@ -7,7 +7,7 @@ import torch
 
 from cgpt_amd import ops
 from oracle import cpu_ops, oracle64
-from tests.util import DTYPES, DTYPE_IDS, TOL, assert_close, randint, randn, to_np
+from tests.util import DTYPES, DTYPE_IDS, TOL, assert_close, launches, randint, randn, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -493,3 +493,44 @@ def test_cross_entropy_of_more_logits_than_the_memory_cache_gives_the_rows_of_fe
     only = torch.empty(1, device=device)
     ops.cross_entropy_forward(only, logits, targets, rows)
     assert only.item() == loss.item()
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1003), (torch.float32, 9000), (torch.float16, 140000)], ids=["bf16", "f32", "f16"])
+@pytest.mark.parametrize("rows", [1, 2, 127, 128, 129])
+def test_mean_loss_of_few_rows_comes_from_the_rows_launch(device, dtype, vocab, rows):
+    """Up to 128 rows the last workgroup takes the mean (longer rows than the registers hold: a launch of its own). Three calls in a row
+    and three replays: the workgroups' counter is left as it was found. The bound is the rounding of a row's loss, 2^-24 of values around
+    log V and of the largest logit, in rows and in their mean, and that of the fast exponential and logarithm, a few units each."""
+    logits = randn((rows, vocab), dtype, rows + vocab)
+    targets = randint(vocab, (rows,), rows)
+    wide = logits.double()
+    want = (torch.logsumexp(wide, 1) - wide.gather(1, targets.long()[:, None])[:, 0]).mean().item()
+    z, y = dev(logits, device), dev(targets, device)
+    loss, gradient = torch.empty(1, device=device), torch.empty_like(z)
+    for with_gradient in (True, False):
+        def call():
+            if with_gradient:
+                ops.cross_entropy_forward_backward(loss, gradient, z, y, rows)
+            else:
+                ops.cross_entropy_forward(loss, z, y, rows)
+        seen = set()
+        for _ in range(3):
+            loss.fill_(float("nan"))
+            call()
+            seen.add(loss.item())
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            call()
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                call()
+            for _ in range(3):
+                loss.fill_(float("nan"))
+                graph.replay()
+                call()
+                seen.add(loss.item())
+        assert len(seen) == 1
+        assert abs(seen.pop() - want) <= 2e-6 * max(1.0, abs(want))
+    long_rows = vocab > 131072 and dtype != torch.float32
+    assert launches(lambda: ops.cross_entropy_forward(loss, z, y, rows)) == (1 if rows <= 128 and not long_rows else 2)
