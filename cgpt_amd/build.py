@@ -114,7 +114,7 @@ def build_dispatch(force: bool = True) -> pathlib.Path:
     libraries = cpp_extension.library_paths()
     cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f"-I{path}" for path in includes), str(DISPATCH_SOURCE), "-o", str(DISPATCH_PATH),
-           *(f"-L{path}" for path in libraries), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           f"-L{LIB_DIR}", "-lcgptx", "-Wl,-rpath,$ORIGIN/lib", *(f"-L{path}" for path in libraries), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
            *(f"-Wl,-rpath,{path}" for path in libraries)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

@@ -69,6 +69,22 @@ def _load_dispatch():
     globals().update(_tensors=_dispatch.tensors, _same_shape=_dispatch.same_shape, _adamw_entries=_dispatch.adamw_entries)
 
 
+class _Native:
+    """The native operator calls of host/dispatch.cpp, loaded on first use. Each takes a call as programs make it as a rule and gives
+    the library's status, or None, having done nothing, for one that the functions below look at themselves."""
+
+    def __getattr__(self, name):
+        capi.lib()  # says what is missing where the library is
+        _load_dispatch()
+        from . import _dispatch
+        function = getattr(_dispatch, name)
+        setattr(self, name, function)
+        return function
+
+
+_native = _Native()
+
+
 def _tensors(*tensors):  # replaced by the native function on first use
     _load_dispatch()
     return _tensors(*tensors)
@@ -158,6 +174,11 @@ class AdamWOptions:  # include/optim/adamw.h:12-27
 # --------------------------------------------------------------------------- backward
 def rmsnorm_backward(grad_input, grad_weight, grad_output, input, weight, epsilon, stream=None):
     """include/ops/backward/rmsnorm_backward.h:21-29."""
+    status = _native.rmsnorm_backward(grad_input, grad_weight, grad_output, input, weight, epsilon, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "rmsnorm_backward"
     if not (math.isfinite(epsilon) and epsilon > 0):
         raise ValueError(f"{name}: epsilon must be finite and positive")
@@ -187,6 +208,12 @@ def _rope_check(name, q, k, cos_cache, sin_cache, options):
 def rope_backward(grad_query, grad_key, grad_rotated_query, grad_rotated_key, cos_cache, sin_cache, stream=None,
                   rope_options: RopeOptions = RopeOptions()):
     """include/ops/backward/rope_backward.h:22-31."""
+    status = _native.rope_backward(grad_query, grad_key, grad_rotated_query, grad_rotated_key, cos_cache, sin_cache, rope_options.rotary_dim,
+                                   rope_options.position_offset, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "rope_backward"
     code, gq, gk, rq, rk, cos, sin = \
         _tensors(grad_query, grad_key, grad_rotated_query, grad_rotated_key, cos_cache, sin_cache) or \
@@ -202,6 +229,11 @@ def rope_backward(grad_query, grad_key, grad_rotated_query, grad_rotated_key, co
 def swiglu_backward(grad_gate, grad_up, grad_output, gate, up, stream=None,
                     options: SwiGLUBackwardOptions = SwiGLUBackwardOptions()):
     """include/ops/backward/swiglu_backward.h:30-38."""
+    status = _native.swiglu_backward(grad_gate, grad_up, grad_output, gate, up, options.accumulate_gate, options.accumulate_up, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "swiglu_backward"
     code, dg, du, dy, g, u = _tensors(grad_gate, grad_up, grad_output, gate, up) or \
         _reject(name, grad_gate, grad_up, grad_output, gate, up)
@@ -229,6 +261,12 @@ def swiglu_backward_packed(grad_gate_up, grad_output, gate_up, stream=None,
 def linear_backward(grad_input, grad_weight, grad_bias, grad_output, input, weight, gemm_context=None, stream=None,
                     options: LinearBackwardOptions = LinearBackwardOptions()):
     """include/ops/backward/linear_backward.h:36-46 (gemm_context stands where the cuBLASLt context is)."""
+    status = _native.linear_backward(grad_input, grad_weight, grad_bias, grad_output, input, weight, options.accumulate_input,
+                                     options.accumulate_weight, options.accumulate_bias, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "linear_backward"
     code, dx, dw, db, dy, x, w = _tensors(grad_input, grad_weight, grad_bias, grad_output, input, weight) or \
         _reject(name, grad_input, grad_weight, grad_bias, grad_output, input, weight)
@@ -251,6 +289,12 @@ def linear_backward(grad_input, grad_weight, grad_bias, grad_output, input, weig
 def embedding_backward(grad_weight, grad_output, device_token_ids, token_count, stream=None,
                        options: EmbeddingBackwardOptions = EmbeddingBackwardOptions()):
     """include/ops/backward/embedding_backward.h:35-42."""
+    status = _native.embedding_backward(grad_weight, grad_output, device_token_ids, token_count, options.bounds_check,
+                                        options.accumulate_weight, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "embedding_backward"
     code, dw, dy = _tensors(grad_weight, grad_output) or _reject(name, grad_weight, grad_output)
     if token_count == 0:
@@ -275,6 +319,11 @@ def _ce_check(name, loss, logits, targets, target_count):
 def cross_entropy_forward_backward(loss, gradient, logits, device_targets, target_count, stream=None,
                                    gradient_scale: float = 1.0):
     """include/ops/cross_entropy.h:25-32."""
+    status = _native.cross_entropy_forward_backward(loss, gradient, logits, device_targets, target_count, gradient_scale, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "cross_entropy_forward_backward"
     code, g, z = _tensors(gradient, logits) or _reject(name, gradient, logits)
     _ce_check(name, loss, logits, device_targets, target_count)
@@ -287,6 +336,11 @@ def cross_entropy_forward_backward(loss, gradient, logits, device_targets, targe
 
 def cross_entropy_forward(loss, logits, device_targets, target_count, stream=None):
     """include/ops/cross_entropy.h:37-42."""
+    status = _native.cross_entropy_forward(loss, logits, device_targets, target_count, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "cross_entropy_forward"
     code, z = _tensors(logits) or _reject(name, logits)
     _ce_check(name, loss, logits, device_targets, target_count)
@@ -298,6 +352,12 @@ def cut_cross_entropy_forward_backward(loss, input_gradient, classifier_gradient
                                        target_count, stream=None, gradient_scale: float = 1.0,
                                        accumulate_classifier: bool = False):
     """include/ops/cut_cross_entropy.h:25-33; gradient_scale and accumulate_classifier are extensions."""
+    status = _native.cut_cross_entropy_forward_backward(loss, input_gradient, classifier_gradient, input, classifier, device_targets,
+                                                        target_count, gradient_scale, accumulate_classifier, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "cut_cross_entropy_forward_backward"
     code, dx, dc, x, c = _tensors(input_gradient, classifier_gradient, input, classifier) or \
         _reject(name, input_gradient, classifier_gradient, input, classifier)
@@ -332,6 +392,12 @@ def flash_gqa_attention_backward_with_lse(grad_query, grad_key, grad_value, grad
                                           options: FlashAttentionOptions = FlashAttentionOptions(),
                                           accumulate_grads: bool = False):
     """include/ops/backward/attention_backward.h:57-70."""
+    status = _native.attention_backward_with_lse(grad_query, grad_key, grad_value, grad_output, output, logsumexp, query, key, value,
+                                                 options, accumulate_grads, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "flash_gqa_attention_backward_with_lse"
     code, dq, dk, dv, do, o, q, k, v = \
         _tensors(grad_query, grad_key, grad_value, grad_output, output, query, key, value) or \
@@ -351,6 +417,11 @@ def flash_gqa_attention_backward(grad_query, grad_key, grad_value, grad_output, 
                                  options: FlashAttentionOptions = FlashAttentionOptions(),
                                  accumulate_grads: bool = False):
     """include/ops/backward/attention_backward.h:24-35."""
+    status = _native.attention_backward(grad_query, grad_key, grad_value, grad_output, query, key, value, options, accumulate_grads, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "flash_gqa_attention_backward"
     code, dq, dk, dv, do, q, k, v = _tensors(grad_query, grad_key, grad_value, grad_output, query, key, value) or \
         _reject(name, grad_query, grad_key, grad_value, grad_output, query, key, value)
@@ -491,6 +562,11 @@ def adamw_step(parameter, gradient, state: AdamWState, options: AdamWOptions = A
 # ---------------------------------------------------------------------------- forward
 def rmsnorm_forward(output, input, weight, epsilon, stream=None):
     """include/ops/rmsnorm.h."""
+    status = _native.rmsnorm_forward(output, input, weight, epsilon, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "rmsnorm_forward"
     if not (math.isfinite(epsilon) and epsilon > 0):
         raise ValueError(f"{name}: epsilon must be finite and positive")
@@ -503,6 +579,11 @@ def rmsnorm_forward(output, input, weight, epsilon, stream=None):
 
 def rope_forward(query, key, cos_cache, sin_cache, stream=None, rope_options: RopeOptions = RopeOptions()):
     """include/ops/rope.h:32-39 (in place)."""
+    status = _native.rope_forward(query, key, cos_cache, sin_cache, rope_options.rotary_dim, rope_options.position_offset, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "rope_forward"
     code, q, k, cos, sin = _tensors(query, key, cos_cache, sin_cache) or _reject(name, query, key, cos_cache, sin_cache)
     _rope_check(name, query, key, cos_cache, sin_cache, rope_options)
@@ -515,6 +596,12 @@ def swiglu_forward(output, gate, up=None, stream=None):
     """include/ops/swiglu.h: (output, gate, up) or, with up omitted, (output, gate_up) with the
     projections concatenated along the last dimension."""
     name = "swiglu_forward"
+    if up is not None:
+        status = _native.swiglu_forward(output, gate, up, stream)
+        if status == 0:
+            return
+        if status:
+            capi.check(status)
     if up is None:
         gate_up = gate
         code, y, gu = _tensors(output, gate_up) or _reject(name, output, gate_up)
@@ -536,6 +623,11 @@ def swiglu_forward(output, gate, up=None, stream=None):
 
 def linear_forward(output, input, weight, gemm_context=None, stream=None, bias=None):
     """include/ops/linear.h."""
+    status = _native.linear_forward(output, input, weight, bias, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "linear_forward"
     code, y, x, w, b = _tensors(output, input, weight, bias) or _reject(name, output, input, weight, bias)
     x_shape, w_shape, y_shape = input.shape, weight.shape, output.shape
@@ -603,6 +695,11 @@ def linear_backward_weights_stacked(grad_weight, grad_output, input, stream=None
 
 def embedding_forward(output, device_token_ids, token_count, weight, stream=None):
     """include/ops/embedding.h."""
+    status = _native.embedding_forward(output, device_token_ids, token_count, weight, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "embedding_forward"
     code, y, w = _tensors(output, weight) or _reject(name, output, weight)
     _ids(name, device_token_ids, token_count)
@@ -615,6 +712,11 @@ def embedding_forward(output, device_token_ids, token_count, weight, stream=None
 def flash_gqa_attention_forward_with_lse(output, logsumexp, query, key, value, stream=None,
                                          options: FlashAttentionOptions = FlashAttentionOptions()):
     """include/ops/attention.h:70-78."""
+    status = _native.attention_forward(output, logsumexp, query, key, value, options, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "flash_gqa_attention_forward_with_lse"
     code, o, q, k, v = _tensors(output, query, key, value) or _reject(name, output, query, key, value)
     if logsumexp is not None:
@@ -636,6 +738,11 @@ def flash_gqa_attention_forward(output, query, key, value, stream=None,
 
 def add_tensors(output, a, b, stream=None):
     """src/core/transformer_block.cu:242-248."""
+    status = _native.add(output, a, b, stream)
+    if status == 0:
+        return
+    if status:
+        capi.check(status)
     name = "add"
     code, y, x1, x2 = _tensors(output, a, b) or _reject(name, output, a, b)
     if not _same_shape(a, output, b):
