@@ -179,8 +179,23 @@ struct ColumnReduceSink {
 // most, for q's and k's rows together.
 enum class NormPass { plain, with_rope, dual };
 std::size_t rmsnorm_backward_sink_bytes(NormPass pass, std::size_t rows, std::size_t hidden, int dtype);
-// Runs the reductions recorded in `table` (device copy of `entries`).
-int run_column_reductions(const ColumnReduceEntry* table, const std::vector<ColumnReduceEntry>& entries, hipStream_t stream);
+// A mean loss to be taken from rows' losses (null: none).
+struct MeanEntry {
+    float* loss = nullptr;
+    const float* row_losses = nullptr;
+    unsigned int rows = 0;
+};
+// Runs the reductions recorded in `table` (device copy of `entries`), and takes the mean in the same launch.
+int run_column_reductions(const ColumnReduceEntry* table, const std::vector<ColumnReduceEntry>& entries, const MeanEntry& mean, hipStream_t stream);
+
+// The lookup of a step's tokens and, where few enough that a launch costs more than its work (*grouped), the grouping that the
+// scatter of their gradient starts from, as workgroups of the same launch. groups: embedding_groups_bytes(...) of memory that stays until
+// the scatter; given no groups the scatter makes its own.
+std::size_t embedding_groups_bytes(std::size_t token_count, std::size_t vocab);
+int embedding_forward_and_group(void* output, const std::uint32_t* token_ids, std::size_t token_count, const void* weight, std::size_t vocab,
+                                std::size_t hidden, void* groups, int dtype, hipStream_t stream, bool* grouped);
+int embedding_backward_grouped(void* grad_weight, const void* grad_output, const std::uint32_t* token_ids, std::size_t token_count,
+                               std::size_t vocab, std::size_t hidden, int accumulate_weight, void* groups, int dtype, hipStream_t stream);
 
 // ---- fused variants used by the composed train step --------------------------
 // rmsnorm backward with grad_input = (norm gradient) + residual; residual may be null or alias
@@ -198,7 +213,10 @@ struct LinearParts {
 int linear_backward(void* grad_input, void* grad_weight, void* grad_bias, const void* grad_output, const void* input,
                     const void* weight, std::size_t rows, std::size_t in_features, std::size_t out_features,
                     int accumulate_input, int accumulate_weight, int accumulate_bias, int dtype, hipStream_t stream,
-                    LinearParts* parts, bool large_pairs = true);
+                    LinearParts* parts, bool large_pairs = true, std::size_t grad_output_pitch = 0);
+// The row length at which linear_backward reads an output gradient as it lies (grad_output_pitch; zeros past out_features), where it
+// would copy rows of out_features elements to such rows first. out_features: it would not. Tensors on 16-byte boundaries.
+std::size_t linear_backward_pitch(std::size_t rows, std::size_t in_features, std::size_t out_features, int dtype);
 
 // Per-head RMSNorm and rotary embedding of q and k in one pass over their [rows = tokens x heads, head_dim]:
 //   forward   output = rope(rmsnorm(input));   backward   output = the gradient of that, with the weight gradient.

@@ -48,31 +48,6 @@ __device__ __forceinline__ MaxSum block_combine(MaxSum v, MaxSum* stage) {
     return total;
 }
 
-// (Σ row_loss) / rows by a workgroup of THREADS. 1024 partial sums of four running ones each: the order of additions is fixed by
-// the rows alone, so the result is reproducible. read: how a row's loss is read.
-constexpr int kMeanSums = 1024;
-template <int THREADS, typename Read>
-__device__ __forceinline__ void mean_of_rows(float* __restrict__ loss, Read&& read, unsigned int rows, float inv_rows, double* stage) {
-    for (unsigned int t = threadIdx.x; t < kMeanSums; t += THREADS) {
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-        unsigned int i = t;
-        for (; i + 3 * kMeanSums < rows; i += 4 * kMeanSums) {
-            s0 += static_cast<double>(read(i));
-            s1 += static_cast<double>(read(i + kMeanSums));
-            s2 += static_cast<double>(read(i + 2 * kMeanSums));
-            s3 += static_cast<double>(read(i + 3 * kMeanSums));
-        }
-        for (; i < rows; i += kMeanSums) s0 += static_cast<double>(read(i));
-        stage[t] = (s0 + s1) + (s2 + s3);
-    }
-    __syncthreads();
-    for (unsigned int stride = kMeanSums / 2; stride > 0; stride >>= 1) {
-        for (unsigned int t = threadIdx.x; t < stride; t += THREADS) stage[t] += stage[t + stride];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) loss[0] = static_cast<float>(stage[0]) * inv_rows;
-}
-
 // The mean that the last workgroup of a row launch takes, in place of a launch that begins when all of this one has ended: bf16 [16, 1000] 8.3 -> 6.2 us,
 // [100, 32000] 9.8 -> 7.8. The workgroups meet on one counter, which takes one of them every 12 ns: [4096, 1000] would take 52 us for 12, fp32
 // [512, 50257] 24 for 22.
@@ -299,7 +274,7 @@ __global__ __launch_bounds__(1024) void mean_reduce_kernel(float* __restrict__ l
 // Per-row pass: row_loss[r] and (optionally) the gradient, factor = gradient_scale / total_rows.
 int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient, const void* logits, std::size_t ld_logits,
                        const std::uint32_t* targets, std::size_t rows, std::size_t vocab, float factor, int dtype,
-                       hipStream_t stream, float* loss) {
+                       hipStream_t stream, float* loss, bool* mean_taken) {
     MeanArgs mean{loss, nullptr, 1.0f / static_cast<float>(rows)};
     if (loss != nullptr && rows <= kMostMeanRows) mean.counter = tickets(stream);
     const auto r = static_cast<unsigned int>(rows), v = static_cast<unsigned int>(vocab);
@@ -322,7 +297,8 @@ int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient,
                                factor, same_phase);
         }
         CGPTX_LAUNCH_CHECK();
-        return loss != nullptr && mean.counter == nullptr ? mean_reduce(loss, row_loss, rows, stream) : CGPTX_OK;
+        if (mean_taken != nullptr) *mean_taken = mean.counter != nullptr;
+        return CGPTX_OK;
     });
 }
 
@@ -350,8 +326,11 @@ int run(float* loss, void* gradient, const void* logits, const std::uint32_t* ta
     if (int s = scratch(stream, rows * sizeof(float), &mem)) return s;
     auto* row_loss = static_cast<float*>(mem);
     const float factor = gradient_scale / static_cast<float>(rows);
-    return cross_entropy_rows(row_loss, with_gradient ? gradient : nullptr, vocab, logits, vocab, targets, rows, vocab, factor,
-                              dtype, stream, loss);
+    bool mean_taken = false;
+    if (int s = cross_entropy_rows(row_loss, with_gradient ? gradient : nullptr, vocab, logits, vocab, targets, rows, vocab, factor,
+                                   dtype, stream, loss, &mean_taken))
+        return s;
+    return mean_taken ? CGPTX_OK : mean_reduce(loss, row_loss, rows, stream);
 }
 
 }  // namespace

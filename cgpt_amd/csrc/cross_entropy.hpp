@@ -7,12 +7,42 @@ namespace cgptx {
 
 // row_loss[r] = [y_r < V](logsumexp z_r − z_{r,y_r}); gradient (may be null, may be the logits' own memory) =
 // (softmax − onehot)·factor. Rows are ld_logits and ld_gradient elements apart; gradient columns from vocab to
-// ld_gradient are cleared. loss (may be null): where the mean over these rows goes, see mean_reduce.
+// ld_gradient are cleared. loss (may be null): where the mean over these rows goes if they are few (*mean_taken; see mean_reduce).
 int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient, const void* logits, std::size_t ld_logits,
                        const std::uint32_t* targets, std::size_t rows, std::size_t vocab, float factor, int dtype,
-                       hipStream_t stream, float* loss = nullptr);
+                       hipStream_t stream, float* loss = nullptr, bool* mean_taken = nullptr);
 
 // loss[0] = (Σ row_loss) / rows, summed in a fixed order.
 int mean_reduce(float* loss, const float* row_loss, std::size_t rows, hipStream_t stream);
+
+// cgptx_cut_cross_entropy_forward_backward whose rows' losses are left in row_losses; the mean is the caller's to take.
+int cut_cross_entropy(float* row_losses, void* input_gradient, void* classifier_gradient, const void* input, const void* classifier,
+                      const std::uint32_t* targets, std::size_t rows, std::size_t hidden, std::size_t vocab, float gradient_scale,
+                      int dtype, hipStream_t stream);
+
+// (Σ row_loss) / rows by a workgroup of THREADS. 1024 partial sums of four running ones each: the order of additions is fixed by
+// the rows alone, so the result is reproducible. read: how a row's loss is read.
+constexpr int kMeanSums = 1024;
+template <int THREADS, typename Read>
+__device__ __forceinline__ void mean_of_rows(float* __restrict__ loss, Read&& read, unsigned int rows, float inv_rows, double* stage) {
+    for (unsigned int t = threadIdx.x; t < kMeanSums; t += THREADS) {
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+        unsigned int i = t;
+        for (; i + 3 * kMeanSums < rows; i += 4 * kMeanSums) {
+            s0 += static_cast<double>(read(i));
+            s1 += static_cast<double>(read(i + kMeanSums));
+            s2 += static_cast<double>(read(i + 2 * kMeanSums));
+            s3 += static_cast<double>(read(i + 3 * kMeanSums));
+        }
+        for (; i < rows; i += kMeanSums) s0 += static_cast<double>(read(i));
+        stage[t] = (s0 + s1) + (s2 + s3);
+    }
+    __syncthreads();
+    for (unsigned int stride = kMeanSums / 2; stride > 0; stride >>= 1) {
+        for (unsigned int t = threadIdx.x; t < stride; t += THREADS) stage[t] += stage[t + stride];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) loss[0] = static_cast<float>(stage[0]) * inv_rows;
+}
 
 }  // namespace cgptx

@@ -25,15 +25,16 @@
 #include <cstdlib>
 #include <limits>
 
-extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input_gradient, void* classifier_gradient,
-                                                        const void* input, const void* classifier,
-                                                        const uint32_t* targets, size_t rows, size_t hidden,
-                                                        size_t vocab, float gradient_scale,
-                                                        int accumulate_classifier, int dtype, cgptx_stream stream_) {
-    using namespace cgptx;
+namespace cgptx {
+namespace {
+
+// row_losses: null, or where the rows' losses are left, in place of their mean in `loss`.
+int run(float* loss, float* row_losses, void* input_gradient, void* classifier_gradient, const void* input, const void* classifier,
+        const std::uint32_t* targets, std::size_t rows, std::size_t hidden, std::size_t vocab, float gradient_scale,
+        int accumulate_classifier, int dtype, hipStream_t stream) {
     const char* name = "cut_cross_entropy";
     if (!valid_dtype(dtype)) return fail(CGPTX_INVALID_ARGUMENT, std::string(name) + ": unsupported dtype");
-    if (loss == nullptr || input_gradient == nullptr || classifier_gradient == nullptr || input == nullptr ||
+    if ((loss == nullptr && row_losses == nullptr) || input_gradient == nullptr || classifier_gradient == nullptr || input == nullptr ||
         classifier == nullptr || targets == nullptr || rows == 0 || hidden == 0 || vocab == 0)
         return fail(CGPTX_INVALID_ARGUMENT,
                     std::string(name) + ": input and classifier must be non-empty matrices with gradients and targets");
@@ -42,7 +43,6 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
     constexpr std::size_t i32max = std::numeric_limits<int>::max();
     if (rows > i32max || hidden > i32max || vocab > i32max)
         return fail(CGPTX_OVERFLOW, std::string(name) + ": dimension exceeds int range");
-    auto stream = static_cast<hipStream_t>(stream_);
     const std::size_t elem = dtype_size(dtype);
     // Rows are processed in chunks so that the logits scratch stays within 1 GiB whatever the number of rows
     // (CGPTX_CUT_CE_LOGITS_BYTES, read per call, sets another bound, up to 2 GiB - 1 MiB: the streamed contraction
@@ -128,11 +128,12 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
     }
     split_bytes = std::min(split_bytes, (held - needed()) & ~std::size_t{255});
     auto* base = static_cast<char*>(mem);
-    auto* row_loss = reinterpret_cast<float*>(base);
+    auto* row_loss = row_losses != nullptr ? row_losses : reinterpret_cast<float*>(base);
     auto* acc = reinterpret_cast<float*>(base + loss_bytes);
     void* split_room = split_bytes != 0 ? base + loss_bytes + acc_bytes : nullptr;
     void* logits = base + loss_bytes + acc_bytes + split_bytes;
     const float factor = gradient_scale / static_cast<float>(rows);
+    bool mean_taken = false;
     for (std::size_t r0 = 0; r0 < rows; r0 += chunk) {
         const std::size_t r = std::min(chunk, rows - r0);
         const void* x = static_cast<const char*>(input) + r0 * hidden * elem;
@@ -150,7 +151,8 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         z.dtype = dtype;
         z.no_split = true;
         if (int s = gemm(z, stream)) return s;
-        if (int s = cross_entropy_rows(row_loss + r0, logits, pitch, logits, pitch, targets + r0, r, vocab, factor, dtype, stream, r == rows ? loss : nullptr))
+        if (int s = cross_entropy_rows(row_loss + r0, logits, pitch, logits, pitch, targets + r0, r, vocab, factor, dtype, stream,
+                                       single ? loss : nullptr, &mean_taken))
             return s;
         GemmArgs dx = input_gradient_call(r0, r);
         dx.a = logits;
@@ -176,5 +178,25 @@ extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input
         dc.split_workspace_bytes = split_bytes;
         if (int s = gemm(dc, stream)) return s;
     }
-    return single ? CGPTX_OK : mean_reduce(loss, row_loss, rows, stream);
+    return mean_taken || row_losses != nullptr ? CGPTX_OK : mean_reduce(loss, row_loss, rows, stream);
+}
+
+}  // namespace
+
+int cut_cross_entropy(float* row_losses, void* input_gradient, void* classifier_gradient, const void* input, const void* classifier,
+                      const std::uint32_t* targets, std::size_t rows, std::size_t hidden, std::size_t vocab, float gradient_scale,
+                      int dtype, hipStream_t stream) {
+    return run(nullptr, row_losses, input_gradient, classifier_gradient, input, classifier, targets, rows, hidden, vocab, gradient_scale,
+               0, dtype, stream);
+}
+
+}  // namespace cgptx
+
+extern "C" int cgptx_cut_cross_entropy_forward_backward(float* loss, void* input_gradient, void* classifier_gradient,
+                                                        const void* input, const void* classifier,
+                                                        const uint32_t* targets, size_t rows, size_t hidden,
+                                                        size_t vocab, float gradient_scale,
+                                                        int accumulate_classifier, int dtype, cgptx_stream stream) {
+    return cgptx::run(loss, nullptr, input_gradient, classifier_gradient, input, classifier, targets, rows, hidden, vocab,
+                      gradient_scale, accumulate_classifier, dtype, static_cast<hipStream_t>(stream));
 }

@@ -22,7 +22,21 @@ int validate(const char* name, std::size_t rows, std::size_t in_features, std::s
     return CGPTX_OK;
 }
 
+// An output gradient in rows of whole K tiles.
+std::size_t padded(std::size_t out_features) { return (out_features + 31) / 32 * 32; }
+// Whether both contractions of a backward pass then stream: whole chunks of input and weight, the streamed kernels' 32-bit offsets.
+bool copies_stream(std::size_t rows, std::size_t in_features, std::size_t out_features, std::size_t elem) {
+    constexpr std::size_t kSpan = (std::size_t{1} << 31) - (std::size_t{1} << 21);
+    return in_features * elem % 16 == 0 && rows * (out_features + 32 + in_features) * elem < kSpan && out_features * in_features * elem < kSpan;
+}
+
 }  // namespace
+
+std::size_t linear_backward_pitch(std::size_t rows, std::size_t in_features, std::size_t out_features, int dtype) {
+    const std::size_t elem = dtype_size(dtype);
+    return out_features * elem % 16 != 0 && copies_stream(rows, in_features, out_features, elem) ? padded(out_features) : out_features;
+}
+
 }  // namespace cgptx
 
 extern "C" int cgptx_linear_forward(void* output, const void* input, const void* weight, const void* bias,
@@ -163,7 +177,7 @@ extern "C" int cgptx_linear_backward(void* grad_input, void* grad_weight, void* 
 int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias, const void* grad_output, const void* input,
                            const void* weight, std::size_t rows, std::size_t in_features, std::size_t out_features,
                            int accumulate_input, int accumulate_weight, int accumulate_bias, int dtype, hipStream_t stream,
-                           LinearParts* parts, bool large_pairs) {
+                           LinearParts* parts, bool large_pairs, std::size_t grad_output_pitch) {
     if (int s = validate("linear_backward", rows, in_features, out_features, dtype)) return s;
     if (grad_output == nullptr || (grad_input != nullptr && weight == nullptr) ||
         (grad_weight != nullptr && input == nullptr))
@@ -172,7 +186,7 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
     // make its own otherwise).
     const std::size_t elem = dtype_size(dtype);
     const void* dy = grad_output;
-    std::size_t dy_pitch = out_features;
+    std::size_t dy_pitch = grad_output_pitch != 0 ? grad_output_pitch : out_features;
     void* split_room = nullptr;
     std::size_t split_bytes = 0;
     auto input_gradient = [&]() {  // dX[rows, in] = dY[rows, out] · W[out, in]
@@ -216,11 +230,10 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
         g.split_workspace_bytes = split_bytes;
         return g;
     };
-    constexpr std::size_t kSpan = (std::size_t{1} << 31) - (std::size_t{1} << 21);  // the streamed kernels' 32-bit offsets
-    if (grad_input != nullptr && grad_weight != nullptr &&
-        (out_features * elem % 16 != 0 || !is_aligned16(grad_output)) && in_features * elem % 16 == 0 && is_aligned16(weight) &&
-        is_aligned16(input) && rows * (out_features + 32 + in_features) * elem < kSpan && out_features * in_features * elem < kSpan) {
-        dy_pitch = (out_features + 31) / 32 * 32;
+    if (grad_output_pitch == 0 && grad_input != nullptr && grad_weight != nullptr &&
+        (out_features * elem % 16 != 0 || !is_aligned16(grad_output)) && is_aligned16(weight) && is_aligned16(input) &&
+        copies_stream(rows, in_features, out_features, elem)) {
+        dy_pitch = padded(out_features);
         const std::size_t copy_bytes = (rows * dy_pitch * elem + 255) & ~std::size_t{255};
         split_bytes = std::max(gemm_split_bytes(input_gradient()), gemm_split_bytes(weight_gradient())) + 256;
         void* mem = nullptr;
@@ -238,7 +251,7 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
     if (grad_input != nullptr && grad_weight != nullptr) {
         // Small calls: both gradients, and the bias's, in one launch, whose parts run in no order. None may write what another
         // one reads, nor what another one writes: overlapping results hold what the last of the separate launches leaves.
-        const std::size_t dy_bytes = rows * out_features * elem, x_bytes = rows * in_features * elem, w_bytes = out_features * in_features * elem;
+        const std::size_t dy_bytes = rows * std::max(out_features, grad_output_pitch) * elem, x_bytes = rows * in_features * elem, w_bytes = out_features * in_features * elem;
         const std::size_t bias_bytes = out_features * elem;
         auto apart = [](const void* a, std::size_t a_bytes, const void* b, std::size_t b_bytes) {
             const auto x = reinterpret_cast<std::uintptr_t>(a), y = reinterpret_cast<std::uintptr_t>(b);
@@ -268,6 +281,8 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
         if (parts != nullptr)
             if (int s = parts->done(LinearParts::weight)) return s;
     }
+    if (grad_bias != nullptr && grad_output_pitch != 0 && grad_output_pitch != out_features)
+        return fail(CGPTX_RUNTIME, "linear_backward: no bias gradient of an output gradient in padded rows");
     if (grad_bias != nullptr) {  // db[out] = Σ_rows dY
         const int cols = static_cast<int>(out_features);
         const int slices = rows < 256 ? 1 : (rows < 65536 ? 64 : 256);

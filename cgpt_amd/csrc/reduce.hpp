@@ -1,7 +1,7 @@
 // Column reductions shared by the norm and linear kernels.
 #pragma once
 
-#include "common.hpp"
+#include "cross_entropy.hpp"
 
 namespace cgptx {
 
@@ -130,8 +130,16 @@ __device__ __forceinline__ void column_partial_reduce_entry(const ColumnReduceEn
     else column_partial_reduce_body<T, 32>(static_cast<T*>(e.out), e.partial, e.parts, e.hidden, 0, group, units, folded, stage);
 }
 static __global__ __launch_bounds__(kFinishThreads) void column_partial_reduce_table_kernel(
-    const ColumnReduceEntry* __restrict__ table, int units) {
-    __shared__ float folded[kFolded], stage[4 * 32];
+    const ColumnReduceEntry* __restrict__ table, int entries, int units, MeanEntry mean) {
+    __shared__ __align__(8) float folded[kFolded];
+    __shared__ float stage[4 * 32];
+    static_assert(sizeof(folded) >= kMeanSums * sizeof(double), "the mean's sums fit");
+    if (static_cast<int>(blockIdx.y) == entries) {  // a launch of its own would take a step of 300 tokens 4 us
+        if (blockIdx.x == 0)
+            mean_of_rows<kFinishThreads>(mean.loss, [&](unsigned int i) { return mean.row_losses[i]; }, mean.rows,
+                                         1.0f / static_cast<float>(mean.rows), reinterpret_cast<double*>(folded));
+        return;
+    }
     const ColumnReduceEntry e = table[blockIdx.y];
     const int group = static_cast<int>(blockIdx.x);
     if (group * finish_columns(e.hidden) >= e.hidden) return;

@@ -771,12 +771,13 @@ int reduce_columns(ColumnReduceSink* sink, bool deferred, T* dw, const float* pa
     return CGPTX_OK;
 }
 
-int run_column_reductions(const ColumnReduceEntry* table, const std::vector<ColumnReduceEntry>& entries, hipStream_t stream) {
-    if (entries.empty()) return CGPTX_OK;
+int run_column_reductions(const ColumnReduceEntry* table, const std::vector<ColumnReduceEntry>& entries, const MeanEntry& mean, hipStream_t stream) {
+    if (entries.empty()) return mean.rows != 0 ? mean_reduce(mean.loss, mean.row_losses, mean.rows, stream) : CGPTX_OK;
     int groups = 1;
     for (const ColumnReduceEntry& e : entries) groups = std::max(groups, (e.hidden + finish_columns(e.hidden) - 1) / finish_columns(e.hidden));
-    hipLaunchKernelGGL(column_partial_reduce_table_kernel, dim3(groups, static_cast<unsigned int>(entries.size())), dim3(kFinishThreads),
-                       0, stream, table, compute_units());
+    const auto count = static_cast<unsigned int>(entries.size());
+    hipLaunchKernelGGL(column_partial_reduce_table_kernel, dim3(groups, count + (mean.rows != 0 ? 1u : 0u)), dim3(kFinishThreads), 0, stream, table,
+                       static_cast<int>(count), compute_units(), mean);
     CGPTX_LAUNCH_CHECK();
     return CGPTX_OK;
 }

@@ -17,6 +17,7 @@
 //     ahead of each replay.
 #include "cgptx_train.h"
 #include "common.hpp"
+#include "cross_entropy.hpp"
 #include "gemm.hpp"
 
 #include <charconv>
@@ -103,6 +104,9 @@ struct cgptx_model {
     void* normalized = nullptr;
     void* logits = nullptr;       // dense loss only, allocated on first use
     void* grad_logits = nullptr;
+    std::size_t grad_logits_pitch = 0;  // row length: what the classifier's gradients read as it lies
+    float* row_losses = nullptr;        // their mean is taken beside the norms' reductions
+    void* token_groups = nullptr;       // the tokens by id, made beside their lookup where they are few
     void *cos_cache = nullptr, *sin_cache = nullptr;
     std::uint32_t *tokens = nullptr, *targets = nullptr;
     float* loss = nullptr;
@@ -332,11 +336,11 @@ constexpr const char* kClassifierLabels[3] = CGPTX_GRADIENT_LABELS("classifier")
 // type one by one, passes on enlarged whatever other order of additions the layers above it take.
 int linear_gradients(cgptx_model* m, void* dx, void* dw, const void* dy, const void* x, const void* w, std::size_t rows,
                      std::size_t in_features, std::size_t out_features, int accumulate_input, int dt, hipStream_t stream,
-                     const char* const (&labels)[3]) {
+                     const char* const (&labels)[3], std::size_t grad_output_pitch = 0) {
     TimedParts timed(m, stream, labels);
     if (m->profiling) CGPTX_TRY(timed.start());
     return linear_backward(dx, dw, nullptr, dy, x, w, rows, in_features, out_features, accumulate_input, 0, 0, dt, stream,
-                           m->profiling ? &timed : nullptr, false);
+                           m->profiling ? &timed : nullptr, false, grad_output_pitch);
 }
 
 // Y = X·Wᵀ + residual (accumulate: + Y): the block's residual additions ride in the projection's
@@ -573,7 +577,7 @@ cgptx::ColumnReduceSink* norm_reduction_sink(cgptx_model* m) {
 // device copy of the table is written once, by the first pass, outside any capture. The sink's memory and the
 // table are sized when the model is created; should a pass still find the memory too small (it then reduced at
 // once, from the arena), the memory grows here and the caller repeats the pass before recording it.
-int finish_norm_reductions(cgptx_model* m, hipStream_t stream) {
+int finish_norm_reductions(cgptx_model* m, const MeanEntry& mean, hipStream_t stream) {
     auto& sink = m->norm_reductions;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (stream != nullptr) CGPTX_HIP(hipStreamIsCapturing(stream, &capture));
@@ -586,7 +590,9 @@ int finish_norm_reductions(cgptx_model* m, hipStream_t stream) {
             step.exec = nullptr;
         }
     };
-    if (!sink.entries.empty()) {
+    if (sink.entries.empty()) {
+        if (int s = run_column_reductions(nullptr, sink.entries, mean, stream)) return s;
+    } else {
         if (!(sink.entries == m->norm_reduction_uploaded)) {
             if (capturing) return fail(CGPTX_RUNTIME, "model: the table of norm reductions changed under graph capture");
             CGPTX_HIP(hipStreamSynchronize(stream));  // earlier launches may still read the table
@@ -602,7 +608,7 @@ int finish_norm_reductions(cgptx_model* m, hipStream_t stream) {
                                 hipMemcpyHostToDevice));
             m->norm_reduction_uploaded = sink.entries;
         }
-        if (int s = run_column_reductions(m->norm_reduction_table, sink.entries, stream))
+        if (int s = run_column_reductions(m->norm_reduction_table, sink.entries, mean, stream))
             return s;
     }
     m->norm_reductions_resized = false;
@@ -782,7 +788,9 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
     const bool fused_qkv = dt != CGPTX_F32 && QW % 256 == 0 && KW % 256 == 0 && H % 32 == 0;
 
     // ------------------------------------------------------------------ forward
-    CGPTX_OP("embedding_fwd", cgptx_embedding_forward(m->hidden[0], m->tokens, N, m->embedding.value, c.vocabulary_size, H, dt, s));
+    bool grouped = false;
+    CGPTX_OP("embedding_fwd", embedding_forward_and_group(m->hidden[0], m->tokens, N, m->embedding.value, c.vocabulary_size, H,
+                                                          m->token_groups, dt, stream, &grouped));
     for (std::size_t l = 0; l < c.num_layers; ++l) {
         const auto& w = m->layers[l];
         const auto& a = m->acts[l];
@@ -853,15 +861,14 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
 
     // --------------------------------------------------------- loss + classifier
     if (loss_mode == CGPTX_LOSS_CUT) {
-        CGPTX_OP("cut_ce", cgptx_cut_cross_entropy_forward_backward(m->loss, m->d_normalized, m->embedding.gradient,
-                                                           m->normalized, m->embedding.value, m->targets, N, H,
-                                                           c.vocabulary_size, loss_scale, 0, dt, s));
+        CGPTX_OP("cut_ce", cut_cross_entropy(m->row_losses, m->d_normalized, m->embedding.gradient, m->normalized, m->embedding.value,
+                                             m->targets, N, H, c.vocabulary_size, loss_scale, dt, stream));
     } else {
         CGPTX_OP("gemm_fwd.classifier", cgptx_linear_forward(m->logits, m->normalized, m->embedding.value, nullptr, N, H,
                                        c.vocabulary_size, dt, s));
-        CGPTX_OP("dense_ce", cgptx_cross_entropy_forward_backward(m->loss, m->grad_logits, m->logits, m->targets, N,
-                                                       c.vocabulary_size, loss_scale, dt, s));
-        CGPTX_TRY(linear_gradients(m, m->d_normalized, m->embedding.gradient, m->grad_logits, m->normalized, m->embedding.value, N, H, c.vocabulary_size, 0, dt, stream, kClassifierLabels));
+        CGPTX_OP("dense_ce", cross_entropy_rows(m->row_losses, m->grad_logits, m->grad_logits_pitch, m->logits, c.vocabulary_size, m->targets,
+                                                N, c.vocabulary_size, loss_scale / static_cast<float>(N), dt, stream));
+        CGPTX_TRY(linear_gradients(m, m->d_normalized, m->embedding.gradient, m->grad_logits, m->normalized, m->embedding.value, N, H, c.vocabulary_size, 0, dt, stream, kClassifierLabels, m->grad_logits_pitch));
     }
 
     // ----------------------------------------------------------------- backward
@@ -1013,8 +1020,9 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
     }
     // Tied embedding: the classifier gradient is already in place; add the lookup's gradient
     // (src/core/transformer_model.cu:375-380).
-    CGPTX_OP("embedding_bwd", cgptx_embedding_backward(m->embedding.gradient, current, m->tokens, N, c.vocabulary_size, H, 1, 1, dt, s));
-    CGPTX_OP("rmsnorm_bwd", finish_norm_reductions(m, stream));
+    CGPTX_OP("embedding_bwd", embedding_backward_grouped(m->embedding.gradient, current, m->tokens, N, c.vocabulary_size, H, 1,
+                                                         grouped ? m->token_groups : nullptr, dt, stream));
+    CGPTX_OP("rmsnorm_bwd", finish_norm_reductions(m, {m->loss, m->row_losses, static_cast<unsigned int>(N)}, stream));
     return CGPTX_OK;
 }
 
@@ -1171,6 +1179,8 @@ extern "C" int cgptx_model_create(cgptx_model** out, const cgptx_model_config* c
         CGPTX_HIP(hipMemset(m->tokens, 0, N * sizeof(std::uint32_t)));
         CGPTX_HIP(hipMemset(m->targets, 0, N * sizeof(std::uint32_t)));
         CGPTX_TRY(allocate_typed(m, &m->loss, 256));
+        CGPTX_TRY(allocate_typed(m, &m->row_losses, N * sizeof(float)));
+        CGPTX_TRY(allocate(m, &m->token_groups, embedding_groups_bytes(N, c.vocabulary_size)));
         CGPTX_HIP(hipMemset(m->loss, 0, 256));
         for (void** p : {&m->d_normalized, &m->grad_a, &m->grad_b, &m->d_norm_in, &m->d_norm_in_f})
             CGPTX_TRY(allocate(m, p, N * H * elem));
@@ -1437,9 +1447,11 @@ int run_step(cgptx_model* m, float loss_scale, int loss_mode, int use_graph, boo
     if (loss_mode != CGPTX_LOSS_DENSE && loss_mode != CGPTX_LOSS_CUT)
         return fail(CGPTX_INVALID_ARGUMENT, "model_forward_backward: unknown loss mode");
     if (loss_mode == CGPTX_LOSS_DENSE && m->logits == nullptr) {
-        const std::size_t bytes = m->rows * m->config.vocabulary_size * dtype_size(m->config.dtype);
-        if (int s = allocate(m, &m->logits, bytes)) return s;
-        if (int s = allocate(m, &m->grad_logits, bytes)) return s;
+        const std::size_t vocab = m->config.vocabulary_size, elem = dtype_size(m->config.dtype);
+        m->grad_logits_pitch = linear_backward_pitch(m->rows, m->config.hidden_size, vocab, m->config.dtype);
+        if (m->grad_logits == nullptr)
+            if (int s = allocate(m, &m->grad_logits, m->rows * m->grad_logits_pitch * elem)) return s;
+        if (int s = allocate(m, &m->logits, m->rows * vocab * elem)) return s;
     }
     if (!use_graph) return enqueue_step(m, loss_scale, loss_mode, with_optimizer, stream);
     if (stream == nullptr)

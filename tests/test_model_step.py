@@ -920,3 +920,43 @@ def test_sharing_launches_changes_no_sum(device, monkeypatch, dtype, batch, seq,
         model.close()
     for (name, a), (_, b) in zip(*results):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("batch,seq,vocab", [(1, 33, 203), (3, 100, 1000), (64, 128, 517), (64, 129, 517)])
+@pytest.mark.parametrize("use_graph", [False, True], ids=["eager", "recorded"])
+def test_launches_that_a_step_shares_give_what_the_operators_give(device, dtype, batch, seq, vocab, use_graph):
+    """The rows' losses are averaged beside the norms' reductions, up to 8192 tokens are grouped beside their lookup, and the dense
+    loss leaves an odd vocabulary's gradient in padded rows: the loss is that of the operator on the step's logits, the classifier's and
+    the table's gradient what the operators make of the step's tensors (sums of 16-bit products in another order: STOL of the scale;
+    fp32 1e-4), with ids so unlike that both kinds of segments occur."""
+    from cgpt_amd import ops
+    from cgpt_amd.model import LOSS_DENSE, Model, ModelConfig
+    from tests.util import STOL
+
+    config = ModelConfig(vocabulary_size=vocab, num_layers=2, hidden_size=128, intermediate_size=192, num_query_heads=4, num_kv_heads=2,
+                         head_dim=32, rotary_dim=32, dtype=dtype)
+    model = Model(config, batch, seq, seed=11, device=device)
+    rows, rng, stream = batch * seq, np.random.default_rng(batch + seq), torch.cuda.Stream(device=device)
+    for call in range(3 if use_graph else 1):
+        tokens = np.minimum(rng.geometric(0.02, size=(batch, seq)) - 1, vocab - 1)
+        tokens[:, ::3] = 7
+        targets = rng.integers(0, vocab, size=(batch, seq))
+        model.set_tokens(tokens, targets)
+        torch.cuda.synchronize()
+        model.forward_backward(32.0, LOSS_DENSE, use_graph=use_graph, stream=stream)
+        loss, _, _ = model.status(stream)
+        logits = model.activation("logits").view(rows, vocab)
+        normalized, d_hidden = (model.activation(name).view(rows, 128) for name in ("normalized", "grad.hidden.0"))
+        ids, wanted = (torch.from_numpy(a.reshape(-1).astype(np.int32)).to(device) for a in (tokens, targets))
+        want_loss, gradient = torch.empty(1, device=device), torch.empty_like(logits)
+        ops.cross_entropy_forward_backward(want_loss, gradient, logits, wanted, rows, gradient_scale=32.0)
+        assert loss == want_loss.item()
+        table = {name: gradient for name, _, gradient in model.parameters()}["model.embed_tokens.weight"].view(vocab, 128)
+        want = torch.empty_like(table)
+        ops.linear_backward(None, want, None, gradient, normalized, torch.zeros(vocab, 128, dtype=dtype, device=device))
+        ops.embedding_backward(want, d_hidden, ids, rows, options=ops.EmbeddingBackwardOptions(accumulate_weight=True))
+        scale = want.float().abs().max().item()
+        assert (table.float() - want.float()).abs().max().item() <= STOL[dtype] * scale
+    model.close()
