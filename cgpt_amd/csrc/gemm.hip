@@ -323,10 +323,11 @@ bool takes_narrow_tiles(const GemmArgs& g) {
            g.ldc < kMostPitch && g.ldr < kMostPitch && g.ld_addend < kMostPitch;
 }
 
-// Whether oblong tiles take a call: 16-bit storage, k-contiguous A, one sum over K, the result stored as it is or with a residual or
-// what C holds added.
+// Whether oblong tiles take a call: 16-bit storage, k-contiguous A, one sum over K, the result stored as it is, with a residual or
+// what C holds added, or (a forward product) with a bias.
 bool takes_oblong_tiles(const GemmArgs& g) {
-    return g.dtype != CGPTX_F32 && g.a_k_contiguous && g.bias == nullptr && g.addend_f32 == nullptr && !g.c_is_f32 && g.a_sums == nullptr &&
+    if (g.bias != nullptr && (!g.b_k_contiguous || g.residual != nullptr || g.accumulate)) return false;
+    return g.dtype != CGPTX_F32 && g.a_k_contiguous && g.addend_f32 == nullptr && !g.c_is_f32 && g.a_sums == nullptr &&
            g.swiglu_out == nullptr && g.swiglu_saved == nullptr && g.batch_rows == 0 && !(g.a_segments.count > 0 && (g.b_k_contiguous || g.residual != nullptr || g.accumulate)) &&
            !(g.residual != nullptr && g.accumulate) && !(g.c_segments.count > 0 && (g.residual != nullptr || g.accumulate)) && c_streams(g, 2);
 }

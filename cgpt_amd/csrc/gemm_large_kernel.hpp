@@ -496,7 +496,8 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     auto sw = [](int row) { return (row / (256 / kRowBytes)) % kRowChunks; };
     const int m_lane = lane & 15, q_lane = lane >> 4;
     // Writes blocks (r, j0 .. j0+JP-1) of kPassRows rows into the wavefront's staging region as element type S.
-    auto stage = [&]<typename S, int JP>(int r, int j0) __attribute__((always_inline)) {
+    constexpr bool kTakesBias = kOblong && A_K && B_K;
+    auto stage = [&]<typename S, int JP>(int r, int j0, const auto&... column_bias) __attribute__((always_inline)) {
         static_assert(JP * 16 * sizeof(S) == kRowBytes, "a pass fills whole staged rows");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -515,6 +516,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
                     if constexpr (!kIsF32) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(x));
                     v[e] = x;
                 }
+                ((v += vec_to_f32<T, 4>(column_bias[j0 + jj])), ...);
                 const int byte = (jj * 16 + q_lane * 4) * static_cast<int>(sizeof(S));
                 unsigned char* slot = write_row + (((byte / 16) ^ sw(row)) * 16) + byte % 16;
                 if constexpr (std::is_same_v<S, float>) *reinterpret_cast<vec_t<float, 4>*>(slot) = v;
@@ -832,7 +834,7 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
             return;
         }
         bool plain = PLAIN;
-        if constexpr (!SPLIT && !plain_apart<BM, SPLIT, RESIDUAL, SWIGLU, GRAD>) plain = stored_as_it_is(p);
+        if constexpr (!PLAIN && !SPLIT && !plain_apart<BM, SPLIT, RESIDUAL, SWIGLU, GRAD>) plain = stored_as_it_is(p);
         if constexpr (!kIsF32 && !SPLIT) if (plain) {
             // Straight-line code, no per-lane predicates or address arithmetic (with one wavefront per
             // SIMD every branch and every dependent wait is exposed): the stores go through a buffer
@@ -850,6 +852,33 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
             const int lane_row = lane / kLanesPerRow, lane_chunk = lane % kLanesPerRow;
             const int row_bytes = static_cast<int>(c_ld * static_cast<long>(sizeof(T)));
             const int voffset = lane_chunk * 8 < cols_left ? lane_row * row_bytes + lane_chunk * 16 : std::numeric_limits<int>::min();
+            if constexpr (kTakesBias) if (p.bias != nullptr) {
+                // A lane's accumulators are the same columns in every block of rows: it holds their bias, added before the rounding.
+                // Square tiles leave a bias to the general epilogue, which takes no longer (2000 x 1024 x 2048 13.3 us either way).
+                // Columns past the matrix are past the buffer's range and get zeros.
+                const __amdgpu_buffer_rsrc_t bias_rsrc = part_rsrc(p.bias, 0, sizeof(T), 1, p.n);
+                vec_t<T, 4> column_bias[TN];
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    column_bias[j] = __builtin_bit_cast(vec_t<T, 4>, __builtin_amdgcn_raw_buffer_load_b64(
+                        bias_rsrc, (w.n0 + col0 + j * 16 + q_lane * 4) * static_cast<int>(sizeof(T)), 0, 0));
+#pragma unroll
+                for (int r = 0; r < kRowBlocks; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (request) request_share(r);
+                    stage.template operator()<T, kStaged>(r, 0, column_bias);
+                    u32x4 data[kRounds];
+#pragma unroll
+                    for (int u = 0; u < kRounds; ++u) {
+                        const int row = u * kRowsPerRound + lane_row;
+                        data[u] = *reinterpret_cast<const u32x4*>(region + row * kRowBytes + ((lane_chunk ^ sw(row)) * 16));
+                    }
+#pragma unroll
+                    for (int u = 0; u < kRounds; ++u)
+                        store_chunk(data[u], rsrc, voffset, (r * kPassRows + u * kRowsPerRound) * row_bytes);
+                }
+                return;
+            }
 #pragma unroll
             for (int r = 0; r < kRowBlocks; ++r) {
                 // Accumulators leave their registers block by block: read ahead of their block they
@@ -1322,7 +1351,8 @@ int launch_narrow(const LargeCall& call, hipStream_t stream) {
 // rounds of square tiles: 5005 x 1024 is 320 tiles of 128 x 128, of which 64 CUs get two, or 80 of 256 x 256. A tile of 160 x 128 is
 // one round. A call of one round costs 6 to 9 us that are no K loop (launch, first loads, store) and then what the L2s deliver
 // (128 columns: 0.25 us a K step, 1.34 PFLOP/s over a full chip) or the matrix cores at the power limit (160 x 256: 0.44 us, 1.5 PFLOP/s). Same
-// sums in the same order as square tiles. Block of 5 x 1001 tokens, 1024 wide, forward and backward 695 -> 671 us.
+// sums in the same order as square tiles. Block of 5 x 1001 tokens, 1024 wide, forward and backward 695 -> 671 us; with a bias 5005 x 2048 x 1024
+// 28.9 -> 23.5, 3000 x 1024 x 4096 31.3 -> 26.2, 16384 x 768 x 768 25.6 -> 23.5.
 template <typename T, int BM, int BN>
 int launch_oblong_tile(const LargeCall& call, hipStream_t stream) {
     KernelArgs p = call.args;
@@ -1332,9 +1362,9 @@ int launch_oblong_tile(const LargeCall& call, hipStream_t stream) {
         p.ldr = p.ldc;
         p.accumulate = 0;
     }
-    if (call.split || !a_k || p.bias != nullptr || p.addend != nullptr || p.accumulate || p.c_f32 || p.ragged || p.act != nullptr ||
-        p.saved != nullptr || p.batch_rows > 0 || (p.residual != nullptr && p.c_seg.count > 0) || (p.a_seg.count > 0 && b_k))
-        return fail(CGPTX_RUNTIME, "gemm: oblong tiles take products that are stored as they are or with a residual");
+    if (call.split || !a_k || (p.bias != nullptr && (!b_k || p.residual != nullptr)) || p.addend != nullptr || p.accumulate || p.c_f32 ||
+        p.ragged || p.act != nullptr || p.saved != nullptr || p.batch_rows > 0 || (p.residual != nullptr && p.c_seg.count > 0) || (p.a_seg.count > 0 && b_k))
+        return fail(CGPTX_RUNTIME, "gemm: oblong tiles take products that are stored as they are, with a bias or with a residual");
     if (p.a_seg.count > 0) return launch_kernel<T, BM, BN, true, false, false, true, false, false, false, false, true>(p, 1, stream);
     if (b_k) return launch_kernel<T, BM, BN, true, true, false, false, false, false, false, false, true>(p, 1, stream);
     return launch_kernel<T, BM, BN, true, false, false, false, false, false, false, false, true>(p, 1, stream);

@@ -520,22 +520,29 @@ def test_gradients_in_k_slices_replay_from_a_graph(device, dtype):
     (12500, 1024, 1024), (13001, 1024, 4096),  # 224 x 256, one round and four
 ])
 def test_oblong_tiles_give_the_bits_of_square_ones(device, rows, k, n, dtype):
-    """Forward products with a bias of zeros run on square tiles of the general epilogue; without one, and as an input gradient,
-    on whatever the plan takes: one sum over K each, in the same order. Integers small enough that all sums are exact check both."""
+    """Results that do not start on 16 bytes run on square tiles of the general epilogue; others, with a bias or without, and as an
+    input gradient, on whatever the plan takes: one sum over K each, in the same order. Integers small enough that all sums are exact
+    check both."""
     g = torch.Generator().manual_seed(rows)
     x = torch.randint(-2, 3, (rows, k), generator=g).to(dtype).to(device)
     w = torch.randint(-1, 2, (n, k), generator=g).to(dtype).to(device)
     for scale in (1.0, 0.37):
         a, b = (x * scale).to(dtype), (w * 0.11 if scale != 1.0 else w).to(dtype)
-        plain, square, dx = (torch.full((rows, n), float("nan"), dtype=dtype, device=device) for _ in range(3))
+        plain, biased, dx = (torch.full((rows, n), float("nan"), dtype=dtype, device=device) for _ in range(3))
+        square = torch.full((rows * n + 4,), float("nan"), dtype=dtype, device=device)[4:].view(rows, n)
+        bias = torch.randint(-9, 10, (n,), generator=g).to(dtype).to(device) * scale
+        ops.linear_forward(biased, a, b, bias=bias)
+        ops.linear_forward(square, a, b, bias=bias)
+        assert torch.equal(biased, square)
         ops.linear_forward(plain, a, b)
-        ops.linear_forward(square, a, b, bias=torch.zeros(n, dtype=dtype, device=device))
+        ops.linear_forward(square, a, b)
         assert torch.equal(plain, square)
         ops.linear_backward(dx, None, None, a, torch.empty_like(dx), b.t().contiguous())
         assert torch.equal(dx, square)
         if scale == 1.0:
             exact = a.float() @ b.float().t()
             assert torch.equal(plain, exact.to(dtype))
+            assert torch.equal(biased, (exact + bias.float()).to(dtype))
             old = torch.randint(-8, 9, (rows, n), generator=g).to(dtype).to(device)
             added = old.clone()
             ops.linear_backward(added, None, None, a, torch.empty_like(dx), b.t().contiguous(),
