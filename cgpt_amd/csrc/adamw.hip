@@ -251,6 +251,11 @@ __global__ __launch_bounds__(kPrepareThreads) void adamw_prepare_kernel(const fl
                                                                        unsigned int partial_count, DeviceState* state,
                                                                        int advance_step) {
     __shared__ double stage[kPrepareThreads];
+    // What the decision needs of the state, while the partial sums are on their way (the flags are the statistics pass's, which has ended).
+    const unsigned int calls = state->calls, parity = calls & 1u;
+    const bool found = state->found_non_finite[parity] != 0u;
+    const float beta1 = state->hyper.beta1, beta2 = state->hyper.beta2, max_grad_norm = state->hyper.max_grad_norm;
+    const unsigned long long next_step = state->step + 1ull;
     // Four independent sums per thread keep four loads in flight (one block adds some 25,000 partials for the 104m
     // model); the order of the additions is fixed by the partial count alone.
     double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
@@ -263,30 +268,28 @@ __global__ __launch_bounds__(kPrepareThreads) void adamw_prepare_kernel(const fl
     }
     for (; i < partial_count; i += kPrepareThreads) s0 += static_cast<double>(partial[i]);
     stage[threadIdx.x] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    for (int stride = kPrepareThreads / 2; stride > 0; stride >>= 1) {
-        if (threadIdx.x < stride) stage[threadIdx.x] += stage[threadIdx.x + stride];
-        __syncthreads();
+    float correction1 = 1.0f, correction2 = 1.0f;
+    if (threadIdx.x < kWave) {  // not sixteen wavefronts
+        correction1 = 1.0f - powf(beta1, static_cast<float>(next_step));
+        correction2 = 1.0f - powf(beta2, static_cast<float>(next_step));
     }
+    __syncthreads();
+    if (threadIdx.x >= kWave) return;
+    const float squared = static_cast<float>(tree_sum_1024(stage));
     if (threadIdx.x != 0) return;
-    const float squared = static_cast<float>(stage[0]);
     state->squared_norm = squared;
-    const unsigned int parity = state->calls & 1u;
-    const bool found = state->found_non_finite[parity] != 0u;
     state->found_non_finite[parity ^ 1u] = 0u;  // the flag of the next call
-    state->calls += 1u;
+    state->calls = calls + 1u;
     if (found || !isfinite(squared)) {
         state->non_finite = 1u;
         state->observed_non_finite = 1u;
         return;
     }
     state->non_finite = 0u;
-    const float beta1 = state->hyper.beta1, beta2 = state->hyper.beta2, max_grad_norm = state->hyper.max_grad_norm;
     if (advance_step) {
-        const unsigned long long next_step = state->step + 1ull;
         state->step = next_step;
-        state->scalars[0] = 1.0f - powf(beta1, static_cast<float>(next_step));
-        state->scalars[1] = 1.0f - powf(beta2, static_cast<float>(next_step));
+        state->scalars[0] = correction1;
+        state->scalars[1] = correction2;
     }
     if (isinf(max_grad_norm)) {
         state->scalars[2] = 1.0f;

@@ -22,7 +22,7 @@ int cut_cross_entropy(float* row_losses, void* input_gradient, void* classifier_
 
 // (Σ row_loss) / rows by a workgroup of THREADS. 1024 partial sums of four running ones each: the order of additions is fixed by
 // the rows alone, so the result is reproducible. read: how a row's loss is read.
-constexpr int kMeanSums = 1024;
+constexpr int kMeanSums = 1024;  // what tree_sum_1024 adds up
 template <int THREADS, typename Read>
 __device__ __forceinline__ void mean_of_rows(float* __restrict__ loss, Read&& read, unsigned int rows, float inv_rows, double* stage) {
     for (unsigned int t = threadIdx.x; t < kMeanSums; t += THREADS) {
@@ -38,11 +38,9 @@ __device__ __forceinline__ void mean_of_rows(float* __restrict__ loss, Read&& re
         stage[t] = (s0 + s1) + (s2 + s3);
     }
     __syncthreads();
-    for (unsigned int stride = kMeanSums / 2; stride > 0; stride >>= 1) {
-        for (unsigned int t = threadIdx.x; t < stride; t += THREADS) stage[t] += stage[t + stride];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) loss[0] = static_cast<float>(stage[0]) * inv_rows;
+    if (threadIdx.x >= kWave) return;
+    const double sum = tree_sum_1024(stage);
+    if (threadIdx.x == 0) loss[0] = static_cast<float>(sum) * inv_rows;
 }
 
 }  // namespace cgptx

@@ -495,6 +495,22 @@ def test_cross_entropy_of_more_logits_than_the_memory_cache_gives_the_rows_of_fe
     assert only.item() == loss.item()
 
 
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 128, 129, 1023, 1024, 1025, 2049, 4096, 4097, 9001])
+def test_mean_loss_counts_every_row_once(device, rows):
+    """Rows of equal logits all have the loss that one of them has alone, and rows whose target lies outside the vocabulary have none: their
+    sum in 64 bits is exact in any order, so the mean is known to the last bit, at the edges of the tree of 1024 sums that takes it."""
+    vocab = 40
+    z = torch.full((rows, vocab), 0.5, device=device)
+    for seed in range(3):
+        keep = randint(2, (rows,), rows + seed) == 1
+        y = torch.where(keep, 7, vocab).to(torch.int32).to(device)
+        one, loss = torch.empty(1, device=device), torch.empty(1, device=device)
+        ops.cross_entropy_forward(one, z[:1], torch.full((1,), 7, dtype=torch.int32, device=device), 1)
+        ops.cross_entropy_forward(loss, z, y, rows)
+        total = np.float32(float(one.item()) * int(keep.sum()))
+        assert loss.item() == total * (np.float32(1.0) / np.float32(rows))
+
+
 @pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1003), (torch.float32, 9000), (torch.float16, 140000)], ids=["bf16", "f32", "f16"])
 @pytest.mark.parametrize("rows", [1, 2, 127, 128, 129])
 def test_mean_loss_of_few_rows_comes_from_the_rows_launch(device, dtype, vocab, rows):
