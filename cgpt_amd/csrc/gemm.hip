@@ -79,27 +79,51 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(void* __restric
     }
 }
 
-// Copies a [rows, cols] matrix to rows of `pitch` elements (whole 16-byte chunks), zeros past cols: the streamed kernels
-// read whole chunks. One chunk per thread; the source may start anywhere.
+// Copies [rows, cols] matrices to rows of `pitch` elements (whole 16-byte chunks), zeros past cols: the streamed kernels
+// read whole chunks. One chunk per thread; a source may start anywhere. Two copies, those of a product of odd K, share a launch: the first
+// first_blocks workgroups take one, the others the other.
+struct PadJob {
+    void* dst;
+    const void* src;
+    long rows, ld;
+    int cols, pitch;
+};
 template <typename E>
-__global__ __launch_bounds__(kThreads) void pad_rows_kernel(E* __restrict__ dst, const E* __restrict__ src, long rows, int cols,
-                                                            long ld, int pitch) {
+__global__ __launch_bounds__(kThreads) void pad_rows_kernel(PadJob first, PadJob second, int first_blocks) {
     constexpr int VEC = kVec128<E>;
-    const int chunks = pitch / VEC;
-    const long total = rows * chunks;
-    for (long q = static_cast<long>(blockIdx.x) * kThreads + threadIdx.x; q < total; q += static_cast<long>(gridDim.x) * kThreads) {
+    const bool other = static_cast<int>(blockIdx.x) >= first_blocks;
+    const PadJob job = other ? second : first;
+    const long block = static_cast<int>(blockIdx.x) - (other ? first_blocks : 0);
+    const long blocks = other ? static_cast<int>(gridDim.x) - first_blocks : first_blocks;
+    const E* const src = static_cast<const E*>(job.src);
+    E* const dst = static_cast<E*>(job.dst);
+    const int chunks = job.pitch / VEC;
+    const long total = job.rows * chunks;
+    for (long q = block * kThreads + threadIdx.x; q < total; q += blocks * kThreads) {
         const long row = q / chunks;
         const int col = static_cast<int>(q - row * chunks) * VEC;
-        const E* from = src + row * ld + col;
+        const E* from = src + row * job.ld + col;
         vec_t<E, VEC> v;
-        if (col + VEC <= cols) {
+        if (col + VEC <= job.cols) {
             __builtin_memcpy(&v, from, 16);
         } else {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) v[e] = col + e < cols ? from[e] : E{0};
+            for (int e = 0; e < VEC; ++e) v[e] = col + e < job.cols ? from[e] : E{0};
         }
-        store_vec<E, VEC>(dst + row * pitch + col, v);
+        store_vec<E, VEC>(dst + row * job.pitch + col, v);
     }
+}
+int launch_pad_rows(const PadJob& first, const PadJob* second, int dtype, hipStream_t stream) {
+    auto blocks_of = [&](const PadJob& job) {
+        const long chunks = job.rows * (job.pitch * static_cast<long>(dtype_size(dtype)) / 16);
+        return static_cast<int>(std::min<long>((chunks + kThreads - 1) / kThreads, static_cast<long>(compute_units()) * 16));
+    };
+    const int blocks = blocks_of(first);
+    const dim3 grid(static_cast<unsigned int>(blocks + (second != nullptr ? blocks_of(*second) : 0)));
+    auto kernel = dtype == CGPTX_F32 ? pad_rows_kernel<std::uint32_t> : pad_rows_kernel<std::uint16_t>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, first, second != nullptr ? *second : first, blocks);
+    CGPTX_LAUNCH_CHECK();
+    return CGPTX_OK;
 }
 
 // ---- fp32 matrix-core kernel for everything the streamed path does not take ----------------------
@@ -733,16 +757,22 @@ int run_padded(const GemmArgs& g, bool pad_a, bool pad_b, hipStream_t stream, bo
     *taken = held >= a_bytes + b_bytes;
     if (!*taken) return CGPTX_OK;
     auto* base = static_cast<char*>(mem);
+    // Both operands' copies in one launch, graphs of calls: bf16 16 x 1379 x 256 8.3 -> 6.5 us, 1000 x 1021 x 1024 14.1 -> 12.4.
+    PadJob jobs[2];
+    int copies = 0;
+    auto copy = [&](void* to, const void* from, bool k_contiguous, std::size_t extent, std::size_t ld, std::size_t pitch) {
+        jobs[copies++] = PadJob{to, from, static_cast<long>(k_contiguous ? extent : g.k), static_cast<long>(ld),
+                                static_cast<int>(k_contiguous ? g.k : extent), static_cast<int>(pitch)};
+    };
     if (pad_a) {
         padded.a = base;
-        const std::size_t rows = g.a_k_contiguous ? g.m : g.k, cols = g.a_k_contiguous ? g.k : g.m;
-        if (int s = pad_rows(base, g.a, rows, cols, g.lda, padded.lda, g.dtype, stream)) return s;
+        copy(base, g.a, g.a_k_contiguous, g.m, g.lda, padded.lda);
     }
     if (pad_b) {
         padded.b = base + a_bytes;
-        const std::size_t rows = g.b_k_contiguous ? g.n : g.k, cols = g.b_k_contiguous ? g.k : g.n;
-        if (int s = pad_rows(base + a_bytes, g.b, rows, cols, g.ldb, padded.ldb, g.dtype, stream)) return s;
+        copy(base + a_bytes, g.b, g.b_k_contiguous, g.n, g.ldb, padded.ldb);
     }
+    if (int s = launch_pad_rows(jobs[0], copies > 1 ? &jobs[1] : nullptr, g.dtype, stream)) return s;
     padded.no_split = true;
     padded.split_workspace = split_bytes != 0 ? base + a_bytes + b_bytes : nullptr;
     padded.split_workspace_bytes = std::min(split_bytes, held - a_bytes - b_bytes);
@@ -1162,16 +1192,8 @@ bool gemm_takes_batch(const GemmArgs& g) {
 
 int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, int dtype,
              hipStream_t stream) {
-    const std::size_t chunks = rows * (pitch * dtype_size(dtype) / 16);
-    const dim3 grid(static_cast<unsigned int>(std::min<std::size_t>((chunks + kThreads - 1) / kThreads, static_cast<std::size_t>(compute_units()) * 16)));
-    auto launch = [&]<typename E>() {
-        hipLaunchKernelGGL((pad_rows_kernel<E>), grid, dim3(kThreads), 0, stream, static_cast<E*>(dst), static_cast<const E*>(src),
-                           static_cast<long>(rows), static_cast<int>(cols), static_cast<long>(ld), static_cast<int>(pitch));
-    };
-    if (dtype == CGPTX_F32) launch.template operator()<std::uint32_t>();
-    else launch.template operator()<std::uint16_t>();
-    CGPTX_LAUNCH_CHECK();
-    return CGPTX_OK;
+    return launch_pad_rows(PadJob{dst, src, static_cast<long>(rows), static_cast<long>(ld), static_cast<int>(cols), static_cast<int>(pitch)}, nullptr,
+                           dtype, stream);
 }
 
 std::size_t gemm_split_bytes(const GemmArgs& g) { return make_plan(g).partial_bytes(g); }

@@ -550,6 +550,21 @@ def test_oblong_tiles_give_the_bits_of_square_ones(device, rows, k, n, dtype):
             assert torch.equal(added, (exact + old.float()).to(dtype))
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("rows,k,n", [(1, 7, 8), (16, 1379, 256), (300, 517, 770), (257, 65, 3), (700, 4097, 64)])
+def test_both_operands_of_odd_k_are_copied_in_one_launch(device, rows, k, n, dtype):
+    """The copy of the input and that of the weight, and the product over them (in K slices: and their sum). Operands that start
+    anywhere; integers small enough that all sums are exact."""
+    g = torch.Generator().manual_seed(rows)
+    x = torch.empty(rows * k + 1, dtype=dtype, device=device)[1:].view(rows, k)
+    x.copy_(torch.randint(-1, 2, (rows, k), generator=g))
+    w = torch.randint(-1, 2, (n, k), generator=g).to(dtype).to(device)
+    y = torch.full((rows, n), float("nan"), dtype=dtype, device=device)
+    ops.linear_forward(y, x, w)
+    assert torch.equal(y, (x.float() @ w.float().t()).to(dtype))
+    assert launches(lambda: ops.linear_forward(y, x, w)) <= 3
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("rows,fin,fout", [
     (5005, 1024, 2048), (6983, 760, 2048),   # dX on 224 x 256, dW in two and three slices; rows, columns and K end inside tiles
