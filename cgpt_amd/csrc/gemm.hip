@@ -1196,6 +1196,13 @@ int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std
                            dtype, stream);
 }
 
+int pad_rows_of_two(void* dst0, const void* src0, std::size_t rows0, void* dst1, const void* src1, std::size_t rows1, std::size_t cols,
+                    std::size_t pitch, int dtype, hipStream_t stream) {
+    const PadJob second{dst1, src1, static_cast<long>(rows1), static_cast<long>(cols), static_cast<int>(cols), static_cast<int>(pitch)};
+    return launch_pad_rows(PadJob{dst0, src0, static_cast<long>(rows0), static_cast<long>(cols), static_cast<int>(cols), static_cast<int>(pitch)}, &second,
+                           dtype, stream);
+}
+
 std::size_t gemm_split_bytes(const GemmArgs& g) { return make_plan(g).partial_bytes(g); }
 
 int gemm(const GemmArgs& g, hipStream_t stream) {

@@ -106,6 +106,9 @@ std::size_t gemm_split_bytes(const GemmArgs& args);
 // Copies [rows, cols] elements (row stride ld) to rows of `pitch` elements (whole 16-byte chunks), zeros past cols.
 int pad_rows(void* dst, const void* src, std::size_t rows, std::size_t cols, std::size_t ld, std::size_t pitch, int dtype,
              hipStream_t stream);
+// Two dense matrices of the same columns, in one launch.
+int pad_rows_of_two(void* dst0, const void* src0, std::size_t rows0, void* dst1, const void* src1, std::size_t rows1, std::size_t cols,
+                    std::size_t pitch, int dtype, hipStream_t stream);
 // Whether gemm() serves args.swiglu_out for this call (shape, layout and alignment of the fused kernel).
 bool gemm_fuses_swiglu(const GemmArgs& args);
 bool gemm_fuses_swiglu_gradient(const GemmArgs& args);

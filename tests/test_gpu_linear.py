@@ -565,6 +565,32 @@ def test_both_operands_of_odd_k_are_copied_in_one_launch(device, rows, k, n, dty
     assert launches(lambda: ops.linear_forward(y, x, w)) <= 3
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("rows,fin,fout", [(1, 9, 8), (16, 1379, 256), (33, 517, 771), (257, 65, 40), (700, 1021, 200)])
+@pytest.mark.parametrize("accumulate", [False, True], ids=["overwrite", "accumulate"])
+def test_gradients_over_odd_rows_share_a_launch(device, rows, fin, fout, accumulate, dtype):
+    """Weight and input of odd rows are copied together (an output gradient whose columns end inside a K tile in a launch of its own), and
+    both gradients and the bias's come from one launch over the copies. A result on top of the input keeps the contractions' order: the
+    weight gradient is that of what the input gradient left there. Integers small enough that all sums are exact."""
+    g = torch.Generator().manual_seed(rows + fin)
+    draw = lambda *shape: torch.randint(-1, 2, shape, generator=g).to(dtype).to(device)
+    dy, x, w = draw(rows, fout), draw(rows, fin), draw(fout, fin)
+    old = [draw(rows, fin), draw(fout, fin), draw(fout)]
+    options = ops.LinearBackwardOptions(accumulate_input=accumulate, accumulate_weight=accumulate, accumulate_bias=accumulate)
+    outputs = [t.clone() for t in old]
+    ops.linear_backward(*outputs, dy, x, w, options=options)
+    exact = [dy.float() @ w.float(), dy.float().t() @ x.float(), dy.float().sum(0)]
+    for out, before, want in zip(outputs, old, exact):
+        assert torch.equal(out, (want + before.float() if accumulate else want).to(dtype))
+    assert launches(lambda: ops.linear_backward(*outputs, dy, x, w, options=options)) <= (3 if dtype != torch.float32 else 7)
+    if not accumulate:
+        lying = x.clone()
+        ops.linear_backward(lying, outputs[1], None, dy, lying, w)
+        assert torch.equal(lying, exact[0].to(dtype))
+        want = dy.double().t() @ lying.double()
+        assert (outputs[1].double() - want).abs().max() <= 2.0 ** -7 * max(1.0, want.abs().max().item())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("rows,fin,fout", [
     (5005, 1024, 2048), (6983, 760, 2048),   # dX on 224 x 256, dW in two and three slices; rows, columns and K end inside tiles
