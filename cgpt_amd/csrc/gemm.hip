@@ -243,11 +243,14 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma_kernel(KernelArgs p, i
 // ------------------------------------------------------------------- host side
 
 // Oblong tiles run one block per CU: us before and after a block's K loop, of a further one, of a K step on an idle chip and what a
-// full one (whose clock and L2s are shared) adds. Measured as predicted_us says, K from 128 to 4096 and 0.4 to 4 rounds: within 8 per
-// cent. They are taken where they are predicted to take 5 per cent less than the best square tiles or 256 x 192 ones. [M, N] x K, us,
-// best of those and chosen: 5005 x 1024 x 1024 17.7 -> 15.7 (160 x 128), x 2048 27.4 -> 22.5; 7000 x 768 x 2048 28.2 -> 25.2 (192 x 128);
-// 5005 x 2048 x 1024 26.4 -> 23.3 (160 x 256), 10000 x 1024 x 1024 26.3 -> 22.3; 13000 x 4096 x 1024 109 -> 99 (224 x 256). Where a call's
-// square tiles fill the chip they stay: 16384 x 1024 x 1024 30.6 and 35.5 (256 x 128), 2000 x 2048 x 1024 12.0 (128 x 128) and 12.9.
+// full one (whose clock and L2s are shared) adds. Measured as predicted_us says, K from 128 to 4096: within 8 per cent where one round of
+// blocks is enough, and short by up to 20 where many rounds run at the power limit. How much less than the best square tiles or 256 x 192
+// ones they have to be predicted to take is oblong_has_to_beat's. [M, N] x K, us, operands rotated,
+// best of those and chosen: 5005 x 1024 x 1024 17.3 -> 14.6 (160 x 128), x 2048 27.4 -> 22.6; 7000 x 768 x 2048 27.9 -> 24.1 (192 x 128);
+// 5005 x 2048 x 1024 26.4 -> 22.8 (160 x 256), 10000 x 1024 x 1024 26.8 -> 22.4; 13000 x 4096 x 1024 108 -> 98 (224 x 256). Full rounds
+// of 256 x 128 gain little: 8192 x 1024 x 1024 19.1 - 20.7 and 18.6 - 20.2, its input gradient 19.6 - 20.7 and 19.3 - 20.1, 4096 x 2048 x 1024
+// 19.3 - 19.9 and 19.0 - 20.3; with a bias, which square tiles add in their general epilogue, 21.3 - 22.6 and 19.2 - 20.3. Where square
+// tiles fill the chip they stay: 16384 x 1024 x 1024 30.6 and 35.5 (256 x 128), 2000 x 2048 x 1024 12.0 (128 x 128) and 12.9.
 struct OblongCost {
     int tile;
     double first, further, step, step_full;
@@ -259,6 +262,23 @@ const OblongCost& oblong_cost(int tile) {
     for (const OblongCost& c : kOblongCosts)
         if (c.tile == tile) return c;
     return kOblongCosts[0];
+}
+// What square tiles have to be predicted to take at least for an oblong one to be taken: more where its prediction is known to be short. Of several
+// rounds of tiles of 128 columns those predicted to gain 6 per cent lost 3 (19504 x 640 x 4096 100 -> 104 us, 33416 x 640 x 2048 93.5 -> 96), those
+// predicted to gain 7 to 13 gained 2 to 8; beyond four rounds of sums longer than 512 5 to 7 per cent predicted were -2 to 0
+// (28856 x 2048 x 2048 202 -> 205, 30304 x 4096 x 768 178 -> 180) and 15 were 3 to 8. With a bias all of these gain (19105 x 640 x 4096 90.3 -> 84.6).
+double oblong_has_to_beat(int tile, double predicted, long tiles, long k_tiles, bool bias, long units) {
+    if (bias) return 1.05 * predicted;
+    if (tiles > 4 * units && k_tiles > 16) return 1.10 * predicted;
+    return (tiles > units && tile_columns(tile) == 128 ? 1.07 : 1.05) * predicted;
+}
+// What a call of 128 x 128 tiles with a CU each takes, closer than predicted_us has it where K is long: many small blocks bring in more at once
+// than few large ones. Of such calls 16 of 16 lost 2 to 10 per cent on oblong tiles (2000 x 1280 x 4096 29.0 -> 31.8, 3000 x 1024 x 4096 31.1 -> 32.8,
+// its input gradient 32.3 -> 35.3, 1552 x 1536 x 1024 11.6 -> 12.4) unless a bias is added (1670 x 1280 x 1024 13.6 -> 12.8, 3000 x
+// 1024 x 4096 32.0 -> 32.6). Within 6 per cent.
+double lone_blocks_us(long tiles, long k_tiles, bool bias, long units) {
+    const double load = static_cast<double>(tiles) / static_cast<double>(units);
+    return 5.9 + static_cast<double>(k_tiles) * (0.15 + 0.06 * load) + (bias ? 2.0 : 0.0);
 }
 
 // CGPTX_GEMM_TILE=32|64|128|192|256|160128|... pins the tile size (for experiments); anything else = automatic, and so is a size that a call's
@@ -379,7 +399,8 @@ Plan make_plan(const GemmArgs& g) {
     auto try_oblong = [&](double best) {
         for (const OblongCost& c : kOblongCosts) {
             if (pinned > 256 && c.tile != pinned) continue;
-            const double time = 1.05 * predicted_us(c.tile, tiles_of(c.tile), 1, k_tiles, 0.0, f32, true, g.b_k_contiguous, units);
+            const double time = oblong_has_to_beat(c.tile, predicted_us(c.tile, tiles_of(c.tile), 1, k_tiles, 0.0, f32, true, g.b_k_contiguous, units),
+                                                   tiles_of(c.tile), k_tiles, g.bias != nullptr, units);
             if (pinned == 0 && time >= best) continue;
             best = time;
             plan.tile = c.tile;
@@ -444,7 +465,7 @@ Plan make_plan(const GemmArgs& g) {
         }
     }
     if (takes_oblong_tiles(g) && (forced > 256 || (forced == 0 && large))) {
-        try_oblong(best);
+        try_oblong(tiles_of(128) <= units ? std::min(best, lone_blocks_us(tiles_of(128), k_tiles, g.bias != nullptr, units)) : best);
         best_slices = plan.tile > 256 ? 1 : best_slices;
     }
     set_slices(best_slices);

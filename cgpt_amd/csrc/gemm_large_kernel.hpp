@@ -1352,7 +1352,7 @@ int launch_narrow(const LargeCall& call, hipStream_t stream) {
 // one round. A call of one round costs 6 to 9 us that are no K loop (launch, first loads, store) and then what the L2s deliver
 // (128 columns: 0.25 us a K step, 1.34 PFLOP/s over a full chip) or the matrix cores at the power limit (160 x 256: 0.44 us, 1.5 PFLOP/s). Same
 // sums in the same order as square tiles. Block of 5 x 1001 tokens, 1024 wide, forward and backward 695 -> 671 us; with a bias 5005 x 2048 x 1024
-// 28.9 -> 23.5, 3000 x 1024 x 4096 31.3 -> 26.2, 16384 x 768 x 768 25.6 -> 23.5.
+// 30.6 -> 23.1, 10000 x 1024 x 1024 30.8 -> 22.7, 16384 x 768 x 768 31.2 -> 22.3.
 template <typename T, int BM, int BN>
 int launch_oblong_tile(const LargeCall& call, hipStream_t stream) {
     KernelArgs p = call.args;

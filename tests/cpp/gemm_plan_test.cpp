@@ -124,12 +124,31 @@ void check_oblong() {
                             const std::string name = name_of(g) + ": tiles of " + std::to_string(plan.tile);
                             expect((extra < 3 || (extra == 3 && kind == Kind::forward)) && dtype != CGPTX_F32 && kind != Kind::weight_gradient && plan.slices == 1, name);
                             expect(tile_rows(plan.tile) % 32 == 0 && tile_columns(plan.tile) % 128 == 0, name);
+                            expect(Plan::tiles_of(g, 128) > compute_units() || g.bias != nullptr, name + " where every square one has a CU");
                             GemmArgs square = g;  // as it was planned without them
                             square.c = address(8);
                             const Plan other = make_plan(square);
                             expect(other.slices == 1 && other.tile >= 128, name + " for " + std::to_string(other.tile) + " in " + std::to_string(other.slices));
                         }
     expect(taken > 500, std::to_string(taken) + " calls on oblong tiles");
+    // Measured (see kOblongCosts, oblong_has_to_beat, lone_blocks_us): who gains and who loses by them.
+    struct {
+        std::size_t m, n, k;
+        bool gains, gains_with_bias;
+    } const measured[] = {{5005, 1024, 1024, true, true},    {5005, 1024, 2048, true, true},    {5005, 2048, 1024, true, true},
+                          {7000, 768, 2048, true, true},     {10000, 1024, 1024, true, true},   {13000, 4096, 1024, true, true},
+                          {16384, 768, 768, true, true},     {8192, 1024, 2048, true, true},    {30304, 2048, 256, true, true},
+                          {22226, 640, 4096, true, true},    {3000, 1024, 4096, false, false},  {2000, 1280, 4096, false, false},
+                          {1552, 1536, 1024, false, true},   {1670, 1280, 1024, false, true},   {5984, 512, 4096, false, false},
+                          {19504, 640, 4096, false, true},   {33416, 640, 2048, false, true},   {28856, 2048, 2048, false, true},
+                          {30304, 4096, 768, false, true},   {16384, 1024, 1024, false, false}, {2000, 2048, 1024, false, false}};
+    for (const auto& call : measured)
+        for (const int added : {0, 1, 2}) {
+            GemmArgs g = contraction(added == 1 ? Kind::input_gradient : Kind::forward, call.m, call.n, call.k, CGPTX_BF16);
+            if (added == 2) g.bias = address();
+            const int tile = make_plan(g).tile;
+            expect((tile > 256) == (added == 2 ? call.gains_with_bias : call.gains), name_of(g) + (added == 2 ? " + bias" : "") + ": tiles of " + std::to_string(tile));
+        }
     // Both gradients of a projection: one round of workgroups, C of either in whole aligned chunks.
     int pairs_taken = 0;
     for (std::size_t rows = 500; rows <= 20000; rows += rows / 9)
