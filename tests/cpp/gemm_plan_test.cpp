@@ -149,11 +149,11 @@ void check_oblong() {
             const int tile = make_plan(g).tile;
             expect((tile > 256) == (added == 2 ? call.gains_with_bias : call.gains), name_of(g) + (added == 2 ? " + bias" : "") + ": tiles of " + std::to_string(tile));
         }
-    // Both gradients of a projection: one round of workgroups, C of either in whole aligned chunks.
+    // Both gradients of a projection: one round of workgroups on every XCD, C of either in whole aligned chunks.
     int pairs_taken = 0;
-    for (std::size_t rows = 500; rows <= 20000; rows += rows / 9)
-        for (const std::size_t in : {640, 768, 1000, 1024, 2048})
-            for (const std::size_t out : {256, 1024, 2048, 4096})
+    for (std::size_t rows = 500; rows <= 20000; rows += rows / 23)
+        for (const std::size_t in : {576, 640, 768, 1000, 1024, 1152, 1408, 2048, 2304})
+            for (const std::size_t out : {256, 1024, 1792, 2048, 2304, 2560, 3584, 4096})
                 for (const int extra : {0, 1, 2, 3, 4}) {
                     GemmArgs calls[2] = {contraction(Kind::input_gradient, rows, in, out, CGPTX_BF16), contraction(Kind::weight_gradient, out, in, rows, CGPTX_BF16)};
                     if (extra == 1) calls[0].accumulate = true;
@@ -163,8 +163,9 @@ void check_oblong() {
                     const GemmGroup plan = plan_group(calls, 2, true);
                     if (!plan.pair || plan.tile[0] <= 256) continue;
                     ++pairs_taken;
-                    const long items = Plan::tiles_of(calls[0], plan.tile[0]) + tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns) * plan.slices;
-                    expect(extra < 3 && items <= compute_units(), name_of(calls[0]) + ": " + std::to_string(items) + " workgroups for a pair");
+                    const long input = Plan::tiles_of(calls[0], plan.tile[0]), weight = tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns) * plan.slices;
+                    expect(extra < 3 && ((input + 7) / 8 + (weight + 7) / 8) * 8 <= compute_units(),
+                           name_of(calls[0]) + ": " + std::to_string(input) + " and " + std::to_string(weight) + " workgroups for a pair");
                 }
     expect(pairs_taken > 20, std::to_string(pairs_taken) + " pairs on oblong tiles");
     // Columns in segments are whole tiles of 256; an input gradient's segments along K take nothing added.
