@@ -286,12 +286,12 @@ int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient,
         if (vectors <= 2u * 512) launch_resident<T, 512, 2>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
         else if (vectors <= 8u * 512) launch_resident<T, 512, 8>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
         else if (vectors <= 16u * 512) launch_resident<T, 512, 16>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
-        else if (vectors <= 16u * 1024) launch_resident<T, 1024, 16>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
+        else if (vectors <= kMostHeldVectors) launch_resident<T, 1024, 16>(row_loss, g, z, targets, r, v, ld_logits, ld_gradient, factor, mean, stream);
         else {
             mean.counter = nullptr;
             // The streaming kernel finds each row's own 16-byte boundary; logits and gradient rows must share it.
             const bool same_phase = g == nullptr || (((reinterpret_cast<std::uintptr_t>(z) ^ reinterpret_cast<std::uintptr_t>(g)) & 15u) == 0 &&
-                                                     (ld_logits - ld_gradient) % kVec128<T> == 0);
+                                                     cross_entropy_in_vectors(vocab, ld_logits, ld_gradient, dtype));
             auto kernel = g != nullptr ? cross_entropy_row_kernel<T, true> : cross_entropy_row_kernel<T, false>;
             hipLaunchKernelGGL(kernel, dim3(r), dim3(kThreads), 0, stream, row_loss, g, z, targets, v, ld_logits, ld_gradient,
                                factor, same_phase);
@@ -300,6 +300,11 @@ int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient,
         if (mean_taken != nullptr) *mean_taken = mean.counter != nullptr;
         return CGPTX_OK;
     });
+}
+
+std::size_t cross_entropy_gradient_pitch(std::size_t rows, std::size_t hidden, std::size_t vocab, int dtype) {
+    const std::size_t pitch = linear_backward_pitch(rows, hidden, vocab, dtype);
+    return cross_entropy_in_vectors(vocab, vocab, pitch, dtype) ? pitch : vocab;
 }
 
 int mean_reduce(float* loss, const float* row_loss, std::size_t rows, hipStream_t stream) {

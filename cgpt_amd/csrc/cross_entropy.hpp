@@ -12,6 +12,18 @@ int cross_entropy_rows(float* row_loss, void* gradient, std::size_t ld_gradient,
                        const std::uint32_t* targets, std::size_t rows, std::size_t vocab, float factor, int dtype,
                        hipStream_t stream, float* loss = nullptr, bool* mean_taken = nullptr);
 
+// Rows of up to this many 16-byte vectors stay in registers between the row pass's two passes; longer ones are streamed twice.
+constexpr std::size_t kMostHeldVectors = 16 * 1024;
+// Whether the row pass accesses logits and gradient, both on 16 bytes and in rows of these lengths, by whole vectors: streamed rows only where
+// a logits' row and its gradient's lie alike within their vectors (else by elements).
+inline bool cross_entropy_in_vectors(std::size_t vocab, std::size_t ld_logits, std::size_t ld_gradient, int dtype) {
+    const std::size_t vec = 16 / dtype_size(dtype);
+    return vocab / vec <= kMostHeldVectors || (ld_logits - ld_gradient) % vec == 0;
+}
+// The row length of the gradient that a dense loss over logits in rows of `vocab` leaves for linear_backward: what that reads as it lies, but
+// where rows are streamed that of the logits (linear_backward then copies it).
+std::size_t cross_entropy_gradient_pitch(std::size_t rows, std::size_t hidden, std::size_t vocab, int dtype);
+
 // loss[0] = (Σ row_loss) / rows, summed in a fixed order.
 int mean_reduce(float* loss, const float* row_loss, std::size_t rows, hipStream_t stream);
 

@@ -868,7 +868,8 @@ int enqueue_forward_backward(cgptx_model* m, float loss_scale, int loss_mode, hi
                                        c.vocabulary_size, dt, s));
         CGPTX_OP("dense_ce", cross_entropy_rows(m->row_losses, m->grad_logits, m->grad_logits_pitch, m->logits, c.vocabulary_size, m->targets,
                                                 N, c.vocabulary_size, loss_scale / static_cast<float>(N), dt, stream));
-        CGPTX_TRY(linear_gradients(m, m->d_normalized, m->embedding.gradient, m->grad_logits, m->normalized, m->embedding.value, N, H, c.vocabulary_size, 0, dt, stream, kClassifierLabels, m->grad_logits_pitch));
+        const std::size_t pitch = m->grad_logits_pitch != c.vocabulary_size ? m->grad_logits_pitch : 0;
+        CGPTX_TRY(linear_gradients(m, m->d_normalized, m->embedding.gradient, m->grad_logits, m->normalized, m->embedding.value, N, H, c.vocabulary_size, 0, dt, stream, kClassifierLabels, pitch));
     }
 
     // ----------------------------------------------------------------- backward
@@ -1448,7 +1449,7 @@ int run_step(cgptx_model* m, float loss_scale, int loss_mode, int use_graph, boo
         return fail(CGPTX_INVALID_ARGUMENT, "model_forward_backward: unknown loss mode");
     if (loss_mode == CGPTX_LOSS_DENSE && m->logits == nullptr) {
         const std::size_t vocab = m->config.vocabulary_size, elem = dtype_size(m->config.dtype);
-        m->grad_logits_pitch = linear_backward_pitch(m->rows, m->config.hidden_size, vocab, m->config.dtype);
+        m->grad_logits_pitch = cross_entropy_gradient_pitch(m->rows, m->config.hidden_size, vocab, m->config.dtype);
         if (m->grad_logits == nullptr)
             if (int s = allocate(m, &m->grad_logits, m->rows * m->grad_logits_pitch * elem)) return s;
         if (int s = allocate(m, &m->logits, m->rows * vocab * elem)) return s;

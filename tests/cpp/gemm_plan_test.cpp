@@ -7,6 +7,7 @@
 #include <string>
 #include <vector>
 
+#include "cross_entropy.hpp"
 #include "gemm.hip"
 
 namespace {
@@ -270,6 +271,24 @@ void check_counters() {
         }
 }
 
+// The rows in which a step's dense loss leaves its gradient never take its row pass from whole vectors to elements, and are whole chunks
+// wherever that costs nothing.
+void check_loss_rows() {
+    int streamed = 0;
+    for (const int dtype : {CGPTX_F32, CGPTX_F16, CGPTX_BF16}) {
+        const std::size_t vec = 16 / dtype_size(dtype), held = kMostHeldVectors * vec;
+        for (const std::size_t vocab : {std::size_t{203}, std::size_t{50257}, held - 1, held, held + 1, held + vec - 1, held + vec, held + vec + 1, held + 3 * vec + 2, 2 * held - 1})
+            for (const std::size_t rows : {1, 33, 512}) {
+                const std::size_t pitch = cross_entropy_gradient_pitch(rows, 128, vocab, dtype);
+                const std::string name = std::to_string(rows) + " rows of " + std::to_string(vocab) + " logits of type " + std::to_string(dtype);
+                expect(cross_entropy_in_vectors(vocab, vocab, pitch, dtype), name + ": by elements, gradient in rows of " + std::to_string(pitch));
+                if (vocab / vec > kMostHeldVectors) ++streamed;
+                else expect(pitch == linear_backward_pitch(rows, 128, vocab, dtype), name + ": gradient in rows of " + std::to_string(pitch));
+            }
+    }
+    expect(streamed >= 30, std::to_string(streamed) + " streamed shapes");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -279,6 +298,7 @@ int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "oblong") == 0) check_oblong();
     if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
     if (argc > 1 && std::strcmp(argv[1], "predictions") == 0) check_predictions();
+    if (argc > 1 && std::strcmp(argv[1], "loss_rows") == 0) check_loss_rows();
     std::printf("%d failure(s)\n", failures);
     return failures == 0 ? 0 : 1;
 }

@@ -146,3 +146,9 @@ def test_predictions_that_stop_short_decide_as_whole_ones():
     """tests/cpp/gemm_plan_test.cpp: what both gradients of a projection take in one launch, predicted only as far as the answer
     can matter."""
     run_plan_test("predictions")
+
+
+def test_a_steps_dense_loss_streams_long_rows_in_vectors():
+    """tests/cpp/gemm_plan_test.cpp: the gradient of more logits than the registers hold lies in rows like the logits' own (in rows padded
+    for the contractions, an odd vocabulary's were read and written element by element)."""
+    run_plan_test("loss_rows")

@@ -960,3 +960,10 @@ def test_launches_that_a_step_shares_give_what_the_operators_give(device, dtype,
         scale = want.float().abs().max().item()
         assert (table.float() - want.float()).abs().max().item() <= STOL[dtype] * scale
     model.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 131083), (torch.float16, 131080), (torch.float32, 65541)], ids=["bf16", "f16", "f32"])
+def test_a_dense_step_over_longer_rows_than_registers_hold_gives_what_the_operators_give(device, dtype, vocab):
+    """The loss's gradient keeps rows like the logits' there, and the classifier's gradients read a copy in padded ones."""
+    test_launches_that_a_step_shares_give_what_the_operators_give(device, dtype, 1, 33, vocab, False)
