@@ -300,6 +300,7 @@ std::size_t round_up(std::size_t v, std::size_t unit) { return (v + unit - 1) / 
 // How a call of the streamed kernels is cut: tile, K slices per tile and K steps per slice.
 struct Plan {
     int tile = 256;  // see tile_rows
+    int replaced = 0;  // the tile that an oblong one took the place of
     static long tiles_of(const GemmArgs& g, int tile) {
         const std::size_t rows = tile_rows(tile), columns = tile_columns(tile);
         return static_cast<long>((g.m + rows - 1) / rows) * static_cast<long>((g.n + columns - 1) / columns);
@@ -397,6 +398,7 @@ Plan make_plan(const GemmArgs& g) {
     const int pinned = forced_tile();
     // Oblong tiles in place of plan.tile's, predicted to take `best`: the same sums in the same order.
     auto try_oblong = [&](double best) {
+        plan.replaced = plan.tile;
         for (const OblongCost& c : kOblongCosts) {
             if (pinned > 256 && c.tile != pinned) continue;
             const double time = oblong_has_to_beat(c.tile, predicted_us(c.tile, tiles_of(c.tile), 1, k_tiles, 0.0, f32, true, g.b_k_contiguous, units),
@@ -870,12 +872,26 @@ double predicted_pair_us(long tiles_x, long steps_x, long tiles_w, long steps_w,
     return time();
 }
 
-// The same with an oblong tile for the input gradient and 256 x 128 for the weight gradient, where every workgroup has a CU to itself:
-// the longer of the two. Both operands of the weight gradient are read transposed from LDS, 0.30 - 0.39 us a K step. Fitted to 16 shapes from
-// 3000 x 1024 x 4096 to 12000 x 768 x 768, six tiles and one to four slices each: within 5 per cent where one round is enough; what several
-// rounds take varies by a third with the order in which workgroups end, so those keep to 128 x 128 tiles, and so do short sums, whose
-// slices cost more to add up than the tiles save. us, 128 x 128 and chosen: 5005 x 1024 x 2048 53.4 -> 45.7, 6000 x 1024 x 2048 59.1 -> 52.0,
-// 7000 x 768 x 2048 52.0 -> 47.4, 3000 x 1024 x 4096 52.7 -> 47.8; 5005 x 1024 x 1024 30.8 and 33.6, 4096 x 768 x 2048 33.6 and 34.8.
+// What oblong pairs are held against: the same, closer, where all workgroups have a slot at once. Two that share a CU take 0.28 us a K step there
+// and not 0.47. Fitted to 2472 launches of 1298 drawn shapes, three sets of operands in turn: 2 per cent short, standard deviation 6 (predicted_pair_us
+// 9 per cent too long, 11).
+double pair_us_of_one_round(long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units) {
+    const long kt = slices > 1 ? slice_steps(steps_w, slices) : steps_w, items_w = tiles_w * slices, items = tiles_x + items_w;
+    const bool weight_first = kt >= steps_x;
+    const long longest = weight_first ? kt : steps_x, most = weight_first ? items_w : tiles_x;
+    const long beside = items <= units ? 0 : most > units ? longest : weight_first ? steps_x : kt;
+    if (items <= units && slices > 1)  // few workgroups, in short slices: they do not slow each other down
+        return 8.0 + 1.2 * static_cast<double>(slices) + static_cast<double>(longest) * (0.13 + 0.07 * static_cast<double>(items) / static_cast<double>(units));
+    const double work = static_cast<double>(tiles_x * steps_x + items_w * kt) / static_cast<double>(units);
+    return (slices > 1 ? 8.0 + 0.9 * static_cast<double>(slices) : 5.0) + 0.22 * static_cast<double>(longest - beside) + 0.28 * static_cast<double>(beside) +
+           0.05 * work;
+}
+
+// A pair with an oblong tile for the input gradient and 256 x 128 for the weight gradient, where every workgroup has a CU to itself:
+// the longer of the two, and what the shorter one takes of the L2s and the power meanwhile. Both operands of the weight gradient are read transposed
+// from LDS, 0.30 - 0.39 us a K step; adding its slices up takes some 5 us, and longer the later the input gradient's tiles let go of the memory. Fitted to
+// 6070 launches of 1510 drawn shapes: standard deviation 3 per cent in one slice, 5 in two and three. What several rounds take varies by a third with
+// the order in which workgroups end, so those keep to 128 x 128 tiles.
 double predicted_oblong_pair_us(const OblongCost& c, long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units) {
     const long items = tiles_x + tiles_w * slices;
     // Workgroups go to the XCDs in turn and each call's tiles are dealt out to them by itself: one round is one that every XCD's share of
@@ -884,10 +900,22 @@ double predicted_oblong_pair_us(const OblongCost& c, long tiles_x, long steps_x,
     if (on_an_xcd > units / kXcds) return std::numeric_limits<double>::infinity();
     const long kt = slices > 1 ? slice_steps(steps_w, slices) : steps_w;
     const double filled = static_cast<double>(items) / static_cast<double>(units);
-    const double fold = slices > 1 ? 3.6 * static_cast<double>(slices * tiles_w * slices) / static_cast<double>(units) : 0.0;
-    const double input = 4.2 + static_cast<double>(steps_x) * (1.09 * c.step + 0.565 * c.step_full * filled);
-    const double weight = 6.5 + static_cast<double>(kt) * (0.30 + 0.087 * filled) + fold;
-    return 4.5 + std::max(input, weight);
+    const double input = static_cast<double>(steps_x) * (1.09 * c.step + 0.565 * c.step_full * filled);
+    const double weight = static_cast<double>(kt) * (0.30 + 0.087 * filled);
+    const double longer = std::max(input, weight), shorter = std::min(input, weight);
+    return slices == 1 ? 7.2 + 0.93 * longer + 0.20 * shorter
+                       : 7.6 + 0.54 * static_cast<double>(slices) + 0.77 * longer + 0.30 * shorter + 15.7 * static_cast<double>(tiles_x) / static_cast<double>(units);
+}
+
+// What a pair on oblong tiles has to be predicted to take in place of one of 128 x 128 predicted at `pair_us`: 5 per cent less where all workgroups of that one
+// have a slot at once, 12 where not (predicted_pair_us is longest there just where some CUs get one more). Of 1252 drawn shapes with such a pair 294 take oblong
+// tiles, 0.90 of the time in the mean, and 5 lose 1 to 3 per cent; of 140 others 2, by 1 and 4.5. Asked for 6 per cent less than predicted_pair_us says, 114 of
+// 270 lost, up to 20. us, 128 x 128 and chosen: 5005 x 1024 x 2048 50.5 -> 46.5, 6000 x 1024 x 2048 60.0 -> 52.1, 6983 x 760 x 2048 53.3 -> 48.6, 7000 x
+// 768 x 2048 50.5 -> 48.5. That stay: 5005 x 1024 x 1024 30.4 and 31.5, 4096 x 768 x 2048 34.3 and 35.9, 2816 x 896 x 2944 36.2 and 41.7, 1615 x 1792 x
+// 1472 24.5 and 28.6, 3357 x 1024 x 2688 41.3 and 48.1; and, for want of a closer prediction, 3000 x 1024 x 4096 50.8 and 46.9.
+double oblong_pair_has_to_beat(double pair_us, long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units) {
+    if (tiles_x + tiles_w * slices > 2 * units) return pair_us / 1.12;
+    return pair_us_of_one_round(tiles_x, steps_x, tiles_w, steps_w, slices, units) / 1.05;
 }
 
 // A group's tiles: those whose predicted time in one launch is least. The launch takes as long as its longest workgroup or
@@ -914,10 +942,13 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
         const GemmArgs& g = calls[i];
         const Plan plan = make_plan(g);
         f32_group = f32_group && (count > 2 || plan.slices == 1);
-        const long tiles = Plan::tiles_of(g, plan.tile);
+        // An input gradient by itself on oblong tiles counts with those that they replace: what they promise is less than the error of a pair's
+        // prediction. Pairs given up for it lost 5 to 27 per cent (17175 x 256 x 640 31.2 -> 39.5 us, with the bias 4469 x 1728 x 2880 92 -> 114).
+        const int tile = plan.tile > 256 ? plan.replaced : plan.tile;
+        const long tiles = Plan::tiles_of(g, tile);
         const bool f32 = g.dtype == CGPTX_F32;
         const long k_step = f32 ? kBK<float> : kBK<bf16_t>, k_tiles = (static_cast<long>(g.k) + k_step - 1) / k_step;
-        separate += predicted_us(plan.tile, tiles, plan.slices, k_tiles, static_cast<double>(plan.partial_bytes(g)) * 1e-6, f32,
+        separate += predicted_us(tile, tiles, plan.slices, k_tiles, static_cast<double>(plan.partial_bytes(g)) * 1e-6, f32,
                                  g.a_k_contiguous, g.b_k_contiguous, compute_units());
         if (g.a_sums != nullptr) separate += 6.0;  // two launches of their own
     }
@@ -936,12 +967,14 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
         }
         if (takes_oblong_tiles(calls[0]) && calls[0].a_segments.count == 0 && c_streams(calls[1], 2)) {
             const long tiles = tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns);
+            double most = best_plan.pair ? oblong_pair_has_to_beat(best, tiles_x, steps_x, tiles_w, steps_w, best_plan.slices, compute_units()) : best / 1.08;
             for (const OblongCost& c : kOblongCosts)
                 for (long s = 1; s <= 3; ++s) {
                     if (s > 1 && slice_steps(steps_w, s) * (s - 1) >= steps_w) continue;
-                    const double time = 1.06 * predicted_oblong_pair_us(c, Plan::tiles_of(calls[0], c.tile), steps_x, tiles, steps_w, s, compute_units());
-                    if (time >= best) continue;
-                    best = time;
+                    const double time = predicted_oblong_pair_us(c, Plan::tiles_of(calls[0], c.tile), steps_x, tiles, steps_w, s, compute_units());
+                    if (time >= most) continue;
+                    most = time;
+                    best = std::min(best, 1.08 * time);
                     best_plan.joined = best_plan.pair = true;
                     best_plan.tile[0] = c.tile;
                     best_plan.slices = static_cast<int>(s);

@@ -177,6 +177,45 @@ void check_oblong() {
     expect(make_plan(g).tile <= 256, "segments along K, added to C");
 }
 
+// Both gradients of a projection (rows, in, out), measured in one launch: each tile and slice count of the pairs on oblong tiles at ragged shapes, those
+// that gain by them, and those that do not and keep 128 x 128 tiles.
+void check_oblong_pairs() {
+    struct {
+        std::size_t rows, in, out;
+        int tile, slices;
+    } const ragged[] = {{732, 1368, 2208, 160128, 1},  {2323, 648, 3104, 160128, 2},  {3691, 400, 2208, 160128, 3}, {779, 3960, 1184, 160256, 1},
+                        {3336, 1040, 1824, 160256, 2}, {2957, 720, 1184, 160256, 3},  {2646, 944, 2784, 192128, 1}, {3226, 600, 1632, 192128, 3},
+                        {1080, 3624, 1056, 192256, 1}, {3910, 1048, 1568, 192256, 2}, {5188, 904, 1440, 192256, 3}, {1196, 3616, 1056, 224256, 1},
+                        {3965, 1160, 1440, 224256, 2}, {4010, 1192, 1248, 224256, 3}, {3004, 792, 1184, 256128, 3}};
+    auto plan_of = [](std::size_t rows, std::size_t in, std::size_t out, int dtype, bool accumulate, bool bias) {
+        GemmArgs calls[2] = {contraction(Kind::input_gradient, rows, in, out, dtype), contraction(Kind::weight_gradient, out, in, rows, dtype)};
+        calls[0].accumulate = calls[1].accumulate = accumulate;
+        if (bias) calls[1].a_sums = address();
+        return plan_group(calls, 2, true);
+    };
+    auto named = [](std::size_t rows, std::size_t in, std::size_t out, const GemmGroup& plan) {
+        return std::to_string(rows) + " x " + std::to_string(in) + " x " + std::to_string(out) + (plan.pair ? ": pair of tile " : plan.joined ? ": group of tile " : ": apart, ") +
+               std::to_string(plan.tile[0]) + " in " + std::to_string(plan.slices);
+    };
+    for (const auto& shape : ragged)
+        for (const int dtype : {CGPTX_BF16, CGPTX_F16})
+            for (const bool accumulate : {false, true}) {
+                const GemmGroup plan = plan_of(shape.rows, shape.in, shape.out, dtype, accumulate, true);
+                expect(plan.pair && plan.tile[0] == shape.tile && plan.slices == shape.slices, named(shape.rows, shape.in, shape.out, plan));
+            }
+    struct {
+        std::size_t rows, in, out;
+        bool gains;
+    } const measured[] = {{5005, 1024, 2048, true},  {6000, 1024, 2048, true},  {6983, 760, 2048, true},   {7000, 768, 2048, true},   {3425, 1536, 3072, true},
+                          {5862, 896, 3840, true},   {5005, 1024, 1024, false}, {4096, 768, 2048, false},  {2816, 896, 2944, false},  {1615, 1792, 1472, false},
+                          {3357, 1024, 2688, false}, {6546, 384, 2944, false},  {1508, 1408, 1792, false}, {17175, 256, 640, false},
+                          {26156, 768, 1920, false}, {4978, 256, 3840, false}};
+    for (const auto& shape : measured) {
+        const GemmGroup plan = plan_of(shape.rows, shape.in, shape.out, CGPTX_BF16, false, false);
+        expect(plan.pair && (plan.tile[0] > 256) == shape.gains, named(shape.rows, shape.in, shape.out, plan));
+    }
+}
+
 // q's, k's and v's gradients over `rows` tokens as one group: their input gradients as one call in segments, then the weight gradients.
 struct Gradients {
     GemmArgs calls[4], input[3];
@@ -296,6 +335,7 @@ int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "chains") == 0) check_chains();
     if (argc > 1 && std::strcmp(argv[1], "narrow") == 0) check_narrow();
     if (argc > 1 && std::strcmp(argv[1], "oblong") == 0) check_oblong();
+    if (argc > 1 && std::strcmp(argv[1], "oblong_pairs") == 0) check_oblong_pairs();
     if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
     if (argc > 1 && std::strcmp(argv[1], "predictions") == 0) check_predictions();
     if (argc > 1 && std::strcmp(argv[1], "loss_rows") == 0) check_loss_rows();

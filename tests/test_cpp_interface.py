@@ -152,3 +152,9 @@ def test_a_steps_dense_loss_streams_long_rows_in_vectors():
     """tests/cpp/gemm_plan_test.cpp: the gradient of more logits than the registers hold lies in rows like the logits' own (in rows padded
     for the contractions, an odd vocabulary's were read and written element by element)."""
     run_plan_test("loss_rows")
+
+
+def test_pairs_on_oblong_tiles_are_those_that_gain():
+    """tests/cpp/gemm_plan_test.cpp: gradients that lost up to a fifth on oblong tiles, or apart because of them, share a launch of 128 x 128
+    ones, and the ragged shapes of tests/test_gpu_linear.py reach every tile."""
+    run_plan_test("oblong_pairs")
