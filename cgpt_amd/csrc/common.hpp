@@ -100,6 +100,12 @@ __device__ __forceinline__ float wave_sum(float v) {
     if constexpr (width >= 2) v += row_exchange<1>(v);
     return v;
 }
+// The last six levels of such a tree, of a value per lane; valid in lane 0.
+__device__ __forceinline__ double tree_sum_64(double v) {
+#pragma unroll
+    for (int offset = kWave / 2; offset > 0; offset /= 2) v += __shfl_down(v, offset, kWave);
+    return v;
+}
 // The sum of a workgroup's 1024 partial sums as a tree (t and t + 512, then t and t + 256, down to 0 and 1), for the lanes of its
 // first wavefront, which stand behind the barrier that follows the sums' stores; valid in lane 0. A barrier per level of the tree took a
 // workgroup of 1024 threads some 1.5 us; a wavefront adds the first four levels in registers and exchanges the rest: mean of the losses of
@@ -114,9 +120,7 @@ __device__ __forceinline__ double tree_sum_1024(const double* stage) {
     for (int half = kEach / 2; half > 0; half /= 2)
 #pragma unroll
         for (int k = 0; k < half; ++k) v[k] += v[k + half];
-#pragma unroll
-    for (int offset = kWave / 2; offset > 0; offset /= 2) v[0] += __shfl_down(v[0], offset, kWave);
-    return v[0];
+    return tree_sum_64(v[0]);
 }
 template <int width = kWave>
 __device__ __forceinline__ float wave_max(float v) {
@@ -318,11 +322,11 @@ __host__ __device__ constexpr unsigned int fold_share(int slice, int slices) {
     return slice == 0 ? 0u - even * static_cast<unsigned int>(slices - 1) : even;
 }
 // A thread leaves a value that the last workgroup of the launch reads, behind the L2s (each XCD has its own), and counts its
-// workgroup: true for the last one. Every workgroup calls it once, with one thread.
-__device__ __forceinline__ bool leave_and_count(float* where, float value, unsigned int* counter, unsigned int share) {
+// workgroup. Every workgroup calls it once, with one thread; the last one gets 0 - share, on which nothing waits before it is looked at.
+__device__ __forceinline__ unsigned int leave_and_count(float* where, float value, unsigned int* counter, unsigned int share) {
     __hip_atomic_store(where, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    return __hip_atomic_fetch_add(counter, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + share == 0u;
+    return __hip_atomic_fetch_add(counter, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // What leave_and_count left.
 __device__ __forceinline__ float read_left(const float* where) { return __hip_atomic_load(where, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }

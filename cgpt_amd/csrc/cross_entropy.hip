@@ -48,15 +48,17 @@ __device__ __forceinline__ MaxSum block_combine(MaxSum v, MaxSum* stage) {
     return total;
 }
 
-// The mean that the last workgroup of a row launch takes, in place of a launch that begins when all of this one has ended: bf16 [16, 1000] 9.6 -> 5.6 us,
-// [128, 2000] 9.5 -> 6.2. The workgroups meet on one counter, which takes one of them every 12 ns: [4096, 1000] would take 52 us for 12, fp32
-// [512, 50257] 24 for 22.
+// The mean that the last workgroup of a row launch takes, in place of a launch that begins when all of this one has ended: its first wavefront, which
+// looks at the counter behind the gradient's stores. bf16 [16, 900] 7.5 -> 4.6 us a call, [128, 2000] 7.5 -> 5.5. In a graph of calls, where a launch
+// takes no host time, 5.5 -> 4.7, at 64 rows 5.6 -> 5.1, at 128 5.5 -> 5.7 (with both of a lane's losses read at once; one after the other, the tree
+// of sums on all threads and the counter awaited before the gradient 6.1), [128, 50257] 13.7 -> 12.0. The workgroups meet on one counter, which takes one
+// of them every 12 ns: [4096, 1000] would take 52 us for 12, fp32 [512, 50257] 24 for 22.
 struct MeanArgs {
     float* loss;
     unsigned int* counter;  // null: no mean
     float inv_rows;
 };
-constexpr std::size_t kMostMeanRows = 128;
+constexpr std::size_t kMostMeanRows = kFewMeanRows;
 
 // Streaming kernel for rows that are too long to hold: each row is split into the elements before its first
 // 16-byte boundary (a vocabulary that is not a multiple of the vector width moves every row's start), whole 128-bit
@@ -166,8 +168,6 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
     constexpr int VEC = kVec128<T>;
     constexpr int WAVES = THREADS / kWave;
     __shared__ MaxSum stage[WAVES];
-    __shared__ double mean_stage[kMeanSums];
-    __shared__ bool last;
     const T* row = logits + blockIdx.x * ld_logits;
     const unsigned int vectors = vocab / VEC, tail = vectors * VEC + threadIdx.x;  // tail: this thread's element behind them
     const std::uint32_t target = targets[blockIdx.x];
@@ -202,11 +202,13 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
         if (tail < vocab) acc.s += __expf(held_tail - acc.m);
     }
     const MaxSum total = block_combine<WAVES>(acc, stage);
+    const unsigned int share = fold_share(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+    unsigned int counted = 0;
     if (threadIdx.x == 0) {
         float loss = 0.0f;
         if (target < vocab) loss = __logf(total.s) + total.m - target_logit;
         if (mean.counter != nullptr)  // before the gradient's stores, which it would wait for
-            last = leave_and_count(row_loss + blockIdx.x, loss, mean.counter, fold_share(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)));
+            counted = leave_and_count(row_loss + blockIdx.x, loss, mean.counter, share);
         else row_loss[blockIdx.x] = loss;
     }
     if constexpr (WithGradient) {
@@ -241,9 +243,9 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
         }
         for (std::size_t i = vocab + threadIdx.x; i < ld_gradient; i += THREADS) out[i] = from_f32<T>(0.0f);
     }
-    if (mean.counter == nullptr) return;
-    __syncthreads();
-    if (last) mean_of_rows<THREADS>(mean.loss, [row_loss](unsigned int i) { return read_left(row_loss + i); }, gridDim.x, mean.inv_rows, mean_stage);
+    if (mean.counter == nullptr || threadIdx.x >= kWave) return;
+    if (static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(counted))) + share != 0u) return;
+    mean_of_few_rows(mean.loss, [row_loss](unsigned int i) { return read_left(row_loss + i); }, gridDim.x, mean.inv_rows);
 }
 
 template <typename T, int THREADS, int SLOTS>

@@ -54,5 +54,14 @@ __device__ __forceinline__ void mean_of_rows(float* __restrict__ loss, Read&& re
     const double sum = tree_sum_1024(stage);
     if (threadIdx.x == 0) loss[0] = static_cast<float>(sum) * inv_rows;
 }
+// The same sum of at most 128 rows, by the first wavefront: the other partial sums, and so the first levels of their tree, are zeros.
+constexpr unsigned int kFewMeanRows = 2 * kWave;
+template <typename Read>
+__device__ __forceinline__ void mean_of_few_rows(float* __restrict__ loss, Read&& read, unsigned int rows, float inv_rows) {
+    const unsigned int lane = threadIdx.x, last = rows - 1;
+    const float first = read(lane < last ? lane : last), second = read(lane + kWave < last ? lane + kWave : last);  // both on their way at once
+    const double sum = tree_sum_64((lane < rows ? 0.0 + static_cast<double>(first) : 0.0) + (lane + kWave < rows ? 0.0 + static_cast<double>(second) : 0.0));
+    if (threadIdx.x == 0) loss[0] = static_cast<float>(sum) * inv_rows;
+}
 
 }  // namespace cgptx
