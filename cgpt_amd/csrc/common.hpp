@@ -211,9 +211,9 @@ struct MeanEntry {
 int run_column_reductions(const ColumnReduceEntry* table, const std::vector<ColumnReduceEntry>& entries, const MeanEntry& mean, hipStream_t stream);
 
 // The lookup of a step's tokens and, where few enough that a launch costs more than its work (*grouped), the grouping that the
-// scatter of their gradient starts from, as workgroups of the same launch. groups: embedding_groups_bytes(...) of memory that stays until
-// the scatter; given no groups the scatter makes its own.
-std::size_t embedding_groups_bytes(std::size_t token_count, std::size_t vocab);
+// scatter of their gradient starts from, as workgroups of the same launch. groups: embedding_groups_ahead_bytes(...) of memory that stays until
+// the scatter (none: 0 bytes, more tokens than that); given no groups the scatter makes its own.
+std::size_t embedding_groups_ahead_bytes(std::size_t token_count, std::size_t vocab);
 int embedding_forward_and_group(void* output, const std::uint32_t* token_ids, std::size_t token_count, const void* weight, std::size_t vocab,
                                 std::size_t hidden, void* groups, int dtype, hipStream_t stream, bool* grouped);
 int embedding_backward_grouped(void* grad_weight, const void* grad_output, const std::uint32_t* token_ids, std::size_t token_count,

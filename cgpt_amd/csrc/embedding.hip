@@ -562,35 +562,36 @@ Grouping plan_grouping(void* mem, const std::uint32_t* token_ids, std::size_t to
     return g;
 }
 
+std::size_t groups_bytes(std::size_t token_count, std::size_t vocab) { return offsets_bytes(vocab) + token_count * sizeof(unsigned int); }
+
 }  // namespace
 
-std::size_t embedding_groups_bytes(std::size_t token_count, std::size_t vocab) {
-    return offsets_bytes(vocab) + token_count * sizeof(unsigned int);
+std::size_t embedding_groups_ahead_bytes(std::size_t token_count, std::size_t vocab) {
+    // Up to the tokens whose lists leave a CU room for a second workgroup. With the mean loss taken beside the norms' reductions and the
+    // logits' gradient written in the rows that its contractions read, four launches less: 3 x 100 tokens, 5003 ids 233.3 -> 225.2 us.
+    constexpr std::size_t kMostTokens = 8192, kMostLds = 48 * 1024;
+    if (token_count == 0 || token_count > kMostTokens || vocab == 0 || vocab > static_cast<std::size_t>(std::numeric_limits<int>::max())) return 0;
+    return plan_grouping(nullptr, nullptr, token_count, vocab).lds <= kMostLds ? groups_bytes(token_count, vocab) : 0;
 }
 
 int embedding_forward_and_group(void* output, const std::uint32_t* token_ids, std::size_t token_count, const void* weight, std::size_t vocab,
                                 std::size_t hidden, void* groups, int dtype, hipStream_t stream, bool* grouped) {
     *grouped = false;
-    // Up to the tokens whose lists leave a CU room for a second workgroup. With the mean loss taken beside the norms' reductions and the
-    // logits' gradient written in the rows that its contractions read, four launches less: 3 x 100 tokens, 5003 ids 233.3 -> 225.2 us.
-    constexpr std::size_t kMostTokens = 8192, kMostLds = 48 * 1024;
-    if (groups != nullptr && valid_dtype(dtype) && output != nullptr && weight != nullptr && token_ids != nullptr && token_count != 0 &&
-        token_count <= kMostTokens && vocab != 0 && vocab <= static_cast<std::size_t>(std::numeric_limits<int>::max()) && hidden != 0) {
+    if (groups != nullptr && valid_dtype(dtype) && output != nullptr && weight != nullptr && token_ids != nullptr && hidden != 0 &&
+        embedding_groups_ahead_bytes(token_count, vocab) != 0) {
         const Grouping g = plan_grouping(groups, token_ids, token_count, vocab);
-        if (g.lds <= kMostLds) {
-            const unsigned int blocks = g.groups + (g.args.count + kGroupThreads / kWave - 1) / (kGroupThreads / kWave);
-            *grouped = true;
-            return dispatch_dtype(dtype, [&]<typename T>() -> int {
-                auto* out = static_cast<T*>(output);
-                auto* w = static_cast<const T*>(weight);
-                const bool vector_ok = hidden % kVec128<T> == 0 && is_aligned16(out) && is_aligned16(w);
-                auto kernel = vector_ok ? embedding_gather_and_group_kernel<T, true> : embedding_gather_and_group_kernel<T, false>;
-                hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kGroupThreads), g.lds, stream, g.args, g.groups, out, w,
-                                   static_cast<unsigned int>(hidden));
-                CGPTX_LAUNCH_CHECK();
-                return CGPTX_OK;
-            });
-        }
+        const unsigned int blocks = g.groups + (g.args.count + kGroupThreads / kWave - 1) / (kGroupThreads / kWave);
+        *grouped = true;
+        return dispatch_dtype(dtype, [&]<typename T>() -> int {
+            auto* out = static_cast<T*>(output);
+            auto* w = static_cast<const T*>(weight);
+            const bool vector_ok = hidden % kVec128<T> == 0 && is_aligned16(out) && is_aligned16(w);
+            auto kernel = vector_ok ? embedding_gather_and_group_kernel<T, true> : embedding_gather_and_group_kernel<T, false>;
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kGroupThreads), g.lds, stream, g.args, g.groups, out, w,
+                               static_cast<unsigned int>(hidden));
+            CGPTX_LAUNCH_CHECK();
+            return CGPTX_OK;
+        });
     }
     return cgptx_embedding_forward(output, token_ids, token_count, weight, vocab, hidden, dtype, stream);
 }
@@ -609,7 +610,7 @@ int embedding_backward_grouped(void* grad_weight, const void* grad_output, const
     const auto v = static_cast<unsigned int>(vocab);
     void* mem = groups;
     if (groups == nullptr)
-        if (int s = scratch(stream, embedding_groups_bytes(token_count, vocab), &mem)) return s;
+        if (int s = scratch(stream, groups_bytes(token_count, vocab), &mem)) return s;
     const Grouping g = plan_grouping(mem, token_ids, token_count, vocab);
     unsigned int *const offsets = g.args.offsets, *const order = g.args.order;
     const unsigned int ids_per_group = g.args.ids_per_group;

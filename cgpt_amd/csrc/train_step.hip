@@ -106,7 +106,7 @@ struct cgptx_model {
     void* grad_logits = nullptr;
     std::size_t grad_logits_pitch = 0;  // row length: what the classifier's gradients read as it lies
     float* row_losses = nullptr;        // their mean is taken beside the norms' reductions
-    void* token_groups = nullptr;       // the tokens by id, made beside their lookup where they are few
+    void* token_groups = nullptr;       // the tokens by id, made beside their lookup; null where they are many
     void *cos_cache = nullptr, *sin_cache = nullptr;
     std::uint32_t *tokens = nullptr, *targets = nullptr;
     float* loss = nullptr;
@@ -1181,7 +1181,7 @@ extern "C" int cgptx_model_create(cgptx_model** out, const cgptx_model_config* c
         CGPTX_HIP(hipMemset(m->targets, 0, N * sizeof(std::uint32_t)));
         CGPTX_TRY(allocate_typed(m, &m->loss, 256));
         CGPTX_TRY(allocate_typed(m, &m->row_losses, N * sizeof(float)));
-        CGPTX_TRY(allocate(m, &m->token_groups, embedding_groups_bytes(N, c.vocabulary_size)));
+        if (const std::size_t bytes = embedding_groups_ahead_bytes(N, c.vocabulary_size); bytes != 0) CGPTX_TRY(allocate(m, &m->token_groups, bytes));
         CGPTX_HIP(hipMemset(m->loss, 0, 256));
         for (void** p : {&m->d_normalized, &m->grad_a, &m->grad_b, &m->d_norm_in, &m->d_norm_in_f})
             CGPTX_TRY(allocate(m, p, N * H * elem));

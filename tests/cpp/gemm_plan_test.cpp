@@ -216,6 +216,18 @@ void check_oblong_pairs() {
     }
 }
 
+// A step holds memory for its tokens by id where they are grouped beside their lookup: up to 8192 tokens.
+void check_token_groups() {
+    for (const std::size_t vocab : {std::size_t{1}, std::size_t{517}, std::size_t{50257}, std::size_t{1} << 20})
+        for (const std::size_t tokens : {1, 300, 4096, 8191, 8192, 8193, 32768, 1 << 20}) {
+            const std::size_t bytes = embedding_groups_ahead_bytes(tokens, vocab), all = (vocab + 1 + tokens) * sizeof(unsigned int);
+            expect(tokens <= 8192 ? bytes == 0 || (bytes >= all && bytes < all + 256) : bytes == 0,
+                   std::to_string(tokens) + " tokens of " + std::to_string(vocab) + " ids: " + std::to_string(bytes) + " bytes");
+            expect(tokens > 4096 || vocab > 50257 || bytes != 0, std::to_string(tokens) + " tokens of " + std::to_string(vocab) + " ids are not grouped ahead");
+        }
+    expect(embedding_groups_ahead_bytes(0, 100) == 0 && embedding_groups_ahead_bytes(100, 0) == 0 && embedding_groups_ahead_bytes(100, std::size_t{1} << 31) == 0, "no such step");
+}
+
 // q's, k's and v's gradients over `rows` tokens as one group: their input gradients as one call in segments, then the weight gradients.
 struct Gradients {
     GemmArgs calls[4], input[3];
@@ -338,6 +350,7 @@ int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "oblong_pairs") == 0) check_oblong_pairs();
     if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
     if (argc > 1 && std::strcmp(argv[1], "predictions") == 0) check_predictions();
+    if (argc > 1 && std::strcmp(argv[1], "token_groups") == 0) check_token_groups();
     if (argc > 1 && std::strcmp(argv[1], "loss_rows") == 0) check_loss_rows();
     std::printf("%d failure(s)\n", failures);
     return failures == 0 ? 0 : 1;

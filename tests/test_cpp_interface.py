@@ -158,3 +158,8 @@ def test_pairs_on_oblong_tiles_are_those_that_gain():
     """tests/cpp/gemm_plan_test.cpp: gradients that lost up to a fifth on oblong tiles, or apart because of them, share a launch of 128 x 128
     ones, and the ragged shapes of tests/test_gpu_linear.py reach every tile."""
     run_plan_test("oblong_pairs")
+
+
+def test_a_step_of_many_tokens_holds_no_memory_for_their_groups():
+    """tests/cpp/gemm_plan_test.cpp: a step's tokens by id have memory of their own only where they are grouped beside their lookup."""
+    run_plan_test("token_groups")
