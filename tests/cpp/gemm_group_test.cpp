@@ -378,6 +378,104 @@ void check_narrow_epilogue(int dtype, hipStream_t stream) {
     }
 }
 
+// What oblong tiles take beside plain products, ragged both ways and along K: an input gradient whose operand comes from three buffers, a forward
+// product into three, and a residual that is not C. The shapes' tiles are held by gemm_plan_test.cpp. Some rows are compared, and all guards.
+void check_oblong_forms(std::size_t rows, std::size_t columns, std::size_t k, int dtype, hipStream_t stream) {
+    const std::string name = "oblong tiles, " + std::to_string(rows) + " x " + std::to_string(columns) + " x " + std::to_string(k) + (dtype == CGPTX_F16 ? " f16" : " bf16");
+    std::printf("%s\n", name.c_str());
+    std::fflush(stdout);
+    std::mt19937 rng(static_cast<unsigned int>(rows + k));
+    std::vector<std::size_t> some;
+    for (std::size_t r = 0; r < rows; r += 997) some.push_back(r);
+    for (std::size_t r = rows - 3; r < rows; ++r) some.push_back(r);
+    auto expect_rows = [&](const Bits& got, std::size_t width, const Bits& want, std::size_t want_width, std::size_t first, const char* what) {
+        for (std::size_t i = 0; i < some.size(); ++i)
+            expect(std::memcmp(&got[some[i] * width], &want[i * want_width + first], width * 2) == 0, name + ", " + what + ": row " + std::to_string(some[i]));
+    };
+    auto launch = [&](const GemmArgs& g, const char* what) {
+        expect(cgptx::gemm(g, stream) == CGPTX_OK, name + ", " + what + ": launch");
+        hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    };
+    {
+        const std::size_t n = columns - 8, width[3] = {k / 2, k / 4, k / 4}, first[3] = {0, k / 2, k / 4 * 3};
+        const Matrix w = random_matrix(k, n, rng), dy[3] = {random_matrix(rows, width[0], rng), random_matrix(rows, width[1], rng), random_matrix(rows, width[2], rng)};
+        const Buffer on_w(w, dtype), on_dq(dy[0], dtype), on_dk(dy[1], dtype), on_dv(dy[2], dtype);
+        const Buffer* on_dy[3] = {&on_dq, &on_dk, &on_dv};
+        Buffer dx(rows * n);
+        GemmArgs g;
+        g.b = on_w.data();
+        g.c = dx.data();
+        g.m = rows;
+        g.n = g.ldb = g.ldc = n;
+        g.k = k;
+        g.b_k_contiguous = false;
+        g.dtype = dtype;
+        g.a_segments.count = 3;
+        for (int i = 0; i < 3; ++i) {
+            g.a_segments.ptr[i] = on_dy[i]->data();
+            g.a_segments.ld[i] = g.a_segments.cols[i] = width[i];
+        }
+        launch(g, "three operands");
+        const Bits want = product(some.size(), n, k, dtype, [&](std::size_t i, std::size_t t) {
+            const int s = t < first[1] ? 0 : t < first[2] ? 1 : 2;
+            return dy[s].at(some[i], t - first[s]);
+        }, [&](std::size_t t, std::size_t j) { return w.at(t, j); });
+        Bits got;
+        expect(dx.copy(got), name + ", three operands: guards");
+        expect_rows(got, n, want, n, 0, "three operands");
+    }
+    const std::size_t short_k = k - 32;  // ends inside a K tile
+    const Matrix x = random_matrix(rows, short_k, rng), w = random_matrix(columns, short_k, rng);
+    const Buffer on_x(x, dtype), on_w(w, dtype);
+    GemmArgs forward;
+    forward.a = on_x.data();
+    forward.b = on_w.data();
+    forward.m = rows;
+    forward.k = forward.lda = forward.ldb = short_k;
+    forward.dtype = dtype;
+    const Bits want = product(some.size(), columns, short_k, dtype, [&](std::size_t i, std::size_t t) { return x.at(some[i], t); },
+                              [&](std::size_t t, std::size_t j) { return w.at(j, t); });
+    {
+        const std::size_t q = columns - 512;
+        Buffer y_q(rows * q), y_k(rows * 256), y_v(rows * 256);
+        Buffer* const y[3] = {&y_q, &y_k, &y_v};
+        const std::size_t width[3] = {q, 256, 256}, first[3] = {0, q, q + 256};
+        GemmArgs g = forward;
+        g.n = columns;
+        g.c_segments.count = 3;
+        for (int i = 0; i < 3; ++i) {
+            g.c_segments.ptr[i] = y[i]->data();
+            g.c_segments.ld[i] = g.c_segments.cols[i] = width[i];
+        }
+        launch(g, "three results");
+        for (int i = 0; i < 3; ++i) {
+            Bits got;
+            expect(y[i]->copy(got), name + ", three results: guards");
+            expect_rows(got, width[i], want, columns, first[i], "three results");
+        }
+    }
+    {
+        const std::size_t n = columns - 8;
+        const Matrix residual = random_matrix(rows, n, rng);
+        const Buffer on_residual(residual, dtype);
+        Buffer y(rows * n);
+        GemmArgs g = forward;
+        g.n = g.ldc = g.ldr = n;
+        g.c = y.data();
+        g.residual = on_residual.data();
+        launch(g, "residual");
+        Bits got, sum(some.size() * n);
+        expect(y.copy(got), name + ", residual: guards");
+        for (std::size_t i = 0; i < some.size(); ++i)
+            for (std::size_t j = 0; j < n; ++j) {
+                int exact = residual.at(some[i], j);
+                for (std::size_t t = 0; t < short_k; ++t) exact += x.at(some[i], t) * w.at(j, t);
+                sum[i * n + j] = rounded(exact, dtype);
+            }
+        expect_rows(got, n, sum, n, 0, "residual");
+    }
+}
+
 }  // namespace
 
 int main() {
@@ -392,6 +490,12 @@ int main() {
             check(300, 512, 512, 64, 224, dtype, stream);   // more rows than one tile of either size
             check_many_rows(16300, 760, 1024, 512, 512, dtype, stream);
             check_narrow_epilogue(dtype, stream);
+            check_oblong_forms(5003, 1024, 1024, dtype, stream);   // 160 x 128
+            check_oblong_forms(6999, 768, 2048, dtype, stream);    // 192 x 128
+            check_oblong_forms(8161, 1024, 4096, dtype, stream);   // 256 x 128
+            check_oblong_forms(9999, 1024, 1024, dtype, stream);   // 160 x 256
+            check_oblong_forms(11871, 1024, 1024, dtype, stream);  // 192 x 256
+            check_oblong_forms(12470, 1024, 1024, dtype, stream);  // 224 x 256
         }
         check_segment_sums(300, 512, 512, 512, stream);
         check_segment_sums(131, 768, 768, 256, stream);

@@ -150,11 +150,11 @@ void check_oblong() {
             const int tile = make_plan(g).tile;
             expect((tile > 256) == (added == 2 ? call.gains_with_bias : call.gains), name_of(g) + (added == 2 ? " + bias" : "") + ": tiles of " + std::to_string(tile));
         }
-    // Both gradients of a projection: one round of workgroups on every XCD, C of either in whole aligned chunks.
+    // Both gradients of a projection: one round of workgroups, C of either in whole aligned chunks.
     int pairs_taken = 0;
-    for (std::size_t rows = 500; rows <= 20000; rows += rows / 23)
-        for (const std::size_t in : {576, 640, 768, 1000, 1024, 1152, 1408, 2048, 2304})
-            for (const std::size_t out : {256, 1024, 1792, 2048, 2304, 2560, 3584, 4096})
+    for (std::size_t rows = 500; rows <= 20000; rows += rows / 9)
+        for (const std::size_t in : {640, 768, 1000, 1024, 2048})
+            for (const std::size_t out : {256, 1024, 2048, 4096})
                 for (const int extra : {0, 1, 2, 3, 4}) {
                     GemmArgs calls[2] = {contraction(Kind::input_gradient, rows, in, out, CGPTX_BF16), contraction(Kind::weight_gradient, out, in, rows, CGPTX_BF16)};
                     if (extra == 1) calls[0].accumulate = true;
@@ -164,17 +164,76 @@ void check_oblong() {
                     const GemmGroup plan = plan_group(calls, 2, true);
                     if (!plan.pair || plan.tile[0] <= 256) continue;
                     ++pairs_taken;
-                    const long input = Plan::tiles_of(calls[0], plan.tile[0]), weight = tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns) * plan.slices;
-                    expect(extra < 3 && ((input + 7) / 8 + (weight + 7) / 8) * 8 <= compute_units(),
-                           name_of(calls[0]) + ": " + std::to_string(input) + " and " + std::to_string(weight) + " workgroups for a pair");
+                    const long items = Plan::tiles_of(calls[0], plan.tile[0]) + tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns) * plan.slices;
+                    expect(extra < 3 && items <= compute_units(), name_of(calls[0]) + ": " + std::to_string(items) + " workgroups for a pair");
                 }
     expect(pairs_taken > 20, std::to_string(pairs_taken) + " pairs on oblong tiles");
+    // One on every XCD: either call's tiles are dealt out by themselves.
+    for (std::size_t rows = 500; rows <= 20000; rows += rows / 23)
+        for (const std::size_t in : {576, 640, 768, 1000, 1024, 1152, 1408, 2048, 2304})
+            for (const std::size_t out : {256, 1024, 1792, 2048, 2304, 2560, 3584, 4096}) {
+                const GemmArgs calls[2] = {contraction(Kind::input_gradient, rows, in, out, CGPTX_BF16), contraction(Kind::weight_gradient, out, in, rows, CGPTX_BF16)};
+                const GemmGroup plan = plan_group(calls, 2, true);
+                if (!plan.pair || plan.tile[0] <= 256) continue;
+                const long input = Plan::tiles_of(calls[0], plan.tile[0]), weight = tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns) * plan.slices;
+                expect(((input + 7) / 8 + (weight + 7) / 8) * 8 <= compute_units(),
+                       name_of(calls[0]) + ": " + std::to_string(input) + " and " + std::to_string(weight) + " workgroups for a pair");
+            }
     // Columns in segments are whole tiles of 256; an input gradient's segments along K take nothing added.
     GemmArgs g = contraction(Kind::input_gradient, 5005, 1024, 1536, CGPTX_BF16);
     g.a_segments.count = 3;
     expect(make_plan(g).tile > 256, "segments along K");
     g.accumulate = true;
     expect(make_plan(g).tile <= 256, "segments along K, added to C");
+}
+
+// The tiles that tests of values are there for: tests/test_gpu_linear.py's products (forward, with a bias, as an input gradient, added to C) and
+// gemm_group_test.cpp's (an operand or a result in three buffers, a residual).
+void check_oblong_shapes() {
+    struct Shape {
+        std::size_t rows, k, n;
+        int tile;
+    };
+    auto expect_tile = [](const GemmArgs& g, int tile, const char* what) {
+        const int taken = make_plan(g).tile;
+        expect(taken == tile, name_of(g) + ", " + what + ": tiles of " + std::to_string(taken));
+    };
+    for (const int dtype : {CGPTX_BF16, CGPTX_F16}) {
+        for (const Shape& s : {Shape{5005, 1024, 1024, 160128}, {4833, 992, 1000, 160128}, {7000, 2048, 768, 192128}, {8999, 1728, 640, 192128}, {8161, 4096, 1024, 256128},
+                               {5005, 1024, 2048, 160256}, {10000, 1024, 1016, 160256}, {11900, 1024, 1024, 192256}, {11871, 992, 1016, 192256}, {12500, 1024, 1024, 224256},
+                               {13001, 1024, 4096, 224256}}) {
+            GemmArgs g = contraction(Kind::forward, s.rows, s.n, s.k, dtype);
+            expect_tile(g, s.tile, "forward");
+            g.bias = address();
+            expect_tile(g, s.tile, "bias");
+            g = contraction(Kind::input_gradient, s.rows, s.n, s.k, dtype);
+            expect_tile(g, s.tile, "input gradient");
+            g.accumulate = true;
+            expect_tile(g, s.tile, "added");
+        }
+        for (const Shape& s : {Shape{5003, 1024, 1024, 160128}, {6999, 2048, 768, 192128}, {8161, 4096, 1024, 256128}, {9999, 1024, 1024, 160256}, {11871, 1024, 1024, 192256},
+                               {12470, 1024, 1024, 224256}}) {
+            GemmArgs g = contraction(Kind::input_gradient, s.rows, s.n - 8, s.k, dtype);
+            g.a = nullptr;
+            g.a_segments.count = 3;
+            for (int i = 0; i < 3; ++i) {
+                g.a_segments.ptr[i] = address();
+                g.a_segments.ld[i] = g.a_segments.cols[i] = i == 0 ? s.k / 2 : s.k / 4;
+            }
+            expect_tile(g, s.tile, "three operands");
+            g = contraction(Kind::forward, s.rows, s.n, s.k - 32, dtype);
+            g.c_segments.count = 3;
+            for (int i = 0; i < 3; ++i) {
+                g.c_segments.ptr[i] = address();
+                g.c_segments.ld[i] = g.c_segments.cols[i] = i == 0 ? s.n - 512 : 256;
+            }
+            expect_tile(g, s.tile, "three results");
+            g = contraction(Kind::forward, s.rows, s.n - 8, s.k - 32, dtype);
+            g.residual = address();
+            g.ldr = s.n - 8;
+            expect_tile(g, s.tile, "residual");
+        }
+    }
 }
 
 // Both gradients of a projection (rows, in, out), measured in one launch: each tile and slice count of the pairs on oblong tiles at ragged shapes, those
@@ -350,6 +409,7 @@ int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "oblong_pairs") == 0) check_oblong_pairs();
     if (argc > 1 && std::strcmp(argv[1], "counters") == 0) check_counters();
     if (argc > 1 && std::strcmp(argv[1], "predictions") == 0) check_predictions();
+    if (argc > 1 && std::strcmp(argv[1], "oblong_shapes") == 0) check_oblong_shapes();
     if (argc > 1 && std::strcmp(argv[1], "token_groups") == 0) check_token_groups();
     if (argc > 1 && std::strcmp(argv[1], "loss_rows") == 0) check_loss_rows();
     std::printf("%d failure(s)\n", failures);

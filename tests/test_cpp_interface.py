@@ -163,3 +163,9 @@ def test_pairs_on_oblong_tiles_are_those_that_gain():
 def test_a_step_of_many_tokens_holds_no_memory_for_their_groups():
     """tests/cpp/gemm_plan_test.cpp: a step's tokens by id have memory of their own only where they are grouped beside their lookup."""
     run_plan_test("token_groups")
+
+
+def test_shapes_that_are_there_for_oblong_tiles_reach_them():
+    """tests/cpp/gemm_plan_test.cpp: the shapes whose values tests/test_gpu_linear.py and tests/cpp/gemm_group_test.cpp check on oblong tiles are
+    planned for those tiles (11871 x 352 x 1024, once meant for 192 x 256, is not)."""
+    run_plan_test("oblong_shapes")

@@ -550,3 +550,30 @@ def test_mean_loss_of_few_rows_comes_from_the_rows_launch(device, dtype, vocab, 
         assert abs(seen.pop() - want) <= 2e-6 * max(1.0, abs(want))
     long_rows = vocab > 131072 and dtype != torch.float32
     assert launches(lambda: ops.cross_entropy_forward(loss, z, y, rows)) == (1 if rows <= 128 and not long_rows else 2)
+
+
+@pytest.mark.parametrize("dtype,rows,vocab", [(torch.bfloat16, 3011, 50257), (torch.float16, 1201, 131071), (torch.float32, 4721, 16381)],
+                         ids=["bf16", "f16", "f32"])
+def test_cross_entropy_without_a_gradient_or_in_place_over_the_memory_cache(device, dtype, rows, vocab):
+    """More than 288 MiB of logits alone: the loss without a gradient, and with the gradient in the logits' own place, are those of calls over
+    few rows, which access them otherwise."""
+    assert rows * vocab * dtype.itemsize > 288 << 20
+    generator = torch.Generator(device=device).manual_seed(6)
+    logits = torch.randn(rows, vocab, device=device, generator=generator).to(dtype)
+    targets = torch.randint(0, vocab, (rows,), device=device, generator=generator, dtype=torch.int32)
+    loss, total = torch.empty(1, device=device), 0.0
+    want = torch.empty_like(logits)
+    for first in range(0, rows, 300):
+        part = slice(first, min(first + 300, rows))
+        few = part.stop - part.start
+        ops.cross_entropy_forward_backward(loss, want[part], logits[part], targets[part].contiguous(), few, gradient_scale=float(few))
+        only = torch.empty(1, device=device)
+        ops.cross_entropy_forward(only, logits[part], targets[part].contiguous(), few)
+        assert only.item() == loss.item()
+        total += loss.item() * few
+    ops.cross_entropy_forward(loss, logits, targets, rows)
+    assert abs(loss.item() - total / rows) <= 1e-6 * abs(loss.item())
+    in_place = torch.empty(1, device=device)
+    ops.cross_entropy_forward_backward(in_place, logits, logits, targets, rows, gradient_scale=float(rows))
+    assert in_place.item() == loss.item()
+    assert torch.equal(logits, want)

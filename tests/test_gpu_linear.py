@@ -614,3 +614,9 @@ def test_both_gradients_on_oblong_tiles_share_a_launch(device, rows, fin, fout, 
 def test_both_gradients_on_every_oblong_tile(device, rows, fin, fout, accumulate, dtype):
     """Rows, columns and K end inside tiles."""
     test_both_gradients_on_large_tiles_share_a_launch(device, rows, fin, fout, accumulate, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_oblong_tiles_of_192_x_256_end_anywhere(device, dtype):
+    """Rows, columns and K end inside tiles."""
+    test_oblong_tiles_give_the_bits_of_square_ones(device, 11871, 992, 1016, dtype)
