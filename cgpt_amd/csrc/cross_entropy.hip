@@ -202,13 +202,12 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
         if (tail < vocab) acc.s += __expf(held_tail - acc.m);
     }
     const MaxSum total = block_combine<WAVES>(acc, stage);
-    const unsigned int share = fold_share(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
     unsigned int counted = 0;
     if (threadIdx.x == 0) {
         float loss = 0.0f;
         if (target < vocab) loss = __logf(total.s) + total.m - target_logit;
         if (mean.counter != nullptr)  // before the gradient's stores, which it would wait for
-            counted = leave_and_count(row_loss + blockIdx.x, loss, mean.counter, share);
+            counted = leave_and_count(row_loss + blockIdx.x, loss, mean.counter, fold_share(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)));
         else row_loss[blockIdx.x] = loss;
     }
     if constexpr (WithGradient) {
@@ -244,7 +243,8 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_row_resident_kernel(
         for (std::size_t i = vocab + threadIdx.x; i < ld_gradient; i += THREADS) out[i] = from_f32<T>(0.0f);
     }
     if (mean.counter == nullptr || threadIdx.x >= kWave) return;
-    if (static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(counted))) + share != 0u) return;
+    counted = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(counted)));
+    if (counted + fold_share(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) != 0u) return;
     mean_of_few_rows(mean.loss, [row_loss](unsigned int i) { return read_left(row_loss + i); }, gridDim.x, mean.inv_rows);
 }
 
