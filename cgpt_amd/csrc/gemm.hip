@@ -909,8 +909,8 @@ double predicted_oblong_pair_us(const OblongCost& c, long tiles_x, long steps_x,
 
 // What a pair on oblong tiles has to be predicted to take in place of one of 128 x 128 predicted at `pair_us`: 5 per cent less where all workgroups of that one
 // have a slot at once, 12 where not (predicted_pair_us is longest there just where some CUs get one more). Of 1252 drawn shapes with such a pair 294 take oblong
-// tiles, 0.90 of the time in the mean, and 5 lose 1 to 3 per cent; of 140 others 2, by 1 and 4.5. Asked for 6 per cent less than predicted_pair_us says, 114 of
-// 270 lost, up to 20. us, 128 x 128 and chosen: 5005 x 1024 x 2048 50.5 -> 46.5, 6000 x 1024 x 2048 60.0 -> 52.1, 6983 x 760 x 2048 53.3 -> 48.6, 7000 x
+// tiles, 0.90 of the time in the mean, and 5 lose 1 to 3 per cent; of 140 others 2, by 2 and 4. Asked for 6 per cent less than predicted_pair_us says, 114 of
+// 270 lost, up to 20. us, 128 x 128 and chosen: 5005 x 1024 x 2048 50.5 -> 46.2, 6000 x 1024 x 2048 60.0 -> 52.1, 6983 x 760 x 2048 53.3 -> 48.6, 7000 x
 // 768 x 2048 50.5 -> 48.5. That stay: 5005 x 1024 x 1024 30.4 and 31.5, 4096 x 768 x 2048 34.3 and 35.9, 2816 x 896 x 2944 36.2 and 41.7, 1615 x 1792 x
 // 1472 24.5 and 28.6, 3357 x 1024 x 2688 41.3 and 48.1; and, for want of a closer prediction, 3000 x 1024 x 4096 50.8 and 46.9.
 double oblong_pair_has_to_beat(double pair_us, long tiles_x, long steps_x, long tiles_w, long steps_w, long slices, long units) {
@@ -967,18 +967,23 @@ GemmGroup plan_group(const GemmArgs* calls, int count, bool pair) {
         }
         if (takes_oblong_tiles(calls[0]) && calls[0].a_segments.count == 0 && c_streams(calls[1], 2)) {
             const long tiles = tiles_of_size(calls[1], kPairWeightRows, kPairWeightColumns);
-            double most = best_plan.pair ? oblong_pair_has_to_beat(best, tiles_x, steps_x, tiles_w, steps_w, best_plan.slices, compute_units()) : best / 1.08;
-            for (const OblongCost& c : kOblongCosts)
+            const double most = best_plan.pair ? oblong_pair_has_to_beat(best, tiles_x, steps_x, tiles_w, steps_w, best_plan.slices, compute_units()) : best / 1.08;
+            double least = most;
+            for (const OblongCost& c : kOblongCosts) {
+                // Of two that are predicted within 2 per cent the larger one: 5005 x 1024 x 2048 47.1 us on 192 x 256, 46.2 on 224 x 256.
+                double own = std::min(most, 1.02 * least);
                 for (long s = 1; s <= 3; ++s) {
                     if (s > 1 && slice_steps(steps_w, s) * (s - 1) >= steps_w) continue;
                     const double time = predicted_oblong_pair_us(c, Plan::tiles_of(calls[0], c.tile), steps_x, tiles, steps_w, s, compute_units());
-                    if (time >= most) continue;
-                    most = time;
+                    if (time >= own) continue;
+                    own = time;
+                    least = std::min(least, time);
                     best = std::min(best, 1.08 * time);
                     best_plan.joined = best_plan.pair = true;
                     best_plan.tile[0] = c.tile;
                     best_plan.slices = static_cast<int>(s);
                 }
+            }
         }
     }
     if (fewest > kGroupBlocksPerUnit * units) return best_plan;

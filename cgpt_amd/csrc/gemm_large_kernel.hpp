@@ -477,12 +477,12 @@ __device__ __forceinline__ void contract(const KernelArgs& p, int item, const in
     // Epilogue staging. acc[i][j][e] holds C[m, n] with m = lane%16, n = 4*(lane/16) + e, relative
     // to the 16 x 16 block (i, j) of the wavefront's WM x WN part of the tile. Each wavefront passes
     // its part through a private part of A's last LDS slot (the only one the first K tiles of
-    // the next item do not fill), 32 rows at a time, and stores it row by row: whole contiguous
-    // row segments of C per instruction instead of 32 separate 8-byte pieces, and no workgroup
-    // barrier. When bias, residual or the old C are added (or the output is fp32 / a split-K
+    // the next item do not fill), 32 rows at a time (16 of an oblong tile), and stores it row by row:
+    // whole contiguous row segments of C per instruction instead of 32 separate 8-byte pieces, and no
+    // workgroup barrier. When bias, residual or the old C are added (or the output is fp32 / a split-K
     // partial) the staging is fp32, half the columns per pass, and rounding to the storage dtype
-    // still happens once, after the additions; otherwise the values are rounded in registers and
-    // staged in the storage dtype. A staged row is kRowBytes long; its 16-byte chunk c sits at
+    // still happens once, after the additions; otherwise (and on oblong tiles with a bias, which is
+    // added there) the values are rounded in registers and staged in the storage dtype. A staged row is kRowBytes long; its 16-byte chunk c sits at
     // chunk position c ^ sw(row), which spreads both the column-wise writes and the row-wise reads
     // over all banks.
     constexpr bool kIsF32 = std::is_same_v<T, float>;
@@ -1204,8 +1204,8 @@ __global__ __launch_bounds__(kThreads, DEEP ? 1 : 2) void gemm_pair_kernel(PairA
 }
 
 // The same with tiles of 256 x 128 of the weight gradient and oblong ones of the input gradient, one workgroup per CU and one round of
-// them: 40 per cent less operand traffic per product than 128 x 128 tiles, which the path from the L2s binds. 5005 x 1024 x 2048 is 108 tiles of 192 x 256
-// and 64 of 256 x 128 in two slices, 236 workgroups: 50.5 -> 46.5 us.
+// them: 40 per cent less operand traffic per product than 128 x 128 tiles, which the path from the L2s binds. 5005 x 1024 x 2048 is 92 tiles of 224 x 256
+// and 64 of 256 x 128 in two slices, 220 workgroups: 50.5 -> 46.2 us.
 template <typename T, int BM, int BN>
 __global__ __launch_bounds__(kThreads, 1) void gemm_oblong_pair_kernel(PairArgs pair) {
     extern __shared__ __align__(1024) unsigned char smem_raw[];
