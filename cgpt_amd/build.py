@@ -101,7 +101,8 @@ DISPATCH_PATH = ROOT / "cgpt_amd" / "_dispatch.so"
 
 
 def build_dispatch(force: bool = True) -> pathlib.Path:
-    """Compiles the Python extension behind cgpt_amd/ops.py (host code only: tensor checks against torch's C++ API)."""
+    """Compiles the Python extension behind cgpt_amd/ops.py (host code only: tensor checks against torch's C++ API, and the operators' calls
+    of the library)."""
     deps = [DISPATCH_SOURCE, ROOT / "include" / "cgptx.h"]
     if not force and DISPATCH_PATH.exists() and all(DISPATCH_PATH.stat().st_mtime >= d.stat().st_mtime for d in deps):
         return DISPATCH_PATH

@@ -373,7 +373,7 @@ __device__ __forceinline__ void update_chunk(const DeviceEntry& entry, unsigned 
 
 // ONCE: the state and the gradients are accessed as what is used once (the parameter is not: the next forward pass reads it). Then the
 // statistics pass of the next call does not share the memory with the write-back of this one's state either: 100 M bf16 parameters in
-// 134 tensors, update 512 -> 459 us, statistics 71 -> 43, the call 593 -> 518; 50 M 304 -> 246.
+// 134 tensors, update 513 -> 433 us, statistics 72 -> 57, the call 593 -> 522; 50 M 304 -> 246.
 template <bool ONCE>
 __global__ __launch_bounds__(kThreads) void adamw_update_kernel(const DeviceEntry* __restrict__ entries,
                                                                const unsigned int* __restrict__ chunk_begin,

@@ -189,8 +189,9 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
         (grad_weight != nullptr && input == nullptr))
         return fail(CGPTX_INVALID_ARGUMENT, "linear_backward: null tensor");
     // An output gradient whose rows are not whole 16-byte chunks feeds both contractions from one padded copy (each would
-    // make its own otherwise). So do weight and input of such rows: copied together, they leave the contractions free to share a launch.
-    // Forward and backward, eager, six to nine launches before: bf16 16 x 1379 x 256 with bias 27 - 33 -> 17.5 us, 1000 x 1021 x 1024 with bias, added
+    // make its own otherwise). So do weight and input of such rows: copied together, they leave the contractions free to share a launch, but for
+    // pairs on large tiles whose weight gradient is cut along K: the scratch beside the copies holds no partial tiles for those, and their contractions go one
+    // after the other (9000 x 2047 x 200 128 -> 122.6 us). Forward and backward, eager, six to nine launches before: bf16 16 x 1379 x 256 with bias 27 - 33 -> 17.5 us, 1000 x 1021 x 1024 with bias, added
     // to old gradients 48 -> 35, 5005 x 1023 x 2048 118 -> 99, fp32 200 x 1001 x 500 53 -> 35.
     const std::size_t elem = dtype_size(dtype);
     const void *dy = grad_output, *w = weight, *x = input;
@@ -268,7 +269,8 @@ int cgptx::linear_backward(void* grad_input, void* grad_weight, void* grad_bias,
         const std::size_t dy_copy = pad_out ? bytes_of(rows, dy_pitch) : 0, w_copy = pad_in ? bytes_of(out_features, in_pitch) : 0;
         const std::size_t copy_bytes = dy_copy + w_copy + (pad_in ? bytes_of(rows, in_pitch) : 0);
         split_bytes = std::max(gemm_split_bytes(input_gradient()), gemm_split_bytes(weight_gradient()));
-        // fp32 sums in K slices keep them: 2000 x 65 x 67 in one launch, in one sum over 2000 rows, is 4.0e-7 off the sums in 64 bits, in slices 1.4e-7.
+        // fp32 sums in K slices keep them: 2000 x 65 x 67 in one launch, in one sum over 2000 rows, is 4.0e-7 off the sums in 64 bits, in slices 1.4e-7. In 16-bit
+        // storage, whose rounding is five hundred times that (f16 2000 x 65 x 67 2.011e-4 off either way), such a sum may be one chain.
         const bool keeps_slices = pad_in && dtype == CGPTX_F32 && split_bytes != 0;
         split_bytes += 256;
         void* mem = nullptr;
