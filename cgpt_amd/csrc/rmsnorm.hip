@@ -543,7 +543,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_dual_rows_kernel(
 // --------------------------------------------------------------- generic path
 template <typename T, bool Backward>
 __global__ __launch_bounds__(kThreads) void rmsnorm_row_generic_kernel(
-    T* __restrict__ out, float* __restrict__ inv_rms, const T* __restrict__ dy, const T* __restrict__ x,
+    T* out, float* __restrict__ inv_rms, const T* __restrict__ dy, const T* residual /* may be null or alias out */, const T* __restrict__ x,
     const T* __restrict__ w, int rows, int hidden, float inv_hidden, float eps) {
     __shared__ float red[2][kWavesPerBlock];
     const int lane = threadIdx.x & (kWave - 1);
@@ -576,8 +576,8 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_row_generic_kernel(
             const float corr = dd * inv * inv * inv * inv_hidden;
             if (threadIdx.x == 0) inv_rms[row] = inv;
             for (int col = threadIdx.x; col < hidden; col += kThreads) {
-                out[base + col] = from_f32<T>(to_f32(dy[base + col]) * to_f32(w[col]) * inv -
-                                              to_f32(x[base + col]) * corr);
+                const float gradient = to_f32(dy[base + col]) * to_f32(w[col]) * inv - to_f32(x[base + col]) * corr;
+                out[base + col] = from_f32<T>(residual != nullptr ? gradient + to_f32(residual[base + col]) : gradient);
             }
         } else {
             for (int col = threadIdx.x; col < hidden; col += kThreads) {
@@ -1064,14 +1064,13 @@ int rmsnorm_backward_impl(void* grad_input, void* grad_weight, const void* grad_
         auto* partial = reinterpret_cast<float*>(static_cast<char*>(mem) + inv_bytes);
         const int row_blocks = r < compute_units() * 8 ? r : compute_units() * 8;
         hipLaunchKernelGGL((rmsnorm_row_generic_kernel<T, true>), dim3(row_blocks), dim3(kThreads), 0, stream, dx,
-                           inv_rms, dy, x, w, r, h, 1.0f / static_cast<float>(h), epsilon);
+                           inv_rms, dy, res, x, w, r, h, 1.0f / static_cast<float>(h), epsilon);
         CGPTX_LAUNCH_CHECK();
         hipLaunchKernelGGL((rmsnorm_dgamma_generic_kernel<T>), dim3(reduce_blocks, slices), dim3(kThreads), 0, stream,
                            partial, dy, x, inv_rms, r, h, rows_per_slice);
         CGPTX_LAUNCH_CHECK();
         launch_column_partial_reduce<T>(dw, partial, slices, h, 0, stream);
         CGPTX_LAUNCH_CHECK();
-        if (res != nullptr) return cgptx_add(dx, dx, res, rows * hidden, dtype, stream);
         return CGPTX_OK;
     });
 }
@@ -1184,7 +1183,7 @@ extern "C" int cgptx_rmsnorm_forward(void* output, const void* input, const void
         }
         const int row_blocks = r < compute_units() * 8 ? r : compute_units() * 8;
         hipLaunchKernelGGL((rmsnorm_row_generic_kernel<T, false>), dim3(row_blocks), dim3(kThreads), 0, stream, y,
-                           nullptr, nullptr, x, w, r, h, 1.0f / static_cast<float>(h), epsilon);
+                           nullptr, nullptr, nullptr, x, w, r, h, 1.0f / static_cast<float>(h), epsilon);
         CGPTX_LAUNCH_CHECK();
         return CGPTX_OK;
     });

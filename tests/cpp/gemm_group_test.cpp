@@ -1,7 +1,8 @@
 // The projections of q, k and v as the step of a small model makes them: several contractions in one launch
 // (cgpt_amd/csrc/gemm.hpp), forward as a group of three, backward as one of four whose input gradient reads its operand from
 // three buffers. Operands of -1 .. 1: sums of at most 8192 products are exact in fp32 in any order, so every result is the
-// rounded exact value. Built by `python -m cgpt_amd.build`; run by tests/test_cpp_interface.py on the GPU.
+// rounded exact value. Built by `python -m cgpt_amd.build`; run by tests/test_cpp_interface.py on the GPU. Also what else of a step's parts no
+// entry point of the library reaches: a norm's gradient added to the residual stream's.
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -476,6 +477,55 @@ void check_oblong_forms(std::size_t rows, std::size_t columns, std::size_t k, in
     }
 }
 
+// A norm's input gradient on top of the residual stream's: into a buffer of its own, and in place of it, as a step's blocks add their
+// second branch. Without an output gradient the residual comes out as it went in; with one, both ways give the same bits.
+void check_residual_in_place(std::size_t rows, std::size_t hidden, int dtype, hipStream_t stream) {
+    const std::string name = "norm gradient on a residual, " + std::to_string(rows) + " x " + std::to_string(hidden) + ", type " + std::to_string(dtype);
+    std::printf("%s\n", name.c_str());
+    std::fflush(stdout);
+    const std::size_t elem = dtype == CGPTX_F32 ? 4 : 2, count = rows * hidden;
+    std::mt19937 rng(static_cast<unsigned int>(rows + hidden));
+    using Bytes = std::vector<unsigned char>;
+    auto numbers = [&](std::size_t n, int most) {
+        Bytes bytes(n * elem);
+        for (std::size_t i = 0; i < n; ++i) {
+            const int value = static_cast<int>(rng() % (2 * most + 1)) - most;
+            const auto f = static_cast<float>(value);
+            const std::uint16_t half = rounded(value, dtype);
+            std::memcpy(&bytes[i * elem], elem == 4 ? static_cast<const void*>(&f) : &half, elem);
+        }
+        return bytes;
+    };
+    std::vector<void*> held;
+    auto on_device = [&](const Bytes& bytes) {
+        void* p = nullptr;
+        hip_ok(hipMalloc(&p, bytes.size()), "hipMalloc");
+        hip_ok(hipMemcpy(p, bytes.data(), bytes.size(), hipMemcpyHostToDevice), "hipMemcpy");
+        held.push_back(p);
+        return p;
+    };
+    const Bytes residual = numbers(count, 100), nothing(count * elem);
+    void* const x = on_device(numbers(count, 5));
+    void* const w = on_device(numbers(hidden, 3));
+    void* const dw = on_device(Bytes(hidden * elem));
+    void* const apart = on_device(residual);
+    for (const Bytes& gradient : {nothing, numbers(count, 7)}) {
+        void* const dy = on_device(gradient);
+        void* const out = on_device(nothing);
+        void* const in_place = on_device(residual);
+        expect(cgptx::rmsnorm_backward_residual(out, dw, dy, x, w, apart, rows, hidden, 1e-5f, dtype, stream) == CGPTX_OK, name + ": launch");
+        expect(cgptx::rmsnorm_backward_residual(in_place, dw, dy, x, w, in_place, rows, hidden, 1e-5f, dtype, stream) == CGPTX_OK, name + ": launch in place");
+        hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        Bytes got(count * elem), got_in_place(count * elem);
+        hip_ok(hipMemcpy(got.data(), out, got.size(), hipMemcpyDeviceToHost), "hipMemcpy");
+        hip_ok(hipMemcpy(got_in_place.data(), in_place, got.size(), hipMemcpyDeviceToHost), "hipMemcpy");
+        expect(got == got_in_place, name + ": in place");
+        if (gradient == nothing) expect(got == residual, name + ": no gradient");
+        else if (hidden > 1) expect(got != residual, name + ": a gradient");  // of one column it is next to nothing
+    }
+    for (void* p : held) (void)hipFree(p);
+}
+
 }  // namespace
 
 int main() {
@@ -497,6 +547,9 @@ int main() {
             check_oblong_forms(11871, 1024, 1024, dtype, stream);  // 192 x 256
             check_oblong_forms(12470, 1024, 1024, dtype, stream);  // 224 x 256
         }
+        for (const int dtype : {CGPTX_F32, CGPTX_F16, CGPTX_BF16})
+            for (const std::size_t hidden : {1, 18, 20, 36, 64, 180, 1021, 1024, 5003})  // rows of whole vectors and others
+                for (const std::size_t rows : {1, 130, 2500}) check_residual_in_place(rows, hidden, dtype, stream);
         check_segment_sums(300, 512, 512, 512, stream);
         check_segment_sums(131, 768, 768, 256, stream);
         check_segment_sums(70, 224, 96, 32, stream);  // wavefronts without a K tile of some segments
